@@ -197,10 +197,12 @@ def work(case):
 
 def tolerance(case):
     if case["kind"] == "decoder":
-        # int8 codes behind bf16 norms: evaluating the two RMSNorms in 64 bits moves single gradients by up to 4.7e-2, the
-        # linears' products in 64 bits by up to 2.8e-2
-        return {"rel": 1e-1}
+        # int8 codes behind bf16 activations: the linears' products in 64 bits move single gradients by up to 2.8e-2 (and the
+        # two RMSNorms without their rounding to bf16 in the middle by 4.7e-2), single elements by their own size
+        return {"rel": 3e-2, "max": 0.99}
     double = case["scheme"] == "double_channel" if "scheme" in case else case["api"] == "double_channel"
     if double and not case.get("bias", False):
         return "exact"                          # int32 sums and a fixed order of roundings: one right answer
-    return {"rel": 1.2e-4}                      # the products in 64 bits: up to 3.3e-5 away, bf16 outputs that round the other way
+    # the products in 64 bits: up to 3.3e-5 away.  Those are bf16 outputs that round the other way, each by one ulp (at most
+    # 2^-7 of the value); a bias rounds a second time, and what is left after it may be smaller than what was rounded before
+    return {"rel": 1.2e-4, "max": 4e-2 if case.get("bias", False) else 2e-2}
