@@ -126,7 +126,8 @@ enum ti8_gemm_kernel {
     TI8_KERNEL_ONE_TILE = 1,          /* one workgroup per output tile */
     TI8_KERNEL_ONE_TILE_MULTI = 2,    /* the same, several GEMMs in one launch */
     TI8_KERNEL_PERSISTENT_CHAIN = 3,  /* persistent workgroups, chained block-channel promotion (256 x 256 tiles) */
-    TI8_KERNEL_FEW_ROWS = 4           /* M <= 256: 32 x 32 blocks, K split over the waves */
+    TI8_KERNEL_FEW_ROWS = 4,          /* M <= 256: 32 x 32 blocks, K split over the waves */
+    TI8_KERNEL_MID = 5                /* 128 x 128 tiles, two K tiles at a time on two groups of four waves */
 };
 #define TI8_KERNEL_KIND(id) ((id) & 0xff)
 int ti8_last_gemm_kernel(void);
@@ -316,8 +317,8 @@ int ti8_fwht_t_quant_row(const void* x, int64_t ldx, void* scratch, int8_t* q, i
  *       C = bf16(acc * out_scale) (out_scale = 1 for none).
  * N, K multiples of 128.  M a multiple of 128, or any multiple of 32 up to 256 (decode
  * shapes: only the first M rows of a quantised, zero-padded operand are multiplied; block
- * scales are indexed by row / 128 as usual).  Those M are served by the few-rows kernel
- * only, i.e. not with TI8_GEMM_STRICT / TI8_GEMM_TILED, TI8_SCALE_ROW_K128 or K > 32768. */
+ * scales are indexed by row / 128 as usual).  Those M are served by the few-rows and the
+ * medium-size kernel only, i.e. not with TI8_GEMM_STRICT / TI8_GEMM_TILED, TI8_SCALE_ROW_K128 or K > 32768. */
 int ti8_gemm_i8_nt(const int8_t* A, int64_t bsa, int64_t lda,
                    const int8_t* B, int64_t bsb, int64_t ldb,
                    void* C, int64_t bsc, int64_t ldc,
@@ -333,9 +334,8 @@ int ti8_gemm_i8_nt(const int8_t* A, int64_t bsa, int64_t lda,
  * triton/block_channel_bwd33.py:72) when all their operands are at hand.  Every field means what the
  * argument of that name means in ti8_gemm_i8_nt; `problems` is a HOST array, read before the call
  * returns.  Each GEMM runs the kernel that ti8_gemm_i8_nt with TI8_GEMM_TILED selects for its shape
- * and scale modes, so results are bit-identical to such separate calls; one launch serves them when
- * they all select the same kernel (not TI8_GEMM_STRICT, not TI8_SCALE_ROW_K128), otherwise they are
- * launched one after the other.  TI8_GEMM_SKINNY is refused. */
+ * and scale modes, so results are bit-identical to such separate calls; those that select the same
+ * kernel share one launch (not TI8_GEMM_STRICT, not TI8_SCALE_ROW_K128).  TI8_GEMM_SKINNY is refused. */
 typedef struct ti8_gemm_problem {
     const int8_t* A; int64_t bsa, lda;
     const int8_t* B; int64_t bsb, ldb;

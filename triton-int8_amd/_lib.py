@@ -60,7 +60,7 @@ COMBINE_MUL_MUL, COMBINE_MUL_PROD, COMBINE_DIV_PROD = 0, 1, 2
 GEMM_STRICT, GEMM_TILED, GEMM_SKINNY, GEMM_LARGE_TILES, GEMM_ONE_TILE = 1, 2, 4, 8, 16
 NOALLOC_MAX_ROWS_PLUS_COLS = 65536
 SCHEME_BLOCK_CHANNEL, SCHEME_DOUBLE_CHANNEL = 0, 2
-KERNEL_NONE, KERNEL_ONE_TILE, KERNEL_ONE_TILE_MULTI, KERNEL_PERSISTENT_CHAIN, KERNEL_FEW_ROWS = 0, 1, 2, 3, 4
+KERNEL_NONE, KERNEL_ONE_TILE, KERNEL_ONE_TILE_MULTI, KERNEL_PERSISTENT_CHAIN, KERNEL_FEW_ROWS, KERNEL_MID = 0, 1, 2, 3, 4, 5
 
 _lib = None
 
@@ -154,7 +154,8 @@ _EPILOGUES = ("int32 out", "per-row scales, int32 over the whole K", "promotion 
 _KINDS = {KERNEL_NONE: "none", KERNEL_ONE_TILE: "gemm_i8_kernel (one workgroup per tile)",
           KERNEL_ONE_TILE_MULTI: "gemm_i8_multi_kernel (one workgroup per tile, several GEMMs per launch)",
           KERNEL_PERSISTENT_CHAIN: "gemm_i8_chain_kernel (persistent workgroups)",
-          KERNEL_FEW_ROWS: "gemm_i8_wavering_kernel (few rows)"}
+          KERNEL_FEW_ROWS: "gemm_i8_wavering_kernel (few rows)",
+          KERNEL_MID: "gemm_i8_mid_kernel (two K tiles at a time)"}
 
 
 def describe_gemm_kernel(kernel_id=None):

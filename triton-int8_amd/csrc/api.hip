@@ -37,6 +37,7 @@ extern "C" int ti8_init(void) {
     (void)device_cu_count();
     if (int e = init_gemm_kernels()) return e;
     if (int e = init_skinny_kernels()) return e;
+    if (int e = init_mid_kernels()) return e;
     if (int e = init_fwht_kernels()) return e;
     if (int e = init_quant_scratch()) return e;
     // last: a device that refuses the persistent kernel's 160 KiB of LDS is not an error (the one-tile kernel serves

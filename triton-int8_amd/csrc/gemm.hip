@@ -726,6 +726,12 @@ static int launch_tiled(const char* fn, const GemmArgs& a, int64_t batch, const 
         const int rc = try_chain_persistent(m, &batch, st);
         if (rc != CHAIN_UNAVAILABLE) return rc;
     }
+    if (c.mid) {
+        GemmMulti m;
+        m.count = 1;
+        m.g[0] = a;
+        return launch_mid(m, batch, c.epi == EPI_ROWS, st);
+    }
 #define TI8_GEMM_CASE(BM, BN, WM, WN, EPI) \
     if (c.bm == BM && c.bn == BN && c.epi == EPI) return launch<BM, BN, WM, WN, EPI>(a, batch, st)
     TI8_GEMM_CASE(128, 128, 2, 2, EPI_ROWS);
@@ -738,6 +744,27 @@ static int launch_tiled(const char* fn, const GemmArgs& a, int64_t batch, const 
     TI8_GEMM_CASE(128, 128, 2, 2, EPI_PROMOTE);
 #undef TI8_GEMM_CASE
     return fail(TI8_ERR_MODE, "%s: no kernel for tile %d x %d, epilogue %d", fn, c.bm, c.bn, c.epi);
+}
+
+// GEMMs of batch 1 that all selected the kernel `c`: one launch where that kernel has a several-GEMMs form
+static int launch_group(const char* fn, GemmMulti& m, const idx::GemmConfig& c, bool persistent, hipStream_t st) {
+    if (c.mid) return launch_mid(m, 1, c.epi == EPI_ROWS, st);
+    if (c.epi == EPI_PROMOTE_CHAIN && persistent) {
+        const int64_t ones[GEMM_MULTI_MAX] = {1, 1, 1};
+        const int rc = try_chain_persistent(m, ones, st);
+        if (rc != CHAIN_UNAVAILABLE) return rc;
+    }
+#define TI8_GEMM_CASE(BM, BN, WM, WN, EPI) \
+    if (c.bm == BM && c.bn == BN && c.epi == EPI) return launch_multi<BM, BN, WM, WN, EPI>(m, st)
+    TI8_GEMM_CASE(128, 128, 2, 2, EPI_ROWS);
+    TI8_GEMM_CASE(256, 256, 2, 4, EPI_ROWS);
+    TI8_GEMM_CASE(256, 256, 2, 4, EPI_PROMOTE_CHAIN);
+    TI8_GEMM_CASE(256, 128, 4, 2, EPI_PROMOTE);
+    TI8_GEMM_CASE(128, 128, 2, 2, EPI_PROMOTE);
+#undef TI8_GEMM_CASE
+    for (int i = 0; i < m.count; ++i)
+        if (int e = launch_tiled(fn, m.g[i], 1, c, persistent, st)) return e;
+    return TI8_OK;
 }
 
 }  // namespace ti8
@@ -758,7 +785,15 @@ extern "C" int ti8_gemm_i8_nt(const int8_t* A, int64_t bsa, int64_t lda, const i
     // few rows: too few 256-row tiles to fill the machine, take the kernel that splits N and K finer
     const bool large = (gemm_flags & TI8_GEMM_LARGE_TILES) != 0;
     const bool want_skinny = (gemm_flags & TI8_GEMM_SKINNY) || (!(gemm_flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES)) && M <= 256);
-    if (want_skinny && !a.strict && skinny_supported(a)) return launch_skinny(a, batch, acc_i32_full != 0, st);
+    if (want_skinny && !a.strict && skinny_supported(a)) {
+        if (!(gemm_flags & TI8_GEMM_SKINNY) && idx::gemm_few_rows_prefers_mid(M, N, K, batch, device_cu_count())) {
+            GemmMulti m;
+            m.count = 1;
+            m.g[0] = a;
+            return launch_mid(m, batch, acc_i32_full != 0, st);
+        }
+        return launch_skinny(a, batch, acc_i32_full != 0, st);
+    }
     if (M % 128)
         return fail(TI8_ERR_SHAPE, "%s: M = %lld is not a multiple of 128, which only the few-rows kernel accepts "
                     "(not with TI8_GEMM_STRICT / TI8_GEMM_TILED, per-(row, K tile) scales or K > 32768)", fn, (long long)M);
@@ -774,8 +809,8 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
     GemmMulti m;
     m.count = count;
     idx::GemmConfig c[GEMM_MULTI_MAX];
-    // every GEMM runs the kernel its own shape selects; one launch serves them when they all agree on it
-    bool one_launch = true;
+    // every GEMM runs the kernel its own shape selects (so its bits do not depend on its company); GEMMs that agree on it
+    // share a launch
     for (int i = 0; i < count; ++i) {
         const ti8_gemm_problem& p = problems[i];
         if (int e = prepare_gemm(fn, p, gemm_flags, &m.g[i])) return e;
@@ -783,28 +818,27 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
         if (p.M % 128) return fail(TI8_ERR_SHAPE, "%s: M must be a multiple of 128, GEMM %d has %lld", fn, i, (long long)p.M);
         c[i] = idx::gemm_config(p.M, p.N, p.K, 1, p.acc_i32_full != 0, m.g[i].strict != 0, p.modeA, p.modeB,
                                 (gemm_flags & TI8_GEMM_LARGE_TILES) != 0, device_cu_count());
-        one_launch = one_launch && c[i].bm == c[0].bm && c[i].bn == c[0].bn && c[i].epi == c[0].epi;
     }
-    one_launch = one_launch && c[0].epi != EPI_STRICT && c[0].epi != EPI_PROMOTE_LANE && c[0].epi != EPI_PROMOTE_CHAIN_LANE;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool persistent = !(gemm_flags & TI8_GEMM_ONE_TILE);
-    if (one_launch && c[0].epi == EPI_PROMOTE_CHAIN && persistent) {
-        const int64_t ones[GEMM_MULTI_MAX] = {1, 1, 1};
-        const int rc = try_chain_persistent(m, ones, st);
-        if (rc != CHAIN_UNAVAILABLE) return rc;
+    bool done[GEMM_MULTI_MAX] = {false, false, false}, chains[GEMM_MULTI_MAX];
+    for (int i = 0; i < count; ++i) {
+        GemmMulti one;
+        one.count = 1;
+        one.g[0] = m.g[i];
+        chains[i] = persistent && c[i].epi == EPI_PROMOTE_CHAIN && chain_persistent_supported(one);
     }
-    if (one_launch) {
-#define TI8_GEMM_CASE(BM, BN, WM, WN, EPI) \
-        if (c[0].bm == BM && c[0].bn == BN && c[0].epi == EPI) return launch_multi<BM, BN, WM, WN, EPI>(m, st)
-        TI8_GEMM_CASE(128, 128, 2, 2, EPI_ROWS);
-        TI8_GEMM_CASE(256, 256, 2, 4, EPI_ROWS);
-        TI8_GEMM_CASE(256, 256, 2, 4, EPI_PROMOTE_CHAIN);
-        TI8_GEMM_CASE(256, 128, 4, 2, EPI_PROMOTE);
-        TI8_GEMM_CASE(128, 128, 2, 2, EPI_PROMOTE);
-#undef TI8_GEMM_CASE
+    for (int i = 0; i < count; ++i) {
+        if (done[i]) continue;
+        GemmMulti part;
+        part.count = 0;
+        for (int j = i; j < count; ++j) {
+            if (done[j] || c[j].bm != c[i].bm || c[j].bn != c[i].bn || c[j].epi != c[i].epi || c[j].mid != c[i].mid || chains[j] != chains[i]) continue;
+            part.g[part.count++] = m.g[j];
+            done[j] = true;
+        }
+        if (int e = launch_group(fn, part, c[i], persistent, st)) return e;
     }
-    for (int i = 0; i < count; ++i)
-        if (int e = launch_tiled(fn, m.g[i], 1, c[i], persistent, st)) return e;
     return TI8_OK;
 }
 

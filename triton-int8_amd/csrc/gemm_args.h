@@ -77,6 +77,10 @@ constexpr int CHAIN_UNAVAILABLE = -1;
 bool chain_persistent_supported(const GemmMulti& m);
 int launch_chain_persistent(const GemmMulti& m, int total_tiles, int num_cu, hipStream_t st);
 
+// Kernel for medium sizes (gemm_mid.hip): 128 x 128 tiles, EPI_ROWS (i32_full) or the promotion with factors that are uniform
+// over a wave's tile; K / 128 <= 256.  Fills tiles_m / tiles_n / first of `m`; batch > 1 only with m.count == 1.
+int launch_mid(GemmMulti& m, int64_t batch, bool i32_full, hipStream_t st);
+
 // Kernel for few rows (gemm_skinny.hip): M a multiple of 128, operand A without per-(row, K tile)
 // scales.  i32_full: int32 accumulation over the whole K with per-row scales (bit-exact path).
 bool skinny_supported(const GemmArgs& a);

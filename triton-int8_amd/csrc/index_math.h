@@ -74,6 +74,10 @@ TI8_HD int gemm_wave_first_row(int tile_row0, int wave, int n_instr, int rows) {
     return r >= rows ? r - 128 : r;
 }
 
+// the same for the 32 rows that wave `quarter` (of four) of the medium-size kernel copies; rows is a multiple of 32, and rows
+// past the operand's last re-read its last 32
+TI8_HD int gemm_mid_first_row(int tile_row0, int quarter, int rows) { return imin(tile_row0 + quarter * 32, rows - 32); }
+
 // per-lane byte offset inside the 8-row slab one global->LDS instruction copies: lane l lands at
 // byte 16 l of the 1 KiB LDS slab = (row l/8, physical chunk l%8), and fetches the logical chunk
 // that the XOR swizzle puts there; `parity` = (index of the instruction within the tile) & 1
@@ -255,30 +259,50 @@ TI8_HD int64_t fwht_segment_len(int64_t cols, int64_t n) {
 TI8_HD int fwht_threads(int64_t) { return 256; }   // fwht_kernel: segments of up to 2048 elements (longer ones: fwht_row_kernel)
 
 // LDS-tiled GEMM: tile shape, waves and epilogue kind by shape and scale modes.  `epi` values are
-// the EPI_* constants of gemm_args.h.
+// the EPI_* constants of gemm_args.h; `mid`: the 128 x 128 tiles run on the medium-size kernel (gemm_mid.hip).
 struct GemmConfig {
-    int bm, bn, wm, wn, epi;
+    int bm, bn, wm, wn, epi, mid;
 };
 TI8_HD GemmConfig gemm_config(int64_t M, int64_t N, int64_t K, int64_t batch, bool acc_i32_full, bool strict, int modeA,
                               int modeB, bool large, int num_cu) {
     const int64_t tiles_256x256 = ((M + 255) / 256) * ((N + 255) / 256) * batch;
     const int64_t tiles_256x128 = ((M + 255) / 256) * (N / 128) * batch;
-    if (acc_i32_full) {
-        // medium sizes: when the large tiles would leave CUs without a workgroup, 128 x 128 tiles
-        // (4 waves of 64 x 64, two workgroups per CU)
-        if (!large && tiles_256x256 < num_cu) return GemmConfig{128, 128, 2, 2, 1};
-        return GemmConfig{256, 256, 2, 4, 1};
-    }
-    // the fast promotion keeps at most 256 per-K-tile factors in registers and cannot apply a
-    // factor that varies per row of A inside the loop: those cases take the literal kernel
-    if (strict || modeA == 2 || K > 256 * 128) return GemmConfig{128, 128, 2, 2, 3};
+    const int64_t tiles_128x128 = ((M + 127) / 128) * (N / 128) * batch;
+    // the fast promotion keeps at most 256 per-K-tile factors on chip and cannot apply a factor that varies per row of A
+    // inside the loop: those cases take the literal kernel
+    if (!acc_i32_full && (strict || modeA == 2 || K > 256 * 128)) return GemmConfig{128, 128, 2, 2, 3, 0};
     // operand B scaled per (row, K block): 256 x 256 tiles with the chained promotion where they fill the machine
-    if (modeB == 2) return (large || tiles_256x256 >= num_cu) ? GemmConfig{256, 256, 2, 4, 6} : GemmConfig{256, 128, 4, 2, 4};
-    // 256 x 256 tiles (128 x 64 per wave, float accumulators only) where they fill the machine, else
-    // 256 x 128 (64 x 64 per wave, int32 + float accumulators), else 128 x 128
-    if (large || tiles_256x256 >= num_cu) return GemmConfig{256, 256, 2, 4, 5};
-    if (tiles_256x128 >= num_cu) return GemmConfig{256, 128, 4, 2, 2};
-    return GemmConfig{128, 128, 2, 2, 2};
+    if (!acc_i32_full && modeB == 2) return (large || tiles_256x256 >= num_cu) ? GemmConfig{256, 256, 2, 4, 6, 0} : GemmConfig{256, 128, 4, 2, 4, 0};
+    const GemmConfig big = acc_i32_full ? GemmConfig{256, 256, 2, 4, 1, 0} : GemmConfig{256, 256, 2, 4, 5, 0};
+    const GemmConfig small = acc_i32_full ? GemmConfig{128, 128, 2, 2, 1, 0} : GemmConfig{128, 128, 2, 2, 2, 0};
+    if (large) return big;
+    // Measured at N = 4096, promotion / int32, us.  One 128 x 128 tile per CU at most: the medium-size kernel (1024 rows, K =
+    // 14336: 75.5 / 63.9, four waves 109 / 73.8, 256 x 256 tiles 159 / 121; 384 rows, K = 4096: 24 / 20, 32 / 19, 50 / 39).
+    if (tiles_128x128 <= num_cu) {
+        GemmConfig c = small;
+        c.mid = 1;
+        return c;
+    }
+    // More than half a round of 256 x 256 tiles: idle CUs leave the others a higher clock, and the large tile moves half the
+    // bytes per product (3072 rows, K = 4096, 192 tiles: 61 / 50, 256 x 128 tiles 80, 128 x 128 on four waves - / 55; 768
+    // rows, N = 14336, 168 tiles: 57 / 46 against 79 / 53).
+    if (2 * tiles_256x256 > num_cu) return big;
+    // Exactly one round of 256 x 128 tiles (2048 rows, K = 4096: 46, against 54 on 256 x 256 and 55 on the medium-size kernel)
+    if (!acc_i32_full && tiles_256x128 >= num_cu) return GemmConfig{256, 128, 4, 2, 2, 0};
+    // In between, 128 x 128 tiles on four waves, two workgroups per CU (1536 rows, K = 4096, 384 tiles: 42 / 33, against 52 /
+    // 41 on 256 x 256 tiles and 51 / 42 on the medium-size kernel, whose 129 KiB of LDS leave room for one).
+    return small;
+}
+
+// Up to 256 rows: whether the medium-size kernel beats the few-rows kernel.  The latter's time grows with the bytes its 32 x
+// 32 blocks pull into LDS (0.52 ns per block and K tile on 256 CUs: N = 4096 with 128 rows 10.5 us at K = 4096, 32 us at K = 14336;
+// N = 14336, K = 4096: 31 us at 128 rows, 50 at 256), the former's with the K tiles a workgroup walks (0.85 us per two of them
+// alone, 1.15 with all CUs busy; N = 14336, K = 4096: 22 us at 128 rows, 27 at 256).
+TI8_HD bool gemm_few_rows_prefers_mid(int64_t M, int64_t N, int64_t K, int64_t batch, int num_cu) {
+    const double nk = (double)(K >> 7), blocks = (double)((N / 32) * (M / 32) * batch) * 256.0 / num_cu;
+    const double tiles = (double)(((M + 127) / 128) * (N / 128) * batch) / num_cu;
+    if (tiles > 1.0 || K > 256 * 128) return false;
+    return 7.0 + 0.5 * nk * (0.85 + 0.3 * tiles) < 2.0 + 0.00052 * blocks * nk;
 }
 
 }  // namespace idx

@@ -58,6 +58,7 @@ int device_cu_count();
 int init_gemm_kernels();
 int init_chain_kernel();
 int init_skinny_kernels();
+int init_mid_kernels();
 int init_fwht_kernels();
 int init_quant_scratch();
 
