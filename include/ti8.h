@@ -362,8 +362,8 @@ int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count, int gemm_f
  *                              ti8_gemm_i8_nt_multi(Y, dX, dW; acc_i32_full = 1)
  *   X bf16 [T][K] (ldx), W bf16 [N][K] (ldw), dY bf16 [T][N] (lddy)  ->  Y bf16 [T][N], dX bf16 [T][K], dW bf16 [N][K]
  *   All six 16-byte aligned, leading dimensions multiples of 8 elements; every argument is checked before the first launch.
- *   T, K, N multiples of 128.  `tokens` (1 <= tokens <= T) = the rows of X and dY that hold data when the caller has
- *   zero-padded them to T rows (padded rows change no absmax and add nothing to dW; pass tokens = T otherwise).  With
+ *   T, K, N multiples of 128.  `tokens` (T - 128 < tokens <= T) = the rows of X and dY that exist; the rest of the T rows
+ *   counts as zeros and is not read (zeros change no absmax and add nothing to dW).  With
  *   T <= 256 or N <= 256 the GEMMs are launched one by one, as ti8_gemm_i8_nt would launch them (few-rows kernel up to 256
  *   rows), and Y and dX are computed for the first ceil(tokens / 32) * 32 rows only.
  *   workspace: ti8_linear_fwd_bwd_workspace(T, K, N, scheme) bytes of device memory, 256-byte aligned, contents
@@ -373,6 +373,7 @@ int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count, int gemm_f
  * Nothing is allocated; the call only enqueues kernels, so it may be captured into a graph. */
 enum ti8_scheme {
     TI8_SCHEME_BLOCK_CHANNEL = 0,
+    TI8_SCHEME_ROW_BLOCK = 1,          /* ti8_linear only */
     TI8_SCHEME_DOUBLE_CHANNEL = 2
 };
 /* bytes of workspace the call below needs, or -1 for sizes / a scheme it does not take */
@@ -381,6 +382,49 @@ int ti8_linear_fwd_bwd(const void* X, int64_t ldx, const void* W, int64_t ldw, c
                        void* Y, int64_t ldy, void* dX, int64_t lddx, void* dW, int64_t lddw,
                        int64_t T, int64_t tokens, int64_t K, int64_t N, int scheme, int gemm_flags,
                        void* workspace, int64_t workspace_bytes, ti8_stream_t stream);
+
+/* ---------------------------------------------------------------------------------
+ * The forward, the backward or both of one layer, every scheme and rotation, from one argument block: what a framework's
+ * autograd node enqueues (the reference has no layer; its scripts pay one wrapper per quantiser and per GEMM,
+ * triton/block_channel_fwd32.py:216-241, triton/block_channel_bwd33.py:148-172, triton/double-channle_fwd32.py:269-285).
+ *   X bf16 [tokens][K] (ldx), W bf16 [N][K] (ldw), dY bf16 [tokens][N] (lddy); any number of tokens: the rows between
+ *   `tokens` and T = tokens rounded up to 128 count as zeros and are not read.
+ *   Y bf16 [T][N] (ldy), dX bf16 [T][K] (lddx), dW bf16 [N][K] (lddw); rows of Y and dX from `tokens` on are undefined.
+ *   parts: TI8_PART_FORWARD (X, W -> Y), TI8_PART_BACKWARD (dY, X, W -> dX, dW) or both.  TI8_PART_KEEP: the forward leaves
+ *   what the backward can reuse in `saved` (transposed int8 copies, scales), the backward takes it from there.
+ *   wq, ws: the forward's view of W quantised earlier (int8 [N][K] and its scales in the scheme's layout); W is then not read.
+ *       With TI8_PART_FORWARD alone, without TI8_PART_KEEP.
+ *   hadamard: 0, 128 (block-channel and row-block: H_128 blocks along every contraction dim) or TI8_HADAMARD_FULL (double-channel).
+ *   workspace, saved: sizes from ti8_linear_workspace, 256-byte aligned; contents undefined before and (workspace) after. */
+enum ti8_parts {
+    TI8_PART_FORWARD = 1,
+    TI8_PART_BACKWARD = 2,
+    TI8_PART_KEEP = 4
+};
+enum { TI8_HADAMARD_FULL = -1 };
+typedef struct ti8_linear_args {
+    const void* X; int64_t ldx;
+    const void* W; int64_t ldw;
+    const void* dY; int64_t lddy;
+    void* Y; int64_t ldy;
+    void* dX; int64_t lddx;
+    void* dW; int64_t lddw;
+    const int8_t* wq; const float* ws;
+    int64_t tokens, K, N;
+    int scheme, hadamard, parts, gemm_flags;
+    void* workspace; int64_t workspace_bytes;
+    void* saved; int64_t saved_bytes;
+} ti8_linear_args;
+/* bytes of workspace (and, if `saved_bytes` is not NULL, of saved) that the call needs, or -1 for arguments it does not take;
+ * reads tokens, K, N, scheme, hadamard, parts and whether wq is NULL */
+int64_t ti8_linear_workspace(const ti8_linear_args* a, int64_t* saved_bytes);
+/* enqueue the quantisers only and describe the GEMMs that are left to do in problems[0 .. *count - 1] (at most 3: Y, dX, dW;
+ * M = T for Y and dX), for ti8_gemm_i8_nt_multi */
+int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, int* count, ti8_stream_t stream);
+/* enqueue everything.  With more than 256 (padded) tokens and output features the GEMMs of a call go through
+ * ti8_gemm_i8_nt_multi (TI8_PART_FORWARD alone: ti8_gemm_i8_nt, the same kernel), else they are launched one by one as
+ * ti8_gemm_i8_nt launches them, Y and dX for the first ceil(tokens / 32) * 32 rows only. */
+int ti8_linear(const ti8_linear_args* a, ti8_stream_t stream);
 
 /* Raw int32 accumulators of the same GEMM over the whole K, C int32 [batch][M][N]:
  * the accumulator of int8_gemm_kernel in triton/double-channle_fwd32.py:44,56.

@@ -28,6 +28,14 @@ class GemmProblem(ctypes.Structure):
                 ("out_scale", _f32), ("post_scale", _f32)]
 
 
+class LinearArgs(ctypes.Structure):
+    """ti8_linear_args of include/ti8.h."""
+    _fields_ = [("X", _vp), ("ldx", _i64), ("W", _vp), ("ldw", _i64), ("dY", _vp), ("lddy", _i64), ("Y", _vp), ("ldy", _i64),
+                ("dX", _vp), ("lddx", _i64), ("dW", _vp), ("lddw", _i64), ("wq", _vp), ("ws", _vp),
+                ("tokens", _i64), ("K", _i64), ("N", _i64), ("scheme", _int), ("hadamard", _int), ("parts", _int), ("gemm_flags", _int),
+                ("workspace", _vp), ("workspace_bytes", _i64), ("saved", _vp), ("saved_bytes", _i64)]
+
+
 # name -> argument types, in the order of include/ti8.h
 PROTOTYPES = {
     "ti8_quant_block": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _i64,
@@ -48,9 +56,11 @@ PROTOTYPES = {
     "ti8_gemm_i8_nt_multi": [ctypes.POINTER(GemmProblem), _int, _int, _vp],
     "ti8_gemm_i8_nt_i32": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp],
     "ti8_linear_fwd_bwd": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _i64, _vp],
+    "ti8_linear": [ctypes.POINTER(LinearArgs), _vp],
+    "ti8_linear_quantise": [ctypes.POINTER(LinearArgs), ctypes.POINTER(GemmProblem), ctypes.POINTER(_int), _vp],
     "ti8_probe_mfma": [_vp, _i64, _vp, _int, _int, _int, _int, _vp],
 }
-EXPORTS = ["ti8_version", "ti8_last_error", "ti8_arch", "ti8_init", "ti8_last_gemm_kernel", "ti8_linear_fwd_bwd_workspace"] + list(PROTOTYPES)
+EXPORTS = ["ti8_version", "ti8_last_error", "ti8_arch", "ti8_init", "ti8_last_gemm_kernel", "ti8_linear_fwd_bwd_workspace", "ti8_linear_workspace"] + list(PROTOTYPES)
 
 # enums of include/ti8.h
 Q_CLAMP, Q_EPS_ADD, Q_SCALE_BF16, Q_HAD128, Q_WS_PINGPONG, Q_WS_SECOND, Q_TORCH_ROUND, Q_TORCH_BF16, Q_WS_IS_ZERO = 1, 2, 4, 8, 16, 32, 64, 128, 256
@@ -59,7 +69,9 @@ SCALE_ROW, SCALE_BLOCK128, SCALE_ROW_K128, SCALE_BLOCK_K256 = 0, 1, 2, 3
 COMBINE_MUL_MUL, COMBINE_MUL_PROD, COMBINE_DIV_PROD = 0, 1, 2
 GEMM_STRICT, GEMM_TILED, GEMM_SKINNY, GEMM_LARGE_TILES, GEMM_ONE_TILE = 1, 2, 4, 8, 16
 NOALLOC_MAX_ROWS_PLUS_COLS = 65536
-SCHEME_BLOCK_CHANNEL, SCHEME_DOUBLE_CHANNEL = 0, 2
+SCHEME_BLOCK_CHANNEL, SCHEME_ROW_BLOCK, SCHEME_DOUBLE_CHANNEL = 0, 1, 2
+PART_FORWARD, PART_BACKWARD, PART_KEEP = 1, 2, 4
+HADAMARD_FULL = -1
 KERNEL_NONE, KERNEL_ONE_TILE, KERNEL_ONE_TILE_MULTI, KERNEL_PERSISTENT_CHAIN, KERNEL_FEW_ROWS, KERNEL_MID = 0, 1, 2, 3, 4, 5
 
 _lib = None
@@ -91,6 +103,8 @@ def lib():
         l.ti8_last_gemm_kernel.argtypes = []
         l.ti8_linear_fwd_bwd_workspace.restype = _i64
         l.ti8_linear_fwd_bwd_workspace.argtypes = [_i64, _i64, _i64, _int]
+        l.ti8_linear_workspace.restype = _i64
+        l.ti8_linear_workspace.argtypes = [ctypes.POINTER(LinearArgs), ctypes.POINTER(_i64)]
         for name, args in PROTOTYPES.items():
             fn = getattr(l, name)
             fn.argtypes = args

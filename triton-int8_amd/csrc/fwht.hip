@@ -558,14 +558,15 @@ __global__ __launch_bounds__(NT) void fwht_t_kernel(const uint16_t* __restrict__
 // Thread t reads 8 consecutive columns of row (t / 8) + 32 h; the tile is kept as 32-bit words of
 // two ROWS' elements so that a thread later picks up 8 consecutive rows of one column with 4 reads.
 __global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y,
-                                                             int64_t ldy, int tiles_c) {
+                                                             int64_t ldy, int tiles_c, int64_t valid_rows) {
     __shared__ uint16_t tile[64][64 + 2];   // +2: rows 4 bytes apart modulo the banks
     const int tc = blockIdx.x % tiles_c, tr = blockIdx.x / tiles_c;
     const int tid = threadIdx.x;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
         const int r = (tid >> 3) + 32 * h, c = (tid & 7) * 8;
-        const uint4 v = *reinterpret_cast<const uint4*>(x + ((int64_t)tr * 64 + r) * ldx + (int64_t)tc * 64 + c);
+        uint4 v = make_uint4(0u, 0u, 0u, 0u);   // rows beyond the last (a ragged token count) count as zeros
+        if ((int64_t)tr * 64 + r < valid_rows) v = *reinterpret_cast<const uint4*>(x + ((int64_t)tr * 64 + r) * ldx + (int64_t)tc * 64 + c);
         uint16_t e[8];
         __builtin_memcpy(e, &v, 16);
 #pragma unroll
@@ -655,7 +656,7 @@ extern "C" int ti8_fwht_t(const void* x, int64_t ldx, void* y, int64_t ldy, int6
     // long columns: one or two columns per workgroup would be read 2 or 4 bytes per row and lane; transpose
     // into y with 16-byte accesses instead and transform y in place (the output is the only scratch)
     hipLaunchKernelGGL(transpose_bf16_kernel, dim3((unsigned)((R / 64) * (C / 64))), dim3(256), 0, st, static_cast<const uint16_t*>(x), ldx,
-                       static_cast<uint16_t*>(y), ldy, (int)(C / 64));
+                       static_cast<uint16_t*>(y), ldy, (int)(C / 64), R);
     if (int e = check_launch("ti8_fwht_t")) return e;
     return ti8_fwht(y, ldy, y, ldy, C, R, R, scale, stream);
 }
@@ -715,8 +716,8 @@ extern "C" int ti8_fwht_quant_row(const void* x, int64_t ldx, int8_t* q, int64_t
     return check_launch(fn);
 }
 
-extern "C" int ti8_fwht_t_quant_row(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t C,
-                                    int qflags, int inv_mode, ti8_stream_t stream) {
+int ti8::fwht_t_quant_row_valid(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t valid_rows, int64_t C,
+                                int qflags, int inv_mode, ti8_stream_t stream) {
     const char* fn = "ti8_fwht_t_quant_row";
     if (!x || !scratch || !q || !s) return fail(TI8_ERR_NULL, "%s: x, scratch, q and s are required", fn);
     if (R < 128 || R > 32768 || R % 64 || C <= 0 || C % 64)
@@ -735,7 +736,12 @@ extern "C" int ti8_fwht_t_quant_row(const void* x, int64_t ldx, void* scratch, i
     if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
     if (qflags & (TI8_Q_HAD128 | TI8_Q_SCALE_BF16)) return fail(TI8_ERR_MODE, "%s: only TI8_Q_CLAMP and TI8_Q_EPS_ADD apply here", fn);
     hipLaunchKernelGGL(transpose_bf16_kernel, dim3((unsigned)((R / 64) * (C / 64))), dim3(256), 0, static_cast<hipStream_t>(stream),
-                       static_cast<const uint16_t*>(x), ldx, static_cast<uint16_t*>(scratch), R, (int)(C / 64));
+                       static_cast<const uint16_t*>(x), ldx, static_cast<uint16_t*>(scratch), R, (int)(C / 64), valid_rows);
     if (int e = check_launch(fn)) return e;
     return ti8_fwht_quant_row(scratch, R, q, ldq, s, C, R, n, qflags, inv_mode, stream);
+}
+
+extern "C" int ti8_fwht_t_quant_row(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t C,
+                                    int qflags, int inv_mode, ti8_stream_t stream) {
+    return ti8::fwht_t_quant_row_valid(x, ldx, scratch, q, ldq, s, R, R, C, qflags, inv_mode, stream);
 }

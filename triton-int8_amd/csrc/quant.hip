@@ -95,7 +95,7 @@ template <int NSUB, bool WRITE_Q, bool WRITE_QT, int ARITH = ARITH_KERNEL>
 __device__ __forceinline__ void quant_block_tile(
     const uint16_t* __restrict__ x, int64_t bsx, int64_t ldx, int8_t* __restrict__ q, int64_t bsq, int64_t ldq,
     int8_t* __restrict__ qT, int64_t bsqt, int64_t ldqt, float* __restrict__ s, int64_t ssb, int64_t ssr,
-    int64_t ssc, int nrb, int ncb, const QMode& mode, int tile_index, float* red4, uint32_t* tileT) {
+    int64_t ssc, int nrb, int ncb, int valid_rows, const QMode& mode, int tile_index, float* red4, uint32_t* tileT) {
     const idx::TileId tl = idx::qblock_tile(tile_index, nrb, ncb);
     const int b = tl.b, rb = tl.rb, cb = tl.cb;
 
@@ -110,13 +110,27 @@ __device__ __forceinline__ void quant_block_tile(
     const uint32_t ldx_b = (uint32_t)ldx * 2u;
     const uint32_t x_first = (uint32_t)idx::qblock_row(tid, 0, 0) * ldx_b + (uint32_t)idx::qblock_col(tid) * 2u;
     uint4 v[NSUB][2][4];
+    const int here = valid_rows - rb * 128;   // rows of this tile that exist; the others count as zeros (a ragged token count)
+    if (here >= 128) {
 #pragma unroll
-    for (int u = 0; u < NSUB; ++u)
+        for (int u = 0; u < NSUB; ++u)
 #pragma unroll
-        for (int h = 0; h < 2; ++h)
+            for (int h = 0; h < 2; ++h)
 #pragma unroll
-            for (int j = 0; j < 4; ++j)   // row = idx::qblock_row(tid, h, j) = the first row + 64 h + j
-                v[u][h][j] = *reinterpret_cast<const uint4*>(xt + (x_first + (uint32_t)(idx::qblock_row(0, h, j)) * ldx_b + (uint32_t)(u * 256)));
+                for (int j = 0; j < 4; ++j)   // row = idx::qblock_row(tid, h, j) = the first row + 64 h + j
+                    v[u][h][j] = *reinterpret_cast<const uint4*>(xt + (x_first + (uint32_t)(idx::qblock_row(0, h, j)) * ldx_b + (uint32_t)(u * 256)));
+    } else {
+#pragma unroll
+        for (int u = 0; u < NSUB; ++u)
+#pragma unroll
+            for (int h = 0; h < 2; ++h)
+#pragma unroll
+                for (int j = 0; j < 4; ++j) {
+                    v[u][h][j] = make_uint4(0u, 0u, 0u, 0u);
+                    if (idx::qblock_row(tid, h, j) < here)
+                        v[u][h][j] = *reinterpret_cast<const uint4*>(xt + (x_first + (uint32_t)(idx::qblock_row(0, h, j)) * ldx_b + (uint32_t)(u * 256)));
+                }
+    }
 
     float amax = 0.0f;
 #pragma unroll
@@ -183,7 +197,7 @@ __global__ __launch_bounds__(256) void quant_block_kernel(
     int64_t ssc, int nrb, int ncb, QMode mode) {
     __shared__ float red4[4];
     __shared__ uint32_t tileT[WRITE_QT ? 128 * 33 : 1];
-    quant_block_tile<NSUB, WRITE_Q, WRITE_QT, ARITH>(x, bsx, ldx, q, bsq, ldq, qT, bsqt, ldqt, s, ssb, ssr, ssc, nrb, ncb, mode,
+    quant_block_tile<NSUB, WRITE_Q, WRITE_QT, ARITH>(x, bsx, ldx, q, bsq, ldq, qT, bsqt, ldqt, s, ssb, ssr, ssc, nrb, ncb, nrb * 128, mode,
                                                      blockIdx.x, red4, tileT);
 }
 
@@ -201,6 +215,7 @@ struct QBlockOperand {
     float* s;
     int64_t ssb, ssr, ssc;
     int nrb, ncb;
+    int valid_rows;      // rows of x that exist (128 nrb, or fewer with a batch of one): what is missing of the last tiles counts as zeros
 };
 struct QBlockMulti {
     QBlockOperand op[QBLOCK_MULTI_MAX];
@@ -225,7 +240,7 @@ __global__ __launch_bounds__(256) void quant_block_multi_kernel(const QBlockMult
     const QBlockOperand& o = m.op[i];
     const int local = (int)blockIdx.x - m.first[i];
     quant_block_tile<1, WRITE_Q, WRITE_QT, ARITH_KERNEL>(o.x, o.bsx, o.ldx, o.q, o.bsq, o.ldq, o.qT, o.bsqt, o.ldqt, o.s, o.ssb, o.ssr,
-                                                         o.ssc, o.nrb, o.ncb, mode, local, red4, tileT);
+                                                         o.ssc, o.nrb, o.ncb, o.valid_rows, mode, local, red4, tileT);
 }
 
 
@@ -247,7 +262,7 @@ enum { HAD_BLOCK = 0, HAD_COLMAX = 1, HAD_COL = 2 };
 template <bool ALONG_ROWS, int SCALE = HAD_BLOCK>
 __global__ __launch_bounds__(256) void quant_block_had_kernel(
     const uint16_t* __restrict__ x, int64_t bsx, int64_t ldx, int8_t* __restrict__ q, int64_t bsq, int64_t ldq,
-    float* __restrict__ s, int64_t ssb, int64_t ssr, int64_t ssc, int nrb, int ncb, QMode mode,
+    float* __restrict__ s, int64_t ssb, int64_t ssr, int64_t ssc, int nrb, int ncb, int valid_rows, QMode mode,
     unsigned int* __restrict__ ws = nullptr) {
     static_assert(SCALE == HAD_BLOCK || ALONG_ROWS, "column-wise scales go with the rotation along rows");
     __shared__ float red4[4];
@@ -264,12 +279,23 @@ __global__ __launch_bounds__(256) void quant_block_had_kernel(
     const int lc = ALONG_ROWS ? (tid & 15) : cc;   // chunk of the row that this lane loads
 
     const uint16_t* xt = x + b * bsx + (int64_t)rb * 128 * ldx + (int64_t)cb * 128;
+    const int here = valid_rows - rb * 128;   // rows of this tile that exist, the others count as zeros
     uint4 v[2][4];
+    if (here >= 128) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + lc * 8);
+            for (int j = 0; j < 4; ++j)
+                v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + lc * 8);
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[h][j] = make_uint4(0u, 0u, 0u, 0u);
+                if (h * 64 + rg * 4 + j < here) v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + lc * 8);
+            }
+    }
 
     if (ALONG_ROWS) {
         // tile[row][chunk ^ (row >> 3)]: the 16 lanes that later read one column from 16 different
@@ -416,7 +442,7 @@ __global__ void fill_u32_kernel(unsigned int* p, int n, unsigned int v) {
 __global__ __launch_bounds__(256) void quant_col_t_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                           int8_t* __restrict__ qT, int64_t ldqt,
                                                           float* __restrict__ s, const float* __restrict__ ws,
-                                                          int ncb, QMode mode) {
+                                                          int ncb, int valid_rows, QMode mode) {
     __shared__ uint32_t tileT[128 * 33];
     __shared__ __attribute__((aligned(16))) float sc[128];
     const int cb = blockIdx.x % ncb;
@@ -425,12 +451,23 @@ __global__ __launch_bounds__(256) void quant_col_t_kernel(const uint16_t* __rest
     const int cc = tid & 15, rg = tid >> 4;
     const uint16_t* xt = x + (int64_t)rb * 128 * ldx + (int64_t)cb * 128;
 
+    const int here = valid_rows - rb * 128;   // rows of this tile that exist, the others count as zeros
     uint4 v[2][4];
+    if (here >= 128) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + cc * 8);
+            for (int j = 0; j < 4; ++j)
+                v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + cc * 8);
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[h][j] = make_uint4(0u, 0u, 0u, 0u);
+                if (h * 64 + rg * 4 + j < here) v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + cc * 8);
+            }
+    }
 
     // the tile's 128 column scales: one division each, shared through LDS
     if (tid < 128) {
@@ -510,6 +547,7 @@ template <int TR, bool WITH_ROWS>  // TR: rows of x per workgroup (8, 16, ... 12
 __global__ __launch_bounds__(256) void absmax_kernel(const uint16_t* __restrict__ x, int64_t ldx,
                                                      unsigned int* __restrict__ ws_row,
                                                      unsigned int* __restrict__ ws_col, int64_t R, int C) {
+    // R = rows of x that exist; a row beyond them (a ragged token count) has nothing to add to a maximum
     constexpr int NR = TR / 8;
     __shared__ uint4 part[4][32];  // [wave][chunk]: 8 biased column maxima per chunk
     __shared__ uint32_t rowpart[WITH_ROWS ? TR : 1];  // row maxima of the tile (fp32 bit patterns)
@@ -523,9 +561,17 @@ __global__ __launch_bounds__(256) void absmax_kernel(const uint16_t* __restrict_
     for (int i = 0; i < NR; ++i) rmax[i] = ABS_BIAS2;
     if (c0 < C) {
         uint4 v[NR];
+        if (r0 + TR <= R) {
 #pragma unroll
-        for (int i = 0; i < NR; ++i)
-            v[i] = *reinterpret_cast<const uint4*>(x + (r0 + rg + 8 * i) * ldx + c0);
+            for (int i = 0; i < NR; ++i)
+                v[i] = *reinterpret_cast<const uint4*>(x + (r0 + rg + 8 * i) * ldx + c0);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NR; ++i) {
+                v[i] = make_uint4(0u, 0u, 0u, 0u);
+                if (r0 + rg + 8 * i < R) v[i] = *reinterpret_cast<const uint4*>(x + (r0 + rg + 8 * i) * ldx + c0);
+            }
+        }
 #pragma unroll
         for (int i = 0; i < NR; ++i) {
             const uint32_t a0 = abs_biased2(v[i].x), a1 = abs_biased2(v[i].y), a2 = abs_biased2(v[i].z), a3 = abs_biased2(v[i].w);
@@ -583,7 +629,7 @@ __global__ __launch_bounds__(256) void quant_rowcol_kernel(const uint16_t* __res
                                                            int64_t ldqt, float* __restrict__ s_col,
                                                            const float* __restrict__ ws_row,
                                                            const float* __restrict__ ws_col,
-                                                           float* __restrict__ ws_next, int64_t R, int ncb, QMode mode) {
+                                                           float* __restrict__ ws_next, int64_t R, int ncb, int valid_rows, QMode mode) {
     __shared__ uint32_t tileT[128 * 33];
     __shared__ __attribute__((aligned(16))) float sc[256];  // [0,128): row scales, [128,256): column scales
     const int cb = blockIdx.x % ncb;
@@ -592,12 +638,23 @@ __global__ __launch_bounds__(256) void quant_rowcol_kernel(const uint16_t* __res
     const int cc = tid & 15, rg = tid >> 4;
     const uint16_t* xt = x + (int64_t)rb * 128 * ldx + (int64_t)cb * 128;
 
+    const int here = valid_rows - rb * 128;   // rows of this tile that exist, the others count as zeros
     uint4 v[2][4];
+    if (here >= 128) {
 #pragma unroll
-    for (int h = 0; h < 2; ++h)
+        for (int h = 0; h < 2; ++h)
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-            v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + cc * 8);
+            for (int j = 0; j < 4; ++j)
+                v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + cc * 8);
+    } else {
+#pragma unroll
+        for (int h = 0; h < 2; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                v[h][j] = make_uint4(0u, 0u, 0u, 0u);
+                if (h * 64 + rg * 4 + j < here) v[h][j] = *reinterpret_cast<const uint4*>(xt + (int64_t)(h * 64 + rg * 4 + j) * ldx + cc * 8);
+            }
+    }
 
     // the tile's 128 row scales and 128 column scales: one division per thread, shared through LDS
     {
@@ -707,7 +764,7 @@ extern "C" int ti8_quant_block(const void* x, int64_t bsx, int64_t ldx, int8_t* 
 }
 
 extern "C" int ti8_quant_block_multi(const ti8_qblock_operand* operands, int count, int qflags, int inv_mode, ti8_stream_t stream) {
-    return ti8::quant_block_multi_and_clear(operands, count, qflags, inv_mode, nullptr, 0, stream);
+    return ti8::quant_block_multi_and_clear(operands, nullptr, count, qflags, inv_mode, nullptr, 0, stream);
 }
 
 int ti8::fill_words(unsigned int* p, int64_t words, unsigned int value, hipStream_t st) {
@@ -717,7 +774,7 @@ int ti8::fill_words(unsigned int* p, int64_t words, unsigned int value, hipStrea
     return check_launch("fill");
 }
 
-int ti8::quant_block_multi_and_clear(const ti8_qblock_operand* operands, int count, int qflags, int inv_mode,
+int ti8::quant_block_multi_and_clear(const ti8_qblock_operand* operands, const int64_t* valid_rows, int count, int qflags, int inv_mode,
                                      unsigned int* clear, int64_t clear_words, ti8_stream_t stream) {
     const char* fn = "ti8_quant_block_multi";
     QMode mode;
@@ -733,7 +790,7 @@ int ti8::quant_block_multi_and_clear(const ti8_qblock_operand* operands, int cou
         if ((o.q != nullptr) != (operands[0].q != nullptr) || (o.qT != nullptr) != (operands[0].qT != nullptr))
             return fail(TI8_ERR_MODE, "%s: every operand must ask for the same outputs (q, qT or both)", fn);
         m.op[i] = QBlockOperand{static_cast<const uint16_t*>(o.x), o.bsx, o.ldx, o.q, o.bsq, o.ldq, o.qT, o.bsqt, o.ldqt, o.s,
-                                o.ssb, o.ssr, o.ssc, (int)(o.R / 128), (int)(o.C / 128)};
+                                o.ssb, o.ssr, o.ssc, (int)(o.R / 128), (int)(o.C / 128), (int)(valid_rows ? valid_rows[i] : o.R)};
         m.first[i] = (int)total;
         total += o.B * (o.R / 128) * (o.C / 128);
         if (total > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
@@ -803,8 +860,8 @@ extern "C" int ti8_quant_row(const void* x, int64_t ldx, int8_t* q, int64_t ldq,
     return check_launch("ti8_quant_row");
 }
 
-extern "C" int ti8_quant_col_t(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt, float* s, float* ws,
-                               int64_t R, int64_t C, int qflags, int inv_mode, ti8_stream_t stream) {
+int ti8::quant_col_t_valid(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt, float* s, float* ws,
+                           int64_t R, int64_t valid_rows, int64_t C, int qflags, int inv_mode, ti8_stream_t stream) {
     QMode mode;
     if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
     if (!x || !qT || !s || !ws) return fail(TI8_ERR_NULL, "ti8_quant_col_t: x, qT, s and ws are required");
@@ -824,22 +881,27 @@ extern "C" int ti8_quant_col_t(const void* x, int64_t ldx, int8_t* qT, int64_t l
         // dim): both passes redo the rotation on the tile they read instead of storing it
         const int nrb = (int)(R / 128), ncb = (int)(C / 128);
         hipLaunchKernelGGL((quant_block_had_kernel<true, HAD_COLMAX>), dim3((unsigned)ntiles), dim3(256), 0, st, xp, (int64_t)0, ldx,
-                           qT, (int64_t)0, ldqt, s, (int64_t)0, (int64_t)0, (int64_t)0, nrb, ncb, mode, wsu);
+                           qT, (int64_t)0, ldqt, s, (int64_t)0, (int64_t)0, (int64_t)0, nrb, ncb, (int)valid_rows, mode, wsu);
         hipLaunchKernelGGL((quant_block_had_kernel<true, HAD_COL>), dim3((unsigned)ntiles), dim3(256), 0, st, xp, (int64_t)0, ldx,
-                           qT, (int64_t)0, ldqt, s, (int64_t)0, (int64_t)0, (int64_t)0, nrb, ncb, mode, wsu);
+                           qT, (int64_t)0, ldqt, s, (int64_t)0, (int64_t)0, (int64_t)0, nrb, ncb, (int)valid_rows, mode, wsu);
         return check_launch("ti8_quant_col_t");
     }
     hipLaunchKernelGGL((absmax_kernel<ABSMAX_ROWS, false>), dim3((unsigned)((C + 255) / 256), (unsigned)(R / ABSMAX_ROWS)),
-                       dim3(256), 0, st, xp, ldx, (unsigned int*)nullptr, wsu, R, (int)C);
+                       dim3(256), 0, st, xp, ldx, (unsigned int*)nullptr, wsu, valid_rows, (int)C);
     hipLaunchKernelGGL(quant_col_t_kernel, dim3((unsigned)ntiles), dim3(256), 0, st, xp, ldx, qT, ldqt, s, ws,
-                       (int)(C / 128), mode);
+                       (int)(C / 128), (int)valid_rows, mode);
     return check_launch("ti8_quant_col_t");
 }
 
+extern "C" int ti8_quant_col_t(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt, float* s, float* ws,
+                               int64_t R, int64_t C, int qflags, int inv_mode, ti8_stream_t stream) {
+    return ti8::quant_col_t_valid(x, ldx, qT, ldqt, s, ws, R, R, C, qflags, inv_mode, stream);
+}
+
 // The launches of ti8_quant_row_col_t on a workspace the caller of this function has settled on
-static int quant_row_col_t_impl(const char* fn, const void* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT,
-                                int64_t ldqt, float* s_col, float* ws, int64_t R, int64_t C, int qflags, int inv_mode,
-                                ti8_stream_t stream) {
+int ti8::quant_row_col_t_valid(const char* fn, const void* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT,
+                               int64_t ldqt, float* s_col, float* ws, int64_t R, int64_t valid_rows, int64_t C, int qflags, int inv_mode,
+                               ti8_stream_t stream) {
     const bool pingpong = (qflags & TI8_Q_WS_PINGPONG) != 0, second = (qflags & TI8_Q_WS_SECOND) != 0;
     const bool is_zero = (qflags & TI8_Q_WS_IS_ZERO) != 0;
     if (second && !pingpong) return fail(TI8_ERR_MODE, "%s: TI8_Q_WS_SECOND needs TI8_Q_WS_PINGPONG", fn);
@@ -866,16 +928,16 @@ static int quant_row_col_t_impl(const char* fn, const void* x, int64_t ldx, int8
     if (!pingpong && !is_zero)
         hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)((R + C + 255) / 256)), dim3(256), 0, st, wsu, (int)(R + C), 0u);
     hipLaunchKernelGGL((absmax_kernel<ABSMAX_ROWS, true>), dim3((unsigned)((C + 255) / 256), (unsigned)(R / ABSMAX_ROWS)),
-                       dim3(256), 0, st, xp, ldx, wsu, wsu + R, R, (int)C);
+                       dim3(256), 0, st, xp, ldx, wsu, wsu + R, valid_rows, (int)C);
     hipLaunchKernelGGL(quant_rowcol_kernel, dim3((unsigned)ntiles), dim3(256), 0, st, xp, ldx, q, ldq, s_row, qT, ldqt,
-                       s_col, ws, ws + R, ws_next, R, (int)(C / 128), mode);
+                       s_col, ws, ws + R, ws_next, R, (int)(C / 128), (int)valid_rows, mode);
     return check_launch(fn);
 }
 
 extern "C" int ti8_quant_row_col_t(const void* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT,
                                    int64_t ldqt, float* s_col, float* ws, int64_t R, int64_t C, int qflags,
                                    int inv_mode, ti8_stream_t stream) {
-    return quant_row_col_t_impl("ti8_quant_row_col_t", x, ldx, q, ldq, s_row, qT, ldqt, s_col, ws, R, C, qflags, inv_mode, stream);
+    return ti8::quant_row_col_t_valid("ti8_quant_row_col_t", x, ldx, q, ldq, s_row, qT, ldqt, s_col, ws, R, R, C, qflags, inv_mode, stream);
 }
 
 // ---------------------------------------------------------------------------------
@@ -926,12 +988,12 @@ extern "C" int ti8_quant_row_col_t_noalloc(const void* x, int64_t ldx, int8_t* q
     if (int e = scratch_address(fn, &ws)) return e;
     // the array keeps the last call's maxima: the shared launch sequence starts with the fill kernel
     // that zeroes the R + C words this call uses (a kernel, not a memset, so the call can be captured)
-    return quant_row_col_t_impl(fn, x, ldx, q, ldq, s_row, qT, ldqt, s_col, ws, R, C, qflags, inv_mode, stream);
+    return ti8::quant_row_col_t_valid(fn, x, ldx, q, ldq, s_row, qT, ldqt, s_col, ws, R, R, C, qflags, inv_mode, stream);
 }
 
-extern "C" int ti8_quant_block_had128(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq,
-                                      float* s, int64_t ssb, int64_t ssr, int64_t ssc, int64_t B, int64_t R, int64_t C,
-                                      int along_rows, int qflags, int inv_mode, ti8_stream_t stream) {
+int ti8::quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq,
+                                  float* s, int64_t ssb, int64_t ssr, int64_t ssc, int64_t B, int64_t R, int64_t valid_rows, int64_t C,
+                                  int along_rows, int qflags, int inv_mode, ti8_stream_t stream) {
     QMode mode;
     if (int e = parse_mode(qflags & ~TI8_Q_HAD128, inv_mode, &mode)) return e;
     if (!x || !q || !s) return fail(TI8_ERR_NULL, "ti8_quant_block_had128: x, q and s are required");
@@ -945,8 +1007,14 @@ extern "C" int ti8_quant_block_had128(const void* x, int64_t bsx, int64_t ldx, i
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     if (along_rows)
-        hipLaunchKernelGGL(quant_block_had_kernel<true>, dim3((unsigned)ntiles), dim3(256), 0, st, xp, bsx, ldx, q, bsq, ldq, s, ssb, ssr, ssc, (int)(R / 128), (int)(C / 128), mode);
+        hipLaunchKernelGGL(quant_block_had_kernel<true>, dim3((unsigned)ntiles), dim3(256), 0, st, xp, bsx, ldx, q, bsq, ldq, s, ssb, ssr, ssc, (int)(R / 128), (int)(C / 128), (int)valid_rows, mode);
     else
-        hipLaunchKernelGGL(quant_block_had_kernel<false>, dim3((unsigned)ntiles), dim3(256), 0, st, xp, bsx, ldx, q, bsq, ldq, s, ssb, ssr, ssc, (int)(R / 128), (int)(C / 128), mode);
+        hipLaunchKernelGGL(quant_block_had_kernel<false>, dim3((unsigned)ntiles), dim3(256), 0, st, xp, bsx, ldx, q, bsq, ldq, s, ssb, ssr, ssc, (int)(R / 128), (int)(C / 128), (int)valid_rows, mode);
     return check_launch("ti8_quant_block_had128");
+}
+
+extern "C" int ti8_quant_block_had128(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq,
+                                      float* s, int64_t ssb, int64_t ssr, int64_t ssc, int64_t B, int64_t R, int64_t C,
+                                      int along_rows, int qflags, int inv_mode, ti8_stream_t stream) {
+    return ti8::quant_block_had128_valid(x, bsx, ldx, q, bsq, ldq, s, ssb, ssr, ssc, B, R, R, C, along_rows, qflags, inv_mode, stream);
 }

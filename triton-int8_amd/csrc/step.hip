@@ -1,8 +1,8 @@
-// One training step of the INT8 linear layer -- Y = X W^T, dX = dY W, dW = dY^T X -- enqueued by ONE call:
-// the quantiser launches and the GEMM launch(es) that the Python layer would otherwise issue one entry point at
-// a time, on caller-provided outputs and a caller-provided workspace.  Nothing here computes: the entry points
-// of quant.hip and gemm.hip are called in the order of a step with sub-buffers of the workspace, so every tensor
-// (int8 operands, scales, bf16 outputs) has the bits the separate calls give.
+// The INT8 linear layer -- Y = X W^T, dX = dY W, dW = dY^T X -- enqueued by ONE call: the quantiser launches and the GEMM
+// launch(es) of a forward, a backward or a whole step that the Python layer would otherwise issue one entry point at a time, on
+// caller-provided outputs and a caller-provided workspace.  Nothing here computes: the entry points of quant.hip, fwht.hip and
+// gemm.hip are called in the order of a step with sub-buffers of the workspace, so every tensor (int8 operands, scales, bf16
+// outputs) has the bits the separate calls give.
 #include "ti8_common.h"
 
 namespace ti8 {
@@ -15,100 +15,339 @@ struct Carver {
     int64_t used = 0;
     template <class T>
     T* take(int64_t count) {
-        T* p = base ? reinterpret_cast<T*>(base + used) : nullptr;
+        T* p = reinterpret_cast<T*>(base + used);
         used += (count * (int64_t)sizeof(T) + 255) / 256 * 256;
         return p;
     }
 };
 
-// what one operand needs when it is quantised by rows and by columns (ti8_quant_row_col_t)
-struct RowCol {
-    int8_t* q;
-    int8_t* qT;
-    float* s_row;
-    float* s_col;
-    float* maxima;   // R + C words, zero on entry of the quantiser
-    void carve(Carver& c, int64_t R, int64_t C, bool own_maxima) {
-        q = c.take<int8_t>(R * C);
-        qT = c.take<int8_t>(R * C);
-        s_row = c.take<float>(R);
-        s_col = c.take<float>(C);
-        maxima = own_maxima ? c.take<float>(R + C) : nullptr;
-    }
-};
-
-// what one operand needs when it is quantised by 128 x 128 blocks with a transposed copy (ti8_quant_block)
-struct Blocks {
-    int8_t* q;
-    int8_t* qT;
-    float* s;        // [R / 128][C / 128]
-    void carve(Carver& c, int64_t R, int64_t C) {
-        q = c.take<int8_t>(R * C);
-        qT = c.take<int8_t>(R * C);
-        s = c.take<float>((R / 128) * (C / 128));
-    }
-};
-
-struct BlockChannelLayout {
-    Blocks x, dy;
-    RowCol w;
-    int64_t carve(char* base, int64_t T, int64_t K, int64_t N) {
-        Carver c{base};
-        x.carve(c, T, K);
-        dy.carve(c, T, N);
-        w.carve(c, N, K, true);
-        return c.used;
-    }
-};
-
-struct DoubleChannelLayout {
-    RowCol x, w, dy;
-    float* maxima;     // the three operands' maxima in one piece, so that one fill clears them
+// One call: its arguments with the token dim rounded up, and where every operand lives.
+struct Layer {
+    const ti8_linear_args* a;
+    int64_t T, K, N, tokens;
+    int scheme, had;
+    bool fwd, bwd, keep;
+    // operands of Y = X W^T, dX = dY W, dW = dY^T X and their scales
+    int8_t *xq, *wq, *dq, *wtq, *dytq, *xtq;
+    float *xs, *ws, *ds, *wts, *dyts, *xts;
+    unsigned int* maxima;       // row and column maxima of the operands quantised both ways, in one piece
     int64_t maxima_words;
-    int64_t carve(char* base, int64_t T, int64_t K, int64_t N) {
-        Carver c{base};
-        x.carve(c, T, K, false);
-        w.carve(c, N, K, false);
-        dy.carve(c, T, N, false);
-        maxima_words = (T + K) + (N + K) + (T + N);
-        maxima = c.take<float>(maxima_words);
-        x.maxima = maxima;
-        w.maxima = maxima ? maxima + (T + K) : nullptr;
-        dy.maxima = maxima ? maxima + (T + K) + (N + K) : nullptr;
-        return c.used;
+    uint16_t* scratch;          // transposed bf16 copy in front of a rotation along the rows
+
+    bool block() const { return scheme == TI8_SCHEME_BLOCK_CHANNEL; }
+    bool row_block() const { return scheme == TI8_SCHEME_ROW_BLOCK; }
+    bool dbl() const { return scheme == TI8_SCHEME_DOUBLE_CHANNEL; }
+    // what an unrotated forward quantises for the backward in the same pass
+    bool shares() const { return had == 0 && (keep || (fwd && bwd)); }
+    bool given_w() const { return a->wq != nullptr; }
+
+    // The sizes alone: laid out at an address that is not null (a buffer already placed is told by that) and not used
+    int64_t size(int64_t* saved_bytes) {
+        char* const nowhere = reinterpret_cast<char*>(256);
+        return carve(nowhere, nowhere, saved_bytes);
+    }
+    // Lay the buffers out; returns the bytes of workspace, *saved_bytes those of `saved`.
+    int64_t carve(char* ws_base, char* saved_base, int64_t* saved_bytes) {
+        Carver w{ws_base}, kept{saved_base};
+        Carver& k = keep ? kept : w;
+        const int64_t gk = K / 128, gn = N / 128, gt = T / 128;
+        xq = wq = dq = wtq = dytq = xtq = nullptr;
+        xs = ws = ds = wts = dyts = xts = nullptr;
+        maxima_words = 0;
+        maxima = nullptr;
+        scratch = nullptr;
+        // Reused by the backward (in `saved` when the two are separate calls): block-channel X^T and its grid, W^T by rows;
+        // row-block W^T and its grid; double-channel X^T and W^T by rows
+        const bool shared = shares();
+        if (shared) {
+            if (!row_block()) xtq = k.take<int8_t>(T * K);
+            wtq = k.take<int8_t>(N * K);
+            if (block()) { xs = k.take<float>(gt * gk); wts = k.take<float>(K); }
+            if (row_block()) ws = k.take<float>(gn * gk);
+            if (dbl()) { xts = k.take<float>(K); wts = k.take<float>(K); }
+        }
+        if (fwd) {
+            xq = w.take<int8_t>(T * K);
+            if (!xs) xs = w.take<float>(block() ? gt * gk : T);
+            if (given_w()) {
+                wq = const_cast<int8_t*>(a->wq);
+                ws = const_cast<float*>(a->ws);
+            } else {
+                wq = w.take<int8_t>(N * K);
+                if (!ws) ws = w.take<float>(row_block() ? gn * gk : N);
+            }
+        }
+        if (bwd) {
+            dq = w.take<int8_t>(T * N);
+            ds = w.take<float>(block() ? gt * gn : T);
+            dytq = w.take<int8_t>(T * N);
+            if (block() && had == 0) dyts = ds;
+            else dyts = w.take<float>(block() ? gt * gn : N);
+            if (!wtq) wtq = w.take<int8_t>(N * K);
+            if (!wts) wts = row_block() ? (ws && had == 0 ? ws : w.take<float>(gn * gk)) : w.take<float>(K);
+            if (!xtq) xtq = w.take<int8_t>(T * K);
+            if (!xts) xts = block() && had == 0 && xs ? xs : w.take<float>(dbl() ? K : gt * gk);
+            if (dbl() && had) {
+                int64_t big = N * K;
+                if (T * N > big) big = T * N;
+                if (T * K > big) big = T * K;
+                scratch = w.take<uint16_t>(big);
+            }
+        }
+        // maxima: W by rows and columns in the forward (or W by columns in a backward that found nothing saved), dY and, for
+        // the double-channel scheme, X likewise
+        if (shared && fwd && !row_block()) maxima_words += N + K;
+        if (shared && fwd && dbl()) maxima_words += T + K;
+        if (bwd && had == 0 && !block()) maxima_words += T + N;
+        if (bwd && !shared && !row_block() && !(dbl() && had)) maxima_words += K;      // W^T by columns
+        if (bwd && !shared && dbl() && !had) maxima_words += K;                        // X^T by columns
+        if (bwd && row_block() && had) maxima_words += N;                              // dY^T by rotated columns
+        if (maxima_words) maxima = w.take<unsigned int>(maxima_words);
+        if (saved_bytes) *saved_bytes = kept.used;
+        return w.used;
     }
 };
 
-ti8_gemm_problem gemm2d(const int8_t* A, int64_t lda, const float* sA, int modeA, int64_t sa_rs, int64_t sa_ks,
-                        const int8_t* B, int64_t ldb, const float* sB, int modeB, int64_t sb_rs, int64_t sb_ks,
-                        void* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int acc_i32_full) {
+ti8_gemm_problem gemm2d(const int8_t* A, const float* sA, int modeA, int64_t sa_rs, int64_t sa_ks, const int8_t* B, const float* sB, int modeB,
+                        int64_t sb_rs, int64_t sb_ks, void* C, int64_t ldc, int64_t M, int64_t N, int64_t K, int acc_i32_full, float out_scale, float post_scale) {
     ti8_gemm_problem p;
-    p.A = A; p.bsa = 0; p.lda = lda;
-    p.B = B; p.bsb = 0; p.ldb = ldb;
+    p.A = A; p.bsa = 0; p.lda = K;
+    p.B = B; p.bsb = 0; p.ldb = K;
     p.C = C; p.bsc = 0; p.ldc = ldc;
     p.sA = sA; p.modeA = modeA; p.sa_bs = 0; p.sa_rs = sa_rs; p.sa_ks = sa_ks;
     p.sB = sB; p.modeB = modeB; p.sb_bs = 0; p.sb_rs = sb_rs; p.sb_ks = sb_ks;
     p.batch = 1; p.M = M; p.N = N; p.K = K;
     p.acc_i32_full = acc_i32_full; p.combine = TI8_COMBINE_MUL_MUL;
-    p.out_scale = 1.0f; p.post_scale = 0.0f;
+    p.out_scale = out_scale; p.post_scale = post_scale;
     return p;
 }
 
-int check_step(const char* fn, const void* X, int64_t ldx, const void* W, int64_t ldw, const void* dY, int64_t lddy, const void* Y,
-               int64_t ldy, const void* dX, int64_t lddx, const void* dW, int64_t lddw, int64_t T, int64_t tokens, int64_t K, int64_t N, int scheme) {
-    if (scheme != TI8_SCHEME_BLOCK_CHANNEL && scheme != TI8_SCHEME_DOUBLE_CHANNEL)
-        return fail(TI8_ERR_MODE, "%s: scheme must be TI8_SCHEME_BLOCK_CHANNEL or TI8_SCHEME_DOUBLE_CHANNEL, got %d", fn, scheme);
-    if (!X || !W || !dY || !Y || !dX || !dW) return fail(TI8_ERR_NULL, "%s: X, W, dY, Y, dX and dW are required", fn);
+// Argument checks of every layer call, made before the first launch; fills the part of `L` that describes the call
+int check_layer(const char* fn, const ti8_linear_args* a, int64_t T, Layer* L) {
+    const int KNOWN = TI8_PART_FORWARD | TI8_PART_BACKWARD | TI8_PART_KEEP;
+    L->a = a;
+    L->T = T; L->K = a->K; L->N = a->N; L->tokens = a->tokens;
+    L->scheme = a->scheme; L->had = a->hadamard;
+    L->fwd = (a->parts & TI8_PART_FORWARD) != 0;
+    L->bwd = (a->parts & TI8_PART_BACKWARD) != 0;
+    L->keep = (a->parts & TI8_PART_KEEP) != 0;
+    if (a->scheme < TI8_SCHEME_BLOCK_CHANNEL || a->scheme > TI8_SCHEME_DOUBLE_CHANNEL) return fail(TI8_ERR_MODE, "%s: unknown scheme %d", fn, a->scheme);
+    if (a->hadamard != 0 && a->hadamard != (L->dbl() ? TI8_HADAMARD_FULL : 128)) return fail(TI8_ERR_MODE, "%s: rotation %d does not go with scheme %d", fn, a->hadamard, a->scheme);
+    if ((a->parts & ~KNOWN) || (!L->fwd && !L->bwd) || (L->fwd && L->bwd && L->keep)) return fail(TI8_ERR_MODE, "%s: bad parts 0x%x", fn, a->parts);
+    if (L->given_w() && (L->bwd || L->keep || !a->ws)) return fail(TI8_ERR_MODE, "%s: a weight quantised earlier serves a forward that keeps nothing, and brings its scales", fn);
+    const int64_t K = a->K, N = a->N;
     if (T <= 0 || K <= 0 || N <= 0 || T % 128 || K % 128 || N % 128 || T > 0x3fffffff || K > 0x3fffffff || N > 0x3fffffff)
         return fail(TI8_ERR_SHAPE, "%s: T, K and N must be positive multiples of 128 (zero-pad the tokens); got T=%lld K=%lld N=%lld", fn,
                     (long long)T, (long long)K, (long long)N);
-    if (tokens < 1 || tokens > T) return fail(TI8_ERR_SHAPE, "%s: tokens must be in [1, T]; got tokens=%lld T=%lld", fn, (long long)tokens, (long long)T);
-    if (ldx < K || ldw < K || lddy < N || ldy < N || lddx < K || lddw < K) return fail(TI8_ERR_SHAPE, "%s: leading dimension smaller than the row length", fn);
-    // what the quantisers (inputs) and the GEMM epilogues (outputs) need, checked here so that nothing is launched before a rejection
-    if (!aligned16(X) || !aligned16(W) || !aligned16(dY) || !aligned16(Y) || !aligned16(dX) || !aligned16(dW) || (ldx % 8) || (ldw % 8) ||
-        (lddy % 8) || (ldy % 8) || (lddx % 8) || (lddw % 8))
-        return fail(TI8_ERR_ALIGN, "%s: X, W, dY, Y, dX and dW must be 16-byte aligned with leading dimensions multiples of 8 elements", fn);
+    if (a->tokens < 1 || a->tokens > T) return fail(TI8_ERR_SHAPE, "%s: tokens must be in [1, T]; got tokens=%lld T=%lld", fn, (long long)a->tokens, (long long)T);
     return TI8_OK;
+}
+
+int check_pointers(const char* fn, const ti8_linear_args* a, const Layer& L) {
+    const bool need_w = !L.given_w() && (L.fwd || !L.shares()), need_x = L.fwd || !L.shares() || L.row_block();
+    if ((need_x && !a->X) || (need_w && !a->W) || (L.bwd && (!a->dY || !a->dX || !a->dW)) || (L.fwd && !a->Y))
+        return fail(TI8_ERR_NULL, "%s: X, W, dY, Y, dX and dW are required", fn);
+    const int64_t K = a->K, N = a->N;
+    auto rows_ok = [](const void* p, int64_t ld, int64_t cols) { return !p || ld >= cols; };
+    auto aligned = [](const void* p, int64_t ld) { return !p || (aligned16(p) && ld % 8 == 0); };
+    if (!rows_ok(a->X, a->ldx, K) || !rows_ok(a->W, a->ldw, K) || (L.bwd && (!rows_ok(a->dY, a->lddy, N) || !rows_ok(a->dX, a->lddx, K) || !rows_ok(a->dW, a->lddw, K))) ||
+        (L.fwd && !rows_ok(a->Y, a->ldy, N)))
+        return fail(TI8_ERR_SHAPE, "%s: leading dimension smaller than the row length", fn);
+    // what the quantisers (inputs) and the GEMM epilogues (outputs) need, checked here so that nothing is launched before a rejection
+    if (!aligned(a->X, a->ldx) || !aligned(a->W, a->ldw) || (L.bwd && (!aligned(a->dY, a->lddy) || !aligned(a->dX, a->lddx) || !aligned(a->dW, a->lddw))) ||
+        (L.fwd && !aligned(a->Y, a->ldy)) || !aligned(a->wq, 0))
+        return fail(TI8_ERR_ALIGN, "%s: X, W, dY, Y, dX and dW must be 16-byte aligned with leading dimensions multiples of 8 elements", fn);
+    // limits of the quantisers that this call launches
+    const bool shared = L.shares(), row_k = L.fwd && (L.row_block() || ((L.had || !shared) && !(L.block() && L.given_w())));
+    const bool row_n = L.bwd && L.had && !L.block();
+    if ((row_k && K > 32768) || (row_n && N > 32768) || (L.dbl() && L.had && L.bwd && L.T > 32768))
+        return fail(TI8_ERR_SHAPE, "%s: per-row quantisation takes up to 32768 columns", fn);
+    if ((!L.block() && !L.had && L.T / 32 > 65535) || (!L.row_block() && N / 32 > 65535)) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
+    if (a->gemm_flags & ~(TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES | TI8_GEMM_ONE_TILE)) return fail(TI8_ERR_MODE, "%s: only TI8_GEMM_TILED, TI8_GEMM_LARGE_TILES and TI8_GEMM_ONE_TILE apply here", fn);
+    return TI8_OK;
+}
+
+int64_t next_pow2(int64_t v) {
+    int64_t n = 128;
+    while (n < v) n <<= 1;
+    return n;
+}
+
+// Enqueue the quantisers of a call and describe its GEMMs.  The order is that of linear_forward + linear_backward in the Python layer.
+int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stream_t stream) {
+    const ti8_linear_args& a = *L.a;
+    const int64_t T = L.T, K = L.K, N = L.N, tok = L.tokens;
+    const hipStream_t st = static_cast<hipStream_t>(stream);
+    const int q = TI8_Q_CLAMP, had = L.had == 128 ? TI8_Q_HAD128 : 0;
+    const int inv = L.dbl() ? TI8_INV_AMAX_DIV_127 : TI8_INV_RCP_OF_SCALE;
+    const bool shared = L.shares();
+    unsigned int* mx = L.maxima;
+    auto take_maxima = [&](int64_t words) {
+        unsigned int* p = mx;
+        mx += words;
+        return reinterpret_cast<float*>(p);
+    };
+    auto row_col = [&](const void* x, int64_t ldx, int8_t* oq, float* os, int8_t* oqT, float* osT, int64_t R, int64_t valid, int64_t C) {
+        return quant_row_col_t_valid(fn, x, ldx, oq, C, os, oqT, R, osT, take_maxima(R + C), R, valid, C, q | TI8_Q_WS_IS_ZERO, inv, stream);
+    };
+    auto blocks = [&](const void* x, int64_t ldx, int8_t* oq, int8_t* oqT, float* os, int64_t R, int64_t C) {
+        return ti8_qblock_operand{x, 0, ldx, oq, R * C, C, oqT, R * C, R, os, 0, C / 128, 1, 1, R, C};
+    };
+    int n = 0;
+    // double-channel without rotation, and the row-block backward: one launch clears all maxima (block-channel: the block
+    // quantiser's launch clears them on the side)
+    const bool own_clear = L.maxima_words && L.had == 0 && !L.block();
+    if (own_clear)
+        if (int e = fill_words(L.maxima, L.maxima_words, 0u, st)) return e;
+    const float rot = L.had == 128 ? 0.0078125f : 1.0f;     // 2^-7: both operands carry an un-normalised H_128
+
+    if (L.fwd) {
+        float post = 0.0f;
+        if (L.block() && L.had) {
+            if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xq, T * K, K, L.xs, 0, K / 128, 1, 1, T, tok, K, 0, q, inv, stream)) return e;
+            if (!L.given_w()) if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q | had, inv, stream)) return e;
+        } else if (L.block()) {
+            ti8_qblock_operand o[2] = {blocks(a.X, a.ldx, L.xq, shared ? L.xtq : nullptr, L.xs, T, K)};
+            int64_t valid[2] = {tok, tok};
+            int operands = 1;
+            if (L.bwd) o[operands++] = blocks(a.dY, a.lddy, L.dq, L.dytq, L.ds, T, N);    // both activations at hand: one launch
+            if (int e = quant_block_multi_and_clear(o, valid, operands, q, inv, L.maxima, L.maxima_words, stream)) return e;
+            if (shared) {
+                if (int e = row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K)) return e;     // rows for Y, columns for dX
+            } else if (!L.given_w()) {
+                if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q, inv, stream)) return e;
+            }
+        } else if (L.row_block()) {
+            if (int e = ti8_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, 0, q | had, inv, stream)) return e;
+            if (L.had) {
+                if (!L.given_w()) if (int e = ti8_quant_block_had128(a.W, 0, a.ldw, L.wq, N * K, K, L.ws, 0, K / 128, 1, 1, N, K, 0, q, inv, stream)) return e;
+            } else if (!L.given_w()) {
+                const ti8_qblock_operand o = blocks(a.W, a.ldw, L.wq, shared ? L.wtq : nullptr, L.ws, N, K);
+                if (int e = ti8_quant_block_multi(&o, 1, q, inv, stream)) return e;
+            }
+        } else if (L.had) {
+            post = (float)(1.0 / (double)K);
+            if (int e = ti8_fwht_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, next_pow2(K), q, inv, stream)) return e;
+            if (!L.given_w()) if (int e = ti8_fwht_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, next_pow2(K), q, inv, stream)) return e;
+        } else if (shared) {
+            if (int e = row_col(a.X, a.ldx, L.xq, L.xs, L.xtq, L.xts, T, tok, K)) return e;
+            if (int e = row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K)) return e;
+        } else {
+            if (int e = ti8_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, 0, q, inv, stream)) return e;
+            if (!L.given_w()) if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q, inv, stream)) return e;
+        }
+        const bool xb = L.block(), wb = L.row_block();
+        g[n++] = gemm2d(L.xq, L.xs, xb ? TI8_SCALE_BLOCK128 : TI8_SCALE_ROW, xb ? K / 128 : 1, xb ? 1 : 0,
+                        L.wq, L.ws, wb ? TI8_SCALE_BLOCK128 : TI8_SCALE_ROW, wb ? K / 128 : 1, wb ? 1 : 0, a.Y, a.ldy, T, N, K, L.dbl(), rot, post);
+    }
+    if (L.bwd) {
+        float post_dx = 0.0f, post_dw = 0.0f;
+        int64_t dyts_rs = 1, dyts_ks = 0, xts_rs = 1, xts_ks = 0, wts_rs = 1, wts_ks = 0;
+        int dyt_mode = TI8_SCALE_ROW, xt_mode = TI8_SCALE_ROW, wt_mode = TI8_SCALE_ROW;
+        // a transposed operand's block scales are the transposed grid: no copy
+        auto grid_t = [](int64_t cols, int64_t* rs, int64_t* ks, int* mode) { *rs = 1; *ks = cols / 128; *mode = TI8_SCALE_BLOCK128; };
+        if (L.block() && L.had) {
+            // H_128 along N for dX, along the tokens for dW: two differently rotated copies
+            if (int e = quant_block_had128_valid(a.dY, 0, a.lddy, L.dq, T * N, N, L.ds, 0, N / 128, 1, 1, T, tok, N, 0, q, inv, stream)) return e;
+            if (int e = quant_col_t_valid(a.W, a.ldw, L.wtq, N, L.wts, take_maxima(K), N, N, K, q | had, inv, stream)) return e;
+            if (int e = quant_block_had128_valid(a.dY, 0, a.lddy, L.dytq, T * N, T, L.dyts, 0, N / 128, 1, 1, T, tok, N, 1, 0, inv, stream)) return e;
+            if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xtq, T * K, T, L.xts, 0, K / 128, 1, 1, T, tok, K, 1, 0, inv, stream)) return e;
+        } else if (L.block()) {
+            if (!L.fwd) {
+                ti8_qblock_operand o = blocks(a.dY, a.lddy, L.dq, L.dytq, L.ds, T, N);
+                if (int e = quant_block_multi_and_clear(&o, &tok, 1, q, inv, nullptr, 0, stream)) return e;
+                if (!shared) {
+                    if (int e = quant_col_t_valid(a.W, a.ldw, L.wtq, N, L.wts, take_maxima(K), N, N, K, q, inv, stream)) return e;
+                    o = blocks(a.X, a.ldx, nullptr, L.xtq, L.xts, T, K);
+                    if (int e = quant_block_multi_and_clear(&o, &tok, 1, q, inv, nullptr, 0, stream)) return e;
+                }
+            }
+        } else if (L.row_block() && L.had) {
+            if (int e = ti8_quant_row(a.dY, a.lddy, L.dq, N, L.ds, tok, N, 0, q | had, inv, stream)) return e;
+            if (int e = ti8_quant_block_had128(a.W, 0, a.ldw, L.wtq, N * K, N, L.wts, 0, K / 128, 1, 1, N, K, 1, q, inv, stream)) return e;
+            if (int e = quant_col_t_valid(a.dY, a.lddy, L.dytq, T, L.dyts, take_maxima(N), T, tok, N, q | had, inv, stream)) return e;
+            if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xtq, T * K, T, L.xts, 0, K / 128, 1, 1, T, tok, K, 1, q, inv, stream)) return e;
+        } else if (L.row_block()) {
+            if (int e = row_col(a.dY, a.lddy, L.dq, L.ds, L.dytq, L.dyts, T, tok, N)) return e;
+            ti8_qblock_operand o;
+            if (!shared) {
+                o = blocks(a.W, a.ldw, nullptr, L.wtq, L.wts, N, K);
+                if (int e = ti8_quant_block_multi(&o, 1, q, inv, stream)) return e;
+            }
+            o = blocks(a.X, a.ldx, nullptr, L.xtq, L.xts, T, K);
+            if (int e = quant_block_multi_and_clear(&o, &tok, 1, q, inv, nullptr, 0, stream)) return e;
+        } else if (L.had) {
+            // the transposed operands are rotated along the rows of the tensors as they lie in memory
+            post_dx = (float)(1.0 / (double)N);
+            post_dw = (float)(1.0 / (double)T);
+            if (int e = ti8_fwht_quant_row(a.dY, a.lddy, L.dq, N, L.ds, tok, N, next_pow2(N), q, inv, stream)) return e;
+            if (int e = ti8_fwht_t_quant_row(a.W, a.ldw, L.scratch, L.wtq, N, L.wts, N, K, q, inv, stream)) return e;
+            if (int e = fwht_t_quant_row_valid(a.dY, a.lddy, L.scratch, L.dytq, T, L.dyts, T, tok, N, q, inv, stream)) return e;
+            if (int e = fwht_t_quant_row_valid(a.X, a.ldx, L.scratch, L.xtq, T, L.xts, T, tok, K, q, inv, stream)) return e;
+        } else {
+            if (int e = row_col(a.dY, a.lddy, L.dq, L.ds, L.dytq, L.dyts, T, tok, N)) return e;
+            if (!shared) {
+                if (int e = quant_col_t_valid(a.W, a.ldw, L.wtq, N, L.wts, take_maxima(K), N, N, K, q, inv, stream)) return e;
+                if (int e = quant_col_t_valid(a.X, a.ldx, L.xtq, T, L.xts, take_maxima(K), T, tok, K, q, inv, stream)) return e;
+            }
+        }
+        if (L.block()) { grid_t(N, &dyts_rs, &dyts_ks, &dyt_mode); grid_t(K, &xts_rs, &xts_ks, &xt_mode); }
+        if (L.row_block()) { grid_t(K, &wts_rs, &wts_ks, &wt_mode); grid_t(K, &xts_rs, &xts_ks, &xt_mode); }
+        g[n++] = gemm2d(L.dq, L.ds, L.block() ? TI8_SCALE_BLOCK128 : TI8_SCALE_ROW, L.block() ? N / 128 : 1, L.block() ? 1 : 0,
+                        L.wtq, L.wts, wt_mode, wts_rs, wts_ks, a.dX, a.lddx, T, K, N, L.dbl(), rot, post_dx);
+        g[n++] = gemm2d(L.dytq, L.dyts, dyt_mode, dyts_rs, dyts_ks, L.xtq, L.xts, xt_mode, xts_rs, xts_ks, a.dW, a.lddw, N, K, T, L.dbl(), rot, post_dw);
+    }
+    *count = n;
+    return TI8_OK;
+}
+
+// One GEMM launched alone (what ti8_gemm_i8_nt selects for its shape: the few-rows kernel up to 256 rows).  `live` rows of A are
+// multiplied: with few tokens the padding rows of the 128-row-quantised operand are zeros whose products nobody reads.
+int one_gemm(const ti8_gemm_problem& p, int64_t live, int gemm_flags, ti8_stream_t stream) {
+    return ti8_gemm_i8_nt(p.A, p.bsa, p.lda, p.B, p.bsb, p.ldb, p.C, p.bsc, p.ldc, p.sA, p.modeA, p.sa_bs, p.sa_rs, p.sa_ks,
+                          p.sB, p.modeB, p.sb_bs, p.sb_rs, p.sb_ks, 1, live, p.N, p.K, p.acc_i32_full, p.combine, p.out_scale, p.post_scale,
+                          gemm_flags, stream);
+}
+
+int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t stream) {
+    const int flags = L.a->gemm_flags;
+    // rows of a token operand to multiply: all of them, or with up to 256 (padded) tokens the real ones rounded up to 32
+    auto live_rows = [&](int64_t contraction) {
+        if (L.T > 256 || (flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES)) || contraction > 32768) return L.T;
+        const int64_t r = (L.tokens + 31) / 32 * 32;
+        return r < L.T ? r : L.T;
+    };
+    // they go into one launch where none of them has so few rows that it would take the few-rows kernel
+    if (L.bwd && (L.T < L.N ? L.T : L.N) > 256) return ti8_gemm_i8_nt_multi(g, count, flags, stream);
+    for (int i = 0; i < count; ++i) {
+        const bool token_rows = i + 1 < count || !L.bwd;     // dW, the last of a backward, has one row per output feature
+        if (int e = one_gemm(g[i], token_rows ? live_rows(g[i].K) : g[i].M, flags, stream)) return e;
+    }
+    return TI8_OK;
+}
+
+int run_layer(const char* fn, const ti8_linear_args* a, int64_t T, ti8_gemm_problem* problems, int* count, ti8_stream_t stream) {
+    Layer L;
+    if (int e = check_layer(fn, a, T, &L)) return e;
+    if (int e = check_pointers(fn, a, L)) return e;
+    int64_t need_saved = 0;
+    const int64_t need = L.size(&need_saved);
+    if (!a->workspace || (reinterpret_cast<uintptr_t>(a->workspace) & 255) || a->workspace_bytes < need)
+        return fail(TI8_ERR_SHAPE, "%s: the workspace must be 256-byte aligned and hold %lld bytes (ti8_linear_workspace); got %lld", fn,
+                    (long long)need, (long long)(a->workspace ? a->workspace_bytes : 0));
+    if (need_saved && (!a->saved || (reinterpret_cast<uintptr_t>(a->saved) & 255) || a->saved_bytes < need_saved))
+        return fail(TI8_ERR_SHAPE, "%s: `saved` must be 256-byte aligned and hold %lld bytes (ti8_linear_workspace); got %lld", fn,
+                    (long long)need_saved, (long long)(a->saved ? a->saved_bytes : 0));
+    L.carve(static_cast<char*>(a->workspace), static_cast<char*>(a->saved), nullptr);
+    ti8_gemm_problem g[3];
+    int n = 0;
+    if (int e = quantise(fn, L, g, &n, stream)) return e;
+    if (problems) {
+        for (int i = 0; i < n; ++i) problems[i] = g[i];
+        *count = n;
+        return TI8_OK;
+    }
+    return gemms(L, g, n, stream);
 }
 
 }  // namespace
@@ -116,20 +355,40 @@ int check_step(const char* fn, const void* X, int64_t ldx, const void* W, int64_
 
 using namespace ti8;
 
-extern "C" int64_t ti8_linear_fwd_bwd_workspace(int64_t T, int64_t K, int64_t N, int scheme) {
-    if (T <= 0 || K <= 0 || N <= 0 || T % 128 || K % 128 || N % 128) return -1;
-    if (scheme == TI8_SCHEME_BLOCK_CHANNEL) return BlockChannelLayout().carve(nullptr, T, K, N);
-    if (scheme == TI8_SCHEME_DOUBLE_CHANNEL) return DoubleChannelLayout().carve(nullptr, T, K, N);
-    return -1;
+extern "C" int64_t ti8_linear_workspace(const ti8_linear_args* a, int64_t* saved_bytes) {
+    if (!a || a->tokens < 1) return -1;
+    Layer L;
+    if (check_layer("ti8_linear_workspace", a, (a->tokens + 127) / 128 * 128, &L)) return -1;
+    return L.size(saved_bytes);
 }
 
-// One GEMM of the step launched alone (what ti8_gemm_i8_nt selects for its shape: the few-rows kernel up to 256 rows).
-// `live` rows of A are multiplied: with few tokens the padding rows of the 128-row-quantised operand are zeros whose
-// products nobody reads.
-static int one_gemm(const ti8_gemm_problem& p, int64_t live, int gemm_flags, ti8_stream_t stream) {
-    return ti8_gemm_i8_nt(p.A, p.bsa, p.lda, p.B, p.bsb, p.ldb, p.C, p.bsc, p.ldc, p.sA, p.modeA, p.sa_bs, p.sa_rs, p.sa_ks,
-                          p.sB, p.modeB, p.sb_bs, p.sb_rs, p.sb_ks, 1, live, p.N, p.K, p.acc_i32_full, p.combine, p.out_scale, p.post_scale,
-                          gemm_flags, stream);
+extern "C" int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, int* count, ti8_stream_t stream) {
+    const char* fn = "ti8_linear_quantise";
+    if (!a || !problems || !count) return fail(TI8_ERR_NULL, "%s: args, problems and count are required", fn);
+    return run_layer(fn, a, (a->tokens + 127) / 128 * 128, problems, count, stream);
+}
+
+extern "C" int ti8_linear(const ti8_linear_args* a, ti8_stream_t stream) {
+    const char* fn = "ti8_linear";
+    if (!a) return fail(TI8_ERR_NULL, "%s: args is required", fn);
+    return run_layer(fn, a, (a->tokens + 127) / 128 * 128, nullptr, nullptr, stream);
+}
+
+// The whole step on a token dim that the caller has rounded up itself
+static ti8_linear_args step_args(int64_t tokens, int64_t K, int64_t N, int scheme) {
+    ti8_linear_args a = {};
+    a.tokens = tokens; a.K = K; a.N = N;
+    a.scheme = scheme;
+    a.parts = TI8_PART_FORWARD | TI8_PART_BACKWARD;
+    return a;
+}
+
+extern "C" int64_t ti8_linear_fwd_bwd_workspace(int64_t T, int64_t K, int64_t N, int scheme) {
+    if (scheme != TI8_SCHEME_BLOCK_CHANNEL && scheme != TI8_SCHEME_DOUBLE_CHANNEL) return -1;
+    const ti8_linear_args a = step_args(T, K, N, scheme);
+    Layer L;
+    if (check_layer("ti8_linear_fwd_bwd_workspace", &a, T, &L)) return -1;
+    return L.size(nullptr);
 }
 
 extern "C" int ti8_linear_fwd_bwd(const void* X, int64_t ldx, const void* W, int64_t ldw, const void* dY, int64_t lddy,
@@ -137,61 +396,12 @@ extern "C" int ti8_linear_fwd_bwd(const void* X, int64_t ldx, const void* W, int
                                   int64_t T, int64_t tokens, int64_t K, int64_t N, int scheme, int gemm_flags,
                                   void* workspace, int64_t workspace_bytes, ti8_stream_t stream) {
     const char* fn = "ti8_linear_fwd_bwd";
-    if (int e = check_step(fn, X, ldx, W, ldw, dY, lddy, Y, ldy, dX, lddx, dW, lddw, T, tokens, K, N, scheme)) return e;
-    const int64_t need = ti8_linear_fwd_bwd_workspace(T, K, N, scheme);
-    if (!workspace || (reinterpret_cast<uintptr_t>(workspace) & 255) || workspace_bytes < need)
-        return fail(TI8_ERR_SHAPE, "%s: the workspace must be 256-byte aligned and hold %lld bytes (ti8_linear_fwd_bwd_workspace); got %lld", fn,
-                    (long long)need, (long long)(workspace ? workspace_bytes : 0));
-    if (gemm_flags & ~(TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES | TI8_GEMM_ONE_TILE)) return fail(TI8_ERR_MODE, "%s: only TI8_GEMM_TILED, TI8_GEMM_LARGE_TILES and TI8_GEMM_ONE_TILE apply here", fn);
-    char* base = static_cast<char*>(workspace);
-    const int q = TI8_Q_CLAMP;
-    // rows of the token operands that Y and dX multiply: all of them, or with up to 256 (padded) tokens the real ones
-    // rounded up to 32, which the few-rows kernel takes
-    auto live_rows = [&](int64_t contraction) {
-        if (T > 256 || (gemm_flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES)) || contraction > 32768) return T;
-        const int64_t r = (tokens + 31) / 32 * 32;
-        return r < T ? r : T;
-    };
-    // the three GEMMs go into one launch where none of them has so few rows that it would take the few-rows kernel
-    const bool one_launch = (T < N ? T : N) > 256;
-
-    if (scheme == TI8_SCHEME_BLOCK_CHANNEL) {
-        // triton/block_channel_fwd32.py:221-222 on (X, W) and on (dY, W^T), triton/block_channel_bwd33.py:153-154 on (dY^T, X^T):
-        // X and dY per 128 x 128 block (one read each; the transposed copies are the dW GEMM's K-contiguous operands and
-        // their scale grids the transposed grids), W per row and per column
-        BlockChannelLayout L;
-        L.carve(base, T, K, N);
-        const ti8_qblock_operand ops[2] = {
-            {X, 0, ldx, L.x.q, T * K, K, L.x.qT, T * K, T, L.x.s, 0, K / 128, 1, 1, T, K},
-            {dY, 0, lddy, L.dy.q, T * N, N, L.dy.qT, T * N, T, L.dy.s, 0, N / 128, 1, 1, T, N}};
-        // the same launch clears the words in which W's maxima are collected next
-        if (int e = quant_block_multi_and_clear(ops, 2, q, TI8_INV_RCP_OF_SCALE, reinterpret_cast<unsigned int*>(L.w.maxima), N + K, stream)) return e;
-        if (int e = ti8_quant_row_col_t(W, ldw, L.w.q, K, L.w.s_row, L.w.qT, N, L.w.s_col, L.w.maxima, N, K, q | TI8_Q_WS_IS_ZERO, TI8_INV_RCP_OF_SCALE, stream)) return e;
-        const ti8_gemm_problem g[3] = {
-            gemm2d(L.x.q, K, L.x.s, TI8_SCALE_BLOCK128, K / 128, 1, L.w.q, K, L.w.s_row, TI8_SCALE_ROW, 1, 0, Y, ldy, T, N, K, 0),
-            gemm2d(L.dy.q, N, L.dy.s, TI8_SCALE_BLOCK128, N / 128, 1, L.w.qT, N, L.w.s_col, TI8_SCALE_ROW, 1, 0, dX, lddx, T, K, N, 0),
-            gemm2d(L.dy.qT, T, L.dy.s, TI8_SCALE_BLOCK128, 1, N / 128, L.x.qT, T, L.x.s, TI8_SCALE_BLOCK128, 1, K / 128, dW, lddw, N, K, T, 0)};
-        if (one_launch) return ti8_gemm_i8_nt_multi(g, 3, gemm_flags, stream);
-        if (int e = one_gemm(g[0], live_rows(K), gemm_flags, stream)) return e;
-        if (int e = one_gemm(g[1], live_rows(N), gemm_flags, stream)) return e;
-        return one_gemm(g[2], N, gemm_flags, stream);
-    }
-
-    // double-channel: every operand per row and per column (triton/double-channle_fwd32.py:277-278 on (X, W) and (dY, W^T),
-    // triton/double_channel_bwd33.py:193-194 on (dY^T, X^T)), int32 accumulation over the whole K
-    DoubleChannelLayout L;
-    L.carve(base, T, K, N);
-    if (int e = fill_words(reinterpret_cast<unsigned int*>(L.maxima), L.maxima_words, 0u, static_cast<hipStream_t>(stream))) return e;
-    const int qz = q | TI8_Q_WS_IS_ZERO;
-    if (int e = ti8_quant_row_col_t(X, ldx, L.x.q, K, L.x.s_row, L.x.qT, T, L.x.s_col, L.x.maxima, T, K, qz, TI8_INV_AMAX_DIV_127, stream)) return e;
-    if (int e = ti8_quant_row_col_t(W, ldw, L.w.q, K, L.w.s_row, L.w.qT, N, L.w.s_col, L.w.maxima, N, K, qz, TI8_INV_AMAX_DIV_127, stream)) return e;
-    if (int e = ti8_quant_row_col_t(dY, lddy, L.dy.q, N, L.dy.s_row, L.dy.qT, T, L.dy.s_col, L.dy.maxima, T, N, qz, TI8_INV_AMAX_DIV_127, stream)) return e;
-    const ti8_gemm_problem g[3] = {
-        gemm2d(L.x.q, K, L.x.s_row, TI8_SCALE_ROW, 1, 0, L.w.q, K, L.w.s_row, TI8_SCALE_ROW, 1, 0, Y, ldy, T, N, K, 1),
-        gemm2d(L.dy.q, N, L.dy.s_row, TI8_SCALE_ROW, 1, 0, L.w.qT, N, L.w.s_col, TI8_SCALE_ROW, 1, 0, dX, lddx, T, K, N, 1),
-        gemm2d(L.dy.qT, T, L.dy.s_col, TI8_SCALE_ROW, 1, 0, L.x.qT, T, L.x.s_col, TI8_SCALE_ROW, 1, 0, dW, lddw, N, K, T, 1)};
-    if (one_launch) return ti8_gemm_i8_nt_multi(g, 3, gemm_flags, stream);
-    if (int e = one_gemm(g[0], live_rows(K), gemm_flags, stream)) return e;
-    if (int e = one_gemm(g[1], live_rows(N), gemm_flags, stream)) return e;
-    return one_gemm(g[2], N, gemm_flags, stream);
+    if (scheme != TI8_SCHEME_BLOCK_CHANNEL && scheme != TI8_SCHEME_DOUBLE_CHANNEL)
+        return fail(TI8_ERR_MODE, "%s: scheme must be TI8_SCHEME_BLOCK_CHANNEL or TI8_SCHEME_DOUBLE_CHANNEL, got %d", fn, scheme);
+    ti8_linear_args a = step_args(tokens, K, N, scheme);
+    a.X = X; a.ldx = ldx; a.W = W; a.ldw = ldw; a.dY = dY; a.lddy = lddy;
+    a.Y = Y; a.ldy = ldy; a.dX = dX; a.lddx = lddx; a.dW = dW; a.lddw = lddw;
+    a.gemm_flags = gemm_flags;
+    a.workspace = workspace; a.workspace_bytes = workspace_bytes;
+    return run_layer(fn, &a, T, nullptr, nullptr, stream);
 }

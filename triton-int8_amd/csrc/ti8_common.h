@@ -62,10 +62,22 @@ int init_mid_kernels();
 int init_fwht_kernels();
 int init_quant_scratch();
 
-// ---- pieces of quant.hip that the one-call step (step.hip) uses --------------------
+// ---- pieces of quant.hip and fwht.hip that the layer calls (step.hip) use ----------
+// `valid_rows` (of R, the rest counts as zeros and is not read): an activation whose token count is no multiple of the tile
+// needs no zero-padded copy.  NULL / R: all of them.
 // ti8_quant_block_multi that also zeroes `clear_words` 32-bit words at `clear` (NULL: nothing) in the same launch
-int quant_block_multi_and_clear(const ti8_qblock_operand* operands, int count, int qflags, int inv_mode,
+int quant_block_multi_and_clear(const ti8_qblock_operand* operands, const int64_t* valid_rows, int count, int qflags, int inv_mode,
                                 unsigned int* clear, int64_t clear_words, ti8_stream_t stream);
+int quant_row_col_t_valid(const char* fn, const void* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT,
+                          int64_t ldqt, float* s_col, float* ws, int64_t R, int64_t valid_rows, int64_t C, int qflags, int inv_mode,
+                          ti8_stream_t stream);
+int quant_col_t_valid(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt, float* s, float* ws, int64_t R, int64_t valid_rows, int64_t C,
+                      int qflags, int inv_mode, ti8_stream_t stream);
+int quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq, float* s, int64_t ssb, int64_t ssr,
+                             int64_t ssc, int64_t B, int64_t R, int64_t valid_rows, int64_t C, int along_rows, int qflags, int inv_mode,
+                             ti8_stream_t stream);
+int fwht_t_quant_row_valid(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t valid_rows, int64_t C,
+                           int qflags, int inv_mode, ti8_stream_t stream);
 int fill_words(unsigned int* p, int64_t words, unsigned int value, hipStream_t st);
 
 // ---- which kernel served the last GEMM call of this thread (ti8_last_gemm_kernel) ---

@@ -28,7 +28,7 @@ column-absmax kernel that never materialises W^T in bf16.
 import torch
 
 from . import ops
-from ._lib import (COMBINE_MUL_MUL, INV_AMAX_DIV_127, INV_RCP_OF_SCALE, SCALE_BLOCK128, SCALE_ROW)
+from ._lib import (COMBINE_MUL_MUL, INV_AMAX_DIV_127, INV_RCP_OF_SCALE, PART_BACKWARD, PART_FORWARD, PART_KEEP, SCALE_BLOCK128, SCALE_ROW)
 
 __all__ = ["quantize_weight", "linear_forward", "linear_backward", "linear_fwd_bwd", "pad_tokens", "Int8LinearFunction", "Int8Linear", "SCHEMES"]
 
@@ -273,15 +273,28 @@ def _one_launch(scheme, hadamard, padded_tokens, out_features):
 
 
 # Schemes whose whole step is one library call (ops.linear_step: the same launches, queued from C) when nothing is
-# rotated.  False: the step is assembled here from the separate entry points (same bits; the tests run both).
+# rotated; the other modes take two (ops.linear_call: the quantisers, then the GEMMs).  False: the step is assembled here from
+# the separate entry points (same bits; the tests run both).
 ONE_CALL_STEP = True
 ONE_CALL_SCHEMES = ("block_channel", "double_channel")
 
 
+def _from_c():
+    """Whether a layer's launches are queued by the library (the few-rows kernel by name is for the separate entry points only)."""
+    return ONE_CALL_STEP and ops.GEMM_PATH in ("auto", "tiled", "large")
+
+
+def _layer_dims(x2, weight, dy2=None):
+    """(tokens, K, N) of a layer call, or ValueError."""
+    if x2.shape[1] != weight.shape[1] or (dy2 is not None and tuple(dy2.shape) != (x2.shape[0], weight.shape[0])):
+        raise ValueError(f"shapes do not fit: X {tuple(x2.shape)}, W {tuple(weight.shape)}" + ("" if dy2 is None else f", dY {tuple(dy2.shape)}"))
+    return x2.shape[0], x2.shape[1], weight.shape[0]
+
+
 def linear_fwd_bwd(X, W, dY, scheme="block_channel", hadamard=None, out=None, workspace=None):
     """One forward + backward of the layer: returns (Y, dX, dW) for X [B,M,K] or [M,K].
-    Any number of tokens is accepted (zero-padded to a multiple of 128, see :func:`pad_tokens`);
-    K and N must be multiples of 128.  ``out`` = (Y [T,N], dX [T,K], dW [N,K]) bf16 tensors to write into and
+    Any number of tokens is accepted (what is missing of the last 128 counts as zeros, see :func:`pad_tokens`; no padded copies are
+    made); K and N must be multiples of 128.  ``out`` = (Y [T,N], dX [T,K], dW [N,K]) bf16 tensors to write into and
     ``workspace`` (``ops.linear_step_workspace_bytes``) are taken where the step is one library call and the token
     count a multiple of 128 (else ValueError): a caller that runs many steps of one shape allocates them once."""
     _check(scheme, hadamard)
@@ -291,15 +304,18 @@ def linear_fwd_bwd(X, W, dY, scheme="block_channel", hadamard=None, out=None, wo
     T = X2.shape[0]
     if T == 0:   # nothing to multiply: empty Y and dX, a zero weight gradient (as torch.nn.functional.linear gives)
         return X.new_empty((*lead, N)), X.new_empty((*lead, K)), W.new_zeros((N, K))
-    X2, dY2 = pad_tokens(X2), pad_tokens(dY2)
-    one_call = ONE_CALL_STEP and scheme in ONE_CALL_SCHEMES and hadamard is None and ops.GEMM_PATH in ("auto", "tiled", "large")
+    one_call = _from_c() and scheme in ONE_CALL_SCHEMES and hadamard is None
     if out is not None or workspace is not None:
-        if not one_call or X2.shape[0] != T:
+        if not one_call or T % 128:
             raise ValueError("`out` / `workspace` go with the one-call step: block_channel or double_channel without rotation, "
                              "tokens a multiple of 128")
     if one_call:
-        Y, dX, dW = ops.linear_step(X2, W, dY2, scheme, tokens=T, out=out, workspace=workspace)
+        Y, dX, dW = ops.linear_step(X2, W, dY2, scheme, out=out, workspace=workspace)
         return Y[:T].reshape(*lead, N), dX[:T].reshape(*lead, K), dW
+    if _from_c():
+        Y, dX, dW, _ = ops.linear_call(PART_FORWARD | PART_BACKWARD, scheme, hadamard, *_layer_dims(X2, W, dY2), X=X2, W=W, dY=dY2)
+        return Y[:T].reshape(*lead, N), dX[:T].reshape(*lead, K), dW
+    X2, dY2 = pad_tokens(X2), pad_tokens(dY2)
     gemms = [] if _one_launch(scheme, hadamard, X2.shape[0], N) else None
     pre = None
     if scheme == "block_channel" and hadamard is None:
@@ -322,35 +338,42 @@ class Int8LinearFunction(torch.autograd.Function):
     def forward(ctx, x, weight, bias, scheme, hadamard):
         K, N = x.shape[-1], weight.shape[0]
         x2 = x.reshape(-1, K)
-        ctx.tokens = x2.shape[0]
+        ctx.tokens = tokens = x2.shape[0]
         ctx.has_bias = bias is not None
-        if ctx.tokens == 0:   # an empty batch: empty output, zero gradients
-            ctx.save_for_backward(x2, weight)
-            return x.new_empty((*x.shape[:-1], N))
-        x2 = pad_tokens(x2)
-        need_bwd = any(ctx.needs_input_grad[:2])
-        y, saved = linear_forward(x2, weight, scheme, hadamard, need_backward=need_bwd, tokens=ctx.tokens)
-        ctx.scheme, ctx.hadamard, ctx.saved_q = scheme, hadamard, saved
-        ctx.has_bias = bias is not None
+        ctx.scheme, ctx.hadamard, ctx.saved_q = scheme, hadamard, None
         ctx.save_for_backward(x2, weight)
-        y = y[:ctx.tokens]
+        if tokens == 0:   # an empty batch: empty output, zero gradients
+            return x.new_empty((*x.shape[:-1], N))
+        need_bwd = any(ctx.needs_input_grad[:2])
+        if _from_c():
+            y, _, _, ctx.saved_q = ops.linear_call(PART_FORWARD | (PART_KEEP if need_bwd else 0), scheme, hadamard,
+                                                   *_layer_dims(x2, weight), X=x2, W=weight)
+        else:
+            y, ctx.saved_q = linear_forward(pad_tokens(x2), weight, scheme, hadamard, need_backward=need_bwd, tokens=tokens)
+        y = y[:tokens]
         if bias is not None:
-            y = y + bias
+            y += bias       # the GEMM's own output: in place
         return y.reshape(*x.shape[:-1], N)
 
     @staticmethod
     def backward(ctx, dy):
         x2, weight = ctx.saved_tensors
         N = weight.shape[0]
-        if ctx.tokens == 0:
+        tokens = ctx.tokens
+        if tokens == 0:
             return dy.new_empty((*dy.shape[:-1], x2.shape[1])), torch.zeros_like(weight), (dy.new_zeros((N,)) if ctx.has_bias else None), None, None
-        dy2 = pad_tokens(dy.reshape(-1, N).contiguous())
-        gemms = [] if _one_launch(ctx.scheme, ctx.hadamard, x2.shape[0], N) else None
-        dx, dw = linear_backward(dy2, x2, weight, ctx.scheme, ctx.hadamard, ctx.saved_q, tokens=ctx.tokens, gemms=gemms)
-        if gemms:
-            ops.gemm_i8_nt_multi(gemms)   # dX and dW in one launch
+        dy2 = dy.reshape(-1, N)
+        if isinstance(ctx.saved_q, torch.Tensor) or (ctx.saved_q is None and _from_c()):
+            _, dx, dw, _ = ops.linear_call(PART_BACKWARD | (PART_KEEP if ctx.saved_q is not None else 0), ctx.scheme, ctx.hadamard,
+                                           *_layer_dims(x2, weight, dy2), X=x2, W=weight, dY=dy2, saved=ctx.saved_q)
+        else:
+            dyp, xp = pad_tokens(dy2.contiguous()), pad_tokens(x2)
+            gemms = [] if _one_launch(ctx.scheme, ctx.hadamard, xp.shape[0], N) else None
+            dx, dw = linear_backward(dyp, xp, weight, ctx.scheme, ctx.hadamard, ctx.saved_q, tokens=tokens, gemms=gemms)
+            if gemms:
+                ops.gemm_i8_nt_multi(gemms)   # dX and dW in one launch
         db = dy2.sum(dim=0).to(dy.dtype) if ctx.has_bias else None
-        return dx[:ctx.tokens].reshape(*dy.shape[:-1], x2.shape[1]), dw, db, None, None
+        return dx[:tokens].reshape(*dy.shape[:-1], x2.shape[1]), dw, db, None, None
 
 
 class Int8Linear(torch.nn.Module):
@@ -380,13 +403,17 @@ class Int8Linear(torch.nn.Module):
         key = (self.weight._version, self.weight.data_ptr(), self.scheme, self.hadamard)
         if self._wq_key != key:
             self._wq, self._wq_key = quantize_weight(self.weight.detach(), self.scheme, self.hadamard), key
-        K = x.shape[-1]
-        x2 = x.reshape(-1, K)
+        x2 = x.reshape(-1, x.shape[-1])
         tokens = x2.shape[0]
-        y, _ = linear_forward(pad_tokens(x2), None, self.scheme, self.hadamard, need_backward=False, wq=self._wq, tokens=tokens)
+        if _from_c():
+            if x2.shape[1] != self.in_features:
+                raise ValueError(f"expected {self.in_features} input features, got {x2.shape[1]}")
+            y = ops.linear_call(PART_FORWARD, self.scheme, self.hadamard, tokens, self.in_features, self.out_features, X=x2, wq=self._wq)[0]
+        else:
+            y, _ = linear_forward(pad_tokens(x2), None, self.scheme, self.hadamard, need_backward=False, wq=self._wq, tokens=tokens)
         y = y[:tokens]
         if self.bias is not None:
-            y = y + self.bias
+            y += self.bias      # the GEMM's own output: in place
         return y.reshape(*x.shape[:-1], self.out_features)
 
     def extra_repr(self):

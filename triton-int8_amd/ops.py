@@ -6,6 +6,8 @@ current torch stream and never synchronises.  Arguments the kernels cannot take
 here, before anything is launched.
 """
 import collections
+import ctypes
+import functools
 import threading
 
 import torch
@@ -30,7 +32,8 @@ GEMM_PERSISTENT = True
 
 
 def _stream():
-    return torch.cuda.current_stream().cuda_stream
+    # the raw handle of torch's current stream without building a Stream object (0.2 instead of 1.5 us of every call)
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
 
 
 def _on_gpu(t):
@@ -452,26 +455,95 @@ def linear_step_workspace_bytes(T, K, N, scheme):
     return n
 
 
+def _gemm_flags():
+    return {"tiled": GEMM_TILED, "large": GEMM_LARGE_TILES}.get(GEMM_PATH, 0) | (0 if GEMM_PERSISTENT else GEMM_ONE_TILE)
+
+
+def _rows16(t):
+    """`t` itself where the library can read its rows in place, else a contiguous copy."""
+    if t.stride(1) != 1 or t.stride(0) % 8 or t.data_ptr() % 16:
+        t = t.contiguous()
+    return t
+
+
+def _workspace(nbytes, device):
+    """Uninitialised device memory for one call, 256-byte aligned."""
+    t = torch.empty((nbytes,), dtype=torch.uint8, device=device)
+    if t.data_ptr() % 256:      # never on a device: its allocations start on such boundaries
+        t = torch.empty((nbytes + 256,), dtype=torch.uint8, device=device)
+        t = t[(-t.data_ptr()) % 256:][:nbytes]
+    return t
+
+
+_SCHEMES = {"block_channel": _lib.SCHEME_BLOCK_CHANNEL, "row_block": _lib.SCHEME_ROW_BLOCK, "double_channel": _lib.SCHEME_DOUBLE_CHANNEL}
+_ROTATIONS = {None: 0, 128: 128, "full": _lib.HADAMARD_FULL}
+
+
+@functools.lru_cache(maxsize=1024)
+def _linear_sizes(tokens, K, N, scheme, hadamard, parts, given_w):
+    """(bytes of workspace, bytes of saved) of a ``ti8_linear`` call."""
+    a = _lib.LinearArgs(tokens=tokens, K=K, N=N, scheme=_SCHEMES[scheme], hadamard=_ROTATIONS[hadamard], parts=parts, wq=1 if given_w else None,
+                        ws=1 if given_w else None)
+    saved = ctypes.c_int64(0)
+    n = _lib.lib().ti8_linear_workspace(ctypes.byref(a), ctypes.byref(saved))
+    _need(n >= 0, f"K and N must be positive multiples of 128, got K={K} N={N}")
+    return n, saved.value
+
+
+def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=None, wq=None, saved=None, one_launch=True):
+    """The forward, the backward or both of a layer in one or two library calls (``ti8_linear``; with ``one_launch`` and more than
+    256 tokens and output features the quantisers as one call and the backward's or step's GEMMs as ``ti8_gemm_i8_nt_multi``).
+    X bf16 [tokens, K], W bf16 [N, K], dY bf16 [tokens, N]: any number of tokens, no padded copies.  ``wq`` = (int8 [N, K], scales) of
+    the weight quantised earlier.  Returns (Y [T, N], dX [T, K], dW [N, K], saved) with None for what `parts` does not ask for; T =
+    tokens rounded up to 128, rows from `tokens` on undefined."""
+    for t, name in ((X, "X"), (W, "W"), (dY, "dY")):
+        if t is not None:
+            _check_bf16(t, name)
+    dev = (X if X is not None else dY).device
+    need, need_saved = _linear_sizes(tokens, K, N, scheme, hadamard, parts, wq is not None)
+    X, W, dY = (t if t is None else _rows16(t) for t in (X, W, dY))
+    T = -(-tokens // 128) * 128
+    Y = dX = dW = None
+    if parts & _lib.PART_FORWARD:
+        Y = torch.empty((T, N), dtype=torch.bfloat16, device=dev)
+        if need_saved:
+            saved = _workspace(need_saved, dev)
+    if parts & _lib.PART_BACKWARD:
+        dX = torch.empty((T, K), dtype=torch.bfloat16, device=dev)
+        dW = torch.empty((N, K), dtype=torch.bfloat16, device=dev)
+    workspace = _workspace(need, dev)
+    ptr = lambda t: None if t is None else t.data_ptr()
+    a = _lib.LinearArgs(ptr(X), 0 if X is None else X.stride(0), ptr(W), 0 if W is None else W.stride(0), ptr(dY), 0 if dY is None else dY.stride(0),
+                        ptr(Y), N, ptr(dX), K, ptr(dW), K, ptr(wq[0]) if wq is not None else None, ptr(wq[1]) if wq is not None else None,
+                        tokens, K, N, _SCHEMES[scheme], _ROTATIONS[hadamard], parts, _gemm_flags(), workspace.data_ptr(), need,
+                        ptr(saved), need_saved)
+    stream = _stream()
+    if one_launch and parts & _lib.PART_BACKWARD and min(T, N) > 256:
+        problems, count = (_lib.GemmProblem * 3)(), ctypes.c_int(0)
+        _lib.call("ti8_linear_quantise", ctypes.byref(a), problems, ctypes.byref(count), stream)
+        _lib.call("ti8_gemm_i8_nt_multi", problems, count.value, a.gemm_flags, stream)
+    else:
+        _lib.call("ti8_linear", ctypes.byref(a), stream)
+    return Y, dX, dW, saved
+
+
 def linear_step(X2, W, dY2, scheme, *, tokens=None, out=None, workspace=None):
     """A whole forward + backward of the layer in ONE library call (``ti8_linear_fwd_bwd``): X2 bf16 [T, K],
     W bf16 [N, K], dY2 bf16 [T, N] -> (Y [T, N], dX [T, K], dW [N, K]), the quantisers and GEMMs of
     ``linear.linear_forward`` + ``linear.linear_backward`` enqueued from C with the same bits.
-    T, K, N multiples of 128; ``tokens`` = rows that hold data when the caller has zero-padded X2 and dY2 (with up to
-    256 rows Y and dX are then computed for the first ceil(tokens / 32) * 32 rows only).  ``out`` = (Y, dX, dW) to write into; ``workspace`` = a uint8 tensor of at least
+    K, N multiples of 128, any T: the outputs Y and dX have T rounded up to 128 rows, those beyond T are undefined.  ``tokens`` = rows
+    that hold data when the caller has zero-padded X2 and dY2 (with up to 256 rows Y and dX are then computed for the first
+    ceil(tokens / 32) * 32 rows only).  ``out`` = (Y, dX, dW) to write into; ``workspace`` = a uint8 tensor of at least
     :func:`linear_step_workspace_bytes` bytes (both allocated here when absent)."""
     for t, name in ((X2, "X"), (W, "W"), (dY2, "dY")):
         _check_bf16(t, name)
         _need(t.dim() == 2, f"{name} must be 2-D")
-    T, K = X2.shape
+    rows, K = X2.shape
     N = W.shape[0]
-    _need(W.shape[1] == K and tuple(dY2.shape) == (T, N), f"shapes do not fit: X {tuple(X2.shape)}, W {tuple(W.shape)}, dY {tuple(dY2.shape)}")
+    _need(W.shape[1] == K and tuple(dY2.shape) == (rows, N), f"shapes do not fit: X {tuple(X2.shape)}, W {tuple(W.shape)}, dY {tuple(dY2.shape)}")
+    T = -(-rows // 128) * 128
     need = linear_step_workspace_bytes(T, K, N, scheme)
-
-    def rows(t):
-        if t.stride(1) != 1 or t.stride(0) % 8 or t.data_ptr() % 16:
-            t = t.contiguous()
-        return t
-    X2, W, dY2 = rows(X2), rows(W), rows(dY2)
+    X2, W, dY2 = _rows16(X2), _rows16(W), _rows16(dY2)
     dev = X2.device
     if out is None:
         out = (torch.empty((T, N), dtype=torch.bfloat16, device=dev), torch.empty((T, K), dtype=torch.bfloat16, device=dev),
@@ -480,15 +552,12 @@ def linear_step(X2, W, dY2, scheme, *, tokens=None, out=None, workspace=None):
         for o, shape in zip(out, ((T, N), (T, K), (N, K))):
             _need(tuple(o.shape) == shape and o.dtype == torch.bfloat16 and o.stride(1) == 1 and _on_gpu(o), "bad `out` tensor")
     if workspace is None:
-        workspace = torch.empty((need + 256,), dtype=torch.uint8, device=dev)
-        workspace = workspace[(-workspace.data_ptr()) % 256:][:need]    # device allocations are aligned already: a no-op there
+        workspace = _workspace(need, dev)
     else:
         _need(workspace.dtype == torch.uint8 and workspace.is_contiguous() and workspace.numel() >= need and _on_gpu(workspace)
               and workspace.data_ptr() % 256 == 0, f"`workspace` must be a contiguous, 256-byte aligned uint8 GPU tensor of at least {need} bytes")
     Y, dX, dW = out
     _lib.call("ti8_linear_fwd_bwd", X2.data_ptr(), X2.stride(0), W.data_ptr(), W.stride(0), dY2.data_ptr(), dY2.stride(0),
-              Y.data_ptr(), Y.stride(0), dX.data_ptr(), dX.stride(0), dW.data_ptr(), dW.stride(0), T, T if tokens is None else tokens, K, N,
-              _STEP_SCHEMES[scheme],
-              {"auto": 0, "tiled": GEMM_TILED, "large": GEMM_LARGE_TILES}.get(GEMM_PATH, 0) | (0 if GEMM_PERSISTENT else GEMM_ONE_TILE),
-              workspace.data_ptr(), workspace.numel(), _stream())
+              Y.data_ptr(), Y.stride(0), dX.data_ptr(), dX.stride(0), dW.data_ptr(), dW.stride(0), T, rows if tokens is None else tokens, K, N,
+              _STEP_SCHEMES[scheme], _gemm_flags(), workspace.data_ptr(), need, _stream())
     return Y, dX, dW
