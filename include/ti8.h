@@ -435,6 +435,26 @@ int ti8_gemm_i8_nt_i32(const int8_t* A, int64_t bsa, int64_t lda,
                        int64_t batch, int64_t M, int64_t N, int64_t K, ti8_stream_t stream);
 
 /* ---------------------------------------------------------------------------------
+ * What a decoder layer does between its linears, one pass each (bf16 tensors, contiguous, 16-byte aligned; no counterpart in
+ * the reference).
+ *   ti8_rmsnorm      y[r][c] = bf16(bf16(x[r][c] * rstd[r]) * w[c]), rstd[r] = 1 / sqrt(mean_c(x^2) + eps) (float [rows], written);
+ *                    dim a multiple of 32 up to 8192
+ *   ti8_rmsnorm_bwd  dx bf16 [rows][dim] and dw bf16 [dim] from dy, x, w and the rstd of the forward; workspace of
+ *                    ti8_rmsnorm_bwd_workspace bytes (-1 for sizes it does not take)
+ *   ti8_rope         q and k [tokens][heads * head_dim] rotated by the tables [seq][head_dim / 2] (position = token % seq), halves
+ *                    of a head against each other; backward != 0: by the opposite angle; head_dim a multiple of 16
+ *   ti8_swiglu       out = bf16(bf16(silu(gate)) * up), n elements (a multiple of 8)
+ *   ti8_swiglu_bwd   dgate and dup from d = the gradient of out */
+int ti8_rmsnorm(const void* x, const void* w, void* y, float* rstd, int64_t rows, int64_t dim, float eps, ti8_stream_t stream);
+int64_t ti8_rmsnorm_bwd_workspace(int64_t rows, int64_t dim);
+int ti8_rmsnorm_bwd(const void* dy, const void* x, const void* w, const float* rstd, void* dx, void* dw, void* workspace,
+                    int64_t rows, int64_t dim, ti8_stream_t stream);
+int ti8_rope(const void* q, const void* k, void* out_q, void* out_k, const void* cos_table, const void* sin_table,
+             int64_t tokens, int64_t seq, int64_t heads, int64_t head_dim, int backward, ti8_stream_t stream);
+int ti8_swiglu(const void* gate, const void* up, void* out, int64_t n, ti8_stream_t stream);
+int ti8_swiglu_bwd(const void* d, const void* gate, const void* up, void* dgate, void* dup, int64_t n, ti8_stream_t stream);
+
+/* ---------------------------------------------------------------------------------
  * Measurement aid (no counterpart in the reference; used by bench.py --probe mfma): a loop of nothing
  * but v_mfma_i32_32x32x32_i8 on `workgroups` workgroups of 8 waves, `iters` x 16 MFMAs per wave,
  * operands all zero or pseudo-random, optionally with the block-channel promotion's vector work

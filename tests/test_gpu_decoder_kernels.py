@@ -1,0 +1,88 @@
+"""RMSNorm, rotary embedding and SwiGLU kernels of the decoder layer against the expressions in float64 and the torch bf16 ones."""
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+
+def _rel(got, want):
+    got, want = got.detach().double(), want.detach().double()
+    return float((got - want).norm() / want.norm())
+
+
+@pytest.fixture(scope="module")
+def D():
+    import triton_int8_amd as T
+    return T.decoder
+
+
+# edges: one chunk per thread or none, the register limits (2048, 4096, 8192 elements a row), fewer rows than workgroups and more
+@pytest.mark.parametrize("rows,dim", [(1, 32), (3, 2048), (7, 2080), (1023, 1024), (1025, 512), (2500, 4096), (33, 4128), (5, 8192)])
+def test_rmsnorm(D, dev, rows, dim):
+    gen = torch.Generator(device=dev).manual_seed(rows + dim)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=dev).to(torch.bfloat16)
+    x, w, dy = rand(rows, dim).requires_grad_(True), (1 + 0.1 * rand(dim)).requires_grad_(True), rand(rows, dim)
+    assert D._kernels_take(x, w)
+    y = D._RMSNormFunction.apply(x, w, 1e-5)
+    dx, dw = torch.autograd.grad(y, (x, w), dy)
+    xe, we = x.detach().double().requires_grad_(True), w.detach().double().requires_grad_(True)
+    ye = xe * torch.rsqrt(xe.pow(2).mean(-1, keepdim=True) + 1e-5) * we
+    dxe, dwe = torch.autograd.grad(ye, (xe, we), dy.double())
+    # a rounding to bf16 is off by up to 2^-9 of the value, 2^-9 / sqrt(3) in the norm; two of them in y and in dx, two in dw
+    for got, want in ((y, ye), (dx, dxe), (dw, dwe)):
+        assert _rel(got, want) <= 2 * 2.0 ** -9
+    plain = D._rmsnorm(x, w, 1e-5)
+    if dim <= 4096 and dim % 256 == 0:       # the order of the sum is that of torch's mean
+        assert torch.equal(y, plain)
+    for got, ours, want in zip(torch.autograd.grad(plain, (x, w), dy), (dx, dw), (dxe, dwe)):
+        assert _rel(ours, want) <= 1.05 * _rel(got, want) + 1e-4          # no further from it than the torch expression
+    # differentiated twice: the torch expression's graph
+    g1 = torch.autograd.grad(D._RMSNormFunction.apply(x, w, 1e-5), x, dy, create_graph=True)[0]
+    g0 = torch.autograd.grad(D._rmsnorm(x, w, 1e-5), x, dy, create_graph=True)[0]
+    assert torch.equal(torch.autograd.grad(g1.float().sum(), w)[0], torch.autograd.grad(g0.float().sum(), w)[0])
+
+
+@pytest.mark.parametrize("batch,seq,heads,dim", [(1, 1, 1, 16), (2, 5, 3, 48), (3, 128, 8, 64), (1, 77, 32, 128), (2, 9, 40, 256)])
+def test_rope_bits(D, dev, batch, seq, heads, dim):
+    gen = torch.Generator(device=dev).manual_seed(seq)
+    q, k, dq, dk = (torch.randn(batch, seq, heads, dim, generator=gen, device=dev).to(torch.bfloat16) for _ in range(4))
+    q.requires_grad_(True), k.requires_grad_(True)
+    cos, sin = D.rope_tables(seq, dim, dev)
+    assert D._kernels_take(q, k, cos, sin)
+    outs = [f(q, k, cos, sin) for f in (D._RopeFunction.apply, D._rope_pair)]
+    grads = [torch.autograd.grad(o, (q, k), (dq.transpose(1, 2).contiguous().transpose(1, 2), dk)) for o in outs]
+    for a, b in zip((*outs[0], *grads[0]), (*outs[1], *grads[1])):
+        assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("shape", [(1, 8), (3, 680), (129, 2048), (2, 17, 1024)])
+def test_swiglu(D, dev, shape):
+    gen = torch.Generator(device=dev).manual_seed(shape[-1])
+    gate, up, d = (torch.randn(*shape, generator=gen, device=dev).mul(4).to(torch.bfloat16) for _ in range(3))
+    gate.view(-1)[:4] = torch.tensor([0.0, -100.0, 100.0, -3.0e38], device=dev)
+    gate.requires_grad_(True), up.requires_grad_(True)
+    assert D._kernels_take(gate, up)
+    out = D._SwiGLUFunction.apply(gate, up)
+    got = (out, *torch.autograd.grad(out, (gate, up), d))
+    plain = D._swiglu(gate, up)
+    want = (plain, *torch.autograd.grad(plain, (gate, up), d))
+    ge, ue = gate.detach().double().requires_grad_(True), up.detach().double().requires_grad_(True)
+    exact_out = ge * torch.sigmoid(ge) * ue
+    exact = (exact_out, *torch.autograd.grad(exact_out, (ge, ue), d.double()))
+    for g, w, e in zip(got, want, exact):
+        assert torch.equal(torch.isnan(g), torch.isnan(w))
+        ok = ~torch.isnan(e)
+        assert _rel(g[ok], e[ok]) <= _rel(w[ok], e[ok]) + 1e-5
+
+
+def test_calls_the_kernels_do_not_take(D, dev):
+    x = torch.randn(4, 64, device=dev).to(torch.bfloat16)
+    w = torch.nn.Parameter(torch.ones(64, device=dev, dtype=torch.bfloat16))
+    assert D._kernels_take(x, w)
+    assert not D._kernels_take(x.float(), w) and not D._kernels_take(x.t(), w) and not D._kernels_take(x.cpu(), w)
+    assert not D._kernels_take(torch.randn(257, device=dev).to(torch.bfloat16)[1:], w)       # 2-byte aligned
+    assert not D._kernels_take(x[:0], w)
+    norm = D.RMSNorm(64, device=dev, fused=True)
+    assert torch.equal(torch.func.vmap(norm)(x[:, None]), D.RMSNorm(64, device=dev)(x[:, None]))
+    with torch.autograd.forward_ad.dual_level():
+        assert not D._kernels_take(torch.autograd.forward_ad.make_dual(x, x), w)

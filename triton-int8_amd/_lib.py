@@ -58,9 +58,15 @@ PROTOTYPES = {
     "ti8_linear_fwd_bwd": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _i64, _vp],
     "ti8_linear": [ctypes.POINTER(LinearArgs), _vp],
     "ti8_linear_quantise": [ctypes.POINTER(LinearArgs), ctypes.POINTER(GemmProblem), ctypes.POINTER(_int), _vp],
+    "ti8_rmsnorm": [_vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp],
+    "ti8_rmsnorm_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp],
+    "ti8_rope": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp],
+    "ti8_swiglu": [_vp, _vp, _vp, _i64, _vp],
+    "ti8_swiglu_bwd": [_vp, _vp, _vp, _vp, _vp, _i64, _vp],
     "ti8_probe_mfma": [_vp, _i64, _vp, _int, _int, _int, _int, _vp],
 }
-EXPORTS = ["ti8_version", "ti8_last_error", "ti8_arch", "ti8_init", "ti8_last_gemm_kernel", "ti8_linear_fwd_bwd_workspace", "ti8_linear_workspace"] + list(PROTOTYPES)
+EXPORTS = ["ti8_version", "ti8_last_error", "ti8_arch", "ti8_init", "ti8_last_gemm_kernel", "ti8_linear_fwd_bwd_workspace", "ti8_linear_workspace",
+           "ti8_rmsnorm_bwd_workspace"] + list(PROTOTYPES)
 
 # enums of include/ti8.h
 Q_CLAMP, Q_EPS_ADD, Q_SCALE_BF16, Q_HAD128, Q_WS_PINGPONG, Q_WS_SECOND, Q_TORCH_ROUND, Q_TORCH_BF16, Q_WS_IS_ZERO = 1, 2, 4, 8, 16, 32, 64, 128, 256
@@ -105,6 +111,8 @@ def lib():
         l.ti8_linear_fwd_bwd_workspace.argtypes = [_i64, _i64, _i64, _int]
         l.ti8_linear_workspace.restype = _i64
         l.ti8_linear_workspace.argtypes = [ctypes.POINTER(LinearArgs), ctypes.POINTER(_i64)]
+        l.ti8_rmsnorm_bwd_workspace.restype = _i64
+        l.ti8_rmsnorm_bwd_workspace.argtypes = [_i64, _i64]
         for name, args in PROTOTYPES.items():
             fn = getattr(l, name)
             fn.argtypes = args

@@ -2,12 +2,17 @@
 the training step either side of the hot path, as BASELINE config 5 describes it (hidden 4096,
 32 heads, MLP 14336, bf16 elsewhere).  RMSNorm, rotary embedding, causal attention (torch
 SDPA) and SwiGLU stay in bf16; ``int8=False`` builds the bf16 twin used for loss/grad parity.
+
+In the int8 layer the RMSNorms, the rotary embedding and the SwiGLU product run as one kernel each per direction
+(csrc/decoder.hip); the twin, tensors those kernels do not take and calls under a tracer or a function transform go through the
+torch expressions, which are also what a backward that is differentiated again is made of.
 """
 import math
 
 import torch
 import torch.nn.functional as F
 
+from . import ops
 from .linear import Int8Linear
 
 __all__ = ["DecoderLayer", "rope_tables"]
@@ -27,15 +32,102 @@ def _rope(x, cos, sin):
     return torch.cat((x1 * c - x2 * s, x2 * c + x1 * s), dim=-1)
 
 
+def _rope_pair(q, k, cos, sin):
+    """Both rotated, [B, S, H, D] in and out."""
+    return tuple(_rope(t.transpose(1, 2), cos, sin).transpose(1, 2) for t in (q, k))
+
+
+def _rmsnorm(x, weight, eps):
+    xf = x.float()
+    return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + eps)).to(x.dtype) * weight
+
+
+def _swiglu(gate, up):
+    return F.silu(gate) * up
+
+
+def _kernels_take(*tensors):
+    """Whether tensors can go to the kernels: plain, dense bf16 tensors on the current device, outside tracing and function transforms
+    (to which a kernel launch is invisible)."""
+    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._functorch.peek_interpreter_stack() is not None:
+        return False
+    if torch.autograd.forward_ad._current_level >= 0 or torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
+        return False
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.bfloat16 and t.numel() > 0 and t.is_contiguous()
+               and t.data_ptr() % 16 == 0 and t.device.index == torch._C._cuda_getDevice() for t in tensors)
+
+
+def _dense(t):
+    """A gradient as the kernels read it."""
+    t = t.contiguous()
+    return t if t.data_ptr() % 16 == 0 else t.clone()
+
+
+def _differentiable(expression, inputs, grads):
+    """Gradients as a graph of torch operators, for a backward that will be differentiated again."""
+    with torch.enable_grad():
+        out = expression(*inputs)
+        wanted = [t for t in inputs if t.requires_grad]
+        found = iter(torch.autograd.grad(out, wanted, grads, create_graph=True))
+        return tuple(next(found) if t.requires_grad else None for t in inputs)
+
+
+class _RMSNormFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, weight, eps):
+        y, rstd = ops.rmsnorm(x, weight, eps)
+        ctx.save_for_backward(x, weight, rstd)
+        ctx.eps = eps
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, weight, rstd = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return (*_differentiable(lambda a, w: _rmsnorm(a, w, ctx.eps), (x, weight), dy), None)
+        return (*ops.rmsnorm_backward(_dense(dy), x, weight, rstd), None)
+
+
+class _RopeFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, q, k, cos, sin):
+        ctx.save_for_backward(cos, sin)
+        return ops.rope(q, k, cos, sin)
+
+    @staticmethod
+    def backward(ctx, dq, dk):
+        cos, sin = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return (*_rope_pair(dq, dk, cos, -sin), None, None)     # linear in q and k: the transposed rotation
+        return (*ops.rope(_dense(dq), _dense(dk), cos, sin, backward=True), None, None)
+
+
+class _SwiGLUFunction(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, gate, up):
+        ctx.save_for_backward(gate, up)
+        return ops.swiglu(gate, up)
+
+    @staticmethod
+    def backward(ctx, d):
+        gate, up = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return _differentiable(_swiglu, (gate, up), d)
+        return ops.swiglu_backward(_dense(d), gate, up)
+
+
 class RMSNorm(torch.nn.Module):
-    def __init__(self, dim, eps=1e-5, device=None):
+    def __init__(self, dim, eps=1e-5, device=None, fused=False):
         super().__init__()
         self.weight = torch.nn.Parameter(torch.ones(dim, device=device, dtype=torch.bfloat16))
         self.eps = eps
+        self.fused = fused
 
     def forward(self, x):
-        xf = x.float()
-        return (xf * torch.rsqrt(xf.pow(2).mean(-1, keepdim=True) + self.eps)).to(x.dtype) * self.weight
+        # rows that stay in a workgroup's registers
+        if self.fused and self.weight.numel() <= 8192 and self.weight.numel() % 32 == 0 and x.shape[-1] == self.weight.numel() and _kernels_take(x, self.weight):
+            return _RMSNormFunction.apply(x, self.weight, self.eps)
+        return _rmsnorm(x, self.weight, self.eps)
 
 
 class DecoderLayer(torch.nn.Module):
@@ -53,7 +145,8 @@ class DecoderLayer(torch.nn.Module):
 
         self.q_proj, self.k_proj, self.v_proj, self.o_proj = lin(hidden, hidden), lin(hidden, hidden), lin(hidden, hidden), lin(hidden, hidden)
         self.gate_proj, self.up_proj, self.down_proj = lin(hidden, mlp), lin(hidden, mlp), lin(mlp, hidden)
-        self.input_norm, self.post_norm = RMSNorm(hidden, device=device), RMSNorm(hidden, device=device)
+        self.int8 = int8
+        self.input_norm, self.post_norm = RMSNorm(hidden, device=device, fused=int8), RMSNorm(hidden, device=device, fused=int8)
 
     def copy_weights_from(self, other):
         """Share initial values with another layer (int8 layer <-> bf16 twin)."""
@@ -65,11 +158,13 @@ class DecoderLayer(torch.nn.Module):
         B, S, H = x.shape
         cos, sin = rope_tables(S, self.head_dim, x.device)
         h = self.input_norm(x)
-        q = self.q_proj(h).view(B, S, self.heads, self.head_dim).transpose(1, 2)
-        k = self.k_proj(h).view(B, S, self.heads, self.head_dim).transpose(1, 2)
-        v = self.v_proj(h).view(B, S, self.heads, self.head_dim).transpose(1, 2)
-        q, k = _rope(q, cos, sin), _rope(k, cos, sin)
+        q, k, v = (p(h).view(B, S, self.heads, self.head_dim) for p in (self.q_proj, self.k_proj, self.v_proj))
+        rotate = _RopeFunction.apply if self.int8 and self.head_dim % 16 == 0 and _kernels_take(q, k, cos, sin) else _rope_pair
+        q, k = rotate(q, k, cos, sin)
+        q, k, v = (t.transpose(1, 2) for t in (q, k, v))
         a = F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=1.0 / math.sqrt(self.head_dim))
         x = x + self.o_proj(a.transpose(1, 2).reshape(B, S, H))
         h = self.post_norm(x)
-        return x + self.down_proj(F.silu(self.gate_proj(h)) * self.up_proj(h))
+        gate, up = self.gate_proj(h), self.up_proj(h)
+        product = _SwiGLUFunction.apply if self.int8 and _kernels_take(gate, up) else _swiglu
+        return x + self.down_proj(product(gate, up))

@@ -561,3 +561,39 @@ def linear_step(X2, W, dY2, scheme, *, tokens=None, out=None, workspace=None):
               Y.data_ptr(), Y.stride(0), dX.data_ptr(), dX.stride(0), dW.data_ptr(), dW.stride(0), T, rows if tokens is None else tokens, K, N,
               _STEP_SCHEMES[scheme], _gemm_flags(), workspace.data_ptr(), need, _stream())
     return Y, dX, dW
+
+
+def rmsnorm(x, weight, eps):
+    """``bf16(x * rstd) * weight`` over the last dim of a contiguous bf16 tensor; returns it and rstd (float32, one per row)."""
+    y, rstd = torch.empty_like(x), torch.empty(x.shape[:-1], dtype=torch.float32, device=x.device)
+    _lib.call("ti8_rmsnorm", x.data_ptr(), weight.data_ptr(), y.data_ptr(), rstd.data_ptr(), rstd.numel(), x.shape[-1], eps, _stream())
+    return y, rstd
+
+
+def rmsnorm_backward(dy, x, weight, rstd):
+    dx, dw = torch.empty_like(x), torch.empty_like(weight)
+    rows, dim = rstd.numel(), x.shape[-1]
+    workspace = torch.empty((_lib.lib().ti8_rmsnorm_bwd_workspace(rows, dim),), dtype=torch.uint8, device=x.device)
+    _lib.call("ti8_rmsnorm_bwd", dy.data_ptr(), x.data_ptr(), weight.data_ptr(), rstd.data_ptr(), dx.data_ptr(), dw.data_ptr(), workspace.data_ptr(),
+              rows, dim, _stream())
+    return dx, dw
+
+
+def rope(q, k, cos, sin, backward=False):
+    """q and k [batch, seq, heads, head_dim] (contiguous bf16) rotated by the tables [seq, head_dim / 2], or rotated back."""
+    B, S, H, D = q.shape
+    oq, ok = torch.empty_like(q), torch.empty_like(k)
+    _lib.call("ti8_rope", q.data_ptr(), k.data_ptr(), oq.data_ptr(), ok.data_ptr(), cos.data_ptr(), sin.data_ptr(), B * S, S, H, D, 1 if backward else 0, _stream())
+    return oq, ok
+
+
+def swiglu(gate, up):
+    out = torch.empty_like(gate)
+    _lib.call("ti8_swiglu", gate.data_ptr(), up.data_ptr(), out.data_ptr(), gate.numel(), _stream())
+    return out
+
+
+def swiglu_backward(d, gate, up):
+    dgate, dup = torch.empty_like(gate), torch.empty_like(up)
+    _lib.call("ti8_swiglu_bwd", d.data_ptr(), gate.data_ptr(), up.data_ptr(), dgate.data_ptr(), dup.data_ptr(), gate.numel(), _stream())
+    return dgate, dup
