@@ -394,6 +394,8 @@ int ti8_linear_fwd_bwd(const void* X, int64_t ldx, const void* W, int64_t ldw, c
  *   what the backward can reuse in `saved` (transposed int8 copies, scales), the backward takes it from there.
  *   wq, ws: the forward's view of W quantised earlier (int8 [N][K] and its scales in the scheme's layout); W is then not read.
  *       With TI8_PART_FORWARD alone, without TI8_PART_KEEP.
+ *   bias: bf16 [N], 16-byte aligned, added to Y's rows (a bf16 sum of the rounded Y and the bias), or NULL; not with
+ *       ti8_linear_quantise.
  *   hadamard: 0, 128 (block-channel and row-block: H_128 blocks along every contraction dim) or TI8_HADAMARD_FULL (double-channel).
  *   workspace, saved: sizes from ti8_linear_workspace, 256-byte aligned; contents undefined before and (workspace) after. */
 enum ti8_parts {
@@ -414,6 +416,7 @@ typedef struct ti8_linear_args {
     int scheme, hadamard, parts, gemm_flags;
     void* workspace; int64_t workspace_bytes;
     void* saved; int64_t saved_bytes;
+    const void* bias;
 } ti8_linear_args;
 /* bytes of workspace (and, if `saved_bytes` is not NULL, of saved) that the call needs, or -1 for arguments it does not take;
  * reads tokens, K, N, scheme, hadamard, parts and whether wq is NULL */
@@ -425,6 +428,10 @@ int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, in
  * ti8_gemm_i8_nt_multi (TI8_PART_FORWARD alone: ti8_gemm_i8_nt, the same kernel), else they are launched one by one as
  * ti8_gemm_i8_nt launches them, Y and dX for the first ceil(tokens / 32) * 32 rows only. */
 int ti8_linear(const ti8_linear_args* a, ti8_stream_t stream);
+/* Column sums of x bf16 [rows][cols] (ldx), added up in fp32 and rounded once: the gradient of a bias.  cols a multiple of 32;
+ * workspace: ti8_column_sum_workspace bytes (-1 for sizes it does not take), 16-byte aligned. */
+int64_t ti8_column_sum_workspace(int64_t rows, int64_t cols);
+int ti8_column_sum(const void* x, int64_t ldx, void* out, void* workspace, int64_t rows, int64_t cols, ti8_stream_t stream);
 
 /* Raw int32 accumulators of the same GEMM over the whole K, C int32 [batch][M][N]:
  * the accumulator of int8_gemm_kernel in triton/double-channle_fwd32.py:44,56.

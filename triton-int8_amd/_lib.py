@@ -33,7 +33,7 @@ class LinearArgs(ctypes.Structure):
     _fields_ = [("X", _vp), ("ldx", _i64), ("W", _vp), ("ldw", _i64), ("dY", _vp), ("lddy", _i64), ("Y", _vp), ("ldy", _i64),
                 ("dX", _vp), ("lddx", _i64), ("dW", _vp), ("lddw", _i64), ("wq", _vp), ("ws", _vp),
                 ("tokens", _i64), ("K", _i64), ("N", _i64), ("scheme", _int), ("hadamard", _int), ("parts", _int), ("gemm_flags", _int),
-                ("workspace", _vp), ("workspace_bytes", _i64), ("saved", _vp), ("saved_bytes", _i64)]
+                ("workspace", _vp), ("workspace_bytes", _i64), ("saved", _vp), ("saved_bytes", _i64), ("bias", _vp)]
 
 
 # name -> argument types, in the order of include/ti8.h
@@ -57,6 +57,7 @@ PROTOTYPES = {
     "ti8_gemm_i8_nt_i32": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp],
     "ti8_linear_fwd_bwd": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _i64, _vp],
     "ti8_linear": [ctypes.POINTER(LinearArgs), _vp],
+    "ti8_column_sum": [_vp, _i64, _vp, _vp, _i64, _i64, _vp],
     "ti8_linear_quantise": [ctypes.POINTER(LinearArgs), ctypes.POINTER(GemmProblem), ctypes.POINTER(_int), _vp],
     "ti8_rmsnorm": [_vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp],
     "ti8_rmsnorm_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp],
@@ -66,7 +67,7 @@ PROTOTYPES = {
     "ti8_probe_mfma": [_vp, _i64, _vp, _int, _int, _int, _int, _vp],
 }
 EXPORTS = ["ti8_version", "ti8_last_error", "ti8_arch", "ti8_init", "ti8_last_gemm_kernel", "ti8_linear_fwd_bwd_workspace", "ti8_linear_workspace",
-           "ti8_rmsnorm_bwd_workspace"] + list(PROTOTYPES)
+           "ti8_rmsnorm_bwd_workspace", "ti8_column_sum_workspace"] + list(PROTOTYPES)
 
 # enums of include/ti8.h
 Q_CLAMP, Q_EPS_ADD, Q_SCALE_BF16, Q_HAD128, Q_WS_PINGPONG, Q_WS_SECOND, Q_TORCH_ROUND, Q_TORCH_BF16, Q_WS_IS_ZERO = 1, 2, 4, 8, 16, 32, 64, 128, 256
@@ -113,6 +114,8 @@ def lib():
         l.ti8_linear_workspace.argtypes = [ctypes.POINTER(LinearArgs), ctypes.POINTER(_i64)]
         l.ti8_rmsnorm_bwd_workspace.restype = _i64
         l.ti8_rmsnorm_bwd_workspace.argtypes = [_i64, _i64]
+        l.ti8_column_sum_workspace.restype = _i64
+        l.ti8_column_sum_workspace.argtypes = [_i64, _i64]
         for name, args in PROTOTYPES.items():
             fn = getattr(l, name)
             fn.argtypes = args

@@ -1,0 +1,111 @@
+// The bias of a linear layer: adding it to the output of a GEMM whose epilogue does not, and its gradient, the column sums of dY.
+#include "ti8_common.h"
+
+namespace ti8 {
+
+namespace {
+
+constexpr int THREADS = 256;
+constexpr int SUM_COLS = 512;       // columns per workgroup of column_partial_kernel: 64 lanes x 8, a row's share is 1 KiB
+
+}  // namespace
+
+// y[r][c] = bf16(y[r][c] + bias[c]), 8 columns per thread.  Streams y once each way; torch's broadcast add reads the bias through
+// its strided path: 1500 x 5632 (34 MB) 11 us, this 6.
+__global__ __launch_bounds__(THREADS) void add_bias_kernel(uint16_t* __restrict__ y, int64_t ldy, const uint16_t* __restrict__ bias, int rows, int chunks) {
+    const int c = (int)blockIdx.x * THREADS + (int)threadIdx.x;      // group of 8 columns
+    if (c >= chunks) return;
+    const uint4 b = *reinterpret_cast<const uint4*>(bias + c * 8);
+    const int r0 = (int)blockIdx.y * 4;
+    uint16_t* const p = y + (int64_t)r0 * ldy + c * 8;
+    uint4 v[4];
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (r0 + k < rows) v[k] = *reinterpret_cast<const uint4*>(p + (int64_t)k * ldy);
+#pragma unroll
+    for (int k = 0; k < 4; ++k)
+        if (r0 + k < rows)
+            *reinterpret_cast<uint4*>(p + (int64_t)k * ldy) =
+                make_uint4(add_bf16x2(v[k].x, b.x), add_bf16x2(v[k].y, b.y), add_bf16x2(v[k].z, b.z), add_bf16x2(v[k].w, b.w));
+}
+
+// partial[g][c] = sum of x[r][c] over rows r = g * per .. of workgroup row g: each of the four waves takes every fourth row, LDS
+// adds their sums.  One read of x; the column sums of a [1500][5632] dY take 4 + 3 us in the two launches (torch's reduction with
+// the two memory fills in front of it: 23).
+__global__ __launch_bounds__(THREADS) void column_partial_kernel(const uint16_t* __restrict__ x, int64_t ldx, int rows, int per, int cols, float* __restrict__ partial) {
+    __shared__ float acc[4][SUM_COLS];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int c0 = (int)blockIdx.x * SUM_COLS + lane * 8;
+    const int r0 = (int)blockIdx.y * per, r1 = min(r0 + per, rows);
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = 0.0f;
+    if (c0 < cols) {
+#pragma unroll 4
+        for (int r = r0 + wave; r < r1; r += 4) {
+            const uint4 v = *reinterpret_cast<const uint4*>(x + (int64_t)r * ldx + c0);
+            const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                s[2 * e] += bf16_lo(w[e]);
+                s[2 * e + 1] += bf16_hi(w[e]);
+            }
+        }
+    }
+#pragma unroll
+    for (int e = 0; e < 8; e += 4) *reinterpret_cast<float4*>(&acc[wave][lane * 8 + e]) = make_float4(s[e], s[e + 1], s[e + 2], s[e + 3]);
+    __syncthreads();
+    const int c = threadIdx.x * 2, col = (int)blockIdx.x * SUM_COLS + c;
+    if (col >= cols) return;
+    *reinterpret_cast<float2*>(partial + (int64_t)blockIdx.y * cols + col) =
+        make_float2((acc[0][c] + acc[1][c]) + (acc[2][c] + acc[3][c]), (acc[0][c + 1] + acc[1][c + 1]) + (acc[2][c + 1] + acc[3][c + 1]));
+}
+
+int add_bias(void* y, int64_t ldy, const void* bias, int64_t rows, int64_t cols, ti8_stream_t stream) {
+    const int chunks = (int)(cols / 8);
+    for (int64_t r = 0; r < rows; r += 4 * 65535) {     // a launch has at most 65535 workgroup rows
+        const int64_t n = rows - r < 4 * 65535 ? rows - r : 4 * 65535;
+        hipLaunchKernelGGL(add_bias_kernel, dim3((unsigned)((chunks + THREADS - 1) / THREADS), (unsigned)((n + 3) / 4)), dim3(THREADS), 0,
+                           static_cast<hipStream_t>(stream), static_cast<uint16_t*>(y) + r * ldy, ldy, static_cast<const uint16_t*>(bias), (int)n, chunks);
+        if (int e = check_launch("ti8_linear")) return e;
+    }
+    return TI8_OK;
+}
+
+// Rows per workgroup: about 1024 workgroups, no fewer than 16 rows each (the partial sums are then at most an eighth of the bytes read)
+static int64_t rows_per_group(int64_t rows, int64_t cols) {
+    const int64_t strips = (cols + SUM_COLS - 1) / SUM_COLS;
+    const int64_t wanted = strips < 1024 ? 1024 / strips : 1;
+    const int64_t per = (rows + wanted - 1) / wanted;
+    return per < 16 ? 16 : per;
+}
+
+static bool column_sum_takes(int64_t rows, int64_t cols) {
+    return rows > 0 && rows <= 0x3fffffff && cols > 0 && cols % 32 == 0 && cols <= 0x3fffffff;
+}
+
+}  // namespace ti8
+
+using namespace ti8;
+
+extern "C" int64_t ti8_column_sum_workspace(int64_t rows, int64_t cols) {
+    if (!column_sum_takes(rows, cols)) return -1;
+    const int64_t per = rows_per_group(rows, cols);
+    return (rows + per - 1) / per * cols * (int64_t)sizeof(float);
+}
+
+extern "C" int ti8_column_sum(const void* x, int64_t ldx, void* out, void* workspace, int64_t rows, int64_t cols, ti8_stream_t stream) {
+    const char* fn = "ti8_column_sum";
+    if (!x || !out || !workspace) return fail(TI8_ERR_NULL, "%s: x, out and the workspace are required", fn);
+    if (!column_sum_takes(rows, cols) || ldx < cols)
+        return fail(TI8_ERR_SHAPE, "%s: need rows>0, cols a positive multiple of 32 and ldx>=cols; got rows=%lld cols=%lld ldx=%lld", fn, (long long)rows, (long long)cols, (long long)ldx);
+    if (!aligned16(x) || ldx % 8 || !aligned16(out) || !aligned16(workspace)) return fail(TI8_ERR_ALIGN, "%s: x, out and the workspace must be 16-byte aligned, ldx a multiple of 8", fn);
+    const int64_t per = rows_per_group(rows, cols);
+    const int groups = (int)((rows + per - 1) / per);
+    float* const partial = static_cast<float*>(workspace);
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    hipLaunchKernelGGL(column_partial_kernel, dim3((unsigned)((cols + SUM_COLS - 1) / SUM_COLS), (unsigned)groups), dim3(THREADS), 0, st,
+                       static_cast<const uint16_t*>(x), ldx, (int)rows, (int)per, (int)cols, partial);
+    if (int e = check_launch(fn)) return e;
+    return sum_partials(fn, partial, groups, cols, out, st);
+}

@@ -292,6 +292,11 @@ void with_chunks(int64_t dim, F f) {
 }
 
 }  // namespace
+int sum_partials(const char* fn, const float* partial, int groups, int64_t dim, void* out, hipStream_t st) {
+    hipLaunchKernelGGL(column_sum_kernel, dim3((unsigned)(dim / SUM_COLS)), dim3(1024), 0, st, partial, groups, (int)dim, static_cast<uint16_t*>(out));
+    return check_launch(fn);
+}
+
 }  // namespace ti8
 
 using namespace ti8;
@@ -329,8 +334,7 @@ extern "C" int ti8_rmsnorm_bwd(const void* dy, const void* x, const void* w, con
                            static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), rstd, static_cast<uint16_t*>(dx), partial, rows, (int)dim);
     });
     if (int e = check_launch(fn)) return e;
-    hipLaunchKernelGGL(column_sum_kernel, dim3((unsigned)(dim / SUM_COLS)), dim3(1024), 0, st, partial, groups, (int)dim, static_cast<uint16_t*>(dw));
-    return check_launch(fn);
+    return sum_partials(fn, partial, groups, dim, dw, st);
 }
 
 extern "C" int ti8_rope(const void* q, const void* k, void* out_q, void* out_k, const void* cos_table, const void* sin_table, int64_t tokens, int64_t seq,

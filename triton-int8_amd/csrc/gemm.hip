@@ -677,6 +677,7 @@ static int prepare_gemm(const char* fn, const ti8_gemm_problem& p, int gemm_flag
     a.combine = p.combine;
     a.strict = (gemm_flags & TI8_GEMM_STRICT) ? 1 : 0;
     a.out_scale = p.out_scale; a.post_scale = p.post_scale;
+    a.bias = nullptr;
     *out = a;
     return TI8_OK;
 }
@@ -771,34 +772,50 @@ static int launch_group(const char* fn, GemmMulti& m, const idx::GemmConfig& c, 
 
 using namespace ti8;
 
+// One GEMM on the kernel that its shape selects.  `bias` (bf16 [N], 16-byte aligned, may be null) is handed to the kernels whose
+// epilogue adds it; *added says whether it was one of those.
+int ti8::gemm_nt_bias(const ti8_gemm_problem& p, const void* bias, int gemm_flags, bool* added, ti8_stream_t stream) {
+    const char* fn = "ti8_gemm_i8_nt";
+    const int64_t M = p.M, N = p.N, K = p.K, batch = p.batch;
+    const bool i32_full = p.acc_i32_full != 0;
+    GemmArgs a;
+    if (int e = prepare_gemm(fn, p, gemm_flags, &a)) return e;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    *added = false;
+    auto with_bias = [&]() {
+        a.bias = static_cast<const uint16_t*>(bias);
+        *added = bias != nullptr;
+    };
+    // few rows: too few 256-row tiles to fill the machine, take the kernel that splits N and K finer
+    const bool large = (gemm_flags & TI8_GEMM_LARGE_TILES) != 0;
+    const bool want_skinny = (gemm_flags & TI8_GEMM_SKINNY) || (!(gemm_flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES)) && M <= 256);
+    if (want_skinny && !a.strict && skinny_supported(a)) {
+        with_bias();
+        if (!(gemm_flags & TI8_GEMM_SKINNY) && idx::gemm_few_rows_prefers_mid(M, N, K, batch, device_cu_count())) {
+            GemmMulti m;
+            m.count = 1;
+            m.g[0] = a;
+            return launch_mid(m, batch, i32_full, st);
+        }
+        return launch_skinny(a, batch, i32_full, st);
+    }
+    if (M % 128)
+        return fail(TI8_ERR_SHAPE, "%s: M = %lld is not a multiple of 128, which only the few-rows kernel accepts "
+                    "(not with TI8_GEMM_STRICT / TI8_GEMM_TILED, per-(row, K tile) scales or K > 32768)", fn, (long long)M);
+    const idx::GemmConfig c = idx::gemm_config(M, N, K, batch, i32_full, a.strict != 0, p.modeA, p.modeB, large, device_cu_count());
+    if (c.mid) with_bias();
+    return launch_tiled(fn, a, batch, c, !(gemm_flags & TI8_GEMM_ONE_TILE), st);
+}
+
 extern "C" int ti8_gemm_i8_nt(const int8_t* A, int64_t bsa, int64_t lda, const int8_t* B, int64_t bsb, int64_t ldb,
                               void* C, int64_t bsc, int64_t ldc, const float* sA, int modeA, int64_t sa_bs,
                               int64_t sa_rs, int64_t sa_ks, const float* sB, int modeB, int64_t sb_bs, int64_t sb_rs,
                               int64_t sb_ks, int64_t batch, int64_t M, int64_t N, int64_t K, int acc_i32_full,
                               int combine, float out_scale, float post_scale, int gemm_flags, ti8_stream_t stream) {
-    const char* fn = "ti8_gemm_i8_nt";
     const ti8_gemm_problem p = {A, bsa, lda, B, bsb, ldb, C, bsc, ldc, sA, modeA, sa_bs, sa_rs, sa_ks, sB, modeB, sb_bs, sb_rs, sb_ks,
                                 batch, M, N, K, acc_i32_full, combine, out_scale, post_scale};
-    GemmArgs a;
-    if (int e = prepare_gemm(fn, p, gemm_flags, &a)) return e;
-    hipStream_t st = static_cast<hipStream_t>(stream);
-    // few rows: too few 256-row tiles to fill the machine, take the kernel that splits N and K finer
-    const bool large = (gemm_flags & TI8_GEMM_LARGE_TILES) != 0;
-    const bool want_skinny = (gemm_flags & TI8_GEMM_SKINNY) || (!(gemm_flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES)) && M <= 256);
-    if (want_skinny && !a.strict && skinny_supported(a)) {
-        if (!(gemm_flags & TI8_GEMM_SKINNY) && idx::gemm_few_rows_prefers_mid(M, N, K, batch, device_cu_count())) {
-            GemmMulti m;
-            m.count = 1;
-            m.g[0] = a;
-            return launch_mid(m, batch, acc_i32_full != 0, st);
-        }
-        return launch_skinny(a, batch, acc_i32_full != 0, st);
-    }
-    if (M % 128)
-        return fail(TI8_ERR_SHAPE, "%s: M = %lld is not a multiple of 128, which only the few-rows kernel accepts "
-                    "(not with TI8_GEMM_STRICT / TI8_GEMM_TILED, per-(row, K tile) scales or K > 32768)", fn, (long long)M);
-    return launch_tiled(fn, a, batch, idx::gemm_config(M, N, K, batch, acc_i32_full != 0, a.strict != 0, modeA, modeB, large, device_cu_count()),
-                        !(gemm_flags & TI8_GEMM_ONE_TILE), st);
+    bool added = false;
+    return gemm_nt_bias(p, nullptr, gemm_flags, &added, stream);
 }
 
 extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count, int gemm_flags, ti8_stream_t stream) {
@@ -854,6 +871,6 @@ extern "C" int ti8_gemm_i8_nt_i32(const int8_t* A, int64_t bsa, int64_t lda, con
     a.sb = a.sa;
     a.M = (int)M; a.N = (int)N; a.K = (int)K;
     a.tiles_m = a.tiles_n = 0;
-    a.combine = 0; a.strict = 0; a.out_scale = 1.0f; a.post_scale = 0.0f;
+    a.combine = 0; a.strict = 0; a.out_scale = 1.0f; a.post_scale = 0.0f; a.bias = nullptr;
     return launch<256, 256, 2, 4, EPI_I32>(a, batch, static_cast<hipStream_t>(stream));
 }

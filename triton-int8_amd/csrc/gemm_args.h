@@ -22,6 +22,7 @@ struct GemmArgs {
     int combine;
     int strict;
     float out_scale, post_scale;
+    const uint16_t* bias;   // bf16 [N], added to the rounded result and rounded again; the few-rows and the medium kernel only (else null)
 };
 
 // EPI_PROMOTE: the per-K-tile factor is uniform over a wave's tile (block or per-row scales

@@ -252,6 +252,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m)
         v = col_part ? v : 1.0f;
         coln[c] = divide ? 1.0f / v : v;
     }
+    uint4 bias = make_uint4(0, 0, 0, 0);
+    if (g.bias) bias = *reinterpret_cast<const uint4*>(g.bias + n0 + wn * WCOLS + rb_col);
     // every load has landed and every wave is past its last fragment read: the buffers become exchange slabs
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
@@ -312,8 +314,10 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m)
             for (int c = 0; c < 8; ++c) v[c] = __uint_as_float(pack_bf16x2(v[c], 0.0f) << 16) * g.post_scale;
         }
         uint16_t* const row = dst + (int64_t)(8 * k) * g.ldc;
-        *reinterpret_cast<uint2*>(row) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
-        *reinterpret_cast<uint2*>(row + 4) = make_uint2(pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+        uint4 o = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+        if (g.bias) o = make_uint4(add_bf16x2(o.x, bias.x), add_bf16x2(o.y, bias.y), add_bf16x2(o.z, bias.z), add_bf16x2(o.w, bias.w));
+        *reinterpret_cast<uint2*>(row) = make_uint2(o.x, o.y);
+        *reinterpret_cast<uint2*>(row + 4) = make_uint2(o.z, o.w);
     }
 }
 

@@ -120,6 +120,9 @@ __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g)
         for (int c = 0; c < 4; ++c) coln[c] = 1.0f / coln[c];
     }
 
+    // the bias of those 4 columns (without one: 8 bytes of B, dropped)
+    const uint2 bias = *reinterpret_cast<const uint2*>(g.bias ? reinterpret_cast<const void*>(g.bias + n0 + e_col) : reinterpret_cast<const void*>(g.B));
+
     const int fr_row = lane & 31, fr_half = lane >> 5;
     const int sw = (lane & 7) ^ ((lane >> 3) & 1);
     int choff[4];
@@ -139,6 +142,8 @@ __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g)
     // for nothing else): a load still pending at the loop's entry makes the compiler drain the
     // whole load queue at the top of every iteration
     asm volatile("" : "+v"(rowm));
+    uint32_t bias_lo = bias.x, bias_hi = bias.y;
+    asm volatile("" : "+v"(bias_lo), "+v"(bias_hi));
 #pragma unroll
     for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(coln[c]));
 
@@ -221,6 +226,10 @@ __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g)
     uint2 o;
     o.x = pack_bf16x2(t[0], t[1]);
     o.y = pack_bf16x2(t[2], t[3]);
+    if (g.bias) {
+        o.x = add_bf16x2(o.x, bias_lo);
+        o.y = add_bf16x2(o.y, bias_hi);
+    }
     *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.C) + (int64_t)batch * g.bsc + (int64_t)(m0 + e_row) * g.ldc + n0 + e_col) = o;
 }
 

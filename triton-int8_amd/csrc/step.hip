@@ -155,8 +155,8 @@ int check_pointers(const char* fn, const ti8_linear_args* a, const Layer& L) {
         return fail(TI8_ERR_SHAPE, "%s: leading dimension smaller than the row length", fn);
     // what the quantisers (inputs) and the GEMM epilogues (outputs) need, checked here so that nothing is launched before a rejection
     if (!aligned(a->X, a->ldx) || !aligned(a->W, a->ldw) || (L.bwd && (!aligned(a->dY, a->lddy) || !aligned(a->dX, a->lddx) || !aligned(a->dW, a->lddw))) ||
-        (L.fwd && !aligned(a->Y, a->ldy)) || !aligned(a->wq, 0))
-        return fail(TI8_ERR_ALIGN, "%s: X, W, dY, Y, dX and dW must be 16-byte aligned with leading dimensions multiples of 8 elements", fn);
+        (L.fwd && (!aligned(a->Y, a->ldy) || !aligned(a->bias, 0))) || !aligned(a->wq, 0))
+        return fail(TI8_ERR_ALIGN, "%s: X, W, dY, Y, dX, dW and the bias must be 16-byte aligned with leading dimensions multiples of 8 elements", fn);
     // limits of the quantisers that this call launches
     const bool shared = L.shares(), row_k = L.fwd && (L.row_block() || ((L.had || !shared) && !(L.block() && L.given_w())));
     const bool row_n = L.bwd && L.had && !L.block();
@@ -303,10 +303,12 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
 
 // One GEMM launched alone (what ti8_gemm_i8_nt selects for its shape: the few-rows kernel up to 256 rows).  `live` rows of A are
 // multiplied: with few tokens the padding rows of the 128-row-quantised operand are zeros whose products nobody reads.
-int one_gemm(const ti8_gemm_problem& p, int64_t live, int gemm_flags, ti8_stream_t stream) {
-    return ti8_gemm_i8_nt(p.A, p.bsa, p.lda, p.B, p.bsb, p.ldb, p.C, p.bsc, p.ldc, p.sA, p.modeA, p.sa_bs, p.sa_rs, p.sa_ks,
-                          p.sB, p.modeB, p.sb_bs, p.sb_rs, p.sb_ks, 1, live, p.N, p.K, p.acc_i32_full, p.combine, p.out_scale, p.post_scale,
-                          gemm_flags, stream);
+int one_gemm(const ti8_gemm_problem& p, int64_t live, const void* bias, int64_t tokens, int gemm_flags, ti8_stream_t stream) {
+    ti8_gemm_problem q = p;
+    q.M = live;
+    bool added = false;
+    if (int e = gemm_nt_bias(q, bias, gemm_flags, &added, stream)) return e;
+    return bias && !added ? add_bias(p.C, p.ldc, bias, tokens, p.N, stream) : TI8_OK;
 }
 
 int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t stream) {
@@ -318,10 +320,13 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
         return r < L.T ? r : L.T;
     };
     // they go into one launch where none of them has so few rows that it would take the few-rows kernel
-    if (L.bwd && (L.T < L.N ? L.T : L.N) > 256) return ti8_gemm_i8_nt_multi(g, count, flags, stream);
+    if (L.bwd && (L.T < L.N ? L.T : L.N) > 256) {
+        if (int e = ti8_gemm_i8_nt_multi(g, count, flags, stream)) return e;
+        return L.fwd && L.a->bias ? add_bias(L.a->Y, L.a->ldy, L.a->bias, L.tokens, L.N, stream) : TI8_OK;
+    }
     for (int i = 0; i < count; ++i) {
         const bool token_rows = i + 1 < count || !L.bwd;     // dW, the last of a backward, has one row per output feature
-        if (int e = one_gemm(g[i], token_rows ? live_rows(g[i].K) : g[i].M, flags, stream)) return e;
+        if (int e = one_gemm(g[i], token_rows ? live_rows(g[i].K) : g[i].M, L.fwd && i == 0 ? L.a->bias : nullptr, L.tokens, flags, stream)) return e;
     }
     return TI8_OK;
 }
@@ -365,6 +370,7 @@ extern "C" int64_t ti8_linear_workspace(const ti8_linear_args* a, int64_t* saved
 extern "C" int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, int* count, ti8_stream_t stream) {
     const char* fn = "ti8_linear_quantise";
     if (!a || !problems || !count) return fail(TI8_ERR_NULL, "%s: args, problems and count are required", fn);
+    if (a->bias) return fail(TI8_ERR_MODE, "%s: the GEMMs that a bias goes with are the caller's", fn);
     return run_layer(fn, a, (a->tokens + 127) / 128 * 128, problems, count, stream);
 }
 

@@ -79,6 +79,11 @@ int quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q,
 int fwht_t_quant_row_valid(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t valid_rows, int64_t C,
                            int qflags, int inv_mode, ti8_stream_t stream);
 int fill_words(unsigned int* p, int64_t words, unsigned int value, hipStream_t st);
+// ti8_gemm_i8_nt with a bias for the kernels whose epilogue adds one (*added: this was one); y += bias behind the others (bias.hip)
+int gemm_nt_bias(const ti8_gemm_problem& p, const void* bias, int gemm_flags, bool* added, ti8_stream_t stream);
+int add_bias(void* y, int64_t ldy, const void* bias, int64_t rows, int64_t cols, ti8_stream_t stream);
+// out[c] = bf16(sum over g of partial[g][c]), dim a multiple of 32 (decoder.hip)
+int sum_partials(const char* fn, const float* partial, int groups, int64_t dim, void* out, hipStream_t st);
 
 // ---- which kernel served the last GEMM call of this thread (ti8_last_gemm_kernel) ---
 void note_gemm_kernel(int kind, int bm, int bn, int epi);
@@ -108,6 +113,9 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float lo, float hi) {
     const ti8_f32x2 v = {lo, hi};
     return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, ti8_bf16x2));
 }
+
+// sums of two pairs of bf16, each rounded to bf16
+__device__ __forceinline__ uint32_t add_bf16x2(uint32_t a, uint32_t b) { return pack_bf16x2(bf16_lo(a) + bf16_lo(b), bf16_hi(a) + bf16_hi(b)); }
 
 // Reductions over lanes with DPP moves (no LDS traffic).
 // max(v, v of the lane that DPP control CTRL names) in the rows of ROW_MASK; other lanes keep v

@@ -331,6 +331,13 @@ def linear_fwd_bwd(X, W, dY, scheme="block_channel", hadamard=None, out=None, wo
     return Y[:T].reshape(*lead, N), dX[:T].reshape(*lead, K), dW
 
 
+def _in_the_call(bias, features):
+    """Whether a bias goes into the layer call: a plain, dense bf16 vector that nothing else has to see being added."""
+    return (bias is not None and type(bias) in (torch.Tensor, torch.nn.Parameter) and bias.dtype == torch.bfloat16 and bias.is_cuda and tuple(bias.shape) == (features,)
+            and bias.is_contiguous() and bias.data_ptr() % 16 == 0 and bias.device.index == torch._C._cuda_getDevice()
+            and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None)
+
+
 class Int8LinearFunction(torch.autograd.Function):
     """y = x W^T (+ bias) with every GEMM of forward and backward on the INT8 path."""
 
@@ -346,8 +353,11 @@ class Int8LinearFunction(torch.autograd.Function):
             return x.new_empty((*x.shape[:-1], N))
         need_bwd = any(ctx.needs_input_grad[:2])
         if _from_c():
+            inside = _in_the_call(bias, N)
             y, _, _, ctx.saved_q = ops.linear_call(PART_FORWARD | (PART_KEEP if need_bwd else 0), scheme, hadamard,
-                                                   *_layer_dims(x2, weight), X=x2, W=weight)
+                                                   *_layer_dims(x2, weight), X=x2, W=weight, bias=bias if inside else None)
+            if inside:
+                bias = None
         else:
             y, ctx.saved_q = linear_forward(pad_tokens(x2), weight, scheme, hadamard, need_backward=need_bwd, tokens=tokens)
         y = y[:tokens]
@@ -372,7 +382,10 @@ class Int8LinearFunction(torch.autograd.Function):
             dx, dw = linear_backward(dyp, xp, weight, ctx.scheme, ctx.hadamard, ctx.saved_q, tokens=tokens, gemms=gemms)
             if gemms:
                 ops.gemm_i8_nt_multi(gemms)   # dX and dW in one launch
-        db = dy2.sum(dim=0).to(dy.dtype) if ctx.has_bias else None
+        db = None
+        if ctx.has_bias:
+            # (a backward that is differentiated again needs the sum as a torch operator)
+            db = ops.column_sum(dy2) if dy2.dtype == torch.bfloat16 and dy2.is_cuda and not torch.is_grad_enabled() else dy2.sum(dim=0).to(dy.dtype)
         return dx[:tokens].reshape(*dy.shape[:-1], x2.shape[1]), dw, db, None, None
 
 
@@ -408,11 +421,14 @@ class Int8Linear(torch.nn.Module):
         if _from_c():
             if x2.shape[1] != self.in_features:
                 raise ValueError(f"expected {self.in_features} input features, got {x2.shape[1]}")
-            y = ops.linear_call(PART_FORWARD, self.scheme, self.hadamard, tokens, self.in_features, self.out_features, X=x2, wq=self._wq)[0]
+            inside = _in_the_call(self.bias, self.out_features)
+            y = ops.linear_call(PART_FORWARD, self.scheme, self.hadamard, tokens, self.in_features, self.out_features, X=x2, wq=self._wq,
+                                bias=self.bias if inside else None)[0]
         else:
+            inside = False
             y, _ = linear_forward(pad_tokens(x2), None, self.scheme, self.hadamard, need_backward=False, wq=self._wq, tokens=tokens)
         y = y[:tokens]
-        if self.bias is not None:
+        if self.bias is not None and not inside:
             y += self.bias      # the GEMM's own output: in place
         return y.reshape(*x.shape[:-1], self.out_features)
 

@@ -490,11 +490,11 @@ def _linear_sizes(tokens, K, N, scheme, hadamard, parts, given_w):
     return n, saved.value
 
 
-def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=None, wq=None, saved=None, one_launch=True):
+def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=None, wq=None, saved=None, one_launch=True, bias=None):
     """The forward, the backward or both of a layer in one or two library calls (``ti8_linear``; with ``one_launch`` and more than
     256 tokens and output features the quantisers as one call and the backward's or step's GEMMs as ``ti8_gemm_i8_nt_multi``).
     X bf16 [tokens, K], W bf16 [N, K], dY bf16 [tokens, N]: any number of tokens, no padded copies.  ``wq`` = (int8 [N, K], scales) of
-    the weight quantised earlier.  Returns (Y [T, N], dX [T, K], dW [N, K], saved) with None for what `parts` does not ask for; T =
+    the weight quantised earlier, ``bias`` bf16 [N] is added to Y (a forward alone).  Returns (Y [T, N], dX [T, K], dW [N, K], saved) with None for what `parts` does not ask for; T =
     tokens rounded up to 128, rows from `tokens` on undefined."""
     for t, name in ((X, "X"), (W, "W"), (dY, "dY")):
         if t is not None:
@@ -516,7 +516,7 @@ def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=Non
     a = _lib.LinearArgs(ptr(X), 0 if X is None else X.stride(0), ptr(W), 0 if W is None else W.stride(0), ptr(dY), 0 if dY is None else dY.stride(0),
                         ptr(Y), N, ptr(dX), K, ptr(dW), K, ptr(wq[0]) if wq is not None else None, ptr(wq[1]) if wq is not None else None,
                         tokens, K, N, _SCHEMES[scheme], _ROTATIONS[hadamard], parts, _gemm_flags(), workspace.data_ptr(), need,
-                        ptr(saved), need_saved)
+                        ptr(saved), need_saved, ptr(bias))
     stream = _stream()
     if one_launch and parts & _lib.PART_BACKWARD and min(T, N) > 256:
         problems, count = (_lib.GemmProblem * 3)(), ctypes.c_int(0)
@@ -525,6 +525,16 @@ def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=Non
     else:
         _lib.call("ti8_linear", ctypes.byref(a), stream)
     return Y, dX, dW, saved
+
+
+def column_sum(x):
+    """``x.sum(0)`` of a bf16 matrix, added up in fp32; columns a multiple of 32."""
+    x = _rows16(x)
+    rows, cols = x.shape
+    out = torch.empty((cols,), dtype=torch.bfloat16, device=x.device)
+    workspace = torch.empty((_lib.lib().ti8_column_sum_workspace(rows, cols),), dtype=torch.uint8, device=x.device)
+    _lib.call("ti8_column_sum", x.data_ptr(), x.stride(0), out.data_ptr(), workspace.data_ptr(), rows, cols, _stream())
+    return out
 
 
 def linear_step(X2, W, dY2, scheme, *, tokens=None, out=None, workspace=None):
