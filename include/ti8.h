@@ -95,6 +95,8 @@ enum ti8_gemm_flags {
     TI8_GEMM_LARGE_TILES = 8, /* LDS-tiled kernel with the largest tiles (256 x 256) whatever the shape */
     TI8_GEMM_ONE_TILE = 16,   /* one workgroup per output tile also where the block-channel promotion would run on
                                  persistent workgroups (one per CU walking its tiles); same bits either way */
+    TI8_GEMM_TOGETHER = 32,   /* ti8_gemm_i8_nt_multi: choose the kernels for the launch as a whole, not as each GEMM's shape
+                                 alone would; the promoted sums may then associate differently from a separate call's */
     TI8_GEMM_SKINNY = 4   /* take the few-rows kernel (no LDS staging, K split over waves) whenever
                              it supports the scale modes; by default it is used for M <= 256.  Both
                              kernels give bit-identical results with acc_i32_full; otherwise their
@@ -334,7 +336,7 @@ int ti8_gemm_i8_nt(const int8_t* A, int64_t bsa, int64_t lda,
  * triton/block_channel_bwd33.py:72) when all their operands are at hand.  Every field means what the
  * argument of that name means in ti8_gemm_i8_nt; `problems` is a HOST array, read before the call
  * returns.  Each GEMM runs the kernel that ti8_gemm_i8_nt with TI8_GEMM_TILED selects for its shape
- * and scale modes, so results are bit-identical to such separate calls; those that select the same
+ * and scale modes, so results are bit-identical to such separate calls (not with TI8_GEMM_TOGETHER); those that select the same
  * kernel share one launch (not TI8_GEMM_STRICT, not TI8_SCALE_ROW_K128).  TI8_GEMM_SKINNY is refused. */
 typedef struct ti8_gemm_problem {
     const int8_t* A; int64_t bsa, lda;

@@ -74,7 +74,7 @@ Q_CLAMP, Q_EPS_ADD, Q_SCALE_BF16, Q_HAD128, Q_WS_PINGPONG, Q_WS_SECOND, Q_TORCH_
 INV_RCP_OF_SCALE, INV_AMAX_DIV_127, INV_AMAX_MUL_RCP127, INV_MULTIPLIER = 0, 1, 2, 3
 SCALE_ROW, SCALE_BLOCK128, SCALE_ROW_K128, SCALE_BLOCK_K256 = 0, 1, 2, 3
 COMBINE_MUL_MUL, COMBINE_MUL_PROD, COMBINE_DIV_PROD = 0, 1, 2
-GEMM_STRICT, GEMM_TILED, GEMM_SKINNY, GEMM_LARGE_TILES, GEMM_ONE_TILE = 1, 2, 4, 8, 16
+GEMM_STRICT, GEMM_TILED, GEMM_SKINNY, GEMM_LARGE_TILES, GEMM_ONE_TILE, GEMM_TOGETHER = 1, 2, 4, 8, 16, 32
 NOALLOC_MAX_ROWS_PLUS_COLS = 65536
 SCHEME_BLOCK_CHANNEL, SCHEME_ROW_BLOCK, SCHEME_DOUBLE_CHANNEL = 0, 1, 2
 PART_FORWARD, PART_BACKWARD, PART_KEEP = 1, 2, 4

@@ -823,6 +823,8 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
     if (!problems) return fail(TI8_ERR_NULL, "%s: problems is required", fn);
     if (count < 1 || count > GEMM_MULTI_MAX) return fail(TI8_ERR_SHAPE, "%s: between 1 and %d GEMMs, got %d", fn, GEMM_MULTI_MAX, count);
     if (gemm_flags & TI8_GEMM_SKINNY) return fail(TI8_ERR_MODE, "%s: the few-rows kernel is not offered here", fn);
+    const bool together = (gemm_flags & TI8_GEMM_TOGETHER) != 0;
+    gemm_flags &= ~TI8_GEMM_TOGETHER;
     GemmMulti m;
     m.count = count;
     idx::GemmConfig c[GEMM_MULTI_MAX];
@@ -839,12 +841,34 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
     hipStream_t st = static_cast<hipStream_t>(stream);
     const bool persistent = !(gemm_flags & TI8_GEMM_ONE_TILE);
     bool done[GEMM_MULTI_MAX] = {false, false, false}, chains[GEMM_MULTI_MAX];
+    if (together) {
+        // The medium-size kernel is one workgroup per CU: in a second round of 128 x 128 tiles the four-wave kernel, two workgroups per
+        // CU, hides their turn-over (step of 2048 tokens, 2048 -> 2048, 768 tiles: 61 us against 76; 1280 tokens, 1408 -> 2432, 519
+        // tiles: 46 / 52; 2048 tokens, 1024 -> 1024, 320 tiles: 37 / 41; 384 tokens, 1408 -> 2432, 299 tiles: 39 / 36)
+        int64_t tiles = 0;
+        for (int i = 0; i < count; ++i)
+            if (c[i].bm == 128 && c[i].bn == 128) tiles += (problems[i].M / 128) * (problems[i].N / 128);
+        if (4 * tiles >= 5 * device_cu_count())
+            for (int i = 0; i < count; ++i) c[i].mid = 0;
+    }
     for (int i = 0; i < count; ++i) {
         GemmMulti one;
         one.count = 1;
         one.g[0] = m.g[i];
         chains[i] = persistent && c[i].epi == EPI_PROMOTE_CHAIN && chain_persistent_supported(one);
     }
+    // Both kernels of the chained promotion in one call (an odd number of K tiles keeps a GEMM off the persistent one; same bits on
+    // either): apart, the persistent kernel's last round is paid for in full, so they go apart only where it fills its rounds (8576
+    // tokens, 2944 -> 12800, H_128, dX alone 408 tiles on 256 CUs: apart 1450 us, together 1406)
+    int64_t chain_tiles = 0, others = 0;
+    for (int i = 0; i < count; ++i) {
+        if (c[i].epi != EPI_PROMOTE_CHAIN) continue;
+        if (chains[i]) chain_tiles += ((problems[i].M + 255) / 256) * ((problems[i].N + 255) / 256);
+        else ++others;
+    }
+    const int64_t cus = device_cu_count(), rounds = (chain_tiles + cus - 1) / cus;
+    if (others && chain_tiles * 20 < rounds * cus * 19)
+        for (int i = 0; i < count; ++i) chains[i] = false;
     for (int i = 0; i < count; ++i) {
         if (done[i]) continue;
         GemmMulti part;
@@ -854,7 +878,7 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
             part.g[part.count++] = m.g[j];
             done[j] = true;
         }
-        if (int e = launch_group(fn, part, c[i], persistent, st)) return e;
+        if (int e = launch_group(fn, part, c[i], chains[i], st)) return e;
     }
     return TI8_OK;
 }

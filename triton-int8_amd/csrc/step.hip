@@ -321,7 +321,7 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
     };
     // they go into one launch where none of them has so few rows that it would take the few-rows kernel
     if (L.bwd && (L.T < L.N ? L.T : L.N) > 256) {
-        if (int e = ti8_gemm_i8_nt_multi(g, count, flags, stream)) return e;
+        if (int e = ti8_gemm_i8_nt_multi(g, count, flags | TI8_GEMM_TOGETHER, stream)) return e;
         return L.fwd && L.a->bias ? add_bias(L.a->Y, L.a->ldy, L.a->bias, L.tokens, L.N, stream) : TI8_OK;
     }
     for (int i = 0; i < count; ++i) {

@@ -327,7 +327,7 @@ def linear_fwd_bwd(X, W, dY, scheme="block_channel", hadamard=None, out=None, wo
         saved["dYq"] = pre[1]
     dX, dW = linear_backward(dY2, X2, W, scheme, hadamard, saved, tokens=T, gemms=gemms)
     if gemms:
-        ops.gemm_i8_nt_multi(gemms)   # Y, dX and dW, into the tensors handed out above
+        ops.gemm_i8_nt_multi(gemms, together=True)   # Y, dX and dW, into the tensors handed out above
     return Y[:T].reshape(*lead, N), dX[:T].reshape(*lead, K), dW
 
 
@@ -381,7 +381,7 @@ class Int8LinearFunction(torch.autograd.Function):
             gemms = [] if _one_launch(ctx.scheme, ctx.hadamard, xp.shape[0], N) else None
             dx, dw = linear_backward(dyp, xp, weight, ctx.scheme, ctx.hadamard, ctx.saved_q, tokens=tokens, gemms=gemms)
             if gemms:
-                ops.gemm_i8_nt_multi(gemms)   # dX and dW in one launch
+                ops.gemm_i8_nt_multi(gemms, together=True)   # dX and dW in one launch
         db = None
         if ctx.has_bias:
             # (a backward that is differentiated again needs the sum as a torch operator)

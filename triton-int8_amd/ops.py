@@ -13,7 +13,7 @@ import threading
 import torch
 
 from . import _lib
-from ._lib import (COMBINE_DIV_PROD, COMBINE_MUL_MUL, COMBINE_MUL_PROD, GEMM_LARGE_TILES, GEMM_ONE_TILE, GEMM_SKINNY, GEMM_STRICT, GEMM_TILED, INV_AMAX_DIV_127,
+from ._lib import (COMBINE_DIV_PROD, COMBINE_MUL_MUL, COMBINE_MUL_PROD, GEMM_LARGE_TILES, GEMM_ONE_TILE, GEMM_SKINNY, GEMM_STRICT, GEMM_TILED, GEMM_TOGETHER, INV_AMAX_DIV_127,
                    INV_AMAX_MUL_RCP127, INV_MULTIPLIER, INV_RCP_OF_SCALE, Q_CLAMP, Q_EPS_ADD, Q_HAD128, Q_SCALE_BF16, Q_TORCH_BF16, Q_TORCH_ROUND,
                    Q_WS_PINGPONG, Q_WS_SECOND,
                    SCALE_BLOCK128, SCALE_BLOCK_K256, SCALE_ROW, SCALE_ROW_K128)
@@ -393,11 +393,12 @@ def gemm_i8_nt(A, B, sA, modeA, sB, modeB, *, acc_i32_full=False, combine=COMBIN
     return out
 
 
-def gemm_i8_nt_multi(problems):
+def gemm_i8_nt_multi(problems, together=False):
     """Up to 3 GEMMs ``dequant(A @ B^T)`` with A int8 [M, K] and B int8 [N, K] in ONE launch; `problems`
     is a list of dicts with the keys A, B, sA, modeA, sB, modeB and optionally acc_i32_full, combine,
     out_scale, post_scale, out (meaning as in ``gemm_i8_nt``).  Returns the bf16 outputs [M, N],
-    bit-identical to separate calls.  The GEMMs must select the same kernel (else RuntimeError)."""
+    bit-identical to separate calls; with ``together`` the kernels are chosen for the launch as a whole, and a promoted sum may
+    associate differently."""
     _need(1 <= len(problems) <= 3, "between 1 and 3 GEMMs")
     descs, outs, keep = (_lib.GemmProblem * len(problems))(), [], []
     for i, p in enumerate(problems):
@@ -423,7 +424,7 @@ def gemm_i8_nt_multi(problems):
                                     float(p.get("out_scale", 1.0)), float(p.get("post_scale", 0.0)))
         outs.append(out)
         keep.append((A, B, sAv, sBv))     # contiguous copies stay alive until the launch is queued
-    _lib.call("ti8_gemm_i8_nt_multi", descs, len(problems), {"auto": 0, "tiled": GEMM_TILED, "large": GEMM_LARGE_TILES}.get(GEMM_PATH, 0) | (0 if GEMM_PERSISTENT else GEMM_ONE_TILE), _stream())
+    _lib.call("ti8_gemm_i8_nt_multi", descs, len(problems), _gemm_flags() | (GEMM_TOGETHER if together else 0), _stream())
     return outs
 
 
@@ -521,7 +522,7 @@ def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=Non
     if one_launch and parts & _lib.PART_BACKWARD and min(T, N) > 256:
         problems, count = (_lib.GemmProblem * 3)(), ctypes.c_int(0)
         _lib.call("ti8_linear_quantise", ctypes.byref(a), problems, ctypes.byref(count), stream)
-        _lib.call("ti8_gemm_i8_nt_multi", problems, count.value, a.gemm_flags, stream)
+        _lib.call("ti8_gemm_i8_nt_multi", problems, count.value, a.gemm_flags | GEMM_TOGETHER, stream)
     else:
         _lib.call("ti8_linear", ctypes.byref(a), stream)
     return Y, dX, dW, saved
