@@ -59,6 +59,7 @@ enum ti8_qflags {
                                reference's pure-torch quantisers instead of its Triton kernels' -- scale =
                                reciprocal(max(amax, 1e-4)) * 127, q = clamp(round_half_even(x * scale), -127, 127), stored
                                scale = reciprocal(scale) (per_block_cast_to_int8 of tilelang/block_channel_bwd.py:96-104) */
+    TI8_Q_SCALE_T = 512,    /* ti8_quant_row with group = 128 only: scales stored as s[cols/128][rows] */
     TI8_Q_TORCH_BF16 = 128  /* the same with every intermediate rounded to bf16, the product x * scale included: what torch
                                computes when the input is bf16 and nothing widens it (per_token_cast_to_int8 /
                                per_block_cast_to_int8 of tilelang/block_channel_fwd.py:215-230) */

@@ -720,7 +720,7 @@ static int try_chain_persistent(GemmMulti& m, const int64_t* batch, hipStream_t 
 
 // One GEMM on the LDS-tiled kernel that `c` names
 static int launch_tiled(const char* fn, const GemmArgs& a, int64_t batch, const idx::GemmConfig& c, bool persistent, hipStream_t st) {
-    if (c.epi == EPI_PROMOTE_CHAIN && persistent) {
+    if ((c.epi == EPI_PROMOTE_CHAIN || c.epi == EPI_PROMOTE_CHAIN_LANE) && persistent) {
         GemmMulti m;
         m.count = 1;
         m.g[0] = a;

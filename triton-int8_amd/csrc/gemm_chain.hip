@@ -15,6 +15,10 @@
 // tile's K tiles alternate between the two LDS buffers from a fixed start, which makes every LDS address a register
 // plus an immediate; one register holds the per-K-tile factors of 64 K tiles and is refilled every 64; the launcher
 // sends other shapes to the one-tile kernel).
+//
+// The body is shared by two kernels: gemm_i8_chain_kernel, whose per-K-tile factor is uniform over a wave's tile, and
+// gemm_i8_chain_lane_kernel, for operand B scaled per (row, K tile) (EPI_PROMOTE_CHAIN_LANE), where every lane fetches the
+// scales of its two columns one K tile ahead -- with the operand loads of that K tile, across tile boundaries too.
 #include <type_traits>
 #include "gemm_args.h"
 
@@ -71,9 +75,10 @@ struct Tile {
     uint32_t col_s;          // their stride (0 when B has none)
 };
 
-}  // namespace
-
-__global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti m, const int total_tiles) {
+// LANEB: operand B has one scale per (row, K tile); `col_p` / `col_s` then lead to the K tile 0 scales of the wave tile's
+// columns, `fb_ks` from one K tile to the next.
+template <bool LANEB>
+__device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_tiles) {
     extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
     // layout: [A buf0][A buf1][B buf0][B buf1][epilogue slab]
     int8_t* const ldsA = smem;
@@ -132,7 +137,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
         t.fa_ks = a_in ? (uint32_t)g.sa.ks : 0u;
         t.fb_ks = b_in ? (uint32_t)g.sb.ks : 0u;
         t.wide = __builtin_amdgcn_readfirstlane((g.sa.mode == TI8_SCALE_BLOCK_K256 ? 1 : 0) | (g.sb.mode == TI8_SCALE_BLOCK_K256 ? 2 : 0));
-        t.col_s = b_in ? 0u : (uint32_t)g.sb.rs;
+        t.col_s = b_in && !LANEB ? 0u : (uint32_t)g.sb.rs;
         t.col_p = g.sb.p + idx::epi_col_scale_index(t.batch, g.sb.bs, idx::chain_col_scale_first(t.n0 + wn * WCOLS, g.N), g.N, t.col_s);
         return t;
     };
@@ -158,16 +163,20 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
     auto load_raw_factors = [&](const Tile& t, int block64, float& ra, float& rb) {
         const uint32_t kt = (uint32_t)idx::gemm_factor_kt(block64, opaque_lane(), t.nk);
         ra = t.fa_p[(kt >> (t.wide & 1)) * t.fa_ks];
-        rb = t.fb_p[(kt >> ((t.wide >> 1) & 1)) * t.fb_ks];
+        rb = LANEB ? 1.0f : t.fb_p[(kt >> ((t.wide >> 1) & 1)) * t.fb_ks];
     };
     // the same two loads written out, for the place where the compiler must not count them: it would wait for the
     // epilogue's stores along with them (the caller waits with the counts it knows, then calls `landed`)
     auto load_raw_factors_uncounted = [&](const Tile& t, float& ra, float& rb) {
         const uint32_t kt = (uint32_t)idx::gemm_factor_kt(0, opaque_lane(), t.nk);
         const float* pa = t.fa_p + (kt >> (t.wide & 1)) * t.fa_ks;
-        const float* pb = t.fb_p + (kt >> ((t.wide >> 1) & 1)) * t.fb_ks;
         asm volatile("global_load_dword %0, %1, off" : "=v"(ra) : "v"(pa) : "memory");
-        asm volatile("global_load_dword %0, %1, off" : "=v"(rb) : "v"(pb) : "memory");
+        if constexpr (!LANEB) {
+            const float* pb = t.fb_p + (kt >> ((t.wide >> 1) & 1)) * t.fb_ks;
+            asm volatile("global_load_dword %0, %1, off" : "=v"(rb) : "v"(pb) : "memory");
+        } else {
+            rb = 1.0f;
+        }
     };
     auto landed = [&](float& ra, float& rb) { asm volatile("" : "+v"(ra), "+v"(rb)); };
     // 16 bytes from LDS that the compiler does not count (the caller waits for lgkmcnt itself)
@@ -180,6 +189,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
     auto finish_factors = [&](const Tile& t, float ra, float rb) {
         const GemmArgs& g = m.g[t.gi];
         float f = g.sa.mode != TI8_SCALE_ROW ? ra : 1.0f;
+        if (LANEB) return f;   // B's part, and the reciprocal of the product, per lane in the K loop
         if (g.sb.mode != TI8_SCALE_ROW) f = f * rb;
         if (g.combine == TI8_COMBINE_DIV_PROD) f = 1.0f / f;
         return f;
@@ -212,12 +222,23 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
 #pragma unroll
         for (int j = 0; j < TN; ++j) fbv[j][ks] = *reinterpret_cast<const v4i*>(smem + bbase[ks] + (stage * B_BYTES + j * 4096));
     };
-    float f_cur = 1.0f;
+    // factors of the K tile being folded, one per block column (the same wave-uniform value without LANEB)
+    float f_cur = 1.0f, f_lane[TN] = {1.0f, 1.0f};
     auto fold = [&](int i, const v16i& d0, const v16i& d1) {
+        const float f0 = LANEB ? f_lane[0] : f_cur, f1 = LANEB ? f_lane[1] : f_cur;
 #pragma unroll
-        for (int r = 0; r < 16; ++r) accf[i][0][r] = __builtin_fmaf(static_cast<float>(d0[r]), f_cur, accf[i][0][r]);
+        for (int r = 0; r < 16; ++r) accf[i][0][r] = __builtin_fmaf(static_cast<float>(d0[r]), f0, accf[i][0][r]);
 #pragma unroll
-        for (int r = 0; r < 16; ++r) accf[i][1][r] = __builtin_fmaf(static_cast<float>(d1[r]), f_cur, accf[i][1][r]);
+        for (int r = 0; r < 16; ++r) accf[i][1][r] = __builtin_fmaf(static_cast<float>(d1[r]), f1, accf[i][1][r]);
+    };
+    // LANEB: B's scales of this lane's two columns in the next K tile to be multiplied
+    float fb_next[TN] = {1.0f, 1.0f};
+    bool divide_by_f = false;
+    auto load_lane_factors = [&](const Tile& t, int kt) {
+        const float* p = t.col_p + (uint64_t)((uint32_t)kt * t.fb_ks);
+        const uint32_t c0 = (uint32_t)(opaque_lane() & 31) * t.col_s;
+#pragma unroll
+        for (int j = 0; j < TN; ++j) fb_next[j] = (p + (uint64_t)(32u * (uint32_t)j * t.col_s))[c0];
     };
 
     // One K tile in LDS buffer `parity` (a tile's K tile kt sits in buffer kt & 1); the B half of the K tile
@@ -237,6 +258,18 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
         constexpr int cur = decltype(parity_tag)::value;
         constexpr int stA = cur, stAn = cur ^ 1, stBn = cur ^ 1;
         f_cur = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fvec), kt & 63));
+        if constexpr (LANEB) {
+            // this K tile's factors, and its successor's scales on their way: ahead of the operand loads that the wait in front
+            // of the barrier covers (behind a tile's first K tile the compiler waits for them in the next one)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) f_lane[j] = f_cur * fb_next[j];
+            load_lane_factors(nb, koff_b >> 7);
+#pragma unroll
+            for (int j = 0; j < TN; ++j) {
+                const float rf = 1.0f / f_lane[j];
+                f_lane[j] = divide_by_f ? rf : f_lane[j];
+            }
+        }
         if (!FIRST) load_b(nb, koff_b, wB + (cur ^ 1) * B_BYTES);
 #pragma unroll
         for (int i = 0; i < TM - 1; ++i) {
@@ -304,7 +337,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
         const int rb_col = idx::epi_col_of_lane(el, WCOLS), rb_row = idx::epi_row_of_lane(el, WCOLS);
         const int e_row = el & 31, e_half = el >> 5;
         const bool divide = g.combine == TI8_COMBINE_DIV_PROD;
-        const bool row_part = g.sa.mode == TI8_SCALE_ROW, col_part = g.sb.mode == TI8_SCALE_ROW;
+        const bool row_part = g.sa.mode == TI8_SCALE_ROW, col_part = !LANEB && g.sb.mode == TI8_SCALE_ROW;
         float cm[8];
 #pragma unroll
         for (int c = 0; c < 8; ++c) {
@@ -401,6 +434,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
         load_b(cur, 0, wB);
         float ra, rb;
         load_raw_factors(cur, 0, ra, rb);
+        if (LANEB) load_lane_factors(cur, 0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
         fvec = finish_factors(cur, ra, rb);
@@ -413,6 +447,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
     bool stored = false;   // whether this wave's previous epilogue left stores behind
     while (true) {
         const int nk = cur.nk;
+        if (LANEB) divide_by_f = m.g[cur.gi].combine == TI8_COMBINE_DIV_PROD;
         // all but the last K tile: B of kt + 1 from this tile (for kt = 0 it is under way already); A of kt + 2 from this tile,
         // in the last of them K tile 0 of the next
         using T_ = std::true_type;
@@ -445,8 +480,8 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
             kt += 2;
         }
         // last K tile: the column scales of this tile's epilogue travel beside it
-        float coln[4];
-        load_col_scales(cur, coln);
+        float coln[4] = {1.0f, 1.0f, 1.0f, 1.0f};
+        if (!LANEB) load_col_scales(cur, coln);
         __builtin_amdgcn_sched_barrier(0);
         ktile_p(F_{}, F_{}, P1{}, false, fvec, nk - 1, nxt, 0, nxt, 128);
         // the accumulators are complete HERE: without this the optimiser moves the last K tile's convert + fma behind
@@ -494,11 +529,27 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti 
     __builtin_amdgcn_s_waitcnt(0);
 }
 
+}  // namespace
+
+__global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti m, const int total_tiles) {
+    chain_tiles<false>(m, total_tiles);
+}
+
+__global__ __launch_bounds__(64 * NW) void gemm_i8_chain_lane_kernel(const GemmMulti m, const int total_tiles) {
+    chain_tiles<true>(m, total_tiles);
+}
+
+// operand B scaled per (row, K tile): all GEMMs of a launch or none
+static bool lane_scales(const GemmMulti& m) { return m.g[0].sb.mode == TI8_SCALE_ROW_K128; }
+
 bool chain_persistent_supported(const GemmMulti& m) {
     for (int i = 0; i < m.count; ++i) {
         const int nk = m.g[i].K >> 7;
         if (nk < 2 || nk > 256 || (nk & 1) || m.g[i].strict) return false;
-        if (m.g[i].sa.mode == TI8_SCALE_ROW_K128 || m.g[i].sb.mode == TI8_SCALE_ROW_K128) return false;
+        if (m.g[i].sa.mode == TI8_SCALE_ROW_K128 || (m.g[i].sb.mode == TI8_SCALE_ROW_K128) != lane_scales(m)) return false;
+        // row by row, a wave's scales lie in 32 cache lines per load and bound either kernel (4 x 8192^3, whole call: 2835 us here, 2769
+        // on one workgroup per tile); column by column 2361 against 2496 us for the GEMM
+        if (lane_scales(m) && m.g[i].sb.rs != 1) return false;
         // the epilogue stores 16 bytes per lane and row (the one-tile kernels store 8)
         if ((reinterpret_cast<uintptr_t>(m.g[i].C) & 15) || (m.g[i].ldc % 8) || (m.g[i].bsc % 8)) return false;
         // per-lane offsets into the scale arrays are kept in 32 bits: 64 K blocks x stride, 64 columns x stride
@@ -512,11 +563,13 @@ bool chain_persistent_supported(const GemmMulti& m) {
 // its batch count; one workgroup per CU (fewer when there are fewer tiles)
 // Whether the current device grants the kernel its 160 KiB of LDS (asked once per device).  A refusal is remembered
 // and reported through ti8_last_error() by the call that met it; callers then take the one-tile kernel.
+template <bool LANEB>
 static bool chain_kernel_available() {
     static OncePerDevice granted, refused;
     const uint64_t bit = 1ull << (current_device() & 63);
     if (refused.done.load(std::memory_order_acquire) & bit) return false;
-    const hipError_t e = raise_lds_limit(granted, reinterpret_cast<const void*>(gemm_i8_chain_kernel), LDS_BYTES);
+    const void* kern = LANEB ? reinterpret_cast<const void*>(gemm_i8_chain_lane_kernel) : reinterpret_cast<const void*>(gemm_i8_chain_kernel);
+    const hipError_t e = raise_lds_limit(granted, kern, LDS_BYTES);
     if (e == hipSuccess) return true;
     refused.done.fetch_or(bit, std::memory_order_release);
     (void)fail(TI8_OK, "gemm: device %d refuses %d bytes of LDS for the persistent kernel (%s); one workgroup per tile serves its shapes",
@@ -525,15 +578,18 @@ static bool chain_kernel_available() {
 }
 
 int init_chain_kernel() {
-    (void)chain_kernel_available();
+    (void)chain_kernel_available<false>();
+    (void)chain_kernel_available<true>();
     return TI8_OK;
 }
 
 int launch_chain_persistent(const GemmMulti& m, int total_tiles, int num_cu, hipStream_t st) {
-    if (!chain_kernel_available()) return CHAIN_UNAVAILABLE;
+    const bool lane = lane_scales(m);
+    if (!(lane ? chain_kernel_available<true>() : chain_kernel_available<false>())) return CHAIN_UNAVAILABLE;
     const int grid = total_tiles < num_cu ? total_tiles : num_cu;
-    hipLaunchKernelGGL(gemm_i8_chain_kernel, dim3((unsigned)grid), dim3(64 * NW), LDS_BYTES, st, m, total_tiles);
-    note_gemm_kernel(TI8_KERNEL_PERSISTENT_CHAIN, BM, BN, EPI_PROMOTE_CHAIN);
+    const auto kernel = lane ? gemm_i8_chain_lane_kernel : gemm_i8_chain_kernel;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * NW), LDS_BYTES, st, m, total_tiles);
+    note_gemm_kernel(TI8_KERNEL_PERSISTENT_CHAIN, BM, BN, lane ? EPI_PROMOTE_CHAIN_LANE : EPI_PROMOTE_CHAIN);
     return check_launch("ti8_gemm_i8_nt");
 }
 

@@ -410,7 +410,7 @@ __global__ __launch_bounds__(256) void quant_row_kernel(const uint16_t* __restri
             const float scale = 127.0f / amax;
             if (c < nchunk) {
                 *reinterpret_cast<uint2*>(qr + c * 8) = quant8(v[i], scale * lane_sign);
-                if ((c & 15) == 0) s[row * ngrp + (c >> 4)] = stored_scale(amax, scale, mode);
+                if ((c & 15) == 0) s[mode.scale_t ? (int64_t)(c >> 4) * rows + row : row * ngrp + (c >> 4)] = stored_scale(amax, scale, mode);
             }
         }
         return;
@@ -821,8 +821,11 @@ extern "C" int ti8_quant_row(const void* x, int64_t ldx, int8_t* q, int64_t ldq,
                              int64_t cols, int group, int qflags, int inv_mode, ti8_stream_t stream) {
     QMode mode;
     const int arith = arith_of(qflags);
-    qflags &= ~(TI8_Q_TORCH_ROUND | TI8_Q_TORCH_BF16);
+    const bool scale_t = (qflags & TI8_Q_SCALE_T) != 0;
+    qflags &= ~(TI8_Q_TORCH_ROUND | TI8_Q_TORCH_BF16 | TI8_Q_SCALE_T);
     if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
+    mode.scale_t = scale_t;
+    if (scale_t && group != 128) return fail(TI8_ERR_MODE, "ti8_quant_row: TI8_Q_SCALE_T goes with group = 128");
     if (arith != ARITH_KERNEL && (group != 0 || (qflags & (TI8_Q_EPS_ADD | TI8_Q_SCALE_BF16 | TI8_Q_HAD128)) || inv_mode != TI8_INV_RCP_OF_SCALE))
         return fail(TI8_ERR_MODE, "ti8_quant_row: the torch arithmetic goes with group = 0, no other flag and TI8_INV_RCP_OF_SCALE");
     if (!x || !q || !s) return fail(TI8_ERR_NULL, "ti8_quant_row: x, q and s are required");

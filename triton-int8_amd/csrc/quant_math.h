@@ -12,6 +12,7 @@ struct QMode {
     int eps_add;     // TI8_Q_EPS_ADD
     int scale_bf16;  // TI8_Q_SCALE_BF16
     int inv_mode;    // ti8_inv_mode
+    int scale_t = 0; // TI8_Q_SCALE_T (per-row quantiser with groups)
 };
 
 // Arithmetic of the conversion.  ARITH_KERNEL is that of the reference's Triton kernels.  The

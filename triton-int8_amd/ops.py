@@ -14,7 +14,7 @@ import torch
 
 from . import _lib
 from ._lib import (COMBINE_DIV_PROD, COMBINE_MUL_MUL, COMBINE_MUL_PROD, GEMM_LARGE_TILES, GEMM_ONE_TILE, GEMM_SKINNY, GEMM_STRICT, GEMM_TILED, GEMM_TOGETHER, INV_AMAX_DIV_127,
-                   INV_AMAX_MUL_RCP127, INV_MULTIPLIER, INV_RCP_OF_SCALE, Q_CLAMP, Q_EPS_ADD, Q_HAD128, Q_SCALE_BF16, Q_TORCH_BF16, Q_TORCH_ROUND,
+                   INV_AMAX_MUL_RCP127, INV_MULTIPLIER, INV_RCP_OF_SCALE, Q_CLAMP, Q_EPS_ADD, Q_HAD128, Q_SCALE_BF16, Q_SCALE_T, Q_TORCH_BF16, Q_TORCH_ROUND,
                    Q_WS_PINGPONG, Q_WS_SECOND,
                    SCALE_BLOCK128, SCALE_BLOCK_K256, SCALE_ROW, SCALE_ROW_K128)
 
@@ -165,9 +165,10 @@ def quant_block_had128(x, *, along_rows=False, clamp=True, inv_mode=INV_RCP_OF_S
 
 
 def quant_row(x, *, clamp=True, group=0, eps_add=False, scale_bf16=False, inv_mode=INV_RCP_OF_SCALE, hadamard128=False,
-              torch_arith=None):
+              torch_arith=None, scale_t=False):
     """Per-row (``group=0``) or per-(row, 128 columns) absmax quantisation of the last dim.
-    ``x``: bf16 [..., cols].  Returns ``(q, s)`` with ``s`` fp32 [...] or [..., cols/128].
+    ``x``: bf16 [..., cols].  Returns ``(q, s)`` with ``s`` fp32 [...] or [..., cols/128]; with ``scale_t`` (2-D x, group 128)
+    ``s`` [rows, cols/128] lies in memory column by column, where a GEMM's lanes find neighbouring rows side by side.
     ``hadamard128`` rotates every group of 128 columns by H_128 first (fused, one read)."""
     _check_bf16(x, "x")
     _need(x.dim() >= 1 and x.numel() > 0, "x must be a non-empty tensor")
@@ -178,9 +179,12 @@ def quant_row(x, *, clamp=True, group=0, eps_add=False, scale_bf16=False, inv_mo
         x2 = x2.contiguous()
     rows = x2.shape[0]
     q = torch.empty((rows, cols), dtype=torch.int8, device=x.device)
-    s = torch.empty((rows, cols // 128) if group else (rows,), dtype=torch.float32, device=x.device)
+    _need(not scale_t or (group and x.dim() == 2), "scale_t needs a 2-D x and groups of 128 columns")
+    s = torch.empty((cols // 128, rows) if scale_t else (rows, cols // 128) if group else (rows,), dtype=torch.float32, device=x.device)
     _lib.call("ti8_quant_row", x2.data_ptr(), x2.stride(0), q.data_ptr(), cols, s.data_ptr(), rows, cols, group,
-              _qflags(clamp, eps_add, scale_bf16, torch_arith) | (Q_HAD128 if hadamard128 else 0), inv_mode, _stream())
+              _qflags(clamp, eps_add, scale_bf16, torch_arith) | (Q_HAD128 if hadamard128 else 0) | (Q_SCALE_T if scale_t else 0), inv_mode, _stream())
+    if scale_t:
+        return q, s.t()
     lead = x.shape[:-1]
     return q.reshape(*lead, cols), s.reshape(*lead, cols // 128) if group else s.reshape(*lead)
 
