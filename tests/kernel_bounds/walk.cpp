@@ -592,6 +592,41 @@ int walk_gemm_chain(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t 
     return r.bad;
 }
 
+// Tiles of the persistent chained kernel's workgroups, round by round: each of `total` exactly once
+int walk_chain_rounds(int total, int grid, int several, int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    std::vector<int> seen((size_t)total, 0);
+    for (int w = 0; w < grid; ++w) {
+        ++seen[(size_t)w];
+        for (int base = grid;; base += grid) {
+            const int t = chain_tile_of_round(base, grid, total, w, several != 0);
+            if (t >= total) break;
+            if (t < base || t >= base + grid) r.fail("chain rounds: workgroup %d takes tile %d in the round from %d", w, t, base);
+            ++seen[(size_t)t];
+        }
+    }
+    for (int t = 0; t < total && !r.bad; ++t) {
+        if (seen[(size_t)t] != 1) r.fail("chain rounds: tile %d is taken %d times", t, seen[(size_t)t]);
+        ++r.checked;
+    }
+    *n_checked = r.checked;
+    return r.bad;
+}
+
+// Choice of kernels for a launch of several GEMMs of shapes shape[i] = {M, N, K}: cfg[3 i ..] = bm, bn, mid of GEMM i alone, then of the
+// launch (9 values each)
+void walk_configs_together(const int64_t* shape, int count, int i32, int num_cu, int* cfg) {
+    GemmConfig c[3];
+    int64_t s[3][3];
+    for (int i = 0; i < count; ++i) {
+        for (int d = 0; d < 3; ++d) s[i][d] = shape[3 * i + d];
+        c[i] = gemm_config(s[i][0], s[i][1], s[i][2], 1, i32 != 0, false, i32 ? 0 : 1, i32 ? 0 : 1, false, num_cu);
+        cfg[3 * i] = c[i].bm; cfg[3 * i + 1] = c[i].bn; cfg[3 * i + 2] = c[i].mid;
+    }
+    gemm_configs_together(s, count, false, num_cu, c);
+    for (int i = 0; i < count; ++i) { cfg[9 + 3 * i] = c[i].bm; cfg[9 + 3 * i + 1] = c[i].bn; cfg[9 + 3 * i + 2] = c[i].mid; }
+}
+
 // Workgroup -> (GEMM, tile) map of a several-GEMM launch (gemm.hip: gemm_i8_multi_kernel, launch_multi):
 // tiles[i] = workgroups of GEMM i.  Every workgroup of the grid must land in a GEMM i < count with
 // a tile index in [0, tiles[i]), and every (GEMM, tile) must be taken exactly once.

@@ -44,6 +44,9 @@ def walker(tmp_path_factory):
     lib.walk_quant_block.argtypes = [i64, i64, ci, i64, i64, ci, i64, i64, i64, i64, i64, i64, i64, i64, ci, i64, i64, i64, i64, p64, cp, ci]
     lib.walk_gemm.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] * 5 + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_gemm_chain.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] + [i64] * 3 + [p64, cp, ci]
+    lib.walk_chain_rounds.argtypes = [ci, ci, ci, p64, cp, ci]
+    lib.walk_configs_together.argtypes = [p64, ci, ci, ci, ctypes.POINTER(ci)]
+    lib.walk_configs_together.restype = None
     lib.walk_gemm_multi_map.argtypes = [ctypes.POINTER(ci), ci, p64, cp, ci]
     return lib
 
@@ -367,3 +370,34 @@ def test_persistent_chain_kernel_geometries(walker, M, N, K, batch, mA, mB, grid
     rc = walker.walk_gemm_chain(M * K, K, N * K, K, M * N, N, ctypes.byref(sa), ctypes.byref(sb), batch, M, N, K, grid,
                                 batch * M * K - K, batch * N * K, batch * M * N, ctypes.byref(n), msg, 512)
     assert rc != 0 and b"gemm chain A" in msg.value
+
+
+@pytest.mark.parametrize("several", [0, 1])
+@pytest.mark.parametrize("total,grid", [(1, 1), (255, 255), (256, 256), (257, 256), (356, 256), (512, 256), (1000, 256), (1280, 256), (40, 7)])
+def test_rounds_of_the_persistent_kernel(walker, total, grid, several):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    assert walker.walk_chain_rounds(total, grid, several, ctypes.byref(n), msg, 512) == 0, msg.value.decode()
+    assert n.value == total
+
+
+@pytest.mark.parametrize("i32", [0, 1])
+def test_kernels_of_a_launch_as_a_whole(walker, i32):
+    """The GEMMs either keep the kernels that their shapes choose or share one that has a several-GEMMs form, whatever their order."""
+    tokens, features = (128, 384, 640, 1280, 2176, 4096, 9088), (128, 1024, 1408, 4096, 14336)
+    shared = 0
+    for t in tokens:
+        for k in features:
+            for n in features:
+                step = [(t, n, k), (t, k, n), (n, k, t)]
+                seen = set()
+                for shapes in (step, step[1:], step[::-1]):
+                    cfg = (ctypes.c_int * 18)()
+                    walker.walk_configs_together((ctypes.c_int64 * 9)(*sum(shapes, ())), len(shapes), i32, 256, cfg)
+                    alone = [tuple(cfg[3 * i:3 * i + 3]) for i in range(len(shapes))]
+                    launch = [tuple(cfg[9 + 3 * i:12 + 3 * i]) for i in range(len(shapes))]
+                    assert launch == alone or (len(set(launch)) == 1 and launch[0] in ((128, 128, 0), (256, 256, 0))), shapes
+                    shared += launch != alone
+                    if len(shapes) == 3:
+                        seen.add(tuple(launch if shapes is step else launch[::-1]))
+                assert len(seen) == 1, step
+    assert shared > 20

@@ -16,6 +16,7 @@
 // for both operands, which is all an NT dot product needs); result register r of lane
 // l is C[8*(r/4) + 4*(l/32) + r%4][l % 32] with rows from A and columns from B.
 #include <type_traits>
+#include <algorithm>
 #include "gemm_args.h"
 
 namespace ti8 {
@@ -842,14 +843,13 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
     const bool persistent = !(gemm_flags & TI8_GEMM_ONE_TILE);
     bool done[GEMM_MULTI_MAX] = {false, false, false}, chains[GEMM_MULTI_MAX];
     if (together) {
-        // The medium-size kernel is one workgroup per CU: in a second round of 128 x 128 tiles the four-wave kernel, two workgroups per
-        // CU, hides their turn-over (step of 2048 tokens, 2048 -> 2048, 768 tiles: 61 us against 76; 1280 tokens, 1408 -> 2432, 519
-        // tiles: 46 / 52; 2048 tokens, 1024 -> 1024, 320 tiles: 37 / 41; 384 tokens, 1408 -> 2432, 299 tiles: 39 / 36)
-        int64_t tiles = 0;
-        for (int i = 0; i < count; ++i)
-            if (c[i].bm == 128 && c[i].bn == 128) tiles += (problems[i].M / 128) * (problems[i].N / 128);
-        if (4 * tiles >= 5 * device_cu_count())
-            for (int i = 0; i < count; ++i) c[i].mid = 0;
+        int64_t shape[GEMM_MULTI_MAX][3];
+        for (int i = 0; i < count; ++i) {
+            shape[i][0] = problems[i].M;
+            shape[i][1] = problems[i].N;
+            shape[i][2] = problems[i].K;
+        }
+        idx::gemm_configs_together(shape, count, (gemm_flags & TI8_GEMM_LARGE_TILES) != 0, device_cu_count(), c);
     }
     for (int i = 0; i < count; ++i) {
         GemmMulti one;
@@ -878,6 +878,12 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
             part.g[part.count++] = m.g[j];
             done[j] = true;
         }
+        // The longest K first, so that the launch does not end on it; whole rounds of 256 x 256 tiles stay in their order (8192
+        // tokens, 4096 -> 4096, five rounds: 467 us, dW in front of Y and dX 473)
+        int64_t tiles = 0;
+        for (int k = 0; k < part.count; ++k) tiles += (((int64_t)part.g[k].M + c[i].bm - 1) / c[i].bm) * (((int64_t)part.g[k].N + c[i].bn - 1) / c[i].bn);
+        if (together && (c[i].bn != 256 || tiles % cus != 0))
+            std::stable_sort(part.g, part.g + part.count, [](const GemmArgs& x, const GemmArgs& y) { return x.K > y.K; });
         if (int e = launch_group(fn, part, c[i], chains[i], st)) return e;
     }
     return TI8_OK;

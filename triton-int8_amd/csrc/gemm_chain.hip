@@ -422,12 +422,14 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         return true;
     };
 
+    const auto tile_of_round = [&](int base) { return idx::chain_tile_of_round(base, stride_t, total_tiles, (int)blockIdx.x, m.count > 1); };
+
     // ---- first tile: operands of K tile 0 into LDS and registers, K tile 1's A half in flight ------------
-    int T = blockIdx.x;
-    Tile cur = locate(T);
+    int base = 0;      // first tile of the round of `cur`
+    Tile cur = locate(blockIdx.x);
     // without a next tile the loads that run ahead fetch this tile's K tiles 0 and 1 again (nobody reads them)
-    bool more = T + stride_t < total_tiles;
-    Tile nxt = more ? locate(T + stride_t) : cur;
+    bool more = tile_of_round(stride_t) < total_tiles;
+    Tile nxt = more ? locate(tile_of_round(stride_t)) : cur;
     float fvec;
     {
         load_a(cur, 0, wA);
@@ -514,10 +516,10 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         for (int ks = 0; ks < 4; ++ks) read_b(0, ks);
         read_a(0, 0, 0);
         // the accumulators are free: the place for the integer divisions that find the tile after the next
-        T += stride_t;
+        base += stride_t;
         cur = nxt;
-        more = T + stride_t < total_tiles;
-        if (more) nxt = locate(T + stride_t);
+        more = tile_of_round(base + stride_t) < total_tiles;
+        if (more) nxt = locate(tile_of_round(base + stride_t));
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll

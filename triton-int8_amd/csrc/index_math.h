@@ -123,6 +123,12 @@ TI8_HD int epi_scale_lane(int lane, int c) { return 2 * (lane % 8) + (c >> 2); }
 // first column whose per-row scale of B a wave of the persistent kernel fetches: its tile's first column, or, for a
 // tile outside the operand (N is a multiple of 128, the wave tile has 64 columns), the operand's last 64 columns
 TI8_HD int chain_col_scale_first(int first_col_of_wave_tile, int ncols) { return imin(first_col_of_wave_tile, ncols - 64); }
+// tile that workgroup `w` of `grid` takes in the round that starts at tile `base`: its own number, in a partly filled last round of a
+// launch of several GEMMs counted from the other end -- the longest K comes first there, so that round goes to the workgroups
+// whose tiles before it were short.  Past the last tile: no tile (>= total), and none in any later round.
+TI8_HD int chain_tile_of_round(int base, int grid, int total, int w, bool several) {
+    return several && base + grid > total ? base + grid - 1 - w : base + w;
+}
 TI8_HD int epi_chain_slab_row(int e, int fr_half) { return 8 * (e >> 2) + 4 * fr_half + (e & 3); }
 TI8_HD int epi_chain_slab_word(int row, int col) { return row * 64 + (col ^ (4 * (row & 1))); }
 // index of the column scale of column `col` (clamped to the last column; stride 0 when absent)
@@ -292,6 +298,121 @@ TI8_HD GemmConfig gemm_config(int64_t M, int64_t N, int64_t K, int64_t batch, bo
     // In between, 128 x 128 tiles on four waves, two workgroups per CU (1536 rows, K = 4096, 384 tiles: 42 / 33, against 52 /
     // 41 on 256 x 256 tiles and 51 / 42 on the medium-size kernel, whose 129 KiB of LDS leave room for one).
     return small;
+}
+
+// ---- several GEMMs in one launch: the kernel for all of them ----------------------------------------------------------------
+// A GEMM of its own pays for the last round of its tiles in full, so GEMMs that choose by their own shape and end up on different
+// kernels leave CUs idle several times (640 tokens, 2048 -> 5632, three GEMMs of a step: 63 us, on one kernel together 48; 1280
+// tokens, 1280 -> 1280: 25.6 / 18.3; 2560 tokens, 2048 -> 8192: 187 / 158).  The times below are fits, in us on 256 CUs, to 40
+// launches of 2 and 3 GEMMs of 384 .. 7040 tokens and 1024 .. 14336 features: a constant, the K tiles of the busiest CU, the mean
+// over the CUs, and what a tile or a round costs besides; off by 4 % in the mean and 11 % at most (int32: 21 %, on tiles that
+// leave most CUs idle).  Against the choice by shape alone the launches take 0.93 of the time in the mean and 1.01 at worst.
+struct GemmSet {
+    int64_t M[3], N[3], nk[3];   // nk (K tiles) descending: the order of the launch
+    int count;
+};
+TI8_HD int64_t gemm_set_tiles(const GemmSet& s, int i, int bm) { return ((s.M[i] + bm - 1) / bm) * ((s.N[i] + bm - 1) / bm); }
+// 128 x 128 tiles on four waves, two workgroups per CU
+TI8_HD double gemm_set_time_small(const GemmSet& s, bool i32, int num_cu) {
+    const double slots = 2.0 * num_cu;
+    double tiles = 0, work = 0;
+    for (int i = 0; i < s.count; ++i) {
+        tiles += (double)gemm_set_tiles(s, i, 128);
+        work += (double)(gemm_set_tiles(s, i, 128) * s.nk[i]);
+    }
+    const double mean = work / slots, over = tiles <= slots ? mean : mean + 0.5 * (double)s.nk[s.count - 1];
+    const double longest = over > (double)s.nk[0] ? over : (double)s.nk[0];
+    // (a tile alone on its CU waits through its K loop, however little the others have to do)
+    const double alone = i32 ? 5.0 + 0.62 * (double)s.nk[0] : 6.0 + 0.87 * (double)s.nk[0];
+    const double t = i32 ? 5.0 + 0.28 * longest + 0.71 * mean + 2.9 * tiles / slots : 6.3 + 0.37 * longest + 0.96 * mean + 1.84 * tiles / slots;
+    return t > alone ? t : alone;
+}
+// 256 x 256 tiles.  The busiest CU: workgroup w takes tile w of every round, in the last one counted from the end (as the persistent
+// kernel does); its load changes only where a GEMM begins, so those workgroups are looked at.
+TI8_HD double gemm_set_time_large(const GemmSet& s, bool i32, int num_cu) {
+    int64_t first[4] = {0, 0, 0, 0};
+    double work = 0;
+    for (int i = 0; i < s.count; ++i) {
+        first[i + 1] = first[i] + gemm_set_tiles(s, i, 256);
+        work += (double)(gemm_set_tiles(s, i, 256) * s.nk[i]);
+    }
+    const int64_t total = first[s.count], rounds = (total + num_cu - 1) / num_cu;
+    int64_t busiest = 0;
+    for (int q = 0; q < 4 * (s.count + 1); ++q) {
+        int64_t w = (first[q >> 2] + num_cu - 1 + (q & 1)) % num_cu;   // the last workgroup in front of GEMM q / 4, or its first
+        if (q & 2) w = num_cu - 1 - w;
+        int64_t load = 0;
+        for (int64_t r = 0; r < rounds; ++r) {
+            const int64_t t = r * num_cu + (r == rounds - 1 && s.count > 1 ? num_cu - 1 - w : w);
+            if (t < total) load += s.nk[t < first[1] ? 0 : (t < first[2] || s.count < 3 ? 1 : 2)];
+        }
+        if (load > busiest) busiest = load;
+    }
+    const double mean = work / num_cu, longest = (double)busiest;
+    if (i32) return 8.6 + 0.71 * longest + 0.95 * mean + 1.2 * (double)rounds;
+    // an odd number of K tiles keeps the launch off the persistent kernel
+    bool odd = false;
+    for (int i = 0; i < s.count; ++i) odd = odd || (s.nk[i] & 1);
+    return (7.7 + 1.15 * longest + 0.9 * mean + 0.4 * (double)rounds) * (odd ? 1.04 : 1.0);
+}
+// the medium-size kernel, one workgroup per CU: past one round a workgroup's turn-over is not hidden
+TI8_HD double gemm_set_time_mid(const GemmSet& s, bool i32, int num_cu) {
+    double tiles = 0, work = 0;
+    for (int i = 0; i < s.count; ++i) {
+        tiles += (double)gemm_set_tiles(s, i, 128) / num_cu;
+        work += (double)(gemm_set_tiles(s, i, 128) * s.nk[i]) / num_cu;
+    }
+    if (tiles > 1.0) work += (double)s.nk[s.count - 1] + 10.0;   // the last tiles, and 6 us of turn-over
+    const double longest = work > (double)s.nk[0] ? work : (double)s.nk[0];
+    return 7.0 + 0.5 * longest * (0.85 + 0.3 * (tiles < 1.0 ? tiles : 1.0)) * (i32 ? 0.85 : 1.0);
+}
+
+// 256 x 128 tiles, one workgroup per CU
+TI8_HD double gemm_set_time_half(const GemmSet& s, int num_cu) {
+    double work = 0;
+    for (int i = 0; i < s.count; ++i) work += (double)(((s.M[i] + 255) / 256) * (s.N[i] / 128) * s.nk[i]) / num_cu;
+    return 6.0 + 1.25 * (work > (double)s.nk[0] ? work : (double)s.nk[0]);
+}
+
+// `c` holds what gemm_config selects for each shape {M, N, K}, and becomes what the launch is to use
+TI8_HD void gemm_configs_together(const int64_t (*shape)[3], int count, bool large, int num_cu, GemmConfig* c) {
+    if (large || count < 2) return;
+    const bool i32 = c[0].epi == 1;
+    GemmSet all = {}, mids = {}, bigs = {}, halves = {}, smalls = {};
+    int order[3] = {0, 1, 2};
+    for (int i = 1; i < count; ++i)
+        for (int j = i; j > 0 && shape[order[j]][2] > shape[order[j - 1]][2]; --j) {
+            const int t = order[j];
+            order[j] = order[j - 1];
+            order[j - 1] = t;
+        }
+    int64_t mid_tiles = 0;
+    for (int q = 0; q < count; ++q) {
+        const int i = order[q];
+        // EPI_ROWS, or EPI_PROMOTE / EPI_PROMOTE_CHAIN: kernels that take each other's GEMMs
+        if (i32 ? c[i].epi != 1 : (c[i].epi != 2 && c[i].epi != 5)) return;
+        GemmSet* const sets[2] = {&all, c[i].mid ? &mids : (c[i].bn == 256 ? &bigs : (c[i].bm == 256 ? &halves : &smalls))};
+        for (int k = 0; k < 2; ++k) {
+            GemmSet& s = *sets[k];
+            s.M[s.count] = shape[i][0];
+            s.N[s.count] = shape[i][1];
+            s.nk[s.count++] = shape[i][2] >> 7;
+        }
+        if (c[i].mid) mid_tiles += gemm_set_tiles(all, q, 128);
+    }
+    if (bigs.count == count || (mids.count == count && mid_tiles <= num_cu)) return;
+    const double small = gemm_set_time_small(all, i32, num_cu), big = gemm_set_time_large(all, i32, num_cu);
+    // A launch for each kernel chosen; not for several rounds of medium-size tiles, and with 15 % on top where the four-wave kernel is
+    // among them (measured over predicted: 369 / 336 us, 193 / 168, 185 / 160 at 3200, 6016 and 2176 tokens)
+    double apart = mids.count == count && 4 * mid_tiles >= 5 * (int64_t)num_cu ? 1e30 : 0.0;
+    if (mids.count) apart += gemm_set_time_mid(mids, i32, num_cu);
+    if (bigs.count) apart += gemm_set_time_large(bigs, i32, num_cu);
+    if (halves.count) apart += gemm_set_time_half(halves, num_cu);
+    if (smalls.count) apart = 1.15 * (apart + gemm_set_time_small(smalls, i32, num_cu));
+    const double margin = 1.04;   // what the fits are off by
+    if (apart <= margin * small && apart <= margin * big) return;
+    for (int i = 0; i < count; ++i)
+        c[i] = big < small ? GemmConfig{256, 256, 2, 4, i32 ? 1 : 5, 0} : GemmConfig{128, 128, 2, 2, i32 ? 1 : 2, 0};
 }
 
 // Up to 256 rows: whether the medium-size kernel beats the few-rows kernel.  The latter's time grows with the bytes its 32 x

@@ -174,6 +174,11 @@ def linear_backward(dY2, X2, W, scheme="block_channel", hadamard=None, saved=Non
     _check(scheme, hadamard)
     saved = saved or {}
     T, N = dY2.shape
+    if gemms is None and _one_launch(scheme, hadamard, T, N):
+        gemms = []
+        grads = linear_backward(dY2, X2, W, scheme, hadamard, saved, tokens, gemms)
+        ops.gemm_i8_nt_multi(gemms, together=True)   # dX and dW, on the kernels that the layer's own backward takes
+        return grads
     K = X2.shape[1]
     if scheme == "block_channel":
         if hadamard == 128:
