@@ -808,6 +808,25 @@ int ti8::gemm_nt_bias(const ti8_gemm_problem& p, const void* bias, int gemm_flag
     return launch_tiled(fn, a, batch, c, !(gemm_flags & TI8_GEMM_ONE_TILE), st);
 }
 
+// Two GEMMs of batch 1 as one launch of the few-rows kernel, the bias with the first, if that is the kernel both would get alone
+// (same bits); *launched says whether they were.
+int ti8::gemm_nt_pair(const ti8_gemm_problem& p, const void* bias, const ti8_gemm_problem& q, int gemm_flags, bool* launched, ti8_stream_t stream) {
+    *launched = false;
+    if (gemm_flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES | TI8_GEMM_STRICT)) return TI8_OK;
+    GemmMulti m;
+    m.count = 2;
+    const ti8_gemm_problem* const both[2] = {&p, &q};
+    for (int i = 0; i < 2; ++i) {
+        const ti8_gemm_problem& x = *both[i];
+        if (x.M > 256 || x.batch != 1 || (x.acc_i32_full != 0) != (p.acc_i32_full != 0)) return TI8_OK;
+        if (int e = prepare_gemm("ti8_gemm_i8_nt", x, gemm_flags, &m.g[i])) return e;
+        if (!skinny_supported(m.g[i]) || idx::gemm_few_rows_prefers_mid(x.M, x.N, x.K, 1, device_cu_count())) return TI8_OK;
+    }
+    m.g[0].bias = static_cast<const uint16_t*>(bias);
+    *launched = true;
+    return launch_skinny_multi(m, p.acc_i32_full != 0, static_cast<hipStream_t>(stream));
+}
+
 extern "C" int ti8_gemm_i8_nt(const int8_t* A, int64_t bsa, int64_t lda, const int8_t* B, int64_t bsb, int64_t ldb,
                               void* C, int64_t bsc, int64_t ldc, const float* sA, int modeA, int64_t sa_bs,
                               int64_t sa_rs, int64_t sa_ks, const float* sB, int modeB, int64_t sb_bs, int64_t sb_rs,

@@ -86,5 +86,7 @@ int launch_mid(GemmMulti& m, int64_t batch, bool i32_full, hipStream_t st);
 // scales.  i32_full: int32 accumulation over the whole K with per-row scales (bit-exact path).
 bool skinny_supported(const GemmArgs& a);
 int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t st);
+// several GEMMs of batch 1 in one launch; fills first[] of `m`
+int launch_skinny_multi(GemmMulti& m, bool i32_full, hipStream_t st);
 
 }  // namespace ti8

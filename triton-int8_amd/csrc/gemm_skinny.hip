@@ -31,22 +31,22 @@ constexpr int WS_STAGES = 2;
 constexpr int WS_STAGE_BYTES = 2 * 32 * 128;
 constexpr int WS_LOADS = 8;  // global->LDS instructions per wave and stage
 
+// `block_x` = index of the workgroup among the blocks of this GEMM and batch.
 template <bool I32FULL>
-__global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g) {
+__device__ __forceinline__ void wavering_block(const GemmArgs& g, const int block_x, const int batch) {
     extern __shared__ __attribute__((aligned(1024))) int8_t smem[];  // 4 waves x WS_STAGES x 8 KiB
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int batch = blockIdx.y;
     const int mtiles = g.M >> 5, nstrips = g.N >> 5;
     int strip, mt;
     if ((nstrips & 7) == 0) {   // workgroups that share a strip of B on one XCD (ids 8 apart)
-        const int xcd = blockIdx.x & 7, idx = blockIdx.x >> 3;
+        const int xcd = block_x & 7, idx = block_x >> 3;
         strip = (idx / mtiles) * 8 + xcd;
         mt = idx % mtiles;
     } else {
-        strip = blockIdx.x / mtiles;
-        mt = blockIdx.x % mtiles;
+        strip = block_x / mtiles;
+        mt = block_x % mtiles;
     }
     const int n0 = strip * 32, m0 = mt * 32;
     const int nk = g.K >> 7;
@@ -69,7 +69,7 @@ __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g)
     int8_t* const ring = smem + wave * (WS_STAGES * WS_STAGE_BYTES);
     // step i of this wave's walk is K tile kbeg + (i + rot) mod nq: workgroups start at different
     // tiles so that they do not ask the same memory channels for their lines at the same time
-    const int rot = nq > 0 ? (int)(((blockIdx.x >> 3) * 3u + blockIdx.y) % (unsigned)nq) : 0;
+    const int rot = nq > 0 ? (int)((((unsigned)block_x >> 3) * 3u + (unsigned)batch) % (unsigned)nq) : 0;
     auto tile_of_step = [&](int i) {
         int j = min(i, max(nq - 1, 0)) + rot;   // past the end: the last one again, into a free stage
         if (j >= nq) j -= nq;
@@ -233,6 +233,19 @@ __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g)
     *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.C) + (int64_t)batch * g.bsc + (int64_t)(m0 + e_row) * g.ldc + n0 + e_col) = o;
 }
 
+template <bool I32FULL>
+__global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g) {
+    wavering_block<I32FULL>(g, blockIdx.x, blockIdx.y);
+}
+
+// Several GEMMs (batch of one each) in one launch: Y and dX of a step on few tokens, which have few blocks each and wait for their
+// loads most of the time (16 tokens, 4096 -> 4096: 128 blocks and 7.4 us each on 256 CUs; the step 50.3 us apart, 44.6 together).
+template <bool I32FULL>
+__global__ __launch_bounds__(256) void gemm_i8_wavering_multi_kernel(const GemmMulti m) {
+    const int i = idx::gemm_multi_pick((int)blockIdx.x, m.first[1], m.first[2], m.count);
+    wavering_block<I32FULL>(m.g[i], (int)blockIdx.x - m.first[i], 0);
+}
+
 bool skinny_supported(const GemmArgs& a) {
     // factors that vary inside a 32 x 32 block (one scale per row or column AND K tile) and more
     // than 256 K tiles are left to the tiled kernels
@@ -244,9 +257,11 @@ bool skinny_supported(const GemmArgs& a) {
 constexpr size_t WAVERING_LDS_BYTES = (size_t)4 * WS_STAGES * WS_STAGE_BYTES;
 
 int init_skinny_kernels() {
-    static OncePerDevice once_i32, once_promote;
+    static OncePerDevice once_i32, once_promote, once_i32_multi, once_promote_multi;
     hipError_t e = raise_lds_limit(once_i32, reinterpret_cast<const void*>(gemm_i8_wavering_kernel<true>), (int)WAVERING_LDS_BYTES);
     if (e == hipSuccess) e = raise_lds_limit(once_promote, reinterpret_cast<const void*>(gemm_i8_wavering_kernel<false>), (int)WAVERING_LDS_BYTES);
+    if (e == hipSuccess) e = raise_lds_limit(once_i32_multi, reinterpret_cast<const void*>(gemm_i8_wavering_multi_kernel<true>), (int)WAVERING_LDS_BYTES);
+    if (e == hipSuccess) e = raise_lds_limit(once_promote_multi, reinterpret_cast<const void*>(gemm_i8_wavering_multi_kernel<false>), (int)WAVERING_LDS_BYTES);
     if (e != hipSuccess) return fail(TI8_ERR_HIP, "gemm: cannot raise the LDS limit to %zu: %s", WAVERING_LDS_BYTES, hipGetErrorString(e));
     return TI8_OK;
 }
@@ -265,6 +280,22 @@ static int launch_wavering(const GemmArgs& a, int64_t batch, bool i32_full, hipS
 
 int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t st) {
     return launch_wavering(a, batch, i32_full, st);
+}
+
+int launch_skinny_multi(GemmMulti& m, bool i32_full, hipStream_t st) {
+    if (int e = init_skinny_kernels()) return e;
+    int64_t total = 0;
+    for (int i = 0; i < m.count; ++i) {
+        m.first[i] = (int)total;
+        total += (int64_t)(m.g[i].N / 32) * (m.g[i].M / 32);
+    }
+    if (total > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "gemm: too many blocks");
+    for (int i = m.count; i <= GEMM_MULTI_MAX; ++i) m.first[i] = (int)total;
+    for (int i = m.count; i < GEMM_MULTI_MAX; ++i) m.g[i] = m.g[0];
+    const auto kernel = i32_full ? gemm_i8_wavering_multi_kernel<true> : gemm_i8_wavering_multi_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), WAVERING_LDS_BYTES, st, m);
+    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
+    return check_launch("ti8_gemm_i8_nt");
 }
 
 }  // namespace ti8

@@ -324,7 +324,16 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
         if (int e = ti8_gemm_i8_nt_multi(g, count, flags | TI8_GEMM_TOGETHER, stream)) return e;
         return L.fwd && L.a->bias ? add_bias(L.a->Y, L.a->ldy, L.a->bias, L.tokens, L.N, stream) : TI8_OK;
     }
-    for (int i = 0; i < count; ++i) {
+    int first = 0;
+    if (count == 3) {   // Y and dX have few rows both: one launch where the few-rows kernel takes them
+        ti8_gemm_problem y = g[0], dx = g[1];
+        y.M = live_rows(y.K);
+        dx.M = live_rows(dx.K);
+        bool launched = false;
+        if (int e = gemm_nt_pair(y, L.a->bias, dx, flags, &launched, stream)) return e;
+        if (launched) first = 2;
+    }
+    for (int i = first; i < count; ++i) {
         const bool token_rows = i + 1 < count || !L.bwd;     // dW, the last of a backward, has one row per output feature
         if (int e = one_gemm(g[i], token_rows ? live_rows(g[i].K) : g[i].M, L.fwd && i == 0 ? L.a->bias : nullptr, L.tokens, flags, stream)) return e;
     }
