@@ -450,7 +450,8 @@ int ti8_gemm_i8_nt_i32(const int8_t* A, int64_t bsa, int64_t lda,
  *   ti8_rmsnorm      y[r][c] = bf16(bf16(x[r][c] * rstd[r]) * w[c]), rstd[r] = 1 / sqrt(mean_c(x^2) + eps) (float [rows], written);
  *                    dim a multiple of 32 up to 8192
  *   ti8_rmsnorm_bwd  dx bf16 [rows][dim] and dw bf16 [dim] from dy, x, w and the rstd of the forward; workspace of
- *                    ti8_rmsnorm_bwd_workspace bytes (-1 for sizes it does not take)
+ *                    ti8_rmsnorm_bwd_workspace bytes (-1 for sizes it does not take), which starts with the rounded products
+ *                    bf16(dy * bf16(x rstd)) [rows][dim] that dw adds up.  dw NULL: the products only (2 * rows * dim bytes suffice)
  *   ti8_rope         q and k [tokens][heads * head_dim] rotated by the tables [seq][head_dim / 2] (position = token % seq), halves
  *                    of a head against each other; backward != 0: by the opposite angle; head_dim a multiple of 16
  *   ti8_swiglu       out = bf16(bf16(silu(gate)) * up), n elements (a multiple of 8)

@@ -42,6 +42,69 @@ def test_rmsnorm(D, dev, rows, dim):
     assert torch.equal(torch.autograd.grad(g1.float().sum(), w)[0], torch.autograd.grad(g0.float().sum(), w)[0])
 
 
+# the smallest and largest rows and row counts that the layer hands to the kernels, steps of 256 that no power of two covers
+@pytest.mark.parametrize("shape", [(8, 256), (9, 4096), (3, 5, 768), (16, 2816), (2, 1000, 1024), (1025, 3840), (4097, 512)])
+def test_rmsnorm_bits(D, dev, shape):
+    gen = torch.Generator(device=dev).manual_seed(sum(shape))
+    rand = lambda *s: torch.randn(*s, generator=gen, device=dev).to(torch.bfloat16)
+    x, dy = rand(*shape).requires_grad_(True), rand(*shape)
+    norms = [D.RMSNorm(shape[-1], device=dev, fused=fused) for fused in (True, False)]
+    with torch.no_grad():
+        norms[0].weight.add_(0.1 * rand(shape[-1]))
+        norms[1].weight.copy_(norms[0].weight)
+    outs = [n(x) for n in norms]
+    assert [type(y.grad_fn).__name__ == "_RMSNormFunctionBackward" for y in outs] == [True, False]
+    for got, want in zip(*((y.detach(), *torch.autograd.grad(y, (x, n.weight), dy)) for y, n in zip(outs, norms))):
+        assert torch.equal(got, want)
+
+
+@pytest.mark.parametrize("shape", [(7, 1024), (1, 256), (64, 640), (16, 8192)])
+def test_rmsnorm_sizes_left_to_the_expression(D, dev, shape):
+    x = torch.randn(*shape, generator=torch.Generator(device=dev).manual_seed(1), device=dev).to(torch.bfloat16).requires_grad_(True)
+    got, want = (D.RMSNorm(shape[-1], device=dev, fused=fused)(x) for fused in (True, False))
+    assert torch.equal(got, want) and type(got.grad_fn) is type(want.grad_fn)
+
+
+def test_rmsnorm_backward_in_a_graph(D, dev):
+    gen = torch.Generator(device=dev).manual_seed(3)
+    rand = lambda *s: torch.randn(*s, generator=gen, device=dev).to(torch.bfloat16)
+    x, w, dy = rand(4096, 512), 1 + 0.1 * rand(512), rand(4096, 512)
+    _, rstd = D.ops.rmsnorm(x, w, 1e-5)
+    D.ops.rmsnorm_backward(dy, x, w, rstd)
+    torch.cuda.synchronize()
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph):
+        got = D.ops.rmsnorm_backward(dy, x, w, rstd)
+    for _ in range(4):
+        dy.copy_(rand(4096, 512))
+        graph.replay()
+        dx, dw = D.ops.rmsnorm_backward(dy, x, w, rstd)
+        assert torch.equal(got[0], dx)
+        # the same products in another order: (rows + 1) roundings of 2^-24 of their magnitudes, and one to bf16 either side
+        mag = (dy.double() * x.double() * rstd.double()[:, None]).abs().sum(0)
+        assert bool(((got[1].double() - dw.double()).abs() <= 2.0 ** -8 * dw.double().abs() + 4097 * 2.0 ** -23 * mag).all())
+        torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("batch,seq,hidden,heads,mlp", [(2, 40, 512, 8, 1024), (1, 648, 1024, 8, 2816), (2, 512, 2048, 16, 5504)])
+def test_decoder_layer_bits(D, dev, monkeypatch, batch, seq, hidden, heads, mlp):
+    """Output and every gradient of the layer with its kernels and with the torch expressions in their place."""
+    gen = torch.Generator(device=dev).manual_seed(seq)
+    layer = D.DecoderLayer(hidden, heads, mlp, device=dev)
+    x = torch.randn(batch, seq, hidden, generator=gen, device=dev).to(torch.bfloat16).requires_grad_(True)
+    dy = (1e-3 * torch.randn(batch, seq, hidden, generator=gen, device=dev)).to(torch.bfloat16)
+    wanted = [x, *layer.parameters()]
+
+    def outputs():
+        y = layer(x)
+        return [y.detach(), *torch.autograd.grad(y, wanted, dy)]
+    got = outputs()
+    monkeypatch.setattr(D, "_kernels_take", lambda *tensors: False)
+    names = ["y", "x", *(n for n, _ in layer.named_parameters())]
+    for name, a, b in zip(names, got, outputs()):
+        assert torch.equal(a, b), name
+
+
 @pytest.mark.parametrize("batch,seq,heads,dim", [(1, 1, 1, 16), (2, 5, 3, 48), (3, 128, 8, 64), (1, 77, 32, 128), (2, 9, 40, 256)])
 def test_rope_bits(D, dev, batch, seq, heads, dim):
     gen = torch.Generator(device=dev).manual_seed(seq)

@@ -3,8 +3,8 @@
 //
 // All are bound by HBM.  Written as torch expressions they are 60 launches that carry every intermediate through memory, the
 // RMSNorm's in fp32: 6.0 ms of a 28 ms layer step (4 x 4096 tokens, hidden 4096, MLP 14336).  Here a tensor is read once and
-// a result written once.  Intermediates that the expressions round to bf16 are rounded to bf16 here too (in registers), so
-// that the rotary embedding and the SwiGLU product give the bits of the expressions; sums run in fp32.
+// a result written once.  Intermediates that the expressions round to bf16 are rounded to bf16 here too (in registers) and rows
+// are added up in their order, so that the layer's output and gradients have the bits of the expressions.
 #include <type_traits>
 #include "ti8_common.h"
 
@@ -13,12 +13,8 @@ namespace ti8 {
 namespace {
 
 constexpr int THREADS = 256;
-constexpr int NORM_MAX_CHUNKS = 4;                          // 16-byte chunks per thread: rows of up to 8192 elements in registers
-constexpr int NORM_MAX_DIM = THREADS * 8 * NORM_MAX_CHUNKS;
-// Workgroups of the RMSNorm backward; each owns every GROUPS-th row and keeps its share of the weight gradient in registers.
-// 1024 = 4 workgroups on each CU (16 waves cover the latency of a row's loads), and the fp32 partial sums they leave
-// (GROUPS x dim) are read back in 3 % of the time of the pass at 16384 rows.
-constexpr int NORM_BWD_GROUPS = 1024;
+constexpr int NORM_STEP = 2048;                 // RMSNorm: elements of a row per 8 loads of 4 elements that a wave's lanes make
+constexpr int NORM_MAX_DIM = 4 * NORM_STEP;     // rows that fit a wave's registers
 
 __device__ __forceinline__ void unpack8(const uint4& v, float* f) {
     f[0] = bf16_lo(v.x); f[1] = bf16_hi(v.x); f[2] = bf16_lo(v.y); f[3] = bf16_hi(v.y);
@@ -33,19 +29,19 @@ __device__ __forceinline__ void round8(float* f) {
     unpack8(v, f);
 }
 
-// sum over the workgroup, in every thread; `red` holds one word per wave.  Two calls in a row need two different `red`.
-__device__ __forceinline__ float block_sum_256(float v, float* red) {
+// Sum over a row that a wave holds 4 elements per lane and step, s[e] the lane's sum over its elements e of every step; in every lane.
+// The order is that in which torch adds up an fp32 row of up to 4096 elements (lane l: elements 4 l .. 4 l + 3 of every 256, each
+// position on its own; then the four, then neighbouring lanes).
+__device__ __forceinline__ float row_sum(const float (&s)[4]) {
+    float sum = ((s[0] + s[1]) + s[2]) + s[3];
 #pragma unroll
-    for (int m = 32; m; m >>= 1) v += __shfl_xor(v, m, 64);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-    __syncthreads();
-    return (red[0] + red[1]) + (red[2] + red[3]);
+    for (int m = 1; m < 64; m <<= 1) sum += __shfl_xor(sum, m, 64);
+    return sum;
 }
 
 // y = bf16(x * rstd) * w, rstd = 1 / sqrt(mean(x^2) + eps); one wave per row, the row in registers, 4 elements per lane and load.
-// The squares are added up in the order in which torch's mean over a row of up to 4096 elements adds them (lane l: elements 4 l ..
-// 4 l + 3 of every 256, each position on its own; then the four, then neighbouring lanes): rstd, and with it y, has the bits of
-// the torch expression.  A difference in its last bit would move int8 codes behind it, which the layers that follow spread.
+// The squares are added up in torch's order (row_sum): rstd, and with it y, has the bits of the torch expression.  A difference in
+// its last bit would move int8 codes behind it, which the layers that follow spread.
 // 16384 x 4096: 56 us (4.8 TB/s; 46 us with 16-byte loads and a workgroup per row, in another order) against about 320 us for the
 // seven launches of the expression.
 template <int NV>
@@ -70,9 +66,7 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_kernel(const uint16_t* __rest
 #pragma unroll
         for (int e = 0; e < 4; ++e) s[e] += f[e] * f[e];
     }
-    float sum = ((s[0] + s[1]) + s[2]) + s[3];
-#pragma unroll
-    for (int m = 1; m < 64; m <<= 1) sum += __shfl_xor(sum, m, 64);
+    const float sum = row_sum(s);
     const float r = (float)(1.0 / sqrt((double)(sum * (1.0f / (float)dim) + eps)));   // rounded once; v_rsq_f32 is off by one bit in 7 % of the rows
     if (lane == 0) rstd[row] = r;
     uint2* yr = reinterpret_cast<uint2*>(y + row * dim);
@@ -87,82 +81,62 @@ __global__ __launch_bounds__(THREADS) void rmsnorm_kernel(const uint16_t* __rest
     }
 }
 
-// 16384 x 4096: 70 us (5.8 TB/s) + 6 us for the partial sums, against about 640 us of launches.
-// dx = rstd * (dn - x * rstd^2 * mean(dn x)) with dn = bf16(dy w); partial[g] = sum over the rows of workgroup g of dy * bf16(x rstd)
+// dx = g rstd + k (2 x) with g = bf16(dy w) and k = -1/2 (sum of g x) rstd^3 / dim, and the products bf16(dy * bf16(x rstd)) whose
+// column sums are the weight's gradient: what autograd makes of the expression, rounding by rounding and with the row's sum in torch's
+// order (row_sum), so that dx and the products have its bits.  dx goes on into the attention's gradients and the int8 codes behind
+// them: summed in another order, dQ and dK came out up to 3.6e-3 away (16384 x 4096).
+// The products go through memory because a sum of them in this kernel would be a sum in another order.  One wave per row, the row in
+// registers as in the forward.  16384 x 4096: 86 us (6.2 TB/s), and 39 us for torch's sum of the products; the sums in registers with
+// 16-byte loads and a workgroup per row took 76 us in all, the launches of the expression about 640.
 template <int NV>
 __global__ __launch_bounds__(THREADS) void rmsnorm_bwd_kernel(const uint16_t* __restrict__ dy, const uint16_t* __restrict__ x, const uint16_t* __restrict__ w,
-                                                              const float* __restrict__ rstd, uint16_t* __restrict__ dx, float* __restrict__ partial,
+                                                              const float* __restrict__ rstd, uint16_t* __restrict__ dx, uint16_t* __restrict__ prod,
                                                               int64_t rows, int dim) {
-    __shared__ float red[2][4];
-    const int nchunk = dim >> 3;
-    const uint4* wr = reinterpret_cast<const uint4*>(w);
-    uint4 wv[NV];
-    float dw[NV][8];
+    const int lane = threadIdx.x & 63;
+    const int64_t row = (int64_t)blockIdx.x * (THREADS / 64) + (threadIdx.x >> 6);
+    if (row >= rows) return;
+    const int nchunk = dim >> 2;
+    const uint2* xr = reinterpret_cast<const uint2*>(x + row * dim);
+    const uint2* dr = reinterpret_cast<const uint2*>(dy + row * dim);
+    const uint2* wr = reinterpret_cast<const uint2*>(w);
+    uint2* pr = reinterpret_cast<uint2*>(prod + row * dim);
+    const float r = rstd[row];
+    uint2 xv[NV], g[NV];
 #pragma unroll
     for (int i = 0; i < NV; ++i) {
-        const int c = threadIdx.x + i * THREADS;
-        wv[i] = c < nchunk ? wr[c] : make_uint4(0, 0, 0, 0);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) dw[i][e] = 0.0f;
-    }
-    const float inv_dim = 1.0f / (float)dim;
-    int turn = 0;
-    for (int64_t row = blockIdx.x; row < rows; row += gridDim.x, turn ^= 1) {
-        const uint4* xr = reinterpret_cast<const uint4*>(x + row * dim);
-        const uint4* dr = reinterpret_cast<const uint4*>(dy + row * dim);
-        const float r = rstd[row];
-        uint4 xv[NV], dv[NV];
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int c = threadIdx.x + i * THREADS;
-            xv[i] = dv[i] = make_uint4(0, 0, 0, 0);
-            if (c < nchunk) {
-                xv[i] = xr[c];
-                dv[i] = dr[c];
-            }
-        }
-        float dot = 0.0f;
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            float xf[8], df[8], wf[8], n[8];
-            unpack8(xv[i], xf);
-            unpack8(dv[i], df);
-            unpack8(wv[i], wf);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) n[e] = xf[e] * r;
-            round8(n);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                dw[i][e] = __builtin_fmaf(df[e], n[e], dw[i][e]);
-                df[e] = df[e] * wf[e];
-            }
-            dv[i] = pack8(df);
-            unpack8(dv[i], df);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) dot = __builtin_fmaf(df[e], xf[e], dot);
-        }
-        // the two reduction buffers alternate: a wave may write this row's while another still reads the last row's
-        const float k = block_sum_256(dot, red[turn]) * inv_dim * r * r;
-        uint4* out = reinterpret_cast<uint4*>(dx + row * dim);
-#pragma unroll
-        for (int i = 0; i < NV; ++i) {
-            const int c = threadIdx.x + i * THREADS;
-            float xf[8], df[8];
-            unpack8(xv[i], xf);
-            unpack8(dv[i], df);
-#pragma unroll
-            for (int e = 0; e < 8; ++e) df[e] = r * __builtin_fmaf(-k, xf[e], df[e]);
-            if (c < nchunk) out[c] = pack8(df);
-        }
-    }
-    float* p = partial + (int64_t)blockIdx.x * dim;
-#pragma unroll
-    for (int i = 0; i < NV; ++i) {
-        const int c = threadIdx.x + i * THREADS;
+        const int c = lane + i * 64;
+        xv[i] = g[i] = make_uint2(0, 0);
         if (c < nchunk) {
-            *reinterpret_cast<float4*>(p + c * 8) = make_float4(dw[i][0], dw[i][1], dw[i][2], dw[i][3]);
-            *reinterpret_cast<float4*>(p + c * 8 + 4) = make_float4(dw[i][4], dw[i][5], dw[i][6], dw[i][7]);
+            xv[i] = xr[c];
+            g[i] = dr[c];
         }
+    }
+    float s[4] = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = lane + i * 64;
+        if (c < nchunk) {
+            const uint2 wv = wr[c];
+            const uint32_t n0 = pack_bf16x2(bf16_lo(xv[i].x) * r, bf16_hi(xv[i].x) * r), n1 = pack_bf16x2(bf16_lo(xv[i].y) * r, bf16_hi(xv[i].y) * r);
+            pr[c] = make_uint2(pack_bf16x2(bf16_lo(g[i].x) * bf16_lo(n0), bf16_hi(g[i].x) * bf16_hi(n0)),
+                               pack_bf16x2(bf16_lo(g[i].y) * bf16_lo(n1), bf16_hi(g[i].y) * bf16_hi(n1)));
+            g[i] = make_uint2(pack_bf16x2(bf16_lo(g[i].x) * bf16_lo(wv.x), bf16_hi(g[i].x) * bf16_hi(wv.x)),
+                              pack_bf16x2(bf16_lo(g[i].y) * bf16_lo(wv.y), bf16_hi(g[i].y) * bf16_hi(wv.y)));
+            s[0] += bf16_lo(g[i].x) * bf16_lo(xv[i].x);
+            s[1] += bf16_hi(g[i].x) * bf16_hi(xv[i].x);
+            s[2] += bf16_lo(g[i].y) * bf16_lo(xv[i].y);
+            s[3] += bf16_hi(g[i].y) * bf16_hi(xv[i].y);
+        }
+    }
+    const float k = ((-0.5f * row_sum(s)) * ((r * r) * r)) * (1.0f / (float)dim);
+    uint2* out = reinterpret_cast<uint2*>(dx + row * dim);
+    const auto grad = [&](float gf, float xf) { return gf * r + k * (2.0f * xf); };
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        const int c = lane + i * 64;
+        if (c < nchunk)
+            out[c] = make_uint2(pack_bf16x2(grad(bf16_lo(g[i].x), bf16_lo(xv[i].x)), grad(bf16_hi(g[i].x), bf16_hi(xv[i].x))),
+                                pack_bf16x2(grad(bf16_lo(g[i].y), bf16_lo(xv[i].y)), grad(bf16_hi(g[i].y), bf16_hi(xv[i].y))));
     }
 }
 
@@ -283,12 +257,12 @@ int check_norm(const char* fn, int64_t rows, int64_t dim) {
     return TI8_OK;
 }
 
+// f(loads per lane of a row of `dim` elements)
 template <class F>
 void with_chunks(int64_t dim, F f) {
-    const int nv = (int)((dim + THREADS * 8 - 1) / (THREADS * 8));
-    if (nv == 1) f(std::integral_constant<int, 1>{});
-    else if (nv == 2) f(std::integral_constant<int, 2>{});
-    else f(std::integral_constant<int, 4>{});
+    if (dim <= NORM_STEP) f(std::integral_constant<int, 8>{});
+    else if (dim <= 2 * NORM_STEP) f(std::integral_constant<int, 16>{});
+    else f(std::integral_constant<int, 32>{});
 }
 
 }  // namespace
@@ -306,35 +280,36 @@ extern "C" int ti8_rmsnorm(const void* x, const void* w, void* y, float* rstd, i
     if (!x || !w || !y || !rstd) return fail(TI8_ERR_NULL, "%s: x, w, y and rstd are required", fn);
     if (int e = check_norm(fn, rows, dim)) return e;
     if (!aligned16(x) || !aligned16(w) || !aligned16(y)) return fail(TI8_ERR_ALIGN, "%s: x, w and y must be 16-byte aligned", fn);
-    // a row's 4-element chunks per lane: 8 per step of the backward's, which has 256 threads with 8 elements each
     with_chunks(dim, [&](auto nv) {
-        hipLaunchKernelGGL((rmsnorm_kernel<8 * decltype(nv)::value>), dim3((unsigned)((rows + 3) / 4)), dim3(THREADS), 0, static_cast<hipStream_t>(stream),
+        hipLaunchKernelGGL((rmsnorm_kernel<decltype(nv)::value>), dim3((unsigned)((rows + 3) / 4)), dim3(THREADS), 0, static_cast<hipStream_t>(stream),
                            static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), static_cast<uint16_t*>(y), rstd, rows, (int)dim, eps);
     });
     return check_launch(fn);
 }
 
+// the products, then the partial sums of their column sums
+static int64_t norm_products_bytes(int64_t rows, int64_t dim) { return (rows * dim * 2 + 255) / 256 * 256; }
+
 extern "C" int64_t ti8_rmsnorm_bwd_workspace(int64_t rows, int64_t dim) {
     if (check_norm("ti8_rmsnorm_bwd_workspace", rows, dim)) return -1;
-    return (rows < NORM_BWD_GROUPS ? rows : NORM_BWD_GROUPS) * dim * (int64_t)sizeof(float);
+    const int64_t sums = ti8_column_sum_workspace(rows, dim);
+    return sums < 0 ? -1 : norm_products_bytes(rows, dim) + sums;
 }
 
 extern "C" int ti8_rmsnorm_bwd(const void* dy, const void* x, const void* w, const float* rstd, void* dx, void* dw, void* workspace, int64_t rows,
                                int64_t dim, ti8_stream_t stream) {
     const char* fn = "ti8_rmsnorm_bwd";
-    if (!dy || !x || !w || !rstd || !dx || !dw || !workspace) return fail(TI8_ERR_NULL, "%s: dy, x, w, rstd, dx, dw and workspace are required", fn);
+    if (!dy || !x || !w || !rstd || !dx || !workspace) return fail(TI8_ERR_NULL, "%s: dy, x, w, rstd, dx and workspace are required", fn);
     if (int e = check_norm(fn, rows, dim)) return e;
     if (!aligned16(dy) || !aligned16(x) || !aligned16(w) || !aligned16(dx) || !aligned16(dw) || !aligned16(workspace))
         return fail(TI8_ERR_ALIGN, "%s: dy, x, w, dx, dw and workspace must be 16-byte aligned", fn);
-    const int groups = (int)(rows < NORM_BWD_GROUPS ? rows : NORM_BWD_GROUPS);
-    const hipStream_t st = static_cast<hipStream_t>(stream);
-    float* const partial = static_cast<float*>(workspace);
     with_chunks(dim, [&](auto nv) {
-        hipLaunchKernelGGL((rmsnorm_bwd_kernel<decltype(nv)::value>), dim3((unsigned)groups), dim3(THREADS), 0, st, static_cast<const uint16_t*>(dy),
-                           static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), rstd, static_cast<uint16_t*>(dx), partial, rows, (int)dim);
+        hipLaunchKernelGGL((rmsnorm_bwd_kernel<decltype(nv)::value>), dim3((unsigned)((rows + 3) / 4)), dim3(THREADS), 0, static_cast<hipStream_t>(stream),
+                           static_cast<const uint16_t*>(dy), static_cast<const uint16_t*>(x), static_cast<const uint16_t*>(w), rstd, static_cast<uint16_t*>(dx),
+                           static_cast<uint16_t*>(workspace), rows, (int)dim);
     });
     if (int e = check_launch(fn)) return e;
-    return sum_partials(fn, partial, groups, dim, dw, st);
+    return dw ? ti8_column_sum(workspace, dim, dw, static_cast<char*>(workspace) + norm_products_bytes(rows, dim), rows, dim, stream) : TI8_OK;
 }
 
 extern "C" int ti8_rope(const void* q, const void* k, void* out_q, void* out_k, const void* cos_table, const void* sin_table, int64_t tokens, int64_t seq,

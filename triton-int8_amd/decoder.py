@@ -124,8 +124,10 @@ class RMSNorm(torch.nn.Module):
         self.fused = fused
 
     def forward(self, x):
-        # rows that stay in a workgroup's registers
-        if self.fused and self.weight.numel() <= 8192 and self.weight.numel() % 32 == 0 and x.shape[-1] == self.weight.numel() and _kernels_take(x, self.weight):
+        # rows that the kernels add up in the order of torch's sum over the last dim, so that results and gradients have the bits of the
+        # expression (fewer than 8 rows, or longer ones, torch splits over more threads)
+        dim = self.weight.numel()
+        if self.fused and dim <= 4096 and dim % 256 == 0 and x.shape[-1] == dim and x.numel() >= 8 * dim and _kernels_take(x, self.weight):
             return _RMSNormFunction.apply(x, self.weight, self.eps)
         return _rmsnorm(x, self.weight, self.eps)
 

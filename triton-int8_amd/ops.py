@@ -586,11 +586,18 @@ def rmsnorm(x, weight, eps):
 
 
 def rmsnorm_backward(dy, x, weight, rstd):
-    dx, dw = torch.empty_like(x), torch.empty_like(weight)
+    """dx and the weight's gradient with the bits that autograd gives for the torch expression."""
+    dx = torch.empty_like(x)
     rows, dim = rstd.numel(), x.shape[-1]
+    args = dy.data_ptr(), x.data_ptr(), weight.data_ptr(), rstd.data_ptr(), dx.data_ptr()
+    if not torch.cuda.is_current_stream_capturing():
+        products = torch.empty_like(x)
+        _lib.call("ti8_rmsnorm_bwd", *args, None, products.data_ptr(), rows, dim, _stream())
+        return dx, products.sum(dim=tuple(range(x.dim() - 1)))
+    # torch's sum over many rows clears its counters by memset nodes, which a replayed graph must not hold: summed in another order
+    dw = torch.empty_like(weight)
     workspace = torch.empty((_lib.lib().ti8_rmsnorm_bwd_workspace(rows, dim),), dtype=torch.uint8, device=x.device)
-    _lib.call("ti8_rmsnorm_bwd", dy.data_ptr(), x.data_ptr(), weight.data_ptr(), rstd.data_ptr(), dx.data_ptr(), dw.data_ptr(), workspace.data_ptr(),
-              rows, dim, _stream())
+    _lib.call("ti8_rmsnorm_bwd", *args, dw.data_ptr(), workspace.data_ptr(), rows, dim, _stream())
     return dx, dw
 
 
