@@ -426,7 +426,8 @@ class Int8Linear(torch.nn.Module):
         if _from_c():
             if x2.shape[1] != self.in_features:
                 raise ValueError(f"expected {self.in_features} input features, got {x2.shape[1]}")
-            inside = _in_the_call(self.bias, self.out_features)
+            # a bias that wants its gradient is added by torch, which autograd sees
+            inside = _in_the_call(self.bias, self.out_features) and not (torch.is_grad_enabled() and self.bias.requires_grad)
             y = ops.linear_call(PART_FORWARD, self.scheme, self.hadamard, tokens, self.in_features, self.out_features, X=x2, wq=self._wq,
                                 bias=self.bias if inside else None)[0]
         else:
