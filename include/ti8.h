@@ -97,7 +97,7 @@ enum ti8_gemm_flags {
     TI8_GEMM_ONE_TILE = 16,   /* one workgroup per output tile also where the block-channel promotion would run on
                                  persistent workgroups (one per CU walking its tiles); same bits either way */
     TI8_GEMM_TOGETHER = 32,   /* ti8_gemm_i8_nt_multi: choose the kernels for the launch as a whole, not as each GEMM's shape
-                                 alone would; the promoted sums may then associate differently from a separate call's */
+                                 alone would (same bits: the LDS-tiled kernels all add up the K tiles in order) */
     TI8_GEMM_SKINNY = 4   /* take the few-rows kernel (no LDS staging, K split over waves) whenever
                              it supports the scale modes; by default it is used for M <= 256.  Both
                              kernels give bit-identical results with acc_i32_full; otherwise their
@@ -130,7 +130,7 @@ enum ti8_gemm_kernel {
     TI8_KERNEL_ONE_TILE_MULTI = 2,    /* the same, several GEMMs in one launch */
     TI8_KERNEL_PERSISTENT_CHAIN = 3,  /* persistent workgroups, chained block-channel promotion (256 x 256 tiles) */
     TI8_KERNEL_FEW_ROWS = 4,          /* M <= 256: 32 x 32 blocks, K split over the waves */
-    TI8_KERNEL_MID = 5                /* 128 x 128 tiles, two K tiles at a time on two groups of four waves */
+    TI8_KERNEL_MID = 5                /* 128 x 128 tiles on two groups of four waves, half a K tile apart */
 };
 #define TI8_KERNEL_KIND(id) ((id) & 0xff)
 int ti8_last_gemm_kernel(void);

@@ -1,4 +1,4 @@
-"""The medium-size GEMM kernel (gemm_i8_mid_kernel: 128 x 128 tiles, the K tiles of either parity on a group of four waves)
+"""The medium-size GEMM kernel (gemm_i8_mid_kernel: 128 x 128 tiles on two groups of four waves, half a K tile apart)
 against the oracle: int32 path bit for bit, promotion per element within the bar of an fp32 sum in another order
 (``assert_promoted_close``), over NaN-filled outputs."""
 import pytest
@@ -81,3 +81,24 @@ def test_step_whose_gemms_take_different_kernels(T, dev):
         Y0, saved = T.linear.linear_forward(X, W, scheme)
         dX0, dW0 = T.linear.linear_backward(dY, X, W, scheme, None, saved)
         assert torch.equal(Y, Y0) and torch.equal(dX, dX0) and torch.equal(dW, dW0), scheme
+
+
+# 1 to 9 K tiles (the loop takes four at a time), the longest K, batches, tile counts no multiple of 8
+@pytest.mark.parametrize("M,N,K,batch", [*((256, 384, 128 * nk, 1) for nk in range(1, 10)), (128, 256, 32768, 1), (384, 1152, 1408, 3), (1024, 2048, 5632, 1)])
+def test_bits_do_not_depend_on_the_kernel(T, dev, monkeypatch, M, N, K, batch):
+    """Promoted sums on the medium-size kernel and on 256 x 256 tiles: the K tiles in the same order, so the same bits."""
+    from triton_int8_amd import ops
+    from triton_int8_amd._lib import COMBINE_DIV_PROD, KERNEL_MID, SCALE_BLOCK128, SCALE_ROW
+    g = torch.Generator(device=dev).manual_seed(M + N + K)
+    A, B = (torch.randint(-127, 128, s, generator=g, dtype=torch.int8, device=dev) for s in ((batch, M, K), (N, K)))
+    pos = lambda *shape: torch.rand(*shape, generator=g, device=dev) + 1e-2
+    sa_row, sb_row, sa_blk, sb_blk = pos(batch, M), pos(N), pos(batch, M // 128, K // 128), pos(N // 128, K // 128)
+    for sA, mA, sB, mB, kw in ((sa_blk, SCALE_BLOCK128, sb_row, SCALE_ROW, {}), (sa_blk, SCALE_BLOCK128, sb_blk, SCALE_BLOCK128, {}),
+                               (sa_row, SCALE_ROW, sb_blk, SCALE_BLOCK128, {"out_scale": 2.0 ** -7}),
+                               (sa_blk, SCALE_BLOCK128, sb_blk, SCALE_BLOCK128, {"combine": COMBINE_DIV_PROD})):
+        outs = [torch.full((batch, M, N), float("nan"), dtype=torch.bfloat16, device=dev) for _ in range(2)]
+        for path, out in zip(("tiled", "large"), outs):
+            monkeypatch.setattr(ops, "GEMM_PATH", path)
+            ops.gemm_i8_nt(A, B, sA, mA, sB, mB, out=out, **kw)
+            assert (T.last_gemm_kernel() == KERNEL_MID) == (path == "tiled")
+        assert torch.equal(*outs)

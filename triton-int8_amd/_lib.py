@@ -180,7 +180,7 @@ _KINDS = {KERNEL_NONE: "none", KERNEL_ONE_TILE: "gemm_i8_kernel (one workgroup p
           KERNEL_ONE_TILE_MULTI: "gemm_i8_multi_kernel (one workgroup per tile, several GEMMs per launch)",
           KERNEL_PERSISTENT_CHAIN: "gemm_i8_chain_kernel (persistent workgroups)",
           KERNEL_FEW_ROWS: "gemm_i8_wavering_kernel (few rows)",
-          KERNEL_MID: "gemm_i8_mid_kernel (two K tiles at a time)"}
+          KERNEL_MID: "gemm_i8_mid_kernel (two groups of waves half a K tile apart)"}
 
 
 def describe_gemm_kernel(kernel_id=None):

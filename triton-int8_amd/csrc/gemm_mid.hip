@@ -1,30 +1,29 @@
-// INT8 NT GEMM for medium sizes: 128 x 128 tiles, two K tiles at a time on two groups of four waves.
+// INT8 NT GEMM for medium sizes: 128 x 128 tiles on eight waves in two groups, half a K tile apart.
 //
 // Up to one 128 x 128 tile per CU the time of a GEMM is the time ONE workgroup takes for its K loop, and the tile on four
 // waves (gemm.hip, one wave per SIMD) spends that loop waiting: load -> barrier -> LDS read -> MFMA -> convert + fma, one
-// after the other, 1.0 us per K tile where the MFMAs take 0.22.  Here group g of a workgroup's eight waves takes the K
-// tiles of parity g, each wave a 64 x 64 quarter of the tile with its own accumulators: every SIMD holds two waves, and a K
-// tile costs no more LDS reads or convert + fma than on four waves (eight smaller quarters would read half again as much).
+// after the other, 1.0 us per K tile where the MFMAs take 0.22.  Here each of eight waves owns 32 rows x 64 columns of the
+// tile, the upper or lower block row of a 64 x 64 quarter by its group, and every SIMD holds a wave of either group.
 //
-//  * The groups run half a step apart.  Phase M: the products of a K tile whose fragments are in registers, the previous
-//    tile's second block row folded between the MFMAs of the first (8 vector instructions per MFMA), the loads of the tile
-//    after the next one per MFMA of the second.  Phase F: the next tile's fragments out of LDS, the first block row folded
-//    between the reads.  While one group is in M the other is in F, so that MFMAs, vector instructions, LDS reads and loads
-//    run at the same time; ONE barrier per phase.  (Both groups in step: 10 % slower.  Everything folded in F: 19 % slower,
-//    a single wave per SIMD issues a vector instruction every 7 cycles only, two waves one every 4.)
-//  * All fragments of a K tile are read in one phase, so its LDS buffer is free for three phases: a load has one and a half
-//    steps to land, and two K tiles per group (64 to 128 KiB per CU) are in flight.
-//  * The order inside the phases is written out between scheduling barriers: left to itself the compiler gathers the
-//    conversions in front and spills.
-//  * The sums of the two groups meet once, in LDS, behind the loop: each wave hands over one of its two block rows and
-//    finishes the other.
+//  * The groups run half a K tile apart.  Phase M: the products of a K tile whose fragments are in registers, the previous
+//    tile's second block folded between the MFMAs (4 vector instructions per MFMA; a second set of product registers lets
+//    the MFMAs of both blocks alternate), the loads of the K tile three on.  Phase F: the next tile's fragments out of LDS,
+//    the first block folded between the reads.  While one group is in M the other is in F, so that MFMAs, vector
+//    instructions, LDS reads and loads run at the same time; ONE barrier per phase.  (A single wave per SIMD issues a vector
+//    instruction every 7 cycles only, two waves one every 4.)
+//  * All fragments of a K tile are read in one phase, so a stage is free again when the second group has read it; with four
+//    stages a load has three phases and more to land, and two to three K tiles (64 to 96 KiB per CU) are in flight.
+//  * The order inside the phases is written out between scheduling barriers, and nothing branches inside a K tile: left to
+//    itself the compiler gathers the conversions in front and spills, or sinks them to the end of the loop.
 //
-// What bounds it: 64 KiB per step and CU from L2 into LDS (alone 0.66 us of the 1.15 us that a step takes with all CUs
-// busy) in the LDS that 128 KiB of fragments are read from, beside 1024 cycles of MFMA per SIMD.  1024 rows, K = 14336, N =
-// 4096: promotion 75.5 us = 1.59 POP/s (four waves: 109), int32 63.9 us (73.8); K = 4096: 28 us (33.6).
+// Every sum runs over the K tiles in order, as on the other LDS-tiled kernels, so a GEMM has the same bits on all of them:
+// which one serves it is a matter of speed alone.  (The K tiles of either parity on a group of their own, their sums added at
+// the end, read a third less from LDS and is no faster; its other association moved the gradients of a decoder layer by up to
+// 1.8e-2 through the int8 codes behind them.)
 //
-// Arithmetic: the int32 path (I32) is exact and bit-identical to the other kernels; the promotion adds the K tiles of each
-// parity in order and then the two sums (fp32 association only, no rounding more).
+// What bounds it: 32 KiB per K tile and CU from L2 into LDS, 96 KiB of fragments out of it, and 512 cycles of MFMA per SIMD
+// beside as many of convert + fma.  1024 rows, K = 14336, N = 4096: promotion 84 us = 1.43 POP/s (four waves 109; parities
+// apart 82), int32 62 us (74; 71); K = 4096: 27 / 22 us (34 / - ; 28 / 25); 2048 x 2048 x 2048: 16.2 / 13.3 (- ; 16.9 / 15.5).
 #include <type_traits>
 #include "gemm_args.h"
 
@@ -32,28 +31,27 @@ namespace ti8 {
 
 namespace {
 
-constexpr int BM = 128, BN = 128, NGROUP = 2, WN = 2, NW = 8;
-constexpr int TM = 2, TN = 2;                       // 32 x 32 blocks per wave
+constexpr int BM = 128, BN = 128, WN = 2, NW = 8;
+constexpr int TN = 2;                               // 32 x 32 blocks per wave: one block row of two
 constexpr int WCOLS = TN * 32;
-constexpr int INSTR = 4;                            // global -> LDS instructions per wave, operand and K tile (32 rows)
+constexpr int INSTR = 2;                            // global -> LDS instructions per wave, operand and K tile (16 rows)
 constexpr int A_BYTES = BM * 128;
 constexpr int STAGE_BYTES = A_BYTES + BN * 128;     // one K tile of both operands
-constexpr int GROUP_BYTES = 2 * STAGE_BYTES;        // double buffered, per group
+constexpr int STAGES = 4;
 constexpr int MAX_K_TILES = 256;
-constexpr int LDS_BYTES = NGROUP * GROUP_BYTES + MAX_K_TILES * 4;   // 128 KiB of operands, one factor per K tile
-// vmcnt(2 * INSTR): all but the youngest K tile's loads of this wave
-constexpr int WAIT_ALL_BUT_ONE_TILE = 0xf70 | (2 * INSTR);
+constexpr int LDS_BYTES = STAGES * STAGE_BYTES + MAX_K_TILES * 4;   // 128 KiB of operands, one factor per K tile
+constexpr int WAIT_ALL_BUT_ONE_TILE = 0xf70 | (2 * INSTR);     // vmcnt: all but the youngest K tile's loads of this wave
 static_assert(2 * INSTR < 16, "vmcnt[3:0]");
 constexpr int WAIT_LDS = 0xc07f;                    // lgkmcnt(0)
 constexpr int SLAB_LD = idx::EPI_SLAB_LD(WCOLS);    // words per row of a wave's 32 x 64 slab
-static_assert(NW * 32 * SLAB_LD * 4 <= NGROUP * GROUP_BYTES, "the exchange slabs lie over the operand buffers");
+static_assert(NW * 32 * SLAB_LD * 4 <= STAGES * STAGE_BYTES, "the epilogue's slabs lie over the operand buffers");
 
 }  // namespace
 
 template <bool I32>
 __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m) {
     extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
-    // layout: [group][buffer][A 16 KiB][B 16 KiB], then the factors
+    // layout: [stage][A 16 KiB][B 16 KiB], then the factors
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -64,7 +62,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m)
     const int batch = blockIdx.y;
     const idx::TileCoord tc = idx::gemm_tile_of((int)blockIdx.x - m.first[gi], g.tiles_m, g.tiles_n, idx::gemm_group_rows(BM));
     const int m0 = tc.tile_m * BM, n0 = tc.tile_n * BN;
-    const int nk = g.K >> 7;
+    const int nk = g.K >> 7, klast = (nk - 1) * 128;
 
     // ---- global -> LDS: the slab layout and swizzle of the other kernels (gemm.hip) -----------
     uint32_t voffA[2], voffB[2];
@@ -73,35 +71,21 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m)
         voffA[p] = idx::gemm_lane_offset_bytes(lane, p, (int)g.lda);
         voffB[p] = idx::gemm_lane_offset_bytes(lane, p, (int)g.ldb);
     }
-    const int8_t* const baseA = g.A + (int64_t)batch * g.bsa + (int64_t)idx::gemm_mid_first_row(m0, quarter, g.M) * g.lda;
-    const int8_t* const baseB = g.B + (int64_t)batch * g.bsb + (int64_t)idx::gemm_mid_first_row(n0, quarter, g.N) * g.ldb;
+    const int8_t* const baseA = g.A + (int64_t)batch * g.bsa + (int64_t)idx::gemm_mid_first_row(m0, wave, g.M) * g.lda;
+    const int8_t* const baseB = g.B + (int64_t)batch * g.bsb + (int64_t)idx::gemm_mid_first_row(n0, wave, g.N) * g.ldb;
     const int64_t strideA8 = 8 * g.lda, strideB8 = 8 * g.ldb;
-    int8_t* const wdst = smem + grp * GROUP_BYTES + quarter * INSTR * 1024;
-    // byte offset along K of this group's tile t; past the end (the odd group's last step when nk is odd, and the loads that
-    // run ahead) the last K tile is fetched again, into a buffer whose products are dropped or never made
-    auto k_offset = [&](int t) { return min(2 * t + grp, nk - 1) * 128; };
-    auto issue = [&](int t, int buf) {
-        issue_tile_loads<INSTR>(baseA + k_offset(t), strideA8, voffA, 0, wdst + buf * STAGE_BYTES);
-        issue_tile_loads<INSTR>(baseB + k_offset(t), strideB8, voffB, 0, wdst + buf * STAGE_BYTES + A_BYTES);
+    int8_t* const wdst = smem + wave * INSTR * 1024;
+    // instruction q (of 4) of K tile t; a tile past the end is the last one again, into a buffer whose products nobody makes
+    auto issue_one = [&](int t, int stage, int q) {
+        const int koff = idx::gemm_k_offset(t, klast);
+        if (q < INSTR) issue_tile_loads<1>(baseA + koff + q * strideA8, strideA8, voffA, q, wdst + stage * STAGE_BYTES + q * 1024);
+        else issue_tile_loads<1>(baseB + koff + (q - INSTR) * strideB8, strideB8, voffB, q - INSTR, wdst + stage * STAGE_BYTES + A_BYTES + (q - INSTR) * 1024);
     };
-    issue(0, 0);
-
-    // ---- LDS -> registers ------------------------------------------------------------------
-    const int fr_row = lane & 31, fr_half = lane >> 5;
-    const int sw = (lane & 7) ^ ((lane >> 3) & 1);
-    uint32_t abase[4], bbase[4];
-#pragma unroll
-    for (int ks = 0; ks < 4; ++ks) {
-        const int choff = ((ks * 2 + fr_half) ^ sw) * 16;
-        abase[ks] = (uint32_t)(grp * GROUP_BYTES + (wm * TM * 32 + fr_row) * 128 + choff);
-        bbase[ks] = (uint32_t)(grp * GROUP_BYTES + A_BYTES + (wn * TN * 32 + fr_row) * 128 + choff);
-        asm volatile("" : "+v"(abase[ks]), "+v"(bbase[ks]));
-    }
 
     // ---- per-K-tile factors of the promotion: f_kt = fa_kt * fb_kt (an operand scaled per row contributes its vector in the
     // epilogue instead), the same for the whole tile, through LDS
     const bool divide = !I32 && g.combine == TI8_COMBINE_DIV_PROD;
-    float* const factors = reinterpret_cast<float*>(smem + NGROUP * GROUP_BYTES);
+    float* const factors = reinterpret_cast<float*>(smem + STAGES * STAGE_BYTES);
     if (!I32 && threadIdx.x < MAX_K_TILES) {
         const int kt = min((int)threadIdx.x, nk - 1);
         float f = 1.0f;
@@ -110,135 +94,137 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m)
         if (divide) f = 1.0f / f;
         factors[threadIdx.x] = f;
     }
+#pragma unroll
+    for (int t = 0; t < 3; ++t)
+#pragma unroll
+        for (int q = 0; q < 2 * INSTR; ++q) issue_one(t, t, q);
+
+    // ---- LDS -> registers ------------------------------------------------------------------
+    // addresses of the first two stages and, 64 KiB on (past the reach of an instruction's offset), of the last two
+    const int fr_row = lane & 31, fr_half = lane >> 5;
+    const int sw = (lane & 7) ^ ((lane >> 3) & 1);
+    uint32_t abase[2][4], bbase[2][4];
+#pragma unroll
+    for (int h = 0; h < 2; ++h)
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            const int choff = ((ks * 2 + fr_half) ^ sw) * 16;
+            abase[h][ks] = (uint32_t)(2 * h * STAGE_BYTES + ((wm * 2 + grp) * 32 + fr_row) * 128 + choff);
+            bbase[h][ks] = (uint32_t)(2 * h * STAGE_BYTES + A_BYTES + (wn * TN * 32 + fr_row) * 128 + choff);
+            asm volatile("" : "+v"(abase[h][ks]), "+v"(bbase[h][ks]));
+        }
 
     const v16i vzero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    v16i acc[TM][TN];       // I32: the sums; else the products of the K tile at hand
-    float accf[I32 ? 1 : TM][I32 ? 1 : TN][16];
+    v16i acc[I32 ? 1 : 2][TN];           // I32: the sums; else the products of the last two K tiles, by parity
+    float accf[I32 ? 1 : TN][16];
 #pragma unroll
-    for (int i = 0; i < TM; ++i)
+    for (int j = 0; j < TN; ++j) acc[0][j] = acc[I32 ? 0 : 1][j] = vzero;
 #pragma unroll
-        for (int j = 0; j < TN; ++j) acc[i][j] = vzero;
+    for (int j = 0; j < (I32 ? 1 : TN); ++j)
 #pragma unroll
-    for (int i = 0; i < (I32 ? 1 : TM); ++i)
-#pragma unroll
-        for (int j = 0; j < (I32 ? 1 : TN); ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) accf[i][j][r] = 0.0f;
+        for (int r = 0; r < 16; ++r) accf[j][r] = 0.0f;
 
-    v4i fa[TM][4], fb[TN][4];
-    // instruction pair q (of 8) of a K tile's fragment reads
-    auto read_pair = [&](int buf, int q) {
-        const int ks = q >> 1, b = q & 1;
-        fa[b][ks] = *reinterpret_cast<const v4i*>(smem + abase[ks] + (buf * STAGE_BYTES + b * 4096));
-        fb[b][ks] = *reinterpret_cast<const v4i*>(smem + bbase[ks] + (buf * STAGE_BYTES + b * 4096));
+    v4i fa[4], fb[TN][4];
+    // instruction q (of 12) of a K tile's fragment reads
+    auto read_one = [&](int stage, int q) {
+        const int ks = q / 3, b = q % 3, h = stage >> 1, off = (stage & 1) * STAGE_BYTES;
+        if (b == 0) fa[ks] = *reinterpret_cast<const v4i*>(smem + abase[h][ks] + off);
+        else fb[b - 1][ks] = *reinterpret_cast<const v4i*>(smem + bbase[h][ks] + (off + (b - 1) * 4096));
     };
     // the fragments are in registers HERE: without this the optimiser may move the reads behind the wait, to where the
     // fragments are used, past the point at which their buffer is given back
     auto frags_landed = [&]() {
         __builtin_amdgcn_s_waitcnt(WAIT_LDS);
 #pragma unroll
-        for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(fa[0][ks]), "+v"(fa[1][ks]), "+v"(fb[0][ks]), "+v"(fb[1][ks])::"memory");
+        for (int ks = 0; ks < 4; ++ks) asm volatile("" : "+v"(fa[ks]), "+v"(fb[0][ks]), "+v"(fb[1][ks])::"memory");
     };
-    // MFMA q (of 8) of block row i; piece q (of 8) of folding block row i in
-    auto mfma = [&](int i, int q) {
-        const int ks = q >> 1, j = q & 1;
-        acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[i][ks], fb[j][ks], (!I32 && ks == 0) ? vzero : acc[i][j], 0, 0, 0);
+    // MFMA ks (of 4) of block j into product set p; piece q (of 8) of folding its block j in
+    auto mfma = [&](int p, int j, int ks) {
+        acc[I32 ? 0 : p][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[ks], fb[j][ks], (!I32 && ks == 0) ? vzero : acc[I32 ? 0 : p][j], 0, 0, 0);
     };
-    auto fold = [&](int i, int q, float f) {
+    auto fold = [&](int p, int j, int q, float f) {
         if (I32) return;
-        const int j = q >> 2;
 #pragma unroll
-        for (int r = (q & 3) * 4; r < (q & 3) * 4 + 4; ++r)
-            accf[I32 ? 0 : i][I32 ? 0 : j][r] = __builtin_fmaf(static_cast<float>(acc[i][j][r]), f, accf[I32 ? 0 : i][I32 ? 0 : j][r]);
+        for (int r = q * 2; r < q * 2 + 2; ++r) accf[I32 ? 0 : j][r] = __builtin_fmaf(static_cast<float>(acc[I32 ? 0 : p][j][r]), f, accf[I32 ? 0 : j][r]);
     };
-    float f_cur = 0.0f, f_next = 0.0f;      // factor of the K tile whose products are in acc; the one read last
+    float f_cur = 0.0f, f_next = 0.0f;      // factor of the K tile whose products are being folded; the one read last
     auto read_factor = [&](int t) {
-        if (!I32) f_next = factors[min(2 * t + grp, MAX_K_TILES - 1)];
+        if (!I32) f_next = factors[min(t, MAX_K_TILES - 1)];
     };
-    // phase M of K tile `t` of this group (its fragments are in registers, its LDS buffer BUF is free again): the products,
-    // the loads of tile t + 2; at the end tile t + 1 (all but the 8 youngest loads) has landed
-    auto phase_m = [&](auto buf_tag, int t) {
-        constexpr int BUF = decltype(buf_tag)::value;
-        const bool live = 2 * t + grp < nk;     // wave-uniform
-        if (!I32 || live) {                     // a promoted tile past the end is dropped by its factor instead
-#pragma unroll
-            for (int q = 0; q < 8; ++q) {
-                __builtin_amdgcn_sched_barrier(0);
-                mfma(0, q);
-                __builtin_amdgcn_sched_barrier(0);
-                fold(1, q, f_cur);
-            }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-        if (!I32) f_cur = live ? f_next : 0.0f;
-        const int8_t* const pA = baseA + k_offset(t + 2);
-        const int8_t* const pB = baseB + k_offset(t + 2);
-        int8_t* const dst = wdst + BUF * STAGE_BYTES;
+    // phase M of K tile t (its fragments are in registers): the products, the loads of tile t + 3 into the stage that both
+    // groups are past
+    auto phase_m = [&](auto stage_tag, int t) {
+        constexpr int STAGE = decltype(stage_tag)::value, P = STAGE & 1;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             __builtin_amdgcn_sched_barrier(0);
-            if (!I32 || live) mfma(1, q);
-            if (q < INSTR) issue_tile_loads<1>(pA + q * strideA8, strideA8, voffA, q, dst + q * 1024);
-            else issue_tile_loads<1>(pB + (q - INSTR) * strideB8, strideB8, voffB, q, dst + A_BYTES + (q - INSTR) * 1024);
+            mfma(P, q & 1, q >> 1);
+            __builtin_amdgcn_sched_barrier(0);
+            fold(P ^ 1, 1, q, f_cur);
+            if (q & 1) issue_one(t + 3, (STAGE + 3) % STAGES, q >> 1);
         }
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(WAIT_ALL_BUT_ONE_TILE);
+        f_cur = f_next;
     };
-    // phase F behind it: the fragments of tile t + 1 out of buffer BUF ^ 1
-    auto phase_f = [&](auto buf_tag, int t) {
-        constexpr int BUF = decltype(buf_tag)::value;
+    // phase F behind it: the fragments of tile t + 1
+    auto phase_f = [&](auto stage_tag, int t) {
+        constexpr int NEXT = (decltype(stage_tag)::value + 1) % STAGES;
         read_factor(t + 1);
 #pragma unroll
-        for (int q = 0; q < 8; ++q) {
+        for (int q = 0; q < 4; ++q) {
             __builtin_amdgcn_sched_barrier(0);
-            read_pair(BUF ^ 1, q);
+#pragma unroll
+            for (int k = 0; k < 3; ++k) read_one(NEXT, 3 * q + k);
             __builtin_amdgcn_sched_barrier(0);
-            fold(0, q, f_cur);
+            fold(decltype(stage_tag)::value & 1, 0, 2 * q, f_cur);
+            fold(decltype(stage_tag)::value & 1, 0, 2 * q + 1, f_cur);
         }
         __builtin_amdgcn_sched_barrier(0);
+        __builtin_amdgcn_s_waitcnt(WAIT_ALL_BUT_ONE_TILE);      // tile t + 2: group 0 reads it in the phase after group 1 waited here
         frags_landed();
     };
     // the barrier is written out: in front of the one it knows the compiler waits for every load in flight
     auto barrier = [&]() { asm volatile("s_barrier" ::: "memory"); };
-    using B0 = std::integral_constant<int, 0>;
-    using B1 = std::integral_constant<int, 1>;
+    auto k_tile = [&](auto stage_tag, int t) {
+        barrier();
+        phase_m(stage_tag, t);
+        barrier();
+        phase_f(stage_tag, t);
+    };
+    using S0 = std::integral_constant<int, 0>;
+    using S1 = std::integral_constant<int, 1>;
+    using S2 = std::integral_constant<int, 2>;
+    using S3 = std::integral_constant<int, 3>;
 
     // ---- K loop --------------------------------------------------------------------------------
-    const int steps = (nk + 1) >> 1;
-    __builtin_amdgcn_s_waitcnt(0);      // tile 0 and the factors
-    __syncthreads();
-    issue(1, 1);
+    __builtin_amdgcn_s_waitcnt(WAIT_LDS & WAIT_ALL_BUT_ONE_TILE);      // tiles 0 and 1 and the factors
+    barrier();
 #pragma unroll
-    for (int q = 0; q < 8; ++q) read_pair(0, q);
+    for (int q = 0; q < 12; ++q) read_one(0, q);
     read_factor(0);
     frags_landed();
-    if (grp == 1) barrier();            // half a step behind group 0 from here on
+    if (grp == 1) barrier();            // half a K tile behind group 0 from here on
     int t = 0;
-    for (; t + 1 < steps; t += 2) {     // (one exit at the end: with a second one in the middle the accumulators are copied)
-        barrier();
-        phase_m(B0{}, t);
-        barrier();
-        phase_f(B0{}, t);
-        barrier();
-        phase_m(B1{}, t + 1);
-        barrier();
-        phase_f(B1{}, t + 1);
+    for (; t + 4 <= nk; t += 4) {
+        k_tile(S0{}, t);
+        k_tile(S1{}, t + 1);
+        k_tile(S2{}, t + 2);
+        k_tile(S3{}, t + 3);
     }
-    if (t < steps) {
-        barrier();
-        phase_m(B0{}, t);
-        barrier();
-        phase_f(B0{}, t);
-    }
+    if (t < nk) k_tile(S0{}, t);
+    if (t + 1 < nk) k_tile(S1{}, t + 1);
+    if (t + 2 < nk) k_tile(S2{}, t + 2);
     if (grp == 0) barrier();            // both groups have met the same number of barriers
 #pragma unroll
-    for (int q = 0; q < 8; ++q) fold(1, q, f_cur);
+    for (int q = 0; q < 8; ++q) {
+        if (nk & 1) fold(0, 1, q, f_cur);
+        else fold(1, 1, q, f_cur);
+    }
 
-    // ---- epilogue: what this wave finishes is block row `grp` of its quarter, 32 rows x 64 columns, 8 columns per lane ----
-    const int e_row0 = m0 + wm * TM * 32 + grp * 32;
+    // ---- epilogue: 32 rows x 64 columns per wave, 8 columns per lane ----
+    const int e_row0 = m0 + (wm * 2 + grp) * 32;
     const int rb_col = idx::epi_col_of_lane(lane, WCOLS), rb_row = idx::epi_row_of_lane(lane, WCOLS);
     const bool row_part = I32 || g.sa.mode == TI8_SCALE_ROW, col_part = I32 || g.sb.mode == TI8_SCALE_ROW;
-    // (scale loads behind the loop: 12 registers that the loop has no room for)
     float rowm[4], coln[8];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
@@ -254,45 +240,17 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m)
     }
     uint4 bias = make_uint4(0, 0, 0, 0);
     if (g.bias) bias = *reinterpret_cast<const uint4*>(g.bias + n0 + wn * WCOLS + rb_col);
-    // every load has landed and every wave is past its last fragment read: the buffers become exchange slabs
+    // every load has landed and every wave is past its last fragment read: the buffers become the waves' slabs
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    // wave (grp, quarter) puts block row 1 - grp into its slab and adds to its block row `grp` what the partner wave put
-    // there for it
     uint32_t* const slab = reinterpret_cast<uint32_t*>(smem) + wave * (32 * SLAB_LD);
-    auto put = [&](int i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int rr = 8 * (r >> 2) + 4 * fr_half + (r & 3);
-                slab[rr * SLAB_LD + j * 32 + fr_row] = I32 ? static_cast<uint32_t>(acc[i][j][r]) : __float_as_uint(accf[I32 ? 0 : i][I32 ? 0 : j][r]);
-            }
-    };
-    if (grp == 0) put(1);
-    else put(0);
-    __syncthreads();
-    const uint32_t* const other = reinterpret_cast<const uint32_t*>(smem) + (wave ^ 4) * (32 * SLAB_LD);
-    uint32_t theirs[TN][16];
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) theirs[j][r] = other[(8 * (r >> 2) + 4 * fr_half + (r & 3)) * SLAB_LD + j * 32 + fr_row];
-    __syncthreads();
-    auto sum_into_slab = [&](int i) {
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int rr = 8 * (r >> 2) + 4 * fr_half + (r & 3);
-                uint32_t w;
-                if (I32) w = static_cast<uint32_t>(acc[i][j][r]) + theirs[j][r];
-                else w = __float_as_uint(accf[I32 ? 0 : i][I32 ? 0 : j][r] + __uint_as_float(theirs[j][r]));
-                slab[rr * SLAB_LD + j * 32 + fr_row] = w;
-            }
-    };
-    if (grp == 0) sum_into_slab(0);
-    else sum_into_slab(1);
+        for (int r = 0; r < 16; ++r) {
+            const int rr = 8 * (r >> 2) + 4 * fr_half + (r & 3);
+            slab[rr * SLAB_LD + j * 32 + fr_row] = I32 ? static_cast<uint32_t>(acc[0][j][r]) : __float_as_uint(accf[I32 ? 0 : j][r]);
+        }
     __builtin_amdgcn_s_waitcnt(WAIT_LDS);   // the wave reads back what it wrote itself
     __builtin_amdgcn_wave_barrier();
     if (e_row0 >= g.M) return;              // M is a multiple of 32: a wave's 32 rows are all inside or all outside

@@ -74,9 +74,9 @@ TI8_HD int gemm_wave_first_row(int tile_row0, int wave, int n_instr, int rows) {
     return r >= rows ? r - 128 : r;
 }
 
-// the same for the 32 rows that wave `quarter` (of four) of the medium-size kernel copies; rows is a multiple of 32, and rows
-// past the operand's last re-read its last 32
-TI8_HD int gemm_mid_first_row(int tile_row0, int quarter, int rows) { return imin(tile_row0 + quarter * 32, rows - 32); }
+// the same for the 16 rows that each wave (of eight) of the medium-size kernel copies; rows is a multiple of 32, and rows past
+// the operand's last re-read its last 16
+TI8_HD int gemm_mid_first_row(int tile_row0, int wave, int rows) { return imin(tile_row0 + wave * 16, rows - 16); }
 
 // per-lane byte offset inside the 8-row slab one global->LDS instruction copies: lane l lands at
 // byte 16 l of the 1 KiB LDS slab = (row l/8, physical chunk l%8), and fetches the logical chunk

@@ -267,7 +267,7 @@ def pad_tokens(x2, multiple=128):
 
 # Schemes whose whole step (linear_fwd_bwd with more than 256 tokens and output features) runs its three GEMMs as
 # one call (ops.gemm_i8_nt_multi): on large sizes one launch of persistent workgroups walks the tiles of all three.  The kernels are
-# chosen for the call as a whole, so a promoted sum may associate differently than in a GEMM launched alone.
+# chosen for the call as a whole; all of them give the same bits.
 ONE_LAUNCH_SCHEMES = ("block_channel", "row_block", "double_channel")
 
 

@@ -401,8 +401,7 @@ def gemm_i8_nt_multi(problems, together=False):
     """Up to 3 GEMMs ``dequant(A @ B^T)`` with A int8 [M, K] and B int8 [N, K] in ONE launch; `problems`
     is a list of dicts with the keys A, B, sA, modeA, sB, modeB and optionally acc_i32_full, combine,
     out_scale, post_scale, out (meaning as in ``gemm_i8_nt``).  Returns the bf16 outputs [M, N],
-    bit-identical to separate calls; with ``together`` the kernels are chosen for the launch as a whole, and a promoted sum may
-    associate differently."""
+    bit-identical to separate calls on the same (LDS-tiled) kernels; with ``together`` the kernels are chosen for the launch as a whole."""
     _need(1 <= len(problems) <= 3, "between 1 and 3 GEMMs")
     descs, outs, keep = (_lib.GemmProblem * len(problems))(), [], []
     for i, p in enumerate(problems):
