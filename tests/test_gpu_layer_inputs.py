@@ -45,3 +45,44 @@ def test_bias_gradient_behind_a_frozen_weight(T, dev, scheme, had, tokens, align
     with torch.no_grad():
         assert torch.equal(y, lin(x)) and not lin(x).requires_grad
     assert not lin.requires_grad_(False)(x).requires_grad
+
+
+def step_and_module(T, lin, scheme, had, x, dy, backward):
+    """What the entry points return for the tensors as they are: the one-call step, the module without autograd and with it."""
+    bias, lin.bias = lin.bias, None
+    with torch.no_grad():
+        outs = [*T.linear_fwd_bwd(x, lin.weight.detach(), dy, scheme, had), lin(x)]
+    lin.bias = bias
+    leaf = x.detach().requires_grad_(True)
+    assert leaf.stride() == x.stride() and leaf.data_ptr() == x.data_ptr()
+    y = lin(leaf)
+    return [*outs, y.detach(), *backward(y, (leaf, lin.weight, lin.bias))]
+
+
+def compare_with_dense(T, dev, scheme, had, lin, x, dy, backward):
+    dense = [torch.empty(t.shape, dtype=t.dtype, device=dev).copy_(t) for t in (x, dy)]
+    want = step_and_module(T, lin, scheme, had, *dense, lambda y, leaves: torch.autograd.grad(y, leaves, dense[1]))
+    got = step_and_module(T, lin, scheme, had, x, dy, backward)
+    for name, a, b in zip(("Y", "dX", "dW", "y without autograd", "y", "dx", "dw", "db"), got, want):
+        assert torch.isfinite(a).all() and torch.equal(a, b), name
+
+
+@pytest.mark.parametrize("tokens", [1, 5, 128, 300, 512])
+@pytest.mark.parametrize("scheme,had", MODES)
+def test_rows_broadcast_from_one(T, dev, scheme, had, tokens):
+    """One row for all tokens: the gradient that a sum over the tokens sends back, and an activation expanded over a batch."""
+    g = make_gen(tokens)
+    lin = layer(T, g, dev, scheme, had)
+    row_x, row_dy = randn_bf16(g, 7, K).to(dev), randn_bf16(g, N, std=1e-3).to(dev)
+    x, dy = row_x[3:4].expand(8 * tokens, K)[:tokens], row_dy.expand(8 * tokens, N)[:tokens]
+    assert x.stride(0) == dy.stride(0) == 0
+    compare_with_dense(T, dev, scheme, had, lin, x, dy, lambda y, leaves: torch.autograd.grad(y.sum(0), leaves, row_dy))
+
+
+@pytest.mark.parametrize("tokens", [1, 300, 512])
+@pytest.mark.parametrize("scheme,had", MODES)
+def test_rows_that_overlap(T, dev, scheme, had, tokens):
+    g = make_gen(tokens)
+    lin = layer(T, g, dev, scheme, had)
+    x, dy = randn_bf16(g, 8 * tokens + K).to(dev).as_strided((tokens, K), (8, 1)), randn_bf16(g, 8 * tokens + N, std=1e-3).to(dev).as_strided((tokens, N), (8, 1))
+    compare_with_dense(T, dev, scheme, had, lin, x, dy, lambda y, leaves: torch.autograd.grad(y, leaves, dy))

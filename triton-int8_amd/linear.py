@@ -377,12 +377,12 @@ class Int8LinearFunction(torch.autograd.Function):
         tokens = ctx.tokens
         if tokens == 0:
             return dy.new_empty((*dy.shape[:-1], x2.shape[1])), torch.zeros_like(weight), (dy.new_zeros((N,)) if ctx.has_bias else None), None, None
-        dy2 = dy.reshape(-1, N)
+        dy2 = ops.rows16(dy.reshape(-1, N))
         if isinstance(ctx.saved_q, torch.Tensor) or (ctx.saved_q is None and _from_c()):
             _, dx, dw, _ = ops.linear_call(PART_BACKWARD | (PART_KEEP if ctx.saved_q is not None else 0), ctx.scheme, ctx.hadamard,
                                            *_layer_dims(x2, weight, dy2), X=x2, W=weight, dY=dy2, saved=ctx.saved_q)
         else:
-            dyp, xp = pad_tokens(dy2.contiguous()), pad_tokens(x2)
+            dyp, xp = pad_tokens(dy2), pad_tokens(x2)
             gemms = [] if _one_launch(ctx.scheme, ctx.hadamard, xp.shape[0], N) else None
             dx, dw = linear_backward(dyp, xp, weight, ctx.scheme, ctx.hadamard, ctx.saved_q, tokens=tokens, gemms=gemms)
             if gemms:

@@ -463,9 +463,10 @@ def _gemm_flags():
     return {"tiled": GEMM_TILED, "large": GEMM_LARGE_TILES}.get(GEMM_PATH, 0) | (0 if GEMM_PERSISTENT else GEMM_ONE_TILE)
 
 
-def _rows16(t):
-    """`t` itself where the library can read its rows in place, else a contiguous copy."""
-    if t.stride(1) != 1 or t.stride(0) % 8 or t.data_ptr() % 16:
+def rows16(t):
+    """`t` itself where the library can read its rows in place, else a contiguous copy (rows that overlap, too: those of a tensor
+    expanded over its rows, as autograd sends it back through a sum, are one and the same)."""
+    if t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1] or t.data_ptr() % 16:
         t = t.contiguous()
     return t
 
@@ -505,7 +506,7 @@ def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=Non
             _check_bf16(t, name)
     dev = (X if X is not None else dY).device
     need, need_saved = _linear_sizes(tokens, K, N, scheme, hadamard, parts, wq is not None)
-    X, W, dY = (t if t is None else _rows16(t) for t in (X, W, dY))
+    X, W, dY = (t if t is None else rows16(t) for t in (X, W, dY))
     T = -(-tokens // 128) * 128
     Y = dX = dW = None
     if parts & _lib.PART_FORWARD:
@@ -533,7 +534,7 @@ def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=Non
 
 def column_sum(x):
     """``x.sum(0)`` of a bf16 matrix, added up in fp32; columns a multiple of 32."""
-    x = _rows16(x)
+    x = rows16(x)
     rows, cols = x.shape
     out = torch.empty((cols,), dtype=torch.bfloat16, device=x.device)
     workspace = torch.empty((_lib.lib().ti8_column_sum_workspace(rows, cols),), dtype=torch.uint8, device=x.device)
@@ -557,7 +558,7 @@ def linear_step(X2, W, dY2, scheme, *, tokens=None, out=None, workspace=None):
     _need(W.shape[1] == K and tuple(dY2.shape) == (rows, N), f"shapes do not fit: X {tuple(X2.shape)}, W {tuple(W.shape)}, dY {tuple(dY2.shape)}")
     T = -(-rows // 128) * 128
     need = linear_step_workspace_bytes(T, K, N, scheme)
-    X2, W, dY2 = _rows16(X2), _rows16(W), _rows16(dY2)
+    X2, W, dY2 = rows16(X2), rows16(W), rows16(dY2)
     dev = X2.device
     if out is None:
         out = (torch.empty((T, N), dtype=torch.bfloat16, device=dev), torch.empty((T, K), dtype=torch.bfloat16, device=dev),
