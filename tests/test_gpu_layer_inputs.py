@@ -86,3 +86,16 @@ def test_rows_that_overlap(T, dev, scheme, had, tokens):
     lin = layer(T, g, dev, scheme, had)
     x, dy = randn_bf16(g, 8 * tokens + K).to(dev).as_strided((tokens, K), (8, 1)), randn_bf16(g, 8 * tokens + N, std=1e-3).to(dev).as_strided((tokens, N), (8, 1))
     compare_with_dense(T, dev, scheme, had, lin, x, dy, lambda y, leaves: torch.autograd.grad(y, leaves, dy))
+
+
+@pytest.mark.parametrize("tokens", [1, 5, 128, 300])
+@pytest.mark.parametrize("scheme,had", MODES)
+def test_rows_at_odd_offsets(T, dev, scheme, had, tokens):
+    """Dense tensors that do not start on 16 bytes, and a single row out of rows whose distance is no multiple of 16 bytes."""
+    g = make_gen(tokens)
+    lin = layer(T, g, dev, scheme, had)
+    x, dy = randn_bf16(g, tokens * K + 1).to(dev)[1:].view(tokens, K), randn_bf16(g, tokens * N + 3, std=1e-3).to(dev)[3:].view(tokens, N)
+    assert x.is_contiguous() and x.data_ptr() % 16 and dy.is_contiguous() and dy.data_ptr() % 16
+    compare_with_dense(T, dev, scheme, had, lin, x, dy, lambda y, leaves: torch.autograd.grad(y, leaves, dy))
+    x, dy = randn_bf16(g, tokens, K + 4).to(dev)[:, :K], randn_bf16(g, tokens, N + 4, std=1e-3).to(dev)[:, :N]
+    compare_with_dense(T, dev, scheme, had, lin, x, dy, lambda y, leaves: torch.autograd.grad(y, leaves, dy))

@@ -464,10 +464,11 @@ def _gemm_flags():
 
 
 def rows16(t):
-    """`t` itself where the library can read its rows in place, else a contiguous copy (rows that overlap, too: those of a tensor
+    """`t` itself where the library can read its rows in place, else a dense copy (rows that overlap, too: those of a tensor
     expanded over its rows, as autograd sends it back through a sum, are one and the same)."""
     if t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1] or t.data_ptr() % 16:
-        t = t.contiguous()
+        # (contiguous() returns a dense tensor that starts at an odd offset, and a single row whatever its stride, as it is)
+        t = t.clone(memory_format=torch.contiguous_format)
     return t
 
 
