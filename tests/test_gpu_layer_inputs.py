@@ -99,3 +99,31 @@ def test_rows_at_odd_offsets(T, dev, scheme, had, tokens):
     compare_with_dense(T, dev, scheme, had, lin, x, dy, lambda y, leaves: torch.autograd.grad(y, leaves, dy))
     x, dy = randn_bf16(g, tokens, K + 4).to(dev)[:, :K], randn_bf16(g, tokens, N + 4, std=1e-3).to(dev)[:, :N]
     compare_with_dense(T, dev, scheme, had, lin, x, dy, lambda y, leaves: torch.autograd.grad(y, leaves, dy))
+
+
+@pytest.mark.parametrize("tokens", [5, 300])
+@pytest.mark.parametrize("scheme,had", MODES)
+def test_bias_of_another_type(T, dev, scheme, had, tokens):
+    """A float32 bias: the sum is made and returned in float32, with and without autograd."""
+    g = make_gen(tokens)
+    lin = layer(T, g, dev, scheme, had, bias=False)
+    x, b = randn_bf16(g, tokens, K).to(dev), torch.randn(N, generator=g).to(dev)
+    with torch.no_grad():
+        want = lin(x) + b
+    lin.bias = torch.nn.Parameter(b)
+    with torch.no_grad():
+        y = lin(x)
+        assert y.dtype == torch.float32 and torch.equal(y, want)
+    y = lin(x)
+    assert y.dtype == torch.float32 and torch.equal(y, want)
+
+
+def test_a_batch_of_biases(T, dev):
+    """vmap over the bias: one GEMM, a sum for each bias."""
+    g = make_gen(2)
+    lin = layer(T, g, dev, "block_channel", None)
+    x, biases = randn_bf16(g, 300, K).to(dev), randn_bf16(g, 3, N).to(dev)
+    with torch.no_grad():
+        got = torch.func.vmap(lambda b: torch.func.functional_call(lin, {"bias": b}, (x,)))(biases)
+        for y, b in zip(got, biases):
+            assert torch.equal(y, torch.func.functional_call(lin, {"bias": b}, (x,)))

@@ -338,9 +338,10 @@ def linear_fwd_bwd(X, W, dY, scheme="block_channel", hadamard=None, out=None, wo
 
 def _in_the_call(bias, features):
     """Whether a bias goes into the layer call: a plain, dense bf16 vector that nothing else has to see being added."""
-    return (bias is not None and type(bias) in (torch.Tensor, torch.nn.Parameter) and bias.dtype == torch.bfloat16 and bias.is_cuda and tuple(bias.shape) == (features,)
-            and bias.is_contiguous() and bias.data_ptr() % 16 == 0 and bias.device.index == torch._C._cuda_getDevice()
-            and torch.autograd.forward_ad._current_level < 0 and torch._C._functorch.peek_interpreter_stack() is None)
+    # (function transforms first: inside one a tensor may have no address)
+    return (bias is not None and torch._C._functorch.peek_interpreter_stack() is None and torch.autograd.forward_ad._current_level < 0
+            and type(bias) in (torch.Tensor, torch.nn.Parameter) and bias.dtype == torch.bfloat16 and bias.is_cuda and tuple(bias.shape) == (features,)
+            and bias.is_contiguous() and bias.data_ptr() % 16 == 0 and bias.device.index == torch._C._cuda_getDevice())
 
 
 class Int8LinearFunction(torch.autograd.Function):
@@ -367,7 +368,7 @@ class Int8LinearFunction(torch.autograd.Function):
             y, ctx.saved_q = linear_forward(pad_tokens(x2), weight, scheme, hadamard, need_backward=need_bwd, tokens=tokens)
         y = y[:tokens]
         if bias is not None:
-            y += bias       # the GEMM's own output: in place
+            y = y + bias
         return y.reshape(*x.shape[:-1], N)
 
     @staticmethod
@@ -435,7 +436,7 @@ class Int8Linear(torch.nn.Module):
             y, _ = linear_forward(pad_tokens(x2), None, self.scheme, self.hadamard, need_backward=False, wq=self._wq, tokens=tokens)
         y = y[:tokens]
         if self.bias is not None and not inside:
-            y += self.bias      # the GEMM's own output: in place
+            y = y + self.bias
         return y.reshape(*x.shape[:-1], self.out_features)
 
     def extra_repr(self):
