@@ -127,3 +127,29 @@ def test_a_batch_of_biases(T, dev):
         got = torch.func.vmap(lambda b: torch.func.functional_call(lin, {"bias": b}, (x,)))(biases)
         for y, b in zip(got, biases):
             assert torch.equal(y, torch.func.functional_call(lin, {"bias": b}, (x,)))
+
+
+@pytest.mark.parametrize("scheme", ["row_block", "double_channel"])
+def test_more_tokens_than_a_column_pass_takes(T, dev, scheme):
+    """Per-row scales: a forward quantises its rows only, and no launch of it has one workgroup row per 32 tokens (at most 65535)."""
+    g = make_gen(4)
+    tokens, k, n = 65535 * 32 + 129, 128, 128
+    lin = T.Int8Linear(k, n, scheme=scheme, device=dev)
+    x = torch.randn(tokens, k, generator=torch.Generator(device=dev).manual_seed(4), device=dev, dtype=torch.bfloat16)
+    with torch.no_grad():
+        y = lin(x)
+        for rows in (slice(0, 512), slice(tokens // 2, tokens // 2 + 512), slice(tokens - 512, tokens)):
+            assert torch.equal(y[rows], lin(x[rows]))
+
+
+def test_what_a_column_pass_does_not_take_is_refused(T, dev):
+    """The same token counts where an operand is quantised by columns."""
+    from triton_int8_amd import ops
+    from triton_int8_amd._lib import PART_BACKWARD, PART_FORWARD, PART_KEEP
+    tokens, k, n = 65535 * 32 + 1, 128, 128
+    big = torch.empty(tokens, k, device=dev, dtype=torch.bfloat16)
+    w = torch.empty(n, k, device=dev, dtype=torch.bfloat16)
+    for scheme, had, parts in (("row_block", None, PART_BACKWARD), ("row_block", 128, PART_BACKWARD), ("double_channel", None, PART_BACKWARD),
+                               ("double_channel", None, PART_FORWARD | PART_KEEP), ("row_block", 128, PART_FORWARD | PART_BACKWARD)):
+        with pytest.raises(T._lib.Ti8Error, match="too many tiles"):
+            ops.linear_call(parts, scheme, had, tokens, k, n, X=big, W=w, dY=big, one_launch=False)

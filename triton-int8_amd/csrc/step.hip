@@ -162,7 +162,10 @@ int check_pointers(const char* fn, const ti8_linear_args* a, const Layer& L) {
     const bool row_n = L.bwd && L.had && !L.block();
     if ((row_k && K > 32768) || (row_n && N > 32768) || (L.dbl() && L.had && L.bwd && L.T > 32768))
         return fail(TI8_ERR_SHAPE, "%s: per-row quantisation takes up to 32768 columns", fn);
-    if ((!L.block() && !L.had && L.T / 32 > 65535) || (!L.row_block() && N / 32 > 65535)) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
+    // an operand quantised by columns: a workgroup row per 32 rows of it (the token operands, the weight)
+    const bool tokens_by_columns = (L.row_block() && L.bwd) || (L.dbl() && !L.had && (L.bwd || shared));
+    const bool weight_by_columns = (L.fwd && shared && !L.row_block()) || (L.bwd && !shared && (L.block() || (L.dbl() && !L.had)));
+    if ((tokens_by_columns && L.T / 32 > 65535) || (weight_by_columns && N / 32 > 65535)) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
     if (a->gemm_flags & ~(TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES | TI8_GEMM_ONE_TILE)) return fail(TI8_ERR_MODE, "%s: only TI8_GEMM_TILED, TI8_GEMM_LARGE_TILES and TI8_GEMM_ONE_TILE apply here", fn);
     return TI8_OK;
 }
