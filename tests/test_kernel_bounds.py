@@ -343,6 +343,18 @@ def test_one_call_step_workspace(recorded, scheme, M, K, N):
     assert T._lib.lib().ti8_linear_fwd_bwd_workspace(M + 1, K, N, 0) == -1 and T._lib.lib().ti8_linear_fwd_bwd_workspace(M, K, N, 1) == -1
 
 
+@pytest.mark.parametrize("rows,tokens", [(100, 101), (100, 128), (128, 129), (128, 0), (5, -1)])
+def test_one_call_step_reads_no_more_rows_than_there_are(recorded, rows, tokens):
+    """`tokens` between the rows of X and dY and the multiple of 128 above them: the library would read up to `tokens` rows."""
+    T, allocs, calls = recorded
+    X, W, dY = (allocs.add(torch.empty(s, dtype=torch.bfloat16)) for s in ((rows, 256), (384, 256), (rows, 384)))
+    with pytest.raises(ValueError, match="tokens"):
+        T.ops.linear_step(X, W, dY, "block_channel", tokens=tokens)
+    assert not calls
+    T.ops.linear_step(X, W, dY, "block_channel", tokens=rows)
+    assert calls[0][1][12] == -(-rows // 128) * 128 and calls[0][1][13] == rows
+
+
 @pytest.mark.parametrize("tiles", [[512, 512, 512], [1, 1, 1], [7, 300, 2], [5], [9, 4]])
 def test_multi_launch_map(walker, tiles):
     msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)

@@ -557,6 +557,7 @@ def linear_step(X2, W, dY2, scheme, *, tokens=None, out=None, workspace=None):
     rows, K = X2.shape
     N = W.shape[0]
     _need(W.shape[1] == K and tuple(dY2.shape) == (rows, N), f"shapes do not fit: X {tuple(X2.shape)}, W {tuple(W.shape)}, dY {tuple(dY2.shape)}")
+    _need(tokens is None or 1 <= tokens <= rows, f"tokens must be between 1 and the {rows} rows of X and dY, got {tokens}")
     T = -(-rows // 128) * 128
     need = linear_step_workspace_bytes(T, K, N, scheme)
     X2, W, dY2 = rows16(X2), rows16(W), rows16(dY2)
