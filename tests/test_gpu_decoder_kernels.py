@@ -149,3 +149,37 @@ def test_calls_the_kernels_do_not_take(D, dev):
     assert torch.equal(torch.func.vmap(norm)(x[:, None]), D.RMSNorm(64, device=dev)(x[:, None]))
     with torch.autograd.forward_ad.dual_level():
         assert not D._kernels_take(torch.autograd.forward_ad.make_dual(x, x), w)
+
+
+@pytest.mark.parametrize("relayout", ["transposed", "shifted"])
+def test_saved_tensors_in_another_layout(D, dev, relayout):
+    """Hooks that hand a saved tensor back with other strides, or at an odd offset: the same values, so the same gradients."""
+    def unpack(t):
+        if relayout == "transposed":
+            return t.movedim(-1, 0).contiguous().movedim(0, -1)
+        return torch.cat((t.flatten()[:1], t.flatten()))[1:].view(t.shape)
+    gen = torch.Generator(device=dev).manual_seed(7)
+    layer = D.DecoderLayer(512, 8, 1024, device=dev)
+    x = torch.randn(2, 40, 512, generator=gen, device=dev).to(torch.bfloat16).requires_grad_(True)
+    wanted = [x, *layer.parameters()]
+    gate, up = (torch.randn(40, 256, generator=gen, device=dev).to(torch.bfloat16).requires_grad_(True) for _ in range(2))
+    q, k = (torch.randn(1, 40, 2, 64, generator=gen, device=dev).to(torch.bfloat16).requires_grad_(True) for _ in range(2))
+    w = (1 + 0.1 * torch.randn(256, generator=gen, device=dev)).to(torch.bfloat16).requires_grad_(True)
+    tables = D.rope_tables(40, 64, dev)
+    calls = [(lambda: D._RMSNormFunction.apply(gate, w, 1e-5), (gate, w)), (lambda: D._SwiGLUFunction.apply(gate, up), (gate, up)),
+             (lambda: sum(D._RopeFunction.apply(q, k, *tables)), (q, k))]
+    if relayout == "shifted":        # (torch's attention wants the last dim dense)
+        calls.append((lambda: layer(x), wanted))
+    for call, leaves in calls:
+        out = call()
+        d = (1e-2 * torch.randn(*out.shape, generator=gen, device=dev)).to(torch.bfloat16)
+        want = torch.autograd.grad(out, leaves, d)
+        with torch.autograd.graph.saved_tensors_hooks(lambda t: t, unpack):
+            got = torch.autograd.grad(call(), leaves, d)
+        for a, b in zip(got, want):
+            assert torch.equal(a, b)
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: t, lambda t: t.cpu()):
+        for call, leaves in calls[:3]:
+            out = call()
+            with pytest.raises(RuntimeError, match="expected tensors on"):
+                torch.autograd.grad(out, leaves, torch.ones_like(out))

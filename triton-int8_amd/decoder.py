@@ -57,9 +57,12 @@ def _kernels_take(*tensors):
                and t.data_ptr() % 16 == 0 and t.device.index == torch._C._cuda_getDevice() for t in tensors)
 
 
-def _dense(t):
-    """A gradient as the kernels read it."""
-    t = t.contiguous()
+def _dense(t, like, dtype=torch.bfloat16):
+    """A gradient or a saved tensor as the kernels read it, on the device of `like`.  A saved tensor comes back from a hook
+    (torch.autograd.graph.saved_tensors_hooks) in whatever layout, type and place that one gives it."""
+    if t.device != like.device:
+        raise RuntimeError(f"expected tensors on {like.device}, got one on {t.device}")
+    t = t.to(dtype).contiguous()
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 
@@ -85,7 +88,7 @@ class _RMSNormFunction(torch.autograd.Function):
         x, weight, rstd = ctx.saved_tensors
         if torch.is_grad_enabled():
             return (*_differentiable(lambda a, w: _rmsnorm(a, w, ctx.eps), (x, weight), dy), None)
-        return (*ops.rmsnorm_backward(_dense(dy), x, weight, rstd), None)
+        return (*ops.rmsnorm_backward(_dense(dy, dy), _dense(x, dy), _dense(weight, dy), _dense(rstd, dy, torch.float32)), None)
 
 
 class _RopeFunction(torch.autograd.Function):
@@ -99,7 +102,7 @@ class _RopeFunction(torch.autograd.Function):
         cos, sin = ctx.saved_tensors
         if torch.is_grad_enabled():
             return (*_rope_pair(dq, dk, cos, -sin), None, None)     # linear in q and k: the transposed rotation
-        return (*ops.rope(_dense(dq), _dense(dk), cos, sin, backward=True), None, None)
+        return (*ops.rope(*(_dense(t, dq) for t in (dq, dk, cos, sin)), backward=True), None, None)
 
 
 class _SwiGLUFunction(torch.autograd.Function):
@@ -113,7 +116,7 @@ class _SwiGLUFunction(torch.autograd.Function):
         gate, up = ctx.saved_tensors
         if torch.is_grad_enabled():
             return _differentiable(_swiglu, (gate, up), d)
-        return ops.swiglu_backward(_dense(d), gate, up)
+        return ops.swiglu_backward(*(_dense(t, d) for t in (d, gate, up)))
 
 
 class RMSNorm(torch.nn.Module):
