@@ -7,14 +7,16 @@
 //
 //  * The groups run half a K tile apart.  Phase M: the products of a K tile whose fragments are in registers, the previous
 //    tile's second block folded between the MFMAs (4 vector instructions per MFMA; a second set of product registers lets
-//    the MFMAs of both blocks alternate), the loads of the K tile three on.  Phase F: the next tile's fragments out of LDS,
-//    the first block folded between the reads.  While one group is in M the other is in F, so that MFMAs, vector
-//    instructions, LDS reads and loads run at the same time; ONE barrier per phase.  (A single wave per SIMD issues a vector
-//    instruction every 7 cycles only, two waves one every 4.)
-//  * All fragments of a K tile are read in one phase, so a stage is free again when the second group has read it; with four
-//    stages a load has three phases and more to land, and two to three K tiles (64 to 96 KiB per CU) are in flight.
-//  * The order inside the phases is written out between scheduling barriers, and nothing branches inside a K tile: left to
-//    itself the compiler gathers the conversions in front and spills, or sinks them to the end of the loop.
+//    the MFMAs of both blocks alternate).  Phase F: the next tile's fragments out of LDS, the first block folded between the
+//    reads.  While one group is in M the other is in F, so that MFMAs, vector instructions, LDS reads and loads run at the
+//    same time; ONE barrier per phase.  (A single wave per SIMD issues a vector instruction every 7 cycles only, two waves
+//    one every 4.)
+//  * All fragments of a K tile are read in one phase, so a stage is free again when the second group has read it.  Both groups
+//    fetch into it in the phase behind that, one in its M and one in its F: with four stages a load has five phases to land,
+//    and three K tiles (96 KiB per CU) are in flight.  (Both in their M: group 1 a phase later, and a tile count that spreads
+//    badly over the L2s waits: 1280 x 2944 x 8192 int32 44 us, 38 this way.)
+//  * The order inside the phases is written out between scheduling barriers, and nothing branches inside a K tile (a loop for
+//    each group): left to itself the compiler gathers the conversions in front and spills, or sinks them to the loop's end.
 //
 // Every sum runs over the K tiles in order, as on the other LDS-tiled kernels, so a GEMM has the same bits on all of them:
 // which one serves it is a matter of speed alone.  (The K tiles of either parity on a group of their own, their sums added at
@@ -22,8 +24,8 @@
 // 1.8e-2 through the int8 codes behind them.)
 //
 // What bounds it: 32 KiB per K tile and CU from L2 into LDS, 96 KiB of fragments out of it, and 512 cycles of MFMA per SIMD
-// beside as many of convert + fma.  1024 rows, K = 14336, N = 4096: promotion 84 us = 1.43 POP/s (four waves 109; parities
-// apart 82), int32 62 us (74; 71); K = 4096: 27 / 22 us (34 / - ; 28 / 25); 2048 x 2048 x 2048: 16.2 / 13.3 (- ; 16.9 / 15.5).
+// beside as many of convert + fma.  Promotion / int32, us (parities apart): 1024 rows, N = 4096, K = 14336 84 / 66 = 1.43 /
+// 1.82 POP/s (82 / 66; four waves 109 / 74), K = 4096 27 / 23 (27 / 23); 2048 x 2048 x 2048 15.8 / 13.3 (16.6 / 15.4).
 #include <type_traits>
 #include "gemm_args.h"
 
@@ -40,8 +42,8 @@ constexpr int STAGE_BYTES = A_BYTES + BN * 128;     // one K tile of both operan
 constexpr int STAGES = 4;
 constexpr int MAX_K_TILES = 256;
 constexpr int LDS_BYTES = STAGES * STAGE_BYTES + MAX_K_TILES * 4;   // 128 KiB of operands, one factor per K tile
-constexpr int WAIT_ALL_BUT_ONE_TILE = 0xf70 | (2 * INSTR);     // vmcnt: all but the youngest K tile's loads of this wave
-static_assert(2 * INSTR < 16, "vmcnt[3:0]");
+constexpr int WAIT_ALL_BUT_TWO_TILES = 0xf70 | (4 * INSTR);    // vmcnt: all but the youngest two K tiles' loads of this wave
+static_assert(4 * INSTR < 16, "vmcnt[3:0]");
 constexpr int WAIT_LDS = 0xc07f;                    // lgkmcnt(0)
 constexpr int SLAB_LD = idx::EPI_SLAB_LD(WCOLS);    // words per row of a wave's 32 x 64 slab
 static_assert(NW * 32 * SLAB_LD * 4 <= STAGES * STAGE_BYTES, "the epilogue's slabs lie over the operand buffers");
@@ -151,70 +153,83 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m)
     auto read_factor = [&](int t) {
         if (!I32) f_next = factors[min(t, MAX_K_TILES - 1)];
     };
-    // phase M of K tile t (its fragments are in registers): the products, the loads of tile t + 3 into the stage that both
-    // groups are past
-    auto phase_m = [&](auto stage_tag, int t) {
+    // Phase M of K tile t (its fragments are in registers): the products.  Phase F behind it: the fragments of tile t + 1.  Both
+    // groups fetch the same K tile at the same time, group 0 in its M and group 1 in its F, into the stage that both are past;
+    // at the end of that phase all but the youngest two tiles have landed, among them the one that group 0 reads next.
+    auto phase_m = [&](auto grp_tag, auto stage_tag, int t) {
         constexpr int STAGE = decltype(stage_tag)::value, P = STAGE & 1;
+        constexpr bool FETCH = decltype(grp_tag)::value == 0;
 #pragma unroll
         for (int q = 0; q < 8; ++q) {
             __builtin_amdgcn_sched_barrier(0);
             mfma(P, q & 1, q >> 1);
             __builtin_amdgcn_sched_barrier(0);
             fold(P ^ 1, 1, q, f_cur);
-            if (q & 1) issue_one(t + 3, (STAGE + 3) % STAGES, q >> 1);
+            if (FETCH && (q & 1)) issue_one(t + 3, (STAGE + 3) % STAGES, q >> 1);
         }
         __builtin_amdgcn_sched_barrier(0);
         f_cur = f_next;
+        if (FETCH) __builtin_amdgcn_s_waitcnt(WAIT_ALL_BUT_TWO_TILES);
     };
-    // phase F behind it: the fragments of tile t + 1
-    auto phase_f = [&](auto stage_tag, int t) {
-        constexpr int NEXT = (decltype(stage_tag)::value + 1) % STAGES;
+    auto phase_f = [&](auto grp_tag, auto stage_tag, int t) {
+        constexpr int STAGE = decltype(stage_tag)::value, P = STAGE & 1;
+        constexpr bool FETCH = decltype(grp_tag)::value == 1;
         read_factor(t + 1);
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int k = 0; k < 3; ++k) read_one(NEXT, 3 * q + k);
+            for (int k = 0; k < 3; ++k) read_one((STAGE + 1) % STAGES, 3 * q + k);
             __builtin_amdgcn_sched_barrier(0);
-            fold(decltype(stage_tag)::value & 1, 0, 2 * q, f_cur);
-            fold(decltype(stage_tag)::value & 1, 0, 2 * q + 1, f_cur);
+            if (FETCH) issue_one(t + 4, STAGE, q);
+            fold(P, 0, 2 * q, f_cur);
+            fold(P, 0, 2 * q + 1, f_cur);
         }
         __builtin_amdgcn_sched_barrier(0);
-        __builtin_amdgcn_s_waitcnt(WAIT_ALL_BUT_ONE_TILE);      // tile t + 2: group 0 reads it in the phase after group 1 waited here
+        if (FETCH) __builtin_amdgcn_s_waitcnt(WAIT_ALL_BUT_TWO_TILES);
         frags_landed();
     };
     // the barrier is written out: in front of the one it knows the compiler waits for every load in flight
     auto barrier = [&]() { asm volatile("s_barrier" ::: "memory"); };
-    auto k_tile = [&](auto stage_tag, int t) {
+    auto k_tile = [&](auto grp_tag, auto stage_tag, int t) {
         barrier();
-        phase_m(stage_tag, t);
+        phase_m(grp_tag, stage_tag, t);
         barrier();
-        phase_f(stage_tag, t);
+        phase_f(grp_tag, stage_tag, t);
     };
-    using S0 = std::integral_constant<int, 0>;
-    using S1 = std::integral_constant<int, 1>;
-    using S2 = std::integral_constant<int, 2>;
-    using S3 = std::integral_constant<int, 3>;
+    using G0 = std::integral_constant<int, 0>;
+    using G1 = std::integral_constant<int, 1>;
+    auto k_loop = [&](auto grp_tag) {
+        int t = 0;
+        for (; t + 4 <= nk; t += 4) {
+            k_tile(grp_tag, std::integral_constant<int, 0>{}, t);
+            k_tile(grp_tag, std::integral_constant<int, 1>{}, t + 1);
+            k_tile(grp_tag, std::integral_constant<int, 2>{}, t + 2);
+            k_tile(grp_tag, std::integral_constant<int, 3>{}, t + 3);
+        }
+        if (t < nk) k_tile(grp_tag, std::integral_constant<int, 0>{}, t);
+        if (t + 1 < nk) k_tile(grp_tag, std::integral_constant<int, 1>{}, t + 1);
+        if (t + 2 < nk) k_tile(grp_tag, std::integral_constant<int, 2>{}, t + 2);
+    };
 
     // ---- K loop --------------------------------------------------------------------------------
-    __builtin_amdgcn_s_waitcnt(WAIT_LDS & WAIT_ALL_BUT_ONE_TILE);      // tiles 0 and 1 and the factors
+    __builtin_amdgcn_s_waitcnt(WAIT_LDS & WAIT_ALL_BUT_TWO_TILES);      // tile 0 and the factors
     barrier();
 #pragma unroll
     for (int q = 0; q < 12; ++q) read_one(0, q);
     read_factor(0);
-    frags_landed();
-    if (grp == 1) barrier();            // half a K tile behind group 0 from here on
-    int t = 0;
-    for (; t + 4 <= nk; t += 4) {
-        k_tile(S0{}, t);
-        k_tile(S1{}, t + 1);
-        k_tile(S2{}, t + 2);
-        k_tile(S3{}, t + 3);
+    if (grp == 0) {
+        frags_landed();
+        k_loop(G0{});
+        barrier();                      // both groups have met the same number of barriers
+    } else {                            // half a K tile behind group 0
+#pragma unroll
+        for (int q = 0; q < 2 * INSTR; ++q) issue_one(3, 3, q);
+        __builtin_amdgcn_s_waitcnt(WAIT_ALL_BUT_TWO_TILES);
+        frags_landed();
+        barrier();
+        k_loop(G1{});
     }
-    if (t < nk) k_tile(S0{}, t);
-    if (t + 1 < nk) k_tile(S1{}, t + 1);
-    if (t + 2 < nk) k_tile(S2{}, t + 2);
-    if (grp == 0) barrier();            // both groups have met the same number of barriers
 #pragma unroll
     for (int q = 0; q < 8; ++q) {
         if (nk & 1) fold(0, 1, q, f_cur);
