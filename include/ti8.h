@@ -358,14 +358,15 @@ int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count, int gemm_f
  *   dX = fwd_32(dY, W^T)     the same pipeline on the transposed weight
  *   dW = bwd_33(dY^T, X^T)   int8_gemm_pipeline of triton/block_channel_bwd33.py:148-172  /  triton/double_channel_bwd33.py:186-201
  * enqueued back to back from C (the reference pays one Python-side wrapper per quantiser and per GEMM, each with
- * its own allocations).  Same kernels on the same operands as the separate entry points, so the same bits:
+ * its own allocations).  The same quantisers and GEMMs as through the separate entry points, the GEMM kernels chosen for the call
+ * as a whole (TI8_GEMM_TOGETHER), with the same bits:
  *   TI8_SCHEME_BLOCK_CHANNEL   ti8_quant_block_multi(X, dY; q and qT) -> ti8_quant_row_col_t(W) ->
  *                              ti8_gemm_i8_nt_multi(Y, dX, dW)          (3 launches + W's absmax pass)
  *   TI8_SCHEME_DOUBLE_CHANNEL  ti8_quant_row_col_t on X, W, dY (TI8_INV_AMAX_DIV_127) ->
  *                              ti8_gemm_i8_nt_multi(Y, dX, dW; acc_i32_full = 1)
  *   X bf16 [T][K] (ldx), W bf16 [N][K] (ldw), dY bf16 [T][N] (lddy)  ->  Y bf16 [T][N], dX bf16 [T][K], dW bf16 [N][K]
  *   All six 16-byte aligned, leading dimensions multiples of 8 elements; every argument is checked before the first launch.
- *   T, K, N multiples of 128.  `tokens` (T - 128 < tokens <= T) = the rows of X and dY that exist; the rest of the T rows
+ *   T, K, N multiples of 128.  `tokens` (1 <= tokens <= T) = the rows of X and dY that exist; the rest of the T rows
  *   counts as zeros and is not read (zeros change no absmax and add nothing to dW).  With
  *   T <= 256 or N <= 256 the GEMMs are launched one by one, as ti8_gemm_i8_nt would launch them (few-rows kernel up to 256
  *   rows), and Y and dX are computed for the first ceil(tokens / 32) * 32 rows only.

@@ -613,6 +613,87 @@ int walk_chain_rounds(int total, int grid, int several, int64_t* n_checked, char
     return r.bad;
 }
 
+// Medium-size kernel (gemm_mid.hip: gemm_i8_mid_kernel) on one GEMM: 128 x 128 tiles, M a multiple of 32.  Checked: every tile of every
+// batch is computed once; the loads of every K tile, those past the end included, the per-K-tile factors, the scales of the
+// epilogue, the LDS slots of loads, fragments, factors and slabs; every element of C stored once.
+int walk_gemm_mid(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t bsc, int64_t ldc, const ScaleArg* sa, const ScaleArg* sb,
+                  int64_t batch, int64_t M, int64_t N, int64_t K, int i32, int64_t a_elems, int64_t b_elems, int64_t c_elems,
+                  int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    const int STAGES = 4, OPERAND = 128 * 128, STAGE = 2 * OPERAND, FACTORS = 256, WCOLS = 64, SLAB = 32 * EPI_SLAB_LD(WCOLS);
+    const int tiles_m = (int)((M + 127) / 128), tiles_n = (int)(N / 128), nk = (int)(K >> 7), klast = (nk - 1) * 128;
+    if (nk < 1 || nk > FACTORS) r.fail("gemm mid: %d K tiles", nk);
+    std::vector<uint8_t> stored((size_t)c_elems, 0), tile_seen((size_t)tiles_m * tiles_n, 0);
+    for (int64_t by = 0; by < batch && !r.bad; ++by) {
+        std::fill(tile_seen.begin(), tile_seen.end(), 0);
+        for (int bx = 0; bx < tiles_m * tiles_n && !r.bad; ++bx) {
+            const TileCoord tc = gemm_tile_of(bx, tiles_m, tiles_n, gemm_group_rows(128));
+            if (tc.tile_m < 0 || tc.tile_m >= tiles_m || tc.tile_n < 0 || tc.tile_n >= tiles_n) {
+                r.fail("gemm mid: workgroup %d maps to tile (%d, %d) outside %d x %d", bx, tc.tile_m, tc.tile_n, tiles_m, tiles_n);
+                break;
+            }
+            ++tile_seen[(size_t)tc.tile_m * tiles_n + tc.tile_n];
+            const int m0 = tc.tile_m * 128, n0 = tc.tile_n * 128;
+            for (int thread = 0; thread < FACTORS && !i32; ++thread) {
+                const int kt = imin(thread, nk - 1);
+                if (sa->mode != 0) r.access("gemm mid factor A", gemm_factor_index(by, sa->bs, gemm_factor_block(m0, (int)M), sa->rs, kt, sa->mode == 3 ? 1 : 0, sa->ks), 1, sa->elems, bx, thread);
+                if (sb->mode != 0) r.access("gemm mid factor B", gemm_factor_index(by, sb->bs, gemm_factor_block(n0, (int)N), sb->rs, kt, sb->mode == 3 ? 1 : 0, sb->ks), 1, sb->elems, bx, thread);
+            }
+            for (int wave = 0; wave < 8; ++wave) {
+                const int grp = wave >> 2, wm = (wave & 3) / 2, wn = wave & 1;
+                const int rA0 = gemm_mid_first_row(m0, wave, (int)M), rB0 = gemm_mid_first_row(n0, wave, (int)N);
+                for (int lane = 0; lane < 64 && !r.bad; ++lane) {
+                    for (int t = 0; t < nk + 4; t = t == 4 && nk > 8 ? nk - 1 : t + 1) {     // offsets grow with t up to the clamp
+                        const int koff = gemm_k_offset(t, klast);
+                        for (int i = 0; i < 2; ++i) {
+                            r.access("gemm mid A", by * bsa + gemm_load_offset_bytes(rA0, lda, koff, i, gemm_lane_offset_bytes(lane, i & 1, (int)lda)), 16, a_elems, bx, wave, lane, t);
+                            r.access("gemm mid B", by * bsb + gemm_load_offset_bytes(rB0, ldb, koff, i, gemm_lane_offset_bytes(lane, i & 1, (int)ldb)), 16, b_elems, bx, wave, lane, t);
+                            r.access("gemm mid LDS", (t % STAGES) * STAGE + OPERAND + wave * 2048 + i * 1024 + lane * 16, 16, STAGES * STAGE, bx, wave, lane, t);
+                        }
+                    }
+                    const int fr_row = lane & 31, fr_half = lane >> 5, sw = (lane & 7) ^ ((lane >> 3) & 1);
+                    for (int ks = 0; ks < 4; ++ks) {
+                        const int choff = ((ks * 2 + fr_half) ^ sw) * 16;
+                        r.access("gemm mid fragment A", ((wm * 2 + grp) * 32 + fr_row) * 128 + choff, 16, OPERAND, bx, wave, lane, ks);
+                        for (int j = 0; j < 2; ++j) r.access("gemm mid fragment B", (wn * 64 + j * 32 + fr_row) * 128 + choff, 16, OPERAND, bx, wave, lane, ks);
+                    }
+                    const int row0 = m0 + (wm * 2 + grp) * 32, rb_col = epi_col_of_lane(lane, WCOLS), rb_row = epi_row_of_lane(lane, WCOLS);
+                    const bool row_part = i32 || sa->mode == 0, col_part = i32 || sb->mode == 0;
+                    for (int k = 0; k < 4; ++k)
+                        r.access("gemm mid row scale", epi_row_scale_base(by, sa->bs, imin(row0 + rb_row + 8 * k, (int)M - 1), row_part ? sa->rs : 0), 1, sa->elems, bx, wave, lane, k);
+                    for (int c = 0; c < 8; ++c)
+                        r.access("gemm mid column scale", epi_col_scale_index(by, sb->bs, n0 + wn * WCOLS + rb_col + c, (int)N, col_part ? sb->rs : 0), 1, sb->elems, bx, wave, lane, c);
+                    for (int e = 0; e < 16; ++e)
+                        for (int j = 0; j < 2; ++j)
+                            r.access("gemm mid slab write", (8 * (e >> 2) + 4 * fr_half + (e & 3)) * EPI_SLAB_LD(WCOLS) + j * 32 + fr_row, 1, SLAB, bx, wave, lane, e);
+                    r.access("gemm mid slabs", (int64_t)(wave + 1) * SLAB * 4 - 1, 1, STAGES * STAGE, bx, wave);
+                    if (row0 >= M) continue;
+                    for (int k = 0; k < 4; ++k) {
+                        r.access("gemm mid slab read", (rb_row + 8 * k) * EPI_SLAB_LD(WCOLS) + rb_col, 8, SLAB, bx, wave, lane, k);
+                        const int64_t off = epi_out_offset(by, bsc, row0 + rb_row, ldc, n0 + wn * WCOLS + rb_col) + (int64_t)(8 * k) * ldc;
+                        if (r.access("gemm mid C", off, 8, c_elems, bx, wave, lane, k))
+                            for (int c = 0; c < 8; ++c) ++stored[(size_t)(off + c)];
+                    }
+                }
+            }
+        }
+        for (size_t t = 0; t < tile_seen.size() && !r.bad; ++t)
+            if (tile_seen[t] != 1) r.fail("gemm mid: tile %zu of batch %lld is computed %d times", t, (long long)by, (int)tile_seen[t]);
+    }
+    int64_t total = 0;
+    for (int64_t b = 0; b < batch && !r.bad; ++b)
+        for (int64_t m = 0; m < M; ++m)
+            for (int64_t n = 0; n < N; ++n) {
+                const int times = stored[(size_t)(b * bsc + m * ldc + n)];
+                if (times != 1) r.fail("gemm mid: C[%lld][%lld][%lld] stored %d times", (long long)b, (long long)m, (long long)n, times);
+                total += times;
+            }
+    for (size_t i = 0; i < stored.size(); ++i) total -= stored[i];
+    if (!r.bad && total != 0) r.fail("gemm mid: %lld stores outside C", (long long)-total);
+    *n_checked = r.checked;
+    return r.bad;
+}
+
 // Choice of kernels for a launch of several GEMMs of shapes shape[i] = {M, N, K}: cfg[3 i ..] = bm, bn, mid of GEMM i alone, then of the
 // launch (9 values each)
 void walk_configs_together(const int64_t* shape, int count, int i32, int num_cu, int* cfg) {

@@ -25,7 +25,9 @@ def T():
     (1024, 1024, 1024, 3, "tiled"),    # complete groups of tile rows, 192 tiles over three batches
     (128, 256, 32768, 1, "tiled"),     # 256 K tiles: every factor the kernel keeps
     (224, 14336, 1024, 1, "auto"),     # rows that are no multiple of 128: the last tile re-reads its last 32 rows
-    (32, 16384, 2048, 1, "mid"),       # one block row; chosen by hand, the few-rows kernel is faster here
+    (96, 14336, 14336, 1, "auto"),     # a partial tile only, which the rule sends here for its long K
+    (64, 32768, 2048, 1, "auto"),      # the same for its many columns, every CU busy
+    (32, 16384, 2048, 1, "few"),       # what the rule leaves to the few-rows kernel must agree with the same oracle
 ])
 def test_medium_kernel(T, dev, monkeypatch, M, N, K, batch, path):
     from triton_int8_amd import ops
@@ -40,7 +42,7 @@ def test_medium_kernel(T, dev, monkeypatch, M, N, K, batch, path):
         if kt < nkb:
             sa_blk[:, :, kt] *= 37.0
     Ad, Bd = A.to(dev), B.to(dev)
-    few = path == "mid"                # `path` "mid": what the rule leaves to the few-rows kernel must at least agree
+    few = path == "few"
     monkeypatch.setattr(ops, "GEMM_PATH", "auto" if few else path)
     expected = KERNEL_FEW_ROWS if few else KERNEL_MID
 

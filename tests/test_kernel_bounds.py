@@ -44,6 +44,7 @@ def walker(tmp_path_factory):
     lib.walk_quant_block.argtypes = [i64, i64, ci, i64, i64, ci, i64, i64, i64, i64, i64, i64, i64, i64, ci, i64, i64, i64, i64, p64, cp, ci]
     lib.walk_gemm.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] * 5 + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_gemm_chain.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] + [i64] * 3 + [p64, cp, ci]
+    lib.walk_gemm_mid.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] + [i64] * 3 + [p64, cp, ci]
     lib.walk_chain_rounds.argtypes = [ci, ci, ci, p64, cp, ci]
     lib.walk_configs_together.argtypes = [p64, ci, ci, ci, ctypes.POINTER(ci)]
     lib.walk_configs_together.restype = None
@@ -382,6 +383,30 @@ def test_persistent_chain_kernel_geometries(walker, M, N, K, batch, mA, mB, grid
     rc = walker.walk_gemm_chain(M * K, K, N * K, K, M * N, N, ctypes.byref(sa), ctypes.byref(sb), batch, M, N, K, grid,
                                 batch * M * K - K, batch * N * K, batch * M * N, ctypes.byref(n), msg, 512)
     assert rc != 0 and b"gemm chain A" in msg.value
+
+
+# rows of a partial tile only, of one behind a full tile, K tiles from one on (the loads run three and four ahead), the most K tiles that
+# it keeps factors of, batches, rows of the operands further apart than K
+@pytest.mark.parametrize("M,N,K,batch,gap", [(32, 256, 128, 1, 0), (64, 128, 256, 2, 0), (96, 384, 384, 1, 16), (128, 128, 512, 3, 0), (224, 256, 640, 1, 0),
+                                             (384, 1152, 1408, 2, 0), (256, 384, 1024, 1, 128), (160, 128, 32768, 1, 0)])
+@pytest.mark.parametrize("mA,mB,i32", [(0, 0, 1), (1, 0, 0), (1, 1, 0), (0, 1, 0), (3, 1, 0)])
+def test_medium_kernel_geometries(walker, M, N, K, batch, gap, mA, mB, i32):
+    nkb, ld = K // 128, K + gap
+    mA = 1 if mA == 3 and nkb % 2 else mA       # (256-wide scale blocks need an even number of K tiles)
+
+    def desc(mode, rows, batched):
+        per = {0: rows, 1: -(-rows // 128) * nkb, 3: -(-rows // 128) * (nkb // 2)}[mode]
+        return ScaleArg(mode, per if batched else 0, {0: 1, 1: nkb, 3: nkb // 2}[mode], 0 if mode == 0 else 1, per * (batch if batched else 1))
+    sa, sb = desc(mA, M, True), desc(mB, N, False)
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    run = lambda a_rows, b_rows, c_el: walker.walk_gemm_mid(M * ld, ld, 0, ld, M * N, N, ctypes.byref(sa), ctypes.byref(sb), batch, M, N, K, i32, a_rows * ld - gap,
+                                                            b_rows * ld - gap, c_el, ctypes.byref(n), msg, 512)
+    assert run(batch * M, N, batch * M * N) == 0, msg.value.decode()
+    assert n.value > M * N // 8
+    # one row less of either operand, or of C, than the kernel assumes must be noticed
+    assert run(batch * M - 1, N, batch * M * N) != 0 and b"gemm mid A" in msg.value
+    assert run(batch * M, N - 1, batch * M * N) != 0 and b"gemm mid B" in msg.value
+    assert run(batch * M, N, batch * M * N - N) != 0 and b"gemm mid C" in msg.value
 
 
 @pytest.mark.parametrize("several", [0, 1])

@@ -307,6 +307,8 @@ TI8_HD GemmConfig gemm_config(int64_t M, int64_t N, int64_t K, int64_t batch, bo
 // launches of 2 and 3 GEMMs of 384 .. 7040 tokens and 1024 .. 14336 features: a constant, the K tiles of the busiest CU, the mean
 // over the CUs, and what a tile or a round costs besides; off by 4 % in the mean and 11 % at most (int32: 21 %, on tiles that
 // leave most CUs idle).  Against the choice by shape alone the launches take 0.93 of the time in the mean and 1.01 at worst.
+// With another number of CUs the shares per CU follow it and the constants do not: the order of the kernels is then a guess, the
+// results are the same (all of these kernels give the same bits).
 struct GemmSet {
     int64_t M[3], N[3], nk[3];   // nk (K tiles) descending: the order of the launch
     int count;

@@ -2,7 +2,7 @@
 // launch(es) of a forward, a backward or a whole step that the Python layer would otherwise issue one entry point at a time, on
 // caller-provided outputs and a caller-provided workspace.  Nothing here computes: the entry points of quant.hip, fwht.hip and
 // gemm.hip are called in the order of a step with sub-buffers of the workspace, so every tensor (int8 operands, scales, bf16
-// outputs) has the bits the separate calls give.
+// outputs) has the bits the separate calls give, also where the GEMM kernels are chosen for the call as a whole.
 #include "ti8_common.h"
 
 namespace ti8 {
