@@ -175,7 +175,7 @@ def init():
 
 
 _EPILOGUES = ("int32 out", "per-row scales, int32 over the whole K", "promotion per K tile", "literal arithmetic",
-              "promotion per K tile, per-lane factors", "chained promotion per K tile")
+              "promotion per K tile, per-lane factors", "chained promotion per K tile", "chained promotion per K tile, per-lane factors")
 _KINDS = {KERNEL_NONE: "none", KERNEL_ONE_TILE: "gemm_i8_kernel (one workgroup per tile)",
           KERNEL_ONE_TILE_MULTI: "gemm_i8_multi_kernel (one workgroup per tile, several GEMMs per launch)",
           KERNEL_PERSISTENT_CHAIN: "gemm_i8_chain_kernel (persistent workgroups)",

@@ -550,7 +550,7 @@ bool chain_persistent_supported(const GemmMulti& m) {
         if (nk < 2 || nk > 256 || (nk & 1) || m.g[i].strict) return false;
         if (m.g[i].sa.mode == TI8_SCALE_ROW_K128 || (m.g[i].sb.mode == TI8_SCALE_ROW_K128) != lane_scales(m)) return false;
         // row by row, a wave's scales lie in 32 cache lines per load and bound either kernel (4 x 8192^3, whole call: 2835 us here, 2769
-        // on one workgroup per tile); column by column 2361 against 2496 us for the GEMM
+        // on one workgroup per tile); column by column 2266 against 2382 us for the GEMM
         if (lane_scales(m) && m.g[i].sb.rs != 1) return false;
         // the epilogue stores 16 bytes per lane and row (the one-tile kernels store 8)
         if ((reinterpret_cast<uintptr_t>(m.g[i].C) & 15) || (m.g[i].ldc % 8) || (m.g[i].bsc % 8)) return false;

@@ -60,9 +60,10 @@ def _kernels_take(*tensors):
 def _dense(t, like, dtype=torch.bfloat16):
     """A gradient or a saved tensor as the kernels read it, on the device of `like`.  A saved tensor comes back from a hook
     (torch.autograd.graph.saved_tensors_hooks) in whatever layout, type and place that one gives it."""
-    if t.device != like.device:
+    if t.get_device() != like.get_device():
         raise RuntimeError(f"expected tensors on {like.device}, got one on {t.device}")
-    t = t.to(dtype).contiguous()
+    if t.dtype != dtype or not t.is_contiguous():
+        t = t.to(dtype).contiguous()
     return t if t.data_ptr() % 16 == 0 else t.clone()
 
 

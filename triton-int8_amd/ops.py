@@ -466,7 +466,8 @@ def _gemm_flags():
 def rows16(t):
     """`t` itself where the library can read its rows in place, else a dense copy (rows that overlap, too: those of a tensor
     expanded over its rows, as autograd sends it back through a sum, are one and the same)."""
-    if t.stride(1) != 1 or t.stride(0) % 8 or t.stride(0) < t.shape[1] or t.data_ptr() % 16:
+    row, element = t.stride()
+    if element != 1 or row % 8 or row < t.shape[1] or t.data_ptr() % 16:
         # (contiguous() returns a dense tensor that starts at an odd offset, and a single row whatever its stride, as it is)
         t = t.clone(memory_format=torch.contiguous_format)
     return t
