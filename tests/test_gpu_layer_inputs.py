@@ -153,3 +153,23 @@ def test_what_a_column_pass_does_not_take_is_refused(T, dev):
                                ("double_channel", None, PART_FORWARD | PART_KEEP), ("row_block", 128, PART_FORWARD | PART_BACKWARD)):
         with pytest.raises(T._lib.Ti8Error, match="too many tiles"):
             ops.linear_call(parts, scheme, had, tokens, k, n, X=big, W=w, dY=big, one_launch=False)
+
+
+@pytest.mark.parametrize("scheme,had", MODES)
+def test_a_weight_at_the_address_of_the_last(T, dev, scheme, had):
+    """Weights that come and go, each likely where the one before it lay: the quantised weight is that of the present one."""
+    import copy
+    g = make_gen(6)
+    lin = layer(T, g, dev, scheme, had, bias=False)
+    x = randn_bf16(g, 33, K).to(dev)
+    with torch.no_grad():
+        for _ in range(3):
+            lin(x)
+            lin.weight = torch.nn.Parameter(torch.empty(0, dtype=torch.bfloat16, device=dev))
+            lin.weight = torch.nn.Parameter(randn_bf16(g, N, K, std=0.02).to(dev))
+            fresh = T.Int8Linear(K, N, scheme=scheme, hadamard=had, device=dev)
+            fresh.weight.copy_(lin.weight)
+            assert torch.equal(lin(x), fresh(x))
+        other = copy.deepcopy(lin)
+        other.weight.mul_(2.0)
+        assert torch.equal(other(x), lin(x) * 2.0) and list(lin.state_dict()) == ["weight"]

@@ -400,6 +400,10 @@ class Int8Linear(torch.nn.Module):
     in_features and out_features must be multiples of 128; any number of tokens works
     (zero-padded to the 128-row tile)."""
 
+    # the weight that the forward-only path has quantised (held, because the address of one that is gone may be the next one's; in a
+    # tuple, which a module does not take for a parameter of its own)
+    _wq_of = (None,)
+
     def __init__(self, in_features, out_features, bias=False, scheme="block_channel", hadamard=None,
                  device=None, dtype=torch.bfloat16):
         super().__init__()
@@ -414,14 +418,15 @@ class Int8Linear(torch.nn.Module):
         self._wq, self._wq_key = None, None   # quantised weight of the forward-only path and what it was made from
 
     def forward(self, x):
-        if torch.is_grad_enabled() and (x.requires_grad or self.weight.requires_grad):
-            return Int8LinearFunction.apply(x, self.weight, self.bias, self.scheme, self.hadamard)
+        weight = self.weight
+        if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
+            return Int8LinearFunction.apply(x, weight, self.bias, self.scheme, self.hadamard)
         if x.numel() == 0:
             return x.new_empty((*x.shape[:-1], self.out_features))
         # forward only (inference): the weight is quantised once per weight update, not per call
-        key = (self.weight._version, self.weight.data_ptr(), self.scheme, self.hadamard)
-        if self._wq_key != key:
-            self._wq, self._wq_key = quantize_weight(self.weight.detach(), self.scheme, self.hadamard), key
+        key = (weight._version, weight.data_ptr(), self.scheme, self.hadamard)
+        if self._wq_key != key or self._wq_of[0] is not weight:
+            self._wq, self._wq_key, self._wq_of = quantize_weight(weight.detach(), self.scheme, self.hadamard), key, (weight,)
         x2 = x.reshape(-1, x.shape[-1])
         tokens = x2.shape[0]
         if _from_c():
