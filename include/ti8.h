@@ -466,6 +466,25 @@ int ti8_rope(const void* q, const void* k, void* out_q, void* out_k, const void*
 int ti8_swiglu(const void* gate, const void* up, void* out, int64_t n, ti8_stream_t stream);
 int ti8_swiglu_bwd(const void* d, const void* gate, const void* up, void* dgate, void* dup, int64_t n, ti8_stream_t stream);
 
+/* Backward of causal attention, dense bf16 tensors of `batch` x `heads` x `seq` rows of head_dim (64 or 128) elements, each with
+ * element strides of its own (multiples of 8; the last dim dense; 16-byte aligned).  o and lse = what the forward returned: the
+ * output and, per row, the natural logarithm of the sum over the keys up to the row of exp(scale q k) (float [batch][heads][seq], dense).
+ * Scores, probabilities and their gradients are fp32, rounded to bf16 as operands of the products; sums are fp32 in a fixed order.
+ * workspace: ti8_attention_bwd_workspace bytes (-1 for sizes it does not take), 16-byte aligned. */
+typedef struct {
+    void* p;
+    int64_t stride_b, stride_h, stride_s;
+} ti8_attention_tensor;
+typedef struct {
+    ti8_attention_tensor q, k, v, o, d_o, dq, dk, dv;
+    const float* lse;
+    void* workspace;
+    int64_t batch, heads, seq, head_dim;
+    float scale;
+} ti8_attention_args;
+int64_t ti8_attention_bwd_workspace(int64_t batch, int64_t heads, int64_t seq);
+int ti8_attention_bwd(const ti8_attention_args* a, ti8_stream_t stream);
+
 /* ---------------------------------------------------------------------------------
  * Measurement aid (no counterpart in the reference; used by bench.py --probe mfma): a loop of nothing
  * but v_mfma_i32_32x32x32_i8 on `workgroups` workgroups of 8 waves, `iters` x 16 MFMAs per wave,

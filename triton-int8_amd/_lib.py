@@ -36,6 +36,17 @@ class LinearArgs(ctypes.Structure):
                 ("workspace", _vp), ("workspace_bytes", _i64), ("saved", _vp), ("saved_bytes", _i64), ("bias", _vp)]
 
 
+class AttentionTensor(ctypes.Structure):
+    """ti8_attention_tensor of include/ti8.h."""
+    _fields_ = [("p", _vp), ("stride_b", _i64), ("stride_h", _i64), ("stride_s", _i64)]
+
+
+class AttentionArgs(ctypes.Structure):
+    """ti8_attention_args of include/ti8.h."""
+    _fields_ = [(name, AttentionTensor) for name in ("q", "k", "v", "o", "d_o", "dq", "dk", "dv")] + [
+        ("lse", _vp), ("workspace", _vp), ("batch", _i64), ("heads", _i64), ("seq", _i64), ("head_dim", _i64), ("scale", _f32)]
+
+
 # name -> argument types, in the order of include/ti8.h
 PROTOTYPES = {
     "ti8_quant_block": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _i64,
@@ -64,10 +75,11 @@ PROTOTYPES = {
     "ti8_rope": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp],
     "ti8_swiglu": [_vp, _vp, _vp, _i64, _vp],
     "ti8_swiglu_bwd": [_vp, _vp, _vp, _vp, _vp, _i64, _vp],
+    "ti8_attention_bwd": [ctypes.POINTER(AttentionArgs), _vp],
     "ti8_probe_mfma": [_vp, _i64, _vp, _int, _int, _int, _int, _vp],
 }
 EXPORTS = ["ti8_version", "ti8_last_error", "ti8_arch", "ti8_init", "ti8_last_gemm_kernel", "ti8_linear_fwd_bwd_workspace", "ti8_linear_workspace",
-           "ti8_rmsnorm_bwd_workspace", "ti8_column_sum_workspace"] + list(PROTOTYPES)
+           "ti8_rmsnorm_bwd_workspace", "ti8_column_sum_workspace", "ti8_attention_bwd_workspace"] + list(PROTOTYPES)
 
 # enums of include/ti8.h
 Q_CLAMP, Q_EPS_ADD, Q_SCALE_BF16, Q_HAD128, Q_WS_PINGPONG, Q_WS_SECOND, Q_TORCH_ROUND, Q_TORCH_BF16, Q_WS_IS_ZERO, Q_SCALE_T = 1, 2, 4, 8, 16, 32, 64, 128, 256, 512
@@ -114,6 +126,8 @@ def lib():
         l.ti8_linear_workspace.argtypes = [ctypes.POINTER(LinearArgs), ctypes.POINTER(_i64)]
         l.ti8_rmsnorm_bwd_workspace.restype = _i64
         l.ti8_rmsnorm_bwd_workspace.argtypes = [_i64, _i64]
+        l.ti8_attention_bwd_workspace.restype = _i64
+        l.ti8_attention_bwd_workspace.argtypes = [_i64, _i64, _i64]
         l.ti8_column_sum_workspace.restype = _i64
         l.ti8_column_sum_workspace.argtypes = [_i64, _i64]
         for name, args in PROTOTYPES.items():

@@ -39,6 +39,7 @@ extern "C" int ti8_init(void) {
     if (int e = init_skinny_kernels()) return e;
     if (int e = init_mid_kernels()) return e;
     if (int e = init_fwht_kernels()) return e;
+    if (int e = init_attention_kernels()) return e;
     if (int e = init_quant_scratch()) return e;
     // last: a device that refuses the persistent kernel's 160 KiB of LDS is not an error (the one-tile kernel serves
     // its shapes), but the message says so

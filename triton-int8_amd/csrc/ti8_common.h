@@ -60,6 +60,7 @@ int init_chain_kernel();
 int init_skinny_kernels();
 int init_mid_kernels();
 int init_fwht_kernels();
+int init_attention_kernels();
 int init_quant_scratch();
 
 // ---- pieces of quant.hip and fwht.hip that the layer calls (step.hip) use ----------

@@ -4,7 +4,7 @@ the training step either side of the hot path, as BASELINE config 5 describes it
 SDPA) and SwiGLU stay in bf16; ``int8=False`` builds the bf16 twin used for loss/grad parity.
 
 In the int8 layer the RMSNorms, the rotary embedding and the SwiGLU product run as one kernel each per direction
-(csrc/decoder.hip); the twin, tensors those kernels do not take and calls under a tracer or a function transform go through the
+(csrc/decoder.hip), and the attention's backward as two (csrc/attention.hip); the twin, tensors those kernels do not take and calls under a tracer or a function transform go through the
 torch expressions, which are also what a backward that is differentiated again is made of.
 """
 import math
@@ -46,15 +46,39 @@ def _swiglu(gate, up):
     return F.silu(gate) * up
 
 
-def _kernels_take(*tensors):
-    """Whether tensors can go to the kernels: plain, dense bf16 tensors on the current device, outside tracing and function transforms
-    (to which a kernel launch is invisible)."""
+def _plain(*tensors):
+    """Whether these are plain bf16 tensors on the current device, outside tracing and function transforms (to which a kernel launch is
+    invisible)."""
     if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._functorch.peek_interpreter_stack() is not None:
         return False
     if torch.autograd.forward_ad._current_level >= 0 or torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
         return False
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.bfloat16 and t.numel() > 0 and t.is_contiguous()
-               and t.data_ptr() % 16 == 0 and t.device.index == torch._C._cuda_getDevice() for t in tensors)
+    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.bfloat16 and t.numel() > 0
+               and t.device.index == torch._C._cuda_getDevice() for t in tensors)
+
+
+def _kernels_take(*tensors):
+    """Whether tensors can go to the elementwise kernels: plain ones that are dense and aligned."""
+    return _plain(*tensors) and all(t.is_contiguous() and t.data_ptr() % 16 == 0 for t in tensors)
+
+
+def _rows16(t):
+    """Whether the attention kernels read a [batch, heads, seq, head_dim] tensor in place: rows of bf16 at 16-byte steps, at 32-bit
+    offsets from the first of a (batch, head)."""
+    sb, sh, ss, sd = t.stride()
+    return sd == 1 and not (sb | sh | ss) & 7 and t.data_ptr() % 16 == 0 and t.shape[3] <= ss <= 0x3fffffff // (t.shape[2] + 512)
+
+
+FLASH_ATTENTION = int(torch.nn.attention.SDPBackend.FLASH_ATTENTION)
+
+
+def _attention_kernels_take(q, k, v, scale):
+    """Whether the backward of an attention goes to csrc/attention.hip: where torch would take its flash kernels (whose forward is kept),
+    on shapes and layouts that ours take."""
+    if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)) or torch.is_autocast_enabled("cuda"):
+        return False
+    return (_plain(q, k, v) and q.shape[3] in (64, 128) and all(t.shape == q.shape and _rows16(t) for t in (q, k, v)) and q.shape[2] <= 1 << 24
+            and torch._fused_sdp_choice(q, k, v, None, 0.0, True, scale=scale) == FLASH_ATTENTION)
 
 
 def _dense(t, like, dtype=torch.bfloat16):
@@ -120,6 +144,32 @@ class _SwiGLUFunction(torch.autograd.Function):
         return ops.swiglu_backward(*(_dense(t, d) for t in (d, gate, up)))
 
 
+class _AttentionFunction(torch.autograd.Function):
+    """Causal attention: torch's flash forward, and a backward with its roundings (probabilities and score gradients to bf16) in
+    csrc/attention.hip.  The forward stays torch's: the int8 codes behind it spread every bit in which another one would differ."""
+
+    @staticmethod
+    def forward(ctx, q, k, v, scale):
+        o, lse = torch.ops.aten._scaled_dot_product_flash_attention(q, k, v, 0.0, True, False, scale=scale)[:2]
+        ctx.save_for_backward(q, k, v, o, lse)
+        ctx.scale = scale
+        return o
+
+    @staticmethod
+    def backward(ctx, d_o):
+        q, k, v, o, lse = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            return (*_differentiable(lambda *t: F.scaled_dot_product_attention(*t, is_causal=True, scale=ctx.scale), (q, k, v), d_o), None)
+        q, k, v, o, d_o = (t if t.dtype == torch.bfloat16 and t.device == d_o.device and _rows16(t) else _dense(t, d_o) for t in (q, k, v, o, d_o))
+        return (*ops.attention_backward(d_o, q, k, v, o, _dense(lse, d_o, torch.float32), ctx.scale), None)
+
+
+def _attention(q, k, v, scale):
+    if _attention_kernels_take(q, k, v, scale):
+        return _AttentionFunction.apply(q, k, v, scale)
+    return F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=scale)
+
+
 class RMSNorm(torch.nn.Module):
     def __init__(self, dim, eps=1e-5, device=None, fused=False):
         super().__init__()
@@ -168,7 +218,8 @@ class DecoderLayer(torch.nn.Module):
         rotate = _RopeFunction.apply if self.int8 and self.head_dim % 16 == 0 and _kernels_take(q, k, cos, sin) else _rope_pair
         q, k = rotate(q, k, cos, sin)
         q, k, v = (t.transpose(1, 2) for t in (q, k, v))
-        a = F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=1.0 / math.sqrt(self.head_dim))
+        scale = 1.0 / math.sqrt(self.head_dim)
+        a = _attention(q, k, v, scale) if self.int8 else F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=scale)
         x = x + self.o_proj(a.transpose(1, 2).reshape(B, S, H))
         h = self.post_norm(x)
         gate, up = self.gate_proj(h), self.up_proj(h)
