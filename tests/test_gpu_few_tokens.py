@@ -1,0 +1,30 @@
+"""dW of a step on few tokens, which rides in the launch of Y and dX on 128 x 128 tiles, against the tiled kernels: the same bits."""
+import pytest
+import torch
+
+from conftest import make_gen, randn_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+# one K tile and two, real tokens below and at their edges; one tile of output features beyond the few-rows kernel's 256, uneven grids
+@pytest.mark.parametrize("scheme,hadamard", [("block_channel", None), ("row_block", None), ("double_channel", None), ("block_channel", 128),
+                                             ("row_block", 128), ("double_channel", "full")])
+@pytest.mark.parametrize("tokens,k,n", [(1, 128, 384), (16, 1024, 512), (128, 384, 1152), (129, 640, 384), (256, 128, 2048)])
+def test_dw_of_few_tokens(dev, monkeypatch, tokens, k, n, scheme, hadamard):
+    import triton_int8_amd as T
+    if hadamard == "full":
+        tokens, n = 1 << (tokens - 1).bit_length(), 512
+    g = make_gen(tokens + k + n)
+    X, W, dY = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev), randn_bf16(g, tokens, n, std=1e-3).to(dev)
+    x, w = X.clone().requires_grad_(True), W.clone().requires_grad_(True)
+    step = T.linear_fwd_bwd(X, W, dY, scheme, hadamard)
+    y = T.Int8LinearFunction.apply(x, w, None, scheme, hadamard)
+    layer = (y.detach(), *torch.autograd.grad(y, (x, w), dY))
+    monkeypatch.setattr(T.ops, "GEMM_PATH", "tiled")
+    tiled = T.linear_fwd_bwd(X, W, dY, scheme, hadamard)
+    assert torch.equal(step[2], tiled[2]) and torch.equal(layer[2], tiled[2])
+    for a, b in zip(step, layer):
+        assert torch.equal(a, b)
+    if scheme == "double_channel":      # int32 sums: Y and dX as well
+        assert torch.equal(step[0], tiled[0]) and torch.equal(step[1], tiled[1])

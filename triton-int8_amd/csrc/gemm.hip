@@ -808,23 +808,30 @@ int ti8::gemm_nt_bias(const ti8_gemm_problem& p, const void* bias, int gemm_flag
     return launch_tiled(fn, a, batch, c, !(gemm_flags & TI8_GEMM_ONE_TILE), st);
 }
 
-// Two GEMMs of batch 1 as one launch of the few-rows kernel, the bias with the first, if that is the kernel both would get alone
-// (same bits); *launched says whether they were.
-int ti8::gemm_nt_pair(const ti8_gemm_problem& p, const void* bias, const ti8_gemm_problem& q, int gemm_flags, bool* launched, ti8_stream_t stream) {
-    *launched = false;
+// Those of the GEMMs of a call on few tokens (batch of one each; the last is dW where the call has a backward) that the few-rows kernel
+// takes, and dW where it has one or two K tiles, as one launch (same bits as apart); the bias goes with the first.  launched[i] says which
+// were; a single GEMM on the few-rows kernel is left to gemm_nt_bias.
+int ti8::gemm_nt_few(const ti8_gemm_problem* problems, int count, bool backward, const void* bias, int gemm_flags, bool* launched, ti8_stream_t stream) {
+    for (int i = 0; i < count; ++i) launched[i] = false;
     if (gemm_flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES | TI8_GEMM_STRICT)) return TI8_OK;
+    const bool i32_full = problems[0].acc_i32_full != 0;
     GemmMulti m;
-    m.count = 2;
-    const ti8_gemm_problem* const both[2] = {&p, &q};
-    for (int i = 0; i < 2; ++i) {
-        const ti8_gemm_problem& x = *both[i];
-        if (x.M > 256 || x.batch != 1 || (x.acc_i32_full != 0) != (p.acc_i32_full != 0)) return TI8_OK;
-        if (int e = prepare_gemm("ti8_gemm_i8_nt", x, gemm_flags, &m.g[i])) return e;
-        if (!skinny_supported(m.g[i]) || idx::gemm_few_rows_prefers_mid(x.M, x.N, x.K, 1, device_cu_count())) return TI8_OK;
+    int where[GEMM_MULTI_MAX], few = 0;
+    m.count = 0;
+    for (int i = 0; i < count; ++i) {
+        const ti8_gemm_problem& x = problems[i];
+        const bool is_dw = backward && i + 1 == count;
+        if (x.batch != 1 || (x.acc_i32_full != 0) != i32_full || (!is_dw && x.M > 256)) continue;
+        GemmArgs& g = m.g[m.count];
+        if (int e = prepare_gemm("ti8_gemm_i8_nt", x, gemm_flags, &g)) return e;
+        if (is_dw ? x.M <= 256 || !thin_supported(g, i32_full) : !skinny_supported(g) || idx::gemm_few_rows_prefers_mid(x.M, x.N, x.K, 1, device_cu_count())) continue;
+        if (!is_dw) ++few;
+        if (i == 0) g.bias = static_cast<const uint16_t*>(bias);
+        where[m.count++] = i;
     }
-    m.g[0].bias = static_cast<const uint16_t*>(bias);
-    *launched = true;
-    return launch_skinny_multi(m, p.acc_i32_full != 0, static_cast<hipStream_t>(stream));
+    if (m.count == 0 || (m.count == 1 && few == 1)) return TI8_OK;
+    for (int i = 0; i < m.count; ++i) launched[where[i]] = true;
+    return launch_few(m, few, i32_full, static_cast<hipStream_t>(stream));
 }
 
 extern "C" int ti8_gemm_i8_nt(const int8_t* A, int64_t bsa, int64_t lda, const int8_t* B, int64_t bsb, int64_t ldb,

@@ -238,12 +238,179 @@ __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g)
     wavering_block<I32FULL>(g, blockIdx.x, blockIdx.y);
 }
 
-// Several GEMMs (batch of one each) in one launch: Y and dX of a step on few tokens, which have few blocks each and wait for their
-// loads most of the time (16 tokens, 4096 -> 4096: 128 blocks and 7.4 us each on 256 CUs; the step 50.3 us apart, 44.6 together).
+// A GEMM over few K tiles: dW of a step on up to 256 tokens.  Its products are nothing beside its output, so this is made for
+// writing that: `workers` workgroups share out the 128 x 128 tiles (worker, worker + workers, ...), the next K tile of the walk is fetched
+// while one is multiplied, and a finished tile leaves through LDS in rows of 256 bytes, its stores in flight behind the next tile's
+// products.  Each of the four waves computes 64 x 64 with the operands of the MFMA swapped: a lane then holds four neighbouring
+// columns of a row, eight bytes of the output.  Sums and epilogue are those of the tiled kernels, operation for operation: the same bits.
+// 16 tokens, 4096 -> 4096, Y, dX and dW: 15.6 us in one launch, bound by its 64 MiB (32 of weight, 32 of dW); 8.9 + 11.2 us with dW on
+// 256 x 256 tiles in a launch of its own, 18.0 us with a workgroup for each tile of dW that loads, multiplies and stores in turn.
+// A_ROW: operand A scaled by rows, else by 128 x 128 blocks; operand B by rows (I32FULL) or by blocks.
+constexpr int THIN_K_TILES = 2, THIN_OPERAND = 128 * 128, THIN_STORES = 8;
+template <bool I32FULL, bool A_ROW>
+__device__ __forceinline__ void thin_walk(const GemmArgs& args, const int worker, const int workers) {
+    const GemmArgs g = args;
+    extern __shared__ __attribute__((aligned(1024))) int8_t smem[];  // two stages of [A 16 KiB][B 16 KiB]; a tile [128 rows][256 bytes] on its way out
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int tiles_n = g.N >> 7, tiles = (g.M >> 7) * tiles_n, nk = g.K >> 7;
+    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64;
+
+    const int ld_row = lane >> 3;
+    uint32_t voffA[2], voffB[2];
+#pragma unroll
+    for (int p = 0; p < 2; ++p) {
+        const int ch = (lane & 7) ^ ld_row ^ p;
+        voffA[p] = (uint32_t)(ld_row * (int)g.lda + ch * 16);
+        voffB[p] = (uint32_t)(ld_row * (int)g.ldb + ch * 16);
+    }
+    auto issue = [&](int tile, int kt, int stage) {       // each wave 32 rows of either operand
+        const int m = (tile / tiles_n) * 128 + wave * 32, n = (tile % tiles_n) * 128 + wave * 32;
+        int8_t* const st = smem + stage * 2 * THIN_OPERAND + wave * 4096;
+        issue_tile_loads<4>(g.A + (int64_t)m * g.lda + kt * 128, 8 * g.lda, voffA, 0, st);
+        issue_tile_loads<4>(g.B + (int64_t)n * g.ldb + kt * 128, 8 * g.ldb, voffB, 0, st + THIN_OPERAND);
+    };
+    // (a K tile's factors by scalar loads: they count apart from the tiles in flight)
+    typedef const float __attribute__((address_space(4))) constant_float;
+    constant_float* const fa_p = (constant_float*)(uintptr_t)g.sa.p;
+    constant_float* const fb_p = (constant_float*)(uintptr_t)g.sb.p;
+    const int fr_row = lane & 31, fr_half = lane >> 5;
+    const int sw = (lane & 7) ^ ((lane >> 3) & 1);
+    int at[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) at[ks] = fr_row * 128 + ((ks * 2 + fr_half) ^ sw) * 16;
+    const v16i vzero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
+
+    v16i acc[2][2];
+    float accf[I32FULL ? 1 : 2][I32FULL ? 1 : 2][16];
+    auto clear = [&]() {
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                acc[i][j] = vzero;
+#pragma unroll
+                for (int r = 0; r < 16; ++r) accf[I32FULL ? 0 : i][I32FULL ? 0 : j][r] = 0.0f;
+            }
+    };
+    clear();
+    float rowm[A_ROW ? 2 : 1];
+    float4 cm[I32FULL ? 2 : 1][I32FULL ? 4 : 1];
+    int stage = 0, tile = worker, kt = 0;
+    bool stored = false;
+    issue(tile, kt, stage);
+    for (;;) {
+        const int m0 = (tile / tiles_n) * 128, n0 = (tile % tiles_n) * 128;
+        const bool last = kt + 1 == nk;
+        const int next_tile = last ? tile + workers : tile, next_kt = last ? 0 : kt + 1;
+        // the loads of this K tile are older than the stores of the tile before, which may stay in flight
+        if (stored) TI8_WAIT_VMCNT_LGKM0(THIN_STORES);
+        else TI8_WAIT_VMCNT_LGKM0(0);
+        asm volatile("s_barrier" ::: "memory");
+        int8_t* const st = smem + stage * 2 * THIN_OPERAND;
+        stage ^= 1;
+        if (last) {      // the vectors of the epilogue, in front of the next loads so that they can be waited for alone
+            if (A_ROW)
+#pragma unroll
+                for (int i = 0; i < 2; ++i) rowm[A_ROW ? i : 0] = g.sa.p[(int64_t)(m0 + wm + i * 32 + fr_row) * g.sa.rs];
+            if (I32FULL)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) cm[I32FULL ? j : 0][I32FULL ? q : 0] = *reinterpret_cast<const float4*>(g.sb.p + n0 + wn + j * 32 + 8 * q + 4 * fr_half);
+        }
+        if (next_tile < tiles) issue(next_tile, next_kt, stage);
+        const int8_t* const sa = st + wm * 128;
+        const int8_t* const sb = st + THIN_OPERAND + wn * 128;
+#pragma unroll
+        for (int ks = 0; ks < 4; ++ks) {
+            v4i fa[2], fb[2];
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                fa[i] = *reinterpret_cast<const v4i*>(sa + i * 4096 + at[ks]);
+                fb[i] = *reinterpret_cast<const v4i*>(sb + i * 4096 + at[ks]);
+            }
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fb[j], fa[i], !I32FULL && ks == 0 ? vzero : acc[i][j], 0, 0, 0);
+        }
+        if (!I32FULL) {
+            const float factor = (A_ROW ? 1.0f : fa_p[(int64_t)(m0 >> 7) * g.sa.rs + kt * g.sa.ks]) * fb_p[(int64_t)(n0 >> 7) * g.sb.rs + kt * g.sb.ks];
+#pragma unroll
+            for (int i = 0; i < 2; ++i)
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int r = 0; r < 16; ++r) accf[i][j][r] = __builtin_fmaf(static_cast<float>(acc[i][j][r]), factor, accf[i][j][r]);
+        }
+        if (last) {
+            __builtin_amdgcn_s_waitcnt(0xc07f);     // lgkmcnt(0): this wave's reads of the stage that the tile leaves through
+            asm volatile("s_barrier" ::: "memory");
+            // register 4 q + c of block (i, j): row wm + 32 i + lane % 32, column wn + 32 j + 8 q + 4 (lane / 32) + c.  (Written out: in
+            // front of an LDS write that it knows the compiler waits for all loads in flight, which write LDS too.)
+            const uint32_t slab = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)st;
+#pragma unroll
+            for (int i = 0; i < 2; ++i) {
+                const int row = wm + i * 32 + fr_row;
+#pragma unroll
+                for (int j = 0; j < 2; ++j)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const int col = wn + j * 32 + 8 * q + 4 * fr_half;
+                        const float4 c4 = cm[I32FULL ? j : 0][I32FULL ? q : 0];
+                        const float cn[4] = {c4.x, c4.y, c4.z, c4.w};
+                        float t[4];
+#pragma unroll
+                        for (int c = 0; c < 4; ++c) {
+                            float v;
+                            if (I32FULL) {
+                                v = static_cast<float>(acc[i][j][4 * q + c]) * rowm[A_ROW ? i : 0];
+                                v = v * cn[c];
+                                if (g.post_scale != 0.0f) v = __uint_as_float(pack_bf16x2(v, 0.0f) << 16) * g.post_scale;
+                            } else {
+                                v = accf[I32FULL ? 0 : i][I32FULL ? 0 : j][4 * q + c];
+                                if (A_ROW) v = v * rowm[A_ROW ? i : 0];
+                                v = v * g.out_scale;       // 1 or a power of two
+                            }
+                            t[c] = v;
+                        }
+                        const v2i w = {(int)pack_bf16x2(t[0], t[1]), (int)pack_bf16x2(t[2], t[3])};
+                        asm volatile("ds_write_b64 %0, %1" ::"v"(slab + row * 256 + ((col * 2) ^ ((row & 15) << 4))), "v"(w) : "memory");
+                    }
+            }
+            __builtin_amdgcn_s_waitcnt(0xc07f);
+            asm volatile("s_barrier" ::: "memory");
+            uint16_t* const out = reinterpret_cast<uint16_t*>(g.C) + (int64_t)m0 * g.ldc + n0 + (lane & 15) * 8;
+            // row 16 p + 4 wave + lane / 16, chunk lane % 16
+            const uint32_t from = slab + (wave * 4 + (lane >> 4)) * 256 + (((lane & 15) ^ ((wave * 4 + (lane >> 4)) & 15)) << 4);
+            v4i w[THIN_STORES];
+            asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %8 offset:4096\n\tds_read_b128 %2, %8 offset:8192\n\tds_read_b128 %3, %8 offset:12288\n\t"
+                         "ds_read_b128 %4, %8 offset:16384\n\tds_read_b128 %5, %8 offset:20480\n\tds_read_b128 %6, %8 offset:24576\n\tds_read_b128 %7, %8 offset:28672\n\t"
+                         "s_waitcnt lgkmcnt(0)"
+                         : "=&v"(w[0]), "=&v"(w[1]), "=&v"(w[2]), "=&v"(w[3]), "=&v"(w[4]), "=&v"(w[5]), "=&v"(w[6]), "=&v"(w[7]) : "v"(from) : "memory");
+#pragma unroll
+            for (int p = 0; p < THIN_STORES; ++p) *reinterpret_cast<v4i*>(out + (int64_t)(p * 16 + wave * 4 + (lane >> 4)) * g.ldc) = w[p];
+            if (next_tile >= tiles) break;
+            clear();
+        }
+        stored = last;
+        tile = next_tile;
+        kt = next_kt;
+    }
+}
+
+// The GEMMs of a step, or of its backward, on few tokens (batch of one each) in one launch: Y and dX, which have few blocks each
+// and wait for their loads most of the time, and with m.count > few dW behind them, a workgroup per CU.
 template <bool I32FULL>
-__global__ __launch_bounds__(256) void gemm_i8_wavering_multi_kernel(const GemmMulti m) {
+__global__ __launch_bounds__(256) void gemm_i8_few_kernel(const GemmMulti m, const int few) {
     const int i = idx::gemm_multi_pick((int)blockIdx.x, m.first[1], m.first[2], m.count);
-    wavering_block<I32FULL>(m.g[i], (int)blockIdx.x - m.first[i], 0);
+    if (i < few) wavering_block<I32FULL>(m.g[i], (int)blockIdx.x - m.first[i], 0);
+    else {
+        const int worker = (int)blockIdx.x - m.first[i], workers = (int)gridDim.x - m.first[i];
+        if (I32FULL || m.g[i].sa.mode == TI8_SCALE_ROW) thin_walk<I32FULL, true>(m.g[i], worker, workers);
+        else thin_walk<I32FULL, I32FULL>(m.g[i], worker, workers);
+    }
 }
 
 bool skinny_supported(const GemmArgs& a) {
@@ -254,14 +421,21 @@ bool skinny_supported(const GemmArgs& a) {
     return (int64_t)(a.N / 32) * (a.M / 32) <= 0x7fffffffLL;
 }
 
+bool thin_supported(const GemmArgs& a, bool i32_full) {
+    if (a.K > THIN_K_TILES * 128 || a.M % 128 || a.N % 128 || a.strict || a.combine != TI8_COMBINE_MUL_MUL || !aligned16(a.C) || a.ldc % 8) return false;
+    if (i32_full ? a.sb.rs != 1 || !aligned16(a.sb.p) : a.sb.mode != TI8_SCALE_BLOCK128 || (a.sa.mode != TI8_SCALE_ROW && a.sa.mode != TI8_SCALE_BLOCK128)) return false;
+    return (int64_t)(a.M / 128) * (a.N / 128) <= 0x3fffffff;
+}
+
 constexpr size_t WAVERING_LDS_BYTES = (size_t)4 * WS_STAGES * WS_STAGE_BYTES;
+static_assert(WAVERING_LDS_BYTES >= (size_t)2 * 2 * THIN_OPERAND, "the tiles of dW share the launch");
 
 int init_skinny_kernels() {
     static OncePerDevice once_i32, once_promote, once_i32_multi, once_promote_multi;
     hipError_t e = raise_lds_limit(once_i32, reinterpret_cast<const void*>(gemm_i8_wavering_kernel<true>), (int)WAVERING_LDS_BYTES);
     if (e == hipSuccess) e = raise_lds_limit(once_promote, reinterpret_cast<const void*>(gemm_i8_wavering_kernel<false>), (int)WAVERING_LDS_BYTES);
-    if (e == hipSuccess) e = raise_lds_limit(once_i32_multi, reinterpret_cast<const void*>(gemm_i8_wavering_multi_kernel<true>), (int)WAVERING_LDS_BYTES);
-    if (e == hipSuccess) e = raise_lds_limit(once_promote_multi, reinterpret_cast<const void*>(gemm_i8_wavering_multi_kernel<false>), (int)WAVERING_LDS_BYTES);
+    if (e == hipSuccess) e = raise_lds_limit(once_i32_multi, reinterpret_cast<const void*>(gemm_i8_few_kernel<true>), (int)WAVERING_LDS_BYTES);
+    if (e == hipSuccess) e = raise_lds_limit(once_promote_multi, reinterpret_cast<const void*>(gemm_i8_few_kernel<false>), (int)WAVERING_LDS_BYTES);
     if (e != hipSuccess) return fail(TI8_ERR_HIP, "gemm: cannot raise the LDS limit to %zu: %s", WAVERING_LDS_BYTES, hipGetErrorString(e));
     return TI8_OK;
 }
@@ -282,18 +456,20 @@ int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t s
     return launch_wavering(a, batch, i32_full, st);
 }
 
-int launch_skinny_multi(GemmMulti& m, bool i32_full, hipStream_t st) {
+int launch_few(GemmMulti& m, int few, bool i32_full, hipStream_t st) {
     if (int e = init_skinny_kernels()) return e;
     int64_t total = 0;
+    const int64_t cus = device_cu_count();
     for (int i = 0; i < m.count; ++i) {
         m.first[i] = (int)total;
-        total += (int64_t)(m.g[i].N / 32) * (m.g[i].M / 32);
+        const int64_t tiles = (int64_t)(m.g[i].N / 128) * (m.g[i].M / 128);
+        total += i < few ? (int64_t)(m.g[i].N / 32) * (m.g[i].M / 32) : tiles < cus ? tiles : cus;
+        if (total > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "gemm: too many blocks");
     }
-    if (total > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "gemm: too many blocks");
     for (int i = m.count; i <= GEMM_MULTI_MAX; ++i) m.first[i] = (int)total;
     for (int i = m.count; i < GEMM_MULTI_MAX; ++i) m.g[i] = m.g[0];
-    const auto kernel = i32_full ? gemm_i8_wavering_multi_kernel<true> : gemm_i8_wavering_multi_kernel<false>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), WAVERING_LDS_BYTES, st, m);
+    const auto kernel = i32_full ? gemm_i8_few_kernel<true> : gemm_i8_few_kernel<false>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), WAVERING_LDS_BYTES, st, m, few);
     note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
     return check_launch("ti8_gemm_i8_nt");
 }

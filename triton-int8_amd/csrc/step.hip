@@ -304,19 +304,17 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
     return TI8_OK;
 }
 
-// One GEMM launched alone (what ti8_gemm_i8_nt selects for its shape: the few-rows kernel up to 256 rows).  `live` rows of A are
-// multiplied: with few tokens the padding rows of the 128-row-quantised operand are zeros whose products nobody reads.
-int one_gemm(const ti8_gemm_problem& p, int64_t live, const void* bias, int64_t tokens, int gemm_flags, ti8_stream_t stream) {
-    ti8_gemm_problem q = p;
-    q.M = live;
+// One GEMM launched alone (what ti8_gemm_i8_nt selects for its shape: the few-rows kernel up to 256 rows)
+int one_gemm(const ti8_gemm_problem& q, const void* bias, int64_t tokens, int gemm_flags, ti8_stream_t stream) {
     bool added = false;
     if (int e = gemm_nt_bias(q, bias, gemm_flags, &added, stream)) return e;
-    return bias && !added ? add_bias(p.C, p.ldc, bias, tokens, p.N, stream) : TI8_OK;
+    return bias && !added ? add_bias(q.C, q.ldc, bias, tokens, q.N, stream) : TI8_OK;
 }
 
 int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t stream) {
     const int flags = L.a->gemm_flags;
-    // rows of a token operand to multiply: all of them, or with up to 256 (padded) tokens the real ones rounded up to 32
+    // rows of a token operand to multiply: all of them, or with up to 256 (padded) tokens the real ones rounded up to 32 (the padding
+    // rows of the 128-row-quantised operand are zeros whose products nobody reads)
     auto live_rows = [&](int64_t contraction) {
         if (L.T > 256 || (flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES)) || contraction > 32768) return L.T;
         const int64_t r = (L.tokens + 31) / 32 * 32;
@@ -327,19 +325,17 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
         if (int e = ti8_gemm_i8_nt_multi(g, count, flags | TI8_GEMM_TOGETHER, stream)) return e;
         return L.fwd && L.a->bias ? add_bias(L.a->Y, L.a->ldy, L.a->bias, L.tokens, L.N, stream) : TI8_OK;
     }
-    int first = 0;
-    if (count == 3) {   // Y and dX have few rows both: one launch where the few-rows kernel takes them
-        ti8_gemm_problem y = g[0], dx = g[1];
-        y.M = live_rows(y.K);
-        dx.M = live_rows(dx.K);
-        bool launched = false;
-        if (int e = gemm_nt_pair(y, L.a->bias, dx, flags, &launched, stream)) return e;
-        if (launched) first = 2;
+    ti8_gemm_problem few[3];
+    const void* const bias = L.fwd ? L.a->bias : nullptr;
+    for (int i = 0; i < count; ++i) {
+        few[i] = g[i];
+        if (i + 1 < count || !L.bwd) few[i].M = live_rows(g[i].K);      // dW, the last of a backward, has one row per output feature
     }
-    for (int i = first; i < count; ++i) {
-        const bool token_rows = i + 1 < count || !L.bwd;     // dW, the last of a backward, has one row per output feature
-        if (int e = one_gemm(g[i], token_rows ? live_rows(g[i].K) : g[i].M, L.fwd && i == 0 ? L.a->bias : nullptr, L.tokens, flags, stream)) return e;
-    }
+    bool launched[3];
+    if (int e = gemm_nt_few(few, count, L.bwd, bias, flags, launched, stream)) return e;
+    for (int i = 0; i < count; ++i)
+        if (!launched[i])
+            if (int e = one_gemm(few[i], i == 0 ? bias : nullptr, L.tokens, flags, stream)) return e;
     return TI8_OK;
 }
 

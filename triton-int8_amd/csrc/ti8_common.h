@@ -82,8 +82,8 @@ int fwht_t_quant_row_valid(const void* x, int64_t ldx, void* scratch, int8_t* q,
 int fill_words(unsigned int* p, int64_t words, unsigned int value, hipStream_t st);
 // ti8_gemm_i8_nt with a bias for the kernels whose epilogue adds one (*added: this was one); y += bias behind the others (bias.hip)
 int gemm_nt_bias(const ti8_gemm_problem& p, const void* bias, int gemm_flags, bool* added, ti8_stream_t stream);
-// gemm.hip: Y and dX of a step on few tokens as one launch of the few-rows kernel (see there)
-int gemm_nt_pair(const ti8_gemm_problem& p, const void* bias, const ti8_gemm_problem& q, int gemm_flags, bool* launched, ti8_stream_t stream);
+// gemm.hip: the GEMMs of a call on few tokens as one launch, those that go into it (see there)
+int gemm_nt_few(const ti8_gemm_problem* problems, int count, bool backward, const void* bias, int gemm_flags, bool* launched, ti8_stream_t stream);
 int add_bias(void* y, int64_t ldy, const void* bias, int64_t rows, int64_t cols, ti8_stream_t stream);
 // out[c] = bf16(sum over g of partial[g][c]), dim a multiple of 32 (decoder.hip)
 int sum_partials(const char* fn, const float* partial, int groups, int64_t dim, void* out, hipStream_t st);
