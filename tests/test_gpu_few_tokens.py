@@ -28,3 +28,31 @@ def test_dw_of_few_tokens(dev, monkeypatch, tokens, k, n, scheme, hadamard):
         assert torch.equal(a, b)
     if scheme == "double_channel":      # int32 sums: Y and dX as well
         assert torch.equal(step[0], tiled[0]) and torch.equal(step[1], tiled[1])
+
+
+# workgroups of four 32 x 32 blocks: whole tiles of 64 rows and a last one of 32, a single K tile for four waves, uneven K quarters, strips
+# that are and are not a multiple of 8
+@pytest.mark.parametrize("m,n,k", [(64, 16384, 128), (96, 8192, 384), (160, 4224, 640), (256, 2048, 1152), (192, 5376, 256)])
+@pytest.mark.parametrize("mode", ["double_channel", "block_channel", "row_block", "bias"])
+def test_four_blocks_per_workgroup(dev, monkeypatch, m, n, k, mode):
+    import triton_int8_amd as T
+    g = make_gen(m + n + k)
+    x, w = randn_bf16(g, m, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev)
+    scheme = "block_channel" if mode == "bias" else mode
+    layer = T.Int8Linear(k, n, bias=mode == "bias", scheme=scheme, device=dev)
+    with torch.no_grad():
+        layer.weight.copy_(w)
+        if layer.bias is not None:
+            layer.bias.copy_(randn_bf16(g, n).to(dev))
+        got = layer(x)
+        monkeypatch.setattr(T.ops, "GEMM_PATH", "tiled")
+        want = layer(x)
+    if mode == "double_channel":
+        assert torch.equal(got, want)       # int32 sums
+    else:
+        # the same products in another order: K / 128 roundings of 2^-24 either way, then one of 2^-8 of the value to bf16 (two with a bias, of
+        # values up to the product's and the bias's magnitude)
+        mag = want.float().abs() + (layer.bias.detach().float().abs() if layer.bias is not None else 0.0)
+        spread = (k // 128 + 4) * 2.0 ** -23 * (x.float().abs().amax(1, keepdim=True) * w.float().abs().amax() * k)
+        assert bool(((got.float() - want.float()).abs() <= 2.0 ** -7 * mag + spread).all())
+        assert float((got != want).float().mean()) <= 0.01

@@ -28,17 +28,22 @@ namespace ti8 {
 // shared by the workgroup and one barrier per K tile took 14.4 us where this one takes 11.2 us
 // (128 rows, K = N = 4096).  Two stages = 64 KiB per workgroup, so two workgroups share a CU.
 constexpr int WS_STAGES = 2;
-constexpr int WS_STAGE_BYTES = 2 * 32 * 128;
-constexpr int WS_LOADS = 8;  // global->LDS instructions per wave and stage
 
-// `block_x` = index of the workgroup among the blocks of this GEMM and batch.
-template <bool I32FULL>
+// A workgroup's part of C is MB x NB blocks of 32 x 32, one or four: `block_x` = index of the workgroup among those of this GEMM and
+// batch.  What bounds the kernel is the stream into a CU's LDS (55 bytes per ns, half of what the L2 alone delivers; neither more stages
+// in flight, 3 or 4 instead of 2, nor leaving the MFMAs out makes a difference), and of four blocks the stream is half as long per
+// product.  idx::few_rows_wide says where which is the faster one.  us, one block / four, int32 path: 64 rows, 4096 -> 14336
+// 21.0 / 15.3; 128 rows 4096 -> 4096 10.1 / 10.1, 8192 -> 8192 33.4 / 21.1; 256 rows 4096 -> 4096 16.7 / 10.8, 14336 -> 4096 98 / 36;
+// 64 rows, 14336 -> 14336 46.6 / 32.1 (31.6 for the weight alone).
+template <bool I32FULL, int BLOCKS>
 __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int block_x, const int batch) {
-    extern __shared__ __attribute__((aligned(1024))) int8_t smem[];  // 4 waves x WS_STAGES x 8 KiB
+    constexpr int MB = BLOCKS, NB = BLOCKS;
+    constexpr int STAGE_BYTES = (MB + NB) * 32 * 128;     // per wave
+    extern __shared__ __attribute__((aligned(1024))) int8_t smem[];  // 4 waves x WS_STAGES x STAGE_BYTES
 
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int mtiles = g.M >> 5, nstrips = g.N >> 5;
+    const int mtiles = (g.M + 32 * MB - 1) / (32 * MB), nstrips = g.N / (32 * NB);
     int strip, mt;
     if ((nstrips & 7) == 0) {   // workgroups that share a strip of B on one XCD (ids 8 apart)
         const int xcd = block_x & 7, idx = block_x >> 3;
@@ -48,13 +53,14 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
         strip = block_x / mtiles;
         mt = block_x % mtiles;
     }
-    const int n0 = strip * 32, m0 = mt * 32;
+    const int n0 = strip * 32 * NB, m0 = mt * 32 * MB;
+    const int mblocks = min(MB, (g.M - m0) >> 5);      // blocks of rows that exist; what is computed beyond them is not stored
     const int nk = g.K >> 7;
     const int kbeg = (wave * nk) >> 2, kend = ((wave + 1) * nk) >> 2;
     const int nq = kend - kbeg;
 
-    // ---- global -> LDS (same slab layout and swizzle as the other kernels): 4 instructions of A
-    // (rows 8i .. 8i+7) and 4 of B per stage, all issued by the wave that consumes them
+    // ---- global -> LDS (same slab layout and swizzle as the other kernels): 4 instructions per block
+    // of A's or B's rows (rows 8i .. 8i+7) and stage, all issued by the wave that consumes them
     const int ld_row = lane >> 3;
     uint32_t voffA[2], voffB[2];
 #pragma unroll
@@ -66,20 +72,24 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
     const int8_t* baseA = g.A + (int64_t)batch * g.bsa + (int64_t)m0 * g.lda;
     const int8_t* baseB = g.B + (int64_t)batch * g.bsb + (int64_t)n0 * g.ldb;
     const int64_t strideA8 = 8 * g.lda, strideB8 = 8 * g.ldb;
-    int8_t* const ring = smem + wave * (WS_STAGES * WS_STAGE_BYTES);
-    // step i of this wave's walk is K tile kbeg + (i + rot) mod nq: workgroups start at different
-    // tiles so that they do not ask the same memory channels for their lines at the same time
-    const int rot = nq > 0 ? (int)((((unsigned)block_x >> 3) * 3u + (unsigned)batch) % (unsigned)nq) : 0;
+    int8_t* const ring = smem + wave * (WS_STAGES * STAGE_BYTES);
+    // step i of this wave's walk is K tile kbeg + (i + rot) mod nq: workgroups of one block start at different
+    // tiles so that they do not ask the same memory channels for their lines at the same time.  With more rows what counts is that
+    // the workgroups of an XCD read A's columns together, which then need not all fit its L2 (256 rows, K = 14336, N = 4096:
+    // 36 us, 55 from different tiles on)
+    const int rot = nq > 0 && BLOCKS == 1 ? (int)((((unsigned)block_x >> 3) * 3u + (unsigned)batch) % (unsigned)nq) : 0;
     auto tile_of_step = [&](int i) {
         int j = min(i, max(nq - 1, 0)) + rot;   // past the end: the last one again, into a free stage
         if (j >= nq) j -= nq;
         return min(kbeg + max(j, 0), nk - 1);
     };
     auto issue_stage = [&](int i) {
-        int8_t* st = ring + (i & (WS_STAGES - 1)) * WS_STAGE_BYTES;
+        int8_t* st = ring + (i & (WS_STAGES - 1)) * STAGE_BYTES;
         const int koff = tile_of_step(i) * 128;
-        issue_tile_loads<4>(baseA + koff, strideA8, voffA, 0, st);
-        issue_tile_loads<4>(baseB + koff, strideB8, voffB, 0, st + 4096);
+#pragma unroll
+        for (int b = 0; b < MB; ++b) issue_tile_loads<4>(baseA + koff + min(b, mblocks - 1) * 4 * strideA8, strideA8, voffA, 0, st + b * 4096);
+#pragma unroll
+        for (int b = 0; b < NB; ++b) issue_tile_loads<4>(baseB + koff + b * 4 * strideB8, strideB8, voffB, 0, st + (MB + b) * 4096);
     };
 
     // ---- scales: unconditional loads (an operand that contributes no in-loop factor is read with
@@ -107,45 +117,65 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
             fvec[c] = f;
         }
     }
-    // epilogue scales of the 4 outputs this thread will finish: row t/8, columns 4*(t%8) .. +3
+    // epilogue scales of the outputs this thread will finish: row t/8, columns 4*(t%8) .. +3 of every block
     const int e_row = threadIdx.x >> 3, e_col = (threadIdx.x & 7) * 4;
     const bool row_part = I32FULL || g.sa.mode == TI8_SCALE_ROW, col_part = I32FULL || g.sb.mode == TI8_SCALE_ROW;
-    float rowm = g.sa.p[(int64_t)batch * g.sa.bs + (row_part ? (int64_t)(m0 + e_row) * g.sa.rs : 0)];
-    float coln[4];
+    float rowm[MB], coln[NB][4];
 #pragma unroll
-    for (int c = 0; c < 4; ++c) coln[c] = g.sb.p[(int64_t)batch * g.sb.bs + (col_part ? (int64_t)(n0 + e_col + c) * g.sb.rs : 0)];
+    for (int b = 0; b < MB; ++b)
+        rowm[b] = g.sa.p[(int64_t)batch * g.sa.bs + (row_part ? (int64_t)(m0 + min(b, mblocks - 1) * 32 + e_row) * g.sa.rs : 0)];
+#pragma unroll
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int c = 0; c < 4; ++c) coln[b][c] = g.sb.p[(int64_t)batch * g.sb.bs + (col_part ? (int64_t)(n0 + b * 32 + e_col + c) * g.sb.rs : 0)];
     if (divide) {
-        rowm = 1.0f / rowm;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) coln[c] = 1.0f / coln[c];
+        for (int b = 0; b < MB; ++b) rowm[b] = 1.0f / rowm[b];
+#pragma unroll
+        for (int b = 0; b < NB; ++b)
+#pragma unroll
+            for (int c = 0; c < 4; ++c) coln[b][c] = 1.0f / coln[b][c];
     }
 
-    // the bias of those 4 columns (without one: 8 bytes of B, dropped)
-    const uint2 bias = *reinterpret_cast<const uint2*>(g.bias ? reinterpret_cast<const void*>(g.bias + n0 + e_col) : reinterpret_cast<const void*>(g.B));
+    // the bias of those columns (without one: 8 bytes of B, dropped)
+    uint32_t bias_lo[NB], bias_hi[NB];
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        const uint2 bias = *reinterpret_cast<const uint2*>(g.bias ? reinterpret_cast<const void*>(g.bias + n0 + b * 32 + e_col) : reinterpret_cast<const void*>(g.B));
+        bias_lo[b] = bias.x;
+        bias_hi[b] = bias.y;
+    }
 
     const int fr_row = lane & 31, fr_half = lane >> 5;
     const int sw = (lane & 7) ^ ((lane >> 3) & 1);
-    int choff[4];
+    int at[4];
 #pragma unroll
-    for (int ks = 0; ks < 4; ++ks) choff[ks] = ((ks * 2 + fr_half) ^ sw) * 16;
-    const int a_off = fr_row * 128, b_off = 4096 + fr_row * 128;
+    for (int ks = 0; ks < 4; ++ks) at[ks] = fr_row * 128 + ((ks * 2 + fr_half) ^ sw) * 16;
 
     const v16i vzero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
-    v16i acc = vzero;
-    float accf[16];
+    v16i d[MB][NB];             // int32 sums: of the whole K (I32FULL), or of the step whose products are folded next
+    float accf[I32FULL ? 1 : MB][I32FULL ? 1 : NB][16];
 #pragma unroll
-    for (int i = 0; i < 16; ++i) accf[i] = 0.0f;
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j) {
+            d[i][j] = vzero;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) accf[I32FULL ? 0 : i][I32FULL ? 0 : j][r] = 0.0f;
+        }
 
-#pragma unroll
-    for (int s = 0; s < WS_STAGES - 1; ++s) issue_stage(s);
+    issue_stage(0);
     // pin the scale vectors to registers here (they are older than the tile loads, so this waits
     // for nothing else): a load still pending at the loop's entry makes the compiler drain the
     // whole load queue at the top of every iteration
-    asm volatile("" : "+v"(rowm));
-    uint32_t bias_lo = bias.x, bias_hi = bias.y;
-    asm volatile("" : "+v"(bias_lo), "+v"(bias_hi));
 #pragma unroll
-    for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(coln[c]));
+    for (int b = 0; b < MB; ++b) asm volatile("" : "+v"(rowm[b]));
+#pragma unroll
+    for (int b = 0; b < NB; ++b) {
+        asm volatile("" : "+v"(bias_lo[b]), "+v"(bias_hi[b]));
+#pragma unroll
+        for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(coln[b][c]));
+    }
 
     auto factor_of_step = [&](int i) -> float {
         const int kt = tile_of_step(i);
@@ -156,86 +186,104 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
         const float v3 = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(fvec[3]), l));
         return c == 0 ? v0 : (c == 1 ? v1 : (c == 2 ? v2 : v3));
     };
-    v16i d = vzero;
     float f_prev = 0.0f;
+    auto fold = [&]() {
+#pragma unroll
+        for (int i = 0; i < MB; ++i)
+#pragma unroll
+            for (int j = 0; j < NB; ++j)
+#pragma unroll
+                for (int r = 0; r < 16; ++r) {
+                    float& a = accf[I32FULL ? 0 : i][I32FULL ? 0 : j][r];
+                    a = __builtin_fmaf(static_cast<float>(d[i][j][r]), f_prev, a);
+                }
+    };
     for (int i = 0; i < nq; ++i) {
-        // own loads of step i landed (at most the WS_STAGES - 2 younger steps outstanding); own
-        // LDS reads of step i - 1 returned, so its stage can be refilled.  No barrier: nobody
+        // own loads of step i landed; own LDS reads of step i - 1 returned, so its stage can be refilled.  No barrier: nobody
         // else touches this wave's ring.
-        TI8_WAIT_VMCNT_LGKM0((WS_STAGES - 2) * WS_LOADS);
-        issue_stage(i + WS_STAGES - 1);
-        const int8_t* st = ring + (i & (WS_STAGES - 1)) * WS_STAGE_BYTES;
-        v4i fa[4], fb[4];
+        TI8_WAIT_VMCNT_LGKM0(0);
+        issue_stage(i + 1);
+        const int8_t* st = ring + (i & (WS_STAGES - 1)) * STAGE_BYTES;
+        v4i fa[MB][4], fb[NB][4];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
-            fa[ks] = *reinterpret_cast<const v4i*>(st + a_off + choff[ks]);
-            fb[ks] = *reinterpret_cast<const v4i*>(st + b_off + choff[ks]);
+#pragma unroll
+            for (int b = 0; b < MB; ++b) fa[b][ks] = *reinterpret_cast<const v4i*>(st + b * 4096 + at[ks]);
+#pragma unroll
+            for (int b = 0; b < NB; ++b) fb[b][ks] = *reinterpret_cast<const v4i*>(st + (MB + b) * 4096 + at[ks]);
         }
-        __builtin_amdgcn_sched_barrier(0);   // all eight reads go out before anything else
-        if (I32FULL) {
-#pragma unroll
-            for (int ks = 0; ks < 4; ++ks) acc = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[ks], fb[ks], acc, 0, 0, 0);
-        } else {
-#pragma unroll
-            for (int r = 0; r < 16; ++r) accf[r] = __builtin_fmaf(static_cast<float>(d[r]), f_prev, accf[r]);
+        __builtin_amdgcn_sched_barrier(0);   // all reads go out before anything else
+        if (!I32FULL) {
+            fold();
             __builtin_amdgcn_sched_barrier(0);
-            d = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[0], fb[0], vzero, 0, 0, 0);
-#pragma unroll
-            for (int ks = 1; ks < 4; ++ks) d = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[ks], fb[ks], d, 0, 0, 0);
-            f_prev = factor_of_step(i);
         }
-    }
-    if (!I32FULL) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) accf[r] = __builtin_fmaf(static_cast<float>(d[r]), f_prev, accf[r]);
+        for (int ks = 0; ks < 4; ++ks)
+#pragma unroll
+            for (int a = 0; a < MB; ++a)
+#pragma unroll
+                for (int b = 0; b < NB; ++b) d[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[a][ks], fb[b][ks], !I32FULL && ks == 0 ? vzero : d[a][b], 0, 0, 0);
+        if (!I32FULL) f_prev = factor_of_step(i);
     }
+    if (!I32FULL) fold();
     // every load (the redundant ones of the last steps included) has landed and every wave is
     // done with its ring before the rings are reused for the partial results
     __builtin_amdgcn_s_waitcnt(0);
     __syncthreads();
-    uint32_t* part = reinterpret_cast<uint32_t*>(smem);   // [K quarter][32 rows][32 columns]
+    uint32_t* part = reinterpret_cast<uint32_t*>(smem);   // [block of the workgroup][K quarter][32 rows][32 columns]
 #pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        const int row = 8 * (i >> 2) + 4 * fr_half + (i & 3);
-        part[(wave * 32 + row) * 32 + fr_row] = I32FULL ? static_cast<uint32_t>(acc[i]) : __float_as_uint(accf[i]);
-    }
+    for (int i = 0; i < MB; ++i)
+#pragma unroll
+        for (int j = 0; j < NB; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                const int row = 8 * (r >> 2) + 4 * fr_half + (r & 3);
+                part[(((i * NB + j) * 4 + wave) * 32 + row) * 32 + fr_row] = I32FULL ? static_cast<uint32_t>(d[i][j][r]) : __float_as_uint(accf[I32FULL ? 0 : i][I32FULL ? 0 : j][r]);
+            }
     __syncthreads();
-    uint4 pq[4];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) pq[q] = *reinterpret_cast<const uint4*>(part + (q * 32 + e_row) * 32 + e_col);
-    const uint32_t w0[4] = {pq[0].x, pq[0].y, pq[0].z, pq[0].w}, w1[4] = {pq[1].x, pq[1].y, pq[1].z, pq[1].w};
-    const uint32_t w2[4] = {pq[2].x, pq[2].y, pq[2].z, pq[2].w}, w3[4] = {pq[3].x, pq[3].y, pq[3].z, pq[3].w};
-    float t[4];
+    for (int i = 0; i < MB; ++i) {
+        if (i >= mblocks) break;
 #pragma unroll
-    for (int c = 0; c < 4; ++c) {
-        float v;
-        if (I32FULL) {
-            v = static_cast<float>(static_cast<int32_t>(w0[c] + w1[c] + w2[c] + w3[c])) * rowm;
-            v = v * coln[c];
-            if (g.post_scale != 0.0f) v = __uint_as_float(f32_to_bf16_bits(v) << 16) * g.post_scale;
-        } else {
-            v = __uint_as_float(w0[c]) + __uint_as_float(w1[c]);
-            v = v + __uint_as_float(w2[c]);
-            v = v + __uint_as_float(w3[c]);
-            if (row_part) v = v * rowm;
-            if (col_part) v = v * coln[c];
-            if (g.out_scale != 1.0f) v = v * g.out_scale;
+        for (int j = 0; j < NB; ++j) {
+            uint4 pq[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) pq[q] = *reinterpret_cast<const uint4*>(part + (((i * NB + j) * 4 + q) * 32 + e_row) * 32 + e_col);
+            const uint32_t w0[4] = {pq[0].x, pq[0].y, pq[0].z, pq[0].w}, w1[4] = {pq[1].x, pq[1].y, pq[1].z, pq[1].w};
+            const uint32_t w2[4] = {pq[2].x, pq[2].y, pq[2].z, pq[2].w}, w3[4] = {pq[3].x, pq[3].y, pq[3].z, pq[3].w};
+            float t[4];
+#pragma unroll
+            for (int c = 0; c < 4; ++c) {
+                float v;
+                if (I32FULL) {
+                    v = static_cast<float>(static_cast<int32_t>(w0[c] + w1[c] + w2[c] + w3[c])) * rowm[i];
+                    v = v * coln[j][c];
+                    if (g.post_scale != 0.0f) v = __uint_as_float(f32_to_bf16_bits(v) << 16) * g.post_scale;
+                } else {
+                    v = __uint_as_float(w0[c]) + __uint_as_float(w1[c]);
+                    v = v + __uint_as_float(w2[c]);
+                    v = v + __uint_as_float(w3[c]);
+                    if (row_part) v = v * rowm[i];
+                    if (col_part) v = v * coln[j][c];
+                    if (g.out_scale != 1.0f) v = v * g.out_scale;
+                }
+                t[c] = v;
+            }
+            uint2 o;
+            o.x = pack_bf16x2(t[0], t[1]);
+            o.y = pack_bf16x2(t[2], t[3]);
+            if (g.bias) {
+                o.x = add_bf16x2(o.x, bias_lo[j]);
+                o.y = add_bf16x2(o.y, bias_hi[j]);
+            }
+            *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.C) + (int64_t)batch * g.bsc + (int64_t)(m0 + i * 32 + e_row) * g.ldc + n0 + j * 32 + e_col) = o;
         }
-        t[c] = v;
     }
-    uint2 o;
-    o.x = pack_bf16x2(t[0], t[1]);
-    o.y = pack_bf16x2(t[2], t[3]);
-    if (g.bias) {
-        o.x = add_bf16x2(o.x, bias_lo);
-        o.y = add_bf16x2(o.y, bias_hi);
-    }
-    *reinterpret_cast<uint2*>(reinterpret_cast<uint16_t*>(g.C) + (int64_t)batch * g.bsc + (int64_t)(m0 + e_row) * g.ldc + n0 + e_col) = o;
 }
 
-template <bool I32FULL>
+template <bool I32FULL, int BLOCKS>
 __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g) {
-    wavering_block<I32FULL>(g, blockIdx.x, blockIdx.y);
+    wavering_block<I32FULL, BLOCKS>(g, blockIdx.x, blockIdx.y);
 }
 
 // A GEMM over few K tiles: dW of a step on up to 256 tokens.  Its products are nothing beside its output, so this is made for
@@ -403,14 +451,17 @@ __device__ __forceinline__ void thin_walk(const GemmArgs& args, const int worker
 // The GEMMs of a step, or of its backward, on few tokens (batch of one each) in one launch: Y and dX, which have few blocks each
 // and wait for their loads most of the time, and with m.count > few dW behind them, a workgroup per CU.
 template <bool I32FULL>
-__global__ __launch_bounds__(256) void gemm_i8_few_kernel(const GemmMulti m, const int few) {
+__global__ __launch_bounds__(256) void gemm_i8_few_kernel(const GemmMulti m, const int few, const bool wide) {
     const int i = idx::gemm_multi_pick((int)blockIdx.x, m.first[1], m.first[2], m.count);
-    if (i < few) wavering_block<I32FULL>(m.g[i], (int)blockIdx.x - m.first[i], 0);
-    else {
-        const int worker = (int)blockIdx.x - m.first[i], workers = (int)gridDim.x - m.first[i];
-        if (I32FULL || m.g[i].sa.mode == TI8_SCALE_ROW) thin_walk<I32FULL, true>(m.g[i], worker, workers);
-        else thin_walk<I32FULL, I32FULL>(m.g[i], worker, workers);
+    const int block = (int)blockIdx.x - m.first[i];
+    if (i < few) {
+        if (wide) wavering_block<I32FULL, 2>(m.g[i], block, 0);
+        else wavering_block<I32FULL, 1>(m.g[i], block, 0);
+        return;
     }
+    const int workers = (int)gridDim.x - m.first[i];
+    if (I32FULL || m.g[i].sa.mode == TI8_SCALE_ROW) thin_walk<I32FULL, true>(m.g[i], block, workers);
+    else thin_walk<I32FULL, I32FULL>(m.g[i], block, workers);
 }
 
 bool skinny_supported(const GemmArgs& a) {
@@ -427,51 +478,69 @@ bool thin_supported(const GemmArgs& a, bool i32_full) {
     return (int64_t)(a.M / 128) * (a.N / 128) <= 0x3fffffff;
 }
 
-constexpr size_t WAVERING_LDS_BYTES = (size_t)4 * WS_STAGES * WS_STAGE_BYTES;
-static_assert(WAVERING_LDS_BYTES >= (size_t)2 * 2 * THIN_OPERAND, "the tiles of dW share the launch");
+constexpr int wavering_lds_bytes(bool wide) { return 4 * WS_STAGES * 2 * (wide ? 64 : 32) * 128; }
+static_assert(wavering_lds_bytes(false) >= 2 * 2 * THIN_OPERAND, "the tiles of dW share the launch");
+
+static bool is_wide(const GemmArgs& a, int64_t batch) { return idx::few_rows_wide(a.M, a.N, a.K, batch, device_cu_count()); }
+static int64_t wavering_blocks(const GemmArgs& a, bool wide) { return wide ? (int64_t)(a.N / 64) * ((a.M + 63) / 64) : (int64_t)(a.N / 32) * (a.M / 32); }
 
 int init_skinny_kernels() {
-    static OncePerDevice once_i32, once_promote, once_i32_multi, once_promote_multi;
-    hipError_t e = raise_lds_limit(once_i32, reinterpret_cast<const void*>(gemm_i8_wavering_kernel<true>), (int)WAVERING_LDS_BYTES);
-    if (e == hipSuccess) e = raise_lds_limit(once_promote, reinterpret_cast<const void*>(gemm_i8_wavering_kernel<false>), (int)WAVERING_LDS_BYTES);
-    if (e == hipSuccess) e = raise_lds_limit(once_i32_multi, reinterpret_cast<const void*>(gemm_i8_few_kernel<true>), (int)WAVERING_LDS_BYTES);
-    if (e == hipSuccess) e = raise_lds_limit(once_promote_multi, reinterpret_cast<const void*>(gemm_i8_few_kernel<false>), (int)WAVERING_LDS_BYTES);
-    if (e != hipSuccess) return fail(TI8_ERR_HIP, "gemm: cannot raise the LDS limit to %zu: %s", WAVERING_LDS_BYTES, hipGetErrorString(e));
+    static OncePerDevice all;
+    const uint64_t bit = 1ull << (current_device() & 63);
+    if (all.done.load(std::memory_order_acquire) & bit) return TI8_OK;
+    const void* const kernels[] = {reinterpret_cast<const void*>(gemm_i8_wavering_kernel<false, 2>), reinterpret_cast<const void*>(gemm_i8_wavering_kernel<true, 2>),
+                                   reinterpret_cast<const void*>(gemm_i8_few_kernel<false>), reinterpret_cast<const void*>(gemm_i8_few_kernel<true>)};
+    for (const void* k : kernels) {
+        OncePerDevice once;
+        const hipError_t e = raise_lds_limit(once, k, wavering_lds_bytes(true));
+        if (e != hipSuccess) return fail(TI8_ERR_HIP, "gemm: cannot raise the LDS limit to %d: %s", wavering_lds_bytes(true), hipGetErrorString(e));
+    }
+    static_assert(wavering_lds_bytes(false) <= 64 * 1024, "one block needs no raised limit");
+    all.done.fetch_or(bit, std::memory_order_release);
     return TI8_OK;
 }
 
-static int launch_wavering(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t st) {
-    constexpr size_t shmem = WAVERING_LDS_BYTES;
+int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t st) {
     if (int e = init_skinny_kernels()) return e;
-    dim3 grid((unsigned)((a.N / 32) * (a.M / 32)), (unsigned)batch), block(256);
-    if (i32_full)
-        hipLaunchKernelGGL(gemm_i8_wavering_kernel<true>, grid, block, shmem, st, a);
-    else
-        hipLaunchKernelGGL(gemm_i8_wavering_kernel<false>, grid, block, shmem, st, a);
+    const bool wide = is_wide(a, batch);
+    const dim3 grid((unsigned)wavering_blocks(a, wide), (unsigned)batch);
+    const auto kernel = wide ? (i32_full ? gemm_i8_wavering_kernel<true, 2> : gemm_i8_wavering_kernel<false, 2>)
+                             : (i32_full ? gemm_i8_wavering_kernel<true, 1> : gemm_i8_wavering_kernel<false, 1>);
+    hipLaunchKernelGGL(kernel, grid, dim3(256), wavering_lds_bytes(wide), st, a);
     note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
     return check_launch("ti8_gemm_i8_nt");
 }
 
-int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t st) {
-    return launch_wavering(a, batch, i32_full, st);
-}
-
-int launch_few(GemmMulti& m, int few, bool i32_full, hipStream_t st) {
-    if (int e = init_skinny_kernels()) return e;
+static int launch_few_group(GemmMulti& m, int few, bool wide, bool i32_full, hipStream_t st) {
     int64_t total = 0;
     const int64_t cus = device_cu_count();
     for (int i = 0; i < m.count; ++i) {
         m.first[i] = (int)total;
         const int64_t tiles = (int64_t)(m.g[i].N / 128) * (m.g[i].M / 128);
-        total += i < few ? (int64_t)(m.g[i].N / 32) * (m.g[i].M / 32) : tiles < cus ? tiles : cus;
+        total += i < few ? wavering_blocks(m.g[i], wide) : tiles < cus ? tiles : cus;
         if (total > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "gemm: too many blocks");
     }
     for (int i = m.count; i <= GEMM_MULTI_MAX; ++i) m.first[i] = (int)total;
     for (int i = m.count; i < GEMM_MULTI_MAX; ++i) m.g[i] = m.g[0];
     const auto kernel = i32_full ? gemm_i8_few_kernel<true> : gemm_i8_few_kernel<false>;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), WAVERING_LDS_BYTES, st, m, few);
+    hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), wavering_lds_bytes(wide), st, m, few, wide);
     note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
     return check_launch("ti8_gemm_i8_nt");
+}
+
+int launch_few(GemmMulti& m, int few, bool i32_full, hipStream_t st) {
+    if (int e = init_skinny_kernels()) return e;
+    bool wide[GEMM_MULTI_MAX] = {false, false, false};
+    int wides = 0;
+    for (int i = 0; i < few; ++i) wides += wide[i] = is_wide(m.g[i], 1);
+    if (wides == 0 || wides == few) return launch_few_group(m, few, wides != 0, i32_full, st);
+    // both kinds: four blocks in a launch of their own, whose LDS would leave the others one to a CU (100 tokens, 2048 -> 8192, double
+    // channel: the step 71 us in one launch)
+    GemmMulti four, rest;
+    four.count = rest.count = 0;
+    for (int i = 0; i < m.count; ++i) (wide[i] ? four.g[four.count++] : rest.g[rest.count++]) = m.g[i];
+    if (int e = launch_few_group(four, four.count, true, i32_full, st)) return e;
+    return launch_few_group(rest, few - wides, false, i32_full, st);
 }
 
 }  // namespace ti8

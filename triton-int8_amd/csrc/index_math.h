@@ -417,15 +417,27 @@ TI8_HD void gemm_configs_together(const int64_t (*shape)[3], int count, bool lar
         c[i] = big < small ? GemmConfig{256, 256, 2, 4, i32 ? 1 : 5, 0} : GemmConfig{128, 128, 2, 2, i32 ? 1 : 2, 0};
 }
 
-// Up to 256 rows: whether the medium-size kernel beats the few-rows kernel.  The latter's time grows with the bytes its 32 x
-// 32 blocks pull into LDS (0.52 ns per block and K tile on 256 CUs: N = 4096 with 128 rows 10.5 us at K = 4096, 32 us at K = 14336;
-// N = 14336, K = 4096: 31 us at 128 rows, 50 at 256), the former's with the K tiles a workgroup walks (0.85 us per two of them
-// alone, 1.15 with all CUs busy; N = 14336, K = 4096: 22 us at 128 rows, 27 at 256).
+// Up to 256 rows: us that the few-rows kernel takes with workgroups of one 32 x 32 block or of four.  Bound by the bytes of both
+// operands that pass into a CU's LDS, 55 per ns; workgroups of one block are two to a CU and leave no last round to wait for, those of
+// four are alone on theirs (and a further round costs 6 us more: waiting for its first loads, and the sums of the four waves).
+TI8_HD double few_rows_time(int64_t M, int64_t N, int64_t K, int64_t batch, int num_cu, bool wide) {
+    const int64_t groups = (wide ? ((M + 63) / 64) * (N / 64) : ((M + 31) / 32) * (N / 32)) * batch;
+    const double rounds = wide ? (double)((groups + num_cu - 1) / num_cu) : groups > num_cu ? (double)groups / num_cu : 1.0;
+    return 2.0 + rounds * (wide ? 128.0 : 64.0) * (double)K / 55000.0 + (wide ? 6.0 * (rounds - 1.0) : 0.0);
+}
+// Whether four blocks are the faster ones; over 9 weights and 32 to 256 rows the choice is 0.5 % behind the better of both, and 8 % ahead
+// of one block everywhere.  Equal times go to four: training launches Y and dX together, where one block's two to a CU are taken.
+TI8_HD bool few_rows_wide(int64_t M, int64_t N, int64_t K, int64_t batch, int num_cu) {
+    return M > 32 && few_rows_time(M, N, K, batch, num_cu, true) <= few_rows_time(M, N, K, batch, num_cu, false);
+}
+
+// Up to 256 rows: whether the medium-size kernel beats the few-rows kernel.  Its time grows with the K tiles a workgroup walks (0.85 us
+// per two of them alone, 1.15 with all CUs busy; N = 14336, K = 4096: 25 us at 128 rows, 26 at 256, where the few-rows kernel takes 27
+// and 46).
 TI8_HD bool gemm_few_rows_prefers_mid(int64_t M, int64_t N, int64_t K, int64_t batch, int num_cu) {
-    const double nk = (double)(K >> 7), blocks = (double)((N / 32) * (M / 32) * batch) * 256.0 / num_cu;
-    const double tiles = (double)(((M + 127) / 128) * (N / 128) * batch) / num_cu;
+    const double nk = (double)(K >> 7), tiles = (double)(((M + 127) / 128) * (N / 128) * batch) / num_cu;
     if (tiles > 1.0 || K > 256 * 128) return false;
-    return 7.0 + 0.5 * nk * (0.85 + 0.3 * tiles) < 2.0 + 0.00052 * blocks * nk;
+    return 7.0 + 0.5 * nk * (0.85 + 0.3 * tiles) < few_rows_time(M, N, K, batch, num_cu, few_rows_wide(M, N, K, batch, num_cu));
 }
 
 }  // namespace idx

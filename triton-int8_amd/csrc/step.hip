@@ -331,8 +331,9 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
         few[i] = g[i];
         if (i + 1 < count || !L.bwd) few[i].M = live_rows(g[i].K);      // dW, the last of a backward, has one row per output feature
     }
-    bool launched[3];
-    if (int e = gemm_nt_few(few, count, L.bwd, bias, flags, launched, stream)) return e;
+    bool launched[3] = {false, false, false};
+    if (count > 1)
+        if (int e = gemm_nt_few(few, count, L.bwd, bias, flags, launched, stream)) return e;
     for (int i = 0; i < count; ++i)
         if (!launched[i])
             if (int e = one_gemm(few[i], i == 0 ? bias : nullptr, L.tokens, flags, stream)) return e;
