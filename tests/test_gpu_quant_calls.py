@@ -1,0 +1,64 @@
+"""The quantisers of a layer call in two launches (partial maxima, conversion), against the operands quantised one by one: the same bits."""
+import pytest
+import torch
+
+from conftest import make_gen, randn_bf16
+
+pytestmark = pytest.mark.gpu
+
+
+# one tile each way; parts of one tile; parts of several tiles, the last one shorter (more than 4096 rows or columns), both ways; ragged tokens;
+# operands beyond the Infinity Cache, which go by the atomics form
+@pytest.mark.parametrize("scheme", ["block_channel", "row_block", "double_channel"])
+@pytest.mark.parametrize("tokens,k,n", [(300, 128, 384), (1001, 1152, 640), (4300, 384, 512), (290, 8320, 4224), (9000, 256, 384), (270, 13312, 13056)])
+def test_step_quantised_in_two_launches(dev, monkeypatch, tokens, k, n, scheme):
+    import triton_int8_amd as T
+    g = torch.Generator(device=dev).manual_seed(tokens + k + n)
+    rand = lambda *s: torch.randn(*s, generator=g, device=dev).to(torch.bfloat16)
+    X, W, dY = rand(tokens, k), rand(n, k), rand(tokens, n)
+    X[:, k // 3] *= 40.0        # maxima that sit in one column, one row, the last tile
+    W[n - 1] *= 7.0
+    dY[tokens - 1, n - 1] = 1e4
+    X[tokens // 2, 5] = float("inf")
+    got = T.linear_fwd_bwd(X, W, dY, scheme)
+    x, w = X.clone().requires_grad_(True), W.clone().requires_grad_(True)
+    y = T.Int8LinearFunction.apply(x, w, None, scheme, None)
+    layer = (y.detach(), *torch.autograd.grad(y, (x, w), dY))
+    monkeypatch.setattr(T.linear, "ONE_CALL_STEP", False)
+    want = T.linear_fwd_bwd(X, W, dY, scheme)
+    for name, a, b, c in zip(("Y", "dX", "dW"), got, layer, want):
+        torch.testing.assert_close(a, c, rtol=0, atol=0, equal_nan=True, msg=name)
+        torch.testing.assert_close(b, c, rtol=0, atol=0, equal_nan=True, msg=name)
+
+
+def test_nan_is_left_out_of_partial_maxima(dev, monkeypatch):
+    import triton_int8_amd as T
+    g = make_gen(5)
+    X, W, dY = randn_bf16(g, 400, 256).to(dev), randn_bf16(g, 384, 256).to(dev), randn_bf16(g, 400, 384).to(dev)
+    X[3] = float("nan")
+    W[:, 7] = float("nan")
+    dY[17, 5] = float("nan")
+    got = T.linear_fwd_bwd(X, W, dY, "double_channel")
+    monkeypatch.setattr(T.linear, "ONE_CALL_STEP", False)
+    for a, c in zip(got, T.linear_fwd_bwd(X, W, dY, "double_channel")):
+        torch.testing.assert_close(a, c, rtol=0, atol=0, equal_nan=True)
+
+
+@pytest.mark.parametrize("scheme", ["block_channel", "double_channel"])
+@pytest.mark.parametrize("layout", ["in place", "strided"])
+def test_step_into_given_outputs(dev, scheme, layout):
+    """Outputs hold the partial maxima until the conversion has read them: not where they are the inputs' memory, or not dense."""
+    import triton_int8_amd as T
+    g = make_gen(9)
+    M, K, N = 384, 640, 512
+    X, W, dY = randn_bf16(g, M, K).to(dev), randn_bf16(g, N, K, std=0.02).to(dev), randn_bf16(g, M, N, std=1e-3).to(dev)
+    want = T.linear_fwd_bwd(X, W, dY, scheme)
+    if layout == "in place":
+        out = (dY.clone(), X.clone(), W.clone())
+        got = T.ops.linear_step(out[1], out[2], out[0], scheme, out=out)
+    else:
+        out = tuple(torch.full((r, c + 64), -3.0, dtype=torch.bfloat16, device=dev)[:, :c] for r, c in ((M, N), (M, K), (N, K)))
+        got = T.ops.linear_step(X, W, dY, scheme, out=out)
+        assert all(bool((torch.as_strided(o, (o.shape[0], 64), (o.stride(0), 1), o.storage_offset() + o.shape[1]) == -3.0).all()) for o in out)
+    for a, b in zip(got, want):
+        assert torch.equal(a, b)

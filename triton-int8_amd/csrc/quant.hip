@@ -152,7 +152,7 @@ __device__ __forceinline__ void quant_block_tile(
 #pragma unroll
             for (int j = 0; j < 4; ++j) o[h][j] = quant8<ARITH>(v[u][h][j], scale);
 
-        if (WRITE_Q) {
+        if (WRITE_Q && q) {
             char* qt = reinterpret_cast<char*>(q + idx::qblock_origin(b, bsq, rb, ldq, cb, 128 * NSUB));
             const uint32_t q_first = (uint32_t)idx::qblock_row(tid, 0, 0) * (uint32_t)ldq + (uint32_t)idx::qblock_col(tid) + (uint32_t)(u * 128);
 #pragma unroll
@@ -161,7 +161,7 @@ __device__ __forceinline__ void quant_block_tile(
                 for (int j = 0; j < 4; ++j)
                     *reinterpret_cast<uint2*>(qt + (q_first + (uint32_t)idx::qblock_row(0, h, j) * (uint32_t)ldq)) = o[h][j];
         }
-        if (WRITE_QT) {  // NSUB == 1 only (checked on the host)
+        if (WRITE_QT && qT) {  // NSUB == 1 only (checked on the host)
 #pragma unroll
             for (int h = 0; h < 2; ++h)
             {
@@ -221,26 +221,24 @@ struct QBlockMulti {
     QBlockOperand op[QBLOCK_MULTI_MAX];
     int first[QBLOCK_MULTI_MAX + 1];   // first workgroup of operand i; first[count] = grid size
     int count;
-    unsigned int* clear;               // words that the launch zeroes on the side (thread i of the grid clears word i), or NULL
-    int clear_words;
 };
+
+template <bool WRITE_Q, bool WRITE_QT>
+__device__ __forceinline__ void quant_block_of(const QBlockMulti& m, const int block, const QMode& mode, float* red4, uint32_t* tileT) {
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < QBLOCK_MULTI_MAX; ++k)
+        if (k < m.count && block >= m.first[k]) i = k;
+    const QBlockOperand& o = m.op[i];
+    quant_block_tile<1, WRITE_Q, WRITE_QT, ARITH_KERNEL>(o.x, o.bsx, o.ldx, o.q, o.bsq, o.ldq, o.qT, o.bsqt, o.ldqt, o.s, o.ssb, o.ssr,
+                                                         o.ssc, o.nrb, o.ncb, o.valid_rows, mode, block - m.first[i], red4, tileT);
+}
 
 template <bool WRITE_Q, bool WRITE_QT>
 __global__ __launch_bounds__(256) void quant_block_multi_kernel(const QBlockMulti m, QMode mode) {
     __shared__ float red4[4];
     __shared__ uint32_t tileT[WRITE_QT ? 128 * 33 : 1];
-    {   // the next launch's maxima workspace, cleared here so that no launch exists only to clear it
-        const int64_t w = (int64_t)blockIdx.x * 256 + threadIdx.x;
-        if (w < m.clear_words) m.clear[w] = 0u;
-    }
-    int i = 0;
-#pragma unroll
-    for (int k = 1; k < QBLOCK_MULTI_MAX; ++k)
-        if (k < m.count && (int)blockIdx.x >= m.first[k]) i = k;
-    const QBlockOperand& o = m.op[i];
-    const int local = (int)blockIdx.x - m.first[i];
-    quant_block_tile<1, WRITE_Q, WRITE_QT, ARITH_KERNEL>(o.x, o.bsx, o.ldx, o.q, o.bsq, o.ldq, o.qT, o.bsqt, o.ldqt, o.s, o.ssb, o.ssr,
-                                                         o.ssc, o.nrb, o.ncb, o.valid_rows, mode, local, red4, tileT);
+    quant_block_of<WRITE_Q, WRITE_QT>(m, (int)blockIdx.x, mode, red4, tileT);
 }
 
 
@@ -432,9 +430,17 @@ __global__ __launch_bounds__(256) void quant_row_kernel(const uint16_t* __restri
     }
 }
 
-__global__ void fill_u32_kernel(unsigned int* p, int n, unsigned int v) {
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) p[i] = v;
+struct ClearRanges {    // words to zero, one behind the other
+    unsigned int* p[3];
+    int n[3];
+};
+__global__ void clear_kernel(const ClearRanges r) {
+    int i = blockIdx.x * blockDim.x + threadIdx.x;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        if (i >= 0 && i < r.n[k]) r.p[k][i] = 0u;
+        i -= r.n[k];
+    }
 }
 
 // Quantise a 128x128 tile of x with one scale PER COLUMN (from ws[]) and write it
@@ -622,18 +628,12 @@ __global__ __launch_bounds__(256) void absmax_kernel(const uint16_t* __restrict_
 }
 
 // Quantise a 128x128 tile of x twice: with one scale per ROW into q (same orientation) and
-// with one scale per COLUMN into qT (transposed).  Thread <-> element map of quant_block_kernel.
-__global__ __launch_bounds__(256) void quant_rowcol_kernel(const uint16_t* __restrict__ x, int64_t ldx,
-                                                           int8_t* __restrict__ q, int64_t ldq,
-                                                           float* __restrict__ s_row, int8_t* __restrict__ qT,
-                                                           int64_t ldqt, float* __restrict__ s_col,
-                                                           const float* __restrict__ ws_row,
-                                                           const float* __restrict__ ws_col,
-                                                           float* __restrict__ ws_next, int64_t R, int ncb, int valid_rows, QMode mode) {
-    __shared__ uint32_t tileT[128 * 33];
-    __shared__ __attribute__((aligned(16))) float sc[256];  // [0,128): row scales, [128,256): column scales
-    const int cb = blockIdx.x % ncb;
-    const int rb = blockIdx.x / ncb;
+// with one scale per COLUMN into qT (transposed).  Thread <-> element map of quant_block_kernel.  amax_of() = the absmax of this thread's
+// row (threads 0 .. 127) or column (128 .. 255) of the tile, asked for behind the tile's loads.
+template <class AmaxOf>
+__device__ __forceinline__ void quant_rowcol_tile(const uint16_t* __restrict__ x, int64_t ldx, int8_t* __restrict__ q, int64_t ldq,
+                                                  float* __restrict__ s_row, int8_t* __restrict__ qT, int64_t ldqt, float* __restrict__ s_col,
+                                                  int rb, int cb, int valid_rows, const QMode& mode, uint32_t* tileT, float* sc, AmaxOf amax_of) {
     const int tid = threadIdx.x;
     const int cc = tid & 15, rg = tid >> 4;
     const uint16_t* xt = x + (int64_t)rb * 128 * ldx + (int64_t)cb * 128;
@@ -661,9 +661,7 @@ __global__ __launch_bounds__(256) void quant_rowcol_kernel(const uint16_t* __res
         const bool is_row = tid < 128;
         const int idx = tid & 127;
         const int64_t at = is_row ? (int64_t)rb * 128 + idx : (int64_t)cb * 128 + idx;
-        // two-part workspace: clear the part that the next call will collect its maxima in
-        if (ws_next && (is_row ? cb == 0 : rb == 0)) ws_next[is_row ? at : R + at] = 0.0f;
-        const float amax = amax_floor(is_row ? ws_row[at] : ws_col[at], mode.eps_add);
+        const float amax = amax_floor(amax_of(is_row, idx, at), mode.eps_add);
         const float scale = 127.0f / amax;
         sc[tid] = scale;
         if (is_row ? cb == 0 : rb == 0) (is_row ? s_row : s_col)[at] = stored_scale(amax, scale, mode);
@@ -703,6 +701,192 @@ __global__ __launch_bounds__(256) void quant_rowcol_kernel(const uint16_t* __res
     }
 }
 
+__global__ __launch_bounds__(256) void quant_rowcol_kernel(const uint16_t* __restrict__ x, int64_t ldx,
+                                                           int8_t* __restrict__ q, int64_t ldq,
+                                                           float* __restrict__ s_row, int8_t* __restrict__ qT,
+                                                           int64_t ldqt, float* __restrict__ s_col,
+                                                           const float* __restrict__ ws_row,
+                                                           const float* __restrict__ ws_col,
+                                                           float* __restrict__ ws_next, int64_t R, int ncb, int valid_rows, QMode mode) {
+    __shared__ uint32_t tileT[128 * 33];
+    __shared__ __attribute__((aligned(16))) float sc[256];  // [0,128): row scales, [128,256): column scales
+    const int cb = blockIdx.x % ncb, rb = blockIdx.x / ncb;
+    quant_rowcol_tile(x, ldx, q, ldq, s_row, qT, ldqt, s_col, rb, cb, valid_rows, mode, tileT, sc, [&](bool is_row, int, int64_t at) {
+        // two-part workspace: clear the part that the next call will collect its maxima in
+        if (ws_next && (is_row ? cb == 0 : rb == 0)) ws_next[is_row ? at : R + at] = 0.0f;
+        return is_row ? ws_row[at] : ws_col[at];
+    });
+}
+
+// ---------------------------------------------------------------------------------
+// The quantisers of a layer call in two launches.  An operand that is needed by rows and by columns takes two passes over it, the
+// maxima and the conversion; launched operand by operand these are many short kernels (and one that only clears the maxima).  Here
+// the maxima of all such operands are one launch, together with the block-quantised operands of the call, and the conversions the next.
+// The maxima need no clearing: a workgroup stores those of its rows and of its columns (16 bits each: patterns of |bf16|) beside the other
+// workgroups', at most about 32 of either (quant_maxima_tiles), and the conversion of a 128 x 128 tile takes the largest of what
+// belongs to it, 16 KiB at most from the L2.
+//   rows [nct][R], cols [nrt][C]: maxima over the columns of part ct, over the rows of part rt; a part is tr (tc) times 128
+struct MaxOperand {
+    const uint16_t* x;
+    int64_t ldx;
+    uint16_t *rows, *cols;
+    int8_t* q;          // conversion: by rows, and transposed by columns
+    int64_t ldq;
+    float* s_row;
+    int8_t* qT;
+    int64_t ldqt;
+    float* s_col;
+    int R, C, valid_rows, tr, tc, nrt, nct;
+};
+constexpr int MAX_OPERANDS = 3;
+struct MaxMulti {
+    MaxOperand op[MAX_OPERANDS];
+    int first[MAX_OPERANDS + 1];
+    int count;
+};
+
+// Thread t reads the chunk t % 16 of rows 8 (t / 16) .. + 7 of every 128 x 128 tile of its part
+__device__ __forceinline__ void maxima_part(const MaxOperand& o, const int part, uint16_t* rowmax, uint4 (&colpart)[4][16]) {
+    const int ct = part % o.nct, rt = part / o.nct;
+    const int tid = threadIdx.x, cc = tid & 15, rg = tid >> 4;
+    const int rtiles = min(o.tr, (o.R >> 7) - rt * o.tr), ctiles = min(o.tc, (o.C >> 7) - ct * o.tc);
+    for (int b = 0; b < ctiles; ++b) {
+        const int c0 = (ct * o.tc + b) * 128 + cc * 8;
+        uint32_t m[4] = {ABS_BIAS2, ABS_BIAS2, ABS_BIAS2, ABS_BIAS2};
+        for (int a = 0; a < rtiles; ++a) {
+            const int r0 = (rt * o.tr + a) * 128 + rg * 8;
+            const uint16_t* const xr = o.x + (int64_t)r0 * o.ldx + c0;
+            uint4 v[8];
+            if (r0 + 8 <= o.valid_rows) {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) v[i] = *reinterpret_cast<const uint4*>(xr + i * o.ldx);
+            } else {
+#pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    v[i] = make_uint4(0u, 0u, 0u, 0u);
+                    if (r0 + i < o.valid_rows) v[i] = *reinterpret_cast<const uint4*>(xr + i * o.ldx);
+                }
+            }
+            uint32_t rm[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) {
+                const uint32_t a0 = abs_biased2(v[i].x), a1 = abs_biased2(v[i].y), a2 = abs_biased2(v[i].z), a3 = abs_biased2(v[i].w);
+                m[0] = pk_max_i16(m[0], a0);
+                m[1] = pk_max_i16(m[1], a1);
+                m[2] = pk_max_i16(m[2], a2);
+                m[3] = pk_max_i16(m[3], a3);
+                rm[i] = pk_max_i16(pk_max_i16(a0, a1), pk_max_i16(a2, a3));
+            }
+            // over the 16 lanes that hold the same rows
+#pragma unroll
+            for (int i = 0; i < 8; ++i) rm[i] = dpp_pk_max_i16<0xB1>(rm[i]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) rm[i] = dpp_pk_max_i16<0x4E>(rm[i]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) rm[i] = dpp_pk_max_i16<0x141>(rm[i]);
+#pragma unroll
+            for (int i = 0; i < 8; ++i) rm[i] = dpp_pk_max_i16<0x140>(rm[i]);
+            if (cc == 0) {      // the same thread for these rows in every column tile: no barrier
+                uint32_t w[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) w[i] = unbias_max2(rm[2 * i]) | (unbias_max2(rm[2 * i + 1]) << 16);
+                uint4* const at = reinterpret_cast<uint4*>(rowmax + a * 128 + rg * 8);
+                if (b) {
+                    const uint4 old = *at;
+                    w[0] = pk_max_i16(w[0], old.x); w[1] = pk_max_i16(w[1], old.y); w[2] = pk_max_i16(w[2], old.z); w[3] = pk_max_i16(w[3], old.w);
+                }
+                *at = make_uint4(w[0], w[1], w[2], w[3]);
+            }
+        }
+        // columns: over the 16 threads of a chunk, four in a wave
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+            const auto r16 = __builtin_amdgcn_permlane16_swap(m[k], m[k], false, false);
+            m[k] = pk_max_i16(r16[0], r16[1]);
+            const auto r32 = __builtin_amdgcn_permlane32_swap(m[k], m[k], false, false);
+            m[k] = pk_max_i16(r32[0], r32[1]);
+        }
+#endif
+        if ((tid & 63) < 16) colpart[tid >> 6][cc] = make_uint4(m[0], m[1], m[2], m[3]);
+        __syncthreads();
+        if (tid < 64) {     // dword t: columns 2 t, 2 t + 1
+            const uint32_t* const pw = reinterpret_cast<const uint32_t*>(colpart);
+            const uint32_t u = pk_max_i16(pk_max_i16(pw[tid], pw[64 + tid]), pk_max_i16(pw[128 + tid], pw[192 + tid]));
+            const int lo = static_cast<short>(u & 0xffffu), hi = static_cast<short>(u >> 16);
+            reinterpret_cast<uint32_t*>(o.cols + (int64_t)rt * o.C + (ct * o.tc + b) * 128)[tid] =
+                (uint32_t)(max(lo, 0x7f) - 0x7f) | ((uint32_t)(max(hi, 0x7f) - 0x7f) << 16);
+        }
+        __syncthreads();
+    }
+    if (cc == 0)
+        for (int a = 0; a < rtiles; ++a)
+            *reinterpret_cast<uint4*>(o.rows + (int64_t)ct * o.R + (rt * o.tr + a) * 128 + rg * 8) = *reinterpret_cast<const uint4*>(rowmax + a * 128 + rg * 8);
+}
+
+constexpr int MAXIMA_ROW_TILES = 64;     // 128-row tiles whose row maxima a workgroup keeps in LDS
+__global__ __launch_bounds__(256) void quant_first_kernel(const MaxMulti maxima, const QBlockMulti blocks, QMode mode) {
+    __shared__ float red4[4];
+    __shared__ __attribute__((aligned(16))) uint32_t tileT[128 * 33];
+    __shared__ uint4 colpart[4][16];
+    static_assert(MAXIMA_ROW_TILES * 128 * 2 <= (int)sizeof(tileT), "row maxima share the transposed tile's LDS");
+    const int block_tiles = blocks.first[QBLOCK_MULTI_MAX], part = (int)blockIdx.x - block_tiles;
+    if (part < 0) {
+        if ((int)blockIdx.x < blocks.first[blocks.count]) quant_block_of<true, true>(blocks, (int)blockIdx.x, mode, red4, tileT);
+    } else {
+        int i = 0;
+#pragma unroll
+        for (int k = 1; k < MAX_OPERANDS; ++k)
+            if (k < maxima.count && part >= maxima.first[k]) i = k;
+        const MaxOperand& o = maxima.op[i];
+        if (part - maxima.first[i] < o.nrt * o.nct) maxima_part(o, part - maxima.first[i], reinterpret_cast<uint16_t*>(tileT), colpart);
+    }
+}
+
+__global__ __launch_bounds__(256) void quant_rowcol_multi_kernel(const MaxMulti m, QMode mode) {
+    __shared__ uint32_t tileT[128 * 33];
+    __shared__ __attribute__((aligned(16))) float sc[256];
+    __shared__ uint4 part[2][4][16];    // [rows, columns][wave][chunk]
+    // from the end of the last operand to the beginning of the first, and every tile on the XCD that took its maxima where a part is one
+    // tile: what the launch before read last is still in the caches (4096 x 4096 behind its maxima: 13 us, 16 on another XCD)
+    const int tile = (int)((gridDim.x >> 3) - 1 - (blockIdx.x >> 3)) * 8 + (int)(blockIdx.x & 7);
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < MAX_OPERANDS; ++k)
+        if (k < m.count && tile >= m.first[k]) i = k;
+    const MaxOperand& o = m.op[i];
+    const int ncb = o.C >> 7, local = tile - m.first[i];
+    const int cb = local % ncb, rb = local / ncb;
+    if (rb >= o.R >> 7) return;         // operands start at multiples of 8 tiles
+    quant_rowcol_tile(o.x, o.ldx, o.q, o.ldq, o.s_row, o.qT, o.ldqt, o.s_col, rb, cb, o.valid_rows, mode, tileT, sc, [&](bool is_row, int index, int64_t) {
+        const int chunk = threadIdx.x & 15, p0 = threadIdx.x >> 4;
+#pragma unroll
+        for (int d = 0; d < 2; ++d) {
+            const uint16_t* const from = d ? o.cols + cb * 128 + chunk * 8 : o.rows + rb * 128 + chunk * 8;
+            const int64_t step = d ? o.C : o.R;
+            const int parts = d ? o.nrt : o.nct;
+            uint32_t w[4] = {0u, 0u, 0u, 0u};
+            for (int p = p0; p < parts; p += 16) {
+                const uint4 v = *reinterpret_cast<const uint4*>(from + p * step);
+                w[0] = pk_max_i16(w[0], v.x); w[1] = pk_max_i16(w[1], v.y); w[2] = pk_max_i16(w[2], v.z); w[3] = pk_max_i16(w[3], v.w);
+            }
+#if defined(__HIP_DEVICE_COMPILE__)
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                const auto r16 = __builtin_amdgcn_permlane16_swap(w[k], w[k], false, false);
+                w[k] = pk_max_i16(r16[0], r16[1]);
+                const auto r32 = __builtin_amdgcn_permlane32_swap(w[k], w[k], false, false);
+                w[k] = pk_max_i16(r32[0], r32[1]);
+            }
+#endif
+            if ((threadIdx.x & 63) < 16) part[d][threadIdx.x >> 6][chunk] = make_uint4(w[0], w[1], w[2], w[3]);
+        }
+        __syncthreads();
+        const uint16_t* const mine = reinterpret_cast<const uint16_t*>(part[is_row ? 0 : 1]) + index;
+        return __uint_as_float((uint32_t)max(max(mine[0], mine[128]), max(mine[256], mine[384])) << 16);
+    });
+}
+
 // arithmetic variant a flag set asks for (only ti8_quant_block and ti8_quant_row take the flags)
 static int arith_of(int qflags) {
     return (qflags & TI8_Q_TORCH_BF16) ? ARITH_TORCH_BF16 : ((qflags & TI8_Q_TORCH_ROUND) ? ARITH_TORCH_F32 : ARITH_KERNEL);
@@ -711,6 +895,12 @@ static int arith_of(int qflags) {
 }  // namespace ti8
 
 using namespace ti8;
+
+static void clear(const ClearRanges& r, hipStream_t st) {
+    const int64_t words = (int64_t)r.n[0] + r.n[1] + r.n[2];
+    hipLaunchKernelGGL(clear_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, r);
+}
+static void clear(unsigned int* p, int64_t words, hipStream_t st) { clear(ClearRanges{{p, p, p}, {(int)words, 0, 0}}, st); }
 
 // argument checks of one block-quantiser operand (shared by ti8_quant_block and ti8_quant_block_multi)
 static int check_qblock_operand(const char* fn, const void* x, int64_t bsx, int64_t ldx, const int8_t* q, int64_t bsq, int64_t ldq,
@@ -764,56 +954,152 @@ extern "C" int ti8_quant_block(const void* x, int64_t bsx, int64_t ldx, int8_t* 
 }
 
 extern "C" int ti8_quant_block_multi(const ti8_qblock_operand* operands, int count, int qflags, int inv_mode, ti8_stream_t stream) {
-    return ti8::quant_block_multi_and_clear(operands, nullptr, count, qflags, inv_mode, nullptr, 0, stream);
+    return ti8::quant_block_multi_valid(operands, nullptr, count, qflags, inv_mode, stream);
 }
 
-int ti8::fill_words(unsigned int* p, int64_t words, unsigned int value, hipStream_t st) {
-    if (words <= 0) return TI8_OK;
-    if (!p || words > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "fill: bad buffer");
-    hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)((words + 255) / 256)), dim3(256), 0, st, p, (int)words, value);
-    return check_launch("fill");
+// Maxima collected with atomics in [R rows][C columns] words that are zero, then the conversion
+static void launch_row_col(const uint16_t* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT, int64_t ldqt, float* s_col, unsigned int* ws,
+                           float* ws_next, int64_t R, int64_t valid_rows, int64_t C, const QMode& mode, hipStream_t st) {
+    const float* const maxima = reinterpret_cast<const float*>(ws);
+    hipLaunchKernelGGL((absmax_kernel<ABSMAX_ROWS, true>), dim3((unsigned)((C + 255) / 256), (unsigned)(R / ABSMAX_ROWS)), dim3(256), 0, st, x, ldx, ws, ws + R,
+                       valid_rows, (int)C);
+    hipLaunchKernelGGL(quant_rowcol_kernel, dim3((unsigned)((R / 128) * (C / 128))), dim3(256), 0, st, x, ldx, q, ldq, s_row, qT, ldqt, s_col, maxima, maxima + R,
+                       ws_next, R, (int)(C / 128), (int)valid_rows, mode);
 }
 
-int ti8::quant_block_multi_and_clear(const ti8_qblock_operand* operands, const int64_t* valid_rows, int count, int qflags, int inv_mode,
-                                     unsigned int* clear, int64_t clear_words, ti8_stream_t stream) {
+// Checks of the block-quantised operands of a launch and their kernel arguments
+static int block_operands(const char* fn, const ti8_qblock_operand* operands, const int64_t* valid_rows, int count, QBlockMulti* m, int64_t* total_out) {
+    int64_t total = 0;
+    for (int i = 0; i < count; ++i) {
+        const ti8_qblock_operand& o = operands[i];
+        if (int e = check_qblock_operand(fn, o.x, o.bsx, o.ldx, o.q, o.bsq, o.ldq, o.qT, o.bsqt, o.ldqt, o.s, o.B, o.R, o.C, 128)) return e;
+        m->op[i] = QBlockOperand{static_cast<const uint16_t*>(o.x), o.bsx, o.ldx, o.q, o.bsq, o.ldq, o.qT, o.bsqt, o.ldqt, o.s,
+                                 o.ssb, o.ssr, o.ssc, (int)(o.R / 128), (int)(o.C / 128), (int)(valid_rows ? valid_rows[i] : o.R)};
+        m->first[i] = (int)total;
+        total += o.B * (o.R / 128) * (o.C / 128);
+        if (total > 0x3fffffffLL) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
+    }
+    for (int i = count; i < QBLOCK_MULTI_MAX; ++i) { m->op[i] = count ? m->op[0] : QBlockOperand{}; m->first[i] = (int)total; }
+    m->first[QBLOCK_MULTI_MAX] = (int)total;
+    m->count = count;
+    *total_out = total;
+    return TI8_OK;
+}
+
+int ti8::quant_block_multi_valid(const ti8_qblock_operand* operands, const int64_t* valid_rows, int count, int qflags, int inv_mode, ti8_stream_t stream) {
     const char* fn = "ti8_quant_block_multi";
     QMode mode;
     if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
     if (qflags & TI8_Q_HAD128) return fail(TI8_ERR_MODE, "%s: the Hadamard rotation is not offered here", fn);
     if (!operands) return fail(TI8_ERR_NULL, "%s: operands is required", fn);
     if (count < 1 || count > QBLOCK_MULTI_MAX) return fail(TI8_ERR_SHAPE, "%s: between 1 and %d operands, got %d", fn, QBLOCK_MULTI_MAX, count);
+    for (int i = 0; i < count; ++i)
+        if ((operands[i].q != nullptr) != (operands[0].q != nullptr) || (operands[i].qT != nullptr) != (operands[0].qT != nullptr))
+            return fail(TI8_ERR_MODE, "%s: every operand must ask for the same outputs (q, qT or both)", fn);
     QBlockMulti m;
     int64_t total = 0;
-    for (int i = 0; i < count; ++i) {
-        const ti8_qblock_operand& o = operands[i];
-        if (int e = check_qblock_operand(fn, o.x, o.bsx, o.ldx, o.q, o.bsq, o.ldq, o.qT, o.bsqt, o.ldqt, o.s, o.B, o.R, o.C, 128)) return e;
-        if ((o.q != nullptr) != (operands[0].q != nullptr) || (o.qT != nullptr) != (operands[0].qT != nullptr))
-            return fail(TI8_ERR_MODE, "%s: every operand must ask for the same outputs (q, qT or both)", fn);
-        m.op[i] = QBlockOperand{static_cast<const uint16_t*>(o.x), o.bsx, o.ldx, o.q, o.bsq, o.ldq, o.qT, o.bsqt, o.ldqt, o.s,
-                                o.ssb, o.ssr, o.ssc, (int)(o.R / 128), (int)(o.C / 128), (int)(valid_rows ? valid_rows[i] : o.R)};
-        m.first[i] = (int)total;
-        total += o.B * (o.R / 128) * (o.C / 128);
-        if (total > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
-    }
-    for (int i = count; i < QBLOCK_MULTI_MAX; ++i) { m.op[i] = m.op[0]; m.first[i] = (int)total; }
-    m.first[QBLOCK_MULTI_MAX] = (int)total;
-    m.count = count;
+    if (int e = block_operands(fn, operands, valid_rows, count, &m, &total)) return e;
     hipStream_t st = static_cast<hipStream_t>(stream);
-    m.clear = nullptr;
-    m.clear_words = 0;
-    if (clear && clear_words > 0) {
-        if (clear_words <= total * 256) {
-            m.clear = clear;
-            m.clear_words = (int)clear_words;
-        } else if (int e = fill_words(clear, clear_words, 0u, st)) {   // more words than threads: a launch of its own
-            return e;
-        }
-    }
     dim3 grid((unsigned)total), block(256);
     const bool wq = operands[0].q != nullptr, wqt = operands[0].qT != nullptr;
     if (wq && wqt) hipLaunchKernelGGL((quant_block_multi_kernel<true, true>), grid, block, 0, st, m, mode);
     else if (wq) hipLaunchKernelGGL((quant_block_multi_kernel<true, false>), grid, block, 0, st, m, mode);
     else hipLaunchKernelGGL((quant_block_multi_kernel<false, true>), grid, block, 0, st, m, mode);
+    return check_launch(fn);
+}
+
+// 128 x 128 tiles per part in either direction: about 32 parts, and no more rows than a workgroup's LDS holds maxima of
+static void maxima_tiles(int64_t R, int64_t C, int* tr, int* tc) {
+    const int64_t a = (R / 128 + 31) / 32, b = (C / 128 + 31) / 32;
+    *tr = (int)(a < MAXIMA_ROW_TILES ? a : MAXIMA_ROW_TILES);
+    *tc = (int)b;
+}
+static int64_t round8(int64_t n) { return (n + 7) / 8 * 8; }     // ids 8 apart are workgroups of one XCD
+static int64_t parts_of(int64_t n, int t) { return (n / 128 + t - 1) / t; }
+
+// Up to here: beyond it the maxima of several operands push each other out of the Infinity Cache (256 MiB) before the conversions come,
+// and the shorter parts of the atomics form keep more loads in flight.  Steps, us, these two launches / the atomics form: 16 tokens 4096 ->
+// 4096 block-channel 37.6 / 41; 2000 tokens 4096 -> 4096 double-channel 125 / 138; 1000 tokens 14336 -> 8192 (268 MiB) 510 / 535; 2048
+// tokens 14336 -> 14336 block-channel (392 MiB) 1560 / 1549.
+constexpr int64_t TOGETHER_BYTES = (int64_t)320 << 20;
+
+int64_t ti8::quant_maxima_words(int64_t R, int64_t C) {
+    int tr, tc;
+    maxima_tiles(R, C, &tr, &tc);
+    return (parts_of(C, tc) * R + parts_of(R, tr) * C) / 2;
+}
+
+int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int64_t* block_rows, int nblocks, const QRowColOperand* both, int nboth, int qflags,
+                    int inv_mode, ti8_stream_t stream) {
+    bool same = true;
+    for (int i = 1; i < nblocks; ++i) same = same && !blocks[i].q == !blocks[0].q && !blocks[i].qT == !blocks[0].qT;
+    if (nblocks && !nboth && same) return quant_block_multi_valid(blocks, block_rows, nblocks, qflags, inv_mode, stream);
+    if (!nblocks && !nboth) return TI8_OK;
+    QMode mode;
+    if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
+    int64_t bytes = 0;
+    bool atomics = false;
+    for (int i = 0; i < nboth; ++i) {
+        bytes += both[i].R * both[i].C * 2;
+        atomics = atomics || !both[i].partial;
+    }
+    atomics = atomics || bytes > TOGETHER_BYTES;
+    if (nblocks >= QBLOCK_MULTI_MAX || nboth > MAX_OPERANDS || (qflags & TI8_Q_HAD128)) return fail(TI8_ERR_MODE, "%s: unsupported set of operands", fn);
+    QBlockMulti b;
+    int64_t block_tiles = 0;
+    if (int e = block_operands(fn, blocks, block_rows, nblocks, &b, &block_tiles)) return e;
+    b.first[nblocks] = (int)block_tiles;
+    block_tiles = round8(block_tiles);
+    b.first[QBLOCK_MULTI_MAX] = (int)block_tiles;
+    MaxMulti m;
+    int64_t parts = 0, tiles = 0, first_tile[MAX_OPERANDS + 1];
+    m.count = nboth;
+    for (int i = 0; i < nboth; ++i) {
+        const QRowColOperand& o = both[i];
+        if (!o.x || !o.q || !o.s_row || !o.qT || !o.s_col || !o.maxima) return fail(TI8_ERR_NULL, "%s: x, q, s_row, qT, s_col and maxima are required", fn);
+        if (o.R <= 0 || o.C <= 0 || o.R % 128 || o.C % 128 || o.R > 0x3fffffff || o.C > 0x3fffffff || o.ldx < o.C || o.valid_rows < 0 || o.valid_rows > o.R)
+            return fail(TI8_ERR_SHAPE, "%s: need R%%128==0 and C%%128==0; got R=%lld C=%lld", fn, (long long)o.R, (long long)o.C);
+        if (!aligned16(o.x) || !aligned16(o.q) || !aligned16(o.qT) || !aligned16(o.maxima) || !aligned16(o.partial) || (o.ldx % 8))
+            return fail(TI8_ERR_ALIGN, "%s: pointers must be 16-byte aligned and strides multiples of 16 bytes", fn);
+        if (o.R / ABSMAX_ROWS > 65535) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
+        MaxOperand& x = m.op[i];
+        maxima_tiles(o.R, o.C, &x.tr, &x.tc);
+        x.nrt = (int)parts_of(o.R, x.tr);
+        x.nct = (int)parts_of(o.C, x.tc);
+        x.x = static_cast<const uint16_t*>(o.x); x.ldx = o.ldx;
+        x.rows = reinterpret_cast<uint16_t*>(o.partial);
+        x.cols = x.rows + (int64_t)x.nct * o.R;
+        x.q = o.q; x.ldq = o.C; x.s_row = o.s_row; x.qT = o.qT; x.ldqt = o.R; x.s_col = o.s_col;
+        x.R = (int)o.R; x.C = (int)o.C; x.valid_rows = (int)o.valid_rows;
+        m.first[i] = (int)parts;
+        first_tile[i] = tiles;
+        parts += round8((int64_t)x.nrt * x.nct);
+        tiles += round8((o.R / 128) * (o.C / 128));
+        if (parts + block_tiles > 0x7fffffffLL || tiles > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
+    }
+    for (int i = nboth; i < MAX_OPERANDS; ++i) { m.op[i] = nboth ? m.op[0] : MaxOperand{}; m.first[i] = (int)parts; first_tile[i] = tiles; }
+    m.first[MAX_OPERANDS] = (int)parts;
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (atomics) {
+        ClearRanges r = {};
+        for (int i = 0; i < nboth; ++i) {
+            r.p[i] = both[i].maxima;
+            r.n[i] = (int)(both[i].R + both[i].C);
+        }
+        clear(r, st);
+        for (int i = 0; i < nboth; ++i) {
+            const QRowColOperand& o = both[i];
+            launch_row_col(static_cast<const uint16_t*>(o.x), o.ldx, o.q, o.C, o.s_row, o.qT, o.R, o.s_col, o.maxima, nullptr, o.R, o.valid_rows, o.C, mode, st);
+        }
+        if (int e = check_launch(fn)) return e;
+        return nblocks ? quant_call(fn, blocks, block_rows, nblocks, nullptr, 0, qflags, inv_mode, stream) : TI8_OK;
+    }
+    hipLaunchKernelGGL(quant_first_kernel, dim3((unsigned)(parts + block_tiles)), dim3(256), 0, st, m, b, mode);
+    if (int e = check_launch(fn)) return e;
+    if (!nboth) return TI8_OK;
+    for (int i = 0; i < MAX_OPERANDS; ++i) m.first[i] = (int)first_tile[i];
+    m.first[MAX_OPERANDS] = (int)tiles;
+    hipLaunchKernelGGL(quant_rowcol_multi_kernel, dim3((unsigned)tiles), dim3(256), 0, st, m, mode);
     return check_launch(fn);
 }
 
@@ -878,7 +1164,7 @@ int ti8::quant_col_t_valid(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt,
     hipStream_t st = static_cast<hipStream_t>(stream);
     const uint16_t* xp = static_cast<const uint16_t*>(x);
     unsigned int* wsu = reinterpret_cast<unsigned int*>(ws);
-    hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)((C + 255) / 256)), dim3(256), 0, st, wsu, (int)C, 0u);
+    clear(wsu, C, st);
     if (qflags & TI8_Q_HAD128) {
         // rotate every 128-row segment of every column first (x^T rotated along its contraction
         // dim): both passes redo the rotation on the tile they read instead of storing it
@@ -902,9 +1188,8 @@ extern "C" int ti8_quant_col_t(const void* x, int64_t ldx, int8_t* qT, int64_t l
 }
 
 // The launches of ti8_quant_row_col_t on a workspace the caller of this function has settled on
-int ti8::quant_row_col_t_valid(const char* fn, const void* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT,
-                               int64_t ldqt, float* s_col, float* ws, int64_t R, int64_t valid_rows, int64_t C, int qflags, int inv_mode,
-                               ti8_stream_t stream) {
+static int quant_row_col_t(const char* fn, const void* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT,
+                           int64_t ldqt, float* s_col, float* ws, int64_t R, int64_t C, int qflags, int inv_mode, ti8_stream_t stream) {
     const bool pingpong = (qflags & TI8_Q_WS_PINGPONG) != 0, second = (qflags & TI8_Q_WS_SECOND) != 0;
     const bool is_zero = (qflags & TI8_Q_WS_IS_ZERO) != 0;
     if (second && !pingpong) return fail(TI8_ERR_MODE, "%s: TI8_Q_WS_SECOND needs TI8_Q_WS_PINGPONG", fn);
@@ -929,18 +1214,15 @@ int ti8::quant_row_col_t_valid(const char* fn, const void* x, int64_t ldx, int8_
     }
     unsigned int* wsu = reinterpret_cast<unsigned int*>(ws);
     if (!pingpong && !is_zero)
-        hipLaunchKernelGGL(fill_u32_kernel, dim3((unsigned)((R + C + 255) / 256)), dim3(256), 0, st, wsu, (int)(R + C), 0u);
-    hipLaunchKernelGGL((absmax_kernel<ABSMAX_ROWS, true>), dim3((unsigned)((C + 255) / 256), (unsigned)(R / ABSMAX_ROWS)),
-                       dim3(256), 0, st, xp, ldx, wsu, wsu + R, valid_rows, (int)C);
-    hipLaunchKernelGGL(quant_rowcol_kernel, dim3((unsigned)ntiles), dim3(256), 0, st, xp, ldx, q, ldq, s_row, qT, ldqt,
-                       s_col, ws, ws + R, ws_next, R, (int)(C / 128), (int)valid_rows, mode);
+        clear(wsu, R + C, st);
+    launch_row_col(xp, ldx, q, ldq, s_row, qT, ldqt, s_col, wsu, ws_next, R, R, C, mode, st);
     return check_launch(fn);
 }
 
 extern "C" int ti8_quant_row_col_t(const void* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT,
                                    int64_t ldqt, float* s_col, float* ws, int64_t R, int64_t C, int qflags,
                                    int inv_mode, ti8_stream_t stream) {
-    return ti8::quant_row_col_t_valid("ti8_quant_row_col_t", x, ldx, q, ldq, s_row, qT, ldqt, s_col, ws, R, R, C, qflags, inv_mode, stream);
+    return quant_row_col_t("ti8_quant_row_col_t", x, ldx, q, ldq, s_row, qT, ldqt, s_col, ws, R, C, qflags, inv_mode, stream);
 }
 
 // ---------------------------------------------------------------------------------
@@ -991,7 +1273,7 @@ extern "C" int ti8_quant_row_col_t_noalloc(const void* x, int64_t ldx, int8_t* q
     if (int e = scratch_address(fn, &ws)) return e;
     // the array keeps the last call's maxima: the shared launch sequence starts with the fill kernel
     // that zeroes the R + C words this call uses (a kernel, not a memset, so the call can be captured)
-    return ti8::quant_row_col_t_valid(fn, x, ldx, q, ldq, s_row, qT, ldqt, s_col, ws, R, R, C, qflags, inv_mode, stream);
+    return quant_row_col_t(fn, x, ldx, q, ldq, s_row, qT, ldqt, s_col, ws, R, C, qflags, inv_mode, stream);
 }
 
 int ti8::quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq,

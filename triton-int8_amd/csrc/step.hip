@@ -30,13 +30,16 @@ struct Layer {
     // operands of Y = X W^T, dX = dY W, dW = dY^T X and their scales
     int8_t *xq, *wq, *dq, *wtq, *dytq, *xtq;
     float *xs, *ws, *ds, *wts, *dyts, *xts;
-    unsigned int* maxima;       // row and column maxima of the operands quantised both ways, in one piece
+    unsigned int* maxima;       // scratch of the operands quantised both ways, or by columns: pieces of maxima_piece words
     int64_t maxima_words;
     uint16_t* scratch;          // transposed bf16 copy in front of a rotation along the rows
 
     bool block() const { return scheme == TI8_SCHEME_BLOCK_CHANNEL; }
     bool row_block() const { return scheme == TI8_SCHEME_ROW_BLOCK; }
     bool dbl() const { return scheme == TI8_SCHEME_DOUBLE_CHANNEL; }
+    // R + C maxima, and in a call of one direction the partial ones behind them (a whole step has those in its outputs, see `quantise`)
+    int64_t both_ways_words(int64_t R, int64_t C) const { return maxima_piece(R + C) + (fwd && bwd ? 0 : maxima_piece(quant_maxima_words(R, C))); }
+    static int64_t maxima_piece(int64_t words) { return (words + 63) / 64 * 64; }
     // what an unrotated forward quantises for the backward in the same pass
     bool shares() const { return had == 0 && (keep || (fwd && bwd)); }
     bool given_w() const { return a->wq != nullptr; }
@@ -96,12 +99,12 @@ struct Layer {
         }
         // maxima: W by rows and columns in the forward (or W by columns in a backward that found nothing saved), dY and, for
         // the double-channel scheme, X likewise
-        if (shared && fwd && !row_block()) maxima_words += N + K;
-        if (shared && fwd && dbl()) maxima_words += T + K;
-        if (bwd && had == 0 && !block()) maxima_words += T + N;
-        if (bwd && !shared && !row_block() && !(dbl() && had)) maxima_words += K;      // W^T by columns
-        if (bwd && !shared && dbl() && !had) maxima_words += K;                        // X^T by columns
-        if (bwd && row_block() && had) maxima_words += N;                              // dY^T by rotated columns
+        if (shared && fwd && !row_block()) maxima_words += both_ways_words(N, K);
+        if (shared && fwd && dbl()) maxima_words += both_ways_words(T, K);
+        if (bwd && had == 0 && !block()) maxima_words += both_ways_words(T, N);
+        if (bwd && !shared && !row_block() && !(dbl() && had)) maxima_words += maxima_piece(K);      // W^T by columns
+        if (bwd && !shared && dbl() && !had) maxima_words += maxima_piece(K);                        // X^T by columns
+        if (bwd && row_block() && had) maxima_words += maxima_piece(N);                              // dY^T by rotated columns
         if (maxima_words) maxima = w.take<unsigned int>(maxima_words);
         if (saved_bytes) *saved_bytes = kept.used;
         return w.used;
@@ -170,6 +173,21 @@ int check_pointers(const char* fn, const ti8_linear_args* a, const Layer& L) {
     return TI8_OK;
 }
 
+// Whether the outputs of a whole step share no memory with its inputs
+bool outputs_apart(const ti8_linear_args& a, int64_t T) {
+    struct Range { const char *from, *to; };
+    const auto range = [](const void* p, int64_t rows, int64_t ld, int64_t cols) {
+        const char* const c = static_cast<const char*>(p);
+        return Range{c, p ? c + ((rows - 1) * ld + cols) * 2 : c};
+    };
+    const Range in[3] = {range(a.X, a.tokens, a.ldx, a.K), range(a.W, a.N, a.ldw, a.K), range(a.dY, a.tokens, a.lddy, a.N)};
+    const Range out[3] = {range(a.Y, T, a.ldy, a.N), range(a.dX, T, a.lddx, a.K), range(a.dW, a.N, a.lddw, a.K)};
+    for (const Range& i : in)
+        for (const Range& o : out)
+            if (i.from < o.to && o.from < i.to) return false;
+    return true;
+}
+
 int64_t next_pow2(int64_t v) {
     int64_t n = 128;
     while (n < v) n <<= 1;
@@ -180,28 +198,40 @@ int64_t next_pow2(int64_t v) {
 int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stream_t stream) {
     const ti8_linear_args& a = *L.a;
     const int64_t T = L.T, K = L.K, N = L.N, tok = L.tokens;
-    const hipStream_t st = static_cast<hipStream_t>(stream);
     const int q = TI8_Q_CLAMP, had = L.had == 128 ? TI8_Q_HAD128 : 0;
     const int inv = L.dbl() ? TI8_INV_AMAX_DIV_127 : TI8_INV_RCP_OF_SCALE;
     const bool shared = L.shares();
     unsigned int* mx = L.maxima;
     auto take_maxima = [&](int64_t words) {
         unsigned int* p = mx;
-        mx += words;
+        mx += Layer::maxima_piece(words);
         return reinterpret_cast<float*>(p);
     };
-    auto row_col = [&](const void* x, int64_t ldx, int8_t* oq, float* os, int8_t* oqT, float* osT, int64_t R, int64_t valid, int64_t C) {
-        return quant_row_col_t_valid(fn, x, ldx, oq, C, os, oqT, R, osT, take_maxima(R + C), R, valid, C, q | TI8_Q_WS_IS_ZERO, inv, stream);
+    // Without a rotation, the operands quantised by blocks and those quantised by rows and by columns are collected and go into two
+    // launches for the call, without one that only clears maxima (quant_call: 16 tokens, 4096 -> 4096, block-channel 41 -> 37.6 us;
+    // 3072 tokens row-block 210 -> 204)
+    ti8_qblock_operand by_block[4];
+    int64_t by_block_rows[4];
+    QRowColOperand both[3];
+    int nblocks = 0, nboth = 0;
+    // (`out`, `ldout`: the output of the operand's own shape, which a whole step does not write before its GEMMs; the partial maxima
+    // live there until the conversion has read them, unless the caller's tensors overlap)
+    const bool apart = outputs_apart(a, T);
+    auto row_col = [&](const void* x, int64_t ldx, int8_t* oq, float* os, int8_t* oqT, float* osT, int64_t R, int64_t valid, int64_t C, void* out, int64_t ldout) {
+        unsigned int* const scratch = reinterpret_cast<unsigned int*>(take_maxima(R + C));
+        unsigned int* partial = nullptr;
+        if (!(L.fwd && L.bwd)) partial = reinterpret_cast<unsigned int*>(take_maxima(quant_maxima_words(R, C)));
+        else if (apart && ldout == C) partial = static_cast<unsigned int*>(out);
+        both[nboth++] = QRowColOperand{x, ldx, oq, os, oqT, osT, scratch, partial, R, valid, C};
+    };
+    auto block = [&](const ti8_qblock_operand& o, int64_t valid) {
+        by_block_rows[nblocks] = valid;
+        by_block[nblocks++] = o;
     };
     auto blocks = [&](const void* x, int64_t ldx, int8_t* oq, int8_t* oqT, float* os, int64_t R, int64_t C) {
         return ti8_qblock_operand{x, 0, ldx, oq, R * C, C, oqT, R * C, R, os, 0, C / 128, 1, 1, R, C};
     };
     int n = 0;
-    // double-channel without rotation, and the row-block backward: one launch clears all maxima (block-channel: the block
-    // quantiser's launch clears them on the side)
-    const bool own_clear = L.maxima_words && L.had == 0 && !L.block();
-    if (own_clear)
-        if (int e = fill_words(L.maxima, L.maxima_words, 0u, st)) return e;
     const float rot = L.had == 128 ? 0.0078125f : 1.0f;     // 2^-7: both operands carry an un-normalised H_128
 
     if (L.fwd) {
@@ -210,31 +240,24 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
             if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xq, T * K, K, L.xs, 0, K / 128, 1, 1, T, tok, K, 0, q, inv, stream)) return e;
             if (!L.given_w()) if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q | had, inv, stream)) return e;
         } else if (L.block()) {
-            ti8_qblock_operand o[2] = {blocks(a.X, a.ldx, L.xq, shared ? L.xtq : nullptr, L.xs, T, K)};
-            int64_t valid[2] = {tok, tok};
-            int operands = 1;
-            if (L.bwd) o[operands++] = blocks(a.dY, a.lddy, L.dq, L.dytq, L.ds, T, N);    // both activations at hand: one launch
-            if (int e = quant_block_multi_and_clear(o, valid, operands, q, inv, L.maxima, L.maxima_words, stream)) return e;
-            if (shared) {
-                if (int e = row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K)) return e;     // rows for Y, columns for dX
-            } else if (!L.given_w()) {
+            block(blocks(a.X, a.ldx, L.xq, shared ? L.xtq : nullptr, L.xs, T, K), tok);
+            if (shared) row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K, a.dW, a.lddw);     // rows for Y, columns for dX
+            else if (!L.given_w())
                 if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q, inv, stream)) return e;
-            }
         } else if (L.row_block()) {
             if (int e = ti8_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, 0, q | had, inv, stream)) return e;
             if (L.had) {
                 if (!L.given_w()) if (int e = ti8_quant_block_had128(a.W, 0, a.ldw, L.wq, N * K, K, L.ws, 0, K / 128, 1, 1, N, K, 0, q, inv, stream)) return e;
             } else if (!L.given_w()) {
-                const ti8_qblock_operand o = blocks(a.W, a.ldw, L.wq, shared ? L.wtq : nullptr, L.ws, N, K);
-                if (int e = ti8_quant_block_multi(&o, 1, q, inv, stream)) return e;
+                block(blocks(a.W, a.ldw, L.wq, shared ? L.wtq : nullptr, L.ws, N, K), N);
             }
         } else if (L.had) {
             post = (float)(1.0 / (double)K);
             if (int e = ti8_fwht_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, next_pow2(K), q, inv, stream)) return e;
             if (!L.given_w()) if (int e = ti8_fwht_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, next_pow2(K), q, inv, stream)) return e;
         } else if (shared) {
-            if (int e = row_col(a.X, a.ldx, L.xq, L.xs, L.xtq, L.xts, T, tok, K)) return e;
-            if (int e = row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K)) return e;
+            row_col(a.X, a.ldx, L.xq, L.xs, L.xtq, L.xts, T, tok, K, a.dX, a.lddx);
+            row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K, a.dW, a.lddw);
         } else {
             if (int e = ti8_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, 0, q, inv, stream)) return e;
             if (!L.given_w()) if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q, inv, stream)) return e;
@@ -256,14 +279,10 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
             if (int e = quant_block_had128_valid(a.dY, 0, a.lddy, L.dytq, T * N, T, L.dyts, 0, N / 128, 1, 1, T, tok, N, 1, 0, inv, stream)) return e;
             if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xtq, T * K, T, L.xts, 0, K / 128, 1, 1, T, tok, K, 1, 0, inv, stream)) return e;
         } else if (L.block()) {
-            if (!L.fwd) {
-                ti8_qblock_operand o = blocks(a.dY, a.lddy, L.dq, L.dytq, L.ds, T, N);
-                if (int e = quant_block_multi_and_clear(&o, &tok, 1, q, inv, nullptr, 0, stream)) return e;
-                if (!shared) {
-                    if (int e = quant_col_t_valid(a.W, a.ldw, L.wtq, N, L.wts, take_maxima(K), N, N, K, q, inv, stream)) return e;
-                    o = blocks(a.X, a.ldx, nullptr, L.xtq, L.xts, T, K);
-                    if (int e = quant_block_multi_and_clear(&o, &tok, 1, q, inv, nullptr, 0, stream)) return e;
-                }
+            block(blocks(a.dY, a.lddy, L.dq, L.dytq, L.ds, T, N), tok);
+            if (!shared) {
+                if (int e = quant_col_t_valid(a.W, a.ldw, L.wtq, N, L.wts, take_maxima(K), N, N, K, q, inv, stream)) return e;
+                block(blocks(a.X, a.ldx, nullptr, L.xtq, L.xts, T, K), tok);
             }
         } else if (L.row_block() && L.had) {
             if (int e = ti8_quant_row(a.dY, a.lddy, L.dq, N, L.ds, tok, N, 0, q | had, inv, stream)) return e;
@@ -271,14 +290,9 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
             if (int e = quant_col_t_valid(a.dY, a.lddy, L.dytq, T, L.dyts, take_maxima(N), T, tok, N, q | had, inv, stream)) return e;
             if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xtq, T * K, T, L.xts, 0, K / 128, 1, 1, T, tok, K, 1, q, inv, stream)) return e;
         } else if (L.row_block()) {
-            if (int e = row_col(a.dY, a.lddy, L.dq, L.ds, L.dytq, L.dyts, T, tok, N)) return e;
-            ti8_qblock_operand o;
-            if (!shared) {
-                o = blocks(a.W, a.ldw, nullptr, L.wtq, L.wts, N, K);
-                if (int e = ti8_quant_block_multi(&o, 1, q, inv, stream)) return e;
-            }
-            o = blocks(a.X, a.ldx, nullptr, L.xtq, L.xts, T, K);
-            if (int e = quant_block_multi_and_clear(&o, &tok, 1, q, inv, nullptr, 0, stream)) return e;
+            row_col(a.dY, a.lddy, L.dq, L.ds, L.dytq, L.dyts, T, tok, N, a.Y, a.ldy);
+            if (!shared) block(blocks(a.W, a.ldw, nullptr, L.wtq, L.wts, N, K), N);
+            block(blocks(a.X, a.ldx, nullptr, L.xtq, L.xts, T, K), tok);
         } else if (L.had) {
             // the transposed operands are rotated along the rows of the tensors as they lie in memory
             post_dx = (float)(1.0 / (double)N);
@@ -288,7 +302,7 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
             if (int e = fwht_t_quant_row_valid(a.dY, a.lddy, L.scratch, L.dytq, T, L.dyts, T, tok, N, q, inv, stream)) return e;
             if (int e = fwht_t_quant_row_valid(a.X, a.ldx, L.scratch, L.xtq, T, L.xts, T, tok, K, q, inv, stream)) return e;
         } else {
-            if (int e = row_col(a.dY, a.lddy, L.dq, L.ds, L.dytq, L.dyts, T, tok, N)) return e;
+            row_col(a.dY, a.lddy, L.dq, L.ds, L.dytq, L.dyts, T, tok, N, a.Y, a.ldy);
             if (!shared) {
                 if (int e = quant_col_t_valid(a.W, a.ldw, L.wtq, N, L.wts, take_maxima(K), N, N, K, q, inv, stream)) return e;
                 if (int e = quant_col_t_valid(a.X, a.ldx, L.xtq, T, L.xts, take_maxima(K), T, tok, K, q, inv, stream)) return e;
@@ -301,7 +315,7 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
         g[n++] = gemm2d(L.dytq, L.dyts, dyt_mode, dyts_rs, dyts_ks, L.xtq, L.xts, xt_mode, xts_rs, xts_ks, a.dW, a.lddw, N, K, T, L.dbl(), rot, post_dw);
     }
     *count = n;
-    return TI8_OK;
+    return quant_call(fn, by_block, by_block_rows, nblocks, both, nboth, q, inv, stream);
 }
 
 // One GEMM launched alone (what ti8_gemm_i8_nt selects for its shape: the few-rows kernel up to 256 rows)

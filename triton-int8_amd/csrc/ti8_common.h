@@ -66,12 +66,23 @@ int init_quant_scratch();
 // ---- pieces of quant.hip and fwht.hip that the layer calls (step.hip) use ----------
 // `valid_rows` (of R, the rest counts as zeros and is not read): an activation whose token count is no multiple of the tile
 // needs no zero-padded copy.  NULL / R: all of them.
-// ti8_quant_block_multi that also zeroes `clear_words` 32-bit words at `clear` (NULL: nothing) in the same launch
-int quant_block_multi_and_clear(const ti8_qblock_operand* operands, const int64_t* valid_rows, int count, int qflags, int inv_mode,
-                                unsigned int* clear, int64_t clear_words, ti8_stream_t stream);
-int quant_row_col_t_valid(const char* fn, const void* x, int64_t ldx, int8_t* q, int64_t ldq, float* s_row, int8_t* qT,
-                          int64_t ldqt, float* s_col, float* ws, int64_t R, int64_t valid_rows, int64_t C, int qflags, int inv_mode,
-                          ti8_stream_t stream);
+int quant_block_multi_valid(const ti8_qblock_operand* operands, const int64_t* valid_rows, int count, int qflags, int inv_mode, ti8_stream_t stream);
+// An operand quantised by rows (q [R][C]) and by columns (qT [C][R]).  Scratch: `maxima` R + C words; `partial` quant_maxima_words words
+// (in no more than the operand's own bytes) or null, which leaves the call to the atomics form.
+struct QRowColOperand {
+    const void* x;
+    int64_t ldx;
+    int8_t* q;
+    float* s_row;
+    int8_t* qT;
+    float* s_col;
+    unsigned int *maxima, *partial;
+    int64_t R, valid_rows, C;
+};
+int64_t quant_maxima_words(int64_t R, int64_t C);
+// Block-quantised operands and operands quantised both ways (up to 4 and 3) in two launches, one where there are none of the latter
+int quant_call(const char* fn, const ti8_qblock_operand* blocks, const int64_t* block_rows, int nblocks, const QRowColOperand* both, int nboth, int qflags,
+               int inv_mode, ti8_stream_t stream);
 int quant_col_t_valid(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt, float* s, float* ws, int64_t R, int64_t valid_rows, int64_t C,
                       int qflags, int inv_mode, ti8_stream_t stream);
 int quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq, float* s, int64_t ssb, int64_t ssr,
@@ -79,7 +90,6 @@ int quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q,
                              ti8_stream_t stream);
 int fwht_t_quant_row_valid(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t valid_rows, int64_t C,
                            int qflags, int inv_mode, ti8_stream_t stream);
-int fill_words(unsigned int* p, int64_t words, unsigned int value, hipStream_t st);
 // ti8_gemm_i8_nt with a bias for the kernels whose epilogue adds one (*added: this was one); y += bias behind the others (bias.hip)
 int gemm_nt_bias(const ti8_gemm_problem& p, const void* bias, int gemm_flags, bool* added, ti8_stream_t stream);
 // gemm.hip: the GEMMs of a call on few tokens as one launch, those that go into it (see there)
