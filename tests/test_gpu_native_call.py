@@ -1,0 +1,83 @@
+"""The layer call made from C++ gives what the Python way gives, and leaves to it what it does not take."""
+import pytest
+import torch
+
+import triton_int8_amd as T
+from triton_int8_amd._lib import PART_BACKWARD, PART_FORWARD, PART_KEEP
+
+pytestmark = pytest.mark.gpu
+
+
+class Named(torch.Tensor):
+    pass
+
+
+def _both(monkeypatch, call):
+    assert T._lib.native() is not None
+    made = call()
+    with monkeypatch.context() as m:
+        m.setattr(T._lib, "_native", False)
+        plain = call()
+    return made, plain
+
+
+# the parts a call can have; one tile and several, whole and ragged; rows that are read in place, that begin at an odd address, that overlap
+@pytest.mark.parametrize("scheme, hadamard", [("block_channel", None), ("row_block", 128), ("double_channel", None)])
+@pytest.mark.parametrize("tokens", [1, 128, 300])
+@pytest.mark.parametrize("rows", ["dense", "strided", "odd", "expanded"])
+def test_same_results(dev, monkeypatch, scheme, hadamard, tokens, rows):
+    k, n = 256, 384
+    g = torch.Generator(device=dev).manual_seed(3)
+
+    def matrix(r, c, kind="dense"):
+        x = torch.randn(r, c + 8, generator=g, device=dev).to(torch.bfloat16)
+        return {"dense": x[:, :c].contiguous(), "strided": x[:, :c], "odd": x[:, 1:c + 1], "expanded": x[:1, :c].expand(r, c)}[kind]
+
+    X, W, dY, bias = matrix(tokens, k, rows), matrix(n, k), matrix(tokens, n, rows), matrix(1, n)[0]
+    wq = T.linear.quantize_weight(W, scheme, hadamard)
+
+    def call():
+        Y, _, _, saved = T.ops.linear_call(PART_FORWARD | PART_KEEP, scheme, hadamard, tokens, k, n, X=X, W=W)
+        keep = PART_KEEP if saved is not None else 0
+        _, dX, dW, _ = T.ops.linear_call(PART_BACKWARD | keep, scheme, hadamard, tokens, k, n, X=X, W=W, dY=dY, saved=saved)
+        served = T.ops.linear_call(PART_FORWARD, scheme, hadamard, tokens, k, n, X=X, wq=wq, bias=bias)[0]
+        step = T.linear_fwd_bwd(X, W, dY, scheme, hadamard)
+        assert Y.shape == served.shape == (-(-tokens // 128) * 128, n) and dX.shape[0] == Y.shape[0]
+        return [Y[:tokens], dX[:tokens], dW, served[:tokens], *step]
+
+    for a, b in zip(*_both(monkeypatch, call)):
+        assert a.dtype == b.dtype == torch.bfloat16 and a.stride() == b.stride() and torch.equal(a, b)
+
+
+def test_what_it_leaves_to_the_python_way(dev, monkeypatch):
+    X, W = torch.randn(5, 256, device=dev).to(torch.bfloat16), torch.randn(128, 256, device=dev).to(torch.bfloat16)
+    call = lambda x: T.ops.linear_call(PART_FORWARD, "block_channel", None, 5, 256, 128, X=x, W=W)[0][:5]
+    want = call(X)
+    assert torch.equal(call(X.as_subclass(Named)), want)
+    with T._lib.timed_launches() as record:
+        assert torch.equal(call(X), want)
+    assert list(record) == ["ti8_linear"]
+    for bad in (X.float(), X.cpu()):
+        with pytest.raises(ValueError, match="X must be"):
+            call(bad)
+    def failing():
+        with pytest.raises(T._lib.Ti8Error, match="ti8_linear failed with status .*ti8_linear") as e:
+            T.ops.linear_call(PART_FORWARD, "block_channel", None, 5, 256, 128, X=X)
+        return str(e.value)
+    made, plain = _both(monkeypatch, failing)
+    assert made == plain
+
+
+def test_captured(dev):
+    layer = T.Int8Linear(256, 128, device=dev)
+    x = torch.randn(3, 256, device=dev).to(torch.bfloat16)
+    with torch.no_grad():
+        layer(x)
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            y = layer(x)
+        for seed in range(3):
+            x.copy_(torch.randn(3, 256, device=dev, generator=torch.Generator(device=dev).manual_seed(seed)))
+            graph.replay()
+            assert torch.equal(y, layer(x))
+            torch.cuda.synchronize()

@@ -9,6 +9,7 @@ import os
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libti8.so")
+NATIVE_PATH = os.path.join(_HERE, "_native.so")
 
 _i64, _int, _f32, _vp = ctypes.c_int64, ctypes.c_int, ctypes.c_float, ctypes.c_void_p
 
@@ -173,7 +174,36 @@ def call(name, *args):
         b.record()
         rec.setdefault(name, []).append((a, b))
     if rc != 0:
-        raise Ti8Error(name, rc, l.ti8_last_error().decode())
+        raise failed(name, rc)
+
+
+_native = None  # the extension module, False where there is none
+
+
+def native():
+    """The layer call's host side in C++ (``csrc/native.cpp``) on the entry points of :func:`lib`, or None: while calls are being timed
+    one by one, and where it was built for another torch (the same launches are then made from Python)."""
+    global _native
+    if _timing is not None:
+        return None
+    if _native is None:
+        import importlib.util
+        import torch
+        try:
+            spec = importlib.util.spec_from_file_location("_native", NATIVE_PATH)
+            module = importlib.util.module_from_spec(spec)
+            address = lambda name: ctypes.cast(getattr(lib(), name), _vp).value
+            module.set_up(address("ti8_linear"), address("ti8_linear_quantise"), address("ti8_gemm_i8_nt_multi"), torch.nn.Parameter)
+            _native = module
+        except ImportError:
+            lib()
+            _native = False
+    return _native or None
+
+
+def failed(name, code):
+    """The exception for an entry point of this thread that has just returned a non-zero status."""
+    return Ti8Error(name, code, lib().ti8_last_error().decode())
 
 
 def init():

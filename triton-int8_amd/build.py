@@ -1,6 +1,6 @@
-"""Build ``libti8.so`` (every HIP kernel + the C ABI) for gfx950 with hipcc.
+"""Build ``libti8.so`` (every HIP kernel + the C ABI) for gfx950 with hipcc, and the layer call's host side with g++.
 
-Run as ``python triton-int8_amd/build.py`` or call :func:`build`.  The library is
+Run as ``python triton-int8_amd/build.py`` or call :func:`build`.  The libraries are
 written next to this file; it is cross-compiled, so no GPU is needed to build.
 """
 import os
@@ -10,6 +10,7 @@ import sys
 HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libti8.so")
+NATIVE = os.path.join(HERE, "_native.so")
 SOURCES = ["api.hip", "quant.hip", "fwht.hip", "gemm.hip", "gemm_chain.hip", "gemm_mid.hip", "gemm_skinny.hip", "step.hip", "decoder.hip", "attention.hip", "bias.hip", "probe.hip"]
 
 # -ffp-contract=off: x*scale+0.5 must round twice (bit-exact quantisation); kernels
@@ -33,7 +34,25 @@ def build(verbose: bool = False) -> str:
         raise RuntimeError("hipcc failed:\n" + out)
     if verbose and out:
         print(out)
+    build_native(verbose)
     return LIB
+
+
+def build_native(verbose: bool = False) -> str:
+    """The layer call's host side (csrc/native.cpp), an extension of the Python and the torch that run this: host code only, it is
+    handed the library's entry points when it is loaded."""
+    import sysconfig
+    import torch
+    from torch.utils.cpp_extension import include_paths, library_paths
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}"]
+    cmd += [a for path in [sysconfig.get_paths()["include"], *include_paths()] for a in ("-isystem", path)]
+    cmd += [os.path.join(CSRC, "native.cpp"), "-o", NATIVE, *(f"-L{path}" for path in library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10"]
+    if verbose:
+        print(" ".join(cmd), flush=True)
+    res = subprocess.run(cmd, stdout=subprocess.PIPE, stderr=subprocess.STDOUT, text=True)
+    if res.returncode != 0:
+        raise RuntimeError("g++ failed:\n" + res.stdout)
+    return NATIVE
 
 
 if __name__ == "__main__":

@@ -427,7 +427,8 @@ class Int8Linear(torch.nn.Module):
         key = (weight._version, weight.data_ptr(), self.scheme, self.hadamard)
         if self._wq_key != key or self._wq_of[0] is not weight:
             self._wq, self._wq_key, self._wq_of = quantize_weight(weight.detach(), self.scheme, self.hadamard), key, (weight,)
-        x2 = x.reshape(-1, x.shape[-1])
+        flat = x.dim() == 2
+        x2 = x if flat else x.reshape(-1, x.shape[-1])
         tokens = x2.shape[0]
         if _from_c():
             if x2.shape[1] != self.in_features:
@@ -442,7 +443,7 @@ class Int8Linear(torch.nn.Module):
         y = y[:tokens]
         if self.bias is not None and not inside:
             y = y + self.bias
-        return y.reshape(*x.shape[:-1], self.out_features)
+        return y if flat else y.reshape(*x.shape[:-1], self.out_features)
 
     def extra_repr(self):
         return f"in_features={self.in_features}, out_features={self.out_features}, scheme={self.scheme}, hadamard={self.hadamard}"

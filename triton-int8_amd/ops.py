@@ -497,19 +497,38 @@ def _linear_sizes(tokens, K, N, scheme, hadamard, parts, given_w):
     return n, saved.value
 
 
+def _native_call(parts, scheme, hadamard, tokens, K, N, X, W, dY, wq, saved, apart, bias):
+    """:func:`linear_call` with its allocations and launches made from C++, or None where it takes the Python way.  Calls on few tokens wait
+    for the host: one token through a 4096 x 4096 layer takes 13.3 us, 17.4 with the Python way; 37 tokens, 4096 -> 14336, 16.2 and 17.6."""
+    native = _lib.native()
+    if native is None:
+        return None
+    need, need_saved = _linear_sizes(tokens, K, N, scheme, hadamard, parts, wq is not None)
+    wq, ws = wq or (None, None)
+    out = native.linear_call(parts, _SCHEMES[scheme], _ROTATIONS[hadamard], tokens, K, N, _gemm_flags(), need, need_saved, apart, _stream(),
+                             X, W, dY, wq, ws, saved, bias)
+    if out is not None and len(out) == 2:
+        raise _lib.failed(*out)
+    return out
+
+
 def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=None, wq=None, saved=None, one_launch=True, bias=None):
     """The forward, the backward or both of a layer in one or two library calls (``ti8_linear``; with ``one_launch`` and more than
     256 tokens and output features the quantisers as one call and the backward's or step's GEMMs as ``ti8_gemm_i8_nt_multi``).
     X bf16 [tokens, K], W bf16 [N, K], dY bf16 [tokens, N]: any number of tokens, no padded copies.  ``wq`` = (int8 [N, K], scales) of
     the weight quantised earlier, ``bias`` bf16 [N] is added to Y (a forward alone).  Returns (Y [T, N], dX [T, K], dW [N, K], saved) with None for what `parts` does not ask for; T =
     tokens rounded up to 128, rows from `tokens` on undefined."""
+    T = -(-tokens // 128) * 128
+    apart = one_launch and bool(parts & _lib.PART_BACKWARD) and min(T, N) > 256
+    out = _native_call(parts, scheme, hadamard, tokens, K, N, X, W, dY, wq, saved, apart, bias)
+    if out is not None:
+        return out
     for t, name in ((X, "X"), (W, "W"), (dY, "dY")):
         if t is not None:
             _check_bf16(t, name)
     dev = (X if X is not None else dY).device
     need, need_saved = _linear_sizes(tokens, K, N, scheme, hadamard, parts, wq is not None)
     X, W, dY = (t if t is None else rows16(t) for t in (X, W, dY))
-    T = -(-tokens // 128) * 128
     Y = dX = dW = None
     if parts & _lib.PART_FORWARD:
         Y = torch.empty((T, N), dtype=torch.bfloat16, device=dev)
@@ -525,7 +544,7 @@ def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=Non
                         tokens, K, N, _SCHEMES[scheme], _ROTATIONS[hadamard], parts, _gemm_flags(), workspace.data_ptr(), need,
                         ptr(saved), need_saved, ptr(bias))
     stream = _stream()
-    if one_launch and parts & _lib.PART_BACKWARD and min(T, N) > 256:
+    if apart:
         problems, count = (_lib.GemmProblem * 3)(), ctypes.c_int(0)
         _lib.call("ti8_linear_quantise", ctypes.byref(a), problems, ctypes.byref(count), stream)
         _lib.call("ti8_gemm_i8_nt_multi", problems, count.value, a.gemm_flags | GEMM_TOGETHER, stream)
@@ -561,6 +580,10 @@ def linear_step(X2, W, dY2, scheme, *, tokens=None, out=None, workspace=None):
     _need(tokens is None or 1 <= tokens <= rows, f"tokens must be between 1 and the {rows} rows of X and dY, got {tokens}")
     T = -(-rows // 128) * 128
     need = linear_step_workspace_bytes(T, K, N, scheme)
+    if out is None and workspace is None and tokens is None:
+        made = _native_call(_lib.PART_FORWARD | _lib.PART_BACKWARD, scheme, None, rows, K, N, X2, W, dY2, None, None, False, None)
+        if made is not None:
+            return made[:3]
     X2, W, dY2 = rows16(X2), rows16(W), rows16(dY2)
     dev = X2.device
     if out is None:
