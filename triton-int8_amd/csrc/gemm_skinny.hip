@@ -11,6 +11,7 @@
 // per output, K tiles walked from a workgroup-dependent start).  The int32 path is therefore
 // bit-identical to the tiled kernel, the promoted path differs by fp32 association only.
 #include "gemm_args.h"
+#include "quant_math.h"
 
 namespace ti8 {
 
@@ -28,6 +29,7 @@ namespace ti8 {
 // shared by the workgroup and one barrier per K tile took 14.4 us where this one takes 11.2 us
 // (128 rows, K = N = 4096).  Two stages = 64 KiB per workgroup, so two workgroups share a CU.
 constexpr int WS_STAGES = 2;
+constexpr int DECODE_A_BYTES = DECODE_ROWS * 128;    // a K tile of A that the wave quantises itself
 
 // A workgroup's part of C is MB x NB blocks of 32 x 32, one or four: `block_x` = index of the workgroup among those of this GEMM and
 // batch.  What bounds the kernel is the stream into a CU's LDS (55 bytes per ns, half of what the L2 alone delivers; neither more stages
@@ -35,10 +37,14 @@ constexpr int WS_STAGES = 2;
 // product.  idx::few_rows_wide says where which is the faster one.  us, one block / four, int32 path: 64 rows, 4096 -> 14336
 // 21.0 / 15.3; 128 rows 4096 -> 4096 10.1 / 10.1, 8192 -> 8192 33.4 / 21.1; 256 rows 4096 -> 4096 16.7 / 10.8, 14336 -> 4096 98 / 36;
 // 64 rows, 14336 -> 14336 46.6 / 32.1 (31.6 for the weight alone).
-template <bool I32FULL, int BLOCKS>
-__device__ __forceinline__ void wavering_block(const GemmArgs& g, const int block_x, const int batch) {
+// QUANTISE: operand A is bf16 (g.A, g.lda in elements), 1 to 8 rows, and each wave quantises the 128 columns of its K tile by their
+// absmax (the block quantiser's arithmetic) on the way to LDS, one 16-byte chunk of a row per lane.  The missing ones of the 32 rows are
+// copies of those 8, and missing ones of the 8 copies of the last: rows of C that nobody reads.
+template <bool I32FULL, int BLOCKS, bool QUANTISE = false>
+__device__ __forceinline__ void wavering_block(const GemmArgs& g, const int block_x, const int batch, const int rows = 0) {
+    static_assert(!QUANTISE || (!I32FULL && BLOCKS == 1), "quantised by K tiles, up to 8 rows");
     constexpr int MB = BLOCKS, NB = BLOCKS;
-    constexpr int STAGE_BYTES = (MB + NB) * 32 * 128;     // per wave
+    constexpr int B_AT = QUANTISE ? 0 : MB * 4096, STAGE_BYTES = B_AT + NB * 4096;     // per wave
     extern __shared__ __attribute__((aligned(1024))) int8_t smem[];  // 4 waves x WS_STAGES x STAGE_BYTES
 
     const int lane = threadIdx.x & 63;
@@ -72,7 +78,12 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
     const int8_t* baseA = g.A + (int64_t)batch * g.bsa + (int64_t)m0 * g.lda;
     const int8_t* baseB = g.B + (int64_t)batch * g.bsb + (int64_t)n0 * g.ldb;
     const int64_t strideA8 = 8 * g.lda, strideB8 = 8 * g.ldb;
-    int8_t* const ring = smem + wave * (WS_STAGES * STAGE_BYTES);
+    int8_t* const ring = smem + wave * (WS_STAGES * STAGE_BYTES + (QUANTISE ? DECODE_A_BYTES : 0));
+    // QUANTISE: this lane's 16 elements of a K tile, on their way from memory, and where their codes go
+    const uint16_t* const x = reinterpret_cast<const uint16_t*>(g.A) + (QUANTISE ? min(ld_row, rows - 1) * g.lda + (lane & 7) * 16 : 0);
+    uint4 x_lo = {0, 0, 0, 0}, x_hi = {0, 0, 0, 0};
+    int8_t* const a_tile = ring + WS_STAGES * STAGE_BYTES;
+    const uint32_t a_to = QUANTISE ? (uint32_t)(uintptr_t)(__attribute__((address_space(3))) int8_t*)(a_tile + ld_row * 128 + ((lane & 7) ^ ld_row) * 16) : 0;
     // step i of this wave's walk is K tile kbeg + (i + rot) mod nq: workgroups of one block start at different
     // tiles so that they do not ask the same memory channels for their lines at the same time.  With more rows what counts is that
     // the workgroups of an XCD read A's columns together, which then need not all fit its L2 (256 rows, K = 14336, N = 4096:
@@ -86,10 +97,15 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
     auto issue_stage = [&](int i) {
         int8_t* st = ring + (i & (WS_STAGES - 1)) * STAGE_BYTES;
         const int koff = tile_of_step(i) * 128;
+        if (QUANTISE) {
+            x_lo = *reinterpret_cast<const uint4*>(x + koff);
+            x_hi = *reinterpret_cast<const uint4*>(x + koff + 8);
+        } else {
 #pragma unroll
-        for (int b = 0; b < MB; ++b) issue_tile_loads<4>(baseA + koff + min(b, mblocks - 1) * 4 * strideA8, strideA8, voffA, 0, st + b * 4096);
+            for (int b = 0; b < MB; ++b) issue_tile_loads<4>(baseA + koff + min(b, mblocks - 1) * 4 * strideA8, strideA8, voffA, 0, st + b * 4096);
+        }
 #pragma unroll
-        for (int b = 0; b < NB; ++b) issue_tile_loads<4>(baseB + koff + b * 4 * strideB8, strideB8, voffB, 0, st + (MB + b) * 4096);
+        for (int b = 0; b < NB; ++b) issue_tile_loads<4>(baseB + koff + b * 4 * strideB8, strideB8, voffB, 0, st + B_AT + b * 4096);
     };
 
     // ---- scales: unconditional loads (an operand that contributes no in-loop factor is read with
@@ -98,7 +114,7 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
     const bool divide = !I32FULL && g.combine == TI8_COMBINE_DIV_PROD;
     const bool a_in = !I32FULL && g.sa.mode != TI8_SCALE_ROW, b_in = !I32FULL && g.sb.mode != TI8_SCALE_ROW;
     float fvec[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-    if (!I32FULL) {
+    if (!I32FULL && !QUANTISE) {
         const int sha = g.sa.mode == TI8_SCALE_BLOCK_K256 ? 1 : 0, shb = g.sb.mode == TI8_SCALE_BLOCK_K256 ? 1 : 0;
         const float* pa = g.sa.p + (int64_t)batch * g.sa.bs + (a_in ? (int64_t)(m0 >> 7) * g.sa.rs : 0);
         const float* pb = g.sb.p + (int64_t)batch * g.sb.bs + (b_in ? (int64_t)(n0 >> 7) * g.sb.rs : 0);
@@ -151,6 +167,9 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
     int at[4];
 #pragma unroll
     for (int ks = 0; ks < 4; ++ks) at[ks] = fr_row * 128 + ((ks * 2 + fr_half) ^ sw) * 16;
+    int at_a[4];
+#pragma unroll
+    for (int ks = 0; ks < 4; ++ks) at_a[ks] = QUANTISE ? (lane & 7) * 128 + ((ks * 2 + fr_half) ^ (lane & 7)) * 16 : at[ks];
 
     const v16i vzero = {0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0, 0};
     v16i d[MB][NB];             // int32 sums: of the whole K (I32FULL), or of the step whose products are folded next
@@ -202,15 +221,26 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
         // own loads of step i landed; own LDS reads of step i - 1 returned, so its stage can be refilled.  No barrier: nobody
         // else touches this wave's ring.
         TI8_WAIT_VMCNT_LGKM0(0);
+        const uint4 now_lo = x_lo, now_hi = x_hi;
         issue_stage(i + 1);
         const int8_t* st = ring + (i & (WS_STAGES - 1)) * STAGE_BYTES;
+        float f_now = 0.0f;
+        if (QUANTISE) {
+            const float amax = amax_floor(wave_max(absmax8(now_hi, absmax8(now_lo, 0.0f))), 0);
+            const float scale = 127.0f / amax;
+            f_now = 1.0f / scale;
+            const uint2 lo = quant8(now_lo, scale), hi = quant8(now_hi, scale);
+            const v4i codes = {(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
+            // (a store that the compiler knew of would wait for the loads in flight to LDS; a wave's LDS instructions stay in order)
+            asm volatile("ds_write_b128 %0, %1" ::"v"(a_to), "v"(codes) : "memory");
+        }
         v4i fa[MB][4], fb[NB][4];
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) {
 #pragma unroll
-            for (int b = 0; b < MB; ++b) fa[b][ks] = *reinterpret_cast<const v4i*>(st + b * 4096 + at[ks]);
+            for (int b = 0; b < MB; ++b) fa[b][ks] = *reinterpret_cast<const v4i*>((QUANTISE ? a_tile : st + b * 4096) + at_a[ks]);
 #pragma unroll
-            for (int b = 0; b < NB; ++b) fb[b][ks] = *reinterpret_cast<const v4i*>(st + (MB + b) * 4096 + at[ks]);
+            for (int b = 0; b < NB; ++b) fb[b][ks] = *reinterpret_cast<const v4i*>(st + B_AT + b * 4096 + at[ks]);
         }
         __builtin_amdgcn_sched_barrier(0);   // all reads go out before anything else
         if (!I32FULL) {
@@ -223,7 +253,7 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
             for (int a = 0; a < MB; ++a)
 #pragma unroll
                 for (int b = 0; b < NB; ++b) d[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[a][ks], fb[b][ks], !I32FULL && ks == 0 ? vzero : d[a][b], 0, 0, 0);
-        if (!I32FULL) f_prev = factor_of_step(i);
+        if (!I32FULL) f_prev = QUANTISE ? f_now : factor_of_step(i);
     }
     if (!I32FULL) fold();
     // every load (the redundant ones of the last steps included) has landed and every wave is
@@ -284,6 +314,10 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
 template <bool I32FULL, int BLOCKS>
 __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g) {
     wavering_block<I32FULL, BLOCKS>(g, blockIdx.x, blockIdx.y);
+}
+
+__global__ __launch_bounds__(256) void gemm_i8_decode_kernel(const GemmArgs g, const int rows) {
+    wavering_block<false, 1, true>(g, blockIdx.x, 0, rows);
 }
 
 // A GEMM over few K tiles: dW of a step on up to 256 tokens.  Its products are nothing beside its output, so this is made for
@@ -508,6 +542,14 @@ int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t s
                              : (i32_full ? gemm_i8_wavering_kernel<true, 1> : gemm_i8_wavering_kernel<false, 1>);
     hipLaunchKernelGGL(kernel, grid, dim3(256), wavering_lds_bytes(wide), st, a);
     note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
+    return check_launch("ti8_gemm_i8_nt");
+}
+
+int launch_decode(const GemmArgs& a, int rows, hipStream_t st) {
+    constexpr int lds = 4 * (WS_STAGES * 4096 + DECODE_A_BYTES);
+    static_assert(lds >= 4 * 4096 && lds <= 64 * 1024, "the waves' sums meet there");
+    hipLaunchKernelGGL(gemm_i8_decode_kernel, dim3((unsigned)(a.N / 32)), dim3(256), lds, st, a, rows);
+    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, EPI_PROMOTE);
     return check_launch("ti8_gemm_i8_nt");
 }
 

@@ -440,5 +440,14 @@ TI8_HD bool gemm_few_rows_prefers_mid(int64_t M, int64_t N, int64_t K, int64_t b
     return 7.0 + 0.5 * nk * (0.85 + 0.3 * tiles) < few_rows_time(M, N, K, batch, num_cu, few_rows_wide(M, N, K, batch, num_cu));
 }
 
+// Whether the few-rows kernel quantises up to 8 rows of bf16 itself.  A wave then spends about as long on a K tile's codes as on waiting for
+// the weight's next one: over many K tiles on few CUs that adds up to more than the launch that it saves.  us, apart / in the kernel,
+// 8 rows, calls one after another: K -> N 2048 -> 1024 12.7 / 10.5, 4096 -> 4096 13.3 / 10.3, 4096 -> 14336 15.6 / 11.9, 8192 -> 8192
+// 16.8 / 14.1, 12288 -> 4096 18.4 / 18.2, 14336 -> 1024 18.0 / 18.6, 14336 -> 5120 20.4 / 20.9, 14336 -> 7168 22.1 / 20.8,
+// 14336 -> 14336 35.4 / 31.3.
+TI8_HD bool decode_quantises(int64_t N, int64_t K, int num_cu) {
+    return K / 128 <= 96 || N / 32 * 4 >= (int64_t)num_cu * 3;
+}
+
 }  // namespace idx
 }  // namespace ti8
