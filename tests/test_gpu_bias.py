@@ -36,6 +36,16 @@ def test_bias_is_the_rounded_sum(T, dev, scheme, had, tokens, k, n):
         assert torch.equal(torch.nan_to_num(lin(x)), torch.nan_to_num(want))
 
 
+# what is left of the tilings: 128 x 128 on four waves, a round of 256 x 128; rows of scales on both operands and on neither
+@pytest.mark.parametrize("scheme,had", [("block_channel", None), ("block_channel", 128), ("row_block", None), ("double_channel", None)])
+@pytest.mark.parametrize("tokens,k,n", [(1400, 384, 3072), (2048, 256, 4096), (5000, 256, 2176)])
+def test_bias_in_the_epilogue_of_large_tiles(T, dev, scheme, had, tokens, k, n):
+    g = make_gen(tokens + n)
+    x, w, b = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, n, k).to(dev), randn_bf16(g, n, std=30.0).to(dev)
+    call = lambda bias: T.ops.linear_call(T._lib.PART_FORWARD, scheme, had, tokens, k, n, X=x, W=w, bias=bias)[0][:tokens]
+    assert torch.equal(call(b), call(None) + b)
+
+
 @pytest.mark.parametrize("rows,cols", [(1, 32), (5, 96), (16, 512), (17, 544), (1500, 5632), (4099, 128), (3000, 14336)])
 def test_column_sum(T, dev, rows, cols):
     g = make_gen(rows + cols)

@@ -89,3 +89,18 @@ def test_persistent_chain_kernel_waits_match_its_stores(tmp_path):
     assert str(stores_per_wave) in waits, waits              # first K tile of a tile: everything but the stores
     assert str(stores_per_wave + 4) in waits, waits          # next tile's factors: behind 4 operand loads and the stores
     assert all(int(w) <= stores_per_wave + 4 for w in waits), waits
+
+
+def test_chain_kernel_with_a_bias_waits_like_the_one_without(tmp_path):
+    """The same 16 stores of 16 bytes per wave and variant, nothing branching between them, no more waited for than without the bias,
+    and no scratch."""
+    text = open(compile_to_asm("gemm_chain.hip", tmp_path)).read()
+    body = text[text.index("gemm_i8_chain_bias_kernel"):]
+    body = body[:body.index(".end_amdhsa_kernel")]
+    assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", body)
+    stores = re.findall(r"^\s*(global_store_\w+|buffer_store_\w+|flat_store_\w+|scratch_store_\w+)", body, flags=re.M)
+    assert stores == ["global_store_dwordx4"] * (8 * 16)
+    for block in re.split(r"^\.LBB\S+:|^\s*s_cbranch\w+|^\s*s_branch", body, flags=re.M):
+        assert len(re.findall(r"^\s*global_store_dwordx4", block, flags=re.M)) in (0, 16)
+    waits = {int(w) for w in re.findall(r"s_waitcnt vmcnt\((\d+)\)", body)}
+    assert {16, 20} <= waits and max(waits) == 20

@@ -1,4 +1,5 @@
-// The bias of a linear layer: adding it to the output of a GEMM whose epilogue does not, and its gradient, the column sums of dY.
+// The bias of a linear layer: adding it behind the GEMMs of a whole step (a GEMM launched alone does that in its epilogue), and its
+// gradient, the column sums of dY.
 #include "ti8_common.h"
 
 namespace ti8 {

@@ -22,7 +22,7 @@ struct GemmArgs {
     int combine;
     int strict;
     float out_scale, post_scale;
-    const uint16_t* bias;   // bf16 [N], added to the rounded result and rounded again; the few-rows and the medium kernel only (else null)
+    const uint16_t* bias;   // bf16 [N], added to the rounded result and rounded again, or null; not with scales per (column of C, K tile)
 };
 
 // EPI_PROMOTE: the per-K-tile factor is uniform over a wave's tile (block or per-row scales

@@ -16,7 +16,8 @@
 // plus an immediate; one register holds the per-K-tile factors of 64 K tiles and is refilled every 64; the launcher
 // sends other shapes to the one-tile kernel).
 //
-// The body is shared by two kernels: gemm_i8_chain_kernel, whose per-K-tile factor is uniform over a wave's tile, and
+// The body is shared by three kernels: gemm_i8_chain_kernel, whose per-K-tile factor is uniform over a wave's tile, the same with a
+// bias in its epilogue (gemm_i8_chain_bias_kernel: nothing branches between the stores, whose number the waits count), and
 // gemm_i8_chain_lane_kernel, for operand B scaled per (row, K tile) (EPI_PROMOTE_CHAIN_LANE), where every lane fetches the
 // scales of its two columns one K tile ahead -- with the operand loads of that K tile, across tile boundaries too.
 #include <type_traits>
@@ -77,7 +78,7 @@ struct Tile {
 
 // LANEB: operand B has one scale per (row, K tile); `col_p` / `col_s` then lead to the K tile 0 scales of the wave tile's
 // columns, `fb_ks` from one K tile to the next.
-template <bool LANEB>
+template <bool LANEB, bool BIAS>
 __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_tiles) {
     extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
     // layout: [A buf0][A buf1][B buf0][B buf1][epilogue slab]
@@ -348,6 +349,11 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         const int64_t c_off = idx::epi_out_offset(t.batch, g.bsc, row0, g.ldc, t.n0 + wn * WCOLS + rb_col);
         const int64_t c_step = (int64_t)RPI * g.ldc;
         const float* prow0 = g.sa.p + idx::epi_row_scale_base(t.batch, g.sa.bs, row0, g.sa.rs);
+        uint4 bias = make_uint4(0, 0, 0, 0);     // of this lane's 8 columns, fetched (and waited for) before the first store
+        if (BIAS) {
+            bias = *reinterpret_cast<const uint4*>(g.bias + t.n0 + wn * WCOLS + rb_col);
+            asm volatile("" : "+v"(bias.x), "+v"(bias.y), "+v"(bias.z), "+v"(bias.w));
+        }
         auto store_tile = [&](auto extra_tag, auto mrow_tag, auto mcol_tag) {
             constexpr bool EXTRA = decltype(extra_tag)::value;
             constexpr bool MROW = decltype(mrow_tag)::value;
@@ -399,8 +405,9 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
                             if (EXTRA) v[c] = v[c] * g.out_scale;
                         }
                         // the ONE store of this (pass, k): EPILOGUE_STORES counts these
-                        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(g.C) + off) =
-                            make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+                        uint4 o = make_uint4(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]), pack_bf16x2(v[4], v[5]), pack_bf16x2(v[6], v[7]));
+                        if (BIAS) o = make_uint4(add_bf16x2(o.x, bias.x), add_bf16x2(o.y, bias.y), add_bf16x2(o.z, bias.z), add_bf16x2(o.w, bias.w));
+                        *reinterpret_cast<uint4*>(reinterpret_cast<uint16_t*>(g.C) + off) = o;
                     }
                     __builtin_amdgcn_s_waitcnt(0xc07f);
                     __builtin_amdgcn_wave_barrier();
@@ -534,17 +541,23 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
 }  // namespace
 
 __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti m, const int total_tiles) {
-    chain_tiles<false>(m, total_tiles);
+    chain_tiles<false, false>(m, total_tiles);
+}
+
+// one GEMM, with g.bias
+__global__ __launch_bounds__(64 * NW) void gemm_i8_chain_bias_kernel(const GemmMulti m, const int total_tiles) {
+    chain_tiles<false, true>(m, total_tiles);
 }
 
 __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_lane_kernel(const GemmMulti m, const int total_tiles) {
-    chain_tiles<true>(m, total_tiles);
+    chain_tiles<true, false>(m, total_tiles);
 }
 
 // operand B scaled per (row, K tile): all GEMMs of a launch or none
 static bool lane_scales(const GemmMulti& m) { return m.g[0].sb.mode == TI8_SCALE_ROW_K128; }
 
 bool chain_persistent_supported(const GemmMulti& m) {
+    if (m.g[0].bias && (m.count > 1 || lane_scales(m))) return false;
     for (int i = 0; i < m.count; ++i) {
         const int nk = m.g[i].K >> 7;
         if (nk < 2 || nk > 256 || (nk & 1) || m.g[i].strict) return false;
@@ -565,13 +578,16 @@ bool chain_persistent_supported(const GemmMulti& m) {
 // its batch count; one workgroup per CU (fewer when there are fewer tiles)
 // Whether the current device grants the kernel its 160 KiB of LDS (asked once per device).  A refusal is remembered
 // and reported through ti8_last_error() by the call that met it; callers then take the one-tile kernel.
-template <bool LANEB>
+enum ChainKernel { CHAIN, CHAIN_LANE, CHAIN_BIAS };
+typedef void (*ChainFunction)(GemmMulti, int);
+static ChainFunction chain_function(ChainKernel k) { return k == CHAIN_LANE ? gemm_i8_chain_lane_kernel : k == CHAIN_BIAS ? gemm_i8_chain_bias_kernel : gemm_i8_chain_kernel; }
+
+template <ChainKernel K>
 static bool chain_kernel_available() {
     static OncePerDevice granted, refused;
     const uint64_t bit = 1ull << (current_device() & 63);
     if (refused.done.load(std::memory_order_acquire) & bit) return false;
-    const void* kern = LANEB ? reinterpret_cast<const void*>(gemm_i8_chain_lane_kernel) : reinterpret_cast<const void*>(gemm_i8_chain_kernel);
-    const hipError_t e = raise_lds_limit(granted, kern, LDS_BYTES);
+    const hipError_t e = raise_lds_limit(granted, reinterpret_cast<const void*>(chain_function(K)), LDS_BYTES);
     if (e == hipSuccess) return true;
     refused.done.fetch_or(bit, std::memory_order_release);
     (void)fail(TI8_OK, "gemm: device %d refuses %d bytes of LDS for the persistent kernel (%s); one workgroup per tile serves its shapes",
@@ -580,17 +596,17 @@ static bool chain_kernel_available() {
 }
 
 int init_chain_kernel() {
-    (void)chain_kernel_available<false>();
-    (void)chain_kernel_available<true>();
+    (void)chain_kernel_available<CHAIN>();
+    (void)chain_kernel_available<CHAIN_LANE>();
+    (void)chain_kernel_available<CHAIN_BIAS>();
     return TI8_OK;
 }
 
 int launch_chain_persistent(const GemmMulti& m, int total_tiles, int num_cu, hipStream_t st) {
-    const bool lane = lane_scales(m);
-    if (!(lane ? chain_kernel_available<true>() : chain_kernel_available<false>())) return CHAIN_UNAVAILABLE;
+    const bool lane = lane_scales(m), biased = m.g[0].bias != nullptr;
+    if (!(lane ? chain_kernel_available<CHAIN_LANE>() : biased ? chain_kernel_available<CHAIN_BIAS>() : chain_kernel_available<CHAIN>())) return CHAIN_UNAVAILABLE;
     const int grid = total_tiles < num_cu ? total_tiles : num_cu;
-    const auto kernel = lane ? gemm_i8_chain_lane_kernel : gemm_i8_chain_kernel;
-    hipLaunchKernelGGL(kernel, dim3((unsigned)grid), dim3(64 * NW), LDS_BYTES, st, m, total_tiles);
+    hipLaunchKernelGGL(chain_function(lane ? CHAIN_LANE : biased ? CHAIN_BIAS : CHAIN), dim3((unsigned)grid), dim3(64 * NW), LDS_BYTES, st, m, total_tiles);
     note_gemm_kernel(TI8_KERNEL_PERSISTENT_CHAIN, BM, BN, lane ? EPI_PROMOTE_CHAIN_LANE : EPI_PROMOTE_CHAIN);
     return check_launch("ti8_gemm_i8_nt");
 }

@@ -318,13 +318,6 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
     return quant_call(fn, by_block, by_block_rows, nblocks, both, nboth, q, inv, stream);
 }
 
-// One GEMM launched alone (what ti8_gemm_i8_nt selects for its shape: the few-rows kernel up to 256 rows)
-int one_gemm(const ti8_gemm_problem& q, const void* bias, int64_t tokens, int gemm_flags, ti8_stream_t stream) {
-    bool added = false;
-    if (int e = gemm_nt_bias(q, bias, gemm_flags, &added, stream)) return e;
-    return bias && !added ? add_bias(q.C, q.ldc, bias, tokens, q.N, stream) : TI8_OK;
-}
-
 int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t stream) {
     const int flags = L.a->gemm_flags;
     // rows of a token operand to multiply: all of them, or with up to 256 (padded) tokens the real ones rounded up to 32 (the padding
@@ -350,7 +343,8 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
         if (int e = gemm_nt_few(few, count, L.bwd, bias, flags, launched, stream)) return e;
     for (int i = 0; i < count; ++i)
         if (!launched[i])
-            if (int e = one_gemm(few[i], i == 0 ? bias : nullptr, L.tokens, flags, stream)) return e;
+            // launched alone: what ti8_gemm_i8_nt selects for its shape (the few-rows kernel up to 256 rows)
+            if (int e = gemm_nt_bias(few[i], i == 0 ? bias : nullptr, flags, stream)) return e;
     return TI8_OK;
 }
 

@@ -90,8 +90,8 @@ int quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q,
                              ti8_stream_t stream);
 int fwht_t_quant_row_valid(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t valid_rows, int64_t C,
                            int qflags, int inv_mode, ti8_stream_t stream);
-// ti8_gemm_i8_nt with a bias for the kernels whose epilogue adds one (*added: this was one); y += bias behind the others (bias.hip)
-int gemm_nt_bias(const ti8_gemm_problem& p, const void* bias, int gemm_flags, bool* added, ti8_stream_t stream);
+// ti8_gemm_i8_nt with a bias, which the epilogue adds; y += bias behind the GEMMs of a whole step (bias.hip)
+int gemm_nt_bias(const ti8_gemm_problem& p, const void* bias, int gemm_flags, ti8_stream_t stream);
 // gemm.hip: the GEMMs of a call on few tokens as one launch, those that go into it (see there)
 int gemm_nt_few(const ti8_gemm_problem* problems, int count, bool backward, const void* bias, int gemm_flags, bool* launched, ti8_stream_t stream);
 // Y of 1 to 8 rows of bf16 that the GEMM's kernel quantises itself (`p` describes what it would be with the quantiser apart); *done tells
