@@ -361,15 +361,16 @@ int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count, int gemm_f
  * its own allocations).  The same quantisers and GEMMs as through the separate entry points, the GEMM kernels chosen for the call
  * as a whole (TI8_GEMM_TOGETHER), with the same bits:
  *   TI8_SCHEME_BLOCK_CHANNEL   ti8_quant_block_multi(X, dY; q and qT) -> ti8_quant_row_col_t(W) ->
- *                              ti8_gemm_i8_nt_multi(Y, dX, dW)          (3 launches + W's absmax pass)
+ *                              ti8_gemm_i8_nt_multi(Y, dX, dW)
  *   TI8_SCHEME_DOUBLE_CHANNEL  ti8_quant_row_col_t on X, W, dY (TI8_INV_AMAX_DIV_127) ->
  *                              ti8_gemm_i8_nt_multi(Y, dX, dW; acc_i32_full = 1)
+ * Up to 320 MiB of operands the quantisers are two launches together.
  *   X bf16 [T][K] (ldx), W bf16 [N][K] (ldw), dY bf16 [T][N] (lddy)  ->  Y bf16 [T][N], dX bf16 [T][K], dW bf16 [N][K]
  *   All six 16-byte aligned, leading dimensions multiples of 8 elements; every argument is checked before the first launch.
  *   T, K, N multiples of 128.  `tokens` (1 <= tokens <= T) = the rows of X and dY that exist; the rest of the T rows
  *   counts as zeros and is not read (zeros change no absmax and add nothing to dW).  With
- *   T <= 256 or N <= 256 the GEMMs are launched one by one, as ti8_gemm_i8_nt would launch them (few-rows kernel up to 256
- *   rows), and Y and dX are computed for the first ceil(tokens / 32) * 32 rows only.
+ *   T <= 256 or N <= 256 each GEMM takes the kernel that ti8_gemm_i8_nt would (few-rows kernel up to 256 rows; those on it,
+ *   and dW over one or two K tiles, in one launch), and Y and dX are computed for the first ceil(tokens / 32) * 32 rows only.
  *   workspace: ti8_linear_fwd_bwd_workspace(T, K, N, scheme) bytes of device memory, 256-byte aligned, contents
  *   undefined before and after (it holds the int8 operands, their transposes, scales and maxima; the call clears
  *   what it needs cleared itself, so the same buffer serves any sequence of calls in stream order).
@@ -429,8 +430,8 @@ int64_t ti8_linear_workspace(const ti8_linear_args* a, int64_t* saved_bytes);
  * M = T for Y and dX), for ti8_gemm_i8_nt_multi */
 int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, int* count, ti8_stream_t stream);
 /* enqueue everything.  With more than 256 (padded) tokens and output features the GEMMs of a call go through
- * ti8_gemm_i8_nt_multi (TI8_PART_FORWARD alone: ti8_gemm_i8_nt, the same kernel), else they are launched one by one as
- * ti8_gemm_i8_nt launches them, Y and dX for the first ceil(tokens / 32) * 32 rows only. */
+ * ti8_gemm_i8_nt_multi (TI8_PART_FORWARD alone: ti8_gemm_i8_nt, the same kernel), else each takes the kernel of ti8_gemm_i8_nt
+ * (those on the few-rows kernel in one launch; up to 8 rows may be quantised inside it), Y and dX for the first ceil(tokens / 32) * 32 rows only. */
 int ti8_linear(const ti8_linear_args* a, ti8_stream_t stream);
 /* Column sums of x bf16 [rows][cols] (ldx), added up in fp32 and rounded once: the gradient of a bias.  cols a multiple of 32;
  * workspace: ti8_column_sum_workspace bytes (-1 for sizes it does not take), 16-byte aligned. */

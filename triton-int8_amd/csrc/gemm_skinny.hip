@@ -2,7 +2,7 @@
 //
 // With so few rows the tiled kernel of gemm.hip has only N/128 workgroups, and each walks the
 // whole K behind a two-stage LDS pipeline: its time is load latency, not MFMA.  Here C is cut
-// into 32 x 32 blocks, one per workgroup, (N/32) * (M/32) of them, and K is split over the four
+// into 32 x 32 blocks, one or four per workgroup, and K is split over the four
 // waves of the workgroup, each of which runs its own load -> LDS -> MFMA pipeline with no
 // barrier in the loop.
 //
@@ -19,7 +19,7 @@ namespace ti8 {
 // expcnt untouched (bits 6:4)
 #define TI8_WAIT_VMCNT_LGKM0(n) __builtin_amdgcn_s_waitcnt(((n) & 0xf) | (((n) >> 4) << 14) | 0x0070)
 
-// A workgroup owns 32 x 32 of C and its four waves split K into quarters.  Every wave streams ITS
+// A workgroup owns 32 x 32 of C (or 64 x 64, with twice the stages' bytes) and its four waves split K into quarters.  Every wave streams ITS
 // quarter of both operands through a private LDS ring (WS_STAGES stages of [A 32 rows][B 32 rows]
 // = 8 KiB, filled by global_load_lds in the swizzled layout of the tiled kernel), waits only
 // for its own loads and never for another wave; the four partial results meet in LDS at the end
