@@ -62,3 +62,22 @@ def test_step_into_given_outputs(dev, scheme, layout):
         assert all(bool((torch.as_strided(o, (o.shape[0], 64), (o.stride(0), 1), o.storage_offset() + o.shape[1]) == -3.0).all()) for o in out)
     for a, b in zip(got, want):
         assert torch.equal(a, b)
+
+
+# a wave per row and a workgroup per row, the longest row of either and the shortest of the next (more than 16384: a launch of its own);
+# a whole step, a forward that leaves W^T behind, one that does not
+@pytest.mark.parametrize("k", [4096, 4224, 16384, 16512])
+@pytest.mark.parametrize("tokens", [5, 130])
+def test_rows_beside_the_blocks(dev, monkeypatch, tokens, k):
+    import triton_int8_amd as T
+    from triton_int8_amd._lib import PART_FORWARD, PART_KEEP
+    g = make_gen(tokens + k)
+    n = 256
+    X, W, dY = randn_bf16(g, tokens, k + 8).to(dev)[:, :k], randn_bf16(g, n, k).to(dev), randn_bf16(g, tokens, n).to(dev)
+    X[tokens - 1, k - 1] = 300.0
+    got = T.linear_fwd_bwd(X, W, dY, "row_block")
+    forward = [T.ops.linear_call(PART_FORWARD | keep, "row_block", None, tokens, k, n, X=X, W=W)[0][:tokens] for keep in (0, PART_KEEP)]
+    monkeypatch.setattr(T.linear, "ONE_CALL_STEP", False)
+    for a, c in zip(got, T.linear_fwd_bwd(X, W, dY, "row_block")):
+        assert torch.equal(a, c)
+    assert torch.equal(forward[0], got[0]) and torch.equal(forward[1], got[0])

@@ -373,14 +373,11 @@ __global__ __launch_bounds__(256) void quant_block_had_kernel(
 // NLOAD 16-byte chunks of its row in registers.  GROUP16: one scale per 16 chunks
 // (128 columns) instead of per row.
 template <int NLOAD, bool WG_ROW, bool GROUP16, bool HAD, int ARITH = ARITH_KERNEL>
-__global__ __launch_bounds__(256) void quant_row_kernel(const uint16_t* __restrict__ x, int64_t ldx,
-                                                        int8_t* __restrict__ q, int64_t ldq,
-                                                        float* __restrict__ s, int64_t rows, int cols,
-                                                        QMode mode) {
-    __shared__ float red4[4];
+__device__ __forceinline__ void quant_row_part(const uint16_t* __restrict__ x, int64_t ldx, int8_t* __restrict__ q, int64_t ldq, float* __restrict__ s, int64_t rows,
+                                               int cols, const QMode& mode, const int block, float* red4) {
     constexpr int T = WG_ROW ? 256 : 64;
     const int t = WG_ROW ? threadIdx.x : (threadIdx.x & 63);
-    const int64_t row = idx::qrow_row(blockIdx.x, threadIdx.x >> 6, WG_ROW);
+    const int64_t row = idx::qrow_row(block, threadIdx.x >> 6, WG_ROW);
     if (row >= rows) return;  // whole wave (or workgroup) leaves together
     const int nchunk = cols >> 3;
     const uint16_t* xr = x + row * ldx;
@@ -428,6 +425,13 @@ __global__ __launch_bounds__(256) void quant_row_kernel(const uint16_t* __restri
         const int c = HAD ? idx::had_chunk(idx::qrow_chunk(t, i, T)) : idx::qrow_chunk(t, i, T);
         if (c < nchunk) *reinterpret_cast<uint2*>(qr + c * 8) = quant8<ARITH>(v[i], scale * lane_sign);
     }
+}
+
+template <int NLOAD, bool WG_ROW, bool GROUP16, bool HAD, int ARITH = ARITH_KERNEL>
+__global__ __launch_bounds__(256) void quant_row_kernel(const uint16_t* __restrict__ x, int64_t ldx, int8_t* __restrict__ q, int64_t ldq, float* __restrict__ s,
+                                                        int64_t rows, int cols, QMode mode) {
+    __shared__ float red4[4];
+    quant_row_part<NLOAD, WG_ROW, GROUP16, HAD, ARITH>(x, ldx, q, ldq, s, rows, cols, mode, (int)blockIdx.x, red4);
 }
 
 struct ClearRanges {    // words to zero, one behind the other
@@ -824,15 +828,29 @@ __device__ __forceinline__ void maxima_part(const MaxOperand& o, const int part,
             *reinterpret_cast<uint4*>(o.rows + (int64_t)ct * o.R + (rt * o.tr + a) * 128 + rg * 8) = *reinterpret_cast<const uint4*>(rowmax + a * 128 + rg * 8);
 }
 
+// An operand quantised by rows alone, by workgroups in front of the block tiles (row-block: X, whose rows the same launch reads for X^T).
+// Steps, us, in a launch of its own / here: 16 tokens 4096 -> 4096 37.7 / 33.9, 700 tokens 4096 -> 11008 202 / 198, 3072 tokens 4096 -> 4096
+// 207 / 205.
+struct RowPart {
+    QRowOperand op;
+    int workgroups;     // a multiple of 8
+};
+constexpr int ROW_PART_COLS = 16384;     // 8 chunks per thread of a workgroup
+
 constexpr int MAXIMA_ROW_TILES = 64;     // 128-row tiles whose row maxima a workgroup keeps in LDS
-__global__ __launch_bounds__(256) void quant_first_kernel(const MaxMulti maxima, const QBlockMulti blocks, QMode mode) {
+__global__ __launch_bounds__(256) void quant_first_kernel(const MaxMulti maxima, const QBlockMulti blocks, const RowPart rows, QMode mode) {
     __shared__ float red4[4];
     __shared__ __attribute__((aligned(16))) uint32_t tileT[128 * 33];
     __shared__ uint4 colpart[4][16];
     static_assert(MAXIMA_ROW_TILES * 128 * 2 <= (int)sizeof(tileT), "row maxima share the transposed tile's LDS");
-    const int block_tiles = blocks.first[QBLOCK_MULTI_MAX], part = (int)blockIdx.x - block_tiles;
-    if (part < 0) {
-        if ((int)blockIdx.x < blocks.first[blocks.count]) quant_block_of<true, true>(blocks, (int)blockIdx.x, mode, red4, tileT);
+    const int tile = (int)blockIdx.x - rows.workgroups, part = tile - blocks.first[QBLOCK_MULTI_MAX];
+    if (tile < 0) {
+        const QRowOperand& o = rows.op;
+        const uint16_t* const x = static_cast<const uint16_t*>(o.x);
+        if (o.C <= 4096) quant_row_part<8, false, false, false>(x, o.ldx, o.q, o.C, o.s, o.R, (int)o.C, mode, (int)blockIdx.x, red4);
+        else quant_row_part<8, true, false, false>(x, o.ldx, o.q, o.C, o.s, o.R, (int)o.C, mode, (int)blockIdx.x, red4);
+    } else if (part < 0) {
+        if (tile < blocks.first[blocks.count]) quant_block_of<true, true>(blocks, tile, mode, red4, tileT);
     } else {
         int i = 0;
 #pragma unroll
@@ -1029,14 +1047,8 @@ int64_t ti8::quant_maxima_words(int64_t R, int64_t C) {
     return (parts_of(C, tc) * R + parts_of(R, tr) * C) / 2;
 }
 
-int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int64_t* block_rows, int nblocks, const QRowColOperand* both, int nboth, int qflags,
-                    int inv_mode, ti8_stream_t stream) {
-    bool same = true;
-    for (int i = 1; i < nblocks; ++i) same = same && !blocks[i].q == !blocks[0].q && !blocks[i].qT == !blocks[0].qT;
-    if (nblocks && !nboth && same) return quant_block_multi_valid(blocks, block_rows, nblocks, qflags, inv_mode, stream);
-    if (!nblocks && !nboth) return TI8_OK;
-    QMode mode;
-    if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
+int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int64_t* block_rows, int nblocks, const QRowColOperand* both, int nboth,
+                    const QRowOperand* rows, int qflags, int inv_mode, ti8_stream_t stream) {
     int64_t bytes = 0;
     bool atomics = false;
     for (int i = 0; i < nboth; ++i) {
@@ -1044,6 +1056,16 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
         atomics = atomics || !both[i].partial;
     }
     atomics = atomics || bytes > TOGETHER_BYTES;
+    if (rows && (atomics || nblocks + nboth == 0 || rows->C > ROW_PART_COLS)) {
+        if (int e = ti8_quant_row(rows->x, rows->ldx, rows->q, rows->C, rows->s, rows->R, rows->C, 0, qflags, inv_mode, stream)) return e;
+        rows = nullptr;
+    }
+    bool same = !rows;
+    for (int i = 1; i < nblocks; ++i) same = same && !blocks[i].q == !blocks[0].q && !blocks[i].qT == !blocks[0].qT;
+    if (nblocks && !nboth && same) return quant_block_multi_valid(blocks, block_rows, nblocks, qflags, inv_mode, stream);
+    if (!nblocks && !nboth) return TI8_OK;
+    QMode mode;
+    if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
     if (nblocks >= QBLOCK_MULTI_MAX || nboth > MAX_OPERANDS || (qflags & TI8_Q_HAD128)) return fail(TI8_ERR_MODE, "%s: unsupported set of operands", fn);
     QBlockMulti b;
     int64_t block_tiles = 0;
@@ -1092,9 +1114,15 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
             launch_row_col(static_cast<const uint16_t*>(o.x), o.ldx, o.q, o.C, o.s_row, o.qT, o.R, o.s_col, o.maxima, nullptr, o.R, o.valid_rows, o.C, mode, st);
         }
         if (int e = check_launch(fn)) return e;
-        return nblocks ? quant_call(fn, blocks, block_rows, nblocks, nullptr, 0, qflags, inv_mode, stream) : TI8_OK;
+        return nblocks ? quant_call(fn, blocks, block_rows, nblocks, nullptr, 0, nullptr, qflags, inv_mode, stream) : TI8_OK;
     }
-    hipLaunchKernelGGL(quant_first_kernel, dim3((unsigned)(parts + block_tiles)), dim3(256), 0, st, m, b, mode);
+    RowPart r = {};
+    if (rows) {
+        r.op = *rows;
+        r.workgroups = (int)round8(rows->C <= 4096 ? (rows->R + 3) / 4 : rows->R);
+        if (parts + block_tiles + r.workgroups > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
+    }
+    hipLaunchKernelGGL(quant_first_kernel, dim3((unsigned)(parts + block_tiles + r.workgroups)), dim3(256), 0, st, m, b, r, mode);
     if (int e = check_launch(fn)) return e;
     if (!nboth) return TI8_OK;
     for (int i = 0; i < MAX_OPERANDS; ++i) m.first[i] = (int)first_tile[i];

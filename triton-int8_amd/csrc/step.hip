@@ -214,6 +214,8 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
     int64_t by_block_rows[4];
     QRowColOperand both[3];
     int nblocks = 0, nboth = 0;
+    const QRowOperand x_rows = {a.X, a.ldx, L.xq, L.xs, tok, K};
+    const QRowOperand* by_rows = nullptr;
     // (`out`, `ldout`: the output of the operand's own shape, which a whole step does not write before its GEMMs; the partial maxima
     // live there until the conversion has read them, unless the caller's tensors overlap)
     const bool apart = outputs_apart(a, T);
@@ -245,11 +247,12 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
             else if (!L.given_w())
                 if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q, inv, stream)) return e;
         } else if (L.row_block()) {
-            if (int e = ti8_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, 0, q | had, inv, stream)) return e;
             if (L.had) {
+                if (int e = ti8_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, 0, q | had, inv, stream)) return e;
                 if (!L.given_w()) if (int e = ti8_quant_block_had128(a.W, 0, a.ldw, L.wq, N * K, K, L.ws, 0, K / 128, 1, 1, N, K, 0, q, inv, stream)) return e;
-            } else if (!L.given_w()) {
-                block(blocks(a.W, a.ldw, L.wq, shared ? L.wtq : nullptr, L.ws, N, K), N);
+            } else {
+                by_rows = &x_rows;
+                if (!L.given_w()) block(blocks(a.W, a.ldw, L.wq, shared ? L.wtq : nullptr, L.ws, N, K), N);
             }
         } else if (L.had) {
             post = (float)(1.0 / (double)K);
@@ -315,7 +318,7 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
         g[n++] = gemm2d(L.dytq, L.dyts, dyt_mode, dyts_rs, dyts_ks, L.xtq, L.xts, xt_mode, xts_rs, xts_ks, a.dW, a.lddw, N, K, T, L.dbl(), rot, post_dw);
     }
     *count = n;
-    return quant_call(fn, by_block, by_block_rows, nblocks, both, nboth, q, inv, stream);
+    return quant_call(fn, by_block, by_block_rows, nblocks, both, nboth, by_rows, q, inv, stream);
 }
 
 int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t stream) {

@@ -80,9 +80,18 @@ struct QRowColOperand {
     int64_t R, valid_rows, C;
 };
 int64_t quant_maxima_words(int64_t R, int64_t C);
-// Block-quantised operands and operands quantised both ways (up to 4 and 3) in two launches, one where there are none of the latter
-int quant_call(const char* fn, const ti8_qblock_operand* blocks, const int64_t* block_rows, int nblocks, const QRowColOperand* both, int nboth, int qflags,
-               int inv_mode, ti8_stream_t stream);
+// An operand quantised by rows alone, dense codes
+struct QRowOperand {
+    const void* x;
+    int64_t ldx;
+    int8_t* q;
+    float* s;
+    int64_t R, C;
+};
+// Block-quantised operands, operands quantised both ways (up to 4 and 3) and one quantised by rows (or null) in two launches, one where there
+// are none of the second kind
+int quant_call(const char* fn, const ti8_qblock_operand* blocks, const int64_t* block_rows, int nblocks, const QRowColOperand* both, int nboth,
+               const QRowOperand* rows, int qflags, int inv_mode, ti8_stream_t stream);
 int quant_col_t_valid(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt, float* s, float* ws, int64_t R, int64_t valid_rows, int64_t C,
                       int qflags, int inv_mode, ti8_stream_t stream);
 int quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq, float* s, int64_t ssb, int64_t ssr,
