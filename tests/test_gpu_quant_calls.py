@@ -81,3 +81,22 @@ def test_rows_beside_the_blocks(dev, monkeypatch, tokens, k):
     for a, c in zip(got, T.linear_fwd_bwd(X, W, dY, "row_block")):
         assert torch.equal(a, c)
     assert torch.equal(forward[0], got[0]) and torch.equal(forward[1], got[0])
+
+
+# a workgroup per row up to 256 rows, a wave per row beyond; the shortest and the longest row of the former and their neighbours
+@pytest.mark.parametrize("rows", [1, 255, 256, 257])
+@pytest.mark.parametrize("cols", [512, 640, 4096, 4224])
+def test_few_rows_quantised(dev, rows, cols):
+    import triton_int8_amd as T
+    x = randn_bf16(make_gen(rows + cols), rows, cols + 16).to(dev)[:, :cols]
+    x[rows // 2, cols - 1] = 50.0
+    x[0] = 0.0
+    q, s = T.ops.quant_row(x, inv_mode=T._lib.INV_AMAX_DIV_127)
+    many = torch.zeros((300, cols), dtype=torch.bfloat16, device=dev)       # each row by itself: others do not change it
+    many[:rows] = x
+    want, scale = T.ops.quant_row(many, inv_mode=T._lib.INV_AMAX_DIV_127)
+    assert torch.equal(q, want[:rows]) and torch.equal(s, scale[:rows])
+    amax = x.float().abs().amax(1).clamp(min=1e-4)
+    # tensors on both sides of a division: one rounding (a number over a tensor is 127 times the reciprocal to torch, two)
+    scale = torch.full_like(amax, 127.0) / amax
+    assert torch.equal(q.float(), torch.floor(x.float() * scale[:, None] + 0.5).clamp(-128, 127)) and torch.equal(s, amax / torch.full_like(amax, 127.0))
