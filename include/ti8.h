@@ -431,7 +431,7 @@ int64_t ti8_linear_workspace(const ti8_linear_args* a, int64_t* saved_bytes);
 int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, int* count, ti8_stream_t stream);
 /* enqueue everything.  With more than 256 (padded) tokens and output features the GEMMs of a call go through
  * ti8_gemm_i8_nt_multi (TI8_PART_FORWARD alone: ti8_gemm_i8_nt, the same kernel), else each takes the kernel of ti8_gemm_i8_nt
- * (those on the few-rows kernel in one launch; up to 8 rows may be quantised inside it), Y and dX for the first ceil(tokens / 32) * 32 rows only. */
+ * (those on the few-rows kernel in one launch; up to 8 unrotated rows may be quantised inside it), Y and dX for the first ceil(tokens / 32) * 32 rows only. */
 int ti8_linear(const ti8_linear_args* a, ti8_stream_t stream);
 /* Column sums of x bf16 [rows][cols] (ldx), added up in fp32 and rounded once: the gradient of a bias.  cols a multiple of 32;
  * workspace: ti8_column_sum_workspace bytes (-1 for sizes it does not take), 16-byte aligned. */

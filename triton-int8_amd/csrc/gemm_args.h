@@ -86,9 +86,10 @@ int launch_mid(GemmMulti& m, int64_t batch, bool i32_full, hipStream_t st);
 // scales.  i32_full: int32 accumulation over the whole K with per-row scales (bit-exact path).
 bool skinny_supported(const GemmArgs& a);
 int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t st);
-// The same for up to 8 rows of bf16 (a.A, a.lda in elements) that the kernel quantises by their K tiles itself; operand B by rows
+// The same for up to 8 rows of bf16 (a.A, a.lda in elements) that the kernel quantises itself, as a.sa.mode says: by K tiles
+// (TI8_SCALE_BLOCK128, reciprocal scales) or by rows (absmax / 127 with i32_full, else reciprocal scales)
 constexpr int DECODE_ROWS = 8;
-int launch_decode(const GemmArgs& a, int rows, hipStream_t st);
+int launch_decode(const GemmArgs& a, int rows, bool i32_full, hipStream_t st);
 // GEMMs over at most two K tiles, on 128 x 128 tiles: dW of a step on few tokens
 bool thin_supported(const GemmArgs& a, bool i32_full);
 // several GEMMs of batch 1 in one launch, the first `few` of m.g on the few-rows kernel, one behind them on thin tiles; fills first[] of `m`

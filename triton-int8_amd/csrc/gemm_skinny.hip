@@ -37,12 +37,15 @@ constexpr int DECODE_A_BYTES = DECODE_ROWS * 128;    // a K tile of A that the w
 // product.  idx::few_rows_wide says where which is the faster one.  us, one block / four, int32 path: 64 rows, 4096 -> 14336
 // 21.0 / 15.3; 128 rows 4096 -> 4096 10.1 / 10.1, 8192 -> 8192 33.4 / 21.1; 256 rows 4096 -> 4096 16.7 / 10.8, 14336 -> 4096 98 / 36;
 // 64 rows, 14336 -> 14336 46.6 / 32.1 (31.6 for the weight alone).
-// QUANTISE: operand A is bf16 (g.A, g.lda in elements), 1 to 8 rows, and each wave quantises the 128 columns of its K tile by their
-// absmax (the block quantiser's arithmetic) on the way to LDS, one 16-byte chunk of a row per lane.  The missing ones of the 32 rows are
-// copies of those 8, and missing ones of the 8 copies of the last: rows of C that nobody reads.
-template <bool I32FULL, int BLOCKS, bool QUANTISE = false>
+// QUANTISE: operand A is bf16 (g.A, g.lda in elements), 1 to 8 rows, and each wave quantises the 128 columns of its K tile on the way to
+// LDS, one 16-byte chunk of a row per lane, with the quantisers' own arithmetic: by the absmax of the K tile (BY_TILES), or of the row
+// (BY_ROWS), which every workgroup looks for first.  The missing ones of the 32 rows are copies of those 8, and missing ones of the 8 copies
+// of the last: rows of C that nobody reads.
+enum Quantise { APART, BY_TILES, BY_ROWS };
+template <bool I32FULL, int BLOCKS, Quantise QUANTISE = APART>
 __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int block_x, const int batch, const int rows = 0) {
-    static_assert(!QUANTISE || (!I32FULL && BLOCKS == 1), "quantised by K tiles, up to 8 rows");
+    static_assert(QUANTISE == APART || BLOCKS == 1, "up to 8 rows");
+    static_assert(QUANTISE != BY_TILES || !I32FULL, "a scale per K tile");
     constexpr int MB = BLOCKS, NB = BLOCKS;
     constexpr int B_AT = QUANTISE ? 0 : MB * 4096, STAGE_BYTES = B_AT + NB * 4096;     // per wave
     extern __shared__ __attribute__((aligned(1024))) int8_t smem[];  // 4 waves x WS_STAGES x STAGE_BYTES
@@ -114,7 +117,7 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
     const bool divide = !I32FULL && g.combine == TI8_COMBINE_DIV_PROD;
     const bool a_in = !I32FULL && g.sa.mode != TI8_SCALE_ROW, b_in = !I32FULL && g.sb.mode != TI8_SCALE_ROW;
     float fvec[4] = {1.0f, 1.0f, 1.0f, 1.0f};
-    if (!I32FULL && !QUANTISE) {
+    if (!I32FULL && QUANTISE != BY_TILES) {
         const int sha = g.sa.mode == TI8_SCALE_BLOCK_K256 ? 1 : 0, shb = g.sb.mode == TI8_SCALE_BLOCK_K256 ? 1 : 0;
         const float* pa = g.sa.p + (int64_t)batch * g.sa.bs + (a_in ? (int64_t)(m0 >> 7) * g.sa.rs : 0);
         const float* pb = g.sb.p + (int64_t)batch * g.sb.bs + (b_in ? (int64_t)(n0 >> 7) * g.sb.rs : 0);
@@ -196,6 +199,22 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
         for (int c = 0; c < 4; ++c) asm volatile("" : "+v"(coln[b][c]));
     }
 
+    float row_mult = 0.0f;      // BY_ROWS: of this lane's row of A
+    if (QUANTISE == BY_ROWS) {
+        float amax = 0.0f;
+#pragma unroll 4
+        for (int kt = kbeg; kt < kend; ++kt)
+            amax = absmax8(*reinterpret_cast<const uint4*>(x + kt * 128 + 8), absmax8(*reinterpret_cast<const uint4*>(x + kt * 128), amax));
+        amax = dpp_max<0x141>(dpp_max<0x4E>(dpp_max<0xB1>(amax)));      // over the 8 lanes of a row
+        float* const red = reinterpret_cast<float*>(smem + 4 * (WS_STAGES * STAGE_BYTES + DECODE_A_BYTES));     // [wave][row]
+        if ((lane & 7) == 0) red[wave * DECODE_ROWS + ld_row] = amax;
+        __syncthreads();
+        auto of_row = [&](int r) { return amax_floor(fmaxf(fmaxf(red[r], red[DECODE_ROWS + r]), fmaxf(red[2 * DECODE_ROWS + r], red[3 * DECODE_ROWS + r])), 0); };
+        row_mult = 127.0f / of_row(ld_row);
+        const float out_amax = of_row(e_row & (DECODE_ROWS - 1));
+        rowm[0] = I32FULL ? out_amax / 127.0f : 1.0f / (127.0f / out_amax);
+    }
+
     auto factor_of_step = [&](int i) -> float {
         const int kt = tile_of_step(i);
         const int l = kt & 63, c = kt >> 6;
@@ -226,9 +245,12 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
         const int8_t* st = ring + (i & (WS_STAGES - 1)) * STAGE_BYTES;
         float f_now = 0.0f;
         if (QUANTISE) {
-            const float amax = amax_floor(wave_max(absmax8(now_hi, absmax8(now_lo, 0.0f))), 0);
-            const float scale = 127.0f / amax;
-            f_now = 1.0f / scale;
+            float scale = row_mult;
+            if (QUANTISE == BY_TILES) {
+                const float amax = amax_floor(wave_max(absmax8(now_hi, absmax8(now_lo, 0.0f))), 0);
+                scale = 127.0f / amax;
+                f_now = 1.0f / scale;
+            }
             const uint2 lo = quant8(now_lo, scale), hi = quant8(now_hi, scale);
             const v4i codes = {(int)lo.x, (int)lo.y, (int)hi.x, (int)hi.y};
             // (a store that the compiler knew of would wait for the loads in flight to LDS; a wave's LDS instructions stay in order)
@@ -253,7 +275,7 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
             for (int a = 0; a < MB; ++a)
 #pragma unroll
                 for (int b = 0; b < NB; ++b) d[a][b] = __builtin_amdgcn_mfma_i32_32x32x32_i8(fa[a][ks], fb[b][ks], !I32FULL && ks == 0 ? vzero : d[a][b], 0, 0, 0);
-        if (!I32FULL) f_prev = QUANTISE ? f_now : factor_of_step(i);
+        if (!I32FULL) f_prev = QUANTISE == BY_TILES ? f_now : factor_of_step(i);
     }
     if (!I32FULL) fold();
     // every load (the redundant ones of the last steps included) has landed and every wave is
@@ -316,8 +338,9 @@ __global__ __launch_bounds__(256) void gemm_i8_wavering_kernel(const GemmArgs g)
     wavering_block<I32FULL, BLOCKS>(g, blockIdx.x, blockIdx.y);
 }
 
+template <bool I32FULL, Quantise QUANTISE>
 __global__ __launch_bounds__(256) void gemm_i8_decode_kernel(const GemmArgs g, const int rows) {
-    wavering_block<false, 1, true>(g, blockIdx.x, 0, rows);
+    wavering_block<I32FULL, 1, QUANTISE>(g, blockIdx.x, 0, rows);
 }
 
 // A GEMM over few K tiles: dW of a step on up to 256 tokens.  Its products are nothing beside its output, so this is made for
@@ -545,11 +568,13 @@ int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t s
     return check_launch("ti8_gemm_i8_nt");
 }
 
-int launch_decode(const GemmArgs& a, int rows, hipStream_t st) {
-    constexpr int lds = 4 * (WS_STAGES * 4096 + DECODE_A_BYTES);
+int launch_decode(const GemmArgs& a, int rows, bool i32_full, hipStream_t st) {
+    constexpr int lds = 4 * (WS_STAGES * 4096 + DECODE_A_BYTES) + 4 * DECODE_ROWS * 4;
     static_assert(lds >= 4 * 4096 && lds <= 64 * 1024, "the waves' sums meet there");
-    hipLaunchKernelGGL(gemm_i8_decode_kernel, dim3((unsigned)(a.N / 32)), dim3(256), lds, st, a, rows);
-    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, EPI_PROMOTE);
+    const auto kernel = i32_full ? gemm_i8_decode_kernel<true, BY_ROWS>
+                                 : a.sa.mode == TI8_SCALE_ROW ? gemm_i8_decode_kernel<false, BY_ROWS> : gemm_i8_decode_kernel<false, BY_TILES>;
+    hipLaunchKernelGGL(kernel, dim3((unsigned)(a.N / 32)), dim3(256), lds, st, a, rows);
+    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
     return check_launch("ti8_gemm_i8_nt");
 }
 

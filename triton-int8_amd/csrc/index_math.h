@@ -449,9 +449,11 @@ TI8_HD bool gemm_few_rows_prefers_mid(int64_t M, int64_t N, int64_t K, int64_t b
 // the weight's next one: over many K tiles on few CUs that adds up to more than the launch that it saves.  us, apart / in the kernel,
 // 8 rows, calls one after another: K -> N 2048 -> 1024 12.7 / 10.5, 4096 -> 4096 13.3 / 10.3, 4096 -> 14336 15.6 / 11.9, 8192 -> 8192
 // 16.8 / 14.1, 12288 -> 4096 18.4 / 18.2, 14336 -> 1024 18.0 / 18.6, 14336 -> 5120 20.4 / 20.9, 14336 -> 7168 22.1 / 20.8,
-// 14336 -> 14336 35.4 / 31.3.
-TI8_HD bool decode_quantises(int64_t N, int64_t K, int num_cu) {
-    return K / 128 <= 96 || N / 32 * 4 >= (int64_t)num_cu * 3;
+// 14336 -> 14336 35.4 / 31.3.  By rows, which are read twice: 2048 -> 1024 14.1 / 11.1, 4096 -> 4096 14.0 / 10.8, 4096 -> 14336 14.5 / 12.1,
+// 8192 -> 8192 14.7 / 14.1, 10240 -> 4096 15.4 / 15.1, 11008 -> 1152 13.5 / 13.8, 12288 -> 4096 16.8 / 17.3, 14336 -> 8192 21.9 / 22.0,
+// 14336 -> 10240 30.4 / 27.1, 14336 -> 14336 33.7 / 33.3.
+TI8_HD bool decode_quantises(int64_t N, int64_t K, bool by_rows, int num_cu) {
+    return by_rows ? K / 128 <= 80 || N / 32 > num_cu : K / 128 <= 96 || N / 32 * 4 >= (int64_t)num_cu * 3;
 }
 
 }  // namespace idx

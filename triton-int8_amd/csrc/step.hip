@@ -364,10 +364,12 @@ int run_layer(const char* fn, const ti8_linear_args* a, int64_t T, ti8_gemm_prob
         return fail(TI8_ERR_SHAPE, "%s: `saved` must be 256-byte aligned and hold %lld bytes (ti8_linear_workspace); got %lld", fn,
                     (long long)need_saved, (long long)(a->saved ? a->saved_bytes : 0));
     L.carve(static_cast<char*>(a->workspace), static_cast<char*>(a->saved), nullptr);
-    if (!problems && L.fwd && !L.bwd && L.block() && !L.had && !L.keep && L.given_w()) {
+    if (!problems && L.fwd && !L.bwd && !L.had && !L.keep && L.given_w()) {
         const int64_t K = L.K, N = L.N;
         bool done = false;
-        if (int e = gemm_nt_decode(gemm2d(L.xq, L.xs, TI8_SCALE_BLOCK128, K / 128, 1, L.wq, L.ws, TI8_SCALE_ROW, 1, 0, a->Y, a->ldy, 32, N, K, false, 1.0f, 0.0f),
+        const bool xb = L.block(), wb = L.row_block();
+        if (int e = gemm_nt_decode(gemm2d(L.xq, L.xs, xb ? TI8_SCALE_BLOCK128 : TI8_SCALE_ROW, xb ? K / 128 : 1, xb ? 1 : 0, L.wq, L.ws,
+                                          wb ? TI8_SCALE_BLOCK128 : TI8_SCALE_ROW, wb ? K / 128 : 1, wb ? 1 : 0, a->Y, a->ldy, 32, N, K, L.dbl(), 1.0f, 0.0f),
                                    a->X, a->ldx, L.tokens, a->bias, a->gemm_flags, &done, stream)) return e;
         if (done) return TI8_OK;
     }
