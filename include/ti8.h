@@ -373,7 +373,8 @@ int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count, int gemm_f
  *   and dW over one or two K tiles, in one launch), and Y and dX are computed for the first ceil(tokens / 32) * 32 rows only.
  *   workspace: ti8_linear_fwd_bwd_workspace(T, K, N, scheme) bytes of device memory, 256-byte aligned, contents
  *   undefined before and after (it holds the int8 operands, their transposes, scales and maxima; the call clears
- *   what it needs cleared itself, so the same buffer serves any sequence of calls in stream order).
+ *   what it needs cleared itself, so the same buffer serves any sequence of calls in stream order).  Y, dX and dW are
+ *   scratch memory as well until the GEMMs write them (nothing beyond their rows and columns is touched).
  *   gemm_flags: TI8_GEMM_TILED / TI8_GEMM_LARGE_TILES / TI8_GEMM_ONE_TILE or 0.
  * Nothing is allocated; the call only enqueues kernels, so it may be captured into a graph. */
 enum ti8_scheme {
@@ -427,7 +428,7 @@ typedef struct ti8_linear_args {
  * reads tokens, K, N, scheme, hadamard, parts and whether wq is NULL */
 int64_t ti8_linear_workspace(const ti8_linear_args* a, int64_t* saved_bytes);
 /* enqueue the quantisers only and describe the GEMMs that are left to do in problems[0 .. *count - 1] (at most 3: Y, dX, dW;
- * M = T for Y and dX), for ti8_gemm_i8_nt_multi */
+ * M = T for Y and dX), for ti8_gemm_i8_nt_multi.  Y, dX and dW are not written: what they held stays until the GEMMs */
 int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, int* count, ti8_stream_t stream);
 /* enqueue everything.  With more than 256 (padded) tokens and output features the GEMMs of a call go through
  * ti8_gemm_i8_nt_multi (TI8_PART_FORWARD alone: ti8_gemm_i8_nt, the same kernel), else each takes the kernel of ti8_gemm_i8_nt

@@ -1,0 +1,46 @@
+"""What a step leaves in its output tensors, and when."""
+import ctypes
+
+import pytest
+import torch
+
+import triton_int8_amd as T
+from conftest import make_gen, randn_bf16
+from triton_int8_amd import _lib, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(dev, seed, m, k, n):
+    g = make_gen(seed)
+    return randn_bf16(g, m, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev), randn_bf16(g, m, n, std=1e-3).to(dev)
+
+
+def _linear_args(X, W, dY, out, scheme, need):
+    m, k, n = X.shape[0], X.shape[1], W.shape[0]
+    workspace = ops._workspace(need, X.device)
+    pairs = [v for t in (X, W, dY, *out) for v in (t.data_ptr(), t.stride(0))]
+    return _lib.LinearArgs(*pairs, None, None, m, k, n, ops._SCHEMES[scheme], 0, _lib.PART_FORWARD | _lib.PART_BACKWARD, 0, workspace.data_ptr(), need,
+                           None, 0, None), workspace
+
+
+# partial maxima of one tile and of several; ragged tokens
+@pytest.mark.parametrize("scheme", ["block_channel", "row_block", "double_channel"])
+@pytest.mark.parametrize("tokens,k,n", [(384, 512, 640), (1001, 1152, 384), (300, 4224, 512)])
+def test_quantisers_alone_leave_the_outputs(dev, scheme, tokens, k, n):
+    X, W, dY = _operands(dev, tokens, tokens, k, n)
+    want = T.linear_fwd_bwd(X, W, dY, scheme)
+    rows = -(-tokens // 128) * 128
+    before = [torch.full(s, 7.0, dtype=torch.bfloat16, device=dev) for s in ((rows, n), (rows, k), (n, k))]
+    need, _ = ops._linear_sizes(tokens, k, n, scheme, None, _lib.PART_FORWARD | _lib.PART_BACKWARD, False)
+    a, workspace = _linear_args(X, W, dY, before, scheme, need)
+    problems, count = (_lib.GemmProblem * 3)(), ctypes.c_int(0)
+    _lib.call("ti8_linear_quantise", ctypes.byref(a), problems, ctypes.byref(count), ops._stream())
+    assert count.value == 3 and all(bool((t == 7.0).all()) for t in before)
+    after = [torch.empty_like(t) for t in before]       # the products may go anywhere
+    for p, t in zip(problems, after):
+        p.C = t.data_ptr()
+    _lib.call("ti8_gemm_i8_nt_multi", problems, 3, ops.GEMM_TOGETHER, ops._stream())
+    for a, b in zip(after, want):
+        assert torch.equal(a[:b.shape[0]], b)
+    assert all(bool((t == 7.0).all()) for t in before)

@@ -1041,6 +1041,8 @@ static int64_t parts_of(int64_t n, int t) { return (n / 128 + t - 1) / t; }
 // tokens 14336 -> 14336 block-channel (392 MiB) 1560 / 1549.
 constexpr int64_t TOGETHER_BYTES = (int64_t)320 << 20;
 
+bool ti8::quant_together(int64_t bytes) { return bytes <= TOGETHER_BYTES; }
+
 int64_t ti8::quant_maxima_words(int64_t R, int64_t C) {
     int tr, tc;
     maxima_tiles(R, C, &tr, &tc);
@@ -1055,7 +1057,7 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
         bytes += both[i].R * both[i].C * 2;
         atomics = atomics || !both[i].partial;
     }
-    atomics = atomics || bytes > TOGETHER_BYTES;
+    atomics = atomics || !quant_together(bytes);
     if (rows && (atomics || nblocks + nboth == 0 || rows->C > ROW_PART_COLS)) {
         if (int e = ti8_quant_row(rows->x, rows->ldx, rows->q, rows->C, rows->s, rows->R, rows->C, 0, qflags, inv_mode, stream)) return e;
         rows = nullptr;

@@ -27,6 +27,8 @@ struct Layer {
     int64_t T, K, N, tokens;
     int scheme, had;
     bool fwd, bwd, keep;
+    // a whole step whose workspace has no room for partial maxima (ti8_linear_fwd_bwd): they live in its outputs, see `quantise`
+    bool partials_in_outputs = false;
     // operands of Y = X W^T, dX = dY W, dW = dY^T X and their scales
     int8_t *xq, *wq, *dq, *wtq, *dytq, *xtq;
     float *xs, *ws, *ds, *wts, *dyts, *xts;
@@ -37,9 +39,15 @@ struct Layer {
     bool block() const { return scheme == TI8_SCHEME_BLOCK_CHANNEL; }
     bool row_block() const { return scheme == TI8_SCHEME_ROW_BLOCK; }
     bool dbl() const { return scheme == TI8_SCHEME_DOUBLE_CHANNEL; }
-    // R + C maxima, and in a call of one direction the partial ones behind them (a whole step has those in its outputs, see `quantise`)
-    int64_t both_ways_words(int64_t R, int64_t C) const { return maxima_piece(R + C) + (fwd && bwd ? 0 : maxima_piece(quant_maxima_words(R, C))); }
     static int64_t maxima_piece(int64_t words) { return (words + 63) / 64 * 64; }
+    // bytes of the operands of an unrotated call that are quantised by rows and by columns
+    int64_t both_ways_bytes() const {
+        const int64_t w = shares() && fwd && !row_block() ? N * K : 0, x = shares() && fwd && dbl() ? T * K : 0, dy = bwd && !block() ? T * N : 0;
+        return 2 * (w + x + dy);
+    }
+    // R + C maxima, and the partial ones behind them where those are collected there
+    int64_t partial_words(int64_t R, int64_t C) const { return partials_in_outputs || !quant_together(both_ways_bytes()) ? 0 : maxima_piece(quant_maxima_words(R, C)); }
+    int64_t both_ways_words(int64_t R, int64_t C) const { return maxima_piece(R + C) + partial_words(R, C); }
     // what an unrotated forward quantises for the backward in the same pass
     bool shares() const { return had == 0 && (keep || (fwd && bwd)); }
     bool given_w() const { return a->wq != nullptr; }
@@ -216,13 +224,13 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
     int nblocks = 0, nboth = 0;
     const QRowOperand x_rows = {a.X, a.ldx, L.xq, L.xs, tok, K};
     const QRowOperand* by_rows = nullptr;
-    // (`out`, `ldout`: the output of the operand's own shape, which a whole step does not write before its GEMMs; the partial maxima
-    // live there until the conversion has read them, unless the caller's tensors overlap)
-    const bool apart = outputs_apart(a, T);
+    // (`out`, `ldout`: the output of the operand's own shape, which a whole step does not write before its GEMMs; with
+    // partials_in_outputs the partial maxima live there until the conversion has read them, unless the caller's tensors overlap)
+    const bool apart = L.partials_in_outputs && outputs_apart(a, T);
     auto row_col = [&](const void* x, int64_t ldx, int8_t* oq, float* os, int8_t* oqT, float* osT, int64_t R, int64_t valid, int64_t C, void* out, int64_t ldout) {
         unsigned int* const scratch = reinterpret_cast<unsigned int*>(take_maxima(R + C));
         unsigned int* partial = nullptr;
-        if (!(L.fwd && L.bwd)) partial = reinterpret_cast<unsigned int*>(take_maxima(quant_maxima_words(R, C)));
+        if (L.partial_words(R, C)) partial = reinterpret_cast<unsigned int*>(take_maxima(quant_maxima_words(R, C)));
         else if (apart && ldout == C) partial = static_cast<unsigned int*>(out);
         both[nboth++] = QRowColOperand{x, ldx, oq, os, oqT, osT, scratch, partial, R, valid, C};
     };
@@ -351,9 +359,10 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
     return TI8_OK;
 }
 
-int run_layer(const char* fn, const ti8_linear_args* a, int64_t T, ti8_gemm_problem* problems, int* count, ti8_stream_t stream) {
+int run_layer(const char* fn, const ti8_linear_args* a, int64_t T, ti8_gemm_problem* problems, int* count, ti8_stream_t stream, bool partials_in_outputs = false) {
     Layer L;
     if (int e = check_layer(fn, a, T, &L)) return e;
+    L.partials_in_outputs = partials_in_outputs;
     if (int e = check_pointers(fn, a, L)) return e;
     int64_t need_saved = 0;
     const int64_t need = L.size(&need_saved);
@@ -423,6 +432,7 @@ extern "C" int64_t ti8_linear_fwd_bwd_workspace(int64_t T, int64_t K, int64_t N,
     const ti8_linear_args a = step_args(T, K, N, scheme);
     Layer L;
     if (check_layer("ti8_linear_fwd_bwd_workspace", &a, T, &L)) return -1;
+    L.partials_in_outputs = true;
     return L.size(nullptr);
 }
 
@@ -438,5 +448,5 @@ extern "C" int ti8_linear_fwd_bwd(const void* X, int64_t ldx, const void* W, int
     a.Y = Y; a.ldy = ldy; a.dX = dX; a.lddx = lddx; a.dW = dW; a.lddw = lddw;
     a.gemm_flags = gemm_flags;
     a.workspace = workspace; a.workspace_bytes = workspace_bytes;
-    return run_layer(fn, &a, T, nullptr, nullptr, stream);
+    return run_layer(fn, &a, T, nullptr, nullptr, stream, true);
 }

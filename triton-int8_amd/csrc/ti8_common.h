@@ -80,6 +80,8 @@ struct QRowColOperand {
     int64_t R, valid_rows, C;
 };
 int64_t quant_maxima_words(int64_t R, int64_t C);
+// whether the maxima of so many bytes of such operands are collected in one launch; else `partial` is not looked at
+bool quant_together(int64_t bytes);
 // An operand quantised by rows alone, dense codes
 struct QRowOperand {
     const void* x;
