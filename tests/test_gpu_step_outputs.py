@@ -44,3 +44,25 @@ def test_quantisers_alone_leave_the_outputs(dev, scheme, tokens, k, n):
     for a, b in zip(after, want):
         assert torch.equal(a[:b.shape[0]], b)
     assert all(bool((t == 7.0).all()) for t in before)
+
+
+# one launch for the three products and, on few tokens, another for those that the few-rows kernel takes; dX behind Y in the same memory, dW
+# behind dX, and outputs beside each other in one buffer, which are none of each other's business
+@pytest.mark.parametrize("scheme", ["block_channel", "double_channel"])
+@pytest.mark.parametrize("m", [128, 384])
+def test_outputs_that_share_memory(dev, scheme, m):
+    k = n = m if m > 256 else 512
+    X, W, dY = _operands(dev, m, m, k, n)
+    Y, dX, dW = T.linear_fwd_bwd(X, W, dY, scheme)
+    fresh = lambda: torch.full((max(m, n), k), 5.0, dtype=torch.bfloat16, device=dev)
+    shared, other = fresh(), fresh()
+    T.linear_fwd_bwd(X, W, dY, scheme, out=(shared[:m], shared[:m], other[:n]))
+    assert torch.equal(shared[:m], dX) and torch.equal(other[:n], dW)
+    shared, other = fresh(), fresh()
+    T.linear_fwd_bwd(X, W, dY, scheme, out=(other[:m], shared[:m], shared[:n]))
+    assert torch.equal(other[:m], Y) and torch.equal(shared[:n], dW)
+    wide = torch.full((max(m, n), 3 * k), 5.0, dtype=torch.bfloat16, device=dev)
+    beside = (wide[:m, :k], wide[:m, k:2 * k], wide[:n, 2 * k:])
+    T.linear_fwd_bwd(X, W, dY, scheme, out=beside)
+    for a, b in zip(beside, (Y, dX, dW)):
+        assert torch.equal(a, b)

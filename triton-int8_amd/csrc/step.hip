@@ -181,19 +181,34 @@ int check_pointers(const char* fn, const ti8_linear_args* a, const Layer& L) {
     return TI8_OK;
 }
 
-// Whether the outputs of a whole step share no memory with its inputs
+// A matrix of bf16 in memory
+struct Rows {
+    const char* p;
+    int64_t rows, ld, cols;
+    bool apart(const Rows& o) const {
+        if (!p || !o.p || p + ((rows - 1) * ld + cols) * 2 <= o.p || o.p + ((o.rows - 1) * o.ld + o.cols) * 2 <= p) return true;
+        if (ld != o.ld) return false;
+        const int64_t ahead = ((o.p - p) / 2 % ld + ld) % ld;       // columns of one buffer, beside each other
+        return ahead >= cols && ahead + o.cols <= ld;
+    }
+};
+Rows matrix(const void* p, int64_t rows, int64_t ld, int64_t cols) { return Rows{static_cast<const char*>(p), rows, ld, cols}; }
+
+// Whether the outputs of a call share no memory with each other
 bool outputs_apart(const ti8_linear_args& a, int64_t T) {
-    struct Range { const char *from, *to; };
-    const auto range = [](const void* p, int64_t rows, int64_t ld, int64_t cols) {
-        const char* const c = static_cast<const char*>(p);
-        return Range{c, p ? c + ((rows - 1) * ld + cols) * 2 : c};
-    };
-    const Range in[3] = {range(a.X, a.tokens, a.ldx, a.K), range(a.W, a.N, a.ldw, a.K), range(a.dY, a.tokens, a.lddy, a.N)};
-    const Range out[3] = {range(a.Y, T, a.ldy, a.N), range(a.dX, T, a.lddx, a.K), range(a.dW, a.N, a.lddw, a.K)};
-    for (const Range& i : in)
-        for (const Range& o : out)
-            if (i.from < o.to && o.from < i.to) return false;
-    return true;
+    const bool fwd = (a.parts & TI8_PART_FORWARD) != 0, bwd = (a.parts & TI8_PART_BACKWARD) != 0;
+    const Rows y = matrix(fwd ? a.Y : nullptr, T, a.ldy, a.N), dx = matrix(bwd ? a.dX : nullptr, T, a.lddx, a.K), dw = matrix(bwd ? a.dW : nullptr, a.N, a.lddw, a.K);
+    return y.apart(dx) && y.apart(dw) && dx.apart(dw);
+}
+
+// Whether those of a whole step share none with its inputs, either
+bool step_apart(const ti8_linear_args& a, int64_t T) {
+    const Rows in[3] = {matrix(a.X, a.tokens, a.ldx, a.K), matrix(a.W, a.N, a.ldw, a.K), matrix(a.dY, a.tokens, a.lddy, a.N)};
+    const Rows out[3] = {matrix(a.Y, T, a.ldy, a.N), matrix(a.dX, T, a.lddx, a.K), matrix(a.dW, a.N, a.lddw, a.K)};
+    for (const Rows& i : in)
+        for (const Rows& o : out)
+            if (!i.apart(o)) return false;
+    return outputs_apart(a, T);
 }
 
 int64_t next_pow2(int64_t v) {
@@ -226,7 +241,7 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
     const QRowOperand* by_rows = nullptr;
     // (`out`, `ldout`: the output of the operand's own shape, which a whole step does not write before its GEMMs; with
     // partials_in_outputs the partial maxima live there until the conversion has read them, unless the caller's tensors overlap)
-    const bool apart = L.partials_in_outputs && outputs_apart(a, T);
+    const bool apart = L.partials_in_outputs && step_apart(a, T);
     auto row_col = [&](const void* x, int64_t ldx, int8_t* oq, float* os, int8_t* oqT, float* osT, int64_t R, int64_t valid, int64_t C, void* out, int64_t ldout) {
         unsigned int* const scratch = reinterpret_cast<unsigned int*>(take_maxima(R + C));
         unsigned int* partial = nullptr;
@@ -338,9 +353,12 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
         const int64_t r = (L.tokens + 31) / 32 * 32;
         return r < L.T ? r : L.T;
     };
+    // outputs that share memory: a launch each, so that the last one stands
+    const bool apart = count == 1 || outputs_apart(*L.a, L.T);
     // they go into one launch where none of them has so few rows that it would take the few-rows kernel
     if (L.bwd && (L.T < L.N ? L.T : L.N) > 256) {
-        if (int e = ti8_gemm_i8_nt_multi(g, count, flags | TI8_GEMM_TOGETHER, stream)) return e;
+        for (int i = 0, n = apart ? count : 1; i < count; i += n)
+            if (int e = ti8_gemm_i8_nt_multi(g + i, n, flags | TI8_GEMM_TOGETHER, stream)) return e;
         return L.fwd && L.a->bias ? add_bias(L.a->Y, L.a->ldy, L.a->bias, L.tokens, L.N, stream) : TI8_OK;
     }
     ti8_gemm_problem few[3];
@@ -350,7 +368,7 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
         if (i + 1 < count || !L.bwd) few[i].M = live_rows(g[i].K);      // dW, the last of a backward, has one row per output feature
     }
     bool launched[3] = {false, false, false};
-    if (count > 1)
+    if (count > 1 && apart)
         if (int e = gemm_nt_few(few, count, L.bwd, bias, flags, launched, stream)) return e;
     for (int i = 0; i < count; ++i)
         if (!launched[i])
