@@ -397,6 +397,7 @@ int ti8_linear_fwd_bwd(const void* X, int64_t ldx, const void* W, int64_t ldw, c
  *   X bf16 [tokens][K] (ldx), W bf16 [N][K] (ldw), dY bf16 [tokens][N] (lddy); any number of tokens: the rows between
  *   `tokens` and T = tokens rounded up to 128 count as zeros and are not read.
  *   Y bf16 [T][N] (ldy), dX bf16 [T][K] (lddx), dW bf16 [N][K] (lddw); rows of Y and dX from `tokens` on are undefined.
+ *   Outputs may be the inputs' memory (Y in place of X); those that share memory are written one after the other, Y, dX, dW.
  *   parts: TI8_PART_FORWARD (X, W -> Y), TI8_PART_BACKWARD (dY, X, W -> dX, dW) or both.  TI8_PART_KEEP: the forward leaves
  *   what the backward can reuse in `saved` (transposed int8 copies, scales), the backward takes it from there.
  *   wq, ws: the forward's view of W quantised earlier (int8 [N][K] and its scales in the scheme's layout); W is then not read.

@@ -66,3 +66,23 @@ def test_outputs_that_share_memory(dev, scheme, m):
     T.linear_fwd_bwd(X, W, dY, scheme, out=beside)
     for a, b in zip(beside, (Y, dX, dW)):
         assert torch.equal(a, b)
+
+
+# rows that the product's kernel quantises itself, and nine that have a quantiser; Y over X, and Y's 32 rows over X's last one
+@pytest.mark.parametrize("scheme", ["block_channel", "row_block", "double_channel"])
+@pytest.mark.parametrize("tokens", [1, 3, 8, 9])
+@pytest.mark.parametrize("where", ["in place", "behind"])
+def test_forward_over_its_input(dev, scheme, tokens, where):
+    k = n = 1024
+    X, W, _ = _operands(dev, tokens, tokens, k, n)
+    wq = T.linear.quantize_weight(W, scheme, None)
+    want = ops.linear_call(_lib.PART_FORWARD, scheme, None, tokens, k, n, X=X, wq=wq)[0][:tokens]
+    buffer = torch.zeros((256, k), dtype=torch.bfloat16, device=dev)
+    x, y = buffer[:tokens], buffer[:128] if where == "in place" else buffer[tokens - 1:tokens + 127]
+    x.copy_(X)
+    need, _ = ops._linear_sizes(tokens, k, n, scheme, None, _lib.PART_FORWARD, True)
+    workspace = ops._workspace(need, dev)
+    a = _lib.LinearArgs(x.data_ptr(), k, None, 0, None, 0, y.data_ptr(), n, None, 0, None, 0, wq[0].data_ptr(), wq[1].data_ptr(), tokens, k, n,
+                        ops._SCHEMES[scheme], 0, _lib.PART_FORWARD, 0, workspace.data_ptr(), need, None, 0, None)
+    _lib.call("ti8_linear", ctypes.byref(a), ops._stream())
+    assert torch.equal(y[:tokens], want)

@@ -391,7 +391,8 @@ int run_layer(const char* fn, const ti8_linear_args* a, int64_t T, ti8_gemm_prob
         return fail(TI8_ERR_SHAPE, "%s: `saved` must be 256-byte aligned and hold %lld bytes (ti8_linear_workspace); got %lld", fn,
                     (long long)need_saved, (long long)(a->saved ? a->saved_bytes : 0));
     L.carve(static_cast<char*>(a->workspace), static_cast<char*>(a->saved), nullptr);
-    if (!problems && L.fwd && !L.bwd && !L.had && !L.keep && L.given_w()) {
+    // (a kernel that reads X itself cannot write Y where other workgroups are still reading it)
+    if (!problems && L.fwd && !L.bwd && !L.had && !L.keep && L.given_w() && matrix(a->X, a->tokens, a->ldx, a->K).apart(matrix(a->Y, 32, a->ldy, a->N))) {
         const int64_t K = L.K, N = L.N;
         bool done = false;
         const bool xb = L.block(), wb = L.row_block();
