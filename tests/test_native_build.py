@@ -1,10 +1,13 @@
 """The layer call's host side in C++ loads beside torch without slowing it down."""
+import ctypes
 import importlib.util
 import os
 import struct
 import subprocess
+import sys
 
 import pytest
+import torch
 
 import triton_int8_amd as T
 from conftest import ROOT
@@ -23,6 +26,24 @@ def test_no_thread_local_storage():
 
 
 def test_loaded_on_this_torch():
+    assert T._lib.native() is not None
+
+
+@pytest.mark.parametrize("other", ["torch", "python", "arguments", "problems"])
+def test_built_for_something_else(monkeypatch, other):
+    """Another torch or Python may resolve all its symbols and still keep its fields elsewhere."""
+    monkeypatch.setattr(T._lib, "_native", None)
+    longer = lambda base: type(base.__name__, (ctypes.Structure,), {"_fields_": [*base._fields_, ("more", ctypes.c_int64)]})
+    with monkeypatch.context() as m:
+        if other == "torch":
+            m.setattr(torch, "__version__", torch.__version__ + ".1")
+        elif other == "python":
+            m.setattr(sys, "version_info", (sys.version_info[0], sys.version_info[1] + 1, 0))
+        else:
+            name = "LinearArgs" if other == "arguments" else "GemmProblem"
+            m.setattr(T._lib, name, longer(getattr(T._lib, name)))
+        assert T._lib.native() is None
+    T._lib._native = None
     assert T._lib.native() is not None
 
 

@@ -6,6 +6,7 @@ The library is the product: there is no fallback.  If it has not been built
 import contextlib
 import ctypes
 import os
+import sys
 
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.path.join(_HERE, "libti8.so")
@@ -182,7 +183,8 @@ _native = None  # the extension module, False where there is none
 
 def native():
     """The layer call's host side in C++ (``csrc/native.cpp``) on the entry points of :func:`lib`, or None: while calls are being timed
-    one by one, and where it was built for another torch (the same launches are then made from Python)."""
+    one by one, and where there is none or it was built for another torch, Python or argument block (the same launches are then made
+    from Python)."""
     global _native
     if _timing is not None:
         return None
@@ -192,6 +194,10 @@ def native():
         try:
             spec = importlib.util.spec_from_file_location("_native", NATIVE_PATH)
             module = importlib.util.module_from_spec(spec)
+            here = (str(torch.__version__), sys.version_info[:2], ctypes.sizeof(LinearArgs), ctypes.sizeof(GemmProblem))
+            built_for = getattr(module, "built_for", None)
+            if built_for != here:
+                raise ImportError(f"{NATIVE_PATH} was built for {built_for}, this is {here}")
             address = lambda name: ctypes.cast(getattr(lib(), name), _vp).value
             module.set_up(address("ti8_linear"), address("ti8_linear_quantise"), address("ti8_gemm_i8_nt_multi"), torch.nn.Parameter)
             _native = module

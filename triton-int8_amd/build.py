@@ -51,7 +51,8 @@ def build_native(verbose: bool = False) -> str:
     from torch.utils.cpp_extension import include_paths, library_paths
     # NDEBUG: without it pybind11's headers put a thread-local counter into the library, and once a library with thread-local storage that
     # nobody touches has been loaded, glibc looks every other thread-local variable up the long way (torch's calls take 10 to 20 % longer)
-    cmd = ["g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}"]
+    cmd = ["g++", "-O2", "-DNDEBUG", "-std=c++17", "-fPIC", "-shared", f"-D_GLIBCXX_USE_CXX11_ABI={int(torch.compiled_with_cxx11_abi())}",
+           f'-DTI8_BUILT_FOR_TORCH="{torch.__version__}"']
     cmd += [a for path in [sysconfig.get_paths()["include"], *include_paths()] for a in ("-isystem", path)]
     cmd += [os.path.join(CSRC, "native.cpp"), "-o", NATIVE, *(f"-L{path}" for path in library_paths()), "-ltorch_python", "-ltorch_cpu", "-lc10"]
     if verbose:

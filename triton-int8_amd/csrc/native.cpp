@@ -141,4 +141,15 @@ PyModuleDef module = {PyModuleDef_HEAD_INIT, "_native", nullptr, -1, methods, nu
 
 }  // namespace
 
-PyMODINIT_FUNC PyInit__native(void) { return PyModule_Create(&module); }
+// built_for: what the code above was compiled against, for whoever loads it to compare (fields of torch's and Python's objects and of the
+// library's argument blocks are read and written here without a call)
+PyMODINIT_FUNC PyInit__native(void) {
+    PyObject* const m = PyModule_Create(&module);
+    PyObject* const built_for = Py_BuildValue("(s(ii)nn)", TI8_BUILT_FOR_TORCH, PY_MAJOR_VERSION, PY_MINOR_VERSION, (Py_ssize_t)sizeof(ti8_linear_args), (Py_ssize_t)sizeof(ti8_gemm_problem));
+    if (m && (!built_for || PyModule_AddObject(m, "built_for", built_for) < 0)) {
+        Py_XDECREF(built_for);
+        Py_DECREF(m);
+        return nullptr;
+    }
+    return m;
+}
