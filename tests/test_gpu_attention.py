@@ -97,3 +97,22 @@ def test_attention_backward_in_a_graph(D, dev):
         want = D.ops.attention_backward(do, q, k, v, o, lse, 0.09)
         assert all(torch.equal(a, b) for a, b in zip(got, want))
         torch.cuda.synchronize()
+
+
+# a batch, a head or a row alone, whose stride means nothing: in what comes back through autograd and in what goes in
+@pytest.mark.parametrize("batch,heads,seq", [(1, 3, 40), (2, 1, 33), (2, 3, 1), (1, 1, 1)])
+def test_attention_strides_of_dimensions_of_one(D, dev, batch, heads, seq):
+    gen = torch.Generator(device=dev).manual_seed(11)
+
+    def odd(t):
+        return t.as_strided(t.shape, [s if n > 1 else s + 1 for n, s in zip(t.shape[:3], t.stride()[:3])] + [1], t.storage_offset())
+    q, k, v, do = (torch.randn(batch, heads, seq, 64, generator=gen, device=dev).to(torch.bfloat16) for _ in range(4))
+    want = torch.autograd.grad(D._attention(*(t.requires_grad_(True) for t in (q, k, v)), 0.125), (q, k, v), do)
+    out = D._attention(q, k, v, 0.125)
+    for a, b in zip(torch.autograd.grad(out, (q, k, v), odd(do)), want):
+        assert torch.equal(a, b)
+    x = [odd(t.detach()).requires_grad_(True) for t in (q, k, v)]
+    out = D._attention(*x, 0.125)
+    assert type(out.grad_fn).__name__ == "_AttentionFunctionBackward"
+    for a, b in zip(torch.autograd.grad(out, x, do), want):
+        assert torch.equal(a, b)

@@ -65,8 +65,8 @@ def _kernels_take(*tensors):
 def _rows16(t):
     """Whether the attention kernels read a [batch, heads, seq, head_dim] tensor in place: rows of bf16 at 16-byte steps, at 32-bit
     offsets from the first of a (batch, head)."""
-    sb, sh, ss, sd = t.stride()
-    return sd == 1 and not (sb | sh | ss) & 7 and t.data_ptr() % 16 == 0 and t.shape[3] <= ss <= 0x3fffffff // (t.shape[2] + 512)
+    sb, sh, ss = ops.attention_strides(t)
+    return t.stride(3) == 1 and not (sb | sh | ss) & 7 and t.data_ptr() % 16 == 0 and t.shape[3] <= ss <= 0x3fffffff // (t.shape[2] + 512)
 
 
 FLASH_ATTENTION = int(torch.nn.attention.SDPBackend.FLASH_ATTENTION)

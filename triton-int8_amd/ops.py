@@ -648,13 +648,21 @@ def swiglu_backward(d, gate, up):
     return dgate, dup
 
 
+def attention_strides(t):
+    """Strides between batches, heads and rows of [batch, heads, seq, head_dim] as the attention kernels want them: a dimension of one has
+    any stride in torch, and none that matters."""
+    B, H, S, D = t.shape
+    sb, sh, ss, _ = t.stride()
+    return 0 if B == 1 else sb, 0 if H == 1 else sh, D if S == 1 else ss
+
+
 def attention_backward(d_o, q, k, v, o, lse, scale):
     """Gradients of causal attention (bf16 [batch, heads, seq, head_dim], head_dim 64 or 128, any strides that are multiples of 8 with
     a dense last dim) from its output `o` and `lse` (float32 [batch, heads, seq], dense); each in the memory order [batch, seq, heads, head_dim]."""
     B, H, S, D = q.shape
     dq, dk, dv = (torch.empty((B, S, H, D), dtype=torch.bfloat16, device=q.device).transpose(1, 2) for _ in range(3))
     workspace = torch.empty((_lib.lib().ti8_attention_bwd_workspace(B, H, S),), dtype=torch.uint8, device=q.device)
-    args = _lib.AttentionArgs(*(_lib.AttentionTensor(t.data_ptr(), *t.stride()[:3]) for t in (q, k, v, o, d_o, dq, dk, dv)),
+    args = _lib.AttentionArgs(*(_lib.AttentionTensor(t.data_ptr(), *attention_strides(t)) for t in (q, k, v, o, d_o, dq, dk, dv)),
                               lse.data_ptr(), workspace.data_ptr(), B, H, S, D, scale)
     _lib.call("ti8_attention_bwd", ctypes.byref(args), _stream())
     return dq, dk, dv
