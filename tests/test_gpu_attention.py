@@ -116,3 +116,15 @@ def test_attention_strides_of_dimensions_of_one(D, dev, batch, heads, seq):
     assert type(out.grad_fn).__name__ == "_AttentionFunctionBackward"
     for a, b in zip(torch.autograd.grad(out, x, do), want):
         assert torch.equal(a, b)
+
+
+def test_attention_gradients_beyond_32_bit_offsets_are_torchs(D, dev):
+    """The gradients' rows lie heads * head_dim apart, whatever those of q do."""
+    seq = (1 << 30) // (64 * 128) - 512
+    q = torch.empty((1, 64, seq + 1, 128), dtype=torch.bfloat16, device=dev).requires_grad_(True)
+    assert not D._attention_kernels_take(q, q, q, 0.125)
+    q = q.detach()[:, :, :seq - 1].requires_grad_(True)
+    assert D._attention_kernels_take(q, q, q, 0.125)
+    # more (batch, head) pairs than one call takes
+    assert not D.ops.attention_backward_takes(1 << 21, 8, 16, 64) and not D.ops.attention_backward_takes(1, 8, (1 << 24) + 1, 64)
+    assert D.ops.attention_backward_takes((1 << 21) - 1, 8, 16, 64)

@@ -402,14 +402,14 @@ using namespace ti8;
 
 extern "C" int64_t ti8_attention_bwd_workspace(int64_t batch, int64_t heads, int64_t seq) {
     if (batch <= 0 || heads <= 0 || seq <= 0 || seq > (1 << 24) || batch > 0xffffff || heads > 0xffffff || batch * heads > 0xffffff) return -1;
+    if ((batch * heads + 7) / 8 * 8 * ((seq + 127) / 128) > 0x7fffffff) return -1;      // workgroups of a launch
     return batch * heads * 2 * padded_rows(seq) * (int64_t)sizeof(float);
 }
 
 extern "C" int ti8_attention_bwd(const ti8_attention_args* p, ti8_stream_t stream) {
     const char* fn = "ti8_attention_bwd";
     if (!p || !p->lse || !p->workspace) return fail(TI8_ERR_NULL, "%s: args, lse and workspace are required", fn);
-    if (ti8_attention_bwd_workspace(p->batch, p->heads, p->seq) < 0 || (p->head_dim != 64 && p->head_dim != 128) ||
-        (p->batch * p->heads + 7) / 8 * 8 * ((p->seq + 127) / 128) > 0x7fffffff)
+    if (ti8_attention_bwd_workspace(p->batch, p->heads, p->seq) < 0 || (p->head_dim != 64 && p->head_dim != 128))
         return fail(TI8_ERR_SHAPE, "%s: need batch, heads and seq > 0 and head_dim 64 or 128; got batch=%lld heads=%lld seq=%lld head_dim=%lld", fn,
                     (long long)p->batch, (long long)p->heads, (long long)p->seq, (long long)p->head_dim);
     if (!aligned16(p->workspace) || (reinterpret_cast<uintptr_t>(p->lse) & 3)) return fail(TI8_ERR_ALIGN, "%s: workspace or lse is misaligned", fn);

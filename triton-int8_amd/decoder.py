@@ -77,7 +77,7 @@ def _attention_kernels_take(q, k, v, scale):
     on shapes and layouts that ours take."""
     if not (torch.is_grad_enabled() and (q.requires_grad or k.requires_grad or v.requires_grad)) or torch.is_autocast_enabled("cuda"):
         return False
-    return (_plain(q, k, v) and q.shape[3] in (64, 128) and all(t.shape == q.shape and _rows16(t) for t in (q, k, v)) and q.shape[2] <= 1 << 24
+    return (_plain(q, k, v) and ops.attention_backward_takes(*q.shape) and all(t.shape == q.shape and _rows16(t) for t in (q, k, v))
             and torch._fused_sdp_choice(q, k, v, None, 0.0, True, scale=scale) == FLASH_ATTENTION)
 
 

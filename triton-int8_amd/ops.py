@@ -656,6 +656,12 @@ def attention_strides(t):
     return 0 if B == 1 else sb, 0 if H == 1 else sh, D if S == 1 else ss
 
 
+def attention_backward_takes(batch, heads, seq, head_dim):
+    """Whether :func:`attention_backward` serves these sizes (32-bit offsets into the rows of its outputs among them)."""
+    return (head_dim in (64, 128) and heads * head_dim <= 0x3fffffff // (seq + 512)
+            and _lib.lib().ti8_attention_bwd_workspace(batch, heads, seq) >= 0)
+
+
 def attention_backward(d_o, q, k, v, o, lse, scale):
     """Gradients of causal attention (bf16 [batch, heads, seq, head_dim], head_dim 64 or 128, any strides that are multiples of 8 with
     a dense last dim) from its output `o` and `lse` (float32 [batch, heads, seq], dense); each in the memory order [batch, seq, heads, head_dim]."""
