@@ -264,11 +264,12 @@ int walk_fwht_t(int64_t ldx, int64_t ldy, int64_t R, int64_t C, int64_t x_elems,
 }
 
 // ti8_quant_row -> quant_row_kernel<NLOAD, WG_ROW, GROUP16, HAD> (quant.hip)
-int walk_quant_row(int64_t ldx, int64_t ldq, int64_t rows, int64_t cols, int group, int64_t x_elems, int64_t q_elems,
-                   int64_t s_elems, int64_t* n_checked, char* msg, int msglen) {
+int walk_quant_row_form(int64_t ldx, int64_t ldq, int64_t rows, int64_t cols, int group, int plain, int64_t x_elems, int64_t q_elems,
+                        int64_t s_elems, int* form, int64_t* n_checked, char* msg, int msglen) {
     Report r{msg, msglen};
     const int nchunk = (int)(cols / 8);
-    const QRowConfig cfg = qrow_config(nchunk, group == 128);
+    const QRowConfig cfg = qrow_config(nchunk, group == 128, rows, plain != 0);
+    if (form) { form[0] = cfg.nload; form[1] = cfg.wg_row; }
     const int64_t grid = cfg.wg_row ? rows : (rows + 3) / 4;
     const int T = cfg.wg_row ? 256 : 64;
     const int ngrp = (int)(cols >> 7);
@@ -294,6 +295,10 @@ int walk_quant_row(int64_t ldx, int64_t ldq, int64_t rows, int64_t cols, int gro
         if (seen[(size_t)row] != 1) r.fail("quant_row: row %lld handled %d times", (long long)row, (int)seen[(size_t)row]);
     *n_checked = r.checked;
     return r.bad;
+}
+int walk_quant_row(int64_t ldx, int64_t ldq, int64_t rows, int64_t cols, int group, int64_t x_elems, int64_t q_elems,
+                   int64_t s_elems, int64_t* n_checked, char* msg, int msglen) {
+    return walk_quant_row_form(ldx, ldq, rows, cols, group, 1, x_elems, q_elems, s_elems, nullptr, n_checked, msg, msglen);
 }
 
 // ti8_quant_block -> quant_block_kernel<NSUB, WRITE_Q, WRITE_QT> (quant.hip)

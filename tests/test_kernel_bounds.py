@@ -17,6 +17,7 @@ import pytest
 import torch
 
 from conftest import ROOT
+from triton_int8_amd._lib import Q_HAD128, Q_TORCH_BF16, Q_TORCH_ROUND
 
 CSRC = os.path.join(ROOT, "triton-int8_amd", "csrc")
 SRC = os.path.join(ROOT, "tests", "kernel_bounds", "walk.cpp")
@@ -41,6 +42,7 @@ def walker(tmp_path_factory):
     lib.walk_transpose_bf16.argtypes = [i64] * 6 + [p64, cp, ci]
     lib.walk_fwht_t.argtypes = [i64] * 7 + [p64, cp, ci]
     lib.walk_quant_row.argtypes = [i64] * 4 + [ci] + [i64] * 3 + [p64, cp, ci]
+    lib.walk_quant_row_form.argtypes = [i64] * 4 + [ci, ci] + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_quant_block.argtypes = [i64, i64, ci, i64, i64, ci, i64, i64, i64, i64, i64, i64, i64, i64, ci, i64, i64, i64, i64, p64, cp, ci]
     lib.walk_gemm.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] * 5 + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_gemm_chain.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] + [i64] * 3 + [p64, cp, ci]
@@ -116,8 +118,10 @@ def walk(lib, allocs, name, a):
         x, ldx, y, ldy, R, C = a[:6]
         rc = lib.walk_fwht_t(ldx, ldy, R, C, allocs.room(x, 2), allocs.room(y, 2), LDS_LIMIT, ctypes.byref(n), msg, 512)
     elif name == "ti8_quant_row":
-        x, ldx, q, ldq, s, rows, cols, group = a[:8]
-        rc = lib.walk_quant_row(ldx, ldq, rows, cols, group, allocs.room(x, 2), allocs.room(q, 1), allocs.room(s, 4), ctypes.byref(n), msg, 512)
+        x, ldx, q, ldq, s, rows, cols, group, flags = a[:9]
+        plain = not flags & (Q_HAD128 | Q_TORCH_ROUND | Q_TORCH_BF16)
+        rc = lib.walk_quant_row_form(ldx, ldq, rows, cols, group, plain, allocs.room(x, 2), allocs.room(q, 1), allocs.room(s, 4), None,
+                                     ctypes.byref(n), msg, 512)
     elif name == "ti8_quant_block":
         x, bsx, ldx, q, bsq, ldq, qT, bsqt, ldqt, s, ssb, ssr, ssc, B, R, C, group_c = a[:17]
         rc = lib.walk_quant_block(bsx, ldx, q is not None, bsq, ldq, qT is not None, bsqt, ldqt, ssb, ssr, ssc, B, R, C, group_c,
@@ -243,6 +247,20 @@ def test_gemm_launch_geometries(walker, M, N, K, batch, mA, mB, acc, flags):
     rc = walker.walk_gemm(M * K, K, 0, K, M * N, N, ctypes.byref(sa), ctypes.byref(sb), batch, M, N, K, acc, flags & 1, (flags >> 3) & 1, 0,
                           NUM_CU, batch * M * K, N * K, batch * M * N, picked, ctypes.byref(n), msg, 512)
     assert rc == 0, msg.value.decode()
+
+
+# a workgroup per row up to 256 rows, a wave per row beyond and in the forms that have no other; the shortest row and the longest
+@pytest.mark.parametrize("rows", [1, 255, 256, 257])
+@pytest.mark.parametrize("cols,plain,few", [(512, 1, 0), (640, 1, 1), (4096, 1, 1), (4096, 0, 0), (4224, 1, 0)])
+def test_row_quantiser_launches(walker, rows, cols, plain, few):
+    msg, n, form = ctypes.create_string_buffer(512), ctypes.c_int64(0), (ctypes.c_int * 2)()
+    ld = cols + 16
+    run = lambda x_el, q_el, s_el: walker.walk_quant_row_form(ld, cols, rows, cols, 0, plain, x_el, q_el, s_el, form, ctypes.byref(n), msg, 512)
+    assert run(rows * ld - 16, rows * cols, rows) == 0, msg.value.decode()
+    assert (tuple(form) == (2, 1)) == bool(few and rows <= 256)
+    assert run(rows * ld - 17, rows * cols, rows) == 1 and b"quant_row x" in msg.value
+    assert run(rows * ld - 16, rows * cols - 1, rows) == 1 and b"quant_row q" in msg.value
+    assert run(rows * ld - 16, rows * cols, rows - 1) == 1 and b"quant_row s" in msg.value
 
 
 @pytest.mark.parametrize("R,C", [(128, 8), (128, 520), (2048, 72), (4096, 512), (8192, 1024), (16384, 2048), (32768, 4096), (32768, 64),

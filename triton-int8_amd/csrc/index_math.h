@@ -232,14 +232,14 @@ TI8_HD int qblock_t_col(int t) { return (t & 7) * 16; }
 // per-row quantiser: NLOAD 16-byte chunks per thread, one wave (4 rows per workgroup) or one
 // 256-thread workgroup per row, by the number of 16-byte chunks in a row.  Up to a row per CU (256) the time is that of
 // one row, and a whole workgroup takes it (37 rows of 4096 3.4 us, a wave per row 3.9; the call with its GEMM, 4096 ->
-// 14336, 15.9 and 16.4)
+// 14336, 15.9 and 16.4).  `plain`: no rotation, and the arithmetic of the reference's kernels (the others have no such form).
 struct QRowConfig {
     int nload;
     bool wg_row;
 };
-TI8_HD QRowConfig qrow_config(int nchunk, bool group128, int64_t rows = (int64_t)1 << 31) {
+TI8_HD QRowConfig qrow_config(int nchunk, bool group128, int64_t rows, bool plain) {
     QRowConfig c;
-    if (!group128 && rows <= 256 && nchunk <= 256 * 2 && nchunk > 64) {
+    if (!group128 && plain && rows <= 256 && nchunk <= 256 * 2 && nchunk > 64) {
         c.nload = 2;
         c.wg_row = true;
     } else if (group128) {

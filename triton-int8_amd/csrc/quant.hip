@@ -1162,7 +1162,7 @@ extern "C" int ti8_quant_row(const void* x, int64_t ldx, int8_t* q, int64_t ldq,
          else if (!G16 && arith == ARITH_TORCH_BF16) hipLaunchKernelGGL((quant_row_kernel<NL, WG, false, false, ARITH_TORCH_BF16>), dim3((unsigned)(GRID)), dim3(256), 0, st, xp, ldx, q, ldq, s, rows, c, mode); \
          else if (had) hipLaunchKernelGGL((quant_row_kernel<NL, WG, G16, true>), dim3((unsigned)(GRID)), dim3(256), 0, st, xp, ldx, q, ldq, s, rows, c, mode); \
          else hipLaunchKernelGGL((quant_row_kernel<NL, WG, G16, false>), dim3((unsigned)(GRID)), dim3(256), 0, st, xp, ldx, q, ldq, s, rows, c, mode); } while (0)
-    const idx::QRowConfig cfg = idx::qrow_config(nchunk, group == 128, had || arith != ARITH_KERNEL ? (int64_t)1 << 31 : rows);
+    const idx::QRowConfig cfg = idx::qrow_config(nchunk, group == 128, rows, !had && arith == ARITH_KERNEL);
     const int64_t grid = cfg.wg_row ? rows : (rows + 3) / 4;
     if (group == 128) {
         if (!cfg.wg_row) TI8_LAUNCH_QR(8, false, true, grid);
