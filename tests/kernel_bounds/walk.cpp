@@ -333,6 +333,103 @@ int walk_quant_block(int64_t bsx, int64_t ldx, int has_q, int64_t bsq, int64_t l
     return r.bad;
 }
 
+// Partial maxima of an operand [R][C] (quant.hip: maxima_part, quant_rowcol_multi_kernel): every element that exists read once, every word of
+// both arrays stored once, row maxima inside their LDS, 16-byte accesses on 16-byte boundaries; the conversion of every tile
+// reads all parts' maxima of its own rows and columns.  x_elems elements of x, `words` 32-bit words of scratch.
+int walk_maxima(int64_t R, int64_t C, int64_t valid, int64_t ldx, int64_t x_elems, int64_t words, int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    const MaximaParts m = maxima_parts(R, C);
+    const int64_t cols0 = (int64_t)m.nct * R, halves = 2 * words;
+    std::vector<uint8_t> stored((size_t)halves, 0), read((size_t)((R / 128) * (C / 128)), 0);
+    for (int part = 0; part < m.nrt * m.nct && !r.bad; ++part) {
+        const int ct = part % m.nct, rt = part / m.nct;
+        const int rtiles = imin(m.tr, (int)(R >> 7) - rt * m.tr), ctiles = imin(m.tc, (int)(C >> 7) - ct * m.tc);
+        if (rtiles < 1 || ctiles < 1) { r.fail("maxima: part %d has %d x %d tiles", part, rtiles, ctiles); break; }
+        auto store = [&](const char* what, int64_t at, int n) {
+            if (at % n) r.fail("%s: %lld is not a multiple of %d", what, (long long)at, n);
+            if (r.access(what, at, n, halves, part))
+                for (int e = 0; e < n; ++e) ++stored[(size_t)(at + e)];
+        };
+        for (int a = 0; a < rtiles; ++a)
+            for (int b = 0; b < ctiles; ++b) {
+                ++read[(size_t)((rt * m.tr + a) * (C / 128) + ct * m.tc + b)];
+                for (int tid = 0; tid < 256; ++tid)
+                    for (int i = 0; i < 8; ++i) {
+                        const int64_t row = (rt * m.tr + a) * 128 + (tid >> 4) * 8 + i;
+                        if (row < valid) r.access("maxima x", row * ldx + (ct * m.tc + b) * 128 + (tid & 15) * 8, 8, x_elems, part, tid, i);
+                    }
+            }
+        for (int rg = 0; rg < 16; ++rg)
+            for (int a = 0; a < rtiles; ++a) {
+                r.access("maxima LDS", a * 128 + rg * 8, 8, MAXIMA_ROW_TILES * 128, part, rg, a);
+                store("maxima rows", maxima_rows_at(ct, R, (rt * m.tr + a) * 128 + rg * 8), 8);
+            }
+        for (int b = 0; b < ctiles; ++b)
+            for (int tid = 0; tid < 64; ++tid) store("maxima columns", cols0 + maxima_cols_at(rt, C, (ct * m.tc + b) * 128) + 2 * tid, 2);
+    }
+    for (size_t i = 0; i < read.size() && !r.bad; ++i)
+        if (read[i] != 1) r.fail("maxima: tile %zu is read %d times", i, (int)read[i]);
+    for (size_t i = 0; i < stored.size() && !r.bad; ++i)
+        if (stored[i] != 1) r.fail("maxima: half word %zu is stored %d times", i, (int)stored[i]);
+    for (int64_t tile = 0; tile < (R / 128) * (C / 128) && !r.bad; ++tile) {
+        const int64_t cb = tile % (C / 128), rb = tile / (C / 128);
+        for (int chunk = 0; chunk < 16; ++chunk) {
+            for (int p = 0; p < m.nrt; ++p) r.access("conversion: columns", cols0 + cb * 128 + chunk * 8 + p * C, 8, halves, tile, p);
+            for (int p = 0; p < m.nct; ++p) r.access("conversion: rows", rb * 128 + chunk * 8 + p * R, 8, cols0, tile, p);
+        }
+    }
+    if (cols0 % 8 || C % 8) r.fail("conversion: columns' maxima off 16-byte boundaries");
+    *n_checked = r.checked;
+    return r.bad;
+}
+
+int64_t maxima_scratch_words(int64_t R, int64_t C) { return maxima_words(R, C); }
+
+// Workgroups of the two launches (quant_call, quant_first_kernel, quant_rowcol_multi_kernel) for `count` operands quantised both ways, beside
+// `block_tiles` tiles of block-quantised ones and `row_groups` workgroups of rows: each part and each tile belongs to one workgroup.
+int walk_quant_call(const int64_t* R, const int64_t* C, int count, int block_tiles, int row_groups, int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    int first_part[4] = {0, 0, 0, 0}, first_tile[4] = {0, 0, 0, 0}, parts = 0, tiles = 0;
+    std::vector<std::vector<int>> part_seen(count), tile_seen(count);
+    for (int i = 0; i < 3; ++i) {
+        first_part[i] = parts; first_tile[i] = tiles;
+        if (i >= count) continue;
+        const MaximaParts m = maxima_parts(R[i], C[i]);
+        part_seen[i].assign(m.nrt * m.nct, 0);
+        tile_seen[i].assign((R[i] / 128) * (C[i] / 128), 0);
+        parts += (int)round8(m.nrt * m.nct);
+        tiles += (int)round8((R[i] / 128) * (C[i] / 128));
+    }
+    const int blocks_end = (int)round8(block_tiles), rows_end = (int)round8(row_groups);
+    int blocks = 0;
+    for (int w = 0; w < rows_end + blocks_end + parts && !r.bad; ++w) {
+        const int tile = w - rows_end, part = tile - blocks_end;
+        ++r.checked;
+        if (tile < 0) continue;
+        if (part < 0) { blocks += tile < block_tiles; continue; }
+        const int i = operand_of(part, first_part, count), at = part - first_part[i];
+        if (at < 0 || at >= (int)round8((int64_t)part_seen[i].size())) r.fail("first launch: workgroup %d takes part %d of operand %d", w, at, i);
+        else if (at < (int)part_seen[i].size()) ++part_seen[i][at];
+        if (at == 0 && w % 8) r.fail("first launch: operand %d starts at workgroup %d", i, w);
+    }
+    if (blocks != block_tiles) r.fail("first launch: %d of %d block tiles", blocks, block_tiles);
+    for (int w = 0; w < tiles && !r.bad; ++w) {
+        const int tile = rowcol_multi_tile(w, tiles);
+        ++r.checked;
+        if (tile < 0 || tile >= tiles || tile % 8 != w % 8) { r.fail("conversion: workgroup %d takes tile %d", w, tile); break; }
+        const int i = operand_of(tile, first_tile, count), at = tile - first_tile[i];
+        if (at / (int)(C[i] / 128) < R[i] / 128) ++tile_seen[i][at];
+    }
+    for (int i = 0; i < count && !r.bad; ++i) {
+        for (size_t k = 0; k < part_seen[i].size(); ++k)
+            if (part_seen[i][k] != 1) r.fail("first launch: part %zu of operand %d is taken %d times", k, i, part_seen[i][k]);
+        for (size_t k = 0; k < tile_seen[i].size(); ++k)
+            if (tile_seen[i][k] != 1) r.fail("conversion: tile %zu of operand %d is taken %d times", k, i, tile_seen[i][k]);
+    }
+    *n_checked = r.checked;
+    return r.bad;
+}
+
 struct ScaleArg {
     int mode;
     int64_t bs, rs, ks, elems;

@@ -43,6 +43,10 @@ def walker(tmp_path_factory):
     lib.walk_fwht_t.argtypes = [i64] * 7 + [p64, cp, ci]
     lib.walk_quant_row.argtypes = [i64] * 4 + [ci] + [i64] * 3 + [p64, cp, ci]
     lib.walk_quant_row_form.argtypes = [i64] * 4 + [ci, ci] + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
+    lib.walk_maxima.argtypes = [i64] * 6 + [p64, cp, ci]
+    lib.walk_quant_call.argtypes = [p64, p64, ci, ci, ci, p64, cp, ci]
+    lib.maxima_scratch_words.argtypes = [i64, i64]
+    lib.maxima_scratch_words.restype = i64
     lib.walk_quant_block.argtypes = [i64, i64, ci, i64, i64, ci, i64, i64, i64, i64, i64, i64, i64, i64, ci, i64, i64, i64, i64, p64, cp, ci]
     lib.walk_gemm.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] * 5 + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_gemm_chain.argtypes = [i64] * 6 + [ctypes.POINTER(ScaleArg)] * 2 + [i64] * 4 + [ci] + [i64] * 3 + [p64, cp, ci]
@@ -261,6 +265,28 @@ def test_row_quantiser_launches(walker, rows, cols, plain, few):
     assert run(rows * ld - 17, rows * cols, rows) == 1 and b"quant_row x" in msg.value
     assert run(rows * ld - 16, rows * cols - 1, rows) == 1 and b"quant_row q" in msg.value
     assert run(rows * ld - 16, rows * cols, rows - 1) == 1 and b"quant_row s" in msg.value
+
+
+# one tile; parts of one tile, of several with a shorter last one, both ways; more rows than 32 parts hold the maxima of; ragged rows
+@pytest.mark.parametrize("R,C,valid", [(128, 128, 1), (4096, 4096, 4096), (4224, 4352, 4100), (8448, 256, 8441), (512, 14336, 300), (270336, 128, 270336),
+                                       (300032, 256, 299905)])
+def test_partial_maxima(walker, R, C, valid):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    ld, words = C + 8, walker.maxima_scratch_words(R, C)
+    assert 4 * words <= 2 * R * C       # in no more than the operand's own bytes
+    run = lambda x_el, w: walker.walk_maxima(R, C, valid, ld, x_el, w, ctypes.byref(n), msg, 512)
+    assert run(valid * ld - 8, words) == 0, msg.value.decode()
+    assert run(valid * ld - 9, words) == 1 and b"maxima x" in msg.value
+    assert run(valid * ld - 8, words - 1) == 1 and b"maxima" in msg.value
+    assert run(valid * ld - 8, words + 1) == 1 and b"stored 0 times" in msg.value
+
+
+@pytest.mark.parametrize("operands", [[(128, 128)], [(384, 640), (512, 640)], [(1024, 4096), (4096, 4096), (1024, 4352)], [(128, 384), (384, 128), (8448, 256)]])
+@pytest.mark.parametrize("block_tiles,row_groups", [(0, 0), (5, 0), (64, 13)])
+def test_workgroups_of_a_calls_quantisers(walker, operands, block_tiles, row_groups):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    R, C = ((ctypes.c_int64 * len(operands))(*(o[d] for o in operands)) for d in (0, 1))
+    assert walker.walk_quant_call(R, C, len(operands), block_tiles, row_groups, ctypes.byref(n), msg, 512) == 0, msg.value.decode()
 
 
 @pytest.mark.parametrize("R,C", [(128, 8), (128, 520), (2048, 72), (4096, 512), (8192, 1024), (16384, 2048), (32768, 4096), (32768, 64),

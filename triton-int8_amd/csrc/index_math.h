@@ -227,6 +227,43 @@ TI8_HD int qblock_col(int t) { return (t & 15) * 8; }
 TI8_HD int qblock_t_row(int t, int p) { return p * 32 + (t >> 3); }
 TI8_HD int qblock_t_col(int t) { return (t & 7) * 16; }
 
+// ---- quantisers of a layer call in two launches (quant.hip) -------------------------------------
+// Maxima of an operand [R][C]: a workgroup takes a part of tr x tc tiles of 128 x 128, the last ones in either direction shorter, and stores
+// 16 bits per row of it and per column: rows [nct][R], cols [nrt][C], one array behind the other.  About 32 parts in either
+// direction; a part keeps the maxima of its rows in LDS, so beyond 262144 rows there is one for every 8192.
+constexpr int MAXIMA_ROW_TILES = 64;
+struct MaximaParts {
+    int tr, tc, nrt, nct;
+};
+TI8_HD MaximaParts maxima_parts(int64_t R, int64_t C) {
+    MaximaParts m;
+    const int64_t a = (R / 128 + 31) / 32;
+    m.tr = (int)(a < MAXIMA_ROW_TILES ? a : MAXIMA_ROW_TILES);
+    m.tc = (int)((C / 128 + 31) / 32);
+    m.nrt = (int)((R / 128 + m.tr - 1) / m.tr);
+    m.nct = (int)((C / 128 + m.tc - 1) / m.tc);
+    return m;
+}
+TI8_HD int64_t maxima_rows_at(int ct, int64_t R, int row) { return (int64_t)ct * R + row; }
+TI8_HD int64_t maxima_cols_at(int rt, int64_t C, int col) { return (int64_t)rt * C + col; }
+// 32-bit words of both arrays (R and C are multiples of 128)
+TI8_HD int64_t maxima_words(int64_t R, int64_t C) {
+    const MaximaParts m = maxima_parts(R, C);
+    return (m.nct * R + m.nrt * C) / 2;
+}
+// operands start at multiples of 8 workgroups: ids 8 apart are workgroups of one XCD
+TI8_HD int64_t round8(int64_t n) { return (n + 7) / 8 * 8; }
+// which of up to three operands `at` belongs to, operand i having [first[i], first[i + 1])
+TI8_HD int operand_of(int at, const int* first, int count) {
+    int i = 0;
+    for (int k = 1; k < 3; ++k)
+        if (k < count && at >= first[k]) i = k;
+    return i;
+}
+// the conversion's tile of workgroup `block` of `grid` (a multiple of 8): from the end of the last operand to the beginning of the first, and
+// every tile on the XCD that took its maxima where a part is one tile
+TI8_HD int rowcol_multi_tile(int block, int grid) { return ((grid >> 3) - 1 - (block >> 3)) * 8 + (block & 7); }
+
 // ---- which kernel an entry point launches (decided on the host) ------------------------------
 
 // per-row quantiser: NLOAD 16-byte chunks per thread, one wave (4 rows per workgroup) or one

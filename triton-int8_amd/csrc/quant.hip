@@ -727,8 +727,8 @@ __global__ __launch_bounds__(256) void quant_rowcol_kernel(const uint16_t* __res
 // maxima and the conversion; launched operand by operand these are many short kernels (and one that only clears the maxima).  Here
 // the maxima of all such operands are one launch, together with the block-quantised operands of the call, and the conversions the next.
 // The maxima need no clearing: a workgroup stores those of its rows and of its columns (16 bits each: patterns of |bf16|) beside the other
-// workgroups', at most about 32 of either (quant_maxima_tiles), and the conversion of a 128 x 128 tile takes the largest of what
-// belongs to it, 16 KiB at most from the L2.
+// workgroups' (idx::maxima_parts), and the conversion of a 128 x 128 tile takes the largest of what belongs to it, 256 bytes per part in
+// either direction, from the L2: 16 KiB up to 262144 rows.
 //   rows [nct][R], cols [nrt][C]: maxima over the columns of part ct, over the rows of part rt; a part is tr (tc) times 128
 struct MaxOperand {
     const uint16_t* x;
@@ -742,7 +742,7 @@ struct MaxOperand {
     float* s_col;
     int R, C, valid_rows, tr, tc, nrt, nct;
 };
-constexpr int MAX_OPERANDS = 3;
+constexpr int MAX_OPERANDS = 3;     // (idx::operand_of)
 struct MaxMulti {
     MaxOperand op[MAX_OPERANDS];
     int first[MAX_OPERANDS + 1];
@@ -818,14 +818,14 @@ __device__ __forceinline__ void maxima_part(const MaxOperand& o, const int part,
             const uint32_t* const pw = reinterpret_cast<const uint32_t*>(colpart);
             const uint32_t u = pk_max_i16(pk_max_i16(pw[tid], pw[64 + tid]), pk_max_i16(pw[128 + tid], pw[192 + tid]));
             const int lo = static_cast<short>(u & 0xffffu), hi = static_cast<short>(u >> 16);
-            reinterpret_cast<uint32_t*>(o.cols + (int64_t)rt * o.C + (ct * o.tc + b) * 128)[tid] =
+            reinterpret_cast<uint32_t*>(o.cols + idx::maxima_cols_at(rt, o.C, (ct * o.tc + b) * 128))[tid] =
                 (uint32_t)(max(lo, 0x7f) - 0x7f) | ((uint32_t)(max(hi, 0x7f) - 0x7f) << 16);
         }
         __syncthreads();
     }
     if (cc == 0)
         for (int a = 0; a < rtiles; ++a)
-            *reinterpret_cast<uint4*>(o.rows + (int64_t)ct * o.R + (rt * o.tr + a) * 128 + rg * 8) = *reinterpret_cast<const uint4*>(rowmax + a * 128 + rg * 8);
+            *reinterpret_cast<uint4*>(o.rows + idx::maxima_rows_at(ct, o.R, (rt * o.tr + a) * 128 + rg * 8)) = *reinterpret_cast<const uint4*>(rowmax + a * 128 + rg * 8);
 }
 
 // An operand quantised by rows alone, by workgroups in front of the block tiles (row-block: X, whose rows the same launch reads for X^T).
@@ -837,12 +837,11 @@ struct RowPart {
 };
 constexpr int ROW_PART_COLS = 16384;     // 8 chunks per thread of a workgroup
 
-constexpr int MAXIMA_ROW_TILES = 64;     // 128-row tiles whose row maxima a workgroup keeps in LDS
 __global__ __launch_bounds__(256) void quant_first_kernel(const MaxMulti maxima, const QBlockMulti blocks, const RowPart rows, QMode mode) {
     __shared__ float red4[4];
     __shared__ __attribute__((aligned(16))) uint32_t tileT[128 * 33];
     __shared__ uint4 colpart[4][16];
-    static_assert(MAXIMA_ROW_TILES * 128 * 2 <= (int)sizeof(tileT), "row maxima share the transposed tile's LDS");
+    static_assert(idx::MAXIMA_ROW_TILES * 128 * 2 <= (int)sizeof(tileT), "row maxima share the transposed tile's LDS");
     const int tile = (int)blockIdx.x - rows.workgroups, part = tile - blocks.first[QBLOCK_MULTI_MAX];
     if (tile < 0) {
         const QRowOperand& o = rows.op;
@@ -852,10 +851,7 @@ __global__ __launch_bounds__(256) void quant_first_kernel(const MaxMulti maxima,
     } else if (part < 0) {
         if (tile < blocks.first[blocks.count]) quant_block_of<true, true>(blocks, tile, mode, red4, tileT);
     } else {
-        int i = 0;
-#pragma unroll
-        for (int k = 1; k < MAX_OPERANDS; ++k)
-            if (k < maxima.count && part >= maxima.first[k]) i = k;
+        const int i = idx::operand_of(part, maxima.first, maxima.count);
         const MaxOperand& o = maxima.op[i];
         if (part - maxima.first[i] < o.nrt * o.nct) maxima_part(o, part - maxima.first[i], reinterpret_cast<uint16_t*>(tileT), colpart);
     }
@@ -865,13 +861,9 @@ __global__ __launch_bounds__(256) void quant_rowcol_multi_kernel(const MaxMulti 
     __shared__ uint32_t tileT[128 * 33];
     __shared__ __attribute__((aligned(16))) float sc[256];
     __shared__ uint4 part[2][4][16];    // [rows, columns][wave][chunk]
-    // from the end of the last operand to the beginning of the first, and every tile on the XCD that took its maxima where a part is one
-    // tile: what the launch before read last is still in the caches (4096 x 4096 behind its maxima: 13 us, 16 on another XCD)
-    const int tile = (int)((gridDim.x >> 3) - 1 - (blockIdx.x >> 3)) * 8 + (int)(blockIdx.x & 7);
-    int i = 0;
-#pragma unroll
-    for (int k = 1; k < MAX_OPERANDS; ++k)
-        if (k < m.count && tile >= m.first[k]) i = k;
+    // (what the launch before read last is still in the caches: 4096 x 4096 behind its maxima 13 us, 16 with the tiles on other XCDs)
+    const int tile = idx::rowcol_multi_tile((int)blockIdx.x, (int)gridDim.x);
+    const int i = idx::operand_of(tile, m.first, m.count);
     const MaxOperand& o = m.op[i];
     const int ncb = o.C >> 7, local = tile - m.first[i];
     const int cb = local % ncb, rb = local / ncb;
@@ -1026,15 +1018,6 @@ int ti8::quant_block_multi_valid(const ti8_qblock_operand* operands, const int64
     return check_launch(fn);
 }
 
-// 128 x 128 tiles per part in either direction: about 32 parts, and no more rows than a workgroup's LDS holds maxima of
-static void maxima_tiles(int64_t R, int64_t C, int* tr, int* tc) {
-    const int64_t a = (R / 128 + 31) / 32, b = (C / 128 + 31) / 32;
-    *tr = (int)(a < MAXIMA_ROW_TILES ? a : MAXIMA_ROW_TILES);
-    *tc = (int)b;
-}
-static int64_t round8(int64_t n) { return (n + 7) / 8 * 8; }     // ids 8 apart are workgroups of one XCD
-static int64_t parts_of(int64_t n, int t) { return (n / 128 + t - 1) / t; }
-
 // Up to here: beyond it the maxima of several operands push each other out of the Infinity Cache (256 MiB) before the conversions come,
 // and the shorter parts of the atomics form keep more loads in flight.  Steps, us, these two launches / the atomics form: 16 tokens 4096 ->
 // 4096 block-channel 37.6 / 41; 2000 tokens 4096 -> 4096 double-channel 125 / 138; 1000 tokens 14336 -> 8192 (268 MiB) 510 / 535; 2048
@@ -1043,11 +1026,7 @@ constexpr int64_t TOGETHER_BYTES = (int64_t)320 << 20;
 
 bool ti8::quant_together(int64_t bytes) { return bytes <= TOGETHER_BYTES; }
 
-int64_t ti8::quant_maxima_words(int64_t R, int64_t C) {
-    int tr, tc;
-    maxima_tiles(R, C, &tr, &tc);
-    return (parts_of(C, tc) * R + parts_of(R, tr) * C) / 2;
-}
+int64_t ti8::quant_maxima_words(int64_t R, int64_t C) { return idx::maxima_words(R, C); }
 
 int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int64_t* block_rows, int nblocks, const QRowColOperand* both, int nboth,
                     const QRowOperand* rows, int qflags, int inv_mode, ti8_stream_t stream) {
@@ -1073,7 +1052,7 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
     int64_t block_tiles = 0;
     if (int e = block_operands(fn, blocks, block_rows, nblocks, &b, &block_tiles)) return e;
     b.first[nblocks] = (int)block_tiles;
-    block_tiles = round8(block_tiles);
+    block_tiles = idx::round8(block_tiles);
     b.first[QBLOCK_MULTI_MAX] = (int)block_tiles;
     MaxMulti m;
     int64_t parts = 0, tiles = 0, first_tile[MAX_OPERANDS + 1];
@@ -1087,9 +1066,8 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
             return fail(TI8_ERR_ALIGN, "%s: pointers must be 16-byte aligned and strides multiples of 16 bytes", fn);
         if (o.R / ABSMAX_ROWS > 65535) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
         MaxOperand& x = m.op[i];
-        maxima_tiles(o.R, o.C, &x.tr, &x.tc);
-        x.nrt = (int)parts_of(o.R, x.tr);
-        x.nct = (int)parts_of(o.C, x.tc);
+        const idx::MaximaParts p = idx::maxima_parts(o.R, o.C);
+        x.tr = p.tr; x.tc = p.tc; x.nrt = p.nrt; x.nct = p.nct;
         x.x = static_cast<const uint16_t*>(o.x); x.ldx = o.ldx;
         x.rows = reinterpret_cast<uint16_t*>(o.partial);
         x.cols = x.rows + (int64_t)x.nct * o.R;
@@ -1097,8 +1075,8 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
         x.R = (int)o.R; x.C = (int)o.C; x.valid_rows = (int)o.valid_rows;
         m.first[i] = (int)parts;
         first_tile[i] = tiles;
-        parts += round8((int64_t)x.nrt * x.nct);
-        tiles += round8((o.R / 128) * (o.C / 128));
+        parts += idx::round8((int64_t)x.nrt * x.nct);
+        tiles += idx::round8((o.R / 128) * (o.C / 128));
         if (parts + block_tiles > 0x7fffffffLL || tiles > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
     }
     for (int i = nboth; i < MAX_OPERANDS; ++i) { m.op[i] = nboth ? m.op[0] : MaxOperand{}; m.first[i] = (int)parts; first_tile[i] = tiles; }
@@ -1121,7 +1099,7 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
     RowPart r = {};
     if (rows) {
         r.op = *rows;
-        r.workgroups = (int)round8(rows->C <= 4096 ? (rows->R + 3) / 4 : rows->R);
+        r.workgroups = (int)idx::round8(rows->C <= 4096 ? (rows->R + 3) / 4 : rows->R);
         if (parts + block_tiles + r.workgroups > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
     }
     hipLaunchKernelGGL(quant_first_kernel, dim3((unsigned)(parts + block_tiles + r.workgroups)), dim3(256), 0, st, m, b, r, mode);
