@@ -1,5 +1,5 @@
-"""The bias of the layer: added in the epilogue of the few-rows and the medium GEMM, by a kernel of its own behind the others, and its
-gradient as column sums."""
+"""The bias of the layer: added in the epilogue of the GEMM of a forward, whichever kernel that is, by a kernel of its own behind the
+GEMMs of a whole step on more than 256 tokens and output features, and its gradient as column sums."""
 import pytest
 import torch
 
@@ -44,6 +44,20 @@ def test_bias_in_the_epilogue_of_large_tiles(T, dev, scheme, had, tokens, k, n):
     x, w, b = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, n, k).to(dev), randn_bf16(g, n, std=30.0).to(dev)
     call = lambda bias: T.ops.linear_call(T._lib.PART_FORWARD, scheme, had, tokens, k, n, X=x, W=w, bias=bias)[0][:tokens]
     assert torch.equal(call(b), call(None) + b)
+
+
+# forward and backward in one call: Y beside dX and dW in one launch or two (few tokens), with a launch of its own (few output features), and
+# behind the GEMMs by the kernel that adds a bias
+@pytest.mark.parametrize("scheme", ["block_channel", "row_block", "double_channel"])
+@pytest.mark.parametrize("tokens,k,n", [(16, 512, 640), (16, 1152, 256), (200, 2048, 4096), (300, 512, 256), (1000, 384, 1152)])
+def test_bias_of_a_whole_step(T, dev, scheme, tokens, k, n):
+    g = make_gen(tokens + n)
+    x, w, dy, b = (t.to(dev) for t in (randn_bf16(g, tokens, k), randn_bf16(g, n, k), randn_bf16(g, tokens, n), randn_bf16(g, n, std=30.0)))
+    both = T._lib.PART_FORWARD | T._lib.PART_BACKWARD
+    call = lambda bias: T.ops.linear_call(both, scheme, None, tokens, k, n, X=x, W=w, dY=dy, one_launch=False, bias=bias)
+    (y, dx, dw, _), want = call(b), call(None)
+    assert torch.equal(y[:tokens], want[0][:tokens] + b)
+    assert torch.equal(dx[:tokens], want[1][:tokens]) and torch.equal(dw, want[2])
 
 
 @pytest.mark.parametrize("rows,cols", [(1, 32), (5, 96), (16, 512), (17, 544), (1500, 5632), (4099, 128), (3000, 14336)])

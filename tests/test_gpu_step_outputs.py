@@ -16,12 +16,12 @@ def _operands(dev, seed, m, k, n):
     return randn_bf16(g, m, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev), randn_bf16(g, m, n, std=1e-3).to(dev)
 
 
-def _linear_args(X, W, dY, out, scheme, need):
+def _linear_args(X, W, dY, out, scheme, need, bias=None):
     m, k, n = X.shape[0], X.shape[1], W.shape[0]
     workspace = ops._workspace(need, X.device)
     pairs = [v for t in (X, W, dY, *out) for v in (t.data_ptr(), t.stride(0))]
     return _lib.LinearArgs(*pairs, None, None, m, k, n, ops._SCHEMES[scheme], 0, _lib.PART_FORWARD | _lib.PART_BACKWARD, 0, workspace.data_ptr(), need,
-                           None, 0, None), workspace
+                           None, 0, None if bias is None else bias.data_ptr()), workspace
 
 
 # partial maxima of one tile and of several; ragged tokens
@@ -66,6 +66,23 @@ def test_outputs_that_share_memory(dev, scheme, m):
     T.linear_fwd_bwd(X, W, dY, scheme, out=beside)
     for a, b in zip(beside, (Y, dX, dW)):
         assert torch.equal(a, b)
+
+
+# the bias belongs to Y, and does not outlive it where dX or dW takes its place
+@pytest.mark.parametrize("m", [128, 384])
+def test_bias_of_an_output_that_is_written_over(dev, m):
+    k = n = 384
+    X, W, dY = _operands(dev, m, m, k, n)
+    b = randn_bf16(make_gen(m), n, std=30.0).to(dev)
+    Y, dX, dW = T.linear_fwd_bwd(X, W, dY, "block_channel")
+    need, _ = ops._linear_sizes(m, k, n, "block_channel", None, _lib.PART_FORWARD | _lib.PART_BACKWARD, False)
+    new = lambda rows: torch.empty((rows, k), dtype=torch.bfloat16, device=dev)
+    shared, y, dx, dw = new(max(m, n)), new(m), new(m), new(n)
+    for out, want in (((y, dx, dw), (Y + b, dX, dW)), ((shared[:m], shared[:m], dw), (dX, dX, dW)), ((shared[:m], dx, shared[:n]), (dW[:m], dX, dW))):
+        a, workspace = _linear_args(X, W, dY, out, "block_channel", need, b)
+        _lib.call("ti8_linear", ctypes.byref(a), ops._stream())
+        for got, expected in zip(out, want):
+            assert torch.equal(got[:expected.shape[0]], expected)
 
 
 # rows that the product's kernel quantises itself, and nine that have a quantiser; Y over X, and Y's 32 rows over X's last one

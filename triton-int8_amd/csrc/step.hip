@@ -357,9 +357,12 @@ int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t str
     const bool apart = count == 1 || outputs_apart(*L.a, L.T);
     // they go into one launch where none of them has so few rows that it would take the few-rows kernel
     if (L.bwd && (L.T < L.N ? L.T : L.N) > 256) {
-        for (int i = 0, n = apart ? count : 1; i < count; i += n)
+        for (int i = 0, n = apart ? count : 1; i < count; i += n) {
             if (int e = ti8_gemm_i8_nt_multi(g + i, n, flags | TI8_GEMM_TOGETHER, stream)) return e;
-        return L.fwd && L.a->bias ? add_bias(L.a->Y, L.a->ldy, L.a->bias, L.tokens, L.N, stream) : TI8_OK;
+            if (i == 0 && L.fwd && L.a->bias)       // (before dX or dW may take Y's place)
+                if (int e = add_bias(L.a->Y, L.a->ldy, L.a->bias, L.tokens, L.N, stream)) return e;
+        }
+        return TI8_OK;
     }
     ti8_gemm_problem few[3];
     const void* const bias = L.fwd ? L.a->bias : nullptr;
