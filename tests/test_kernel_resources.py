@@ -104,3 +104,57 @@ def test_chain_kernel_with_a_bias_waits_like_the_one_without(tmp_path):
         assert len(re.findall(r"^\s*global_store_dwordx4", block, flags=re.M)) in (0, 16)
     waits = {int(w) for w in re.findall(r"s_waitcnt vmcnt\((\d+)\)", body)}
     assert {16, 20} <= waits and max(waits) == 20
+
+
+VMEM = r"((?:global|buffer|flat|scratch)_(?:load|store|atomic)\w*)"
+
+
+def kernel_bodies(source, tmp_path, name):
+    text = open(compile_to_asm(source, tmp_path)).read()
+    bodies = {m.group(1): m.group(0) for m in re.finditer(r"^(_Z\w*" + name + r"\w*):.*?\.end_amdhsa_kernel", text, flags=re.S | re.M)}
+    assert bodies
+    return bodies
+
+
+def loops(body):
+    """Text between a label and the last branch back to it."""
+    for m in re.finditer(r"^(\.LBB\w+):", body, flags=re.M):
+        back = list(re.finditer(r"^\s*s_c?branch\w* " + re.escape(m.group(1)) + r"\b", body[m.end():], flags=re.M))
+        if back:
+            yield body[m.end():m.end() + back[-1].end()]
+
+
+def test_few_tokens_kernel_waits_match_its_stores(tmp_path):
+    """The walk over dW's tiles waits with vmcnt(8) for the next K tile while the stores of the tile before may be in flight: safe while
+    a wave issues exactly 8 memory instructions behind that K tile's loads, its stores of 16 bytes, with nothing branching between."""
+    src = open(os.path.join(PKG, "csrc", "gemm_skinny.hip")).read()
+    assert re.search(r"THIN_STORES = 8;", src)
+    for name, body in kernel_bodies("gemm_skinny.hip", tmp_path, "gemm_i8_few_kernel").items():
+        walks = 2 if "ILb0E" in name else 1         # operand A of dW scaled by blocks or by rows; int32 sums: by rows
+        assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", body), name
+        blocks = [re.findall(r"^\s*" + VMEM, b, flags=re.M) for b in re.split(r"^\.LBB\S+:|^\s*s_cbranch\w+|^\s*s_branch", body, flags=re.M)]
+        stores = [b for b in blocks if "global_store_dwordx4" in b]
+        assert stores == [["global_store_dwordx4"] * 8] * walks, (name, stores)
+        assert len(re.findall(r"s_waitcnt vmcnt\(8\) lgkmcnt\(0\)", body)) == walks, name
+        # the eight loads of a K tile, in front of the walk and in it, also in one piece
+        tiles = [b for b in blocks if b == ["global_load_lds_dwordx4"] * 8]
+        assert len(tiles) >= 2 * walks, name
+
+
+def test_attention_kernels_wait_for_what_they_issue(tmp_path):
+    """Every step of the attention's backward waits with vmcnt(n) for its own tile while the next one's n loads may be in flight: it has
+    to issue exactly n loads, all of them to LDS, and nothing else by the wait's barrier.  The kernels keep out of scratch memory in their loops
+    (dK and dV on four waves have one register too many, a store before and a load between them)."""
+    for name, body in kernel_bodies("attention.hip", tmp_path, "attention_d").items():
+        steps = re.findall(r"s_waitcnt vmcnt\((\d+)\) lgkmcnt\(0\)(.*?)(?=^\.LBB|^\s*s_c?branch|\Z)", body, flags=re.S | re.M)
+        assert len(steps) == 2, name            # with and without the mask
+        for n, step in steps:
+            assert re.match(r"[^\n]*\n(?:\s*;[^\n]*\n|\s*\n)*\s*s_barrier\b", step), (name, step[:200])
+            issued = re.findall(r"^\s*" + VMEM + r"([^\n]*)", step, flags=re.M)
+            assert len(issued) == int(n) and all(rest.rstrip().endswith("lds") for _, rest in issued), (name, n, issued)
+        ahead = body[:body.index("s_barrier")]
+        assert len(re.findall(r"^\s*buffer_load_\w+[^\n]* lds\s*$", ahead, flags=re.M)) >= 2 * int(steps[0][0]), name
+        scratch = int(re.search(r"\.amdhsa_private_segment_fixed_size (\d+)", body).group(1))
+        assert scratch <= (8 if "dkdv_kernelILi128ELi4E" in name else 0), (name, scratch)
+        inside = [loop for loop in loops(body) if "mfma" in loop]
+        assert len(inside) >= 2 and not any("scratch_" in loop for loop in inside), name
