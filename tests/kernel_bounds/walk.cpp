@@ -430,6 +430,197 @@ int walk_quant_call(const int64_t* R, const int64_t* C, int count, int block_til
     return r.bad;
 }
 
+// GEMM with few rows (gemm_skinny.hip: wavering_block), workgroups of one 32 x 32 block or of four (`wide`); scales by rows.  rows > 0: up to 8
+// rows of bf16 that it quantises itself (a_elems in bf16).  Every element of C that exists is stored once, every K tile is walked once.
+int walk_few_rows(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int wide, int rows, int64_t a_elems, int64_t b_elems, int64_t c_elems,
+                  int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    const int MB = wide ? 2 : 1, NB = MB, nk = (int)(K >> 7);
+    const int64_t b_at = rows ? 0 : MB * 4096, stage_bytes = b_at + NB * 4096, per_wave = 2 * stage_bytes + (rows ? 1024 : 0);
+    const int64_t lds = rows ? 4 * per_wave + 4 * 8 * 4 : wide ? 131072 : 65536;
+    const int mtiles = (int)((M + 32 * MB - 1) / (32 * MB)), nstrips = (int)(N / (32 * NB));
+    std::vector<uint8_t> stored((size_t)(M * N), 0);
+    const int64_t blocks = few_blocks(M, N, wide != 0);
+    if (rows && M != 32) r.fail("decode: %lld rows of C", (long long)M);
+    for (int64_t block = 0; block < blocks && !r.bad; ++block) {
+        const FewPlace p = few_place((int)block, mtiles, nstrips);
+        const int n0 = p.strip * 32 * NB, m0 = p.mt * 32 * MB, mblocks = imin(MB, ((int)M - m0) >> 5);
+        if (mblocks < 1 || n0 >= N) { r.fail("few rows: workgroup %lld has no block (%d, %d)", (long long)block, m0, n0); break; }
+        std::vector<uint8_t> walked((size_t)nk, 0);
+        for (int wave = 0; wave < 4; ++wave) {
+            const int kbeg = few_k_first(wave, nk), nq = few_k_first(wave + 1, nk) - kbeg;
+            const int rot = nq > 0 && !wide ? (int)((((unsigned)block >> 3) * 3u) % (unsigned)nq) : 0;
+            for (int i = 0; i <= nq; ++i) {         // one stage is fetched ahead
+                const int kt = few_k_tile(i, rot, kbeg, nq, nk);
+                if (kt < 0 || kt >= nk) { r.fail("few rows: K tile %d of %d", kt, nk); break; }
+                if (i < nq) ++walked[(size_t)kt];
+                const int64_t stage = wave * per_wave + (i & 1) * stage_bytes;
+                for (int lane = 0; lane < 64; ++lane) {
+                    const int ld_row = lane >> 3;
+                    if (rows) {
+                        const int64_t at = imin(ld_row, rows - 1) * lda + (lane & 7) * 16 + kt * 128;
+                        r.access("few rows X", at, 8, a_elems, block, wave, lane, kt);
+                        r.access("few rows X", at + 8, 8, a_elems, block, wave, lane, kt);
+                        r.access("few rows LDS codes", wave * per_wave + 2 * stage_bytes + ld_row * 128 + ((lane & 7) ^ ld_row) * 16, 16, lds, block, wave, lane);
+                    }
+                    for (int b = 0; b < MB; ++b)
+                        for (int q = 0; q < 4; ++q) {
+                            const int64_t chunk = ((lane & 7) ^ ld_row ^ (q & 1)) * 16;
+                            if (!rows) {
+                                r.access("few rows A", (m0 + imin(b, mblocks - 1) * 32 + 8 * q + ld_row) * lda + kt * 128 + chunk, 16, a_elems, block, wave, lane, kt);
+                                r.access("few rows LDS A", stage + b * 4096 + q * 1024 + lane * 16, 16, stage + b_at, block, wave, lane, q);
+                            }
+                            r.access("few rows B", (n0 + b * 32 + 8 * q + ld_row) * ldb + kt * 128 + chunk, 16, b_elems, block, wave, lane, kt);
+                            r.access("few rows LDS B", stage + b_at + b * 4096 + q * 1024 + lane * 16, 16, stage + stage_bytes, block, wave, lane, q);
+                        }
+                }
+            }
+            r.access("few rows LDS", wave * per_wave, per_wave, lds, block, wave);
+        }
+        for (int kt = 0; kt < nk && !r.bad; ++kt)
+            if (walked[(size_t)kt] != 1) r.fail("few rows: workgroup %lld walks K tile %d %d times", (long long)block, kt, (int)walked[(size_t)kt]);
+        r.access("few rows LDS sums", 0, (int64_t)MB * NB * 4 * 32 * 32 * 4, lds, block);
+        for (int t = 0; t < 256; ++t)
+            for (int i = 0; i < mblocks; ++i)
+                for (int j = 0; j < NB; ++j) {
+                    const int row = m0 + i * 32 + (t >> 3), col = n0 + j * 32 + (t & 7) * 4;
+                    if (!r.access("few rows C", row * ldc + col, 4, c_elems, block, t, i, j) || row >= M || col + 4 > N) { r.fail("few rows: C(%d, %d)", row, col); continue; }
+                    for (int c = 0; c < 4; ++c) ++stored[(size_t)(row * N + col + c)];
+                }
+    }
+    for (size_t i = 0; i < stored.size() && !r.bad; ++i)
+        if (stored[i] != 1) r.fail("few rows: C(%lld, %lld) is stored %d times", (long long)(i / N), (long long)(i % N), (int)stored[i]);
+    *n_checked = r.checked;
+    return r.bad;
+}
+
+// dW of a step on few tokens (gemm_skinny.hip: thin_walk): every tile belongs to one worker, its rows and K tiles are read, every element stored once
+int walk_thin(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int num_cu, int64_t a_elems, int64_t b_elems, int64_t c_elems,
+              int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    const int tiles_n = (int)(N >> 7), tiles = (int)(M >> 7) * tiles_n, nk = (int)(K >> 7), workers = (int)thin_workers(M, N, num_cu);
+    std::vector<uint8_t> seen((size_t)tiles, 0);
+    for (int worker = 0; worker < workers && !r.bad; ++worker) {
+        if (worker >= tiles) r.fail("thin: worker %d of %d has no tile, and fetches one all the same", worker, workers);
+        for (int tile = worker; tile < tiles && !r.bad; tile += workers) {
+            ++seen[(size_t)tile];
+            const int m0 = (tile / tiles_n) * 128, n0 = (tile % tiles_n) * 128;
+            std::vector<uint8_t> stored(128 * 16, 0), slab(32768 / 16, 0);
+            for (int wave = 0; wave < 4; ++wave)
+                for (int lane = 0; lane < 64; ++lane) {
+                    for (int kt = 0; kt < nk; ++kt)
+                        for (int i = 0; i < 4; ++i) {
+                            const int64_t row = wave * 32 + 8 * i + (lane >> 3), at = kt * 128 + ((lane & 7) ^ (lane >> 3) ^ (i & 1)) * 16;
+                            r.access("thin A", (m0 + row) * lda + at, 16, a_elems, tile, wave, lane, kt);
+                            r.access("thin B", (n0 + row) * ldb + at, 16, b_elems, tile, wave, lane, kt);
+                        }
+                    const int wm = (wave >> 1) * 64, wn = (wave & 1) * 64, fr_row = lane & 31, fr_half = lane >> 5;
+                    for (int i = 0; i < 2; ++i)
+                        for (int j = 0; j < 2; ++j)
+                            for (int q = 0; q < 4; ++q) {
+                                const int row = wm + i * 32 + fr_row, col = wn + j * 32 + 8 * q + 4 * fr_half, at = row * 256 + ((col * 2) ^ ((row & 15) << 4));
+                                if (r.access("thin LDS write", at, 8, 32768, tile, wave, lane)) slab[(size_t)at / 16] += 1;
+                            }
+                    for (int p = 0; p < 8; ++p) {
+                        const int row = p * 16 + wave * 4 + (lane >> 4), chunk = lane & 15;
+                        r.access("thin LDS read", row * 256 + ((chunk ^ (row & 15)) << 4), 16, 32768, tile, wave, lane, p);
+                        r.access("thin C", (m0 + row) * ldc + n0 + chunk * 8, 8, c_elems, tile, wave, lane, p);
+                        ++stored[(size_t)(row * 16 + chunk)];
+                    }
+                }
+            for (size_t i = 0; i < stored.size() && !r.bad; ++i)
+                if (stored[i] != 1 || slab[i] != 2) r.fail("thin: chunk %zu of tile %d is stored %d times, its halves written %d times", i, tile, (int)stored[i], (int)slab[i]);
+        }
+    }
+    for (int t = 0; t < tiles && !r.bad; ++t)
+        if (seen[(size_t)t] != 1) r.fail("thin: tile %d is taken %d times", t, (int)seen[(size_t)t]);
+    *n_checked = r.checked;
+    return r.bad;
+}
+
+// Attention's backward (attention.hip) on tensors of element strides sb, sh, ss: every load lies in its tensor or behind the rows of its pair
+// (where it reads zeros), every tile of scores at or under the diagonal is computed once per kernel, those without a mask lie under it, every
+// row of the results and every word of the workspace is stored once.  *past = rows behind the last that an offset reaches.
+int walk_attention(int64_t batch, int64_t heads, int64_t seq, int D, int64_t sb, int64_t sh, int64_t ss, int waves_dq, int waves_dkdv, int64_t elems,
+                   int64_t words, int64_t* past, int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    const int chunks = D / 8, slabs = 32 * 2 * D / 1024, rows_per_slab = 1024 / (2 * D), pairs = (int)(batch * heads);
+    const int64_t padded = (seq + 31) / 32 * 32, bytes = attention_bytes((int)seq, ss, D);
+    *past = 0;
+    auto load = [&](const char* what, int pair, int64_t row, int at) {
+        if (row - seq > *past) *past = row - seq;
+        const int64_t offset = row * ss * 2 + at;
+        ++r.checked;
+        if (offset >= bytes) return;
+        if (row >= seq || offset + 16 > bytes) r.fail("%s: row %lld, byte %d reaches into the buffer's end", what, (long long)row, at);
+        r.access(what, (pair / heads) * sb + (pair % heads) * sh + offset / 2, 8, elems, pair, row, at);
+    };
+    for (int keys = 0; keys < 2; ++keys) {      // 0: a workgroup owns queries (dQ), 1: keys (dK and dV)
+        const int waves = keys ? waves_dkdv : waves_dq, per_tile = slabs / waves, blocks = (int)((seq + waves * 32 - 1) / (waves * 32));
+        const int all = (int)((seq + 31) / 32);
+        std::vector<uint8_t> done((size_t)pairs * all * all, 0), row_stored((size_t)pairs * seq, 0), word_stored((size_t)(pairs * 2 * padded), 0);
+        for (int w = 0; w < (int)round8(pairs) * blocks && !r.bad; ++w) {
+            const AttentionPlace p = attention_place((uint32_t)w, blocks);
+            if (p.pair >= pairs) continue;
+            const int block = keys ? p.block : blocks - 1 - p.block, row0 = block * waves * 32;
+            if (block < 0 || block >= blocks) { r.fail("attention: workgroup %d takes block %d", w, block); break; }
+            const int first = keys ? row0 / 32 : 0;
+            const int tiles = keys ? all : (int)(((row0 + waves * 32 < seq ? row0 + waves * 32 : seq) + 31) / 32);
+            const int clear = keys ? imin(tiles, first + waves) : row0 / 32;
+            for (int tile = first; tile < tiles + 2; ++tile) {      // two are fetched ahead
+                std::vector<uint8_t> filled((size_t)32 * chunks, 0);
+                for (int wave = 0; wave < waves; ++wave)
+                    for (int lane = 0; lane < 64; ++lane) {
+                        for (int i = 0; i < per_tile; ++i) {
+                            const int row = wave * rows_per_slab + lane / chunks + i * 16;
+                            load("attention tile", p.pair, (int64_t)tile * 32 + row, (lane % chunks) * 16);
+                            const int lds = (wave + i * waves) * 1024 + lane * 16;
+                            if (r.access("attention LDS tile", lds, 16, 64 * D, w, wave, lane)) ++filled[(size_t)lds / 16];
+                            if (lds / (2 * D) != row) r.fail("attention: row %d of a tile lands in row %d", row, lds / (2 * D));
+                        }
+                        if (keys && tile < tiles) r.access("attention rows", p.pair * 2 * padded + (lane & 31) + (lane >> 5) * padded + tile * 32, 1, words, w, tile, lane);
+                    }
+                for (size_t i = 0; i < filled.size() && !r.bad; ++i)
+                    if (filled[i] != 1) r.fail("attention: chunk %zu of a tile is loaded %d times", i, (int)filled[i]);
+            }
+            for (int wave = 0; wave < waves; ++wave) {
+                const int own = row0 + wave * 32;
+                for (int lane = 0; lane < 64; ++lane)
+                    for (int ks = 0; ks < D / 16; ++ks) load("attention operand", p.pair, own + (lane & 31), (lane >> 5) * 16 + ks * 32);
+                for (int tile = first; tile < tiles; ++tile) {
+                    const bool masked = keys ? tile < clear : tile >= clear;
+                    if (masked && (keys ? (tile + 1) * 32 <= own : tile * 32 >= own + 32)) continue;
+                    const int query = keys ? tile * 32 : own, key = keys ? own : tile * 32;
+                    if (query >= seq || key >= seq) continue;       // rows that are zeros
+                    if (!masked && key + 31 > query) r.fail("attention: queries from %d and keys from %d without a mask", query, key);
+                    ++done[((size_t)p.pair * all + query / 32) * all + key / 32];
+                }
+                for (int row = own; row < own + 32; ++row) {
+                    if (row < seq) {
+                        ++row_stored[(size_t)(p.pair * seq + row)];
+                        r.access("attention result", (p.pair / heads) * sb + (p.pair % heads) * sh + row * ss, D, elems, w, row);
+                    }
+                    if (!keys && row < padded)
+                        for (int half = 0; half < 2; ++half)
+                            if (r.access("attention workspace", ((int64_t)p.pair * 2 + half) * padded + row, 1, words, w, row)) ++word_stored[(size_t)((p.pair * 2 + half) * padded + row)];
+                }
+            }
+        }
+        for (int pair = 0; pair < pairs && !r.bad; ++pair)
+            for (int m = 0; m < all; ++m)
+                for (int n = 0; n < all; ++n)
+                    if (done[((size_t)pair * all + m) * all + n] != (n <= m)) r.fail("attention: tile (%d, %d) of pair %d is computed %d times", m, n, pair, (int)done[((size_t)pair * all + m) * all + n]);
+        for (size_t i = 0; i < row_stored.size() && !r.bad; ++i)
+            if (row_stored[i] != 1) r.fail("attention: row %zu is stored %d times", i, (int)row_stored[i]);
+        for (size_t i = 0; !keys && i < word_stored.size() && !r.bad; ++i)
+            if (word_stored[i] != 1) r.fail("attention: word %zu is stored %d times", i, (int)word_stored[i]);
+    }
+    *n_checked = r.checked;
+    return r.bad;
+}
+
+int attention_takes_stride(int64_t stride, int64_t seq, int64_t head_dim) { return attention_stride_ok(stride, seq, head_dim); }
+
 struct ScaleArg {
     int mode;
     int64_t bs, rs, ks, elems;

@@ -45,6 +45,10 @@ def walker(tmp_path_factory):
     lib.walk_quant_row_form.argtypes = [i64] * 4 + [ci, ci] + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_maxima.argtypes = [i64] * 6 + [p64, cp, ci]
     lib.walk_quant_call.argtypes = [p64, p64, ci, ci, ci, p64, cp, ci]
+    lib.walk_few_rows.argtypes = [i64] * 6 + [ci, ci] + [i64] * 3 + [p64, cp, ci]
+    lib.walk_thin.argtypes = [i64] * 6 + [ci] + [i64] * 3 + [p64, cp, ci]
+    lib.walk_attention.argtypes = [i64] * 3 + [ci] + [i64] * 3 + [ci, ci] + [i64] * 2 + [p64, p64, cp, ci]
+    lib.attention_takes_stride.argtypes = [i64] * 3
     lib.maxima_scratch_words.argtypes = [i64, i64]
     lib.maxima_scratch_words.restype = i64
     lib.walk_quant_block.argtypes = [i64, i64, ci, i64, i64, ci, i64, i64, i64, i64, i64, i64, i64, i64, ci, i64, i64, i64, i64, p64, cp, ci]
@@ -287,6 +291,61 @@ def test_workgroups_of_a_calls_quantisers(walker, operands, block_tiles, row_gro
     msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
     R, C = ((ctypes.c_int64 * len(operands))(*(o[d] for o in operands)) for d in (0, 1))
     assert walker.walk_quant_call(R, C, len(operands), block_tiles, row_groups, ctypes.byref(n), msg, 512) == 0, msg.value.decode()
+
+
+# one block and four per workgroup: a last one with half its rows, strips that are and are not a multiple of 8, fewer K tiles than waves
+@pytest.mark.parametrize("M,N,K,wide", [(32, 128, 128, 0), (96, 384, 640, 0), (256, 1024, 1152, 0), (64, 1024, 256, 1), (96, 384, 384, 1), (160, 640, 1152, 1), (32, 128, 128, 1)])
+def test_few_rows_gemm(walker, M, N, K, wide):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    a, b, c = (M - 1) * (K + 16) + K, (N - 1) * K + K, (M - 1) * (N + 8) + N
+    run = lambda *elems: walker.walk_few_rows(M, N, K, K + 16, K, N + 8, wide, 0, *elems, ctypes.byref(n), msg, 512)
+    assert run(a, b, c) == 0, msg.value.decode()
+    for short, what in (((a - 1, b, c), b"few rows A"), ((a, b - 1, c), b"few rows B"), ((a, b, c - 1), b"few rows C")):
+        assert run(*short) == 1 and what in msg.value
+
+
+@pytest.mark.parametrize("rows", [1, 3, 8])
+@pytest.mark.parametrize("N,K", [(128, 128), (384, 640), (1024, 1152)])
+def test_decode_gemm(walker, rows, N, K):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    run = lambda x: walker.walk_few_rows(32, N, K, K + 8, K, N, 0, rows, x, N * K, 32 * N, ctypes.byref(n), msg, 512)
+    x = (rows - 1) * (K + 8) + K
+    assert run(x) == 0, msg.value.decode()
+    assert run(x - 1) == 1 and b"few rows X" in msg.value
+
+
+# fewer tiles than CUs and more, a remainder of the workers' rounds
+@pytest.mark.parametrize("M,N,K,num_cu", [(384, 128, 128, 256), (512, 1024, 256, 256), (640, 1152, 256, 8), (1024, 384, 128, 24)])
+def test_thin_gemm(walker, M, N, K, num_cu):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    a, b, c = M * K, N * K, (M - 1) * (N + 8) + N
+    run = lambda *elems: walker.walk_thin(M, N, K, K, K, N + 8, num_cu, *elems, ctypes.byref(n), msg, 512)
+    assert run(a, b, c) == 0, msg.value.decode()
+    for short, what in (((a - 1, b, c), b"thin A"), ((a, b - 1, c), b"thin B"), ((a, b, c - 1), b"thin C")):
+        assert run(*short) == 1 and what in msg.value
+
+
+# rows: one, tiles' edges, several blocks; pairs that are and are not a multiple of 8; dense and with the heads between the rows
+@pytest.mark.parametrize("batch,heads,seq", [(1, 1, 1), (2, 3, 32), (1, 8, 33), (1, 2, 257), (3, 3, 130), (1, 1, 640)])
+@pytest.mark.parametrize("D,waves", [(64, 4), (128, 4), (128, 8)])
+@pytest.mark.parametrize("rows_dense", [True, False])
+def test_attention_backward_launches(walker, batch, heads, seq, D, waves, rows_dense):
+    msg, n, past = ctypes.create_string_buffer(512), ctypes.c_int64(0), ctypes.c_int64(0)
+    sb, sh, ss = (heads * seq * D, seq * D, D) if rows_dense else (heads * seq * D, D, heads * D)
+    elems, words = batch * heads * seq * D, batch * heads * 2 * (-(-seq // 32) * 32)
+    run = lambda e, w: walker.walk_attention(batch, heads, seq, D, sb, sh, ss, 4, waves, e, w, ctypes.byref(past), ctypes.byref(n), msg, 512)
+    assert run(elems, words) == 0, msg.value.decode()
+    assert past.value <= 352
+    assert run(elems - 1, words) == 1 and b"attention" in msg.value
+    assert run(elems, words - 1) == 1 and b"attention" in msg.value
+
+
+def test_attention_offsets_fit_32_bits(walker):
+    for seq in (1, 100, 4096, 131071, 1 << 20, 1 << 23, 1 << 24):
+        widest = 0x3fffffff // (seq + 512)
+        assert walker.attention_takes_stride(widest, seq, min(widest, 64)) and not walker.attention_takes_stride(widest + 1, seq, 64)
+        assert not walker.attention_takes_stride(63, seq, 64)
+        assert (seq + 352) * widest * 2 + 256 <= 1 << 31        # as signed offsets, too
 
 
 @pytest.mark.parametrize("R,C", [(128, 8), (128, 520), (2048, 72), (4096, 512), (8192, 1024), (16384, 2048), (32768, 4096), (32768, 64),

@@ -18,6 +18,7 @@
 // for dQ, and its dK and dV do not fit the registers.
 #include <type_traits>
 #include "ti8_common.h"
+#include "index_math.h"
 
 namespace ti8 {
 
@@ -83,7 +84,7 @@ typedef __amdgpu_buffer_rsrc_t Rsrc;
 template <int D>
 __device__ __forceinline__ Rsrc rows_of(const Strided& t, int b, int h, int seq) {
     const uint16_t* p = t.p + b * t.sb + h * t.sh;
-    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p), 0, (int)(((int64_t)(seq - 1) * t.ss + D) * 2), 0x00027000);
+    return __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(p), 0, (int)(((int64_t)(seq - 1) * t.ss + D) * 2), 0x00027000);      // = idx::attention_bytes
 }
 __device__ __forceinline__ v8bf load_chunk(Rsrc r, uint32_t offset) { return __builtin_bit_cast(v8bf, __builtin_amdgcn_raw_buffer_load_b128(r, offset, 0, 0)); }
 
@@ -158,11 +159,10 @@ __device__ __forceinline__ void store_rows(const v16f (&x)[Tile<D>::COLS], float
     }
 }
 
-// workgroup -> (batch * head, block): the blocks of a pair on one XCD, whose L2 then serves the rows that they all stream
 __device__ __forceinline__ bool place(const AttentionArgs& a, int& pair, int& block) {
-    const int idx = blockIdx.x >> 3;
-    pair = (idx / a.blocks) * 8 + (blockIdx.x & 7);
-    block = idx % a.blocks;
+    const idx::AttentionPlace p = idx::attention_place(blockIdx.x, a.blocks);
+    pair = p.pair;
+    block = p.block;
     return pair < a.pairs;
 }
 #endif
@@ -376,7 +376,7 @@ int prepare(const char* fn) {
 template <int D, int WAVES_DQ, int WAVES_DKDV>
 int launch(const char* fn, AttentionArgs a, hipStream_t st) {
     if (int err = prepare<D, WAVES_DQ, WAVES_DKDV>(fn)) return err;
-    const int pairs = (a.pairs + 7) / 8 * 8;
+    const int pairs = (int)idx::round8(a.pairs);
     a.blocks = (a.seq + WAVES_DQ * 32 - 1) / (WAVES_DQ * 32);
     hipLaunchKernelGGL((attention_dq_kernel<D, WAVES_DQ>), dim3((unsigned)(pairs * a.blocks)), dim3(WAVES_DQ * 64), (DQ_LDS<D, WAVES_DQ>), st, a);
     if (int err = check_launch(fn)) return err;
@@ -402,7 +402,7 @@ using namespace ti8;
 
 extern "C" int64_t ti8_attention_bwd_workspace(int64_t batch, int64_t heads, int64_t seq) {
     if (batch <= 0 || heads <= 0 || seq <= 0 || seq > (1 << 24) || batch > 0xffffff || heads > 0xffffff || batch * heads > 0xffffff) return -1;
-    if ((batch * heads + 7) / 8 * 8 * ((seq + 127) / 128) > 0x7fffffff) return -1;      // workgroups of a launch
+    if (idx::round8(batch * heads) * ((seq + 127) / 128) > 0x7fffffff) return -1;      // workgroups of a launch
     return batch * heads * 2 * padded_rows(seq) * (int64_t)sizeof(float);
 }
 
@@ -418,8 +418,7 @@ extern "C" int ti8_attention_bwd(const ti8_attention_args* p, ti8_stream_t strea
         if (!x->p) return fail(TI8_ERR_NULL, "%s: q, k, v, o, d_o, dq, dk and dv are required", fn);
         if (!aligned16(x->p) || x->stride_b % 8 || x->stride_h % 8 || x->stride_s % 8)
             return fail(TI8_ERR_ALIGN, "%s: tensors must be 16-byte aligned with strides that are multiples of 8 elements", fn);
-        // (offsets into the rows of one (batch, head) are 32 bits and run up to 352 rows past the last one, where they read zeros)
-        if (x->stride_s < p->head_dim || x->stride_s > 0x3fffffff / (p->seq + 512))
+        if (!idx::attention_stride_ok(x->stride_s, p->seq, p->head_dim))
             return fail(TI8_ERR_SHAPE, "%s: a row stride of %lld elements does not go with %lld rows of %lld", fn, (long long)x->stride_s, (long long)p->seq, (long long)p->head_dim);
     }
     const auto strided = [](const ti8_attention_tensor& x) { return Strided{static_cast<const uint16_t*>(x.p), x.stride_b, x.stride_h, x.stride_s}; };

@@ -53,19 +53,11 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int mtiles = (g.M + 32 * MB - 1) / (32 * MB), nstrips = g.N / (32 * NB);
-    int strip, mt;
-    if ((nstrips & 7) == 0) {   // workgroups that share a strip of B on one XCD (ids 8 apart)
-        const int xcd = block_x & 7, idx = block_x >> 3;
-        strip = (idx / mtiles) * 8 + xcd;
-        mt = idx % mtiles;
-    } else {
-        strip = block_x / mtiles;
-        mt = block_x % mtiles;
-    }
-    const int n0 = strip * 32 * NB, m0 = mt * 32 * MB;
+    const idx::FewPlace place = idx::few_place(block_x, mtiles, nstrips);
+    const int n0 = place.strip * 32 * NB, m0 = place.mt * 32 * MB;
     const int mblocks = min(MB, (g.M - m0) >> 5);      // blocks of rows that exist; what is computed beyond them is not stored
     const int nk = g.K >> 7;
-    const int kbeg = (wave * nk) >> 2, kend = ((wave + 1) * nk) >> 2;
+    const int kbeg = idx::few_k_first(wave, nk), kend = idx::few_k_first(wave + 1, nk);
     const int nq = kend - kbeg;
 
     // ---- global -> LDS (same slab layout and swizzle as the other kernels): 4 instructions per block
@@ -92,11 +84,7 @@ __device__ __forceinline__ void wavering_block(const GemmArgs& g, const int bloc
     // the workgroups of an XCD read A's columns together, which then need not all fit its L2 (256 rows, K = 14336, N = 4096:
     // 36 us, 55 from different tiles on)
     const int rot = nq > 0 && BLOCKS == 1 ? (int)((((unsigned)block_x >> 3) * 3u + (unsigned)batch) % (unsigned)nq) : 0;
-    auto tile_of_step = [&](int i) {
-        int j = min(i, max(nq - 1, 0)) + rot;   // past the end: the last one again, into a free stage
-        if (j >= nq) j -= nq;
-        return min(kbeg + max(j, 0), nk - 1);
-    };
+    auto tile_of_step = [&](int i) { return idx::few_k_tile(i, rot, kbeg, nq, nk); };    // past the end: the last one again, into a free stage
     auto issue_stage = [&](int i) {
         int8_t* st = ring + (i & (WS_STAGES - 1)) * STAGE_BYTES;
         const int koff = tile_of_step(i) * 128;
@@ -539,7 +527,6 @@ constexpr int wavering_lds_bytes(bool wide) { return 4 * WS_STAGES * 2 * (wide ?
 static_assert(wavering_lds_bytes(false) >= 2 * 2 * THIN_OPERAND, "the tiles of dW share the launch");
 
 static bool is_wide(const GemmArgs& a, int64_t batch) { return idx::few_rows_wide(a.M, a.N, a.K, batch, device_cu_count()); }
-static int64_t wavering_blocks(const GemmArgs& a, bool wide) { return wide ? (int64_t)(a.N / 64) * ((a.M + 63) / 64) : (int64_t)(a.N / 32) * (a.M / 32); }
 
 int init_skinny_kernels() {
     static OncePerDevice all;
@@ -560,7 +547,7 @@ int init_skinny_kernels() {
 int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t st) {
     if (int e = init_skinny_kernels()) return e;
     const bool wide = is_wide(a, batch);
-    const dim3 grid((unsigned)wavering_blocks(a, wide), (unsigned)batch);
+    const dim3 grid((unsigned)idx::few_blocks(a.M, a.N, wide), (unsigned)batch);
     const auto kernel = wide ? (i32_full ? gemm_i8_wavering_kernel<true, 2> : gemm_i8_wavering_kernel<false, 2>)
                              : (i32_full ? gemm_i8_wavering_kernel<true, 1> : gemm_i8_wavering_kernel<false, 1>);
     hipLaunchKernelGGL(kernel, grid, dim3(256), wavering_lds_bytes(wide), st, a);
@@ -583,8 +570,7 @@ static int launch_few_group(GemmMulti& m, int few, bool wide, bool i32_full, hip
     const int64_t cus = device_cu_count();
     for (int i = 0; i < m.count; ++i) {
         m.first[i] = (int)total;
-        const int64_t tiles = (int64_t)(m.g[i].N / 128) * (m.g[i].M / 128);
-        total += i < few ? wavering_blocks(m.g[i], wide) : tiles < cus ? tiles : cus;
+        total += i < few ? idx::few_blocks(m.g[i].M, m.g[i].N, wide) : idx::thin_workers(m.g[i].M, m.g[i].N, cus);
         if (total > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "gemm: too many blocks");
     }
     for (int i = m.count; i <= GEMM_MULTI_MAX; ++i) m.first[i] = (int)total;

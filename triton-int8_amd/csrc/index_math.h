@@ -264,6 +264,55 @@ TI8_HD int operand_of(int at, const int* first, int count) {
 // every tile on the XCD that took its maxima where a part is one tile
 TI8_HD int rowcol_multi_tile(int block, int grid) { return ((grid >> 3) - 1 - (block >> 3)) * 8 + (block & 7); }
 
+// ---- GEMM with few rows (gemm_skinny.hip) ------------------------------------------------------
+// Workgroup -> strip of B and rows of A, in blocks of the workgroup's size: those that share a strip on one XCD (ids 8 apart)
+struct FewPlace {
+    int strip, mt;
+};
+TI8_HD FewPlace few_place(int block, int mtiles, int nstrips) {
+    FewPlace p;
+    if ((nstrips & 7) == 0) {
+        const int xcd = block & 7, idx = block >> 3;
+        p.strip = (idx / mtiles) * 8 + xcd;
+        p.mt = idx % mtiles;
+    } else {
+        p.strip = block / mtiles;
+        p.mt = block % mtiles;
+    }
+    return p;
+}
+TI8_HD int64_t few_blocks(int64_t M, int64_t N, bool wide) { return wide ? (N / 64) * ((M + 63) / 64) : (N / 32) * (M / 32); }
+// K tiles of a wave: [few_k_first(wave, nk), few_k_first(wave + 1, nk))
+TI8_HD int few_k_first(int wave, int nk) { return (wave * nk) >> 2; }
+// K tile of step i of a wave's walk over nq of nk, which starts at its tile `rot`; past the end: the last one again
+TI8_HD int few_k_tile(int i, int rot, int kbeg, int nq, int nk) {
+    int j = imin(i, imax(nq - 1, 0)) + rot;
+    if (j >= nq) j -= nq;
+    return imin(kbeg + imax(j, 0), nk - 1);
+}
+// dW beside them: workgroups for its 128 x 128 tiles, worker w taking w, w + workers, ...
+TI8_HD int64_t thin_workers(int64_t M, int64_t N, int64_t num_cu) {
+    const int64_t tiles = (M / 128) * (N / 128);
+    return tiles < num_cu ? tiles : num_cu;
+}
+
+// ---- attention's backward (attention.hip) ---------------------------------------------------------
+// Workgroup -> (batch, head) pair and block of its rows: the blocks of a pair on one XCD, whose L2 then serves the rows that they all
+// stream.  The grid has round8(pairs) * blocks workgroups; those of a pair beyond the last do nothing.
+struct AttentionPlace {
+    int pair, block;
+};
+TI8_HD AttentionPlace attention_place(uint32_t workgroup, int blocks) {
+    const int idx = (int)(workgroup >> 3);
+    return AttentionPlace{(idx / blocks) * 8 + (int)(workgroup & 7), idx % blocks};
+}
+// bytes from the first row of a pair to the last one's end: what lies behind reads as zeros
+TI8_HD int64_t attention_bytes(int seq, int64_t stride, int head_dim) { return ((int64_t)(seq - 1) * stride + head_dim) * 2; }
+TI8_HD bool attention_stride_ok(int64_t stride, int64_t seq, int64_t head_dim) {
+    // (offsets are 32 bits and run up to 352 rows past the last one)
+    return stride >= head_dim && stride <= 0x3fffffff / (seq + 512);
+}
+
 // ---- which kernel an entry point launches (decided on the host) ------------------------------
 
 // per-row quantiser: NLOAD 16-byte chunks per thread, one wave (4 rows per workgroup) or one
