@@ -9,8 +9,10 @@
 // Scores and their gradients go from one product into the next without leaving the wave's registers: a lane's results of a 32 x 32
 // score tile are four rows of every eight in one column, which is an MFMA operand over the rows if the other operand is read in the same
 // order, and the transposing LDS read (ds_read_b64_tr_b16) hands out four rows at a time.  A wave owns 32 rows of one operand in
-// registers; the other is streamed through LDS in tiles of 32 rows, filled two tiles ahead without a trip through registers, which
-// every wave reads twice, in rows for the scores and transposed for the gradients.
+// registers; the other is streamed through LDS in tiles of 32 rows, asked for two tiles ahead without a trip through registers, which
+// every wave reads twice, in rows for the scores and transposed for the gradients.  (In front of a step's first transposing read the
+// compiler waits for all loads, those of the tile two ahead among them: it takes them for what is read.  A tile so has the products of the
+// scores to arrive in.)
 //
 // Bound by the matrix pipe: batch 4, 32 heads, 4096 x 128: dQ 805 us (1.02 PFLOP/s of its own products), dK and dV 1095 us (1.0
 // PFLOP/s), 6.2 ms for torch's three kernels; a large bf16 matrix product reaches 1.17 PFLOP/s.
@@ -71,7 +73,8 @@ constexpr int larger(int a, int b) { return a > b ? a : b; }
 // stages: two tiles, and for dK and dV 64 floats per wave; the results pass through them at the end, 32 rows per wave
 template <int D, int WAVES> constexpr int DKDV_STAGE = 2 * Tile<D>::BYTES + WAVES * 256;
 // MFMA steps over D whose values a wave of the dK / dV kernel keeps in LDS: those that its registers do not hold
-// (two of eight; with all eight in registers the compiler spills: 1170 instead of 1095 us at the size above)
+// (two of eight; with all eight in registers the compiler spills in the loops: 1170 instead of 1095 us at the size above.  Four waves
+// are one register short all the same, and keep it in scratch memory between the loops)
 template <int D> constexpr int V_IN_LDS = D == 128 ? 2 : 0;
 template <int D, int WAVES> constexpr int DKDV_LDS = larger(STAGES * DKDV_STAGE<D, WAVES> + WAVES * V_IN_LDS<D> * 1024, WAVES * Tile<D>::BYTES);
 template <int D, int WAVES> constexpr int DQ_STAGE = 2 * Tile<D>::BYTES;
@@ -257,8 +260,8 @@ __global__ __launch_bounds__(WAVES * 64, 2) void attention_dkdv_kernel(const Att
     int stage = 0;
     auto walk = [&](int from, int to, auto masked) {
         for (int tile = from; tile < to; ++tile) {
-            // own loads of this tile landed (the next tile's may be in flight); behind the barrier everybody's, and nobody reads the
-            // stage of the tile before, which the tile after next goes into
+            // own loads of this tile landed (the next tile's may be in flight: as many as every wave issues for a tile); behind the
+            // barrier everybody's, and nobody reads the stage of the tile before, which the tile after next goes into
             wait_and_meet<LOADS>();
             issue(tile + 2, stage >= 1 ? stage - 1 : 2);
             if (!masked || (tile + 1) * TILE_ROWS > nw) step(smem + stage * DKDV_STAGE<D, WAVES>, tile * TILE_ROWS, masked);
