@@ -517,8 +517,8 @@ def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=Non
     """The forward, the backward or both of a layer in one or two library calls (``ti8_linear``; with ``one_launch`` and more than
     256 tokens and output features the quantisers as one call and the backward's or step's GEMMs as ``ti8_gemm_i8_nt_multi``).
     X bf16 [tokens, K], W bf16 [N, K], dY bf16 [tokens, N]: any number of tokens, no padded copies.  ``wq`` = (int8 [N, K], scales) of
-    the weight quantised earlier, ``bias`` bf16 [N] is added to Y (a forward alone).  Returns (Y [T, N], dX [T, K], dW [N, K], saved) with None for what `parts` does not ask for; T =
-    tokens rounded up to 128, rows from `tokens` on undefined."""
+    the weight quantised earlier, ``bias`` bf16 [N] is added to Y (where the quantisers are no call of their own).  Returns (Y [T, N],
+    dX [T, K], dW [N, K], saved) with None for what `parts` does not ask for; T = tokens rounded up to 128, rows from `tokens` on undefined."""
     T = -(-tokens // 128) * 128
     apart = one_launch and bool(parts & _lib.PART_BACKWARD) and min(T, N) > 256
     out = _native_call(parts, scheme, hadamard, tokens, K, N, X, W, dY, wq, saved, apart, bias)
