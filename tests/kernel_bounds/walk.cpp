@@ -494,6 +494,46 @@ int walk_few_rows(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int
     return r.bad;
 }
 
+// Y of up to 8 rows, 16 columns per workgroup (gemm_decode.hip): every K tile of the rows and of the weight is read where it is and used once by
+// one of the waves, every element of C stored once
+int walk_decode_narrow(int rows, int64_t N, int64_t K, int64_t ldx, int64_t ldb, int64_t ldc, int64_t x_elems, int64_t b_elems, int64_t c_elems,
+                       int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    const int nk = (int)(K >> 7);
+    std::vector<uint8_t> stored((size_t)(rows * N), 0);
+    for (int64_t block = 0; block < N / 16 && !r.bad; ++block) {
+        const int n0 = (int)block * 16;
+        std::vector<uint8_t> used((size_t)nk, 0);
+        for (int wave = 0; wave < 4; ++wave) {
+            const int kbeg = few_k_first(wave, nk), nq = few_k_first(wave + 1, nk) - kbeg, rot = decode_rot(n0, nq);
+            if (rot != (nq > 0 ? (int)((((unsigned)(n0 / 32) >> 3) * 3u) % (unsigned)nq) : 0)) r.fail("decode narrow: another walk than that of the block of 32 columns");
+            for (int batch = 0; batch == 0 || batch * DECODE_BATCH < nq; ++batch)
+                for (int lane = 0; lane < 64; ++lane) {
+                    for (int row = 0; row < rows; ++row) {
+                        const int64_t at = decode_x_offset(row, ldx, few_k_tile(batch * DECODE_BATCH + (lane >> 3), rot, kbeg, nq, nk), lane);
+                        r.access("decode narrow X", at, 8, x_elems, block, wave, lane, batch);
+                        r.access("decode narrow X", at + 8, 8, x_elems, block, wave, lane, batch);
+                    }
+                    for (int t = batch * DECODE_BATCH; t < nq && t < (batch + 1) * DECODE_BATCH; ++t)
+                        for (int h = 0; h < 2; ++h) r.access("decode narrow W", decode_w_offset(n0, ldb, few_k_tile(t, rot, kbeg, nq, nk), lane) + 64 * h, 16, b_elems, block, wave, lane, t);
+                }
+            for (int t = 0; t < nq; ++t) ++used[(size_t)few_k_tile(t, rot, kbeg, nq, nk)];
+        }
+        for (int kt = 0; kt < nk && !r.bad; ++kt)
+            if (used[(size_t)kt] != 1) r.fail("decode narrow: workgroup %lld uses K tile %d %d times", (long long)block, kt, (int)used[(size_t)kt]);
+        for (int lane = 0; lane < 64; ++lane) {
+            const int row = lane & 15, col = n0 + (lane >> 4) * 4;
+            if (row >= rows) continue;
+            if (!r.access("decode narrow C", row * ldc + col, 4, c_elems, block, 0, lane) || col + 4 > N) continue;
+            for (int c = 0; c < 4; ++c) ++stored[(size_t)(row * N + col + c)];
+        }
+    }
+    for (size_t i = 0; i < stored.size() && !r.bad; ++i)
+        if (stored[i] != 1) r.fail("decode narrow: C(%lld, %lld) is stored %d times", (long long)(i / N), (long long)(i % N), (int)stored[i]);
+    *n_checked = r.checked;
+    return r.bad;
+}
+
 // dW of a step on few tokens (gemm_skinny.hip: thin_walk): every tile belongs to one worker, its rows and K tiles are read, every element stored once
 int walk_thin(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int num_cu, int64_t a_elems, int64_t b_elems, int64_t c_elems,
               int64_t* n_checked, char* msg, int msglen) {

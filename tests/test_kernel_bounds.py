@@ -45,6 +45,7 @@ def walker(tmp_path_factory):
     lib.walk_quant_row_form.argtypes = [i64] * 4 + [ci, ci] + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_maxima.argtypes = [i64] * 6 + [p64, cp, ci]
     lib.walk_quant_call.argtypes = [p64, p64, ci, ci, ci, p64, cp, ci]
+    lib.walk_decode_narrow.argtypes = [ci] + [i64] * 8 + [p64, cp, ci]
     lib.walk_few_rows.argtypes = [i64] * 6 + [ci, ci] + [i64] * 3 + [p64, cp, ci]
     lib.walk_thin.argtypes = [i64] * 6 + [ci] + [i64] * 3 + [p64, cp, ci]
     lib.walk_attention.argtypes = [i64] * 3 + [ci] + [i64] * 3 + [ci, ci] + [i64] * 2 + [p64, p64, cp, ci]
@@ -312,6 +313,17 @@ def test_decode_gemm(walker, rows, N, K):
     x = (rows - 1) * (K + 8) + K
     assert run(x) == 0, msg.value.decode()
     assert run(x - 1) == 1 and b"few rows X" in msg.value
+
+
+@pytest.mark.parametrize("rows", [1, 5])
+@pytest.mark.parametrize("N,K", [(128, 128), (384, 640), (512, 4224), (128, 14336)])
+def test_decode_narrow_gemm(walker, rows, N, K):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    run = lambda *elems: walker.walk_decode_narrow(rows, N, K, K + 8, K + 16, N + 8, *elems, ctypes.byref(n), msg, 512)
+    x, b, c = (rows - 1) * (K + 8) + K, (N - 1) * (K + 16) + K, (rows - 1) * (N + 8) + N
+    assert run(x, b, c) == 0, msg.value.decode()
+    for short, what in (((x - 1, b, c), b"narrow X"), ((x, b - 1, c), b"narrow W"), ((x, b, c - 1), b"narrow C")):
+        assert run(*short) == 1 and what in msg.value
 
 
 # fewer tiles than CUs and more, a remainder of the workers' rounds

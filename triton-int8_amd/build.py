@@ -11,7 +11,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 LIB = os.path.join(HERE, "libti8.so")
 NATIVE = os.path.join(HERE, "_native.so")
-SOURCES = ["api.hip", "quant.hip", "fwht.hip", "gemm.hip", "gemm_chain.hip", "gemm_mid.hip", "gemm_skinny.hip", "step.hip", "decoder.hip", "attention.hip", "bias.hip", "probe.hip"]
+SOURCES = ["api.hip", "quant.hip", "fwht.hip", "gemm.hip", "gemm_chain.hip", "gemm_mid.hip", "gemm_skinny.hip", "gemm_decode.hip", "step.hip", "decoder.hip", "attention.hip", "bias.hip", "probe.hip"]
 
 # -ffp-contract=off: x*scale+0.5 must round twice (bit-exact quantisation); kernels
 #   that want an fma ask for one explicitly.

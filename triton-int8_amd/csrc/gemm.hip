@@ -837,20 +837,22 @@ int ti8::gemm_nt_few(const ti8_gemm_problem* problems, int count, bool backward,
 }
 
 // Up to 8 rows through a weight quantised earlier: the GEMM's kernel quantises them itself, each workgroup anew, where
-// idx::decode_quantises says so.  It saves a launch on a path that waits for the host: one token, 4096 -> 4096, 13.3 -> 9.9 us
-// (by rows 14.0 -> 10.8).
+// idx::decode_quantises or idx::decode_narrow says so.  It saves a launch on a path that waits for the host: one token, 4096 -> 4096,
+// 13.3 -> 9.9 us (by rows 14.0 -> 10.8).
 int ti8::gemm_nt_decode(const ti8_gemm_problem& p, const void* X, int64_t ldx, int64_t rows, const void* bias, int gemm_flags, bool* done, ti8_stream_t stream) {
     *done = false;
     if (rows > DECODE_ROWS || (gemm_flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES | TI8_GEMM_STRICT))) return TI8_OK;
     GemmArgs a;
     if (int e = prepare_gemm("ti8_gemm_i8_nt", p, gemm_flags, &a)) return e;
     const int cus = device_cu_count();
-    if (!skinny_supported(a) || idx::gemm_few_rows_prefers_mid(p.M, p.N, p.K, 1, cus) || !idx::decode_quantises(p.N, p.K, p.modeA == TI8_SCALE_ROW, cus)) return TI8_OK;
+    const bool by_rows = p.modeA == TI8_SCALE_ROW, narrow = idx::decode_narrow(p.N, p.K, rows, by_rows, cus);
+    if (!skinny_supported(a) || idx::gemm_few_rows_prefers_mid(p.M, p.N, p.K, 1, cus) || !(narrow || idx::decode_quantises(p.N, p.K, by_rows, cus))) return TI8_OK;
     a.A = static_cast<const int8_t*>(X);
     a.lda = ldx;
     a.bias = static_cast<const uint16_t*>(bias);
     *done = true;
-    return launch_decode(a, (int)rows, p.acc_i32_full != 0, static_cast<hipStream_t>(stream));
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    return narrow ? launch_decode_narrow(a, (int)rows, p.acc_i32_full != 0, st) : launch_decode(a, (int)rows, p.acc_i32_full != 0, st);
 }
 
 extern "C" int ti8_gemm_i8_nt(const int8_t* A, int64_t bsa, int64_t lda, const int8_t* B, int64_t bsb, int64_t ldb,

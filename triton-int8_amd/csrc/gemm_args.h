@@ -90,6 +90,7 @@ int launch_skinny(const GemmArgs& a, int64_t batch, bool i32_full, hipStream_t s
 // (TI8_SCALE_BLOCK128, reciprocal scales) or by rows (absmax / 127 with i32_full, else reciprocal scales)
 constexpr int DECODE_ROWS = 8;
 int launch_decode(const GemmArgs& a, int rows, bool i32_full, hipStream_t st);
+int launch_decode_narrow(const GemmArgs& a, int rows, bool i32_full, hipStream_t st);      // the same on few columns (gemm_decode.hip)
 // GEMMs over at most two K tiles, on 128 x 128 tiles: dW of a step on few tokens
 bool thin_supported(const GemmArgs& a, bool i32_full);
 // several GEMMs of batch 1 in one launch, the first `few` of m.g on the few-rows kernel, one behind them on thin tiles; fills first[] of `m`

@@ -290,6 +290,13 @@ TI8_HD int few_k_tile(int i, int rot, int kbeg, int nq, int nk) {
     if (j >= nq) j -= nq;
     return imin(kbeg + imax(j, 0), nk - 1);
 }
+// ---- Y of up to 8 rows by 16 rows of the weight per workgroup (gemm_decode.hip) --------------------------------------
+constexpr int DECODE_BATCH = 8;       // K tiles whose codes a wave makes together
+// first step of a wave's walk over nq K tiles: that of the 32 x 32 block around these columns
+TI8_HD int decode_rot(int n0, int nq) { return nq > 0 ? (int)((((unsigned)n0 >> 8) * 3u) % (unsigned)nq) : 0; }
+// the lane's 16 columns of a row's K tile, and its 16 bytes of the weight's (the second half of the K tile: 64 bytes on)
+TI8_HD int64_t decode_x_offset(int row, int64_t ldx, int kt, int lane) { return row * ldx + kt * 128 + (lane & 7) * 16; }
+TI8_HD int64_t decode_w_offset(int n0, int64_t ldb, int kt, int lane) { return (int64_t)(n0 + (lane & 15)) * ldb + kt * 128 + (lane >> 4) * 16; }
 // dW beside them: workgroups for its 128 x 128 tiles, worker w taking w, w + workers, ...
 TI8_HD int64_t thin_workers(int64_t M, int64_t N, int64_t num_cu) {
     const int64_t tiles = (M / 128) * (N / 128);
@@ -540,6 +547,16 @@ TI8_HD bool gemm_few_rows_prefers_mid(int64_t M, int64_t N, int64_t K, int64_t b
 // 14336 -> 10240 30.4 / 27.1, 14336 -> 14336 33.7 / 33.3.
 TI8_HD bool decode_quantises(int64_t N, int64_t K, bool by_rows, int num_cu) {
     return by_rows ? K / 128 <= 80 || N / 32 > num_cu : K / 128 <= 96 || N / 32 * 4 >= (int64_t)num_cu * 3;
+}
+
+// Whether up to 8 rows go to the kernel that takes 16 rows of the weight per workgroup (gemm_decode.hip).  Every workgroup makes the codes of
+// all rows: beyond one workgroup per CU that is what it spends its time on.  us, this one / gemm_i8_decode_kernel, at 1 row, 4 and 8:
+// 1024 -> 1024 3.0 3.7 4.7 / 4.0, 2048 -> 1024 3.6 4.3 5.2 / 5.1, 4096 -> 4096 4.9 5.6 6.6 / 7.5, 12288 -> 4096 11.5 13.1 15.6 / 18.3,
+// 14336 -> 5120 18.5 21.4 32.1 / 20.6, 8192 -> 8192 14.2 16.0 21.9 / 13.9, 4096 -> 14336 11.9 14.6 24.5 / 11.0.  By rows: 2048 -> 1024
+// 3.9 4.9 6.3 / 5.7, 4096 -> 4096 5.4 6.6 7.8 / 8.5, 12288 -> 4096 12.2 14.2 17.2 / 17.6; apart, 14336 -> 1024 10.4 12.9 17.9 / 16.6.
+TI8_HD bool decode_narrow(int64_t N, int64_t K, int64_t rows, bool by_rows, int num_cu) {
+    const int64_t nk = K / 128;
+    return N / 16 <= num_cu && (rows <= 4 || (nk >= 24 && (!by_rows || nk <= 96)));
 }
 
 }  // namespace idx
