@@ -49,6 +49,19 @@ def test_same_results(dev, monkeypatch, scheme, hadamard, tokens, rows):
         assert a.dtype == b.dtype == torch.bfloat16 and a.stride() == b.stride() and torch.equal(a, b)
 
 
+@pytest.mark.parametrize("tokens", [1, 8, 9, 128, 300])
+@pytest.mark.parametrize("scheme, hadamard", [("block_channel", None), ("row_block", 128)])
+def test_served(dev, monkeypatch, scheme, hadamard, tokens):
+    k, n = 256, 384
+    X, W = torch.randn(tokens, k, device=dev).to(torch.bfloat16), torch.randn(n, k, device=dev).to(torch.bfloat16)
+    wq = T.linear.quantize_weight(W, scheme, hadamard)
+    want = T.ops.linear_call(PART_FORWARD, scheme, hadamard, tokens, k, n, X=X, wq=wq)[0][:tokens]
+    for y in _both(monkeypatch, lambda: T.ops.linear_served(scheme, hadamard, tokens, k, n, X, wq)):
+        assert y.shape == want.shape and y.stride() == want.stride() and torch.equal(y, want)
+        y.resize_(tokens, n)        # the storage is what the shape needs, or more
+        assert torch.equal(y, want)
+
+
 def test_what_it_leaves_to_the_python_way(dev, monkeypatch):
     X, W = torch.randn(5, 256, device=dev).to(torch.bfloat16), torch.randn(128, 256, device=dev).to(torch.bfloat16)
     call = lambda x: T.ops.linear_call(PART_FORWARD, "block_channel", None, 5, 256, 128, X=x, W=W)[0][:5]

@@ -6,6 +6,8 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ops/empty.h>
+#include <c10/core/Allocator.h>
+#include <c10/core/impl/DeviceGuardImplInterface.h>
 
 #include "../../include/ti8.h"
 
@@ -40,19 +42,36 @@ struct GilReleased {
     ~GilReleased() { PyEval_RestoreThread(state); }
 };
 
+// Device memory that a call needs until its launches are queued, from torch's allocator like a tensor's but without making one
+struct Workspace {
+    c10::DataPtr plain;
+    at::Tensor tensor;
+    void* p;
+    Workspace(int64_t bytes, const at::Device& dev, const at::TensorOptions& options) {
+        if (c10::impl::getDeviceGuardImpl(c10::DeviceType::CUDA)->getDevice() == dev) {
+            plain = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(bytes);
+            p = plain.get();
+        } else {
+            tensor = at::empty({bytes}, options);
+            p = tensor.data_ptr();
+        }
+    }
+};
+
 PyObject* wrap(const at::Tensor& t) {
     if (t.defined()) return THPVariable_Wrap(t);
     Py_RETURN_NONE;
 }
 
-enum { PARTS, SCHEME, HADAMARD, TOKENS, K_, N_, GEMM_FLAGS, NEED, NEED_SAVED, APART, STREAM, NUMBERS, TENSORS = 7 };
+enum { PARTS, SCHEME, HADAMARD, TOKENS, K_, N_, GEMM_FLAGS, NEED, NEED_SAVED, APART, STREAM, SERVED, NUMBERS, TENSORS = 7 };
 
 // linear_call(parts, scheme, hadamard, tokens, K, N, gemm_flags, workspace bytes, saved bytes, whether the GEMMs are a call of their
-// own, stream, X, W, dY, wq, ws, saved, bias) -> (Y, dX, dW, saved), (name, status) of an entry point that failed, or None
+// own, stream, whether only Y is wanted, and of that the rows of tokens alone, X, W, dY, wq, ws, saved, bias) -> (Y, dX, dW, saved) or that Y,
+// (name, status) of an entry point that failed, or None
 PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     HANDLE_TH_ERRORS
     if (nargs != NUMBERS + TENSORS) {
-        PyErr_SetString(PyExc_TypeError, "linear_call takes 18 arguments");
+        PyErr_SetString(PyExc_TypeError, "linear_call takes 19 arguments");
         return nullptr;
     }
     at::Tensor X, W, dY, wq, ws, saved, bias;
@@ -84,7 +103,7 @@ PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
             dX = at::empty({T, K}, bf16);
             dW = at::empty({N, K}, bf16);
         }
-        const at::Tensor workspace = at::empty({v[NEED]}, bytes);
+        const Workspace workspace(v[NEED], dev, bytes);
         const auto ptr = [](const at::Tensor& t) -> void* { return t.defined() ? t.data_ptr() : nullptr; };
         const auto row = [](const at::Tensor& t) -> int64_t { return t.defined() ? t.stride(0) : 0; };
         ti8_linear_args a = {};
@@ -97,7 +116,7 @@ PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         a.wq = static_cast<const int8_t*>(ptr(wq)); a.ws = static_cast<const float*>(ptr(ws));
         a.tokens = tokens; a.K = K; a.N = N;
         a.scheme = (int)v[SCHEME]; a.hadamard = (int)v[HADAMARD]; a.parts = (int)v[PARTS]; a.gemm_flags = (int)v[GEMM_FLAGS];
-        a.workspace = ptr(workspace); a.workspace_bytes = v[NEED];      // (device allocations start on 512-byte boundaries)
+        a.workspace = workspace.p; a.workspace_bytes = v[NEED];      // (device allocations start on 512-byte boundaries)
         a.saved = ptr(saved); a.saved_bytes = v[NEED_SAVED];
         a.bias = ptr(bias);
         ti8_stream_t stream = reinterpret_cast<ti8_stream_t>(static_cast<uintptr_t>(v[STREAM]));
@@ -115,6 +134,10 @@ PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
         }
     }
     if (status != TI8_OK) return Py_BuildValue("(si)", name, status);
+    if (v[SERVED]) {
+        Y.unsafeGetTensorImpl()->set_sizes_contiguous({v[TOKENS], v[N_]});
+        return wrap(Y);
+    }
     return Py_BuildValue("(NNNN)", wrap(Y), wrap(dX), wrap(dW), wrap(saved));
     END_HANDLE_TH_ERRORS
 }

@@ -418,32 +418,34 @@ class Int8Linear(torch.nn.Module):
         self._wq, self._wq_key = None, None   # quantised weight of the forward-only path and what it was made from
 
     def forward(self, x):
-        weight = self.weight
+        # (parameters without the search that such an attribute of a module takes)
+        own = self._parameters
+        weight = own["weight"] if "weight" in own else self.weight
+        bias = own["bias"] if "bias" in own else self.bias
         if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
-            return Int8LinearFunction.apply(x, weight, self.bias, self.scheme, self.hadamard)
+            return Int8LinearFunction.apply(x, weight, bias, self.scheme, self.hadamard)
         if x.numel() == 0:
             return x.new_empty((*x.shape[:-1], self.out_features))
         # forward only (inference): the weight is quantised once per weight update, not per call
         key = (weight._version, weight.data_ptr(), self.scheme, self.hadamard)
         if self._wq_key != key or self._wq_of[0] is not weight:
             self._wq, self._wq_key, self._wq_of = quantize_weight(weight.detach(), self.scheme, self.hadamard), key, (weight,)
-        flat = x.dim() == 2
-        x2 = x if flat else x.reshape(-1, x.shape[-1])
-        tokens = x2.shape[0]
+        shape = x.shape
+        flat = len(shape) == 2
+        x2 = x if flat else x.reshape(-1, shape[-1])
+        tokens = shape[0] if flat else x2.shape[0]
         if _from_c():
-            if x2.shape[1] != self.in_features:
-                raise ValueError(f"expected {self.in_features} input features, got {x2.shape[1]}")
+            if shape[-1] != self.in_features:
+                raise ValueError(f"expected {self.in_features} input features, got {shape[-1]}")
             # a bias that wants its gradient is added by torch, which autograd sees
-            inside = _in_the_call(self.bias, self.out_features) and not (torch.is_grad_enabled() and self.bias.requires_grad)
-            y = ops.linear_call(PART_FORWARD, self.scheme, self.hadamard, tokens, self.in_features, self.out_features, X=x2, wq=self._wq,
-                                bias=self.bias if inside else None)[0]
+            inside = bias is not None and _in_the_call(bias, self.out_features) and not (torch.is_grad_enabled() and bias.requires_grad)
+            y = ops.linear_served(self.scheme, self.hadamard, tokens, self.in_features, self.out_features, x2, self._wq, bias if inside else None)
         else:
             inside = False
-            y, _ = linear_forward(pad_tokens(x2), None, self.scheme, self.hadamard, need_backward=False, wq=self._wq, tokens=tokens)
-        y = y[:tokens]
-        if self.bias is not None and not inside:
-            y = y + self.bias
-        return y if flat else y.reshape(*x.shape[:-1], self.out_features)
+            y = linear_forward(pad_tokens(x2), None, self.scheme, self.hadamard, need_backward=False, wq=self._wq, tokens=tokens)[0][:tokens]
+        if bias is not None and not inside:
+            y = y + bias
+        return y if flat else y.reshape(*shape[:-1], self.out_features)
 
     def extra_repr(self):
         return f"in_features={self.in_features}, out_features={self.out_features}, scheme={self.scheme}, hadamard={self.hadamard}"
