@@ -1044,6 +1044,30 @@ void walk_configs_together(const int64_t* shape, int count, int i32, int num_cu,
 // Workgroup -> (GEMM, tile) map of a several-GEMM launch (gemm.hip: gemm_i8_multi_kernel, launch_multi):
 // tiles[i] = workgroups of GEMM i.  Every workgroup of the grid must land in a GEMM i < count with
 // a tile index in [0, tiles[i]), and every (GEMM, tile) must be taken exactly once.
+// Tile map of the LDS-tiled GEMMs: every tile once, and the workgroups of an XCD (every eighth) on tiles that follow each other
+int walk_gemm_tile_map(int tiles_m, int tiles_n, int group, int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    const int total = tiles_m * tiles_n;
+    std::vector<int> order((size_t)total), seen((size_t)total, 0);       // place of a tile in groups of rows, column by column
+    for (int at = 0, m = 0; m < tiles_m; m += group)
+        for (int n = 0; n < tiles_n; ++n)
+            for (int i = m; i < imin(m + group, tiles_m); ++i) order[(size_t)(i * tiles_n + n)] = at++;
+    for (int xcd = 0; xcd < 8; ++xcd)
+        for (int w = xcd, last = -1; w < total && !r.bad; w += 8) {
+            const TileCoord t = gemm_tile_of(w, tiles_m, tiles_n, group);
+            if (t.tile_m < 0 || t.tile_m >= tiles_m || t.tile_n < 0 || t.tile_n >= tiles_n) { r.fail("tile map: workgroup %d has (%d, %d)", w, t.tile_m, t.tile_n); break; }
+            const int at = order[(size_t)(t.tile_m * tiles_n + t.tile_n)];
+            ++seen[(size_t)at];
+            if (last >= 0 && at != last + 1) r.fail("tile map: workgroup %d is at %d behind %d", w, at, last);
+            last = at;
+            ++r.checked;
+        }
+    for (int t = 0; t < total && !r.bad; ++t)
+        if (seen[(size_t)t] != 1) r.fail("tile map: tile %d is taken %d times", t, seen[(size_t)t]);
+    *n_checked = r.checked;
+    return r.bad;
+}
+
 int walk_gemm_multi_map(const int* tiles, int count, int64_t* n_checked, char* msg, int msglen) {
     Report r{msg, msglen};
     int first[4] = {0, 0, 0, 0};

@@ -45,6 +45,7 @@ def walker(tmp_path_factory):
     lib.walk_quant_row_form.argtypes = [i64] * 4 + [ci, ci] + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_maxima.argtypes = [i64] * 6 + [p64, cp, ci]
     lib.walk_quant_call.argtypes = [p64, p64, ci, ci, ci, p64, cp, ci]
+    lib.walk_gemm_tile_map.argtypes = [ci, ci, ci, p64, cp, ci]
     lib.walk_decode_narrow.argtypes = [ci] + [i64] * 8 + [p64, cp, ci]
     lib.walk_few_rows.argtypes = [i64] * 6 + [ci, ci] + [i64] * 3 + [p64, cp, ci]
     lib.walk_thin.argtypes = [i64] * 6 + [ci] + [i64] * 3 + [p64, cp, ci]
@@ -469,6 +470,13 @@ def test_one_call_step_reads_no_more_rows_than_there_are(recorded, rows, tokens)
     assert not calls
     T.ops.linear_step(X, W, dY, "block_channel", tokens=rows)
     assert calls[0][1][12] == -(-rows // 128) * 128 and calls[0][1][13] == rows
+
+
+@pytest.mark.parametrize("tiles_m,tiles_n,group", [(1, 1, 4), (1, 7, 8), (3, 5, 4), (8, 8, 4), (15, 33, 4), (9, 11, 8), (8, 39, 8)])
+def test_tile_map(walker, tiles_m, tiles_n, group):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    assert walker.walk_gemm_tile_map(tiles_m, tiles_n, group, ctypes.byref(n), msg, 512) == 0, msg.value.decode()
+    assert n.value == tiles_m * tiles_n
 
 
 @pytest.mark.parametrize("tiles", [[512, 512, 512], [1, 1, 1], [7, 300, 2], [5], [9, 4]])
