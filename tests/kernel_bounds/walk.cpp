@@ -838,7 +838,9 @@ int walk_gemm_chain(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t 
     const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN), per_batch = tiles_m * tiles_n;
     const int total = per_batch * (int)batch, nk = (int)(K >> 7), GROUP = gemm_group_rows(BM);
     const int64_t lds_words = (2 * (BM + BN) * 128 + NW * 16 * WCOLS * 4) / 4, slab0 = 2 * (BM + BN) * 128 / 4;
-    if (nk < 2 || nk > 256 || (nk & 1)) { r.fail("gemm chain: K / 128 = %d is odd or outside [2, 256]", nk); *n_checked = 0; return 1; }
+    if (!chain_takes(nk)) { r.fail("gemm chain: not over K / 128 = %d", nk); *n_checked = 0; return 1; }
+    const int walked = chain_walked(nk);
+    if (walked < nk || walked & 1 || walked > 256) r.fail("gemm chain: %d K tiles are walked as %d", nk, walked);
     std::vector<uint8_t> stored(c_elems <= (int64_t)1 << 30 ? (size_t)c_elems : 0, 0);
     std::vector<uint8_t> seen((size_t)total, 0);
     const bool a_in = sa.mode != 0, b_in = sb.mode != 0;
@@ -856,10 +858,10 @@ int walk_gemm_chain(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t 
                 const int wm = wave / WN, wn = wave % WN;
                 const int rA0 = gemm_wave_first_row(m0, wave, A_INSTR, (int)M), rB0 = gemm_wave_first_row(n0, wave, B_INSTR, (int)N);
                 const int tA0 = wave * A_INSTR, tB0 = wave * B_INSTR;
-                const int kts[4] = {0, 1, nk - 2, nk - 1};
+                const int kts[4] = {0, 1, walked - 2, walked - 1};
                 for (int lane = 0; lane < 64; ++lane) {
                     for (int q = 0; q < 4; ++q) {
-                        const int koff = kts[q] * 128;
+                        const int koff = gemm_k_offset(kts[q], (nk - 1) * 128);
                         for (int i = 0; i < A_INSTR; ++i) {
                             const uint32_t vo = gemm_lane_offset_bytes(lane, (tA0 + i) & 1, (int)lda);
                             r.access("gemm chain A", by * bsa + gemm_load_offset_bytes(rA0, lda, koff, i, vo), 16, a_elems, T, wave, lane, kts[q]);
@@ -872,7 +874,7 @@ int walk_gemm_chain(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t 
                     // per-K-tile factors: scalar base + (K tile >> shift) * stride per lane
                     const int64_t fa = gemm_factor_index(by, sa.bs, gemm_factor_block(m0 + wm * TM * 32, (int)M), sa.rs, 0, 0, 0);
                     const int64_t fb = gemm_factor_index(by, sb.bs, gemm_factor_block(n0 + wn * TN * 32, (int)N), sb.rs, 0, 0, 0);
-                    for (int c = 0; c <= (nk - 1) >> 6; ++c) {   // the factor register is refilled every 64 K tiles
+                    for (int c = 0; c <= (walked - 1) >> 6; ++c) {   // the factor register is refilled every 64 K tiles
                         const uint32_t kt = (uint32_t)gemm_factor_kt(c, lane, nk);
                         r.access("gemm chain factor A", fa + (int64_t)((kt >> (sa.mode == 3 ? 1 : 0)) * (uint32_t)(a_in ? sa.ks : 0)), 1, sa.elems, T, wave, lane, c);
                         r.access("gemm chain factor B", fb + (int64_t)((kt >> (sb.mode == 3 ? 1 : 0)) * (uint32_t)(b_in ? sb.ks : 0)), 1, sb.elems, T, wave, lane, c);

@@ -488,7 +488,7 @@ def test_multi_launch_map(walker, tiles):
 
 
 @pytest.mark.parametrize("M,N,K,batch,mA,mB,grid", [(8192, 4096, 4096, 1, 1, 0, 256), (4096, 4096, 8192, 1, 1, 1, 256), (4224, 4480, 256, 1, 1, 0, 256),
-                                                    (2048, 2304, 1024, 3, 0, 1, 256), (1152, 1408, 512, 2, 3, 0, 7), (8192, 8192, 512, 1, 0, 0, 256), (4096, 4096, 16384, 1, 1, 1, 256), (1280, 768, 32768, 1, 1, 0, 15)])
+                                                    (2048, 2304, 1024, 3, 0, 1, 256), (1152, 1408, 512, 2, 3, 0, 7), (640, 768, 128 * 19, 2, 1, 0, 7), (384, 512, 128 * 255, 1, 1, 1, 4), (8192, 8192, 512, 1, 0, 0, 256), (4096, 4096, 16384, 1, 1, 1, 256), (1280, 768, 32768, 1, 1, 0, 15)])
 def test_persistent_chain_kernel_geometries(walker, M, N, K, batch, mA, mB, grid):
     """gemm_i8_chain_kernel: tile lists of persistent workgroups, tiles that hang over M or N, batches, every scale layout."""
     def desc(mode, rows):

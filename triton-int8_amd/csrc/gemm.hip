@@ -903,7 +903,7 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
         one.g[0] = m.g[i];
         chains[i] = persistent && c[i].epi == EPI_PROMOTE_CHAIN && chain_persistent_supported(one);
     }
-    // Both kernels of the chained promotion in one call (an odd number of K tiles keeps a GEMM off the persistent one; same bits on
+    // Both kernels of the chained promotion in one call (few K tiles of an odd number keep a GEMM off the persistent one; same bits on
     // either): apart, the persistent kernel's last round is paid for in full, so they go apart only where it fills its rounds (8576
     // tokens, 2944 -> 12800, H_128, dX alone 408 tiles on 256 CUs: apart 1450 us, together 1406)
     int64_t chain_tiles = 0, others = 0;

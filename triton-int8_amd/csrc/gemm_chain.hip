@@ -11,10 +11,10 @@
 // Per tile this leaves the epilogue's own instructions; measured against one workgroup per tile: the
 // prologue, the workgroup turn-over and most of the store drain.
 // Arithmetic, operand layout in LDS, fragment reads and accumulator layout are those of the chained loop
-// in gemm.hip; results are bit-identical.  Limits: K / 128 even and in [2, 256] for every GEMM of the launch (a
+// in gemm.hip; results are bit-identical.  Limits: K / 128 in [2, 256] for every GEMM of the launch, and walked as an even number (a
 // tile's K tiles alternate between the two LDS buffers from a fixed start, which makes every LDS address a register
-// plus an immediate; one register holds the per-K-tile factors of 64 K tiles and is refilled every 64; the launcher
-// sends other shapes to the one-tile kernel).
+// plus an immediate; one register holds the per-K-tile factors of 64 K tiles and is refilled every 64; idx::chain_takes says
+// which odd numbers the launcher sends here, the others go to the one-tile kernel).
 //
 // The body is shared by three kernels: gemm_i8_chain_kernel, whose per-K-tile factor is uniform over a wave's tile, the same with a
 // bias in its epilogue (gemm_i8_chain_bias_kernel: nothing branches between the stores, whose number the waits count), and
@@ -187,13 +187,13 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         asm volatile("ds_read_b128 %0, %1" : "=v"(v) : "v"(addr) : "memory");
         return v;
     };
-    auto finish_factors = [&](const Tile& t, float ra, float rb) {
+    auto finish_factors = [&](const Tile& t, int block64, float ra, float rb) {
         const GemmArgs& g = m.g[t.gi];
         float f = g.sa.mode != TI8_SCALE_ROW ? ra : 1.0f;
         if (LANEB) return f;   // B's part, and the reciprocal of the product, per lane in the K loop
         if (g.sb.mode != TI8_SCALE_ROW) f = f * rb;
         if (g.combine == TI8_COMBINE_DIV_PROD) f = 1.0f / f;
-        return f;
+        return block64 * 64 + opaque_lane() < t.nk ? f : 0.0f;      // an odd number of K tiles is walked as one more, whose products count for nothing
     };
     // the 4 column scales this lane fetches for the epilogue (16 lanes cover the wave tile's 64 columns)
     auto load_col_scales = [&](const Tile& t, float (&cn)[4]) {
@@ -446,7 +446,7 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         if (LANEB) load_lane_factors(cur, 0);
         __builtin_amdgcn_s_waitcnt(0);
         __syncthreads();
-        fvec = finish_factors(cur, ra, rb);
+        fvec = finish_factors(cur, 0, ra, rb);
         load_a(cur, 128, wA + A_BYTES);
         load_b(cur, 128, wB + B_BYTES);
 #pragma unroll
@@ -455,7 +455,8 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
     }
     bool stored = false;   // whether this wave's previous epilogue left stores behind
     while (true) {
-        const int nk = cur.nk;
+        const int nk = LANEB ? cur.nk : idx::chain_walked(cur.nk);
+        auto k_at = [&](int kt) { return idx::gemm_k_offset(kt, (cur.nk - 1) * 128); };     // past the last one: that one again
         if (LANEB) divide_by_f = m.g[cur.gi].combine == TI8_COMBINE_DIV_PROD;
         // all but the last K tile: B of kt + 1 from this tile (for kt = 0 it is under way already); A of kt + 2 from this tile,
         // in the last of them K tile 0 of the next
@@ -466,26 +467,26 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         // K / 128 is even: a tile starts in LDS buffer 0 and its K tiles alternate 0, 1, 0, 1, ...
         {
             const bool a_next = 2 >= nk;
-            ktile_p(T_{}, T_{}, P0{}, stored, fvec, 0, cur, 128, a_next ? nxt : cur, a_next ? 0 : 256);
+            ktile_p(T_{}, T_{}, P0{}, stored, fvec, 0, cur, 128, a_next ? nxt : cur, a_next ? 0 : k_at(2));
         }
         // K tiles 1 .. nk - 2 in pairs (buffer 1, buffer 0).  The register `fvec` holds the factors of 64 K tiles: the pair that
         // straddles a multiple of 64 sits outside the inner loop and refills it in between (waited for on the spot: once per 64 K tiles)
         for (int kt = 1; kt < nk - 1;) {
             const int last = (kt | 63) - 2 < nk - 3 ? (kt | 63) - 2 : nk - 3;   // last odd K tile whose pair lies inside this block of 64
             for (; kt <= last; kt += 2) {
-                ktile_p(F_{}, T_{}, P1{}, false, fvec, kt, cur, (kt + 1) * 128, cur, (kt + 2) * 128);
+                ktile_p(F_{}, T_{}, P1{}, false, fvec, kt, cur, (kt + 1) * 128, cur, k_at(kt + 2));
                 const bool a_next = kt + 3 >= nk;
-                ktile_p(F_{}, T_{}, P0{}, false, fvec, kt + 1, cur, (kt + 2) * 128, a_next ? nxt : cur, a_next ? 0 : (kt + 3) * 128);
+                ktile_p(F_{}, T_{}, P0{}, false, fvec, kt + 1, cur, k_at(kt + 2), a_next ? nxt : cur, a_next ? 0 : k_at(kt + 3));
             }
             if (kt >= nk - 1) break;
-            ktile_p(F_{}, T_{}, P1{}, false, fvec, kt, cur, (kt + 1) * 128, cur, (kt + 2) * 128);
+            ktile_p(F_{}, T_{}, P1{}, false, fvec, kt, cur, (kt + 1) * 128, cur, k_at(kt + 2));
             {
                 float ra, rb;
                 load_raw_factors(cur, (kt + 1) >> 6, ra, rb);
-                fvec = finish_factors(cur, ra, rb);
+                fvec = finish_factors(cur, (kt + 1) >> 6, ra, rb);
             }
             const bool a_next = kt + 3 >= nk;
-            ktile_p(F_{}, T_{}, P0{}, false, fvec, kt + 1, cur, (kt + 2) * 128, a_next ? nxt : cur, a_next ? 0 : (kt + 3) * 128);
+            ktile_p(F_{}, T_{}, P0{}, false, fvec, kt + 1, cur, k_at(kt + 2), a_next ? nxt : cur, a_next ? 0 : k_at(kt + 3));
             kt += 2;
         }
         // last K tile: the column scales of this tile's epilogue travel beside it
@@ -517,7 +518,7 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         if (stored) __builtin_amdgcn_s_waitcnt(WAIT_FACTORS_BEHIND_STORES);
         else __builtin_amdgcn_s_waitcnt(WAIT_FACTORS);
         landed(ra, rb);
-        fvec = finish_factors(nxt, ra, rb);
+        fvec = finish_factors(nxt, 0, ra, rb);
         // the next tile's K tile 0 has been in LDS since the barrier of the last K tile: its first fragments
 #pragma unroll
         for (int ks = 0; ks < 4; ++ks) read_b(0, ks);
@@ -560,7 +561,7 @@ bool chain_persistent_supported(const GemmMulti& m) {
     if (m.g[0].bias && (m.count > 1 || lane_scales(m))) return false;
     for (int i = 0; i < m.count; ++i) {
         const int nk = m.g[i].K >> 7;
-        if (nk < 2 || nk > 256 || (nk & 1) || m.g[i].strict) return false;
+        if (!idx::chain_takes(nk) || (lane_scales(m) && (nk & 1)) || m.g[i].strict) return false;
         if (m.g[i].sa.mode == TI8_SCALE_ROW_K128 || (m.g[i].sb.mode == TI8_SCALE_ROW_K128) != lane_scales(m)) return false;
         // row by row, a wave's scales lie in 32 cache lines per load and bound either kernel (4 x 8192^3, whole call: 2835 us here, 2769
         // on one workgroup per tile); column by column 2266 against 2382 us for the GEMM

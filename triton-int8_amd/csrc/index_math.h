@@ -124,6 +124,12 @@ TI8_HD int epi_scale_lane(int lane, int c) { return 2 * (lane % 8) + (c >> 2); }
 // first column whose per-row scale of B a wave of the persistent kernel fetches: its tile's first column, or, for a
 // tile outside the operand (N is a multiple of 128, the wave tile has 64 columns), the operand's last 64 columns
 TI8_HD int chain_col_scale_first(int first_col_of_wave_tile, int ncols) { return imin(first_col_of_wave_tile, ncols - 64); }
+// whether the persistent kernel takes a GEMM over so many K tiles.  It walks them in pairs: an odd number as one more, the last one again
+// with a factor of 0, which changes no sum (x + 0 d = x).  us, this way / one workgroup per tile, 8192 x 4096: 9 K tiles 53.2 / 51.6,
+// 13 68.8 / 69.4, 17 85.8 / 85.3, 25 115.5 / 118.2, 57 242 / 253, 91 378 / 400; 2048 x 2048, 64 tiles: 17 33.1 / 33.9, 91 130 / 146.
+TI8_HD bool chain_takes(int nk) { return nk >= 2 && nk <= 256 && ((nk & 1) == 0 || nk >= 19); }
+// K tiles that it walks
+TI8_HD int chain_walked(int nk) { return (nk + 1) & ~1; }
 // tile that workgroup `w` of `grid` takes in the round that starts at tile `base`: its own number, in a partly filled last round of a
 // launch of several GEMMs counted from the other end -- the longest K comes first there, so that round goes to the workgroups
 // whose tiles before it were short.  Past the last tile: no tile (>= total), and none in any later round.
@@ -451,9 +457,9 @@ TI8_HD double gemm_set_time_large(const GemmSet& s, bool i32, int num_cu) {
     }
     const double mean = work / num_cu, longest = (double)busiest;
     if (i32) return 8.6 + 0.71 * longest + 0.95 * mean + 1.2 * (double)rounds;
-    // an odd number of K tiles keeps the launch off the persistent kernel
+    // a GEMM over few K tiles of an odd number keeps the launch off the persistent kernel
     bool odd = false;
-    for (int i = 0; i < s.count; ++i) odd = odd || (s.nk[i] & 1);
+    for (int i = 0; i < s.count; ++i) odd = odd || !chain_takes((int)s.nk[i]);
     return (7.7 + 1.15 * longest + 0.9 * mean + 0.4 * (double)rounds) * (odd ? 1.04 : 1.0);
 }
 // the medium-size kernel, one workgroup per CU: past one round a workgroup's turn-over is not hidden
