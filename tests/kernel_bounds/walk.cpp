@@ -838,7 +838,7 @@ int walk_gemm_chain(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t 
     const int tiles_m = (int)((M + BM - 1) / BM), tiles_n = (int)((N + BN - 1) / BN), per_batch = tiles_m * tiles_n;
     const int total = per_batch * (int)batch, nk = (int)(K >> 7), GROUP = gemm_group_rows(BM);
     const int64_t lds_words = (2 * (BM + BN) * 128 + NW * 16 * WCOLS * 4) / 4, slab0 = 2 * (BM + BN) * 128 / 4;
-    if (!chain_takes(nk)) { r.fail("gemm chain: not over K / 128 = %d", nk); *n_checked = 0; return 1; }
+    if (!chain_takes(nk, true)) { r.fail("gemm chain: not over K / 128 = %d", nk); *n_checked = 0; return 1; }
     const int walked = chain_walked(nk);
     if (walked < nk || walked & 1 || walked > 256) r.fail("gemm chain: %d K tiles are walked as %d", nk, walked);
     std::vector<uint8_t> stored(c_elems <= (int64_t)1 << 30 ? (size_t)c_elems : 0, 0);
@@ -1046,6 +1046,51 @@ void walk_configs_together(const int64_t* shape, int count, int i32, int num_cu,
 // Workgroup -> (GEMM, tile) map of a several-GEMM launch (gemm.hip: gemm_i8_multi_kernel, launch_multi):
 // tiles[i] = workgroups of GEMM i.  Every workgroup of the grid must land in a GEMM i < count with
 // a tile index in [0, tiles[i]), and every (GEMM, tile) must be taken exactly once.
+// Lists of the persistent chained kernel: every tile of every GEMM is on one workgroup's list of one XCD, each list in the order of the
+// launch, no workgroup busier than another by more than a tile that it could have left to it
+int walk_chain_list(const int* tiles, const int* cost, int count, int slots, int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    int n[3], base[4] = {0, 0, 0, 0}, first[CHAIN_LIST_SLOTS + 1];
+    uint16_t order[CHAIN_LIST_MAX];
+    std::vector<std::vector<int>> seen(count);
+    for (int i = 0; i < count; ++i) {
+        n[i] = (tiles[i] + 7) / 8;
+        base[i + 1] = base[i] + 8 * n[i];
+        seen[i].assign(tiles[i], 0);
+    }
+    if (base[count] / 8 > CHAIN_LIST_MAX) { r.fail("chain list: %d entries", base[count] / 8); *n_checked = 0; return 1; }
+    for (int i = count; i < 4; ++i) base[i] = base[count];
+    const int busiest = chain_list(n, cost, count, slots, first, order);
+    if (first[0] != 0 || first[slots] != base[count] / 8) r.fail("chain list: lists from %d to %d", first[0], first[slots]);
+    int most = 0, least_but_last = 0x7fffffff;
+    for (int s = 0; s < slots && !r.bad; ++s) {
+        int load = 0, last = 0;
+        for (int at = first[s]; at < first[s + 1] && !r.bad; ++at) {
+            if (at > first[s] && order[at] <= order[at - 1]) r.fail("chain list: workgroup %d takes %d behind %d", s, order[at], order[at - 1]);
+            for (int xcd = 0; xcd < 8; ++xcd) {
+                const int T = order[at] * 8 + xcd, gi = gemm_multi_pick(T, base[1], base[2], count), local = T - base[gi];
+                if (local < 0 || local >= 8 * n[gi]) r.fail("chain list: entry %d is none of GEMM %d", order[at], gi);
+                else if (local < tiles[gi]) ++seen[gi][(size_t)local], ++r.checked;
+                last = cost[gi];
+            }
+            load += last;
+        }
+        most = imax(most, load);
+        least_but_last = imin(least_but_last, load);
+    }
+    for (int s = 0; s < slots && !r.bad; ++s) {      // its last tile began when nobody else was free
+        int load = 0, last = 0;
+        for (int at = first[s]; at < first[s + 1]; ++at) load += last = cost[gemm_multi_pick(order[at] * 8, base[1], base[2], count)];
+        if (load - last > least_but_last) r.fail("chain list: workgroup %d of load %d took a tile of %d, another has %d in all", s, load, last, least_but_last);
+    }
+    if (!r.bad && most != busiest) r.fail("chain list: the busiest has %d, not %d", most, busiest);
+    for (int i = 0; i < count && !r.bad; ++i)
+        for (int t = 0; t < tiles[i]; ++t)
+            if (seen[i][(size_t)t] != 1) { r.fail("chain list: tile %d of GEMM %d is taken %d times", t, i, seen[i][(size_t)t]); break; }
+    *n_checked = r.checked;
+    return r.bad;
+}
+
 // Tile map of the LDS-tiled GEMMs: every tile once, and the workgroups of an XCD (every eighth) on tiles that follow each other
 int walk_gemm_tile_map(int tiles_m, int tiles_n, int group, int64_t* n_checked, char* msg, int msglen) {
     Report r{msg, msglen};

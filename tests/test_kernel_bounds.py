@@ -45,6 +45,7 @@ def walker(tmp_path_factory):
     lib.walk_quant_row_form.argtypes = [i64] * 4 + [ci, ci] + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_maxima.argtypes = [i64] * 6 + [p64, cp, ci]
     lib.walk_quant_call.argtypes = [p64, p64, ci, ci, ci, p64, cp, ci]
+    lib.walk_chain_list.argtypes = [ctypes.POINTER(ci), ctypes.POINTER(ci), ci, ci, p64, cp, ci]
     lib.walk_gemm_tile_map.argtypes = [ci, ci, ci, p64, cp, ci]
     lib.walk_decode_narrow.argtypes = [ci] + [i64] * 8 + [p64, cp, ci]
     lib.walk_few_rows.argtypes = [i64] * 6 + [ci, ci] + [i64] * 3 + [p64, cp, ci]
@@ -470,6 +471,18 @@ def test_one_call_step_reads_no_more_rows_than_there_are(recorded, rows, tokens)
     assert not calls
     T.ops.linear_step(X, W, dY, "block_channel", tokens=rows)
     assert calls[0][1][12] == -(-rows // 128) * 128 and calls[0][1][13] == rows
+
+
+# fewer tiles than workgroups, one each, a remainder of 8, most of the work in the longest or in the shortest, as many entries as a list has,
+# fewer workgroups than a list has room for
+@pytest.mark.parametrize("tiles,cost", [([3, 2], [9, 7]), ([256, 256, 256], [40, 30, 20]), ([80, 215, 688], [177, 69, 25]), ([75, 144, 1200], [197, 105, 17]),
+                                        ([513, 1, 7], [21, 20, 20]), ([495, 924, 420], [137, 117, 63]), ([1280, 1280, 1280], [64, 40, 11]), ([40], [9])])
+@pytest.mark.parametrize("slots", [32, 5])
+def test_chain_list(walker, tiles, cost, slots):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    array = lambda x: (ctypes.c_int * len(x))(*x)
+    assert walker.walk_chain_list(array(tiles), array(cost), len(tiles), slots, ctypes.byref(n), msg, 512) == 0, msg.value.decode()
+    assert n.value == sum(tiles)
 
 
 @pytest.mark.parametrize("tiles_m,tiles_n,group", [(1, 1, 4), (1, 7, 8), (3, 5, 4), (8, 8, 4), (15, 33, 4), (9, 11, 8), (8, 39, 8)])

@@ -710,9 +710,36 @@ int init_gemm_kernels() {
     return TI8_OK;
 }
 
+// Whether a launch of the persistent kernel is to take its tiles from a list, which is then filled, with `m` in its order: where the
+// busiest workgroup has that much less to do than by rounds.  Tiles of 256 x 256 cost their K tiles and about two and a half more.
+// (GEMMs of batch 1; us, the GEMMs of a step by rounds / by list: 4096 tokens, 11008 -> 1280 228 / 193; 1024, 11392 -> 7680 356 / 301; 768,
+// 12160 -> 6272 241 / 209; 13696, 1664 -> 7424 614 / 573.)
+static bool chain_by_list(GemmMulti& m, ChainList& list, int cus) {
+    std::stable_sort(m.g, m.g + m.count, [](const GemmArgs& x, const GemmArgs& y) { return x.K > y.K; });
+    int n[GEMM_MULTI_MAX], cost[GEMM_MULTI_MAX], entries = 0;
+    int64_t tiles[GEMM_MULTI_MAX], cost64[GEMM_MULTI_MAX];
+    for (int i = 0; i < m.count; ++i) {
+        tiles[i] = (int64_t)m.g[i].tiles_m * m.g[i].tiles_n;
+        if (tiles[i] > 8 * idx::CHAIN_LIST_MAX) return false;
+        n[i] = (int)((tiles[i] + 7) / 8);
+        cost64[i] = cost[i] = 2 * idx::chain_walked(m.g[i].K >> 7) + 5;
+        m.first[i] = entries * 8;
+        entries += n[i];
+        if (entries > idx::CHAIN_LIST_MAX) return false;
+    }
+    for (int i = m.count; i <= GEMM_MULTI_MAX; ++i) m.first[i] = entries * 8;
+    for (int i = m.count; i < GEMM_MULTI_MAX; ++i) m.g[i] = m.g[0];
+    if (cost[0] == cost[m.count - 1]) return false;
+    uint16_t order[idx::CHAIN_LIST_MAX] = {};
+    const int64_t busiest = idx::chain_list(n, cost, m.count, cus / 8, list.first, order);
+    if (busiest * 50 >= idx::chain_rounds_busiest(tiles, cost64, m.count, cus) * 49) return false;
+    for (int v = 0; v < idx::CHAIN_LIST_MAX; v += 2) list.tiles[v / 2] = order[v] | (uint32_t)order[v + 1] << 16;
+    return true;
+}
+
 // The chained promotion on persistent workgroups where its limits allow (gemm_chain.hip); CHAIN_UNAVAILABLE otherwise
 static int try_chain_persistent(GemmMulti& m, const int64_t* batch, hipStream_t st) {
-    if (!chain_persistent_supported(m)) return CHAIN_UNAVAILABLE;
+    if (!chain_persistent_supported(m, m.count > 1)) return CHAIN_UNAVAILABLE;
     int64_t total = 0;
     for (int i = 0; i < m.count; ++i) {
         m.g[i].tiles_m = (m.g[i].M + 255) / 256;
@@ -723,7 +750,16 @@ static int try_chain_persistent(GemmMulti& m, const int64_t* batch, hipStream_t 
     if (total > 0x3fffffff) return CHAIN_UNAVAILABLE;
     for (int i = m.count; i <= GEMM_MULTI_MAX; ++i) m.first[i] = (int)total;
     for (int i = m.count; i < GEMM_MULTI_MAX; ++i) m.g[i] = m.g[0];
-    return launch_chain_persistent(m, (int)total, device_cu_count(), st);
+    const int cus = device_cu_count();
+    if (m.count > 1 && m.g[0].sb.mode != TI8_SCALE_ROW_K128 && cus % 8 == 0 && cus / 8 <= idx::CHAIN_LIST_SLOTS) {
+        GemmMulti by_list = m;
+        ChainList list;
+        if (chain_by_list(by_list, list, cus)) {
+            const int rc = launch_chain_listed(by_list, list, cus, st);
+            if (rc != CHAIN_UNAVAILABLE) return rc;
+        }
+    }
+    return launch_chain_persistent(m, (int)total, cus, st);
 }
 
 // One GEMM on the LDS-tiled kernel that `c` names
@@ -901,7 +937,7 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
         GemmMulti one;
         one.count = 1;
         one.g[0] = m.g[i];
-        chains[i] = persistent && c[i].epi == EPI_PROMOTE_CHAIN && chain_persistent_supported(one);
+        chains[i] = persistent && c[i].epi == EPI_PROMOTE_CHAIN && chain_persistent_supported(one, count > 1);
     }
     // Both kernels of the chained promotion in one call (few K tiles of an odd number keep a GEMM off the persistent one; same bits on
     // either): apart, the persistent kernel's last round is paid for in full, so they go apart only where it fills its rounds (8576

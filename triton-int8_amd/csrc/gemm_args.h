@@ -75,8 +75,15 @@ struct GemmMulti {
 // (first[i + 1] - first[i] = tiles_m * tiles_n * batch of GEMM i).  launch returns TI8_OK, an error, or
 // CHAIN_UNAVAILABLE when the device refuses the 160 KiB of LDS (the caller then takes the one-tile kernel).
 constexpr int CHAIN_UNAVAILABLE = -1;
-bool chain_persistent_supported(const GemmMulti& m);
+bool chain_persistent_supported(const GemmMulti& m, bool several);     // several: on its own, or among others of a call
 int launch_chain_persistent(const GemmMulti& m, int total_tiles, int num_cu, hipStream_t st);
+// What the workgroups of each XCD take, from idx::chain_list (first[i] of the launch at multiples of 8, GEMM i having tiles_m * tiles_n of
+// the numbers from there on).  Two entries of 16 bits to a word: scalar loads.
+struct ChainList {
+    int first[idx::CHAIN_LIST_SLOTS + 1];
+    uint32_t tiles[idx::CHAIN_LIST_MAX / 2];
+};
+int launch_chain_listed(const GemmMulti& m, const ChainList& list, int num_cu, hipStream_t st);
 
 // Kernel for medium sizes (gemm_mid.hip): 128 x 128 tiles, EPI_ROWS (i32_full) or the promotion with factors that are uniform
 // over a wave's tile; K / 128 <= 256.  Fills tiles_m / tiles_n / first of `m`; batch > 1 only with m.count == 1.

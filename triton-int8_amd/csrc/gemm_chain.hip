@@ -16,10 +16,12 @@
 // plus an immediate; one register holds the per-K-tile factors of 64 K tiles and is refilled every 64; idx::chain_takes says
 // which odd numbers the launcher sends here, the others go to the one-tile kernel).
 //
-// The body is shared by three kernels: gemm_i8_chain_kernel, whose per-K-tile factor is uniform over a wave's tile, the same with a
+// The body is shared by four kernels: gemm_i8_chain_kernel, whose per-K-tile factor is uniform over a wave's tile, the same with a
 // bias in its epilogue (gemm_i8_chain_bias_kernel: nothing branches between the stores, whose number the waits count), and
 // gemm_i8_chain_lane_kernel, for operand B scaled per (row, K tile) (EPI_PROMOTE_CHAIN_LANE), where every lane fetches the
-// scales of its two columns one K tile ahead -- with the operand loads of that K tile, across tile boundaries too.
+// scales of its two columns one K tile ahead -- with the operand loads of that K tile, across tile boundaries too.  gemm_i8_chain_listed_kernel
+// takes its tiles from lists (idx::chain_list): where the GEMMs of a launch are over different numbers of K tiles, taking them by rounds
+// leaves most workgroups waiting for those that hold the long ones.
 #include <type_traits>
 #include "gemm_args.h"
 
@@ -78,8 +80,9 @@ struct Tile {
 
 // LANEB: operand B has one scale per (row, K tile); `col_p` / `col_s` then lead to the K tile 0 scales of the wave tile's
 // columns, `fb_ks` from one K tile to the next.
-template <bool LANEB, bool BIAS>
-__device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_tiles) {
+// LISTED: the tiles come from `list`, else by rounds out of `total_tiles`.
+template <bool LANEB, bool BIAS, bool LISTED>
+__device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_tiles, const ChainList* list) {
     extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
     // layout: [A buf0][A buf1][B buf0][B buf1][epilogue slab]
     int8_t* const ldsA = smem;
@@ -112,7 +115,6 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
     }
 
     constexpr int GROUP = idx::gemm_group_rows(BM);
-    const int stride_t = gridDim.x;
 
     // ---- tile T of the launch -> what the loops need --------------------------------------
     auto locate = [&](int T) {
@@ -429,14 +431,33 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         return true;
     };
 
-    const auto tile_of_round = [&](int base) { return idx::chain_tile_of_round(base, stride_t, total_tiles, (int)blockIdx.x, m.count > 1); };
+    // ---- the tiles of this workgroup, one after the other: a number, or -1 behind the last --------------------
+    int at = LISTED ? list->first[blockIdx.x >> 3] : 0;     // entry of the list, or first tile of the round
+    const int end = LISTED ? list->first[(blockIdx.x >> 3) + 1] : total_tiles;
+    const auto next_tile = [&]() {
+        if constexpr (LISTED) {
+            while (at < end) {
+                const int T = (int)((list->tiles[at >> 1] >> (16 * (at & 1))) & 0xffff) * 8 + (int)(blockIdx.x & 7);
+                ++at;
+                const int gi = idx::gemm_multi_pick(T, m.first[1], m.first[2], m.count);
+                if (T - m.first[gi] < m.g[gi].tiles_m * m.g[gi].tiles_n) return T;      // (not every XCD has the last tile of a GEMM)
+            }
+            return -1;
+        } else {
+            const int T = idx::chain_tile_of_round(at, (int)gridDim.x, total_tiles, (int)blockIdx.x, m.count > 1);
+            at += gridDim.x;
+            return T < end ? T : -1;
+        }
+    };
 
     // ---- first tile: operands of K tile 0 into LDS and registers, K tile 1's A half in flight ------------
-    int base = 0;      // first tile of the round of `cur`
-    Tile cur = locate(blockIdx.x);
+    int T = next_tile();
+    if (T < 0) return;
+    Tile cur = locate(T);
     // without a next tile the loads that run ahead fetch this tile's K tiles 0 and 1 again (nobody reads them)
-    bool more = tile_of_round(stride_t) < total_tiles;
-    Tile nxt = more ? locate(tile_of_round(stride_t)) : cur;
+    T = next_tile();
+    bool more = T >= 0;
+    Tile nxt = more ? locate(T) : cur;
     float fvec;
     {
         load_a(cur, 0, wA);
@@ -524,10 +545,10 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         for (int ks = 0; ks < 4; ++ks) read_b(0, ks);
         read_a(0, 0, 0);
         // the accumulators are free: the place for the integer divisions that find the tile after the next
-        base += stride_t;
         cur = nxt;
-        more = tile_of_round(base + stride_t) < total_tiles;
-        if (more) nxt = locate(tile_of_round(base + stride_t));
+        T = next_tile();
+        more = T >= 0;
+        if (more) nxt = locate(T);
 #pragma unroll
         for (int i = 0; i < TM; ++i)
 #pragma unroll
@@ -542,26 +563,31 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
 }  // namespace
 
 __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_kernel(const GemmMulti m, const int total_tiles) {
-    chain_tiles<false, false>(m, total_tiles);
+    chain_tiles<false, false, false>(m, total_tiles, nullptr);
 }
 
 // one GEMM, with g.bias
 __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_bias_kernel(const GemmMulti m, const int total_tiles) {
-    chain_tiles<false, true>(m, total_tiles);
+    chain_tiles<false, true, false>(m, total_tiles, nullptr);
 }
 
 __global__ __launch_bounds__(64 * NW) void gemm_i8_chain_lane_kernel(const GemmMulti m, const int total_tiles) {
-    chain_tiles<true, false>(m, total_tiles);
+    chain_tiles<true, false, false>(m, total_tiles, nullptr);
+}
+
+// GEMMs over different numbers of K tiles
+__global__ __launch_bounds__(64 * NW) void gemm_i8_chain_listed_kernel(const GemmMulti m, const ChainList list) {
+    chain_tiles<false, false, true>(m, 0, &list);
 }
 
 // operand B scaled per (row, K tile): all GEMMs of a launch or none
 static bool lane_scales(const GemmMulti& m) { return m.g[0].sb.mode == TI8_SCALE_ROW_K128; }
 
-bool chain_persistent_supported(const GemmMulti& m) {
+bool chain_persistent_supported(const GemmMulti& m, bool several) {
     if (m.g[0].bias && (m.count > 1 || lane_scales(m))) return false;
     for (int i = 0; i < m.count; ++i) {
         const int nk = m.g[i].K >> 7;
-        if (!idx::chain_takes(nk) || (lane_scales(m) && (nk & 1)) || m.g[i].strict) return false;
+        if (!idx::chain_takes(nk, several) || (lane_scales(m) && (nk & 1)) || m.g[i].strict) return false;
         if (m.g[i].sa.mode == TI8_SCALE_ROW_K128 || (m.g[i].sb.mode == TI8_SCALE_ROW_K128) != lane_scales(m)) return false;
         // row by row, a wave's scales lie in 32 cache lines per load and bound either kernel (4 x 8192^3, whole call: 2835 us here, 2769
         // on one workgroup per tile); column by column 2266 against 2382 us for the GEMM
@@ -579,16 +605,17 @@ bool chain_persistent_supported(const GemmMulti& m) {
 // its batch count; one workgroup per CU (fewer when there are fewer tiles)
 // Whether the current device grants the kernel its 160 KiB of LDS (asked once per device).  A refusal is remembered
 // and reported through ti8_last_error() by the call that met it; callers then take the one-tile kernel.
-enum ChainKernel { CHAIN, CHAIN_LANE, CHAIN_BIAS };
+enum ChainKernel { CHAIN, CHAIN_LANE, CHAIN_BIAS, CHAIN_LISTED };
 typedef void (*ChainFunction)(GemmMulti, int);
 static ChainFunction chain_function(ChainKernel k) { return k == CHAIN_LANE ? gemm_i8_chain_lane_kernel : k == CHAIN_BIAS ? gemm_i8_chain_bias_kernel : gemm_i8_chain_kernel; }
+static const void* chain_address(ChainKernel k) { return k == CHAIN_LISTED ? reinterpret_cast<const void*>(gemm_i8_chain_listed_kernel) : reinterpret_cast<const void*>(chain_function(k)); }
 
 template <ChainKernel K>
 static bool chain_kernel_available() {
     static OncePerDevice granted, refused;
     const uint64_t bit = 1ull << (current_device() & 63);
     if (refused.done.load(std::memory_order_acquire) & bit) return false;
-    const hipError_t e = raise_lds_limit(granted, reinterpret_cast<const void*>(chain_function(K)), LDS_BYTES);
+    const hipError_t e = raise_lds_limit(granted, chain_address(K), LDS_BYTES);
     if (e == hipSuccess) return true;
     refused.done.fetch_or(bit, std::memory_order_release);
     (void)fail(TI8_OK, "gemm: device %d refuses %d bytes of LDS for the persistent kernel (%s); one workgroup per tile serves its shapes",
@@ -600,6 +627,7 @@ int init_chain_kernel() {
     (void)chain_kernel_available<CHAIN>();
     (void)chain_kernel_available<CHAIN_LANE>();
     (void)chain_kernel_available<CHAIN_BIAS>();
+    (void)chain_kernel_available<CHAIN_LISTED>();
     return TI8_OK;
 }
 
@@ -609,6 +637,13 @@ int launch_chain_persistent(const GemmMulti& m, int total_tiles, int num_cu, hip
     const int grid = total_tiles < num_cu ? total_tiles : num_cu;
     hipLaunchKernelGGL(chain_function(lane ? CHAIN_LANE : biased ? CHAIN_BIAS : CHAIN), dim3((unsigned)grid), dim3(64 * NW), LDS_BYTES, st, m, total_tiles);
     note_gemm_kernel(TI8_KERNEL_PERSISTENT_CHAIN, BM, BN, lane ? EPI_PROMOTE_CHAIN_LANE : EPI_PROMOTE_CHAIN);
+    return check_launch("ti8_gemm_i8_nt");
+}
+
+int launch_chain_listed(const GemmMulti& m, const ChainList& list, int num_cu, hipStream_t st) {
+    if (!chain_kernel_available<CHAIN_LISTED>()) return CHAIN_UNAVAILABLE;
+    hipLaunchKernelGGL(gemm_i8_chain_listed_kernel, dim3((unsigned)num_cu), dim3(64 * NW), LDS_BYTES, st, m, list);
+    note_gemm_kernel(TI8_KERNEL_PERSISTENT_CHAIN, BM, BN, EPI_PROMOTE_CHAIN);
     return check_launch("ti8_gemm_i8_nt");
 }
 

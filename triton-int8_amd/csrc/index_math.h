@@ -127,7 +127,9 @@ TI8_HD int chain_col_scale_first(int first_col_of_wave_tile, int ncols) { return
 // whether the persistent kernel takes a GEMM over so many K tiles.  It walks them in pairs: an odd number as one more, the last one again
 // with a factor of 0, which changes no sum (x + 0 d = x).  us, this way / one workgroup per tile, 8192 x 4096: 9 K tiles 53.2 / 51.6,
 // 13 68.8 / 69.4, 17 85.8 / 85.3, 25 115.5 / 118.2, 57 242 / 253, 91 378 / 400; 2048 x 2048, 64 tiles: 17 33.1 / 33.9, 91 130 / 146.
-TI8_HD bool chain_takes(int nk) { return nk >= 2 && nk <= 256 && ((nk & 1) == 0 || nk >= 19); }
+// Beside others in a launch, which it would keep on one workgroup per tile, a GEMM goes there from 13 on (the three of a step: 15360 tokens,
+// 10112 -> 2176, one over 17 K tiles, 1147 us with one workgroup per tile, 1093; 9856, 1664 -> 1792, 13 K tiles 131, 133).
+TI8_HD bool chain_takes(int nk, bool several) { return nk >= 2 && nk <= 256 && ((nk & 1) == 0 || nk >= (several ? 13 : 19)); }
 // K tiles that it walks
 TI8_HD int chain_walked(int nk) { return (nk + 1) & ~1; }
 // tile that workgroup `w` of `grid` takes in the round that starts at tile `base`: its own number, in a partly filled last round of a
@@ -135,6 +137,78 @@ TI8_HD int chain_walked(int nk) { return (nk + 1) & ~1; }
 // whose tiles before it were short.  Past the last tile: no tile (>= total), and none in any later round.
 TI8_HD int chain_tile_of_round(int base, int grid, int total, int w, bool several) {
     return several && base + grid > total ? base + grid - 1 - w : base + w;
+}
+// cost of the busiest of `grid` workgroups that take tiles by rounds (chain_tile_of_round), a tile of GEMM i costing cost[i]: the load changes
+// only where a GEMM begins, so those workgroups are looked at
+TI8_HD int64_t chain_rounds_busiest(const int64_t* tiles, const int64_t* cost, int count, int grid) {
+    int64_t first[4] = {0, 0, 0, 0};
+    for (int i = 0; i < count; ++i) first[i + 1] = first[i] + tiles[i];
+    const int64_t total = first[count], rounds = (total + grid - 1) / grid;
+    int64_t busiest = 0;
+    for (int q = 0; q < 4 * (count + 1); ++q) {
+        int64_t w = (first[q >> 2] + grid - 1 + (q & 1)) % grid;   // the last workgroup in front of GEMM q / 4, or its first
+        if (q & 2) w = grid - 1 - w;
+        int64_t load = 0;
+        for (int64_t r = 0; r < rounds; ++r) {
+            const int64_t t = r * grid + (r == rounds - 1 && count > 1 ? grid - 1 - w : w);
+            if (t < total) load += cost[t < first[1] ? 0 : (t < first[2] || count < 3 ? 1 : 2)];
+        }
+        if (load > busiest) busiest = load;
+    }
+    return busiest;
+}
+// The same for GEMMs over different numbers of K tiles, from a list: tiles in order, the longest K first, each to the workgroup that is
+// free first.  A list serves the workgroups of one XCD (`slots` of them): XCD x takes tiles x, x + 8, ... of every GEMM, whose
+// neighbours in its L2 they then stay, and entry v is tile 8 v + x of the launch, GEMM i having the tiles from 8 (n[0] + .. + n[i - 1]) on.
+// cost[i] descending.  tile[first[s]] .. tile[first[s + 1] - 1]: what workgroup s takes.  Returns the cost of the busiest.
+constexpr int CHAIN_LIST_SLOTS = 32, CHAIN_LIST_MAX = 480;
+inline int chain_list(const int* n, const int* cost, int count, int slots, int* first, uint16_t* tile) {
+    int free_at[CHAIN_LIST_SLOTS] = {}, slot_of[CHAIN_LIST_SLOTS];      // workgroups by the time at which they are free
+    for (int s = 0; s < slots; ++s) slot_of[s] = s;
+    uint8_t taken_by[CHAIN_LIST_MAX];
+    int v = 0, busiest = 0;
+    for (int i = 0; i < count; ++i) {
+        // those that have not taken a tile of this GEMM yet, from `head` on, and those that have, in the order in which they are free again
+        int head = 0, again_at[CHAIN_LIST_SLOTS], again[CHAIN_LIST_SLOTS], begin = 0, held = 0;
+        for (int k = 0; k < n[i]; ++k) {
+            int at, s;
+            if (head < slots && (held == 0 || free_at[head] <= again_at[begin])) {
+                at = free_at[head];
+                s = slot_of[head++];
+            } else {
+                at = again_at[begin];
+                s = again[begin];
+                begin = (begin + 1) % CHAIN_LIST_SLOTS;
+                --held;
+            }
+            const int to = (begin + held++) % CHAIN_LIST_SLOTS;
+            again_at[to] = at + cost[i];
+            again[to] = s;
+            taken_by[v++] = (uint8_t)s;
+        }
+        int merged_at[CHAIN_LIST_SLOTS], merged[CHAIN_LIST_SLOTS];
+        for (int q = 0; q < slots; ++q) {
+            const bool old = head < slots && (held == 0 || free_at[head] <= again_at[begin]);
+            merged_at[q] = old ? free_at[head] : again_at[begin];
+            merged[q] = old ? slot_of[head] : again[begin];
+            if (old) ++head;
+            else {
+                begin = (begin + 1) % CHAIN_LIST_SLOTS;
+                --held;
+            }
+        }
+        for (int q = 0; q < slots; ++q) {
+            free_at[q] = merged_at[q];
+            slot_of[q] = merged[q];
+        }
+        busiest = free_at[slots - 1];
+    }
+    int at[CHAIN_LIST_SLOTS + 1] = {};
+    for (int k = 0; k < v; ++k) ++at[taken_by[k] + 1];
+    for (int s = 0; s < slots; ++s) at[s + 1] += at[s];
+    for (int s = 0; s <= slots; ++s) first[s] = at[s];
+    for (int k = 0; k < v; ++k) tile[at[taken_by[k]]++] = (uint16_t)k;
+    return busiest;
 }
 TI8_HD int epi_chain_slab_row(int e, int fr_half) { return 8 * (e >> 2) + 4 * fr_half + (e & 3); }
 TI8_HD int epi_chain_slab_word(int row, int col) { return row * 64 + (col ^ (4 * (row & 1))); }
@@ -434,32 +508,20 @@ TI8_HD double gemm_set_time_small(const GemmSet& s, bool i32, int num_cu) {
     const double t = i32 ? 5.0 + 0.28 * longest + 0.71 * mean + 2.9 * tiles / slots : 6.3 + 0.37 * longest + 0.96 * mean + 1.84 * tiles / slots;
     return t > alone ? t : alone;
 }
-// 256 x 256 tiles.  The busiest CU: workgroup w takes tile w of every round, in the last one counted from the end (as the persistent
-// kernel does); its load changes only where a GEMM begins, so those workgroups are looked at.
+// 256 x 256 tiles, by rounds
 TI8_HD double gemm_set_time_large(const GemmSet& s, bool i32, int num_cu) {
-    int64_t first[4] = {0, 0, 0, 0};
+    int64_t tiles[3], total = 0;
     double work = 0;
     for (int i = 0; i < s.count; ++i) {
-        first[i + 1] = first[i] + gemm_set_tiles(s, i, 256);
-        work += (double)(gemm_set_tiles(s, i, 256) * s.nk[i]);
+        total += tiles[i] = gemm_set_tiles(s, i, 256);
+        work += (double)(tiles[i] * s.nk[i]);
     }
-    const int64_t total = first[s.count], rounds = (total + num_cu - 1) / num_cu;
-    int64_t busiest = 0;
-    for (int q = 0; q < 4 * (s.count + 1); ++q) {
-        int64_t w = (first[q >> 2] + num_cu - 1 + (q & 1)) % num_cu;   // the last workgroup in front of GEMM q / 4, or its first
-        if (q & 2) w = num_cu - 1 - w;
-        int64_t load = 0;
-        for (int64_t r = 0; r < rounds; ++r) {
-            const int64_t t = r * num_cu + (r == rounds - 1 && s.count > 1 ? num_cu - 1 - w : w);
-            if (t < total) load += s.nk[t < first[1] ? 0 : (t < first[2] || s.count < 3 ? 1 : 2)];
-        }
-        if (load > busiest) busiest = load;
-    }
-    const double mean = work / num_cu, longest = (double)busiest;
+    const int64_t rounds = (total + num_cu - 1) / num_cu;
+    const double mean = work / num_cu, longest = (double)chain_rounds_busiest(tiles, s.nk, s.count, num_cu);
     if (i32) return 8.6 + 0.71 * longest + 0.95 * mean + 1.2 * (double)rounds;
     // a GEMM over few K tiles of an odd number keeps the launch off the persistent kernel
     bool odd = false;
-    for (int i = 0; i < s.count; ++i) odd = odd || !chain_takes((int)s.nk[i]);
+    for (int i = 0; i < s.count; ++i) odd = odd || !chain_takes((int)s.nk[i], false);
     return (7.7 + 1.15 * longest + 0.9 * mean + 0.4 * (double)rounds) * (odd ? 1.04 : 1.0);
 }
 // the medium-size kernel, one workgroup per CU: past one round a workgroup's turn-over is not hidden
