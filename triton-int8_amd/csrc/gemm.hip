@@ -711,7 +711,7 @@ int init_gemm_kernels() {
 }
 
 // Whether a launch of the persistent kernel is to take its tiles from a list, which is then filled, with `m` in its order: where the
-// busiest workgroup has that much less to do than by rounds.  Tiles of 256 x 256 cost their K tiles and about two and a half more.
+// busiest workgroup has that much less to do than by rounds.
 // (GEMMs of batch 1; us, the GEMMs of a step by rounds / by list: 4096 tokens, 11008 -> 1280 228 / 193; 1024, 11392 -> 7680 356 / 301; 768,
 // 12160 -> 6272 241 / 209; 13696, 1664 -> 7424 614 / 573.)
 static bool chain_by_list(GemmMulti& m, ChainList& list, int cus) {
@@ -722,7 +722,7 @@ static bool chain_by_list(GemmMulti& m, ChainList& list, int cus) {
         tiles[i] = (int64_t)m.g[i].tiles_m * m.g[i].tiles_n;
         if (tiles[i] > 8 * idx::CHAIN_LIST_MAX) return false;
         n[i] = (int)((tiles[i] + 7) / 8);
-        cost64[i] = cost[i] = 2 * idx::chain_walked(m.g[i].K >> 7) + 5;
+        cost64[i] = cost[i] = idx::chain_tile_cost(m.g[i].K >> 7);
         m.first[i] = entries * 8;
         entries += n[i];
         if (entries > idx::CHAIN_LIST_MAX) return false;

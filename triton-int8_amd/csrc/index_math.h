@@ -138,6 +138,8 @@ TI8_HD int chain_walked(int nk) { return (nk + 1) & ~1; }
 TI8_HD int chain_tile_of_round(int base, int grid, int total, int w, bool several) {
     return several && base + grid > total ? base + grid - 1 - w : base + w;
 }
+// cost of a tile: its K tiles, and about two and a half more for its end
+TI8_HD int chain_tile_cost(int nk) { return 2 * chain_walked(nk) + 5; }
 // cost of the busiest of `grid` workgroups that take tiles by rounds (chain_tile_of_round), a tile of GEMM i costing cost[i]: the load changes
 // only where a GEMM begins, so those workgroups are looked at
 TI8_HD int64_t chain_rounds_busiest(const int64_t* tiles, const int64_t* cost, int count, int grid) {
@@ -162,7 +164,7 @@ TI8_HD int64_t chain_rounds_busiest(const int64_t* tiles, const int64_t* cost, i
 // neighbours in its L2 they then stay, and entry v is tile 8 v + x of the launch, GEMM i having the tiles from 8 (n[0] + .. + n[i - 1]) on.
 // cost[i] descending.  tile[first[s]] .. tile[first[s + 1] - 1]: what workgroup s takes.  Returns the cost of the busiest.
 constexpr int CHAIN_LIST_SLOTS = 32, CHAIN_LIST_MAX = 480;
-inline int chain_list(const int* n, const int* cost, int count, int slots, int* first, uint16_t* tile) {
+TI8_HD int chain_list(const int* n, const int* cost, int count, int slots, int* first, uint16_t* tile) {
     int free_at[CHAIN_LIST_SLOTS] = {}, slot_of[CHAIN_LIST_SLOTS];      // workgroups by the time at which they are free
     for (int s = 0; s < slots; ++s) slot_of[s] = s;
     uint8_t taken_by[CHAIN_LIST_MAX];
@@ -508,7 +510,8 @@ TI8_HD double gemm_set_time_small(const GemmSet& s, bool i32, int num_cu) {
     const double t = i32 ? 5.0 + 0.28 * longest + 0.71 * mean + 2.9 * tiles / slots : 6.3 + 0.37 * longest + 0.96 * mean + 1.84 * tiles / slots;
     return t > alone ? t : alone;
 }
-// 256 x 256 tiles, by rounds
+// 256 x 256 tiles, by rounds; the persistent kernel by lists where that is less (measured / predicted, us: the GEMMs of a step, 1024 tokens,
+// 4096 -> 11008 156 / 161, 1280, 3200 -> 6528 101 / 101, 1536, 2048 -> 5632 81 / 79; on four waves 165, 112, 90)
 TI8_HD double gemm_set_time_large(const GemmSet& s, bool i32, int num_cu) {
     int64_t tiles[3], total = 0;
     double work = 0;
@@ -522,7 +525,18 @@ TI8_HD double gemm_set_time_large(const GemmSet& s, bool i32, int num_cu) {
     // a GEMM over few K tiles of an odd number keeps the launch off the persistent kernel
     bool odd = false;
     for (int i = 0; i < s.count; ++i) odd = odd || !chain_takes((int)s.nk[i], false);
-    return (7.7 + 1.15 * longest + 0.9 * mean + 0.4 * (double)rounds) * (odd ? 1.04 : 1.0);
+    const double by_rounds = (7.7 + 1.15 * longest + 0.9 * mean + 0.4 * (double)rounds) * (odd ? 1.04 : 1.0);
+    if (odd || s.count < 2 || num_cu % 8 || num_cu / 8 > CHAIN_LIST_SLOTS || total > 8 * (CHAIN_LIST_MAX - s.count)) return by_rounds;
+    int n[3], cost[3], first[CHAIN_LIST_SLOTS + 1];
+    uint16_t order[CHAIN_LIST_MAX];
+    double walked = 0;
+    for (int i = 0; i < s.count; ++i) {
+        n[i] = (int)((tiles[i] + 7) / 8);
+        cost[i] = chain_tile_cost((int)s.nk[i]);
+        walked += (double)(tiles[i] * chain_walked((int)s.nk[i])) / num_cu;
+    }
+    const double by_list = 7.7 + 0.546 * (double)(chain_list(n, cost, s.count, num_cu / 8, first, order) - 3) + 0.9 * walked;
+    return by_list < by_rounds ? by_list : by_rounds;
 }
 // the medium-size kernel, one workgroup per CU: past one round a workgroup's turn-over is not hidden
 TI8_HD double gemm_set_time_mid(const GemmSet& s, bool i32, int num_cu) {
