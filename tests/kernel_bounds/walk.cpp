@@ -1046,6 +1046,18 @@ void walk_configs_together(const int64_t* shape, int count, int i32, int num_cu,
 // Workgroup -> (GEMM, tile) map of a several-GEMM launch (gemm.hip: gemm_i8_multi_kernel, launch_multi):
 // tiles[i] = workgroups of GEMM i.  Every workgroup of the grid must land in a GEMM i < count with
 // a tile index in [0, tiles[i]), and every (GEMM, tile) must be taken exactly once.
+// Column sums in one launch (bias.hip): every strip of columns belongs to one workgroup
+int walk_column_strips(int strips, int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    std::vector<int> seen((size_t)strips, 0);
+    for (int w = 0; w < strips && !r.bad; ++w, ++r.checked) {
+        const int s = column_strip(w, strips);
+        if (s < 0 || s >= strips || seen[(size_t)s]++) r.fail("column strips: workgroup %d takes strip %d of %d", w, s, strips);
+    }
+    *n_checked = r.checked;
+    return r.bad;
+}
+
 // Lists of the persistent chained kernel: every tile of every GEMM is on one workgroup's list of one XCD, each list in the order of the
 // launch, no workgroup busier than another by more than a tile that it could have left to it
 int walk_chain_list(const int* tiles, const int* cost, int count, int slots, int64_t* n_checked, char* msg, int msglen) {

@@ -73,6 +73,12 @@ def test_column_sum(T, dev, rows, cols):
     assert T.ops.column_sum(torch.full((rows, cols), float("inf"), dtype=torch.bfloat16, device=dev)).isinf().all()
 
 
+# the last rows and columns that one launch takes, and the first that two take
+@pytest.mark.parametrize("rows,cols", [(255, 8192), (3072, 1056), (3073, 1056), (1024, 8224), (1025, 8224)])
+def test_column_sum_in_one_launch_and_in_two(T, dev, rows, cols):
+    test_column_sum(T, dev, rows, cols)
+
+
 def test_bias_gradient_can_be_differentiated_again(T, dev):
     lin = T.Int8Linear(256, 128, bias=True, device=dev)
     x, dy = torch.randn(5, 256, device=dev).bfloat16(), torch.ones(5, 128, device=dev).bfloat16().requires_grad_(True)

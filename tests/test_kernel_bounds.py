@@ -45,6 +45,7 @@ def walker(tmp_path_factory):
     lib.walk_quant_row_form.argtypes = [i64] * 4 + [ci, ci] + [i64] * 3 + [ctypes.POINTER(ci), p64, cp, ci]
     lib.walk_maxima.argtypes = [i64] * 6 + [p64, cp, ci]
     lib.walk_quant_call.argtypes = [p64, p64, ci, ci, ci, p64, cp, ci]
+    lib.walk_column_strips.argtypes = [ci, p64, cp, ci]
     lib.walk_chain_list.argtypes = [ctypes.POINTER(ci), ctypes.POINTER(ci), ci, ci, p64, cp, ci]
     lib.walk_gemm_tile_map.argtypes = [ci, ci, ci, p64, cp, ci]
     lib.walk_decode_narrow.argtypes = [ci] + [i64] * 8 + [p64, cp, ci]
@@ -471,6 +472,12 @@ def test_one_call_step_reads_no_more_rows_than_there_are(recorded, rows, tokens)
     assert not calls
     T.ops.linear_step(X, W, dY, "block_channel", tokens=rows)
     assert calls[0][1][12] == -(-rows // 128) * 128 and calls[0][1][13] == rows
+
+
+@pytest.mark.parametrize("strips", [1, 15, 16, 17, 33, 176])
+def test_column_strips(walker, strips):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    assert walker.walk_column_strips(strips, ctypes.byref(n), msg, 512) == 0, msg.value.decode()
 
 
 # fewer tiles than workgroups, one each, a remainder of 8, most of the work in the longest or in the shortest, as many entries as a list has,

@@ -1,6 +1,7 @@
 // The bias of a linear layer: adding it behind the GEMMs of a whole step (a GEMM launched alone does that in its epilogue), and its
 // gradient, the column sums of dY.
 #include "ti8_common.h"
+#include "index_math.h"
 
 namespace ti8 {
 
@@ -62,6 +63,46 @@ __global__ __launch_bounds__(THREADS) void column_partial_kernel(const uint16_t*
         make_float2((acc[0][c] + acc[1][c]) + (acc[2][c] + acc[3][c]), (acc[0][c + 1] + acc[1][c + 1]) + (acc[2][c + 1] + acc[3][c + 1]));
 }
 
+// The same in one launch where a workgroup can take all rows of 32 columns in the time that a second launch takes: 4 lanes to a row's 64 bytes,
+// 256 rows at a time, whose sums meet across the lanes of a wave and then of the 16 waves, in a fixed order.  Strips that share cache
+// lines go to one XCD.  idx::column_sum_narrow says where, with the figures.
+constexpr int NARROW_COLS = 32, NARROW_THREADS = 1024;
+__global__ __launch_bounds__(NARROW_THREADS) void column_sum_narrow_kernel(const uint16_t* __restrict__ x, int64_t ldx, int rows, int strips, uint16_t* __restrict__ out) {
+    __shared__ float acc[NARROW_THREADS / 64][NARROW_COLS];
+    const int strip = idx::column_strip((int)blockIdx.x, strips);
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const uint16_t* const p = x + strip * NARROW_COLS + (lane & 3) * 8;
+    float s[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) s[e] = 0.0f;
+#pragma unroll 8
+    for (int r = (int)threadIdx.x >> 2; r < rows; r += NARROW_THREADS / 4) {
+        const uint4 v = *reinterpret_cast<const uint4*>(p + (int64_t)r * ldx);
+        const uint32_t w[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            s[2 * e] += bf16_lo(w[e]);
+            s[2 * e + 1] += bf16_hi(w[e]);
+        }
+    }
+#pragma unroll
+    for (int m = 4; m < 64; m <<= 1)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s[e] += __shfl_xor(s[e], m, 64);
+    if (lane < 4)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) acc[wave][lane * 8 + e] = s[e];
+    __syncthreads();
+    if (threadIdx.x >= NARROW_COLS / 2) return;
+    float a = 0.0f, b = 0.0f;
+#pragma unroll
+    for (int w = 0; w < NARROW_THREADS / 64; ++w) {
+        a += acc[w][threadIdx.x * 2];
+        b += acc[w][threadIdx.x * 2 + 1];
+    }
+    *reinterpret_cast<uint32_t*>(out + strip * NARROW_COLS + threadIdx.x * 2) = pack_bf16x2(a, b);
+}
+
 int add_bias(void* y, int64_t ldy, const void* bias, int64_t rows, int64_t cols, ti8_stream_t stream) {
     const int chunks = (int)(cols / 8);
     for (int64_t r = 0; r < rows; r += 4 * 65535) {     // a launch has at most 65535 workgroup rows
@@ -101,6 +142,12 @@ extern "C" int ti8_column_sum(const void* x, int64_t ldx, void* out, void* works
     if (!column_sum_takes(rows, cols) || ldx < cols)
         return fail(TI8_ERR_SHAPE, "%s: need rows>0, cols a positive multiple of 32 and ldx>=cols; got rows=%lld cols=%lld ldx=%lld", fn, (long long)rows, (long long)cols, (long long)ldx);
     if (!aligned16(x) || ldx % 8 || !aligned16(out) || !aligned16(workspace)) return fail(TI8_ERR_ALIGN, "%s: x, out and the workspace must be 16-byte aligned, ldx a multiple of 8", fn);
+    if (idx::column_sum_narrow(rows, cols)) {
+        const int strips = (int)(cols / NARROW_COLS);
+        hipLaunchKernelGGL(column_sum_narrow_kernel, dim3((unsigned)strips), dim3(NARROW_THREADS), 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(x), ldx,
+                           (int)rows, strips, static_cast<uint16_t*>(out));
+        return check_launch(fn);
+    }
     const int64_t per = rows_per_group(rows, cols);
     const int groups = (int)((rows + per - 1) / per);
     float* const partial = static_cast<float*>(workspace);

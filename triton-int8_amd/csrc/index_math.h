@@ -386,6 +386,16 @@ TI8_HD int64_t thin_workers(int64_t M, int64_t N, int64_t num_cu) {
     return tiles < num_cu ? tiles : num_cu;
 }
 
+// ---- column sums (bias.hip) -----------------------------------------------------------------------
+// Workgroup -> strip of 32 columns of column_sum_narrow_kernel: two neighbours, which share cache lines, on one XCD
+TI8_HD int column_strip(int block, int strips) {
+    const int group = block & ~15;
+    return group + 16 <= strips ? group + (block & 7) * 2 + ((block >> 3) & 1) : block;
+}
+// Whether that kernel makes the sums in its one launch.  us in a graph, two launches / one: 16 x 4096 4.5 / 3.3, 512 x 14336 6.1 / 5.6,
+// 1500 x 5632 6.2 / 4.7, 3000 x 5632 8.4 / 7.4, 3000 x 1024 5.2 / 5.0; 4096 x 5632 11.3 / 12.0, 1500 x 14336 11.0 / 11.5, 16384 x 4096 25.5 / 35.1.
+TI8_HD bool column_sum_narrow(int64_t rows, int64_t cols) { return rows <= (cols <= 8192 ? 3072 : 1024); }
+
 // ---- attention's backward (attention.hip) ---------------------------------------------------------
 // Workgroup -> (batch, head) pair and block of its rows: the blocks of a pair on one XCD, whose L2 then serves the rows that they all
 // stream.  The grid has round8(pairs) * blocks workgroups; those of a pair beyond the last do nothing.
