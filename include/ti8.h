@@ -436,6 +436,13 @@ int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, in
  * ti8_gemm_i8_nt_multi (TI8_PART_FORWARD alone: ti8_gemm_i8_nt, the same kernel), else each takes the kernel of ti8_gemm_i8_nt
  * (those on the few-rows kernel in one launch; up to 8 unrotated rows may be quantised inside it), Y and dX for the first ceil(tokens / 32) * 32 rows only. */
 int ti8_linear(const ti8_linear_args* a, ti8_stream_t stream);
+/* 2 or 3 layers that multiply the same X (the projections of an attention, gate and up of an MLP), block-channel without rotation or
+ * bias: the forward of all (TI8_PART_FORWARD | TI8_PART_KEEP) or their backward (TI8_PART_BACKWARD | TI8_PART_KEEP), with X quantised once.
+ * Y and dW of each layer have the bits of ti8_linear; the first layer's dX is the sum of the layers' dX, bf16 sums from the last layer to the
+ * first (those that autograd makes of separate calls), the others' dX is not looked at.  `saved` and the workspace of the call are the first
+ * layer's.  parts, X, tokens, K and gemm_flags are those of all; N, W, dY, Y and dW the layer's own, outputs that share no memory. */
+int64_t ti8_linear_group_workspace(const ti8_linear_args* a, int count, int64_t* saved_bytes);
+int ti8_linear_group(const ti8_linear_args* a, int count, ti8_stream_t stream);
 /* Column sums of x bf16 [rows][cols] (ldx), added up in fp32 and rounded once: the gradient of a bias.  cols a multiple of 32;
  * workspace: ti8_column_sum_workspace bytes (-1 for sizes it does not take), 16-byte aligned. */
 int64_t ti8_column_sum_workspace(int64_t rows, int64_t cols);

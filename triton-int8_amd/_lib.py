@@ -70,6 +70,7 @@ PROTOTYPES = {
     "ti8_gemm_i8_nt_i32": [_vp, _i64, _i64, _vp, _i64, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _i64, _vp],
     "ti8_linear_fwd_bwd": [_vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _vp, _i64, _i64, _i64, _i64, _i64, _int, _int, _vp, _i64, _vp],
     "ti8_linear": [ctypes.POINTER(LinearArgs), _vp],
+    "ti8_linear_group": [ctypes.POINTER(LinearArgs), _int, _vp],
     "ti8_column_sum": [_vp, _i64, _vp, _vp, _i64, _i64, _vp],
     "ti8_linear_quantise": [ctypes.POINTER(LinearArgs), ctypes.POINTER(GemmProblem), ctypes.POINTER(_int), _vp],
     "ti8_rmsnorm": [_vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp],
@@ -80,7 +81,7 @@ PROTOTYPES = {
     "ti8_attention_bwd": [ctypes.POINTER(AttentionArgs), _vp],
     "ti8_probe_mfma": [_vp, _i64, _vp, _int, _int, _int, _int, _vp],
 }
-EXPORTS = ["ti8_version", "ti8_last_error", "ti8_arch", "ti8_init", "ti8_last_gemm_kernel", "ti8_linear_fwd_bwd_workspace", "ti8_linear_workspace",
+EXPORTS = ["ti8_version", "ti8_last_error", "ti8_arch", "ti8_init", "ti8_last_gemm_kernel", "ti8_linear_fwd_bwd_workspace", "ti8_linear_workspace", "ti8_linear_group_workspace",
            "ti8_rmsnorm_bwd_workspace", "ti8_column_sum_workspace", "ti8_attention_bwd_workspace"] + list(PROTOTYPES)
 
 # enums of include/ti8.h
@@ -126,6 +127,8 @@ def lib():
         l.ti8_linear_fwd_bwd_workspace.argtypes = [_i64, _i64, _i64, _int]
         l.ti8_linear_workspace.restype = _i64
         l.ti8_linear_workspace.argtypes = [ctypes.POINTER(LinearArgs), ctypes.POINTER(_i64)]
+        l.ti8_linear_group_workspace.restype = _i64
+        l.ti8_linear_group_workspace.argtypes = [ctypes.POINTER(LinearArgs), _int, ctypes.POINTER(_i64)]
         l.ti8_rmsnorm_bwd_workspace.restype = _i64
         l.ti8_rmsnorm_bwd_workspace.argtypes = [_i64, _i64]
         l.ti8_attention_bwd_workspace.restype = _i64

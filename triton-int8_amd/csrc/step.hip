@@ -29,6 +29,8 @@ struct Layer {
     bool fwd, bwd, keep;
     // a whole step whose workspace has no room for partial maxima (ti8_linear_fwd_bwd): they live in its outputs, see `quantise`
     bool partials_in_outputs = false;
+    // layers that multiply the same X (ti8_linear_group): the one that quantises it (null: this one)
+    const Layer* input_of = nullptr;
     // operands of Y = X W^T, dX = dY W, dW = dY^T X and their scales
     int8_t *xq, *wq, *dq, *wtq, *dytq, *xtq;
     float *xs, *ws, *ds, *wts, *dyts, *xts;
@@ -71,14 +73,14 @@ struct Layer {
         // row-block W^T and its grid; double-channel X^T and W^T by rows
         const bool shared = shares();
         if (shared) {
-            if (!row_block()) xtq = k.take<int8_t>(T * K);
+            if (!row_block()) xtq = input_of ? input_of->xtq : k.take<int8_t>(T * K);
             wtq = k.take<int8_t>(N * K);
-            if (block()) { xs = k.take<float>(gt * gk); wts = k.take<float>(K); }
+            if (block()) { xs = input_of ? input_of->xs : k.take<float>(gt * gk); wts = k.take<float>(K); }
             if (row_block()) ws = k.take<float>(gn * gk);
             if (dbl()) { xts = k.take<float>(K); wts = k.take<float>(K); }
         }
         if (fwd) {
-            xq = w.take<int8_t>(T * K);
+            xq = input_of ? input_of->xq : w.take<int8_t>(T * K);
             if (!xs) xs = w.take<float>(block() ? gt * gk : T);
             if (given_w()) {
                 wq = const_cast<int8_t*>(a->wq);
@@ -217,8 +219,25 @@ int64_t next_pow2(int64_t v) {
     return n;
 }
 
-// Enqueue the quantisers of a call and describe its GEMMs.  The order is that of linear_forward + linear_backward in the Python layer.
-int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stream_t stream) {
+// Operands that go into the two quantiser launches of a call: without a rotation, those quantised by blocks and those quantised by rows and by
+// columns, without a launch that only clears maxima (quant_call: 16 tokens, 4096 -> 4096, block-channel 41 -> 37.6 us; 3072 tokens
+// row-block 210 -> 204)
+struct Operands {
+    ti8_qblock_operand by_block[4];
+    int64_t by_block_rows[4];
+    QRowColOperand both[3];
+    int nblocks = 0, nboth = 0;
+    QRowOperand rows;
+    bool by_rows = false;
+};
+int quantise_operands(const char* fn, const Layer& L, const Operands& o, ti8_stream_t stream) {
+    return quant_call(fn, o.by_block, o.by_block_rows, o.nblocks, o.both, o.nboth, o.by_rows ? &o.rows : nullptr, TI8_Q_CLAMP,
+                      L.dbl() ? TI8_INV_AMAX_DIV_127 : TI8_INV_RCP_OF_SCALE, stream);
+}
+
+// Enqueue the quantisers of a call but for those that are added to `o`, and describe its GEMMs.  The order is that of linear_forward +
+// linear_backward in the Python layer.
+int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* count, ti8_stream_t stream) {
     const ti8_linear_args& a = *L.a;
     const int64_t T = L.T, K = L.K, N = L.N, tok = L.tokens;
     const int q = TI8_Q_CLAMP, had = L.had == 128 ? TI8_Q_HAD128 : 0;
@@ -230,15 +249,6 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
         mx += Layer::maxima_piece(words);
         return reinterpret_cast<float*>(p);
     };
-    // Without a rotation, the operands quantised by blocks and those quantised by rows and by columns are collected and go into two
-    // launches for the call, without one that only clears maxima (quant_call: 16 tokens, 4096 -> 4096, block-channel 41 -> 37.6 us;
-    // 3072 tokens row-block 210 -> 204)
-    ti8_qblock_operand by_block[4];
-    int64_t by_block_rows[4];
-    QRowColOperand both[3];
-    int nblocks = 0, nboth = 0;
-    const QRowOperand x_rows = {a.X, a.ldx, L.xq, L.xs, tok, K};
-    const QRowOperand* by_rows = nullptr;
     // (`out`, `ldout`: the output of the operand's own shape, which a whole step does not write before its GEMMs; with
     // partials_in_outputs the partial maxima live there until the conversion has read them, unless the caller's tensors overlap)
     const bool apart = L.partials_in_outputs && step_apart(a, T);
@@ -247,11 +257,11 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
         unsigned int* partial = nullptr;
         if (L.partial_words(R, C)) partial = reinterpret_cast<unsigned int*>(take_maxima(quant_maxima_words(R, C)));
         else if (apart && ldout == C) partial = static_cast<unsigned int*>(out);
-        both[nboth++] = QRowColOperand{x, ldx, oq, os, oqT, osT, scratch, partial, R, valid, C};
+        o.both[o.nboth++] = QRowColOperand{x, ldx, oq, os, oqT, osT, scratch, partial, R, valid, C};
     };
-    auto block = [&](const ti8_qblock_operand& o, int64_t valid) {
-        by_block_rows[nblocks] = valid;
-        by_block[nblocks++] = o;
+    auto block = [&](const ti8_qblock_operand& operand, int64_t valid) {
+        o.by_block_rows[o.nblocks] = valid;
+        o.by_block[o.nblocks++] = operand;
     };
     auto blocks = [&](const void* x, int64_t ldx, int8_t* oq, int8_t* oqT, float* os, int64_t R, int64_t C) {
         return ti8_qblock_operand{x, 0, ldx, oq, R * C, C, oqT, R * C, R, os, 0, C / 128, 1, 1, R, C};
@@ -265,7 +275,7 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
             if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xq, T * K, K, L.xs, 0, K / 128, 1, 1, T, tok, K, 0, q, inv, stream)) return e;
             if (!L.given_w()) if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q | had, inv, stream)) return e;
         } else if (L.block()) {
-            block(blocks(a.X, a.ldx, L.xq, shared ? L.xtq : nullptr, L.xs, T, K), tok);
+            if (!L.input_of) block(blocks(a.X, a.ldx, L.xq, shared ? L.xtq : nullptr, L.xs, T, K), tok);
             if (shared) row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K, a.dW, a.lddw);     // rows for Y, columns for dX
             else if (!L.given_w())
                 if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q, inv, stream)) return e;
@@ -274,7 +284,8 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
                 if (int e = ti8_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, 0, q | had, inv, stream)) return e;
                 if (!L.given_w()) if (int e = ti8_quant_block_had128(a.W, 0, a.ldw, L.wq, N * K, K, L.ws, 0, K / 128, 1, 1, N, K, 0, q, inv, stream)) return e;
             } else {
-                by_rows = &x_rows;
+                o.rows = QRowOperand{a.X, a.ldx, L.xq, L.xs, tok, K};
+                o.by_rows = true;
                 if (!L.given_w()) block(blocks(a.W, a.ldw, L.wq, shared ? L.wtq : nullptr, L.ws, N, K), N);
             }
         } else if (L.had) {
@@ -341,7 +352,7 @@ int quantise(const char* fn, Layer& L, ti8_gemm_problem* g, int* count, ti8_stre
         g[n++] = gemm2d(L.dytq, L.dyts, dyt_mode, dyts_rs, dyts_ks, L.xtq, L.xts, xt_mode, xts_rs, xts_ks, a.dW, a.lddw, N, K, T, L.dbl(), rot, post_dw);
     }
     *count = n;
-    return quant_call(fn, by_block, by_block_rows, nblocks, both, nboth, by_rows, q, inv, stream);
+    return TI8_OK;
 }
 
 int gemms(const Layer& L, const ti8_gemm_problem* g, int count, ti8_stream_t stream) {
@@ -406,13 +417,116 @@ int run_layer(const char* fn, const ti8_linear_args* a, int64_t T, ti8_gemm_prob
     }
     ti8_gemm_problem g[3];
     int n = 0;
-    if (int e = quantise(fn, L, g, &n, stream)) return e;
+    Operands operands;
+    if (int e = quantise(fn, L, operands, g, &n, stream)) return e;
+    if (int e = quantise_operands(fn, L, operands, stream)) return e;
     if (problems) {
         for (int i = 0; i < n; ++i) problems[i] = g[i];
         *count = n;
         return TI8_OK;
     }
     return gemms(L, g, n, stream);
+}
+
+// ---- layers on the same X ----------------------------------------------------------------
+// The seven linears of a decoder layer are three calls of this kind (q, k, v; gate, up) and two alone: X is quantised once for a
+// call, the weights' (the dYs') quantisers are two launches (one) for all of it and the GEMMs one (two).  The whole layer, us apart
+// / so: 3 x 1360 tokens, hidden 2048, MLP 4992 1768 / 1609; 4 x 4096, hidden 4096, MLP 14336 18530 / 18170.
+constexpr int GROUP_MAX = 3;
+struct Group {
+    Layer L[GROUP_MAX];
+    int count;
+    void* dx[GROUP_MAX];        // backward: dX of each layer, [T][K] but for the first, which is the sum's own place
+
+    // As Layer::carve, of the whole call
+    int64_t carve(char* ws_base, char* saved_base, int64_t* saved_bytes) {
+        int64_t used = 0, kept = 0;
+        for (int i = 0; i < count; ++i) {
+            int64_t k = 0;
+            L[i].input_of = i ? &L[0] : nullptr;
+            used += L[i].carve(ws_base + used, saved_base + kept, &k);
+            kept += k;
+        }
+        for (int i = 1; i < count && L[0].bwd; ++i) {
+            dx[i] = ws_base + used;
+            used += (L[0].T * L[0].K * 2 + 255) / 256 * 256;
+        }
+        *saved_bytes = kept;
+        return used;
+    }
+    int64_t size(int64_t* saved_bytes) {
+        char* const nowhere = reinterpret_cast<char*>(256);
+        return carve(nowhere, nowhere, saved_bytes);
+    }
+};
+
+int check_group(const char* fn, const ti8_linear_args* a, int count, Group* g) {
+    if (count < 2 || count > GROUP_MAX) return fail(TI8_ERR_SHAPE, "%s: between 2 and %d layers, got %d", fn, GROUP_MAX, count);
+    g->count = count;
+    for (int i = 0; i < count; ++i) {
+        if (int e = check_layer(fn, a + i, (a[i].tokens + 127) / 128 * 128, &g->L[i])) return e;
+        if (a[i].scheme != TI8_SCHEME_BLOCK_CHANNEL || a[i].hadamard || !g->L[i].keep || a[i].wq || a[i].bias)
+            return fail(TI8_ERR_MODE, "%s: block-channel layers without rotation or bias, forward or backward with TI8_PART_KEEP", fn);
+        if (a[i].parts != a[0].parts || a[i].tokens != a[0].tokens || a[i].K != a[0].K || a[i].X != a[0].X || a[i].ldx != a[0].ldx || a[i].gemm_flags != a[0].gemm_flags)
+            return fail(TI8_ERR_SHAPE, "%s: the layers must have parts, X, tokens, K and gemm_flags in common", fn);
+    }
+    return TI8_OK;
+}
+
+int run_group(const char* fn, const ti8_linear_args* given, int count, ti8_stream_t stream) {
+    Group G;
+    if (int e = check_group(fn, given, count, &G)) return e;
+    const ti8_linear_args& first = given[0];
+    int64_t need_saved = 0;
+    const int64_t need = G.size(&need_saved);
+    if (!first.workspace || (reinterpret_cast<uintptr_t>(first.workspace) & 255) || first.workspace_bytes < need || !first.saved ||
+        (reinterpret_cast<uintptr_t>(first.saved) & 255) || first.saved_bytes < need_saved)
+        return fail(TI8_ERR_SHAPE, "%s: the first layer's workspace and `saved` must be 256-byte aligned and hold %lld and %lld bytes (ti8_linear_group_workspace)",
+                    fn, (long long)need, (long long)need_saved);
+    G.carve(static_cast<char*>(first.workspace), static_cast<char*>(first.saved), &need_saved);
+    const bool fwd = G.L[0].fwd;
+    const int64_t T = G.L[0].T, K = G.L[0].K;
+    ti8_linear_args a[GROUP_MAX];
+    Rows out[2 * GROUP_MAX];
+    int outs = 0;
+    for (int i = 0; i < count; ++i) {
+        a[i] = given[i];
+        if (!fwd && i) {
+            a[i].dX = G.dx[i];
+            a[i].lddx = K;
+        }
+        G.L[i].a = &a[i];
+        if (int e = check_pointers(fn, &a[i], G.L[i])) return e;
+        if (fwd) out[outs++] = matrix(a[i].Y, T, a[i].ldy, a[i].N);
+        else out[outs++] = matrix(a[i].dW, a[i].N, a[i].lddw, K);
+    }
+    if (!fwd) out[outs++] = matrix(first.dX, T, first.lddx, K);
+    for (int i = 0; i < outs; ++i)
+        for (int j = 0; j < i; ++j)
+            if (!out[i].apart(out[j])) return fail(TI8_ERR_SHAPE, "%s: the outputs of the layers must not share memory", fn);
+
+    ti8_gemm_problem g[GROUP_MAX][3], by_kind[3][GROUP_MAX];
+    Operands operands;
+    int n = 0;
+    for (int i = 0; i < count; ++i) {
+        if (int e = quantise(fn, G.L[i], operands, g[i], &n, stream)) return e;
+        for (int k = 0; k < n; ++k) by_kind[k][i] = g[i][k];
+    }
+    if (int e = quantise_operands(fn, G.L[0], operands, stream)) return e;
+    bool large = T > 256;       // (as for one layer: none of them on the few-rows kernel)
+    for (int i = 0; i < count && !fwd; ++i) large = large && a[i].N > 256;
+    if (large) {
+        for (int k = 0; k < n; ++k)
+            if (int e = ti8_gemm_i8_nt_multi(by_kind[k], count, first.gemm_flags | TI8_GEMM_TOGETHER, stream)) return e;
+    } else if (fwd) {
+        if (int e = gemms(G.L[0], by_kind[0], count, stream)) return e;
+    } else {
+        for (int i = 0; i < count; ++i)
+            if (int e = gemms(G.L[i], g[i], n, stream)) return e;
+    }
+    if (fwd) return TI8_OK;
+    // in the order in which autograd adds up the gradients of layers that were called one after the other
+    return add_rows(fn, first.dX, first.lddx, G.dx[1], count > 2 ? G.dx[2] : nullptr, G.L[0].tokens, K, stream);
 }
 
 }  // namespace
@@ -438,6 +552,19 @@ extern "C" int ti8_linear(const ti8_linear_args* a, ti8_stream_t stream) {
     const char* fn = "ti8_linear";
     if (!a) return fail(TI8_ERR_NULL, "%s: args is required", fn);
     return run_layer(fn, a, (a->tokens + 127) / 128 * 128, nullptr, nullptr, stream);
+}
+
+extern "C" int64_t ti8_linear_group_workspace(const ti8_linear_args* a, int count, int64_t* saved_bytes) {
+    if (!a || !saved_bytes || a->tokens < 1) return -1;
+    Group g;
+    if (check_group("ti8_linear_group_workspace", a, count, &g)) return -1;
+    return g.size(saved_bytes);
+}
+
+extern "C" int ti8_linear_group(const ti8_linear_args* a, int count, ti8_stream_t stream) {
+    const char* fn = "ti8_linear_group";
+    if (!a) return fail(TI8_ERR_NULL, "%s: args is required", fn);
+    return run_group(fn, a, count, stream);
 }
 
 // The whole step on a token dim that the caller has rounded up itself

@@ -108,6 +108,8 @@ int gemm_nt_few(const ti8_gemm_problem* problems, int count, bool backward, cons
 // Y of 1 to 8 rows of bf16 that the GEMM's kernel quantises itself (`p` describes what it would be with the quantiser apart); *done tells
 // whether it was launched
 int gemm_nt_decode(const ti8_gemm_problem& p, const void* X, int64_t ldx, int64_t rows, const void* bias, int gemm_flags, bool* done, ti8_stream_t stream);
+// y = bf16(bf16(c + b) + y) on [rows][cols], b and c dense; without c: bf16(b + y) (bias.hip)
+int add_rows(const char* fn, void* y, int64_t ldy, const void* b, const void* c, int64_t rows, int64_t cols, ti8_stream_t stream);
 int add_bias(void* y, int64_t ldy, const void* bias, int64_t rows, int64_t cols, ti8_stream_t stream);
 // out[c] = bf16(sum over g of partial[g][c]), dim a multiple of 32 (decoder.hip)
 int sum_partials(const char* fn, const float* partial, int groups, int64_t dim, void* out, hipStream_t st);

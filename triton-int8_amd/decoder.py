@@ -13,7 +13,7 @@ import torch
 import torch.nn.functional as F
 
 from . import ops
-from .linear import Int8Linear
+from .linear import Int8Linear, LinearGroupFunction, _one_group
 
 __all__ = ["DecoderLayer", "rope_tables"]
 
@@ -170,6 +170,13 @@ def _attention(q, k, v, scale):
     return F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=scale)
 
 
+def _projections(x, *layers):
+    """The layers' outputs for the same x."""
+    if _one_group(x, layers) and _kernels_take(x, *(m.weight for m in layers)):
+        return LinearGroupFunction.apply(x, *(m.weight for m in layers))
+    return tuple(m(x) for m in layers)
+
+
 class RMSNorm(torch.nn.Module):
     def __init__(self, dim, eps=1e-5, device=None, fused=False):
         super().__init__()
@@ -214,7 +221,7 @@ class DecoderLayer(torch.nn.Module):
         B, S, H = x.shape
         cos, sin = rope_tables(S, self.head_dim, x.device)
         h = self.input_norm(x)
-        q, k, v = (p(h).view(B, S, self.heads, self.head_dim) for p in (self.q_proj, self.k_proj, self.v_proj))
+        q, k, v = (t.view(B, S, self.heads, self.head_dim) for t in _projections(h, self.q_proj, self.k_proj, self.v_proj))
         rotate = _RopeFunction.apply if self.int8 and self.head_dim % 16 == 0 and _kernels_take(q, k, cos, sin) else _rope_pair
         q, k = rotate(q, k, cos, sin)
         q, k, v = (t.transpose(1, 2) for t in (q, k, v))
@@ -222,6 +229,6 @@ class DecoderLayer(torch.nn.Module):
         a = _attention(q, k, v, scale) if self.int8 else F.scaled_dot_product_attention(q, k, v, is_causal=True, scale=scale)
         x = x + self.o_proj(a.transpose(1, 2).reshape(B, S, H))
         h = self.post_norm(x)
-        gate, up = self.gate_proj(h), self.up_proj(h)
+        gate, up = _projections(h, self.gate_proj, self.up_proj)
         product = _SwiGLUFunction.apply if self.int8 and _kernels_take(gate, up) else _swiglu
         return x + self.down_proj(product(gate, up))

@@ -395,6 +395,41 @@ class Int8LinearFunction(torch.autograd.Function):
         return dx[:tokens].reshape(*dy.shape[:-1], x2.shape[1]), dw, db, None, None
 
 
+class LinearGroupFunction(torch.autograd.Function):
+    """The products of one x with 2 or 3 weights, block-channel without rotation: :class:`Int8LinearFunction` for each, with x quantised once and
+    the launches of all in one call per direction (``ti8_linear_group``).  Outputs and gradients have the bits of separate calls."""
+
+    @staticmethod
+    def forward(ctx, x, *weights):
+        x2 = x.reshape(-1, x.shape[-1])
+        ctx.save_for_backward(x2, *weights)
+        ys, ctx.saved_q = ops.linear_group_forward(x2, weights)
+        return tuple(y[:x2.shape[0]].reshape(*x.shape[:-1], y.shape[1]) for y in ys)
+
+    @staticmethod
+    def backward(ctx, *dys):
+        x2 = ctx.saved_tensors[0]       # (and the check that no weight has changed since)
+        tokens, K = x2.shape
+        dx, dws = ops.linear_group_backward([d.reshape(tokens, -1) for d in dys], K, ctx.saved_q)
+        return (dx[:tokens].reshape(*dys[0].shape[:-1], K), *dws)
+
+
+def _one_group(x, layers):
+    """Whether layers on the same x (a plain tensor) may run as one call: modules that do just what :class:`Int8Linear` does, in a forward
+    whose backward wants every gradient."""
+    if not (2 <= len(layers) <= 3 and torch.is_grad_enabled() and x.requires_grad and x.numel() and _from_c()) or torch.nn.modules.module._has_any_global_hook():
+        return False
+    for m in layers:
+        own = m.__dict__
+        if type(m) is not Int8Linear or "forward" in own or m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks:
+            return False
+        if m.scheme != "block_channel" or m.hadamard is not None or "weight" not in own["_parameters"] or m.bias is not None or not m.weight.requires_grad:
+            return False
+        if tuple(m.weight.shape) != (m.out_features, x.shape[-1]):
+            return False
+    return True
+
+
 class Int8Linear(torch.nn.Module):
     """``torch.nn.Linear`` whose three GEMMs (Y, dX, dW) run through the INT8 path.
     in_features and out_features must be multiples of 128; any number of tokens works

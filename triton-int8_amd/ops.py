@@ -560,6 +560,62 @@ def linear_call(parts, scheme, hadamard, tokens, K, N, *, X=None, W=None, dY=Non
     return Y, dX, dW, saved
 
 
+@functools.lru_cache(maxsize=256)
+def _group_sizes(tokens, K, features, parts):
+    """(bytes of workspace, bytes of saved) of a ``ti8_linear_group`` call."""
+    args = (_lib.LinearArgs * len(features))(*(_lib.LinearArgs(tokens=tokens, K=K, N=n, scheme=_lib.SCHEME_BLOCK_CHANNEL, parts=parts) for n in features))
+    saved = ctypes.c_int64(0)
+    n = _lib.lib().ti8_linear_group_workspace(args, len(features), ctypes.byref(saved))
+    _need(n >= 0, f"K and N must be positive multiples of 128 and the layers 2 or 3, got K={K} N={features}")
+    return n, saved.value
+
+
+def linear_group_forward(X, weights):
+    """Y of 2 or 3 layers on the same X bf16 [tokens, K] (``ti8_linear_group``, block-channel): ([Y [T, N] ..], saved), as :func:`linear_call`
+    with TI8_PART_KEEP gives them one by one."""
+    tokens, K = X.shape
+    T = -(-tokens // 128) * 128
+    parts = _lib.PART_FORWARD | _lib.PART_KEEP
+    features = tuple(w.shape[0] for w in weights)
+    need, need_saved = _group_sizes(tokens, K, features, parts)
+    for t in (X, *weights):
+        _check_bf16(t, "X and W")
+    X, weights = rows16(X), [rows16(w) for w in weights]
+    dev = X.device
+    Y = [torch.empty((T, n), dtype=torch.bfloat16, device=dev) for n in features]
+    saved, workspace = _workspace(need_saved, dev), _workspace(need, dev)
+    flags, x, ldx = _gemm_flags(), X.data_ptr(), X.stride(0)
+    args = (_lib.LinearArgs * len(features))(*(
+        _lib.LinearArgs(X=x, ldx=ldx, W=w.data_ptr(), ldw=w.stride(0), Y=y.data_ptr(), ldy=n, tokens=tokens, K=K, N=n, scheme=_lib.SCHEME_BLOCK_CHANNEL,
+                        parts=parts, gemm_flags=flags, workspace=workspace.data_ptr(), workspace_bytes=need, saved=saved.data_ptr(), saved_bytes=need_saved)
+        for w, y, n in zip(weights, Y, features)))
+    _lib.call("ti8_linear_group", args, len(features), _stream())
+    return Y, saved
+
+
+def linear_group_backward(dY, K, saved):
+    """(dX [T, K], [dW [N, K] ..]) of the layers whose forward left `saved`; dX is the sum of theirs, last layer first."""
+    tokens = dY[0].shape[0]
+    T = -(-tokens // 128) * 128
+    parts = _lib.PART_BACKWARD | _lib.PART_KEEP
+    features = tuple(d.shape[1] for d in dY)
+    need, need_saved = _group_sizes(tokens, K, features, parts)
+    for d in dY:
+        _check_bf16(d, "dY")
+    dY = [rows16(d) for d in dY]
+    dev = dY[0].device
+    dX = torch.empty((T, K), dtype=torch.bfloat16, device=dev)
+    dW = [torch.empty((n, K), dtype=torch.bfloat16, device=dev) for n in features]
+    workspace = _workspace(need, dev)
+    flags, x = _gemm_flags(), dX.data_ptr()
+    args = (_lib.LinearArgs * len(features))(*(
+        _lib.LinearArgs(dY=d.data_ptr(), lddy=d.stride(0), dX=x, lddx=K, dW=w.data_ptr(), lddw=K, tokens=tokens, K=K, N=n, scheme=_lib.SCHEME_BLOCK_CHANNEL,
+                        parts=parts, gemm_flags=flags, workspace=workspace.data_ptr(), workspace_bytes=need, saved=saved.data_ptr(), saved_bytes=need_saved)
+        for d, w, n in zip(dY, dW, features)))
+    _lib.call("ti8_linear_group", args, len(features), _stream())
+    return dX, dW
+
+
 def column_sum(x):
     """``x.sum(0)`` of a bf16 matrix, added up in fp32; columns a multiple of 32."""
     x = rows16(x)
