@@ -472,6 +472,8 @@ int ti8_rmsnorm(const void* x, const void* w, void* y, float* rstd, int64_t rows
 int64_t ti8_rmsnorm_bwd_workspace(int64_t rows, int64_t dim);
 int ti8_rmsnorm_bwd(const void* dy, const void* x, const void* w, const float* rstd, void* dx, void* dw, void* workspace,
                     int64_t rows, int64_t dim, ti8_stream_t stream);
+/* (tables of ti8_rope, bf16 [seq][(head_dim + 1) / 2]: cos and sin of position * base^(-2 j / head_dim)) */
+int ti8_rope_tables(void* cos_table, void* sin_table, int64_t seq, int64_t head_dim, float base, ti8_stream_t stream);
 int ti8_rope(const void* q, const void* k, void* out_q, void* out_k, const void* cos_table, const void* sin_table,
              int64_t tokens, int64_t seq, int64_t heads, int64_t head_dim, int backward, ti8_stream_t stream);
 int ti8_swiglu(const void* gate, const void* up, void* out, int64_t n, ti8_stream_t stream);

@@ -105,6 +105,13 @@ def test_decoder_layer_bits(D, dev, monkeypatch, batch, seq, hidden, heads, mlp)
         assert torch.equal(a, b), name
 
 
+# one position, the largest angles, head dims that are no power of two, an odd one, another base
+@pytest.mark.parametrize("seq,dim,base", [(1, 2, 10000.0), (5, 48, 10000.0), (777, 96, 10000.0), (4097, 128, 10000.0), (70001, 64, 10000.0), (300, 33, 500000.0)])
+def test_rope_tables_bits(D, dev, seq, dim, base):
+    for got, want in zip(D.rope_tables(seq, dim, dev, base), D._rope_tables(seq, dim, dev, base)):
+        assert got.shape == want.shape and torch.equal(got, want)
+
+
 @pytest.mark.parametrize("batch,seq,heads,dim", [(1, 1, 1, 16), (2, 5, 3, 48), (3, 128, 8, 64), (1, 77, 32, 128), (2, 9, 40, 256)])
 def test_rope_bits(D, dev, batch, seq, heads, dim):
     gen = torch.Generator(device=dev).manual_seed(seq)

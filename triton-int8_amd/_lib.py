@@ -75,6 +75,7 @@ PROTOTYPES = {
     "ti8_linear_quantise": [ctypes.POINTER(LinearArgs), ctypes.POINTER(GemmProblem), ctypes.POINTER(_int), _vp],
     "ti8_rmsnorm": [_vp, _vp, _vp, _vp, _i64, _i64, _f32, _vp],
     "ti8_rmsnorm_bwd": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _vp],
+    "ti8_rope_tables": [_vp, _vp, _i64, _i64, _f32, _vp],
     "ti8_rope": [_vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, _i64, _int, _vp],
     "ti8_swiglu": [_vp, _vp, _vp, _i64, _vp],
     "ti8_swiglu_bwd": [_vp, _vp, _vp, _vp, _vp, _i64, _vp],

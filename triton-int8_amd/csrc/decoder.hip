@@ -169,6 +169,18 @@ __global__ __launch_bounds__(1024) void column_sum_kernel(const float* __restric
     }
 }
 
+// cos and sin [seq][half] of position * base^(-2 j / head_dim), rounded to bf16 at the end, with the roundings of the torch expression
+// (decoder.rope_tables): one launch for its twelve, which the host took 52 us to launch (8 now).
+__global__ __launch_bounds__(THREADS) void rope_tables_kernel(uint16_t* __restrict__ cosv, uint16_t* __restrict__ sinv, int64_t items, int half, float inv_dim, float base) {
+    const int64_t i = (int64_t)blockIdx.x * THREADS + threadIdx.x;
+    if (i >= items) return;
+    const int64_t pos = i / half;
+    const int j = (int)(i - pos * half);
+    const float angle = (float)pos * (1.0f / powf(base, (float)(2 * j) * inv_dim));
+    cosv[i] = (uint16_t)f32_to_bf16_bits(cosf(angle));
+    sinv[i] = (uint16_t)f32_to_bf16_bits(sinf(angle));
+}
+
 // Rotary embedding of q and k [tokens][heads * D], the two halves of a head's D elements rotated against each other by the
 // angle of (position, element); position = token % seq.  One workgroup per token; a thread takes 8 elements of each half.
 // 16384 x 4096, q and k together: 83 us (6.4 TB/s), about 700 us in 12 launches before.
@@ -324,6 +336,17 @@ extern "C" int ti8_rope(const void* q, const void* k, void* out_q, void* out_k, 
     hipLaunchKernelGGL(rope_kernel, dim3((unsigned)tokens, 2), dim3(THREADS), 0, static_cast<hipStream_t>(stream), static_cast<const uint16_t*>(q),
                        static_cast<const uint16_t*>(k), static_cast<uint16_t*>(out_q), static_cast<uint16_t*>(out_k), static_cast<const uint16_t*>(cos_table),
                        static_cast<const uint16_t*>(sin_table), (int)seq, (int)heads, (int)(head_dim / 2), backward ? -1.0f : 1.0f);
+    return check_launch(fn);
+}
+
+extern "C" int ti8_rope_tables(void* cos_table, void* sin_table, int64_t seq, int64_t head_dim, float base, ti8_stream_t stream) {
+    const char* fn = "ti8_rope_tables";
+    if (!cos_table || !sin_table) return fail(TI8_ERR_NULL, "%s: both tables are required", fn);
+    const int64_t half = (head_dim + 1) / 2, items = seq * half;
+    if (seq <= 0 || seq > 0x3fffffff || head_dim <= 0 || head_dim > 0x00ffffff || (items + THREADS - 1) / THREADS > 0x7fffffff)
+        return fail(TI8_ERR_SHAPE, "%s: need 0<seq<2^30 and 0<head_dim<2^24; got seq=%lld head_dim=%lld", fn, (long long)seq, (long long)head_dim);
+    hipLaunchKernelGGL(rope_tables_kernel, dim3((unsigned)((items + THREADS - 1) / THREADS)), dim3(THREADS), 0, static_cast<hipStream_t>(stream),
+                       static_cast<uint16_t*>(cos_table), static_cast<uint16_t*>(sin_table), items, (int)half, 1.0f / (float)head_dim, base);
     return check_launch(fn);
 }
 

@@ -19,6 +19,14 @@ __all__ = ["DecoderLayer", "rope_tables"]
 
 
 def rope_tables(seq_len, head_dim, device, base=10000.0):
+    device = torch.device(device)
+    if (device.type == "cuda" and device.index in (None, torch._C._cuda_getDevice()) and type(base) is float and type(seq_len) is int and seq_len > 0
+            and type(head_dim) is int and head_dim > 0 and _untraced()):
+        return ops.rope_tables(seq_len, head_dim, device, base)
+    return _rope_tables(seq_len, head_dim, device, base)
+
+
+def _rope_tables(seq_len, head_dim, device, base=10000.0):
     inv = 1.0 / (base ** (torch.arange(0, head_dim, 2, device=device, dtype=torch.float32) / head_dim))
     ang = torch.outer(torch.arange(seq_len, device=device, dtype=torch.float32), inv)
     return ang.cos().to(torch.bfloat16), ang.sin().to(torch.bfloat16)
@@ -46,14 +54,15 @@ def _swiglu(gate, up):
     return F.silu(gate) * up
 
 
+def _untraced():
+    """Whether this runs outside tracing and function transforms (to which a kernel launch is invisible)."""
+    return not (torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._functorch.peek_interpreter_stack() is not None
+                or torch.autograd.forward_ad._current_level >= 0 or torch.utils._python_dispatch._get_current_dispatch_mode() is not None)
+
+
 def _plain(*tensors):
-    """Whether these are plain bf16 tensors on the current device, outside tracing and function transforms (to which a kernel launch is
-    invisible)."""
-    if torch.compiler.is_compiling() or torch._C._get_tracing_state() is not None or torch._C._functorch.peek_interpreter_stack() is not None:
-        return False
-    if torch.autograd.forward_ad._current_level >= 0 or torch.utils._python_dispatch._get_current_dispatch_mode() is not None:
-        return False
-    return all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.bfloat16 and t.numel() > 0
+    """Whether these are plain bf16 tensors on the current device, and nothing traces what is done with them."""
+    return _untraced() and all(type(t) in (torch.Tensor, torch.nn.Parameter) and t.is_cuda and t.dtype == torch.bfloat16 and t.numel() > 0
                and t.device.index == torch._C._cuda_getDevice() for t in tensors)
 
 

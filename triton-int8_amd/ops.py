@@ -690,6 +690,13 @@ def rmsnorm_backward(dy, x, weight, rstd):
     return dx, dw
 
 
+def rope_tables(seq_len, head_dim, device, base):
+    """The two tables of :func:`rope`, bf16 [seq_len, (head_dim + 1) // 2] on the current device."""
+    cos, sin = (torch.empty((seq_len, (head_dim + 1) // 2), dtype=torch.bfloat16, device=device) for _ in range(2))
+    _lib.call("ti8_rope_tables", cos.data_ptr(), sin.data_ptr(), seq_len, head_dim, base, _stream())
+    return cos, sin
+
+
 def rope(q, k, cos, sin, backward=False):
     """q and k [batch, seq, heads, head_dim] (contiguous bf16) rotated by the tables [seq, head_dim / 2], or rotated back."""
     B, S, H, D = q.shape
