@@ -377,6 +377,7 @@ int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count, int gemm_f
  *   scratch memory as well until the GEMMs write them (nothing beyond their rows and columns is touched).
  *   They may be the inputs' memory.  Outputs that share memory are written one after the other, Y, dX, dW.
  *   gemm_flags: TI8_GEMM_TILED / TI8_GEMM_LARGE_TILES / TI8_GEMM_ONE_TILE or 0.
+ * A block-channel step on few tokens may quantise its weight inside the GEMMs instead.
  * Nothing is allocated; the call only enqueues kernels, so it may be captured into a graph. */
 enum ti8_scheme {
     TI8_SCHEME_BLOCK_CHANNEL = 0,

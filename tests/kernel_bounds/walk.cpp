@@ -534,6 +534,67 @@ int walk_decode_narrow(int rows, int64_t N, int64_t K, int64_t ldx, int64_t ldb,
     return r.bad;
 }
 
+// parts of a weight's maxima, the larger number of either direction
+int raw_weight_parts(int64_t R, int64_t C) {
+    const MaximaParts p = maxima_parts(R, C);
+    return p.nrt > p.nct ? p.nrt : p.nct;
+}
+
+// Y (cols = 0) or dX of a step on few tokens from the weight itself, W [R][C] (gemm_skinny.hip: raw_block): every element of the weight is read by one
+// lane, every K tile used by one wave of a workgroup against the codes of the same places, every element of the output [tokens] stored once
+int walk_raw_weight(int cols, int tokens, int64_t R, int64_t C, int64_t ldw, int64_t lda, int64_t ldc, int64_t w_elems, int64_t a_elems, int64_t c_elems,
+                    int64_t* n_checked, char* msg, int msglen) {
+    Report r{msg, msglen};
+    const int width = cols ? RAW_STRIP_DX : RAW_STRIP_Y, strips = (int)((cols ? C : R) / width), nk = (int)((cols ? R : C) >> 7), blocks = tokens > 16 ? 2 : 1;
+    const int64_t n = cols ? C : R;
+    std::vector<uint8_t> read((size_t)(R * C), 0), stored((size_t)(tokens * n), 0);
+    for (int block = 0; block < strips && !r.bad; ++block) {
+        const int n0 = (cols ? column_strip(block, strips) : block) * width;
+        for (int wave = 0; wave < 4; ++wave) {
+            const int kbeg = few_k_first(wave, nk), nq = few_k_first(wave + 1, nk) - kbeg, rot = decode_rot(n0, nq);
+            if (nq > 64) r.fail("raw weight: %d K tiles of a wave", nq);
+            for (int step = 0; step < nq; ++step) {
+                const int kt = few_k_tile(step, rot, kbeg, nq, nk);
+                for (int lane = 0; lane < 64; ++lane)
+                    for (int h = 0; h < 2; ++h)
+                        for (int j = 0; j < 16; ++j) {
+                            // byte j of the lane's operand of half h: element of the weight, and of a token's codes
+                            int64_t at, code;
+                            if (cols) {
+                                at = raw_col_base(n0, ldw, kt, h, j) + raw_col_lane_bytes(ldw, lane) / 2;
+                                code = raw_col_codes_offset(0, lda, kt, h, lane) + j;
+                                if (!r.access("raw weight W", at, 2, w_elems, block, wave, lane, kt)) continue;
+                            } else {
+                                const int i = 2 * h + (j >> 3);
+                                at = raw_row_offset(n0, ldw, kt, i, lane) + (j & 7);
+                                code = raw_row_codes_offset(0, lda, kt, i, lane) + (j & 7);
+                                if (!r.access("raw weight W", at, 1, w_elems, block, wave, lane, kt)) continue;
+                            }
+                            for (int b = 0; b < blocks; ++b)
+                                r.access("raw weight codes", code + (b * 16 + (lane & 15)) * lda, 1, a_elems, block, wave, lane, kt);
+                            const int64_t row = at / ldw, col = at % ldw;
+                            if (row >= R || col >= C || code != (cols ? row : col)) { r.fail("raw weight: element (%lld, %lld) meets code %lld", (long long)row, (long long)col, (long long)code); continue; }
+                            for (int e = 0; e < (cols ? 2 : 1); ++e) ++read[(size_t)(row * C + col + e)];
+                        }
+            }
+        }
+        for (int wave = 0; wave < blocks; ++wave)
+            for (int lane = 0; lane < 64; ++lane) {
+                const int token = wave * 16 + (lane & 15), count = cols ? 8 : 4;
+                if (token >= tokens) continue;
+                const int64_t col = n0 + (lane >> 4) * count;
+                if (!r.access("raw weight C", token * ldc + col, count, c_elems, block, wave, lane) || col + count > n) continue;
+                for (int e = 0; e < count; ++e) ++stored[(size_t)(token * n + col + e)];
+            }
+    }
+    for (size_t i = 0; i < read.size() && !r.bad; ++i)
+        if (read[i] != 1) r.fail("raw weight: W(%lld, %lld) is read %d times", (long long)(i / C), (long long)(i % C), (int)read[i]);
+    for (size_t i = 0; i < stored.size() && !r.bad; ++i)
+        if (stored[i] != 1) r.fail("raw weight: C(%lld, %lld) is stored %d times", (long long)(i / n), (long long)(i % n), (int)stored[i]);
+    *n_checked = r.checked;
+    return r.bad;
+}
+
 // dW of a step on few tokens (gemm_skinny.hip: thin_walk): every tile belongs to one worker, its rows and K tiles are read, every element stored once
 int walk_thin(int64_t M, int64_t N, int64_t K, int64_t lda, int64_t ldb, int64_t ldc, int num_cu, int64_t a_elems, int64_t b_elems, int64_t c_elems,
               int64_t* n_checked, char* msg, int msglen) {

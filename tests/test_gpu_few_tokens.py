@@ -56,3 +56,29 @@ def test_four_blocks_per_workgroup(dev, monkeypatch, m, n, k, mode):
         spread = (k // 128 + 4) * 2.0 ** -23 * (x.float().abs().amax(1, keepdim=True) * w.float().abs().amax() * k)
         assert bool(((got.float() - want.float()).abs() <= 2.0 ** -7 * mag + spread).all())
         assert float((got != want).float().mean()) <= 0.01
+
+
+# up to 32 tokens the step's GEMMs read the weight itself: against a layer call whose weight is quantised in memory.  Fewer K tiles than waves, one
+# and several batches of them per wave, uneven quarters, rows of the weight apart
+@pytest.mark.parametrize("scheme", ["block_channel", "double_channel"])
+@pytest.mark.parametrize("tokens,k,n", [(1, 128, 384), (16, 4096, 4096), (17, 640, 1152), (31, 2176, 384), (32, 1152, 5120)])
+def test_step_from_the_weight_itself(dev, tokens, k, n, scheme):
+    import triton_int8_amd as T
+    g = make_gen(tokens + k + n)
+    X, W, dY = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, n, k + 32, std=0.02).to(dev)[:, 16:-16], randn_bf16(g, tokens, n, std=1e-3).to(dev)
+    W[3, 5], W[:, 7] = 1.0, 0.0
+    x, w = X.clone().requires_grad_(True), W.contiguous().requires_grad_(True)
+    y = T.Int8LinearFunction.apply(x, w, None, scheme, None)
+    for got, want in zip(T.linear_fwd_bwd(X, W, dY, scheme), (y.detach(), *torch.autograd.grad(y, (x, w), dY))):
+        assert torch.equal(got, want)
+
+
+def test_step_whose_outputs_are_its_inputs(dev):
+    import triton_int8_amd as T
+    g = make_gen(9)
+    X, W, dY = randn_bf16(g, 128, 512).to(dev), randn_bf16(g, 640, 512, std=0.02).to(dev), randn_bf16(g, 128, 640, std=1e-3).to(dev)
+    X[20:], dY[20:] = 0, 0
+    want = T.ops.linear_step(X, W, dY, "block_channel", tokens=20)
+    got = T.ops.linear_step(X, W, dY, "block_channel", tokens=20, out=(torch.empty_like(dY), X, W))
+    for a, b in zip(got, want):
+        assert torch.equal(a[:20] if a.shape[0] == 128 else a, b[:20] if b.shape[0] == 128 else b)

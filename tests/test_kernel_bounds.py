@@ -50,6 +50,8 @@ def walker(tmp_path_factory):
     lib.walk_gemm_tile_map.argtypes = [ci, ci, ci, p64, cp, ci]
     lib.walk_decode_narrow.argtypes = [ci] + [i64] * 8 + [p64, cp, ci]
     lib.walk_few_rows.argtypes = [i64] * 6 + [ci, ci] + [i64] * 3 + [p64, cp, ci]
+    lib.walk_raw_weight.argtypes = [ci] * 2 + [i64] * 8 + [p64, cp, ci]
+    lib.raw_weight_parts.argtypes = [i64] * 2
     lib.walk_thin.argtypes = [i64] * 6 + [ci] + [i64] * 3 + [p64, cp, ci]
     lib.walk_attention.argtypes = [i64] * 3 + [ci] + [i64] * 3 + [ci, ci] + [i64] * 2 + [p64, p64, cp, ci]
     lib.attention_takes_stride.argtypes = [i64] * 3
@@ -329,6 +331,20 @@ def test_decode_narrow_gemm(walker, rows, N, K):
         assert run(*short) == 1 and what in msg.value
 
 
+# fewer K tiles than waves, uneven quarters, rows of the weight apart
+@pytest.mark.parametrize("cols", [0, 1])
+@pytest.mark.parametrize("tokens", [1, 16, 17, 32])
+@pytest.mark.parametrize("R,C", [(384, 128), (1152, 640), (512, 2176)])
+def test_raw_weight_gemms(walker, cols, tokens, R, C):
+    msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
+    k, out, blocks = (R, C, tokens > 16) if cols else (C, R, tokens > 16)
+    run = lambda *elems: walker.walk_raw_weight(cols, tokens, R, C, C + 24, k, out + 8, *elems, ctypes.byref(n), msg, 512)
+    w, a, c = (R - 1) * (C + 24) + C, (32 if blocks else 16) * k, (tokens - 1) * (out + 8) + out
+    assert run(w, a, c) == 0, msg.value.decode()
+    for short, what in (((w - 1, a, c), b"weight W"), ((w, a - 1, c), b"weight codes"), ((w, a, c - 1), b"weight C")):
+        assert run(*short) == 1 and what in msg.value
+
+
 # fewer tiles than CUs and more, a remainder of the workers' rounds
 @pytest.mark.parametrize("M,N,K,num_cu", [(384, 128, 128, 256), (512, 1024, 256, 256), (640, 1152, 256, 8), (1024, 384, 128, 24)])
 def test_thin_gemm(walker, M, N, K, num_cu):
@@ -581,3 +597,10 @@ def test_kernels_of_a_launch_as_a_whole(walker, i32):
                         seen.add(tuple(launch if shapes is step else launch[::-1]))
                 assert len(seen) == 1, step
     assert shared > 20
+
+
+# every size that the rule lets through has its maxima in as many parts as a lane looks at
+def test_raw_weight_parts(walker):
+    for K in range(128, 32769, 128):
+        for N in (128, 4096, 32640, 32768):
+            assert walker.raw_weight_parts(K, N) <= 32 and walker.raw_weight_parts(N, K) <= 32

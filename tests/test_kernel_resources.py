@@ -139,6 +139,10 @@ def test_few_tokens_kernel_waits_match_its_stores(tmp_path):
         # the eight loads of a K tile, in front of the walk and in it, also in one piece
         tiles = [b for b in blocks if b == ["global_load_lds_dwordx4"] * 8]
         assert len(tiles) >= 2 * walks, name
+    for name, body in kernel_bodies("gemm_skinny.hip", tmp_path, "gemm_i8_raw_weight_kernel").items():      # the same walk, beside other GEMMs
+        assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", body), name
+        blocks = [re.findall(r"^\s*" + VMEM, b, flags=re.M) for b in re.split(r"^\.LBB\S+:|^\s*s_cbranch\w+|^\s*s_branch", body, flags=re.M)]
+        assert sum(b == ["global_store_dwordx4"] * 8 for b in blocks) == 1 and len(re.findall(r"s_waitcnt vmcnt\(8\) lgkmcnt\(0\)", body)) >= 1, name
 
 
 def test_attention_kernels_wait_for_what_they_issue(tmp_path):

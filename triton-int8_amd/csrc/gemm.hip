@@ -872,6 +872,32 @@ int ti8::gemm_nt_few(const ti8_gemm_problem* problems, int count, bool backward,
     return launch_few(m, few, i32_full, static_cast<hipStream_t>(stream));
 }
 
+// Where a block-channel step on few tokens reads its weight twice more, behind the maxima, instead of writing its codes both ways and reading
+// those (idx::raw_weight_takes), and where that gives the same bits: where the few-rows kernel serves Y and dX otherwise, and dW is on thin tiles.
+bool ti8::gemm_raw_weight_takes(int64_t tokens, int64_t K, int64_t N, int64_t ldw) {
+    const int cus = device_cu_count();
+    return idx::raw_weight_takes(tokens, K, N) && N > 256 && ldw <= 0x00ffffff && !idx::gemm_few_rows_prefers_mid(32, N, K, 1, cus) &&
+           !idx::gemm_few_rows_prefers_mid(32, K, N, 1, cus);
+}
+
+int ti8::gemm_nt_raw_weight(const ti8_gemm_problem* problems, const QRowColOperand& w, int64_t tokens, ti8_stream_t stream) {
+    GemmMulti m;
+    m.count = 3;
+    for (int i = 0; i < 3; ++i) {
+        ti8_gemm_problem p = problems[i];
+        if (i < 2) p.M = 32;
+        if (int e = prepare_gemm("ti8_linear", p, 0, &m.g[i])) return e;
+    }
+    if (!thin_supported(m.g[2], false)) return fail(TI8_ERR_SHAPE, "ti8_linear: dW does not fit its kernel");
+    const idx::MaximaParts parts = idx::maxima_parts(w.R, w.C);
+    RawWeight r;
+    r.w = static_cast<const uint16_t*>(w.x); r.ldw = w.ldx;
+    r.rows = reinterpret_cast<const uint16_t*>(w.partial);
+    r.cols = r.rows + (int64_t)parts.nct * w.R;
+    r.R = (int)w.R; r.C = (int)w.C; r.nrt = parts.nrt; r.nct = parts.nct;
+    return launch_raw_weight(m, r, (int)tokens, static_cast<hipStream_t>(stream));
+}
+
 // Up to 8 rows through a weight quantised earlier: the GEMM's kernel quantises them itself, each workgroup anew, where
 // idx::decode_quantises or idx::decode_narrow says so.  It saves a launch on a path that waits for the host: one token, 4096 -> 4096,
 // 13.3 -> 9.9 us (by rows 14.0 -> 10.8).

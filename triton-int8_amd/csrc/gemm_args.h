@@ -100,6 +100,14 @@ int launch_decode(const GemmArgs& a, int rows, bool i32_full, hipStream_t st);
 int launch_decode_narrow(const GemmArgs& a, int rows, bool i32_full, hipStream_t st);      // the same on few columns (gemm_decode.hip)
 // GEMMs over at most two K tiles, on 128 x 128 tiles: dW of a step on few tokens
 bool thin_supported(const GemmArgs& a, bool i32_full);
+// Y (m.g[0]), dX (1) and dW (2) of a block-channel step on few tokens from the weight in bf16; fills first[] of `m`
+struct RawWeight {
+    const uint16_t* w;
+    const uint16_t *rows, *cols;        // partial maxima as MaxOperand (quant.hip) has them: [nct][R], [nrt][C]
+    int64_t ldw;
+    int R, C, nrt, nct;
+};
+int launch_raw_weight(GemmMulti& m, const RawWeight& w, int tokens, hipStream_t st);
 // several GEMMs of batch 1 in one launch, the first `few` of m.g on the few-rows kernel, one behind them on thin tiles; fills first[] of `m`
 int launch_few(GemmMulti& m, int few, bool i32_full, hipStream_t st);
 

@@ -509,6 +509,200 @@ __global__ __launch_bounds__(256) void gemm_i8_few_kernel(const GemmMulti m, con
     else thin_walk<I32FULL, I32FULL>(m.g[i], block, workers);
 }
 
+// Y (16 columns of it, rows of the weight) or, COLS, dX (32 columns of the weight) of up to 16 TB tokens, the weight quantised on its way from
+// memory into the operands of the matrix instructions: by its rows for Y, by its columns for dX.  A weight that is used by so
+// few tokens costs more to quantise into memory (its codes written both ways and read again) than to read twice.  16x16x64 products want 16 codes in a row
+// along the contraction: for Y what two loads bring; for dX a lane loads 2 columns of 16 rows and the conversion, which
+// places single bytes, transposes them (a single column per lane, which gives every CU a workgroup: 22 us for Y and dX instead of 20, the
+// weight's cache lines go to four CUs).  What bounds it is the conversion, 6 instructions per element, on one or two waves per SIMD: 4096 ->
+// 4096, 13 us for Y alone, 14 for dX, 25 with dW in the launch, where the conversion both ways and the GEMMs took 29 in two.  Four waves take
+// the K tiles' quarters, each with two of them on their way; walk, sums and epilogue are those of wavering_block, operation for operation: the
+// same bits.
+template <bool COLS, int TB>
+__device__ __forceinline__ void raw_block(const GemmArgs& g, const RawWeight& w, const int strip, const int tokens) {
+    constexpr int SETS = COLS ? 2 : 1;
+    constexpr int AHEAD = 2, WORDS = COLS ? 32 : 16;
+    extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
+    const int lane = threadIdx.x & 63, low = lane & 15, quad = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = strip * (COLS ? idx::RAW_STRIP_DX : idx::RAW_STRIP_Y), nk = g.K >> 7;
+    const int kbeg = idx::few_k_first(wave, nk), nq = idx::few_k_first(wave + 1, nk) - kbeg;
+    const int rot = idx::decode_rot(n0, nq);
+    auto tile_of_step = [&](int i) { return idx::few_k_tile(i, rot, kbeg, nq, nk); };
+    const float f_all = g.sa.p[(int64_t)tile_of_step(lane) * g.sa.ks];    // of step `lane` (at most 64 per wave)
+
+    // maxima of this lane's row, or two columns
+    // (of up to 32 parts, all asked for at once: one after the other they took longer than the weight)
+    uint32_t parts[idx::RAW_PARTS / 4];
+#pragma unroll
+    for (int i = 0; i < idx::RAW_PARTS / 4; ++i) {
+        const int p = idx::raw_part(i, lane, COLS ? w.nrt : w.nct);
+        if (COLS) parts[i] = *reinterpret_cast<const uint32_t*>(w.cols + idx::maxima_cols_at(p, w.C, n0 + 2 * low));
+        else parts[i] = w.rows[idx::maxima_rows_at(p, w.R, n0 + low)];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+
+    uint32_t raw[AHEAD][WORDS];
+    v4i codes[AHEAD][TB][2];
+    const uint32_t lane_bytes = COLS ? idx::raw_col_lane_bytes(w.ldw, lane) : 0;
+    auto load = [&](int step, uint32_t (&to)[WORDS], v4i (&a)[TB][2]) {
+        const int kt = tile_of_step(step);
+        if constexpr (COLS) {
+            uint32_t at = lane_bytes;
+            asm volatile("" : "+v"(at));        // (a scalar base and a 32-bit offset per load)
+#pragma unroll
+            for (int h = 0; h < 2; ++h) {
+                const char* row = reinterpret_cast<const char*>(w.w + idx::raw_col_base(n0, w.ldw, kt, h, 0));
+#pragma unroll
+                for (int j = 0; j < 16; ++j, row += 2 * w.ldw) to[h * 16 + j] = *reinterpret_cast<const uint32_t*>(row + at);      // (raw_col_base of row j)
+            }
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+#pragma unroll
+                for (int h = 0; h < 2; ++h) a[b][h] = *reinterpret_cast<const v4i*>(g.A + idx::raw_col_codes_offset(b * 16 + low, g.lda, kt, h, lane));
+        } else {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const uint4 v = *reinterpret_cast<const uint4*>(w.w + idx::raw_row_offset(n0, w.ldw, kt, i, lane));
+                to[i * 4] = v.x; to[i * 4 + 1] = v.y; to[i * 4 + 2] = v.z; to[i * 4 + 3] = v.w;
+            }
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const v2i v = *reinterpret_cast<const v2i*>(g.A + idx::raw_row_codes_offset(b * 16 + low, g.lda, kt, i, lane));
+                    a[b][i >> 1][(i & 1) * 2] = v.x;
+                    a[b][i >> 1][(i & 1) * 2 + 1] = v.y;
+                }
+        }
+    };
+#pragma unroll
+    for (int t = 0; t < AHEAD; ++t) load(t, raw[t], codes[t]);     // (past the last one: that one again)
+    __builtin_amdgcn_sched_barrier(0);
+
+    uint32_t m_lo = 0, m_hi = 0;
+#pragma unroll
+    for (int i = 0; i < idx::RAW_PARTS / 4; ++i) {
+        m_lo = max(m_lo, parts[i] & 0xffffu);
+        m_hi = max(m_hi, parts[i] >> 16);
+    }
+    m_lo = max(m_lo, (uint32_t)__shfl_xor((int)m_lo, 16, 64));
+    m_lo = max(m_lo, (uint32_t)__shfl_xor((int)m_lo, 32, 64));
+    const QMode mode = {1, 0, 0, TI8_INV_RCP_OF_SCALE};
+    const float amax_lo = amax_floor(__uint_as_float(m_lo << 16), 0), mult_lo = 127.0f / amax_lo, scale_lo = stored_scale(amax_lo, mult_lo, mode);
+    float mult_hi = 0.0f, scale_hi = 0.0f;
+    if (COLS) {
+        m_hi = max(m_hi, (uint32_t)__shfl_xor((int)m_hi, 16, 64));
+        m_hi = max(m_hi, (uint32_t)__shfl_xor((int)m_hi, 32, 64));
+        const float amax_hi = amax_floor(__uint_as_float(m_hi << 16), 0);
+        mult_hi = 127.0f / amax_hi;
+        scale_hi = stored_scale(amax_hi, mult_hi, mode);
+    }
+
+    const v4i zero = {0, 0, 0, 0};
+    float accf[SETS][TB][4];
+#pragma unroll
+    for (int s = 0; s < SETS; ++s)
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) accf[s][b][r] = 0.0f;
+    auto multiply = [&](int step, const uint32_t (&v)[WORDS], const v4i (&a)[TB][2]) {
+        const float f = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f_all), step));
+        v4i d[SETS][TB];
+#pragma unroll
+        for (int s = 0; s < SETS; ++s)
+#pragma unroll
+            for (int b = 0; b < TB; ++b) d[s][b] = zero;
+#pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            v4i op[SETS];
+            if constexpr (COLS) {
+                uint32_t lo[4] = {0, 0, 0, 0}, hi[4] = {0, 0, 0, 0};
+#pragma unroll
+                for (int j = 0; j < 16; ++j) {
+                    lo[j >> 2] = put_u8(qbiased(bf16_lo(v[h * 16 + j]), mult_lo), j & 3, lo[j >> 2]);
+                    hi[j >> 2] = put_u8(qbiased(bf16_hi(v[h * 16 + j]), mult_hi), j & 3, hi[j >> 2]);
+                }
+                op[0] = v4i{(int)(lo[0] ^ UNBIAS4), (int)(lo[1] ^ UNBIAS4), (int)(lo[2] ^ UNBIAS4), (int)(lo[3] ^ UNBIAS4)};
+                op[SETS - 1] = v4i{(int)(hi[0] ^ UNBIAS4), (int)(hi[1] ^ UNBIAS4), (int)(hi[2] ^ UNBIAS4), (int)(hi[3] ^ UNBIAS4)};
+            } else {
+                const uint32_t* const x = v + h * 8;
+                const uint2 p = quant8(make_uint4(x[0], x[1], x[2], x[3]), mult_lo), q = quant8(make_uint4(x[4], x[5], x[6], x[7]), mult_lo);
+                op[0] = v4i{(int)p.x, (int)p.y, (int)q.x, (int)q.y};
+            }
+#pragma unroll
+            for (int s = 0; s < SETS; ++s)
+#pragma unroll
+                for (int b = 0; b < TB; ++b) d[s][b] = __builtin_amdgcn_mfma_i32_16x16x64_i8(op[s], a[b][h], d[s][b], 0, 0, 0);
+        }
+#pragma unroll
+        for (int s = 0; s < SETS; ++s)
+#pragma unroll
+            for (int b = 0; b < TB; ++b)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) accf[s][b][r] = __builtin_fmaf(static_cast<float>(d[s][b][r]), f, accf[s][b][r]);
+    };
+    // one copy of the code (a kernel's instructions come from memory, too): loads past the last K tile ask for that one again
+    for (int step = 0; step < nq; step += AHEAD)
+#pragma unroll
+        for (int t = 0; t < AHEAD; ++t) {
+            if (step + t < nq) multiply(step + t, raw[t], codes[t]);
+            __builtin_amdgcn_sched_barrier(0);      // the compiler would put off the loads to the end of the batch
+            load(step + AHEAD + t, raw[t], codes[t]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+
+    // lane: token 16 b + low; columns n0 + 4 quad + r, COLS: n0 + 2 (4 quad + r) + set
+    float4* const sums = reinterpret_cast<float4*>(smem);       // [wave][set][b][lane]
+#pragma unroll
+    for (int s = 0; s < SETS; ++s)
+#pragma unroll
+        for (int b = 0; b < TB; ++b)
+            sums[((wave * SETS + s) * TB + b) * 64 + lane] = make_float4(accf[s][b][0], accf[s][b][1], accf[s][b][2], accf[s][b][3]);
+    float scale[SETS][4];       // of those columns
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        scale[0][r] = __shfl(scale_lo, quad * 4 + r, 64);
+        if (COLS) scale[SETS - 1][r] = __shfl(scale_hi, quad * 4 + r, 64);
+    }
+    __syncthreads();
+    const int token = wave * 16 + low;
+    if (wave >= TB || token >= tokens) return;
+    float out[SETS][4];
+#pragma unroll
+    for (int s = 0; s < SETS; ++s) {
+        float part[4][4];
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float4 v = sums[((q * SETS + s) * TB + wave) * 64 + lane];
+            part[q][0] = v.x; part[q][1] = v.y; part[q][2] = v.z; part[q][3] = v.w;
+        }
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+            float v = part[0][r] + part[1][r];
+            v = v + part[2][r];
+            v = v + part[3][r];
+            out[s][r] = v * scale[s][r];
+        }
+    }
+    uint16_t* const to = reinterpret_cast<uint16_t*>(g.C) + (int64_t)token * g.ldc + n0 + quad * (4 * SETS);
+    if constexpr (COLS)
+        *reinterpret_cast<uint4*>(to) = make_uint4(pack_bf16x2(out[0][0], out[SETS - 1][0]), pack_bf16x2(out[0][1], out[SETS - 1][1]),
+                                                   pack_bf16x2(out[0][2], out[SETS - 1][2]), pack_bf16x2(out[0][3], out[SETS - 1][3]));
+    else
+        *reinterpret_cast<uint2*>(to) = make_uint2(pack_bf16x2(out[0][0], out[0][1]), pack_bf16x2(out[0][2], out[0][3]));
+}
+
+// dX first: its workgroups have the most to do, two that share the cache lines of the weight on one XCD
+template <int TB>
+__global__ __launch_bounds__(256) void gemm_i8_raw_weight_kernel(const GemmMulti m, const RawWeight w, const int tokens) {
+    const int block = (int)blockIdx.x;
+    if (block < m.first[1]) raw_block<true, TB>(m.g[1], w, idx::column_strip(block, m.first[1]), tokens);
+    else if (block < m.first[2]) raw_block<false, TB>(m.g[0], w, block - m.first[1], tokens);
+    else thin_walk<false, false>(m.g[2], block - m.first[2], (int)gridDim.x - m.first[2]);
+}
+
 bool skinny_supported(const GemmArgs& a) {
     // factors that vary inside a 32 x 32 block (one scale per row or column AND K tile) and more
     // than 256 K tiles are left to the tiled kernels
@@ -579,6 +773,18 @@ static int launch_few_group(GemmMulti& m, int few, bool wide, bool i32_full, hip
     hipLaunchKernelGGL(kernel, dim3((unsigned)total), dim3(256), wavering_lds_bytes(wide), st, m, few, wide);
     note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
     return check_launch("ti8_gemm_i8_nt");
+}
+
+int launch_raw_weight(GemmMulti& m, const RawWeight& w, int tokens, hipStream_t st) {
+    m.first[0] = 0;
+    m.first[1] = w.C / idx::RAW_STRIP_DX;
+    m.first[2] = m.first[1] + w.R / idx::RAW_STRIP_Y;
+    m.first[3] = m.first[2] + (int)idx::thin_workers(w.R, w.C, device_cu_count());
+    const auto kernel = tokens <= 16 ? gemm_i8_raw_weight_kernel<1> : gemm_i8_raw_weight_kernel<2>;
+    static_assert(4 * 2 * 2 * 64 * 16 <= 2 * 2 * THIN_OPERAND, "the waves' sums share the launch's LDS");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)m.first[3]), dim3(256), 2 * 2 * THIN_OPERAND, st, m, w, tokens);
+    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, EPI_PROMOTE);
+    return check_launch("ti8_linear");
 }
 
 int launch_few(GemmMulti& m, int few, bool i32_full, hipStream_t st) {

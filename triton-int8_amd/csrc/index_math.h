@@ -380,6 +380,28 @@ TI8_HD int decode_rot(int n0, int nq) { return nq > 0 ? (int)((((unsigned)n0 >> 
 // the lane's 16 columns of a row's K tile, and its 16 bytes of the weight's (the second half of the K tile: 64 bytes on)
 TI8_HD int64_t decode_x_offset(int row, int64_t ldx, int kt, int lane) { return row * ldx + kt * 128 + (lane & 7) * 16; }
 TI8_HD int64_t decode_w_offset(int n0, int64_t ldb, int kt, int lane) { return (int64_t)(n0 + (lane & 15)) * ldb + kt * 128 + (lane >> 4) * 16; }
+// ---- Y and dX of a step on few tokens, the weight quantised in the kernel (gemm_skinny.hip: raw_block) ---------------
+// Elements of the weight [R][C] that a lane loads for a K tile.  Y: piece i (of 4) of 8 columns of its row; the 64 columns of a matrix
+// instruction are two pieces of four lanes each, and the codes of the tokens are read the same way.  dX: 2 columns of row j (of 16) of half h.
+constexpr int RAW_STRIP_Y = 16, RAW_STRIP_DX = 32;
+// part of the maxima that a lane looks at as its i-th: every fourth, past the last one that one again.  Up to 32 parts (maxima_parts, up to
+// 32 * 128 * MAXIMA_ROW_TILES rows)
+constexpr int RAW_PARTS = 32;
+TI8_HD int raw_part(int i, int lane, int count) { return imin((lane >> 4) + 4 * i, count - 1); }
+// Whether such a step takes them.  A workgroup walks the whole contraction, so a side much longer than the other leaves few of them with long
+// walks; and for a second block of 16 tokens the codes are read twice as often, which costs on a large weight what the saved launch gains.
+// The step, us, its weight quantised in memory / so: 16 tokens, 4096 -> 4096 37.7 / 32.5, 2048 -> 2048 22.3 / 17.3, 7936 -> 8960 177 / 132,
+// 13440 -> 3200 89.8 / 76.1, 3200 -> 13440 88.6 / 75.0, 10240 -> 1024 37.1 / 34.5, 14336 -> 1024 44.8 / 45.9, 2048 -> 14336 62.7 / 62.4, 1536
+// -> 8960 37.3 / 39.5, 1024 -> 14336 41.5 / 49.1; 32 tokens, 2048 -> 2048 22.3 / 17.2, 2560 -> 2560 26.8 / 22.4, 3072 -> 3072 29.3 / 29.0,
+// 5632 -> 4736 60.8 / 63.7.  (The double-channel step converts X and dY between the maxima and the GEMMs: 17 tokens, 5632 -> 4736 66 / 77.)
+TI8_HD bool raw_weight_takes(int64_t tokens, int64_t K, int64_t N) {
+    return tokens <= 32 && (tokens <= 16 || N * K <= 2560 * 2560) && N <= 5 * K && K <= 10 * N && K <= 32768 && N <= 32768;
+}
+TI8_HD int64_t raw_row_offset(int n0, int64_t ldw, int kt, int i, int lane) { return (int64_t)(n0 + (lane & 15)) * ldw + kt * 128 + i * 32 + (lane >> 4) * 8; }
+TI8_HD int64_t raw_row_codes_offset(int token, int64_t lda, int kt, int i, int lane) { return (int64_t)token * lda + kt * 128 + i * 32 + (lane >> 4) * 8; }
+TI8_HD int64_t raw_col_base(int n0, int64_t ldw, int kt, int h, int j) { return (int64_t)(kt * 128 + h * 64 + j) * ldw + n0; }
+TI8_HD uint32_t raw_col_lane_bytes(int64_t ldw, int lane) { return (uint32_t)((lane >> 4) * 16 * (int)ldw + (lane & 15) * 2) * 2u; }
+TI8_HD int64_t raw_col_codes_offset(int token, int64_t lda, int kt, int h, int lane) { return (int64_t)token * lda + kt * 128 + h * 64 + (lane >> 4) * 16; }
 // dW beside them: workgroups for its 128 x 128 tiles, worker w taking w, w + workers, ...
 TI8_HD int64_t thin_workers(int64_t M, int64_t N, int64_t num_cu) {
     const int64_t tiles = (M / 128) * (N / 128);

@@ -1054,9 +1054,10 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
     b.first[nblocks] = (int)block_tiles;
     block_tiles = idx::round8(block_tiles);
     b.first[QBLOCK_MULTI_MAX] = (int)block_tiles;
-    MaxMulti m;
-    int64_t parts = 0, tiles = 0, first_tile[MAX_OPERANDS + 1];
+    MaxMulti m, conversions;
+    int64_t parts = 0, tiles = 0;
     m.count = nboth;
+    conversions.count = 0;
     for (int i = 0; i < nboth; ++i) {
         const QRowColOperand& o = both[i];
         if (!o.x || !o.q || !o.s_row || !o.qT || !o.s_col || !o.maxima) return fail(TI8_ERR_NULL, "%s: x, q, s_row, qT, s_col and maxima are required", fn);
@@ -1074,13 +1075,20 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
         x.q = o.q; x.ldq = o.C; x.s_row = o.s_row; x.qT = o.qT; x.ldqt = o.R; x.s_col = o.s_col;
         x.R = (int)o.R; x.C = (int)o.C; x.valid_rows = (int)o.valid_rows;
         m.first[i] = (int)parts;
-        first_tile[i] = tiles;
         parts += idx::round8((int64_t)x.nrt * x.nct);
-        tiles += idx::round8((o.R / 128) * (o.C / 128));
+        if (!o.maxima_only) {
+            conversions.op[conversions.count] = x;
+            conversions.first[conversions.count++] = (int)tiles;
+            tiles += idx::round8((o.R / 128) * (o.C / 128));
+        }
         if (parts + block_tiles > 0x7fffffffLL || tiles > 0x7fffffffLL) return fail(TI8_ERR_SHAPE, "%s: too many tiles", fn);
     }
-    for (int i = nboth; i < MAX_OPERANDS; ++i) { m.op[i] = nboth ? m.op[0] : MaxOperand{}; m.first[i] = (int)parts; first_tile[i] = tiles; }
-    m.first[MAX_OPERANDS] = (int)parts;
+    auto fill = [](MaxMulti& to, int64_t total) {
+        for (int i = to.count; i < MAX_OPERANDS; ++i) { to.op[i] = to.count ? to.op[0] : MaxOperand{}; to.first[i] = (int)total; }
+        to.first[MAX_OPERANDS] = (int)total;
+    };
+    fill(m, parts);
+    fill(conversions, tiles);
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (atomics) {
         ClearRanges r = {};
@@ -1104,10 +1112,8 @@ int ti8::quant_call(const char* fn, const ti8_qblock_operand* blocks, const int6
     }
     hipLaunchKernelGGL(quant_first_kernel, dim3((unsigned)(parts + block_tiles + r.workgroups)), dim3(256), 0, st, m, b, r, mode);
     if (int e = check_launch(fn)) return e;
-    if (!nboth) return TI8_OK;
-    for (int i = 0; i < MAX_OPERANDS; ++i) m.first[i] = (int)first_tile[i];
-    m.first[MAX_OPERANDS] = (int)tiles;
-    hipLaunchKernelGGL(quant_rowcol_multi_kernel, dim3((unsigned)tiles), dim3(256), 0, st, m, mode);
+    if (!conversions.count) return TI8_OK;
+    hipLaunchKernelGGL(quant_rowcol_multi_kernel, dim3((unsigned)tiles), dim3(256), 0, st, conversions, mode);
     return check_launch(fn);
 }
 

@@ -31,6 +31,8 @@ struct Layer {
     bool partials_in_outputs = false;
     // layers that multiply the same X (ti8_linear_group): the one that quantises it (null: this one)
     const Layer* input_of = nullptr;
+    // the GEMMs quantise the weight themselves: of its codes there are only the maxima, in their place
+    bool raw_weight = false;
     // operands of Y = X W^T, dX = dY W, dW = dY^T X and their scales
     int8_t *xq, *wq, *dq, *wtq, *dytq, *xtq;
     float *xs, *ws, *ds, *wts, *dyts, *xts;
@@ -257,7 +259,9 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
         unsigned int* partial = nullptr;
         if (L.partial_words(R, C)) partial = reinterpret_cast<unsigned int*>(take_maxima(quant_maxima_words(R, C)));
         else if (apart && ldout == C) partial = static_cast<unsigned int*>(out);
-        o.both[o.nboth++] = QRowColOperand{x, ldx, oq, os, oqT, osT, scratch, partial, R, valid, C};
+        const bool raw = L.raw_weight && x == a.W;
+        if (raw) partial = reinterpret_cast<unsigned int*>(oq);
+        o.both[o.nboth++] = QRowColOperand{x, ldx, oq, os, oqT, osT, scratch, partial, R, valid, C, raw};
     };
     auto block = [&](const ti8_qblock_operand& operand, int64_t valid) {
         o.by_block_rows[o.nblocks] = valid;
@@ -415,11 +419,14 @@ int run_layer(const char* fn, const ti8_linear_args* a, int64_t T, ti8_gemm_prob
                                    a->X, a->ldx, L.tokens, a->bias, a->gemm_flags, &done, stream)) return e;
         if (done) return TI8_OK;
     }
+    L.raw_weight = !problems && T <= 256 && L.fwd && L.bwd && !L.had && L.block() && !a->bias && !(a->gemm_flags & (TI8_GEMM_TILED | TI8_GEMM_LARGE_TILES)) &&
+                   quant_together(L.both_ways_bytes()) && gemm_raw_weight_takes(L.tokens, L.K, L.N, a->ldw) && step_apart(*a, T);
     ti8_gemm_problem g[3];
     int n = 0;
     Operands operands;
     if (int e = quantise(fn, L, operands, g, &n, stream)) return e;
     if (int e = quantise_operands(fn, L, operands, stream)) return e;
+    if (L.raw_weight) return gemm_nt_raw_weight(g, operands.both[0], L.tokens, stream);
     if (problems) {
         for (int i = 0; i < n; ++i) problems[i] = g[i];
         *count = n;

@@ -78,6 +78,7 @@ struct QRowColOperand {
     float* s_col;
     unsigned int *maxima, *partial;
     int64_t R, valid_rows, C;
+    bool maxima_only = false;       // the conversion is somebody else's (with `partial`, not in the atomics form)
 };
 int64_t quant_maxima_words(int64_t R, int64_t C);
 // whether the maxima of so many bytes of such operands are collected in one launch; else `partial` is not looked at
@@ -110,6 +111,10 @@ int gemm_nt_few(const ti8_gemm_problem* problems, int count, bool backward, cons
 int gemm_nt_decode(const ti8_gemm_problem& p, const void* X, int64_t ldx, int64_t rows, const void* bias, int gemm_flags, bool* done, ti8_stream_t stream);
 // y = bf16(bf16(c + b) + y) on [rows][cols], b and c dense; without c: bf16(b + y) (bias.hip)
 int add_rows(const char* fn, void* y, int64_t ldy, const void* b, const void* c, int64_t rows, int64_t cols, ti8_stream_t stream);
+// Y, dX and dW of a block-channel step on up to 32 of up to 256 padded tokens from the weight itself, W [N][K], whose maxima are in `w.partial`, and where that is
+// taken
+bool gemm_raw_weight_takes(int64_t tokens, int64_t K, int64_t N, int64_t ldw);
+int gemm_nt_raw_weight(const ti8_gemm_problem* problems, const QRowColOperand& w, int64_t tokens, ti8_stream_t stream);
 int add_bias(void* y, int64_t ldy, const void* bias, int64_t rows, int64_t cols, ti8_stream_t stream);
 // out[c] = bf16(sum over g of partial[g][c]), dim a multiple of 32 (decoder.hip)
 int sum_partials(const char* fn, const float* partial, int groups, int64_t dim, void* out, hipStream_t st);
