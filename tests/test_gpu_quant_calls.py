@@ -100,3 +100,22 @@ def test_few_rows_quantised(dev, rows, cols):
     # tensors on both sides of a division: one rounding (a number over a tensor is 127 times the reciprocal to torch, two)
     scale = torch.full_like(amax, 127.0) / amax
     assert torch.equal(q.float(), torch.floor(x.float() * scale[:, None] + 0.5).clamp(-128, 127)) and torch.equal(s, amax / torch.full_like(amax, 127.0))
+
+
+# rotated operands of a call in one launch: the forms of the row quantiser (up to 2048, 4096, 8192, 16384 columns, and the rows beyond that keep a launch
+# of their own), tiles with missing tokens, against the separate entry points
+@pytest.mark.parametrize("scheme", ["block_channel", "row_block"])
+@pytest.mark.parametrize("tokens,k,n", [(1, 128, 2176), (37, 2048, 384), (130, 2176, 4096), (300, 4224, 640), (40, 512, 8320), (33, 16512, 256)])
+def test_rotated_operands_in_one_launch(dev, monkeypatch, scheme, tokens, k, n):
+    import triton_int8_amd as T
+    g = make_gen(tokens + k + n)
+    X, W, dY = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev), randn_bf16(g, tokens, n, std=1e-3).to(dev)
+    x, w = X.clone().requires_grad_(True), W.clone().requires_grad_(True)
+
+    def results():
+        y = T.Int8LinearFunction.apply(x, w, None, scheme, 128)
+        return (*T.linear_fwd_bwd(X, W, dY, scheme, 128), y.detach(), *torch.autograd.grad(y, (x, w), dY))
+    got = results()
+    monkeypatch.setattr(T.linear, "ONE_CALL_STEP", False)
+    for a, b in zip(got, results()):
+        assert torch.equal(a, b)

@@ -257,16 +257,14 @@ __global__ __launch_bounds__(256) void quant_block_multi_kernel(const QBlockMult
 // holds and writes them to s[C].
 enum { HAD_BLOCK = 0, HAD_COLMAX = 1, HAD_COL = 2 };
 
-template <bool ALONG_ROWS, int SCALE = HAD_BLOCK>
-__global__ __launch_bounds__(256) void quant_block_had_kernel(
+constexpr int had_tile_elems(bool along_rows) { return along_rows ? 128 * 128 : 8; }
+// tile t; `tile`: had_tile_elems
+template <bool ALONG_ROWS, int SCALE>
+__device__ __forceinline__ void quant_block_had_part(
     const uint16_t* __restrict__ x, int64_t bsx, int64_t ldx, int8_t* __restrict__ q, int64_t bsq, int64_t ldq,
-    float* __restrict__ s, int64_t ssb, int64_t ssr, int64_t ssc, int nrb, int ncb, int valid_rows, QMode mode,
-    unsigned int* __restrict__ ws = nullptr) {
+    float* __restrict__ s, int64_t ssb, int64_t ssr, int64_t ssc, int nrb, int ncb, int valid_rows, const QMode& mode,
+    unsigned int* __restrict__ ws, int t, uint16_t* tile, float* red4) {
     static_assert(SCALE == HAD_BLOCK || ALONG_ROWS, "column-wise scales go with the rotation along rows");
-    __shared__ float red4[4];
-    __shared__ __attribute__((aligned(16))) uint16_t tile[ALONG_ROWS ? 128 * 128 : 8];
-
-    int t = blockIdx.x;
     const int cb = t % ncb;
     t /= ncb;
     const int rb = t % nrb;
@@ -367,6 +365,16 @@ __global__ __launch_bounds__(256) void quant_block_had_kernel(
             *reinterpret_cast<uint2*>(qt + (int64_t)(h * 64 + rg * 4 + j) * ldq + cc * 8) = quant8(v[h][j], lane_scale);
 }
 
+template <bool ALONG_ROWS, int SCALE = HAD_BLOCK>
+__global__ __launch_bounds__(256) void quant_block_had_kernel(
+    const uint16_t* __restrict__ x, int64_t bsx, int64_t ldx, int8_t* __restrict__ q, int64_t bsq, int64_t ldq,
+    float* __restrict__ s, int64_t ssb, int64_t ssr, int64_t ssc, int nrb, int ncb, int valid_rows, QMode mode,
+    unsigned int* __restrict__ ws = nullptr) {
+    __shared__ float red4[4];
+    __shared__ __attribute__((aligned(16))) uint16_t tile[had_tile_elems(ALONG_ROWS)];
+    quant_block_had_part<ALONG_ROWS, SCALE>(x, bsx, ldx, q, bsq, ldq, s, ssb, ssr, ssc, nrb, ncb, valid_rows, mode, ws, (int)blockIdx.x, tile, red4);
+}
+
 // ---------------------------------------------------------------------------------
 // Per-row quantiser, one pass.  WG_ROW = false: one wavefront per row (4 rows per
 // workgroup); WG_ROW = true: one 256-thread workgroup per row.  Each thread keeps
@@ -432,6 +440,44 @@ __global__ __launch_bounds__(256) void quant_row_kernel(const uint16_t* __restri
                                                         int64_t rows, int cols, QMode mode) {
     __shared__ float red4[4];
     quant_row_part<NLOAD, WG_ROW, GROUP16, HAD, ARITH>(x, ldx, q, ldq, s, rows, cols, mode, (int)blockIdx.x, red4);
+}
+
+// The rotating quantisers of a layer call in one launch (one with per-column scales: its maxima here, the conversion behind it): a workgroup per
+// 128 x 128 tile, or per 4 rows or row.  Apart they are up to eight launches, which few tokens wait for, and a tensor that two of
+// them read is no longer in the caches for the second.  Block-channel steps, us, apart / so: 39 tokens, 2176 -> 2560 58.5 / 33.4, 128, 4352 ->
+// 1792 69.9 / 44.9, 1024, 4096 -> 4096 125 / 106, 4096, 4096 -> 4096 298 / 273, 8192, 8192 -> 8192 1840 / 1806.
+struct HadMultiOperand {
+    const uint16_t* x;
+    int8_t* q;
+    float* s;
+    unsigned int* ws;
+    int64_t ldx, ldq;
+    int kind, R, C, valid_rows;     // (by rows: R rows)
+};
+struct HadMulti {
+    HadMultiOperand op[QHAD_MAX];
+    int first[QHAD_MAX];            // of the workgroups; past the last operand: all of them
+};
+__global__ __launch_bounds__(256) void quant_had_multi_kernel(const HadMulti m, const QMode mode) {
+    __shared__ float red4[4];
+    __shared__ __attribute__((aligned(16))) uint16_t tile[had_tile_elems(true)];
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < QHAD_MAX; ++k)
+        if ((int)blockIdx.x >= m.first[k]) i = k;
+    const HadMultiOperand& o = m.op[i];
+    const int t = (int)blockIdx.x - m.first[i];
+    const int ncb = o.C >> 7;
+    switch (o.kind) {
+        case QHAD_BLOCKS: quant_block_had_part<false, HAD_BLOCK>(o.x, 0, o.ldx, o.q, 0, o.ldq, o.s, 0, ncb, 1, o.R >> 7, ncb, o.valid_rows, mode, nullptr, t, tile, red4); break;
+        case QHAD_BLOCKS_T: quant_block_had_part<true, HAD_BLOCK>(o.x, 0, o.ldx, o.q, 0, o.ldq, o.s, 0, ncb, 1, o.R >> 7, ncb, o.valid_rows, mode, nullptr, t, tile, red4); break;
+        case QHAD_COLUMNS: quant_block_had_part<true, HAD_COLMAX>(o.x, 0, o.ldx, o.q, 0, o.ldq, o.s, 0, 0, 0, o.R >> 7, ncb, o.valid_rows, mode, o.ws, t, tile, red4); break;
+        default:            // QHAD_ROWS, in the forms of idx::qrow_config (a row of up to 2048 columns in 4 chunks per lane)
+            if (o.C <= 2048) quant_row_part<4, false, false, true>(o.x, o.ldx, o.q, o.ldq, o.s, o.R, o.C, mode, t, red4);
+            else if (o.C <= 4096) quant_row_part<8, false, false, true>(o.x, o.ldx, o.q, o.ldq, o.s, o.R, o.C, mode, t, red4);
+            else if (o.C <= 8192) quant_row_part<4, true, false, true>(o.x, o.ldx, o.q, o.ldq, o.s, o.R, o.C, mode, t, red4);
+            else quant_row_part<8, true, false, true>(o.x, o.ldx, o.q, o.ldq, o.s, o.R, o.C, mode, t, red4);
+    }
 }
 
 struct ClearRanges {    // words to zero, one behind the other
@@ -961,6 +1007,77 @@ extern "C" int ti8_quant_block(const void* x, int64_t bsx, int64_t ldx, int8_t* 
     else TI8_LAUNCH_QB(1, false, true);
 #undef TI8_LAUNCH_QB
     return check_launch("ti8_quant_block");
+}
+
+// One operand by the entry point of its kind
+static int quant_had_alone(const QHadOperand& o, int qflags, int inv_mode, ti8_stream_t stream) {
+    const int64_t grid = o.C / 128;
+    switch (o.kind) {
+        case QHAD_BLOCKS: return quant_block_had128_valid(o.x, 0, o.ldx, o.q, o.R * o.C, o.C, o.s, 0, grid, 1, 1, o.R, o.valid_rows, o.C, 0, qflags, inv_mode, stream);
+        case QHAD_BLOCKS_T: return quant_block_had128_valid(o.x, 0, o.ldx, o.q, o.R * o.C, o.R, o.s, 0, grid, 1, 1, o.R, o.valid_rows, o.C, 1, qflags, inv_mode, stream);
+        case QHAD_COLUMNS: return quant_col_t_valid(o.x, o.ldx, o.q, o.R, o.s, reinterpret_cast<float*>(o.maxima), o.R, o.valid_rows, o.C, qflags | TI8_Q_HAD128, inv_mode, stream);
+        default: return ti8_quant_row(o.x, o.ldx, o.q, o.C, o.s, o.R, o.C, 0, qflags | TI8_Q_HAD128, inv_mode, stream);
+    }
+}
+
+int ti8::quant_had_call(const char* fn, const QHadOperand* operands, int count, int qflags, int inv_mode, ti8_stream_t stream) {
+    QMode mode;
+    if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
+    if (count < 0 || count > QHAD_MAX) return fail(TI8_ERR_MODE, "%s: unsupported set of operands", fn);
+    // those that read the same tensor behind each other, one with per-column scales (read again by its conversion) last
+    int order[QHAD_MAX], n = 0;
+    int64_t total = 0;
+    const void* last = nullptr;
+    for (int i = 0; i < count; ++i) {
+        const QHadOperand& o = operands[i];
+        if (!o.x || !o.q || !o.s || (o.kind == QHAD_COLUMNS && !o.maxima)) return fail(TI8_ERR_NULL, "%s: x, q, s and maxima are required", fn);
+        if (o.R <= 0 || o.C <= 0 || o.C % 128 || (o.kind != QHAD_ROWS && o.R % 128) || o.R > 0x3fffffff || o.C > 0x3fffffff || o.ldx < o.C || (o.kind == QHAD_ROWS && o.C > 32768))
+            return fail(TI8_ERR_SHAPE, "%s: bad operand of %lld x %lld", fn, (long long)o.R, (long long)o.C);
+        if (!aligned16(o.x) || !aligned16(o.q) || (o.ldx % 8)) return fail(TI8_ERR_ALIGN, "%s: pointers must be 16-byte aligned and strides multiples of 16 bytes", fn);
+        total += o.kind == QHAD_ROWS ? (o.C <= 4096 ? (o.R + 3) / 4 : o.R) : (o.R / 128) * (o.C / 128);
+        if (o.kind == QHAD_COLUMNS) last = o.x;
+    }
+    bool alone = count < 2 || total > 0x7fffffff;
+    for (int i = 0; i < count; ++i) alone = alone || (operands[i].kind == QHAD_ROWS && operands[i].C > 16384);     // (a row in 16 chunks per lane: twice the registers)
+    if (alone) {
+        for (int i = 0; i < count; ++i)
+            if (int e = quant_had_alone(operands[i], qflags, inv_mode, stream)) return e;
+        return TI8_OK;
+    }
+    for (int pass = 0; pass < 2; ++pass)
+        for (int i = 0; i < count; ++i) {
+            bool first = (operands[i].x == last) == (pass == 1);
+            for (int j = 0; j < i; ++j) first = first && operands[j].x != operands[i].x;
+            for (int j = i; first && j < count; ++j)
+                if (operands[j].x == operands[i].x && operands[j].kind != QHAD_COLUMNS) order[n++] = j;
+            for (int j = i; first && j < count; ++j)
+                if (operands[j].x == operands[i].x && operands[j].kind == QHAD_COLUMNS) order[n++] = j;
+        }
+    HadMulti m;
+    ClearRanges r = {};
+    int blocks = 0, columns = 0;
+    for (int i = 0; i < count; ++i) {
+        const QHadOperand& o = operands[order[i]];
+        m.op[i] = HadMultiOperand{static_cast<const uint16_t*>(o.x), o.q, o.s, o.maxima, o.ldx, o.kind == QHAD_BLOCKS || o.kind == QHAD_ROWS ? o.C : o.R, o.kind, (int)o.R, (int)o.C, (int)o.valid_rows};
+        m.first[i] = blocks;
+        blocks += (int)(o.kind == QHAD_ROWS ? (o.C <= 4096 ? (o.R + 3) / 4 : o.R) : (o.R / 128) * (o.C / 128));
+        if (o.kind == QHAD_COLUMNS) {
+            if (columns == 3) return fail(TI8_ERR_MODE, "%s: unsupported set of operands", fn);
+            r.p[columns] = o.maxima;
+            r.n[columns++] = (int)o.C;
+        }
+    }
+    for (int i = count; i < QHAD_MAX; ++i) { m.op[i] = m.op[0]; m.first[i] = 0x7fffffff; }
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (columns) clear(r, st);
+    hipLaunchKernelGGL(quant_had_multi_kernel, dim3((unsigned)blocks), dim3(256), 0, st, m, mode);
+    for (int i = 0; i < count; ++i) {
+        const HadMultiOperand& o = m.op[i];
+        if (o.kind == QHAD_COLUMNS)
+            hipLaunchKernelGGL((quant_block_had_kernel<true, HAD_COL>), dim3((unsigned)((o.R / 128) * (o.C / 128))), dim3(256), 0, st, o.x, (int64_t)0, o.ldx,
+                               o.q, (int64_t)0, o.ldq, o.s, (int64_t)0, (int64_t)0, (int64_t)0, o.R / 128, o.C / 128, o.valid_rows, mode, o.ws);
+    }
+    return check_launch(fn);
 }
 
 extern "C" int ti8_quant_block_multi(const ti8_qblock_operand* operands, int count, int qflags, int inv_mode, ti8_stream_t stream) {

@@ -231,8 +231,11 @@ struct Operands {
     int nblocks = 0, nboth = 0;
     QRowOperand rows;
     bool by_rows = false;
+    QHadOperand rotated[QHAD_MAX];      // with H_128: all of them
+    int nrotated = 0;
 };
 int quantise_operands(const char* fn, const Layer& L, const Operands& o, ti8_stream_t stream) {
+    if (o.nrotated) return quant_had_call(fn, o.rotated, o.nrotated, TI8_Q_CLAMP, TI8_INV_RCP_OF_SCALE, stream);
     return quant_call(fn, o.by_block, o.by_block_rows, o.nblocks, o.both, o.nboth, o.by_rows ? &o.rows : nullptr, TI8_Q_CLAMP,
                       L.dbl() ? TI8_INV_AMAX_DIV_127 : TI8_INV_RCP_OF_SCALE, stream);
 }
@@ -242,7 +245,7 @@ int quantise_operands(const char* fn, const Layer& L, const Operands& o, ti8_str
 int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* count, ti8_stream_t stream) {
     const ti8_linear_args& a = *L.a;
     const int64_t T = L.T, K = L.K, N = L.N, tok = L.tokens;
-    const int q = TI8_Q_CLAMP, had = L.had == 128 ? TI8_Q_HAD128 : 0;
+    const int q = TI8_Q_CLAMP;
     const int inv = L.dbl() ? TI8_INV_AMAX_DIV_127 : TI8_INV_RCP_OF_SCALE;
     const bool shared = L.shares();
     unsigned int* mx = L.maxima;
@@ -263,6 +266,9 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
         if (raw) partial = reinterpret_cast<unsigned int*>(oq);
         o.both[o.nboth++] = QRowColOperand{x, ldx, oq, os, oqT, osT, scratch, partial, R, valid, C, raw};
     };
+    auto rotated = [&](int kind, const void* x, int64_t ldx, int8_t* oq, float* os, int64_t R, int64_t valid, int64_t C, float* maxima = nullptr) {
+        o.rotated[o.nrotated++] = QHadOperand{x, ldx, oq, os, R, valid, C, kind, reinterpret_cast<unsigned int*>(maxima)};
+    };
     auto block = [&](const ti8_qblock_operand& operand, int64_t valid) {
         o.by_block_rows[o.nblocks] = valid;
         o.by_block[o.nblocks++] = operand;
@@ -276,8 +282,8 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
     if (L.fwd) {
         float post = 0.0f;
         if (L.block() && L.had) {
-            if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xq, T * K, K, L.xs, 0, K / 128, 1, 1, T, tok, K, 0, q, inv, stream)) return e;
-            if (!L.given_w()) if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q | had, inv, stream)) return e;
+            rotated(QHAD_BLOCKS, a.X, a.ldx, L.xq, L.xs, T, tok, K);
+            if (!L.given_w()) rotated(QHAD_ROWS, a.W, a.ldw, L.wq, L.ws, N, N, K);
         } else if (L.block()) {
             if (!L.input_of) block(blocks(a.X, a.ldx, L.xq, shared ? L.xtq : nullptr, L.xs, T, K), tok);
             if (shared) row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K, a.dW, a.lddw);     // rows for Y, columns for dX
@@ -285,8 +291,8 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
                 if (int e = ti8_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, 0, q, inv, stream)) return e;
         } else if (L.row_block()) {
             if (L.had) {
-                if (int e = ti8_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, 0, q | had, inv, stream)) return e;
-                if (!L.given_w()) if (int e = ti8_quant_block_had128(a.W, 0, a.ldw, L.wq, N * K, K, L.ws, 0, K / 128, 1, 1, N, K, 0, q, inv, stream)) return e;
+                rotated(QHAD_ROWS, a.X, a.ldx, L.xq, L.xs, tok, tok, K);
+                if (!L.given_w()) rotated(QHAD_BLOCKS, a.W, a.ldw, L.wq, L.ws, N, N, K);
             } else {
                 o.rows = QRowOperand{a.X, a.ldx, L.xq, L.xs, tok, K};
                 o.by_rows = true;
@@ -315,10 +321,10 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
         auto grid_t = [](int64_t cols, int64_t* rs, int64_t* ks, int* mode) { *rs = 1; *ks = cols / 128; *mode = TI8_SCALE_BLOCK128; };
         if (L.block() && L.had) {
             // H_128 along N for dX, along the tokens for dW: two differently rotated copies
-            if (int e = quant_block_had128_valid(a.dY, 0, a.lddy, L.dq, T * N, N, L.ds, 0, N / 128, 1, 1, T, tok, N, 0, q, inv, stream)) return e;
-            if (int e = quant_col_t_valid(a.W, a.ldw, L.wtq, N, L.wts, take_maxima(K), N, N, K, q | had, inv, stream)) return e;
-            if (int e = quant_block_had128_valid(a.dY, 0, a.lddy, L.dytq, T * N, T, L.dyts, 0, N / 128, 1, 1, T, tok, N, 1, 0, inv, stream)) return e;
-            if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xtq, T * K, T, L.xts, 0, K / 128, 1, 1, T, tok, K, 1, 0, inv, stream)) return e;
+            rotated(QHAD_BLOCKS, a.dY, a.lddy, L.dq, L.ds, T, tok, N);
+            rotated(QHAD_COLUMNS, a.W, a.ldw, L.wtq, L.wts, N, N, K, take_maxima(K));
+            rotated(QHAD_BLOCKS_T, a.dY, a.lddy, L.dytq, L.dyts, T, tok, N);
+            rotated(QHAD_BLOCKS_T, a.X, a.ldx, L.xtq, L.xts, T, tok, K);
         } else if (L.block()) {
             block(blocks(a.dY, a.lddy, L.dq, L.dytq, L.ds, T, N), tok);
             if (!shared) {
@@ -326,10 +332,10 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
                 block(blocks(a.X, a.ldx, nullptr, L.xtq, L.xts, T, K), tok);
             }
         } else if (L.row_block() && L.had) {
-            if (int e = ti8_quant_row(a.dY, a.lddy, L.dq, N, L.ds, tok, N, 0, q | had, inv, stream)) return e;
-            if (int e = ti8_quant_block_had128(a.W, 0, a.ldw, L.wtq, N * K, N, L.wts, 0, K / 128, 1, 1, N, K, 1, q, inv, stream)) return e;
-            if (int e = quant_col_t_valid(a.dY, a.lddy, L.dytq, T, L.dyts, take_maxima(N), T, tok, N, q | had, inv, stream)) return e;
-            if (int e = quant_block_had128_valid(a.X, 0, a.ldx, L.xtq, T * K, T, L.xts, 0, K / 128, 1, 1, T, tok, K, 1, q, inv, stream)) return e;
+            rotated(QHAD_ROWS, a.dY, a.lddy, L.dq, L.ds, tok, tok, N);
+            rotated(QHAD_BLOCKS_T, a.W, a.ldw, L.wtq, L.wts, N, N, K);
+            rotated(QHAD_COLUMNS, a.dY, a.lddy, L.dytq, L.dyts, T, tok, N, take_maxima(N));
+            rotated(QHAD_BLOCKS_T, a.X, a.ldx, L.xtq, L.xts, T, tok, K);
         } else if (L.row_block()) {
             row_col(a.dY, a.lddy, L.dq, L.ds, L.dytq, L.dyts, T, tok, N, a.Y, a.ldy);
             if (!shared) block(blocks(a.W, a.ldw, nullptr, L.wtq, L.wts, N, K), N);

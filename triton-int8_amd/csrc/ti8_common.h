@@ -95,6 +95,20 @@ struct QRowOperand {
 // are none of the second kind
 int quant_call(const char* fn, const ti8_qblock_operand* blocks, const int64_t* block_rows, int nblocks, const QRowColOperand* both, int nboth,
                const QRowOperand* rows, int qflags, int inv_mode, ti8_stream_t stream);
+// An operand rotated by H_128 and quantised, dense codes: by 128 x 128 blocks or by rows, rotated along the rows of x [R][C]; by blocks of x^T or by
+// the columns of x (`maxima`: C words of scratch), rotated along the columns, q [C][R].  Up to QHAD_MAX of them in a launch (a clearing one and a
+// conversion more with columns)
+enum { QHAD_BLOCKS = 0, QHAD_BLOCKS_T = 1, QHAD_COLUMNS = 2, QHAD_ROWS = 3, QHAD_MAX = 6 };
+struct QHadOperand {
+    const void* x;
+    int64_t ldx;
+    int8_t* q;
+    float* s;
+    int64_t R, valid_rows, C;       // by rows: R rows
+    int kind;
+    unsigned int* maxima;
+};
+int quant_had_call(const char* fn, const QHadOperand* operands, int count, int qflags, int inv_mode, ti8_stream_t stream);
 int quant_col_t_valid(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt, float* s, float* ws, int64_t R, int64_t valid_rows, int64_t C,
                       int qflags, int inv_mode, ti8_stream_t stream);
 int quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq, float* s, int64_t ssb, int64_t ssr,
