@@ -110,12 +110,26 @@ def test_rotated_operands_in_one_launch(dev, monkeypatch, scheme, tokens, k, n):
     import triton_int8_amd as T
     g = make_gen(tokens + k + n)
     X, W, dY = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev), randn_bf16(g, tokens, n, std=1e-3).to(dev)
+    _against_entry_points(T, monkeypatch, X, W, dY, scheme, 128)
+
+
+def _against_entry_points(T, monkeypatch, X, W, dY, scheme, hadamard):
     x, w = X.clone().requires_grad_(True), W.clone().requires_grad_(True)
 
     def results():
-        y = T.Int8LinearFunction.apply(x, w, None, scheme, 128)
-        return (*T.linear_fwd_bwd(X, W, dY, scheme, 128), y.detach(), *torch.autograd.grad(y, (x, w), dY))
+        y = T.Int8LinearFunction.apply(x, w, None, scheme, hadamard)
+        return (*T.linear_fwd_bwd(X, W, dY, scheme, hadamard), y.detach(), *torch.autograd.grad(y, (x, w), dY))
     got = results()
     monkeypatch.setattr(T.linear, "ONE_CALL_STEP", False)
     for a, b in zip(got, results()):
         assert torch.equal(a, b)
+
+
+# rotated over whole rows: lengths on either kernel, powers of two and between, one for all and all different, missing tokens, 32768 elements, and more
+# than the transposed copies are made together for
+@pytest.mark.parametrize("tokens,k,n", [(1, 128, 128), (200, 2944, 1152), (40, 4096, 5760), (130, 8192, 4096), (20, 32768, 128), (4100, 16384, 1024)])
+def test_rotated_rows_in_one_launch(dev, monkeypatch, tokens, k, n):
+    import triton_int8_amd as T
+    g = make_gen(tokens + k + n)
+    X, W, dY = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev), randn_bf16(g, tokens, n, std=1e-3).to(dev)
+    _against_entry_points(T, monkeypatch, X, W, dY, "double_channel", "full")

@@ -173,18 +173,16 @@ __device__ __forceinline__ void lane_butterflies(float (&a)[16], const LaneStage
 // with the quantiser's own arithmetic on the same bf16-rounded values: the rotated operand never
 // goes to HBM (3 bytes per element instead of 4 + 3).
 template <int NT, bool QUANT>
-__global__ __launch_bounds__(NT) void fwht_kernel(const uint16_t* __restrict__ x, int64_t ldx,
-                                                   uint16_t* __restrict__ y, int64_t ldy, int cols, int logn,
-                                                   int L, float scale, int8_t* __restrict__ q, int64_t ldq,
-                                                   float* __restrict__ s, QMode mode) {
-    extern __shared__ float lds[];
+__device__ __forceinline__ void fwht_part(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy, int cols, int logn,
+                                          int L, float scale, int8_t* __restrict__ q, int64_t ldq, float* __restrict__ s, const QMode& mode,
+                                          const int block, float* lds) {
     const int tid = threadIdx.x;
     // cols < L: one zero-extended row per workgroup (a length that is no power of two, transformed as the next power of
     // two and cut back): elements from `valid` on read as zero and are not stored
     const int valid = cols < L ? cols : L;
     const int segs_per_row = cols < L ? 1 : cols / L;
-    const uint16_t* xr = x + idx::fwht_segment_offset(blockIdx.x, segs_per_row, ldx, L);
-    uint16_t* yr = y + idx::fwht_segment_offset(blockIdx.x, segs_per_row, ldy, L);
+    const uint16_t* xr = x + idx::fwht_segment_offset(block, segs_per_row, ldx, L);
+    uint16_t* yr = y + idx::fwht_segment_offset(block, segs_per_row, ldy, L);
 
     // Segments of 1024 elements and more: bits 0..3 in registers and bits 4..9 across the lanes of a wave, whose 64 lanes
     // hold 64 consecutive chunks (in the order lane_stages wants), then one pass through LDS for what is left.
@@ -275,7 +273,7 @@ __global__ __launch_bounds__(NT) void fwht_kernel(const uint16_t* __restrict__ x
         for (int w = 1; w < NT / 64; ++w) amax = fmaxf(amax, lds[w]);
         amax = amax_floor(amax, mode.eps_add);
         const float mult = 127.0f / amax;
-        const int64_t row = blockIdx.x;
+        const int64_t row = block;
         if (tid == 0) s[row] = stored_scale(amax, mult, mode);
         int8_t* qr = q + row * ldq;
 #pragma unroll
@@ -313,18 +311,17 @@ __global__ __launch_bounds__(NT) void fwht_kernel(const uint16_t* __restrict__ x
 // bf16, or 4 bytes of int8 behind the row's absmax when QUANT): there is no read-back pass, and the exchange buffer is
 // 16 KiB (two of them, so that one barrier per slice is enough) whatever the length.  Same stage order, same roundings as
 // fwht_kernel: bit-identical.
+constexpr int FWHT_ROW_BUF = 4 * 64 * 16;                 // one slice: 4 waves x 64 chunk positions x 16 values (idx::fwht_row_lds)
+constexpr int fwht_row_words(int CH) { return (CH > 1 ? 2 : 1) * FWHT_ROW_BUF; }      // (one buffer and a second barrier per slice measured the same)
 template <int CH, bool QUANT>
-__global__ __launch_bounds__(256) void fwht_row_kernel(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y,
-                                                       int64_t ldy, int cols, float scale, int8_t* __restrict__ q, int64_t ldq,
-                                                       float* __restrict__ s, QMode mode) {
-    constexpr int L = 4096 * CH;
-    constexpr int BUF = 4 * 64 * 16;                      // one slice: 4 waves x 64 chunk positions x 16 values (idx::fwht_row_lds)
-    __shared__ __attribute__((aligned(16))) float xbuf[(CH > 1 ? 2 : 1) * BUF];   // (one buffer and a second barrier per slice measured the same)
+__device__ __forceinline__ void fwht_row_part(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy, int cols, float scale,
+                                              int8_t* __restrict__ q, int64_t ldq, float* __restrict__ s, const QMode& mode, const int block, float* xbuf) {
+    constexpr int L = 4096 * CH, BUF = FWHT_ROW_BUF;
     const int tid = threadIdx.x, lane = tid & 63;
     const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int valid = cols < L ? cols : L;                // cols < L: one zero-extended row per workgroup
     const int segs_per_row = cols < L ? 1 : cols / L;
-    const uint16_t* xr = x + idx::fwht_segment_offset(blockIdx.x, segs_per_row, ldx, L);
+    const uint16_t* xr = x + idx::fwht_segment_offset(block, segs_per_row, ldx, L);
     const LaneStages st = lane_stages(lane, 6);
     const int lp = (lane & ~15) | idx::had_chunk(lane & 15);   // this lane's chunk among the 64 of its wave's 1024 elements
 
@@ -413,7 +410,7 @@ __global__ __launch_bounds__(256) void fwht_row_kernel(const uint16_t* __restric
             o[k][ws] = make_uint2(pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]));
         }
     if (!QUANT) {
-        uint16_t* yr = y + idx::fwht_segment_offset(blockIdx.x, segs_per_row, ldy, L);
+        uint16_t* yr = y + idx::fwht_segment_offset(block, segs_per_row, ldy, L);
 #pragma unroll
         for (int k = 0; k < CH; ++k)
 #pragma unroll
@@ -441,7 +438,7 @@ __global__ __launch_bounds__(256) void fwht_row_kernel(const uint16_t* __restric
     amax = fmaxf(fmaxf(xbuf[0], xbuf[1]), fmaxf(xbuf[2], xbuf[3]));
     amax = amax_floor(amax, mode.eps_add);
     const float mult = 127.0f / amax;
-    const int64_t row = blockIdx.x;
+    const int64_t row = block;
     if (tid == 0) s[row] = stored_scale(amax, mult, mode);
     // everything this thread holds came from chunk position lp of some wave and slice, so it carries this lane's sign
     const float lane_mult = mult * st.sign;
@@ -458,6 +455,45 @@ __global__ __launch_bounds__(256) void fwht_row_kernel(const uint16_t* __restric
             v = put_u8(qbiased(bf16_hi(o[k][ws].y), lane_mult), 3, v);
             *reinterpret_cast<uint32_t*>(qr + first) = v ^ UNBIAS4;
         }
+}
+
+template <int NT, bool QUANT>
+__global__ __launch_bounds__(NT) void fwht_kernel(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy, int cols, int logn,
+                                                  int L, float scale, int8_t* __restrict__ q, int64_t ldq, float* __restrict__ s, QMode mode) {
+    extern __shared__ float lds[];
+    fwht_part<NT, QUANT>(x, ldx, y, ldy, cols, logn, L, scale, q, ldq, s, mode, (int)blockIdx.x, lds);
+}
+
+template <int CH, bool QUANT>
+__global__ __launch_bounds__(256) void fwht_row_kernel(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy, int cols,
+                                                       float scale, int8_t* __restrict__ q, int64_t ldq, float* __restrict__ s, QMode mode) {
+    __shared__ __attribute__((aligned(16))) float xbuf[fwht_row_words(CH)];
+    fwht_row_part<CH, QUANT>(x, ldx, y, ldy, cols, scale, q, ldq, s, mode, (int)blockIdx.x, xbuf);
+}
+
+// Rows of several tensors, of the same length, in one launch: those of a layer call.  Operand i has the workgroups from first[i] on (past the last
+// operand: none).
+struct FwhtMulti {
+    struct { const uint16_t* x; int8_t* q; float* s; int64_t ldx; } op[QFWHT_MAX];      // codes dense
+    int first[QFWHT_MAX];
+};
+__device__ __forceinline__ int fwht_operand(const int (&first)[QFWHT_MAX]) {
+    int i = 0;
+#pragma unroll
+    for (int k = 1; k < QFWHT_MAX; ++k)
+        if ((int)blockIdx.x >= first[k]) i = k;
+    return i;
+}
+__global__ __launch_bounds__(256) void fwht_multi_kernel(const FwhtMulti m, int cols, int logn, int L, QMode mode) {
+    extern __shared__ float lds[];
+    const int i = fwht_operand(m.first);
+    fwht_part<256, true>(m.op[i].x, m.op[i].ldx, nullptr, 0, cols, logn, L, 1.0f, m.op[i].q, cols, m.op[i].s, mode, (int)blockIdx.x - m.first[i], lds);
+}
+template <int CH>
+__global__ __launch_bounds__(256) void fwht_row_multi_kernel(const FwhtMulti m, int cols, QMode mode) {
+    __shared__ __attribute__((aligned(16))) float xbuf[fwht_row_words(CH)];
+    const int i = fwht_operand(m.first);
+    fwht_row_part<CH, true>(m.op[i].x, m.op[i].ldx, nullptr, 0, cols, 1.0f, m.op[i].q, cols, m.op[i].s, mode, (int)blockIdx.x - m.first[i], xbuf);
 }
 
 // ---- transposed input: y[c][r] = sum_r' H[r][r'] x[r'][c], i.e. the transform of x^T along its
@@ -557,10 +593,9 @@ __global__ __launch_bounds__(NT) void fwht_t_kernel(const uint16_t* __restrict__
 // bf16 transpose, 64 x 64 tiles through LDS: x [R][C] -> y [C][R], 16-byte loads and stores.
 // Thread t reads 8 consecutive columns of row (t / 8) + 32 h; the tile is kept as 32-bit words of
 // two ROWS' elements so that a thread later picks up 8 consecutive rows of one column with 4 reads.
-__global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y,
-                                                             int64_t ldy, int tiles_c, int64_t valid_rows) {
-    __shared__ uint16_t tile[64][64 + 2];   // +2: rows 4 bytes apart modulo the banks
-    const int tc = blockIdx.x % tiles_c, tr = blockIdx.x / tiles_c;
+__device__ __forceinline__ void transpose_bf16_part(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y, int64_t ldy, int tiles_c,
+                                                    int64_t valid_rows, const int block, uint16_t (&tile)[64][64 + 2]) {      // +2: rows 4 bytes apart modulo the banks
+    const int tc = block % tiles_c, tr = block / tiles_c;
     const int tid = threadIdx.x;
 #pragma unroll
     for (int h = 0; h < 2; ++h) {
@@ -583,6 +618,20 @@ __global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t* __r
         __builtin_memcpy(&v, e, 16);
         *reinterpret_cast<uint4*>(y + ((int64_t)tc * 64 + c) * ldy + (int64_t)tr * 64 + r) = v;
     }
+}
+__global__ __launch_bounds__(256) void transpose_bf16_kernel(const uint16_t* __restrict__ x, int64_t ldx, uint16_t* __restrict__ y,
+                                                             int64_t ldy, int tiles_c, int64_t valid_rows) {
+    __shared__ uint16_t tile[64][64 + 2];
+    transpose_bf16_part(x, ldx, y, ldy, tiles_c, valid_rows, (int)blockIdx.x, tile);
+}
+struct TransposeMulti {
+    struct { const uint16_t* x; uint16_t* y; int64_t ldx; int R, tiles_c, valid_rows; } op[QFWHT_MAX];      // y [C][R] dense
+    int first[QFWHT_MAX];
+};
+__global__ __launch_bounds__(256) void transpose_bf16_multi_kernel(const TransposeMulti m) {
+    __shared__ uint16_t tile[64][64 + 2];
+    const int i = fwht_operand(m.first);
+    transpose_bf16_part(m.op[i].x, m.op[i].ldx, m.op[i].y, m.op[i].R, m.op[i].tiles_c, m.op[i].valid_rows, (int)blockIdx.x - m.first[i], tile);
 }
 
 }  // namespace ti8
@@ -739,6 +788,81 @@ int ti8::fwht_t_quant_row_valid(const void* x, int64_t ldx, void* scratch, int8_
                        static_cast<const uint16_t*>(x), ldx, static_cast<uint16_t*>(scratch), R, (int)(C / 64), valid_rows);
     if (int e = check_launch(fn)) return e;
     return ti8_fwht_quant_row(scratch, R, q, ldq, s, C, R, n, qflags, inv_mode, stream);
+}
+
+int64_t ti8::next_pow2_128(int64_t v) {
+    int64_t n = 128;
+    while (n < v) n <<= 1;
+    return n;
+}
+
+// The transposes of a call are a launch, and the rows of one length are another: a step's nine launches become two to four, which up to a few
+// thousand tokens is what it waits for.  Steps, us, apart / so: 128 tokens, 4096 -> 1024 63.0 / 49.6, 1024, 2048 -> 1024 64.8 / 46.5, 4096, 4096 ->
+// 4096 319 / 304, 8192, 4096 -> 4096 581 / 555.
+int ti8::quant_fwht_call(const char* fn, const QFwhtOperand* operands, int count, bool together, int qflags, int inv_mode, ti8_stream_t stream) {
+    if (count < 0 || count > QFWHT_MAX) return fail(TI8_ERR_MODE, "%s: unsupported set of operands", fn);
+    QMode mode;
+    if (int e = parse_mode(qflags, inv_mode, &mode)) return e;
+    int64_t tiles = 0, rows = 0;
+    for (int i = 0; i < count; ++i) {
+        const QFwhtOperand& o = operands[i];
+        if (!o.x || !o.q || !o.s || (o.transposed && !o.scratch)) return fail(TI8_ERR_NULL, "%s: x, q, s and scratch are required", fn);
+        const int64_t length = o.transposed ? o.R : o.C;
+        if (o.R <= 0 || o.C <= 0 || o.R > 0x3fffffff || o.C > 0x3fffffff || length % 128 || length > 32768 || (o.transposed && o.C % 64) || o.ldx < o.C)
+            return fail(TI8_ERR_SHAPE, "%s: bad operand of %lld x %lld", fn, (long long)o.R, (long long)o.C);
+        if (!aligned16(o.x) || !aligned16(o.q) || !aligned16(o.scratch) || (o.ldx % 8)) return fail(TI8_ERR_ALIGN, "%s: pointers must be 16-byte aligned and strides multiples of 16 bytes", fn);
+        if (o.transposed) tiles += (o.R / 64) * (o.C / 64);
+        rows += o.transposed ? o.C : o.R;
+    }
+    if (!together || count < 2 || tiles > 0x3fffffff || rows > 0x3fffffff) {
+        for (int i = 0; i < count; ++i) {
+            const QFwhtOperand& o = operands[i];
+            if (int e = o.transposed ? fwht_t_quant_row_valid(o.x, o.ldx, o.scratch, o.q, o.R, o.s, o.R, o.valid_rows, o.C, qflags, inv_mode, stream)
+                                     : ti8_fwht_quant_row(o.x, o.ldx, o.q, o.C, o.s, o.R, o.C, next_pow2_128(o.C), qflags, inv_mode, stream)) return e;
+        }
+        return TI8_OK;
+    }
+    hipStream_t st = static_cast<hipStream_t>(stream);
+    if (tiles) {
+        TransposeMulti m;
+        int n = 0, blocks = 0;
+        for (int i = 0; i < count; ++i) {
+            const QFwhtOperand& o = operands[i];
+            if (!o.transposed) continue;
+            m.op[n] = {static_cast<const uint16_t*>(o.x), static_cast<uint16_t*>(o.scratch), o.ldx, (int)o.R, (int)(o.C / 64), (int)o.valid_rows};
+            m.first[n++] = blocks;
+            blocks += (int)((o.R / 64) * (o.C / 64));
+        }
+        for (int i = n; i < QFWHT_MAX; ++i) { m.op[i] = m.op[0]; m.first[i] = 0x7fffffff; }
+        hipLaunchKernelGGL(transpose_bf16_multi_kernel, dim3((unsigned)blocks), dim3(256), 0, st, m);
+        if (int e = check_launch(fn)) return e;
+    }
+    bool done[QFWHT_MAX] = {};
+    for (int i = 0; i < count; ++i) {
+        if (done[i]) continue;
+        const int64_t cols = operands[i].transposed ? operands[i].R : operands[i].C, n = next_pow2_128(cols);
+        FwhtMulti m;
+        int used = 0, blocks = 0;
+        for (int j = i; j < count; ++j) {
+            const QFwhtOperand& o = operands[j];
+            if (done[j] || (o.transposed ? o.R : o.C) != cols) continue;
+            done[j] = true;
+            m.op[used] = {static_cast<const uint16_t*>(o.transposed ? o.scratch : o.x), o.q, o.s, o.transposed ? o.R : o.ldx};
+            m.first[used++] = blocks;
+            blocks += (int)(o.transposed ? o.C : o.R);
+        }
+        for (int k = used; k < QFWHT_MAX; ++k) { m.op[k] = m.op[0]; m.first[k] = 0x7fffffff; }
+        const dim3 grid((unsigned)blocks), block(256);
+        int logn = 0;
+        while ((1LL << logn) < n) ++logn;
+        if (n < 4096) hipLaunchKernelGGL(fwht_multi_kernel, grid, block, (size_t)idx::fwht_lds_words(n) * sizeof(float), st, m, (int)cols, logn, (int)n, mode);
+        else if (n == 4096) hipLaunchKernelGGL((fwht_row_multi_kernel<1>), grid, block, 0, st, m, (int)cols, mode);
+        else if (n == 8192) hipLaunchKernelGGL((fwht_row_multi_kernel<2>), grid, block, 0, st, m, (int)cols, mode);
+        else if (n == 16384) hipLaunchKernelGGL((fwht_row_multi_kernel<4>), grid, block, 0, st, m, (int)cols, mode);
+        else hipLaunchKernelGGL((fwht_row_multi_kernel<8>), grid, block, 0, st, m, (int)cols, mode);
+        if (int e = check_launch(fn)) return e;
+    }
+    return TI8_OK;
 }
 
 extern "C" int ti8_fwht_t_quant_row(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t C,

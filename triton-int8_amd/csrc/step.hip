@@ -21,6 +21,8 @@ struct Carver {
     }
 };
 
+constexpr int64_t ROTATE_TOGETHER_BYTES = (int64_t)192 << 20;
+
 // One call: its arguments with the token dim rounded up, and where every operand lives.
 struct Layer {
     const ti8_linear_args* a;
@@ -52,6 +54,9 @@ struct Layer {
     // R + C maxima, and the partial ones behind them where those are collected there
     int64_t partial_words(int64_t R, int64_t C) const { return partials_in_outputs || !quant_together(both_ways_bytes()) ? 0 : maxima_piece(quant_maxima_words(R, C)); }
     int64_t both_ways_words(int64_t R, int64_t C) const { return maxima_piece(R + C) + partial_words(R, C); }
+    // whether the transposed copies in front of the rotations are made together (quant_fwht_call): while they find room in the Infinity Cache, and
+    // in a workspace of about the operands' size (8192 tokens, 8192 -> 8192 takes 1807 us either way)
+    bool rotates_together() const { return 2 * (N * K + T * N + T * K) <= ROTATE_TOGETHER_BYTES; }
     // what an unrotated forward quantises for the backward in the same pass
     bool shares() const { return had == 0 && (keep || (fwd && bwd)); }
     bool given_w() const { return a->wq != nullptr; }
@@ -106,7 +111,7 @@ struct Layer {
                 int64_t big = N * K;
                 if (T * N > big) big = T * N;
                 if (T * K > big) big = T * K;
-                scratch = w.take<uint16_t>(big);
+                scratch = w.take<uint16_t>(rotates_together() ? N * K + T * N + T * K : big);
             }
         }
         // maxima: W by rows and columns in the forward (or W by columns in a backward that found nothing saved), dY and, for
@@ -215,12 +220,6 @@ bool step_apart(const ti8_linear_args& a, int64_t T) {
     return outputs_apart(a, T);
 }
 
-int64_t next_pow2(int64_t v) {
-    int64_t n = 128;
-    while (n < v) n <<= 1;
-    return n;
-}
-
 // Operands that go into the two quantiser launches of a call: without a rotation, those quantised by blocks and those quantised by rows and by
 // columns, without a launch that only clears maxima (quant_call: 16 tokens, 4096 -> 4096, block-channel 41 -> 37.6 us; 3072 tokens
 // row-block 210 -> 204)
@@ -233,8 +232,11 @@ struct Operands {
     bool by_rows = false;
     QHadOperand rotated[QHAD_MAX];      // with H_128: all of them
     int nrotated = 0;
+    QFwhtOperand whole[QFWHT_MAX];      // with the rotation over whole rows: likewise
+    int nwhole = 0;
 };
 int quantise_operands(const char* fn, const Layer& L, const Operands& o, ti8_stream_t stream) {
+    if (o.nwhole) return quant_fwht_call(fn, o.whole, o.nwhole, L.rotates_together(), TI8_Q_CLAMP, TI8_INV_AMAX_DIV_127, stream);
     if (o.nrotated) return quant_had_call(fn, o.rotated, o.nrotated, TI8_Q_CLAMP, TI8_INV_RCP_OF_SCALE, stream);
     return quant_call(fn, o.by_block, o.by_block_rows, o.nblocks, o.both, o.nboth, o.by_rows ? &o.rows : nullptr, TI8_Q_CLAMP,
                       L.dbl() ? TI8_INV_AMAX_DIV_127 : TI8_INV_RCP_OF_SCALE, stream);
@@ -269,6 +271,9 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
     auto rotated = [&](int kind, const void* x, int64_t ldx, int8_t* oq, float* os, int64_t R, int64_t valid, int64_t C, float* maxima = nullptr) {
         o.rotated[o.nrotated++] = QHadOperand{x, ldx, oq, os, R, valid, C, kind, reinterpret_cast<unsigned int*>(maxima)};
     };
+    auto whole = [&](const void* x, int64_t ldx, int8_t* oq, float* os, int64_t R, int64_t valid, int64_t C, uint16_t* scratch = nullptr) {
+        o.whole[o.nwhole++] = QFwhtOperand{x, ldx, oq, os, R, valid, C, scratch != nullptr, scratch};
+    };
     auto block = [&](const ti8_qblock_operand& operand, int64_t valid) {
         o.by_block_rows[o.nblocks] = valid;
         o.by_block[o.nblocks++] = operand;
@@ -300,8 +305,8 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
             }
         } else if (L.had) {
             post = (float)(1.0 / (double)K);
-            if (int e = ti8_fwht_quant_row(a.X, a.ldx, L.xq, K, L.xs, tok, K, next_pow2(K), q, inv, stream)) return e;
-            if (!L.given_w()) if (int e = ti8_fwht_quant_row(a.W, a.ldw, L.wq, K, L.ws, N, K, next_pow2(K), q, inv, stream)) return e;
+            whole(a.X, a.ldx, L.xq, L.xs, tok, tok, K);
+            if (!L.given_w()) whole(a.W, a.ldw, L.wq, L.ws, N, N, K);
         } else if (shared) {
             row_col(a.X, a.ldx, L.xq, L.xs, L.xtq, L.xts, T, tok, K, a.dX, a.lddx);
             row_col(a.W, a.ldw, L.wq, L.ws, L.wtq, L.wts, N, N, K, a.dW, a.lddw);
@@ -344,10 +349,11 @@ int quantise(const char* fn, Layer& L, Operands& o, ti8_gemm_problem* g, int* co
             // the transposed operands are rotated along the rows of the tensors as they lie in memory
             post_dx = (float)(1.0 / (double)N);
             post_dw = (float)(1.0 / (double)T);
-            if (int e = ti8_fwht_quant_row(a.dY, a.lddy, L.dq, N, L.ds, tok, N, next_pow2(N), q, inv, stream)) return e;
-            if (int e = ti8_fwht_t_quant_row(a.W, a.ldw, L.scratch, L.wtq, N, L.wts, N, K, q, inv, stream)) return e;
-            if (int e = fwht_t_quant_row_valid(a.dY, a.lddy, L.scratch, L.dytq, T, L.dyts, T, tok, N, q, inv, stream)) return e;
-            if (int e = fwht_t_quant_row_valid(a.X, a.ldx, L.scratch, L.xtq, T, L.xts, T, tok, K, q, inv, stream)) return e;
+            const bool apart_scratch = L.rotates_together();
+            whole(a.dY, a.lddy, L.dq, L.ds, tok, tok, N);
+            whole(a.W, a.ldw, L.wtq, L.wts, N, N, K, L.scratch);
+            whole(a.dY, a.lddy, L.dytq, L.dyts, T, tok, N, L.scratch + (apart_scratch ? N * K : 0));
+            whole(a.X, a.ldx, L.xtq, L.xts, T, tok, K, L.scratch + (apart_scratch ? N * K + T * N : 0));
         } else {
             row_col(a.dY, a.lddy, L.dq, L.ds, L.dytq, L.dyts, T, tok, N, a.Y, a.ldy);
             if (!shared) {

@@ -114,6 +114,21 @@ int quant_col_t_valid(const void* x, int64_t ldx, int8_t* qT, int64_t ldqt, floa
 int quant_block_had128_valid(const void* x, int64_t bsx, int64_t ldx, int8_t* q, int64_t bsq, int64_t ldq, float* s, int64_t ssb, int64_t ssr,
                              int64_t ssc, int64_t B, int64_t R, int64_t valid_rows, int64_t C, int along_rows, int qflags, int inv_mode,
                              ti8_stream_t stream);
+// An operand rotated over the whole row by H and quantised by rows: x [R][C] (R its rows that exist), q [R][C]; or, `transposed`, x^T with x [R][C]
+// transposed into `scratch` first, q [C][R].  Codes dense; up to QFWHT_MAX of a call, `together` (each with scratch of its own) in a launch per
+// length and one for the transposes
+enum { QFWHT_MAX = 6 };
+struct QFwhtOperand {
+    const void* x;
+    int64_t ldx;
+    int8_t* q;
+    float* s;
+    int64_t R, valid_rows, C;
+    bool transposed;
+    void* scratch;
+};
+int64_t next_pow2_128(int64_t v);       // and at least 128
+int quant_fwht_call(const char* fn, const QFwhtOperand* operands, int count, bool together, int qflags, int inv_mode, ti8_stream_t stream);
 int fwht_t_quant_row_valid(const void* x, int64_t ldx, void* scratch, int8_t* q, int64_t ldq, float* s, int64_t R, int64_t valid_rows, int64_t C,
                            int qflags, int inv_mode, ti8_stream_t stream);
 // ti8_gemm_i8_nt with a bias, which the epilogue adds; y += bias behind the GEMMs of a whole step (bias.hip)
