@@ -389,13 +389,15 @@ constexpr int RAW_STRIP_Y = 16, RAW_STRIP_DX = 32;
 constexpr int RAW_PARTS = 32;
 TI8_HD int raw_part(int i, int lane, int count) { return imin((lane >> 4) + 4 * i, count - 1); }
 // Whether such a step takes them.  A workgroup walks the whole contraction, so a side much longer than the other leaves few of them with long
-// walks; and for a second block of 16 tokens the codes are read twice as often, which costs on a large weight what the saved launch gains.
+// walks; and for a second block of 16 tokens the codes are read twice as often, which costs what the saved launch gains, but on a small weight and
+// on one whose codes both ways no longer fit the Infinity Cache beside it.
 // The step, us, its weight quantised in memory / so: 16 tokens, 4096 -> 4096 37.7 / 32.5, 2048 -> 2048 22.3 / 17.3, 7936 -> 8960 177 / 132,
 // 13440 -> 3200 89.8 / 76.1, 3200 -> 13440 88.6 / 75.0, 10240 -> 1024 37.1 / 34.5, 14336 -> 1024 44.8 / 45.9, 2048 -> 14336 62.7 / 62.4, 1536
 // -> 8960 37.3 / 39.5, 1024 -> 14336 41.5 / 49.1; 32 tokens, 2048 -> 2048 22.3 / 17.2, 2560 -> 2560 26.8 / 22.4, 3072 -> 3072 29.3 / 29.0,
-// 5632 -> 4736 60.8 / 63.7.  (The double-channel step converts X and dY between the maxima and the GEMMs: 17 tokens, 5632 -> 4736 66 / 77.)
+// 5632 -> 4736 60.8 / 63.7, 4864 -> 8960 89.6 / 87.1, 14336 -> 4096 123 / 111, 6144 -> 10240 137 / 124, 5120 -> 13312 170 / 133, 11008 ->
+// 11008 291 / 262.  (The double-channel step converts X and dY between the maxima and the GEMMs: 17 tokens, 5632 -> 4736 66 / 77.)
 TI8_HD bool raw_weight_takes(int64_t tokens, int64_t K, int64_t N) {
-    return tokens <= 32 && (tokens <= 16 || N * K <= 2560 * 2560) && N <= 5 * K && K <= 10 * N && K <= 32768 && N <= 32768;
+    return tokens <= 32 && (tokens <= 16 || N * K <= 2560 * 2560 || N * K >= 14336 * 4096) && N <= 5 * K && K <= 10 * N && K <= 32768 && N <= 32768;
 }
 TI8_HD int64_t raw_row_offset(int n0, int64_t ldw, int kt, int i, int lane) { return (int64_t)(n0 + (lane & 15)) * ldw + kt * 128 + i * 32 + (lane >> 4) * 8; }
 TI8_HD int64_t raw_row_codes_offset(int token, int64_t lda, int kt, int i, int lane) { return (int64_t)token * lda + kt * 128 + i * 32 + (lane >> 4) * 8; }
