@@ -757,7 +757,7 @@ int walk_gemm(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t bsc, i
     for (int64_t by = 0; by < batch && !r.bad; ++by) {
         std::fill(tile_seen.begin(), tile_seen.end(), 0);
         for (int bx = 0; bx < tiles_m * tiles_n && !r.bad; ++bx) {
-            const TileCoord tc = gemm_tile_of(bx, tiles_m, tiles_n, GROUP);
+            const TileCoord tc = gemm_tile_of(bx, tiles_m, tiles_n, GROUP, false);
             if (tc.tile_m < 0 || tc.tile_m >= tiles_m || tc.tile_n < 0 || tc.tile_n >= tiles_n) {
                 r.fail("gemm: workgroup %d maps to tile (%d, %d) outside %d x %d", bx, tc.tile_m, tc.tile_n, tiles_m, tiles_n);
                 break;
@@ -909,7 +909,7 @@ int walk_gemm_chain(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t 
         for (int T = w; T < total && !r.bad; T += grid) {
             ++seen[(size_t)T];
             const int64_t by = T / per_batch;
-            const TileCoord tc = gemm_tile_of(T - (int)by * per_batch, tiles_m, tiles_n, GROUP);
+            const TileCoord tc = gemm_tile_of(T - (int)by * per_batch, tiles_m, tiles_n, GROUP, true);
             if (tc.tile_m < 0 || tc.tile_m >= tiles_m || tc.tile_n < 0 || tc.tile_n >= tiles_n) {
                 r.fail("gemm chain: tile %d maps to (%d, %d) outside %d x %d", T, tc.tile_m, tc.tile_n, tiles_m, tiles_n);
                 break;
@@ -1023,7 +1023,7 @@ int walk_gemm_mid(int64_t bsa, int64_t lda, int64_t bsb, int64_t ldb, int64_t bs
     for (int64_t by = 0; by < batch && !r.bad; ++by) {
         std::fill(tile_seen.begin(), tile_seen.end(), 0);
         for (int bx = 0; bx < tiles_m * tiles_n && !r.bad; ++bx) {
-            const TileCoord tc = gemm_tile_of(bx, tiles_m, tiles_n, gemm_group_rows(128));
+            const TileCoord tc = gemm_tile_of(bx, tiles_m, tiles_n, gemm_group_rows(128), false);
             if (tc.tile_m < 0 || tc.tile_m >= tiles_m || tc.tile_n < 0 || tc.tile_n >= tiles_n) {
                 r.fail("gemm mid: workgroup %d maps to tile (%d, %d) outside %d x %d", bx, tc.tile_m, tc.tile_n, tiles_m, tiles_n);
                 break;
@@ -1174,7 +1174,7 @@ int walk_gemm_tile_map(int tiles_m, int tiles_n, int group, int64_t* n_checked, 
             for (int i = m; i < imin(m + group, tiles_m); ++i) order[(size_t)(i * tiles_n + n)] = at++;
     for (int xcd = 0; xcd < 8; ++xcd)
         for (int w = xcd, last = -1; w < total && !r.bad; w += 8) {
-            const TileCoord t = gemm_tile_of(w, tiles_m, tiles_n, group);
+            const TileCoord t = gemm_tile_of(w, tiles_m, tiles_n, group, true);
             if (t.tile_m < 0 || t.tile_m >= tiles_m || t.tile_n < 0 || t.tile_n >= tiles_n) { r.fail("tile map: workgroup %d has (%d, %d)", w, t.tile_m, t.tile_n); break; }
             const int at = order[(size_t)(t.tile_m * tiles_n + t.tile_n)];
             ++seen[(size_t)at];
@@ -1182,8 +1182,13 @@ int walk_gemm_tile_map(int tiles_m, int tiles_n, int group, int64_t* n_checked, 
             last = at;
             ++r.checked;
         }
+    for (int w = 0; w < total && !r.bad; ++w) {      // a GEMM alone: every tile once
+        const TileCoord t = gemm_tile_of(w, tiles_m, tiles_n, group, false);
+        if (t.tile_m < 0 || t.tile_m >= tiles_m || t.tile_n < 0 || t.tile_n >= tiles_n) { r.fail("tile map: workgroup %d alone has (%d, %d)", w, t.tile_m, t.tile_n); break; }
+        ++seen[(size_t)order[(size_t)(t.tile_m * tiles_n + t.tile_n)]];
+    }
     for (int t = 0; t < total && !r.bad; ++t)
-        if (seen[(size_t)t] != 1) r.fail("tile map: tile %d is taken %d times", t, seen[(size_t)t]);
+        if (seen[(size_t)t] != 2) r.fail("tile map: tile %d is taken %d times in both", t, seen[(size_t)t]);
     *n_checked = r.checked;
     return r.bad;
 }

@@ -49,7 +49,7 @@ __device__ __forceinline__ void interleave_hint() {
 // One output tile of one GEMM: the whole kernel body.  `block_x` = index of the workgroup among the
 // tiles of this GEMM, `batch` = batch index.
 template <int BM, int BN, int WM, int WN, int EPI>
-__device__ __forceinline__ void gemm_i8_tile(const GemmArgs& g, const int block_x, const int batch) {
+__device__ __forceinline__ void gemm_i8_tile(const GemmArgs& g, const int block_x, const int batch, const bool several) {
     constexpr int NW = WM * WN;
     constexpr int TM = BM / WM / 32;  // 32x32 blocks per wave along M
     constexpr int TN = BN / WN / 32;
@@ -77,7 +77,7 @@ __device__ __forceinline__ void gemm_i8_tile(const GemmArgs& g, const int block_
     // share are about the same size (256-row tiles: 4 measured 0.4 % faster than 8 and 1 % faster
     // than 16 on 8192 x 4096 x 4096)
     constexpr int GROUP = idx::gemm_group_rows(BM);
-    const idx::TileCoord tc = idx::gemm_tile_of(block_x, g.tiles_m, g.tiles_n, GROUP);
+    const idx::TileCoord tc = idx::gemm_tile_of(block_x, g.tiles_m, g.tiles_n, GROUP, several);
     const int m0 = tc.tile_m * BM, n0 = tc.tile_n * BN;
 
     const int8_t* Ab = g.A + (int64_t)batch * g.bsa;
@@ -575,7 +575,7 @@ __device__ __forceinline__ void gemm_i8_tile(const GemmArgs& g, const int block_
 
 template <int BM, int BN, int WM, int WN, int EPI>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_kernel(const GemmArgs g) {
-    gemm_i8_tile<BM, BN, WM, WN, EPI>(g, blockIdx.x, blockIdx.y);
+    gemm_i8_tile<BM, BN, WM, WN, EPI>(g, blockIdx.x, blockIdx.y, false);
 }
 
 // Several GEMMs (batch of one each) in ONE launch: workgroup w computes tile w - first[i] of the
@@ -586,7 +586,7 @@ template <int BM, int BN, int WM, int WN, int EPI>
 __global__ __launch_bounds__(64 * WM * WN) void gemm_i8_multi_kernel(const GemmMulti m) {
     static_assert(GEMM_MULTI_MAX == 3, "gemm_multi_pick knows three ranges");
     const int i = idx::gemm_multi_pick((int)blockIdx.x, m.first[1], m.first[2], m.count);
-    gemm_i8_tile<BM, BN, WM, WN, EPI>(m.g[i], (int)blockIdx.x - m.first[i], 0);
+    gemm_i8_tile<BM, BN, WM, WN, EPI>(m.g[i], (int)blockIdx.x - m.first[i], 0, m.count > 1);
 }
 
 constexpr size_t tile_lds_bytes(int bm, int bn) { return 2 * (size_t)(bm + bn) * 128; }

@@ -125,7 +125,7 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         const int per_batch = g.tiles_m * g.tiles_n;
         // (divisions of uniform values come out of the vector unit: back into scalar registers)
         t.batch = __builtin_amdgcn_readfirstlane(local / per_batch);
-        const idx::TileCoord tc = idx::gemm_tile_of(local - t.batch * per_batch, g.tiles_m, g.tiles_n, GROUP);
+        const idx::TileCoord tc = idx::gemm_tile_of(local - t.batch * per_batch, g.tiles_m, g.tiles_n, GROUP, true);
         t.m0 = __builtin_amdgcn_readfirstlane(tc.tile_m) * BM;
         t.n0 = __builtin_amdgcn_readfirstlane(tc.tile_n) * BN;
         t.nk = g.K >> 7;

@@ -62,7 +62,7 @@ __global__ __launch_bounds__(64 * NW) void gemm_i8_mid_kernel(const GemmMulti m)
     const int gi = idx::gemm_multi_pick((int)blockIdx.x, m.first[1], m.first[2], m.count);
     const GemmArgs& g = m.g[gi];
     const int batch = blockIdx.y;
-    const idx::TileCoord tc = idx::gemm_tile_of((int)blockIdx.x - m.first[gi], g.tiles_m, g.tiles_n, idx::gemm_group_rows(BM));
+    const idx::TileCoord tc = idx::gemm_tile_of((int)blockIdx.x - m.first[gi], g.tiles_m, g.tiles_n, idx::gemm_group_rows(BM), m.count > 1);
     const int m0 = tc.tile_m * BM, n0 = tc.tile_n * BN;
     const int nk = g.K >> 7, klast = (nk - 1) * 128;
 

@@ -22,17 +22,20 @@ TI8_HD int imax(int a, int b) { return a > b ? a : b; }
 
 // ---- LDS-tiled GEMM (gemm.hip) -------------------------------------------------------------
 
-// workgroup id -> (tile_m, tile_n): one contiguous range of tiles per XCD (ids 8 apart share an
+// workgroup id -> (tile_m, tile_n): mostly one contiguous range of tiles per XCD (ids 8 apart share an
 // XCD; the first ones have a tile more where 8 does not divide their number), then groups of `group` tile rows walked column by
 // column inside a group.  (In their own order, those numbers spread neighbours over all XCDs: three GEMMs of a step in one launch, int32,
 // 512 tokens 2176 -> 4992 40.3 us, 34.6 this way; 640, 8320 -> 1408 55.9 / 48.3; 1152, 8832 -> 3584 135 / 127; 3712, 7168 -> 8320
-// 588 / 570; 13056, 7168 -> 11648 2680 / 2637.)
+// 588 / 570; 13056, 7168 -> 11648 2680 / 2637.  But a GEMM alone on up to 512 tiles of 128 rows, about two per CU, is faster when the XCDs read
+// the same panel of B at the same time: 1144 tokens 3456 -> 1152 24.0 us, 25.8 in ranges; 4143, 1024 -> 1280 17.1 / 18.4; 2300, 1664 -> 3456
+// 27.4 / 28.9; 5000, 1024 -> 2688 31.1 / 30.6.)
 struct TileCoord {
     int tile_m, tile_n;
 };
-TI8_HD TileCoord gemm_tile_of(int block_id, int tiles_m, int tiles_n, int group) {
+TI8_HD TileCoord gemm_tile_of(int block_id, int tiles_m, int tiles_n, int group, bool several) {
     const int ntiles = tiles_m * tiles_n;
-    const int xcd = block_id & 7, pid = xcd * (ntiles >> 3) + imin(xcd, ntiles & 7) + (block_id >> 3);
+    const bool ranges = (ntiles & 7) == 0 || several || group < 8 || ntiles >= 512;      // (several GEMMs in the launch; 8: tiles of 128 rows)
+    const int xcd = block_id & 7, pid = ranges ? xcd * (ntiles >> 3) + imin(xcd, ntiles & 7) + (block_id >> 3) : block_id;
     const int per_group = group * tiles_n;
     const int group_id = pid / per_group;
     const int first_m = group_id * group;
