@@ -541,13 +541,13 @@ int raw_weight_parts(int64_t R, int64_t C) {
 }
 
 // Y (cols = 0) or dX of a step on few tokens from the weight itself, W [R][C] (gemm_skinny.hip: raw_block): every element of the weight is read by one
-// lane, every K tile used by one wave of a workgroup against the codes of the same places, every element of the output [tokens] stored once
+// lane, every K tile used by one wave of a workgroup against the codes of the same places, every element of the output's first 32 rows stored once
 int walk_raw_weight(int cols, int tokens, int64_t R, int64_t C, int64_t ldw, int64_t lda, int64_t ldc, int64_t w_elems, int64_t a_elems, int64_t c_elems,
                     int64_t* n_checked, char* msg, int msglen) {
     Report r{msg, msglen};
     const int width = cols ? RAW_STRIP_DX : RAW_STRIP_Y, strips = (int)((cols ? C : R) / width), nk = (int)((cols ? R : C) >> 7), blocks = tokens > 16 ? 2 : 1;
     const int64_t n = cols ? C : R;
-    std::vector<uint8_t> read((size_t)(R * C), 0), stored((size_t)(tokens * n), 0);
+    std::vector<uint8_t> read((size_t)(R * C), 0), stored((size_t)(32 * n), 0);
     for (int block = 0; block < strips && !r.bad; ++block) {
         const int n0 = (cols ? column_strip(block, strips) : block) * width;
         for (int wave = 0; wave < 4; ++wave) {
@@ -578,10 +578,9 @@ int walk_raw_weight(int cols, int tokens, int64_t R, int64_t C, int64_t ldw, int
                         }
             }
         }
-        for (int wave = 0; wave < blocks; ++wave)
+        for (int wave = 0; wave < 2; ++wave)
             for (int lane = 0; lane < 64; ++lane) {
                 const int token = wave * 16 + (lane & 15), count = cols ? 8 : 4;
-                if (token >= tokens) continue;
                 const int64_t col = n0 + (lane >> 4) * count;
                 if (!r.access("raw weight C", token * ldc + col, count, c_elems, block, wave, lane) || col + count > n) continue;
                 for (int e = 0; e < count; ++e) ++stored[(size_t)(token * n + col + e)];

@@ -82,3 +82,28 @@ def test_step_whose_outputs_are_its_inputs(dev):
     got = T.ops.linear_step(X, W, dY, "block_channel", tokens=20, out=(torch.empty_like(dY), X, W))
     for a, b in zip(got, want):
         assert torch.equal(a[:20] if a.shape[0] == 128 else a, b[:20] if b.shape[0] == 128 else b)
+
+
+# Y and dX are computed for whole blocks of 32 rows, the last of which belong to no token: one block of 16 and two, tokens at and beside their edges; an
+# infinity in X or dY reaches the padding of its 128 x 128 tiles, one in W that of its column of Y or dX (against GEMMs on codes in memory)
+@pytest.mark.parametrize("tokens", [1, 15, 16, 17, 20, 32])
+@pytest.mark.parametrize("infinite", [False, True])
+def test_step_rows_behind_the_tokens(dev, tokens, infinite):
+    import triton_int8_amd as T
+    from triton_int8_amd._lib import PART_BACKWARD, PART_FORWARD, PART_KEEP
+    g = make_gen(tokens)
+    k, n = 640, 1152
+    X, W, dY = randn_bf16(g, 128, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev), randn_bf16(g, 128, n, std=1e-3).to(dev)
+    if infinite:
+        X[0, 200] = dY[0, 900] = float("inf")
+        W[7, 5] = -float("inf")
+    out = tuple(torch.full_like(t, 7.0) for t in (dY, X, W))
+    Y, dX, dW = T.ops.linear_step(X, W, dY, "block_channel", tokens=tokens, out=out)
+    wantY, _, _, saved = T.ops.linear_call(PART_FORWARD | PART_KEEP, "block_channel", None, tokens, k, n, X=X[:tokens], W=W)
+    _, want_dX, want_dW, _ = T.ops.linear_call(PART_BACKWARD | PART_KEEP, "block_channel", None, tokens, k, n, X=X[:tokens], W=W, dY=dY[:tokens], saved=saved)
+    for got, want in ((Y[:32], wantY[:32]), (dX[:32], want_dX[:32]), (dW, want_dW)):
+        assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(nan=0.5), want.nan_to_num(nan=0.5))
+    if not infinite:
+        assert not Y[tokens:32].any() and not dX[tokens:32].any()
+    else:
+        assert tokens == 32 or (Y[tokens:32].isnan().any() and dX[tokens:32].isnan().any())

@@ -339,7 +339,7 @@ def test_raw_weight_gemms(walker, cols, tokens, R, C):
     msg, n = ctypes.create_string_buffer(512), ctypes.c_int64(0)
     k, out, blocks = (R, C, tokens > 16) if cols else (C, R, tokens > 16)
     run = lambda *elems: walker.walk_raw_weight(cols, tokens, R, C, C + 24, k, out + 8, *elems, ctypes.byref(n), msg, 512)
-    w, a, c = (R - 1) * (C + 24) + C, (32 if blocks else 16) * k, (tokens - 1) * (out + 8) + out
+    w, a, c = (R - 1) * (C + 24) + C, (32 if blocks else 16) * k, 31 * (out + 8) + out
     assert run(w, a, c) == 0, msg.value.decode()
     for short, what in (((w - 1, a, c), b"weight W"), ((w, a - 1, c), b"weight codes"), ((w, a, c - 1), b"weight C")):
         assert run(*short) == 1 and what in msg.value

@@ -517,9 +517,9 @@ __global__ __launch_bounds__(256) void gemm_i8_few_kernel(const GemmMulti m, con
 // weight's cache lines go to four CUs).  What bounds it is the conversion, 6 instructions per element, on one or two waves per SIMD: 4096 ->
 // 4096, 13 us for Y alone, 14 for dX, 25 with dW in the launch, where the conversion both ways and the GEMMs took 29 in two.  Four waves take
 // the K tiles' quarters, each with two of them on their way; walk, sums and epilogue are those of wavering_block, operation for operation: the
-// same bits.
+// same bits, in all of its 32 rows: with one block of 16 tokens the others are the sums of zeros.
 template <bool COLS, int TB>
-__device__ __forceinline__ void raw_block(const GemmArgs& g, const RawWeight& w, const int strip, const int tokens) {
+__device__ __forceinline__ void raw_block(const GemmArgs& g, const RawWeight& w, const int strip) {
     constexpr int SETS = COLS ? 2 : 1;
     constexpr int AHEAD = 2, WORDS = COLS ? 32 : 16;
     extern __shared__ __attribute__((aligned(1024))) int8_t smem[];
@@ -660,6 +660,14 @@ __device__ __forceinline__ void raw_block(const GemmArgs& g, const RawWeight& w,
 #pragma unroll
         for (int b = 0; b < TB; ++b)
             sums[((wave * SETS + s) * TB + b) * 64 + lane] = make_float4(accf[s][b][0], accf[s][b][1], accf[s][b][2], accf[s][b][3]);
+    // a quarter's sum over codes of zero: zero, or NaN where a factor is infinite
+    float* const sums_of_zeros = reinterpret_cast<float*>(sums + 4 * SETS * TB * 64);      // [wave]
+    if (TB == 1) {
+        const float z = lane < nq ? 0.0f * f_all : 0.0f;
+        const uint64_t nan = __ballot(z != z);
+        if (lane == 0) sums_of_zeros[wave] = 0.0f;
+        if (nan && lane == __builtin_ctzll(nan)) sums_of_zeros[wave] = z;
+    }
     float scale[SETS][4];       // of those columns
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
@@ -667,15 +675,17 @@ __device__ __forceinline__ void raw_block(const GemmArgs& g, const RawWeight& w,
         if (COLS) scale[SETS - 1][r] = __shfl(scale_hi, quad * 4 + r, 64);
     }
     __syncthreads();
+    if (wave >= 2) return;
     const int token = wave * 16 + low;
-    if (wave >= TB || token >= tokens) return;
     float out[SETS][4];
 #pragma unroll
     for (int s = 0; s < SETS; ++s) {
         float part[4][4];
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
-            const float4 v = sums[((q * SETS + s) * TB + wave) * 64 + lane];
+            float4 v;
+            if (wave < TB) v = sums[((q * SETS + s) * TB + wave) * 64 + lane];
+            else v = make_float4(sums_of_zeros[q], sums_of_zeros[q], sums_of_zeros[q], sums_of_zeros[q]);
             part[q][0] = v.x; part[q][1] = v.y; part[q][2] = v.z; part[q][3] = v.w;
         }
 #pragma unroll
@@ -696,10 +706,10 @@ __device__ __forceinline__ void raw_block(const GemmArgs& g, const RawWeight& w,
 
 // dX first: its workgroups have the most to do, two that share the cache lines of the weight on one XCD
 template <int TB>
-__global__ __launch_bounds__(256) void gemm_i8_raw_weight_kernel(const GemmMulti m, const RawWeight w, const int tokens) {
+__global__ __launch_bounds__(256) void gemm_i8_raw_weight_kernel(const GemmMulti m, const RawWeight w) {
     const int block = (int)blockIdx.x;
-    if (block < m.first[1]) raw_block<true, TB>(m.g[1], w, idx::column_strip(block, m.first[1]), tokens);
-    else if (block < m.first[2]) raw_block<false, TB>(m.g[0], w, block - m.first[1], tokens);
+    if (block < m.first[1]) raw_block<true, TB>(m.g[1], w, idx::column_strip(block, m.first[1]));
+    else if (block < m.first[2]) raw_block<false, TB>(m.g[0], w, block - m.first[1]);
     else thin_walk<false, false>(m.g[2], block - m.first[2], (int)gridDim.x - m.first[2]);
 }
 
@@ -781,8 +791,8 @@ int launch_raw_weight(GemmMulti& m, const RawWeight& w, int tokens, hipStream_t 
     m.first[2] = m.first[1] + w.R / idx::RAW_STRIP_Y;
     m.first[3] = m.first[2] + (int)idx::thin_workers(w.R, w.C, device_cu_count());
     const auto kernel = tokens <= 16 ? gemm_i8_raw_weight_kernel<1> : gemm_i8_raw_weight_kernel<2>;
-    static_assert(4 * 2 * 2 * 64 * 16 <= 2 * 2 * THIN_OPERAND, "the waves' sums share the launch's LDS");
-    hipLaunchKernelGGL(kernel, dim3((unsigned)m.first[3]), dim3(256), 2 * 2 * THIN_OPERAND, st, m, w, tokens);
+    static_assert(4 * 2 * 2 * 64 * 16 + 4 * 4 <= 2 * 2 * THIN_OPERAND, "the waves' sums share the launch's LDS");
+    hipLaunchKernelGGL(kernel, dim3((unsigned)m.first[3]), dim3(256), 2 * 2 * THIN_OPERAND, st, m, w);
     note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, EPI_PROMOTE);
     return check_launch("ti8_linear");
 }
