@@ -19,10 +19,11 @@ __all__ = ["DecoderLayer", "rope_tables"]
 
 
 def rope_tables(seq_len, head_dim, device, base=10000.0):
-    device = torch.device(device)
-    if (device.type == "cuda" and device.index in (None, torch._C._cuda_getDevice()) and type(base) is float and type(seq_len) is int and seq_len > 0
-            and type(head_dim) is int and head_dim > 0 and _untraced()):
-        return ops.rope_tables(seq_len, head_dim, device, base)
+    # (device None: the default one of torch, left to it; the kernel counts in 32 bits)
+    on = torch.device("cpu" if device is None else device)
+    if (on.type == "cuda" and on.index in (None, torch._C._cuda_getDevice()) and type(base) is float and type(seq_len) is int and 0 < seq_len < 1 << 30
+            and type(head_dim) is int and 0 < head_dim < 1 << 24 and _untraced()):
+        return ops.rope_tables(seq_len, head_dim, on, base)
     return _rope_tables(seq_len, head_dim, device, base)
 
 
