@@ -453,10 +453,12 @@ class Int8Linear(torch.nn.Module):
         self._wq, self._wq_key = None, None   # quantised weight of the forward-only path and what it was made from
 
     def forward(self, x):
-        # (parameters without the search that such an attribute of a module takes)
-        own = self._parameters
-        weight = own["weight"] if "weight" in own else self.weight
-        bias = own["bias"] if "bias" in own else self.bias
+        # parameters without the search that such an attribute of a module takes, where nothing stands in front of them: an attribute of the
+        # instance or of a class derived from this one
+        own, shadows = self._parameters, self.__dict__
+        plain = type(self) is Int8Linear
+        weight = own["weight"] if plain and "weight" in own and "weight" not in shadows else self.weight
+        bias = own["bias"] if plain and "bias" in own and "bias" not in shadows else self.bias
         if torch.is_grad_enabled() and (x.requires_grad or weight.requires_grad):
             return Int8LinearFunction.apply(x, weight, bias, self.scheme, self.hadamard)
         if x.numel() == 0:
