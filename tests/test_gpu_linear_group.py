@@ -57,3 +57,19 @@ def test_kept_apart(T, dev):
         layers[0].weight.mul_(2)
     with pytest.raises(RuntimeError, match="modified by an inplace operation"):
         torch.autograd.grad(ys, x, [torch.ones_like(y) for y in ys])
+
+
+# an output that nobody uses: no gradient for its weight, the others' and the input's as those of separate calls
+@pytest.mark.parametrize("unused", [(0,), (2,), (0, 1)])
+@pytest.mark.parametrize("tokens", [37, 300])
+def test_unused_outputs(T, dev, unused, tokens):
+    layers, gen = _layers(T, dev, 256, (256, 384, 640))
+    x = torch.randn(tokens, 256, generator=gen, device=dev).to(torch.bfloat16).requires_grad_(True)
+    dys = [(1e-3 * torch.randn(tokens, m.out_features, generator=gen, device=dev)).to(torch.bfloat16) for m in layers]
+    used = [i for i in range(3) if i not in unused]
+    results = []
+    for ys in (T.decoder._projections(x, *layers), [m(x) for m in layers]):
+        results.append(torch.autograd.grad([ys[i] for i in used], [x, *(m.weight for m in layers)], [dys[i] for i in used], allow_unused=True))
+    assert [g is None for g in results[0]] == [False, *(i in unused for i in range(3))]
+    for a, b in zip(*results):
+        assert (a is None and b is None) or torch.equal(a, b)

@@ -403,15 +403,18 @@ class LinearGroupFunction(torch.autograd.Function):
     def forward(ctx, x, *weights):
         x2 = x.reshape(-1, x.shape[-1])
         ctx.save_for_backward(x2, *weights)
+        ctx.set_materialize_grads(False)
         ys, ctx.saved_q = ops.linear_group_forward(x2, weights)
         return tuple(y[:x2.shape[0]].reshape(*x.shape[:-1], y.shape[1]) for y in ys)
 
     @staticmethod
     def backward(ctx, *dys):
-        x2 = ctx.saved_tensors[0]       # (and the check that no weight has changed since)
+        x2, *weights = ctx.saved_tensors       # (and the check that no weight has changed since)
         tokens, K = x2.shape
-        dx, dws = ops.linear_group_backward([d.reshape(tokens, -1) for d in dys], K, ctx.saved_q)
-        return (dx[:tokens].reshape(*dys[0].shape[:-1], K), *dws)
+        used = next(d for d in dys if d is not None)
+        # (an output that nobody uses: its weight has no gradient)
+        dx, dws = ops.linear_group_backward([used.new_zeros((tokens, w.shape[0])) if d is None else d.reshape(tokens, -1) for d, w in zip(dys, weights)], K, ctx.saved_q)
+        return (dx[:tokens].reshape(*used.shape[:-1], K), *(None if d is None else dw for d, dw in zip(dys, dws)))
 
 
 def _one_group(x, layers):
