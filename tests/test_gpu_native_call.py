@@ -1,6 +1,12 @@
 """The layer call made from C++ gives what the Python way gives, and leaves to it what it does not take."""
+import os
+import subprocess
+import sys
+
 import pytest
 import torch
+
+from conftest import ROOT
 
 import triton_int8_amd as T
 from triton_int8_amd._lib import PART_BACKWARD, PART_FORWARD, PART_KEEP
@@ -94,3 +100,41 @@ def test_captured(dev):
             graph.replay()
             assert torch.equal(y, layer(x))
             torch.cuda.synchronize()
+
+
+ANOTHER_ALLOCATOR = """
+import ctypes, os, sys
+import torch
+hip, made = ctypes.CDLL("libamdhip64.so"), []
+
+@ctypes.CFUNCTYPE(ctypes.c_void_p, ctypes.c_ssize_t, ctypes.c_int, ctypes.c_void_p)
+def take(size, device, stream):
+    p = ctypes.c_void_p()
+    assert hip.hipMalloc(ctypes.byref(p), ctypes.c_size_t(size)) == 0
+    made.append(size)
+    return p.value
+
+@ctypes.CFUNCTYPE(None, ctypes.c_void_p, ctypes.c_ssize_t, ctypes.c_int, ctypes.c_void_p)
+def give(p, size, device, stream):
+    hip.hipFree(ctypes.c_void_p(p))
+
+address = lambda f: ctypes.cast(f, ctypes.c_void_p).value
+torch.cuda.memory.change_current_allocator(torch.cuda.memory._CUDAAllocator(torch._C._cuda_customAllocator(address(take), address(give))))
+import triton_int8_amd as T
+layer = T.Int8Linear(256, 128, device="cuda")
+x = torch.randn(300, 256, device="cuda").bfloat16()
+with torch.no_grad():
+    layer(x)
+    del made[:]
+    layer(x)
+    torch.cuda.synchronize()
+    print(T._lib.native() is not None, len(made), flush=True)
+os._exit(0)     # (nothing is freed behind the callbacks' end)
+"""
+
+
+def test_memory_comes_from_the_programs_own_allocator():
+    """Y and the workspace, in a program that has put another allocator in the place of torch's before anything was allocated."""
+    run = subprocess.run([sys.executable, "-c", ANOTHER_ALLOCATOR], cwd=ROOT, capture_output=True, text=True, timeout=100,
+                         env={**os.environ, "PYTHONPATH": ROOT})
+    assert run.returncode == 0 and run.stdout.split() == ["True", "2"], (run.returncode, run.stdout, run.stderr[-2000:])

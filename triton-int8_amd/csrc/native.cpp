@@ -6,7 +6,7 @@
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ops/empty.h>
-#include <c10/core/Allocator.h>
+#include <ATen/detail/CUDAHooksInterface.h>
 #include <c10/core/impl/DeviceGuardImplInterface.h>
 
 #include "../../include/ti8.h"
@@ -42,14 +42,15 @@ struct GilReleased {
     ~GilReleased() { PyEval_RestoreThread(state); }
 };
 
-// Device memory that a call needs until its launches are queued, from torch's allocator like a tensor's but without making one
+// Device memory that a call needs until its launches are queued, from the allocator that tensors come from at the time (a program may put its own in
+// the place of torch's) but without making one
 struct Workspace {
     c10::DataPtr plain;
     at::Tensor tensor;
     void* p;
     Workspace(int64_t bytes, const at::Device& dev, const at::TensorOptions& options) {
         if (c10::impl::getDeviceGuardImpl(c10::DeviceType::CUDA)->getDevice() == dev) {
-            plain = c10::GetAllocator(c10::DeviceType::CUDA)->allocate(bytes);
+            plain = at::detail::getCUDAHooks().getCUDADeviceAllocator()->allocate(bytes);
             p = plain.get();
         } else {
             tensor = at::empty({bytes}, options);
