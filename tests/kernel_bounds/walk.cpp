@@ -1163,6 +1163,19 @@ int walk_chain_list(const int* tiles, const int* cost, int count, int slots, int
     return r.bad;
 }
 
+// Which GEMMs of a call, over nk[i] K tiles and of tiles[i] 256 x 256 tiles (0: on another kernel), the persistent kernel takes: bit i
+int walk_chains_of_call(const int* nk, const int64_t* tiles, int count, int num_cu) {
+    bool among[3], alone[3], chains[3];
+    int bits = 0;
+    for (int i = 0; i < count; ++i) {
+        among[i] = chain_takes(nk[i], true);
+        alone[i] = chain_takes(nk[i], false);
+    }
+    chains_of_call(among, alone, tiles, count, num_cu, chains);
+    for (int i = 0; i < count; ++i) bits |= chains[i] << i;
+    return bits;
+}
+
 // Tile map of the LDS-tiled GEMMs: every tile once, and the workgroups of an XCD (every eighth) on tiles that follow each other
 int walk_gemm_tile_map(int tiles_m, int tiles_n, int group, int64_t* n_checked, char* msg, int msglen) {
     Report r{msg, msglen};

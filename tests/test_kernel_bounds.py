@@ -47,6 +47,7 @@ def walker(tmp_path_factory):
     lib.walk_quant_call.argtypes = [p64, p64, ci, ci, ci, p64, cp, ci]
     lib.walk_column_strips.argtypes = [ci, p64, cp, ci]
     lib.walk_chain_list.argtypes = [ctypes.POINTER(ci), ctypes.POINTER(ci), ci, ci, p64, cp, ci]
+    lib.walk_chains_of_call.argtypes = [ctypes.POINTER(ci), p64, ci, ci]
     lib.walk_gemm_tile_map.argtypes = [ci, ci, ci, p64, cp, ci]
     lib.walk_decode_narrow.argtypes = [ci] + [i64] * 8 + [p64, cp, ci]
     lib.walk_few_rows.argtypes = [i64] * 6 + [ci, ci] + [i64] * 3 + [p64, cp, ci]
@@ -506,6 +507,15 @@ def test_chain_list(walker, tiles, cost, slots):
     array = lambda x: (ctypes.c_int * len(x))(*x)
     assert walker.walk_chain_list(array(tiles), array(cost), len(tiles), slots, ctypes.byref(n), msg, 512) == 0, msg.value.decode()
     assert n.value == sum(tiles)
+
+
+# an odd number of K tiles from 13 on goes there beside another, alone from 19 on, also where the others of the call are on other kernels or
+# stay on one workgroup per tile; apart only in whole rounds
+@pytest.mark.parametrize("nk,tiles,taken", [([13], [256], 0), ([19], [256], 1), ([13, 15], [256, 40], 3), ([13, 32], [256, 40], 3), ([13, 9], [256, 40], 0), ([19, 9], [256, 40], 1),
+                                            ([19, 9], [200, 40], 0), ([17, 64], [256, 0], 0), ([64, 17], [256, 0], 1), ([13, 17, 9], [256, 256, 7], 3),
+                                            ([13, 9, 300], [256, 256, 256], 0), ([32, 9, 11], [512, 3, 3], 1)])
+def test_gemms_of_a_call_on_the_persistent_kernel(walker, nk, tiles, taken):
+    assert walker.walk_chains_of_call((ctypes.c_int * 3)(*nk), (ctypes.c_int64 * 3)(*tiles), len(nk), 256) == taken
 
 
 @pytest.mark.parametrize("tiles_m,tiles_n,group", [(1, 1, 4), (1, 7, 8), (3, 5, 4), (8, 8, 4), (15, 33, 4), (9, 11, 8), (8, 39, 8)])

@@ -959,24 +959,19 @@ extern "C" int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count,
         }
         idx::gemm_configs_together(shape, count, (gemm_flags & TI8_GEMM_LARGE_TILES) != 0, device_cu_count(), c);
     }
+    bool among[GEMM_MULTI_MAX], alone[GEMM_MULTI_MAX];
+    int64_t chain_tiles[GEMM_MULTI_MAX];
     for (int i = 0; i < count; ++i) {
         GemmMulti one;
         one.count = 1;
         one.g[0] = m.g[i];
-        chains[i] = persistent && c[i].epi == EPI_PROMOTE_CHAIN && chain_persistent_supported(one, count > 1);
+        const bool chained = c[i].epi == EPI_PROMOTE_CHAIN;
+        among[i] = persistent && chained && chain_persistent_supported(one, true);
+        alone[i] = persistent && chained && chain_persistent_supported(one, false);
+        chain_tiles[i] = chained ? ((problems[i].M + 255) / 256) * ((problems[i].N + 255) / 256) : 0;
     }
-    // Both kernels of the chained promotion in one call (few K tiles of an odd number keep a GEMM off the persistent one; same bits on
-    // either): apart, the persistent kernel's last round is paid for in full, so they go apart only where it fills its rounds (8576
-    // tokens, 2944 -> 12800, H_128, dX alone 408 tiles on 256 CUs: apart 1450 us, together 1406)
-    int64_t chain_tiles = 0, others = 0;
-    for (int i = 0; i < count; ++i) {
-        if (c[i].epi != EPI_PROMOTE_CHAIN) continue;
-        if (chains[i]) chain_tiles += ((problems[i].M + 255) / 256) * ((problems[i].N + 255) / 256);
-        else ++others;
-    }
-    const int64_t cus = device_cu_count(), rounds = (chain_tiles + cus - 1) / cus;
-    if (others && chain_tiles * 20 < rounds * cus * 19)
-        for (int i = 0; i < count; ++i) chains[i] = false;
+    const int64_t cus = device_cu_count();
+    idx::chains_of_call(among, alone, chain_tiles, count, (int)cus, chains);
     for (int i = 0; i < count; ++i) {
         if (done[i]) continue;
         GemmMulti part;

@@ -133,6 +133,23 @@ TI8_HD int chain_col_scale_first(int first_col_of_wave_tile, int ncols) { return
 // Beside others in a launch, which it would keep on one workgroup per tile, a GEMM goes there from 13 on (the three of a step: 15360 tokens,
 // 10112 -> 2176, one over 17 K tiles, 1147 us with one workgroup per tile, 1093; 9856, 1664 -> 1792, 13 K tiles 131, 133).
 TI8_HD bool chain_takes(int nk, bool several) { return nk >= 2 && nk <= 256 && ((nk & 1) == 0 || nk >= (several ? 13 : 19)); }
+// Which GEMMs of a call that chain their promotion go there, in one launch, the others staying on one workgroup per tile (same bits on either).
+// among[i], alone[i]: whether it takes GEMM i beside others of its launch, and by itself; tiles[i] of 256 x 256, 0 for GEMMs of other kernels.  Apart, the
+// persistent kernel's last round is paid for in full, so they go apart only where it fills its rounds (8576 tokens, 2944 -> 12800,
+// H_128, dX alone 408 tiles on 256 CUs: apart 1450 us, together 1406)
+TI8_HD void chains_of_call(const bool* among, const bool* alone, const int64_t* tiles, int count, int num_cu, bool* chains) {
+    int together = 0, others = 0;
+    int64_t chain_tiles = 0;
+    for (int i = 0; i < count; ++i) together += chains[i] = tiles[i] && among[i];
+    for (int i = 0; i < count; ++i) {
+        if (together == 1) chains[i] = chains[i] && alone[i];
+        if (chains[i]) chain_tiles += tiles[i];
+        else others += tiles[i] != 0;
+    }
+    const int64_t rounds = (chain_tiles + num_cu - 1) / num_cu;
+    if (others && chain_tiles * 20 < rounds * num_cu * 19)
+        for (int i = 0; i < count; ++i) chains[i] = false;
+}
 // K tiles that it walks
 TI8_HD int chain_walked(int nk) { return (nk + 1) & ~1; }
 // tile that workgroup `w` of `grid` takes in the round that starts at tile `base`: its own number, in a partly filled last round of a
