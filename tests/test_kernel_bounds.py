@@ -614,3 +614,14 @@ def test_raw_weight_parts(walker):
     for K in range(128, 32769, 128):
         for N in (128, 4096, 32640, 32768):
             assert walker.raw_weight_parts(K, N) <= 32 and walker.raw_weight_parts(N, K) <= 32
+
+
+# GEMMs over 13, 15 or 17 K tiles, which the persistent kernel takes beside others, priced as that launch has them: by lists, for a call as a whole
+@pytest.mark.parametrize("tokens,k,n,first,side", [(1664, 2560, 9216, 0, 256), (1920, 4096, 9216, 0, 256), (2085, 3328, 11520, 1, 256), (2761, 1664, 4992, 0, 256),
+                                                   (1664, 1024, 12288, 0, 128), (1920, 12800, 1024, 0, 128), (2780, 3712, 1664, 1, 128)])
+def test_kernels_of_a_call_over_few_odd_numbers_of_k_tiles(walker, tokens, k, n, first, side):
+    t = -(-tokens // 128) * 128
+    shapes = [(t, n, k), (t, k, n), (n, k, t)][first:]
+    cfg = (ctypes.c_int * 18)()
+    walker.walk_configs_together((ctypes.c_int64 * 9)(*sum(shapes, ())), len(shapes), 0, 256, cfg)
+    assert [tuple(cfg[9 + 3 * i:12 + 3 * i]) for i in range(len(shapes))] == [(side, side, 0)] * len(shapes)

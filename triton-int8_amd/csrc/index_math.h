@@ -565,8 +565,12 @@ TI8_HD double gemm_set_time_small(const GemmSet& s, bool i32, int num_cu) {
     return t > alone ? t : alone;
 }
 // 256 x 256 tiles, by rounds; the persistent kernel by lists where that is less (measured / predicted, us: the GEMMs of a step, 1024 tokens,
-// 4096 -> 11008 156 / 161, 1280, 3200 -> 6528 101 / 101, 1536, 2048 -> 5632 81 / 79; on four waves 165, 112, 90)
-TI8_HD double gemm_set_time_large(const GemmSet& s, bool i32, int num_cu) {
+// 4096 -> 11008 156 / 161, 1280, 3200 -> 6528 101 / 101, 1536, 2048 -> 5632 81 / 79; on four waves 165, 112, 90).  `lists`: whether a GEMM over 13, 15 or
+// 17 K tiles, which that kernel takes beside others only, may be in one.  It may where the whole call is priced (whole steps, us, on four
+// waves / so: 1664 tokens, 2560 -> 9216 213 / 183; 1920, 4096 -> 9216 346 / 313; 2176, 2048 -> 7680 187 / 156); by rounds it is no faster there (the backward
+// of 2780 tokens, 3712 -> 1664 79 / 85), and two GEMMs of a call beside a launch of the medium-size kernel lose by going apart with it (1664
+// tokens, 1024 -> 12288 0.955 of the speed, 1920, 12800 -> 1024 0.926, 2176, 1024 -> 11776 0.930).
+TI8_HD double gemm_set_time_large(const GemmSet& s, bool i32, int num_cu, bool lists) {
     int64_t tiles[3], total = 0;
     double work = 0;
     for (int i = 0; i < s.count; ++i) {
@@ -577,10 +581,13 @@ TI8_HD double gemm_set_time_large(const GemmSet& s, bool i32, int num_cu) {
     const double mean = work / num_cu, longest = (double)chain_rounds_busiest(tiles, s.nk, s.count, num_cu);
     if (i32) return 8.6 + 0.71 * longest + 0.95 * mean + 1.2 * (double)rounds;
     // a GEMM over few K tiles of an odd number keeps the launch off the persistent kernel
-    bool odd = false;
-    for (int i = 0; i < s.count; ++i) odd = odd || !chain_takes((int)s.nk[i], false);
+    bool odd = false, listed = s.count > 1;
+    for (int i = 0; i < s.count; ++i) {
+        odd = odd || !chain_takes((int)s.nk[i], false);
+        listed = listed && chain_takes((int)s.nk[i], lists);
+    }
     const double by_rounds = (7.7 + 1.15 * longest + 0.9 * mean + 0.4 * (double)rounds) * (odd ? 1.04 : 1.0);
-    if (odd || s.count < 2 || num_cu % 8 || num_cu / 8 > CHAIN_LIST_SLOTS || total > 8 * (CHAIN_LIST_MAX - s.count)) return by_rounds;
+    if (!listed || num_cu % 8 || num_cu / 8 > CHAIN_LIST_SLOTS || total > 8 * (CHAIN_LIST_MAX - s.count)) return by_rounds;
     int n[3], cost[3], first[CHAIN_LIST_SLOTS + 1];
     uint16_t order[CHAIN_LIST_MAX];
     double walked = 0;
@@ -638,12 +645,12 @@ TI8_HD void gemm_configs_together(const int64_t (*shape)[3], int count, bool lar
         if (c[i].mid) mid_tiles += gemm_set_tiles(all, q, 128);
     }
     if (bigs.count == count || (mids.count == count && mid_tiles <= num_cu)) return;
-    const double small = gemm_set_time_small(all, i32, num_cu), big = gemm_set_time_large(all, i32, num_cu);
+    const double small = gemm_set_time_small(all, i32, num_cu), big = gemm_set_time_large(all, i32, num_cu, true);
     // A launch for each kernel chosen; not for several rounds of medium-size tiles, and with 15 % on top where the four-wave kernel is
     // among them (measured over predicted: 369 / 336 us, 193 / 168, 185 / 160 at 3200, 6016 and 2176 tokens)
     double apart = mids.count == count && 4 * mid_tiles >= 5 * (int64_t)num_cu ? 1e30 : 0.0;
     if (mids.count) apart += gemm_set_time_mid(mids, i32, num_cu);
-    if (bigs.count) apart += gemm_set_time_large(bigs, i32, num_cu);
+    if (bigs.count) apart += gemm_set_time_large(bigs, i32, num_cu, false);
     if (halves.count) apart += gemm_set_time_half(halves, num_cu);
     if (smalls.count) apart = 1.15 * (apart + gemm_set_time_small(smalls, i32, num_cu));
     const double margin = 1.04;   // what the fits are off by
