@@ -121,7 +121,7 @@ const char* ti8_arch(void);
 int ti8_init(void);
 
 /* Which GEMM kernel the last ti8_gemm_i8_nt / _multi / _i32 / ti8_linear_fwd_bwd call of THIS thread launched
- * (the last one when a call launches several): kind | epilogue << 8 | (tile rows / 64) << 16 | (tile columns / 64) << 20.
+ * (the last one when a call launches several): kind | epilogue << 8 | (tile rows / 64) << 16 | (tile columns / 64) << 20 | form << 24.
  * The kernels of one family give bit-identical results whichever of them runs, so a caller (or a test) that
  * cares about WHICH one ran -- the persistent kernel is the fast one -- asks here. */
 enum ti8_gemm_kernel {
@@ -132,7 +132,15 @@ enum ti8_gemm_kernel {
     TI8_KERNEL_FEW_ROWS = 4,          /* M <= 256: 32 x 32 blocks, K split over the waves */
     TI8_KERNEL_MID = 5                /* 128 x 128 tiles on two groups of four waves, half a K tile apart */
 };
+enum ti8_gemm_form {
+    TI8_FORM_PLAIN = 0,
+    TI8_FORM_LISTS = 1,               /* TI8_KERNEL_PERSISTENT_CHAIN: the workgroups take their tiles from lists */
+    TI8_FORM_ROWS = 2,                /* TI8_KERNEL_FEW_ROWS: up to 8 rows of bf16, quantised inside, 32 columns per workgroup */
+    TI8_FORM_ROWS_NARROW = 3,         /* the same, 16 columns per workgroup */
+    TI8_FORM_WEIGHT = 4               /* TI8_KERNEL_FEW_ROWS: a step's weight quantised inside */
+};
 #define TI8_KERNEL_KIND(id) ((id) & 0xff)
+#define TI8_KERNEL_FORM(id) (((id) >> 24) & 0xff)
 int ti8_last_gemm_kernel(void);
 
 /* ---------------------------------------------------------------------------------

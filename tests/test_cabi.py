@@ -158,7 +158,7 @@ def test_latency_harness_shape_rules():
 
 
 def test_gemm_kernel_id_text():
-    """The text for a value of ti8_last_gemm_kernel (kind | epilogue << 8 | rows / 64 << 16 | columns / 64 << 20)."""
+    """The text for a value of ti8_last_gemm_kernel (kind | epilogue << 8 | rows / 64 << 16 | columns / 64 << 20 | form << 24)."""
     import triton_int8_amd
     L = triton_int8_amd._lib
     t = L.describe_gemm_kernel(L.KERNEL_PERSISTENT_CHAIN | 5 << 8 | 4 << 16 | 4 << 20)
@@ -169,6 +169,10 @@ def test_gemm_kernel_id_text():
     assert "gemm_i8_kernel" in t and "256x128" in t
     assert L.describe_gemm_kernel(L.KERNEL_FEW_ROWS) == "gemm_i8_wavering_kernel (few rows)"
     assert L.describe_gemm_kernel(0) == "none"
+    t = L.describe_gemm_kernel(L.KERNEL_PERSISTENT_CHAIN | 5 << 8 | 4 << 16 | 4 << 20 | L.FORM_LISTS << 24)
+    assert "gemm_i8_chain_kernel" in t and "256x256" in t and t.endswith("tiles from lists")
+    for form in (L.FORM_ROWS, L.FORM_ROWS_NARROW, L.FORM_WEIGHT):
+        assert "quantised inside" in L.describe_gemm_kernel(L.KERNEL_FEW_ROWS | form << 24)
 
 
 def test_linear_step_validation(lib):

@@ -3,7 +3,7 @@ import pytest
 import torch
 
 import triton_int8_amd as T
-from triton_int8_amd._lib import PART_FORWARD
+from triton_int8_amd._lib import FORM_ROWS_NARROW, PART_FORWARD, last_gemm_form
 
 pytestmark = pytest.mark.gpu
 
@@ -27,6 +27,8 @@ def test_bits(dev, tokens, k, n, scheme, bias):
     wq = T.linear.quantize_weight(W, scheme, None)
     call = lambda x: T.ops.linear_call(PART_FORWARD, scheme, None, x.shape[0], k, n, X=x, wq=wq, bias=b)[0][:tokens]
     apart = call(wide[:9, :k])
+    assert last_gemm_form() != FORM_ROWS_NARROW
     assert torch.equal(call(wide[:tokens, :k]), apart) and torch.equal(call(wide[:tokens, :k].contiguous()), apart)
+    assert (last_gemm_form() == FORM_ROWS_NARROW) == (n <= 4096 and (tokens <= 4 or k >= 3072))
     wide[0, 5], wide[0, k // 2] = float("nan"), float("inf")
     assert torch.equal(call(wide[:tokens, :k]).view(torch.int16), call(wide[:9, :k]).view(torch.int16))

@@ -59,18 +59,26 @@ def test_four_blocks_per_workgroup(dev, monkeypatch, m, n, k, mode):
 
 
 # up to 32 tokens the step's GEMMs read the weight itself: against a layer call whose weight is quantised in memory.  Fewer K tiles than waves, one
-# and several batches of them per wave, uneven quarters, rows of the weight apart
+# and several batches of them per wave, uneven quarters, rows of the weight apart; the large weights of the second block of 16 tokens, as many K tiles
+# per wave as Y can have (64) and about as many as dX can (57)
 @pytest.mark.parametrize("scheme", ["block_channel", "double_channel"])
-@pytest.mark.parametrize("tokens,k,n", [(1, 128, 384), (16, 4096, 4096), (17, 640, 1152), (31, 2176, 384), (32, 1152, 5120)])
+@pytest.mark.parametrize("tokens,k,n", [(1, 128, 384), (16, 4096, 4096), (17, 640, 1152), (31, 2176, 384), (32, 1152, 5120), (32, 14336, 4096), (20, 32768, 3328),
+                                        (5, 5760, 28800)])
 def test_step_from_the_weight_itself(dev, tokens, k, n, scheme):
     import triton_int8_amd as T
+    from triton_int8_amd._lib import FORM_WEIGHT, last_gemm_form
     g = make_gen(tokens + k + n)
-    X, W, dY = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, n, k + 32, std=0.02).to(dev)[:, 16:-16], randn_bf16(g, tokens, n, std=1e-3).to(dev)
+    X, dY = randn_bf16(g, tokens, k).to(dev), randn_bf16(g, tokens, n, std=1e-3).to(dev)
+    W = (0.02 * torch.randn(n, k + 32, generator=torch.Generator(device=dev).manual_seed(n), device=dev)).to(torch.bfloat16)[:, 16:-16]
     W[3, 5], W[:, 7] = 1.0, 0.0
     x, w = X.clone().requires_grad_(True), W.contiguous().requires_grad_(True)
     y = T.Int8LinearFunction.apply(x, w, None, scheme, None)
-    for got, want in zip(T.linear_fwd_bwd(X, W, dY, scheme), (y.detach(), *torch.autograd.grad(y, (x, w), dY))):
-        assert torch.equal(got, want)
+    want = (y.detach(), *torch.autograd.grad(y, (x, w), dY))
+    assert last_gemm_form() != FORM_WEIGHT
+    step = T.linear_fwd_bwd(X, W, dY, scheme)
+    assert (last_gemm_form() == FORM_WEIGHT) == (scheme == "block_channel")
+    for got, a in zip(step, want):
+        assert torch.equal(got, a)
 
 
 def test_step_whose_outputs_are_its_inputs(dev):
@@ -85,25 +93,26 @@ def test_step_whose_outputs_are_its_inputs(dev):
 
 
 # Y and dX are computed for whole blocks of 32 rows, the last of which belong to no token: one block of 16 and two, tokens at and beside their edges; an
-# infinity in X or dY reaches the padding of its 128 x 128 tiles, one in W that of its column of Y or dX (against GEMMs on codes in memory)
+# infinity in X or dY reaches the padding of its 128 x 128 tiles, one in W that of its column of Y or dX, NaN none (against GEMMs on codes in memory)
 @pytest.mark.parametrize("tokens", [1, 15, 16, 17, 20, 32])
-@pytest.mark.parametrize("infinite", [False, True])
-def test_step_rows_behind_the_tokens(dev, tokens, infinite):
+@pytest.mark.parametrize("special", [None, float("inf"), float("nan")])
+def test_step_rows_behind_the_tokens(dev, tokens, special):
     import triton_int8_amd as T
     from triton_int8_amd._lib import PART_BACKWARD, PART_FORWARD, PART_KEEP
     g = make_gen(tokens)
     k, n = 640, 1152
     X, W, dY = randn_bf16(g, 128, k).to(dev), randn_bf16(g, n, k, std=0.02).to(dev), randn_bf16(g, 128, n, std=1e-3).to(dev)
-    if infinite:
-        X[0, 200] = dY[0, 900] = float("inf")
-        W[7, 5] = -float("inf")
+    if special:
+        X[0, 200] = dY[0, 900] = special
+        W[7, 5] = -special
+        W[9] = W[:, 70] = W[40, 90] if special == float("inf") else special
     out = tuple(torch.full_like(t, 7.0) for t in (dY, X, W))
     Y, dX, dW = T.ops.linear_step(X, W, dY, "block_channel", tokens=tokens, out=out)
     wantY, _, _, saved = T.ops.linear_call(PART_FORWARD | PART_KEEP, "block_channel", None, tokens, k, n, X=X[:tokens], W=W)
     _, want_dX, want_dW, _ = T.ops.linear_call(PART_BACKWARD | PART_KEEP, "block_channel", None, tokens, k, n, X=X[:tokens], W=W, dY=dY[:tokens], saved=saved)
     for got, want in ((Y[:32], wantY[:32]), (dX[:32], want_dX[:32]), (dW, want_dW)):
         assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.nan_to_num(nan=0.5), want.nan_to_num(nan=0.5))
-    if not infinite:
+    if special != float("inf"):
         assert not Y[tokens:32].any() and not dX[tokens:32].any()
     else:
         assert tokens == 32 or (Y[tokens:32].isnan().any() and dX[tokens:32].isnan().any())

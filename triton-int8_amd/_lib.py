@@ -96,6 +96,7 @@ SCHEME_BLOCK_CHANNEL, SCHEME_ROW_BLOCK, SCHEME_DOUBLE_CHANNEL = 0, 1, 2
 PART_FORWARD, PART_BACKWARD, PART_KEEP = 1, 2, 4
 HADAMARD_FULL = -1
 KERNEL_NONE, KERNEL_ONE_TILE, KERNEL_ONE_TILE_MULTI, KERNEL_PERSISTENT_CHAIN, KERNEL_FEW_ROWS, KERNEL_MID = 0, 1, 2, 3, 4, 5
+FORM_PLAIN, FORM_LISTS, FORM_ROWS, FORM_ROWS_NARROW, FORM_WEIGHT = 0, 1, 2, 3, 4
 
 _lib = None
 
@@ -235,17 +236,24 @@ _KINDS = {KERNEL_NONE: "none", KERNEL_ONE_TILE: "gemm_i8_kernel (one workgroup p
           KERNEL_PERSISTENT_CHAIN: "gemm_i8_chain_kernel (persistent workgroups)",
           KERNEL_FEW_ROWS: "gemm_i8_wavering_kernel (few rows)",
           KERNEL_MID: "gemm_i8_mid_kernel (two groups of waves half a K tile apart)"}
+_FORMS = {FORM_LISTS: ", tiles from lists", FORM_ROWS: ", rows quantised inside", FORM_ROWS_NARROW: ", rows quantised inside, 16 columns per workgroup",
+          FORM_WEIGHT: ", weight quantised inside"}
 
 
 def describe_gemm_kernel(kernel_id=None):
-    """Text for a value of ``ti8_last_gemm_kernel`` (default: the current one): kernel, tile, epilogue."""
+    """Text for a value of ``ti8_last_gemm_kernel`` (default: the current one): kernel, tile, epilogue, form."""
     if kernel_id is None:
         kernel_id = lib().ti8_last_gemm_kernel()
     kind, epi, bm, bn = kernel_id & 0xff, (kernel_id >> 8) & 0xff, ((kernel_id >> 16) & 0xf) * 64, ((kernel_id >> 20) & 0xf) * 64
-    name = _KINDS.get(kind, f"kernel kind {kind}")
+    name, form = _KINDS.get(kind, f"kernel kind {kind}"), _FORMS.get(last_gemm_form(kernel_id), "")
     if kind in (KERNEL_NONE, KERNEL_FEW_ROWS):
-        return name
-    return f"{name}, {bm}x{bn} tiles, {_EPILOGUES[epi] if epi < len(_EPILOGUES) else epi}"
+        return name + form
+    return f"{name}, {bm}x{bn} tiles, {_EPILOGUES[epi] if epi < len(_EPILOGUES) else epi}{form}"
+
+
+def last_gemm_form(kernel_id=None):
+    """``FORM_*`` of a value of ``ti8_last_gemm_kernel`` (default: the current one)."""
+    return ((lib().ti8_last_gemm_kernel() if kernel_id is None else kernel_id) >> 24) & 0xff
 
 
 def last_gemm_kernel():

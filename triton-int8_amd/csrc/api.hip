@@ -9,8 +9,8 @@ char* err_buf() {
 }
 
 static thread_local int last_gemm_kernel = TI8_KERNEL_NONE;
-void note_gemm_kernel(int kind, int bm, int bn, int epi) {
-    last_gemm_kernel = kind | (epi << 8) | ((bm / 64) << 16) | ((bn / 64) << 20);
+void note_gemm_kernel(int kind, int bm, int bn, int epi, int form) {
+    last_gemm_kernel = kind | (epi << 8) | ((bm / 64) << 16) | ((bn / 64) << 20) | (form << 24);
 }
 
 int device_cu_count() {

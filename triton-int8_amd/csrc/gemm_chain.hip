@@ -652,7 +652,7 @@ int launch_chain_persistent(const GemmMulti& m, int total_tiles, int num_cu, hip
 int launch_chain_listed(const GemmMulti& m, const ChainList& list, int num_cu, hipStream_t st) {
     if (!chain_kernel_available<CHAIN_LISTED>()) return CHAIN_UNAVAILABLE;
     hipLaunchKernelGGL(gemm_i8_chain_listed_kernel, dim3((unsigned)num_cu), dim3(64 * NW), LDS_BYTES, st, m, list);
-    note_gemm_kernel(TI8_KERNEL_PERSISTENT_CHAIN, BM, BN, EPI_PROMOTE_CHAIN);
+    note_gemm_kernel(TI8_KERNEL_PERSISTENT_CHAIN, BM, BN, EPI_PROMOTE_CHAIN, TI8_FORM_LISTS);
     return check_launch("ti8_gemm_i8_nt");
 }
 

@@ -191,7 +191,7 @@ int launch_decode_narrow(const GemmArgs& a, int rows, bool i32_full, hipStream_t
     if (i32_full) launch_mode<Decode::ROWS_I32>(a, rows, st);
     else if (a.sa.mode == TI8_SCALE_ROW) launch_mode<Decode::ROWS>(a, rows, st);
     else launch_mode<Decode::TILES>(a, rows, st);
-    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
+    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE, TI8_FORM_ROWS_NARROW);
     return check_launch("ti8_gemm_i8_nt");
 }
 

@@ -765,7 +765,7 @@ int launch_decode(const GemmArgs& a, int rows, bool i32_full, hipStream_t st) {
     const auto kernel = i32_full ? gemm_i8_decode_kernel<true, BY_ROWS>
                                  : a.sa.mode == TI8_SCALE_ROW ? gemm_i8_decode_kernel<false, BY_ROWS> : gemm_i8_decode_kernel<false, BY_TILES>;
     hipLaunchKernelGGL(kernel, dim3((unsigned)(a.N / 32)), dim3(256), lds, st, a, rows);
-    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE);
+    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, i32_full ? EPI_ROWS : EPI_PROMOTE, TI8_FORM_ROWS);
     return check_launch("ti8_gemm_i8_nt");
 }
 
@@ -793,7 +793,7 @@ int launch_raw_weight(GemmMulti& m, const RawWeight& w, int tokens, hipStream_t 
     const auto kernel = tokens <= 16 ? gemm_i8_raw_weight_kernel<1> : gemm_i8_raw_weight_kernel<2>;
     static_assert(4 * 2 * 2 * 64 * 16 + 4 * 4 <= 2 * 2 * THIN_OPERAND, "the waves' sums share the launch's LDS");
     hipLaunchKernelGGL(kernel, dim3((unsigned)m.first[3]), dim3(256), 2 * 2 * THIN_OPERAND, st, m, w);
-    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, EPI_PROMOTE);
+    note_gemm_kernel(TI8_KERNEL_FEW_ROWS, 32, 32, EPI_PROMOTE, TI8_FORM_WEIGHT);
     return check_launch("ti8_linear");
 }
 

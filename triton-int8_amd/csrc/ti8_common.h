@@ -149,7 +149,7 @@ int add_bias(void* y, int64_t ldy, const void* bias, int64_t rows, int64_t cols,
 int sum_partials(const char* fn, const float* partial, int groups, int64_t dim, void* out, hipStream_t st);
 
 // ---- which kernel served the last GEMM call of this thread (ti8_last_gemm_kernel) ---
-void note_gemm_kernel(int kind, int bm, int bn, int epi);
+void note_gemm_kernel(int kind, int bm, int bn, int epi, int form = TI8_FORM_PLAIN);
 
 // ---- device helpers --------------------------------------------------------------
 typedef int v4i __attribute__((ext_vector_type(4)));
