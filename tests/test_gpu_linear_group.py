@@ -73,3 +73,21 @@ def test_unused_outputs(T, dev, unused, tokens):
     assert [g is None for g in results[0]] == [False, *(i in unused for i in range(3))]
     for a, b in zip(*results):
         assert (a is None and b is None) or torch.equal(a, b)
+
+
+@pytest.mark.parametrize("special", [float("inf"), float("nan")])
+@pytest.mark.parametrize("tokens", [37, 300])
+def test_non_finite_values(T, dev, special, tokens):
+    layers, gen = _layers(T, dev, 384, (384, 512))
+    x = torch.randn(tokens, 384, generator=gen, device=dev).to(torch.bfloat16)
+    dys = [(1e-3 * torch.randn(tokens, m.out_features, generator=gen, device=dev)).to(torch.bfloat16) for m in layers]
+    x[5, 130], dys[1][7, 3] = special, -special
+    with torch.no_grad():
+        layers[0].weight[9, 70] = special
+        layers[1].weight[:, 300] = special
+    x.requires_grad_(True)
+    wanted = [x, *(m.weight for m in layers)]
+    together, apart = T.decoder._projections(x, *layers), [m(x) for m in layers]
+    assert type(together[0].grad_fn).__name__ == "LinearGroupFunctionBackward"
+    for a, b in zip((*together, *torch.autograd.grad(together, wanted, dys)), (*apart, *torch.autograd.grad(apart, wanted, dys))):
+        assert torch.equal(a.isnan(), b.isnan()) and torch.equal(a.nan_to_num(nan=0.5), b.nan_to_num(nan=0.5))

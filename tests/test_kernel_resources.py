@@ -124,6 +124,21 @@ def loops(body):
             yield body[m.end():m.end() + back[-1].end()]
 
 
+# tiles from lists; operand B scaled per (row, K tile), whose epilogue has no column scales
+@pytest.mark.parametrize("name, variants", [("gemm_i8_chain_listed_kernel", 8), ("gemm_i8_chain_lane_kernel", 4)])
+def test_other_forms_of_the_chain_kernel_wait_like_it(tmp_path, name, variants):
+    """As above: 16 stores of 16 bytes per variant of the epilogue in one piece, waits for 16 and 20, no scratch, two waves per SIMD."""
+    (body,) = kernel_bodies("gemm_chain.hip", tmp_path, name).values()
+    assert re.search(r"\.amdhsa_private_segment_fixed_size 0\b", body)
+    assert int(re.search(r"\.amdhsa_next_free_vgpr (\d+)", body).group(1)) <= 256
+    stores = re.findall(r"^\s*(global_store_\w+|buffer_store_\w+|flat_store_\w+|scratch_store_\w+)", body, flags=re.M)
+    assert stores == ["global_store_dwordx4"] * (variants * 16)
+    for block in re.split(r"^\.LBB\S+:|^\s*s_cbranch\w+|^\s*s_branch", body, flags=re.M):
+        assert len(re.findall(r"^\s*global_store_dwordx4", block, flags=re.M)) in (0, 16)
+    waits = {int(w) for w in re.findall(r"s_waitcnt vmcnt\((\d+)\)", body)}
+    assert {16, 20} <= waits and max(waits) == 20
+
+
 def test_few_tokens_kernel_waits_match_its_stores(tmp_path):
     """The walk over dW's tiles waits with vmcnt(8) for the next K tile while the stores of the tile before may be in flight: safe while
     a wave issues exactly 8 memory instructions behind that K tile's loads, its stores of 16 bytes, with nothing branching between."""
