@@ -68,6 +68,27 @@ def test_served(dev, monkeypatch, scheme, hadamard, tokens):
         assert torch.equal(y, want)
 
 
+@pytest.mark.filterwarnings("ignore::torch.jit.TracerWarning", "ignore:.torch.jit:DeprecationWarning")
+@pytest.mark.parametrize("tokens", [3, 300])
+def test_served_where_operators_are_followed(dev, tokens):
+    """Y's cut to its tokens is an operator that a tracer and a dispatch mode see (the launches are not)."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+    layer, x = T.Int8Linear(256, 384, device=dev), torch.randn(1, tokens, 256, device=dev).to(torch.bfloat16)
+
+    class Names(TorchDispatchMode):
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            names.append(func.overloadpacket.__name__)
+            return func(*args, **(kwargs or {}))
+
+    names = []
+    with torch.no_grad():
+        want = layer(x)
+        assert torch.jit.trace(layer, x, check_trace=False)(x).shape == want.shape
+        with Names():
+            y = layer(x)
+        assert torch.equal(y, want) and "slice" in names
+
+
 def test_what_it_leaves_to_the_python_way(dev, monkeypatch):
     X, W = torch.randn(5, 256, device=dev).to(torch.bfloat16), torch.randn(128, 256, device=dev).to(torch.bfloat16)
     call = lambda x: T.ops.linear_call(PART_FORWARD, "block_channel", None, 5, 256, 128, X=x, W=W)[0][:5]

@@ -7,7 +7,11 @@
 #include <torch/csrc/autograd/python_variable.h>
 #include <ATen/ops/empty.h>
 #include <ATen/detail/CUDAHooksInterface.h>
+#include <ATen/ops/narrow.h>
+#include <ATen/TracerMode.h>
 #include <c10/core/impl/DeviceGuardImplInterface.h>
+#include <c10/core/impl/LocalDispatchKeySet.h>
+#include <c10/core/impl/TorchDispatchModeTLS.h>
 
 #include "../../include/ti8.h"
 
@@ -58,6 +62,12 @@ struct Workspace {
         }
     }
 };
+
+// Whether a tracer, a dispatch mode or a function transform looks at the operators of this thread
+bool followed() {
+    return at::tracer::impl::is_dispatch_enabled() || c10::impl::dispatch_mode_enabled() ||
+           c10::impl::tls_is_dispatch_key_included(c10::DispatchKey::FuncTorchDynamicLayerFrontMode);
+}
 
 PyObject* wrap(const at::Tensor& t) {
     if (t.defined()) return THPVariable_Wrap(t);
@@ -136,7 +146,9 @@ PyObject* linear_call(PyObject*, PyObject* const* args, Py_ssize_t nargs) {
     }
     if (status != TI8_OK) return Py_BuildValue("(si)", name, status);
     if (v[SERVED]) {
-        Y.unsafeGetTensorImpl()->set_sizes_contiguous({v[TOKENS], v[N_]});
+        // (in its own sizes, unless something follows what is made of Y operator by operator)
+        if (followed()) Y = Y.narrow(0, 0, v[TOKENS]);
+        else Y.unsafeGetTensorImpl()->set_sizes_contiguous({v[TOKENS], v[N_]});
         return wrap(Y);
     }
     return Py_BuildValue("(NNNN)", wrap(Y), wrap(dX), wrap(dW), wrap(saved));
