@@ -385,7 +385,7 @@ int ti8_gemm_i8_nt_multi(const ti8_gemm_problem* problems, int count, int gemm_f
  *   scratch memory as well until the GEMMs write them (nothing beyond their rows and columns is touched).
  *   They may be the inputs' memory.  Outputs that share memory are written one after the other, Y, dX, dW.
  *   gemm_flags: TI8_GEMM_TILED / TI8_GEMM_LARGE_TILES / TI8_GEMM_ONE_TILE or 0.
- * A block-channel step on few tokens may quantise its weight inside the GEMMs instead.
+ * A block-channel step on few tokens may quantise its weight inside the GEMMs instead, with the same bits in the same rows.
  * Nothing is allocated; the call only enqueues kernels, so it may be captured into a graph. */
 enum ti8_scheme {
     TI8_SCHEME_BLOCK_CHANNEL = 0,
@@ -443,13 +443,15 @@ int64_t ti8_linear_workspace(const ti8_linear_args* a, int64_t* saved_bytes);
 int ti8_linear_quantise(const ti8_linear_args* a, ti8_gemm_problem* problems, int* count, ti8_stream_t stream);
 /* enqueue everything.  With more than 256 (padded) tokens and output features the GEMMs of a call go through
  * ti8_gemm_i8_nt_multi (TI8_PART_FORWARD alone: ti8_gemm_i8_nt, the same kernel), else each takes the kernel of ti8_gemm_i8_nt
- * (those on the few-rows kernel in one launch; up to 8 unrotated rows may be quantised inside it), Y and dX for the first ceil(tokens / 32) * 32 rows only. */
+ * (those on the few-rows kernel in one launch; up to 8 unrotated rows may be quantised inside it); of Y and dX no more than the first
+ * ceil(tokens / 32) * 32 rows are then written. */
 int ti8_linear(const ti8_linear_args* a, ti8_stream_t stream);
 /* 2 or 3 layers that multiply the same X (the projections of an attention, gate and up of an MLP), block-channel without rotation or
  * bias: the forward of all (TI8_PART_FORWARD | TI8_PART_KEEP) or their backward (TI8_PART_BACKWARD | TI8_PART_KEEP), with X quantised once.
  * Y and dW of each layer have the bits of ti8_linear; the first layer's dX is the sum of the layers' dX, bf16 sums from the last layer to the
  * first (those that autograd makes of separate calls), the others' dX is not looked at.  `saved` and the workspace of the call are the first
- * layer's.  parts, X, tokens, K and gemm_flags are those of all; N, W, dY, Y and dW the layer's own, outputs that share no memory. */
+ * layer's.  parts, X, tokens, K and gemm_flags are those of all; N, W, dY, Y and dW the layer's own, outputs that share no memory.  The workspace of
+ * a backward holds the codes of all dY at once and [T][K] of bf16 for the dX of each layer but the first. */
 int64_t ti8_linear_group_workspace(const ti8_linear_args* a, int count, int64_t* saved_bytes);
 int ti8_linear_group(const ti8_linear_args* a, int count, ti8_stream_t stream);
 /* Column sums of x bf16 [rows][cols] (ldx), added up in fp32 and rounded once: the gradient of a bias.  cols a multiple of 32;

@@ -494,7 +494,7 @@ __device__ __forceinline__ void chain_tiles(const GemmMulti& m, const int total_
         using F_ = std::false_type;
         using P0 = std::integral_constant<int, 0>;
         using P1 = std::integral_constant<int, 1>;
-        // K / 128 is even: a tile starts in LDS buffer 0 and its K tiles alternate 0, 1, 0, 1, ...
+        // nk is even: a tile starts in LDS buffer 0 and its K tiles alternate 0, 1, 0, 1, ...
         {
             const bool a_next = 2 >= nk;
             ktile_p(T_{}, T_{}, P0{}, stored, fvec, 0, cur, 128, a_next ? nxt : cur, a_next ? 0 : k_at(2));

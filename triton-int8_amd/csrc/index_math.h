@@ -24,11 +24,11 @@ TI8_HD int imax(int a, int b) { return a > b ? a : b; }
 
 // workgroup id -> (tile_m, tile_n): mostly one contiguous range of tiles per XCD (ids 8 apart share an
 // XCD; the first ones have a tile more where 8 does not divide their number), then groups of `group` tile rows walked column by
-// column inside a group.  (In their own order, those numbers spread neighbours over all XCDs: three GEMMs of a step in one launch, int32,
-// 512 tokens 2176 -> 4992 40.3 us, 34.6 this way; 640, 8320 -> 1408 55.9 / 48.3; 1152, 8832 -> 3584 135 / 127; 3712, 7168 -> 8320
-// 588 / 570; 13056, 7168 -> 11648 2680 / 2637.  But a GEMM alone on up to 512 tiles of 128 rows, about two per CU, is faster when the XCDs read
-// the same panel of B at the same time: 1144 tokens 3456 -> 1152 24.0 us, 25.8 in ranges; 4143, 1024 -> 1280 17.1 / 18.4; 2300, 1664 -> 3456
-// 27.4 / 28.9; 5000, 1024 -> 2688 31.1 / 30.6.)
+// column inside a group.  A number of tiles that 8 divides is in ranges whatever the launch.  Others, us in their own order, which spreads neighbours
+// over all XCDs / in ranges: three GEMMs of a step in one launch, int32, 512 tokens 2176 -> 4992 40.3 / 34.6; 640, 8320 -> 1408 55.9 / 48.3; 1152,
+// 8832 -> 3584 135 / 127; 3712, 7168 -> 8320 588 / 570; 13056, 7168 -> 11648 2680 / 2637.  A GEMM alone on fewer than 512 tiles of 128 rows, about
+// two per CU, keeps its own order, in which the XCDs read the same panel of B at the same time: 1144 tokens 3456 -> 1152 (81 tiles) 24.0 / 25.8;
+// 4143, 1024 -> 1280 (330) 17.1 / 18.4; 2300, 1664 -> 3456 (486) 27.4 / 28.9; from there on ranges: 5000, 1024 -> 2688 (840) 31.1 / 30.6.
 struct TileCoord {
     int tile_m, tile_n;
 };
@@ -410,7 +410,8 @@ constexpr int RAW_PARTS = 32;
 TI8_HD int raw_part(int i, int lane, int count) { return imin((lane >> 4) + 4 * i, count - 1); }
 // Whether such a step takes them.  A workgroup walks the whole contraction, so a side much longer than the other leaves few of them with long
 // walks; and for a second block of 16 tokens the codes are read twice as often, which costs what the saved launch gains, but on a small weight and
-// on one whose codes both ways no longer fit the Infinity Cache beside it.
+// on one whose codes both ways no longer fit the Infinity Cache (256 MiB) beside it and what the GEMMs write: 4 bytes per element of the weight
+// and 2 of dW, 336 MiB at 14336 x 4096; at 8960 x 4864, 249 MiB, the gain (89.6 / 87.1) is what neighbours lose (5632 x 4736 60.8 / 63.7).
 // The step, us, its weight quantised in memory / so: 16 tokens, 4096 -> 4096 37.7 / 32.5, 2048 -> 2048 22.3 / 17.3, 7936 -> 8960 177 / 132,
 // 13440 -> 3200 89.8 / 76.1, 3200 -> 13440 88.6 / 75.0, 10240 -> 1024 37.1 / 34.5, 14336 -> 1024 44.8 / 45.9, 2048 -> 14336 62.7 / 62.4, 1536
 // -> 8960 37.3 / 39.5, 1024 -> 14336 41.5 / 49.1; 32 tokens, 2048 -> 2048 22.3 / 17.2, 2560 -> 2560 26.8 / 22.4, 3072 -> 3072 29.3 / 29.0,

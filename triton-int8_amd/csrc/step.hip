@@ -55,7 +55,8 @@ struct Layer {
     int64_t partial_words(int64_t R, int64_t C) const { return partials_in_outputs || !quant_together(both_ways_bytes()) ? 0 : maxima_piece(quant_maxima_words(R, C)); }
     int64_t both_ways_words(int64_t R, int64_t C) const { return maxima_piece(R + C) + partial_words(R, C); }
     // whether the transposed copies in front of the rotations are made together (quant_fwht_call): while they find room in the Infinity Cache, and
-    // in a workspace of about the operands' size (8192 tokens, 8192 -> 8192 takes 1807 us either way)
+    // in a workspace of about the operands' size (8192 tokens, 8192 -> 8192 takes 1807 us either way): up to 192 MiB for the copies of a backward, where
+    // one after the other they take the largest one's
     bool rotates_together() const { return 2 * (N * K + T * N + T * K) <= ROTATE_TOGETHER_BYTES; }
     // what an unrotated forward quantises for the backward in the same pass
     bool shares() const { return had == 0 && (keep || (fwd && bwd)); }
@@ -450,7 +451,9 @@ int run_layer(const char* fn, const ti8_linear_args* a, int64_t T, ti8_gemm_prob
 // ---- layers on the same X ----------------------------------------------------------------
 // The seven linears of a decoder layer are three calls of this kind (q, k, v; gate, up) and two alone: X is quantised once for a
 // call, the weights' (the dYs') quantisers are two launches (one) for all of it and the GEMMs one (two).  The whole layer, us apart
-// / so: 3 x 1360 tokens, hidden 2048, MLP 4992 1768 / 1609; 4 x 4096, hidden 4096, MLP 14336 18530 / 18170.
+// / so: 3 x 1360 tokens, hidden 2048, MLP 4992 1634 / 1497; 4 x 4096, hidden 4096, MLP 14336 18270 / 17930.  In memory, the backward holds the codes of
+// all its dY at once (gate and up of 16384 x 14336: 940 MB, apart 470) and a [T][K] dX of each further layer, the layers between the directions
+// X's codes and scales once: peak of the larger layer 4779 MiB, apart 4939, of the smaller 589 / 584.
 constexpr int GROUP_MAX = 3;
 struct Group {
     Layer L[GROUP_MAX];
