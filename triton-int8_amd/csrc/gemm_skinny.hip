@@ -514,8 +514,9 @@ __global__ __launch_bounds__(256) void gemm_i8_few_kernel(const GemmMulti m, con
 // few tokens costs more to quantise into memory (its codes written both ways and read again) than to read twice.  16x16x64 products want 16 codes in a row
 // along the contraction: for Y what two loads bring; for dX a lane loads 2 columns of 16 rows and the conversion, which
 // places single bytes, transposes them (a single column per lane, which gives every CU a workgroup: 22 us for Y and dX instead of 20, the
-// weight's cache lines go to four CUs).  What bounds it is the conversion, 6 instructions per element, on one or two waves per SIMD: 4096 ->
-// 4096, 13 us for Y alone, 14 for dX, 25 with dW in the launch, where the conversion both ways and the GEMMs took 29 in two.  Four waves take
+// weight's cache lines go to four CUs).  What bounds it is the chain of load, conversion (6 instructions per element, about 5 us of issue both ways)
+// and product in one or two waves per SIMD: 4096 -> 4096, 13 us for Y alone, 14 for dX, 25 with dW in the launch, where the conversion both ways and
+// the GEMMs took 29 in two.  Four waves take
 // the K tiles' quarters, each with two of them on their way; walk, sums and epilogue are those of wavering_block, operation for operation: the
 // same bits, in all of its 32 rows: with one block of 16 tokens the others are the sums of zeros.
 template <bool COLS, int TB>
